@@ -19,6 +19,7 @@ import torch
 import torch.nn as nn
 
 from omni_moe.ops.hip import hip_omni_expert_func, hip_omni_mlp_func, hip_omni_moe_fwd_func, hip_omni_router_fwd_func
+from omni_moe.ops.hip.interface import layer_forward
 
 
 _BRANCH_RESOURCES = {}      # (device index, host thread) -> (side stream, fork event, join event)
@@ -136,6 +137,10 @@ class OmniMoE(nn.Module):
         return (mlp_states + experts_states).view(bsz, seq_len, -1)
 
     def forward(self, hidden_states: torch.Tensor, **kwargs) -> torch.Tensor:
+        if hidden_states.is_cuda and type(self) is OmniMoE:
+            out = layer_forward(self, hidden_states)          # the ordinary call; what follows is for everything else
+            if out is not None:
+                return out
         bsz, seq_len, _ = hidden_states.shape
         if torch.is_grad_enabled() and (hidden_states.requires_grad or any(p.requires_grad for p in self.parameters())):
             return self._forward_differentiable(hidden_states)

@@ -8,6 +8,7 @@ is made without a GPU, an exception is raised.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from ctypes import c_char_p, c_float, c_int32, c_int64, c_size_t, c_void_p
 
@@ -83,6 +84,24 @@ def load() -> ctypes.CDLL:
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The torch host path (csrc/torch_ops.cpp), loaded once; it links the library above."""
+    global _native
+    if _native is None:
+        load()
+        path = os.path.join(_HERE, "_native.so")
+        if not os.path.exists(path):
+            raise OmniHipError(f"{path} is missing: build it with `python -m omni_moe.ops.hip.build`")
+        spec = importlib.util.spec_from_file_location("_native", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _native = module
+    return _native
 
 
 def check(code: int, what: str) -> None:

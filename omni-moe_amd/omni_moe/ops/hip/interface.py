@@ -8,6 +8,10 @@ autograd is recording and an input requires grad, the router, expert and MLP ope
 through ``torch.autograd.Function`` wrappers (``OmniRouterFunc``, ``OmniExpertFunc``,
 ``OmniSwiGLUFunc``, ``OmniLinearFunc``) whose backward passes are HIP kernels too (GEMM
 gradients are library matmuls, as in the reference).  Otherwise no graph is built.
+
+The operators that a model calls step after step first offer the call to the native host path (``_lib.native()``,
+``csrc/torch_ops.cpp``), which takes contiguous tensors of matching shapes on one GPU and answers None to anything else:
+what follows here then makes tensors contiguous and raises the contract's errors.
 """
 from __future__ import annotations
 
@@ -34,6 +38,10 @@ def hip_omni_router_func(
     Mirrors ``triton_omni_router_func`` (reference interface.py:32-51) and the input
     contract of ``assert_omni_router_fwd_inputs`` (utils.py:81-104).
     """
+    if router_logits_x.is_cuda and router_logits_y.is_cuda:
+        out = _lib.native().router_select(router_logits_x, router_logits_y, int(num_expert_sqrt), int(num_experts_per_token))
+        if out is not None:
+            return out
     assert router_logits_x.dim() == 2, "router_logits_x must be a 2D tensor of shape (num_tokens, num_expert_sqrt)"
     assert router_logits_y.dim() == 2, "router_logits_y must be a 2D tensor of shape (num_tokens, num_expert_sqrt)"
     assert router_logits_x.size(0) == router_logits_y.size(0), (
@@ -94,7 +102,7 @@ class OmniRouterFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, router_logits_x, router_logits_y, num_expert_sqrt, num_experts_per_token):
-        scores, indices = _router_select(router_logits_x, router_logits_y, num_expert_sqrt, num_experts_per_token)
+        scores, indices = _router_select(router_logits_x, router_logits_y, int(num_expert_sqrt), int(num_experts_per_token))
         ctx.save_for_backward(indices)
         ctx.num_expert_sqrt = num_expert_sqrt
         ctx.mark_non_differentiable(indices)
@@ -154,6 +162,10 @@ def hip_omni_expert_func(
 
     Mirrors ``triton_omni_expert_func`` (reference interface.py:54-72).
     """
+    if x.is_cuda and algo in _ALGOS:
+        y = _lib.native().expert(x, up_weight, down_weight, routing_weights, indices, _ALGOS[algo])
+        if y is not None:
+            return y
     if x.dim() != 2 or up_weight.dim() != 2 or down_weight.dim() != 2:
         raise ValueError("x, up_weight and down_weight must be 2D")
     if routing_weights.shape != indices.shape or routing_weights.dim() != 2 or routing_weights.size(0) != x.size(0):
@@ -241,6 +253,10 @@ def hip_omni_mlp_func(
     counterpart there: the layer uses it to fold its final ``mlp + experts`` add
     (omni_moe.py:102) into the down projection's epilogue.
     """
+    if x.is_cuda:
+        y = _lib.native().mlp(x, gate_weight, up_weight, down_weight, residual)
+        if y is not None:
+            return y
     if x.dim() != 2 or gate_weight.dim() != 2 or up_weight.dim() != 2 or down_weight.dim() != 2:
         raise ValueError("x and the three weights must be 2D")
     T, H = x.shape
@@ -463,6 +479,11 @@ def hip_omni_router_fwd_func(
     Returns (gates [T,k] in x's dtype, indices [T,k] int32[, scores]).  In training mode the
     running buffers are updated in place, as nn.BatchNorm1d does.
     """
+    if x.is_cuda and not return_scores and momentum is not None:
+        out = _lib.native().router_stage(x, weight_x, weight_y, running_mean_x, running_var_x, num_batches_tracked_x, running_mean_y, running_var_y,
+                                         num_batches_tracked_y, int(num_experts_per_token), bool(training), momentum, eps)
+        if out is not None:
+            return out
     if x.dim() != 2 or weight_x.shape != weight_y.shape or weight_x.dim() != 2 or weight_x.size(1) != x.size(1):
         raise ValueError("expected x (tokens, hidden) and two router weights (num_expert_sqrt, hidden)")
     if x.dtype not in _lib.DTYPE_CODE or weight_x.dtype != x.dtype or weight_y.dtype != x.dtype:
@@ -565,6 +586,12 @@ class OmniRouterStageFunc(torch.autograd.Function):
         dw = dz.t().matmul(x) if (ctx.needs_input_grad[1] or ctx.needs_input_grad[2]) else None
         dx = dz.matmul(torch.cat([weight_x, weight_y])) if ctx.needs_input_grad[0] else None
         return (dx, dw[:r] if dw is not None else None, dw[r:] if dw is not None else None) + (None,) * 10
+
+
+def layer_forward(layer, hidden_states: torch.Tensor) -> Optional[torch.Tensor]:
+    """``OmniMoE.forward`` of an unmodified module through the native host path (no-grad: one library call; recording: one
+    differentiable node), or None if it does not take the call."""
+    return _lib.native().layer_forward(layer, hidden_states, _ALGOS)
 
 
 def hip_omni_moe_fwd_func(
