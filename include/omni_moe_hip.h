@@ -160,7 +160,7 @@ OMNI_API int32_t omni_expert_fwd(const void* x, const void* up_weight, const voi
  *   x [T,H]; gate_weight, up_weight [I,H]; down_weight [H,I]; y [T,H]  (bf16, f16 or f32)
  *   residual : NULL, or [T,H] added to the rounded down projection and rounded again
  *              (the layer's final  mlp + experts , omni_moe.py:102)
- *   workspace: omni_mlp_workspace_bytes() bytes (the [T,I] SwiGLU activations)
+ *   workspace: omni_mlp_workspace_bytes() bytes (the [T,I] SwiGLU activations, and fp32 partial sums where a projection is split along K)
  * H and I must be multiples of 8 (of 4 for f32): rows are fetched 16 bytes at a time. */
 OMNI_API size_t omni_mlp_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t dtype);
 OMNI_API int32_t omni_mlp_fwd(const void* x, const void* gate_weight, const void* up_weight, const void* down_weight,
@@ -180,7 +180,7 @@ OMNI_API int32_t omni_swiglu_linear_fwd(const void* x, const void* gate_weight, 
 OMNI_API int32_t omni_linear_fwd(const void* x, const void* weight, const void* residual, void* y, int64_t num_tokens,
                                  int32_t in_features, int32_t out_features, int32_t dtype, void* stream);
 
-/* omni_swiglu_linear_fwd for callers that run other kernels beside it (another stream).  Where the product has at least 256
+/* omni_swiglu_linear_fwd for callers that run other kernels beside it (another stream).  Where the product has more than 256
  * tiles of 256 x 256, omni_swiglu_linear_fwd / omni_linear_fwd / omni_mlp_fwd launch one block per CU that walks its share
  * of the tiles -- faster alone, but it holds every CU until it ends, so a concurrent kernel waits.  This entry launches one
  * block per tile instead (omni_moe_fwd with a side stream uses it for a gate/up projection of at most two rounds of tiles).
@@ -192,7 +192,7 @@ OMNI_API int32_t omni_swiglu_linear_fwd_shared(const void* x, const void* gate_w
 /* omni_swiglu_linear_fwd that also keeps the two projections a backward pass needs (the reference materialises them:
  * interface.py:23-27 calls torch.matmul twice before the SwiGLU function saves gate and up, omni_mlp.py:359-371):
  *   gate_out, up_out [T,I]: x Wg^T and x Wu^T rounded to the storage dtype; h [T,I] their SwiGLU product.
- * bf16 / f16 only, intermediate_size % 8 == 0, hidden_size % 64 == 0, 16-byte aligned outputs; anything else
+ * bf16 / f16 only, intermediate_size and hidden_size multiples of 8, 16-byte aligned pointers; anything else
  * returns OMNI_ERR_UNSUPPORTED (use omni_linear_fwd twice and omni_swiglu_fwd). */
 OMNI_API int32_t omni_swiglu_linear_save_fwd(const void* x, const void* gate_weight, const void* up_weight, void* h,
                                              void* gate_out, void* up_out, int64_t num_tokens, int32_t hidden_size,
@@ -270,6 +270,28 @@ OMNI_API int32_t omni_swiglu_fwd(const void* gate, const void* up, void* out, in
 OMNI_API int32_t omni_swiglu_bwd(const void* dout, const void* gate, const void* up, void* dgate, void* dup,
                                  int64_t num_elements, int32_t dtype, void* stream);
 
+
+/* omni_router_norm_bwd with dz laid out for omni_mlp_bwd: dz [T][2][rp], rp = num_expert_sqrt rounded up to 8 (rows of whole 16-byte pieces), the
+ * columns beyond num_expert_sqrt zero. */
+OMNI_API int32_t omni_router_norm_bwd_padded(const void* dgates, const void* gates, const int32_t* indices, const void* z,
+                                             const float* stats, void* dz, int64_t num_tokens, int32_t num_expert_sqrt,
+                                             int32_t num_experts_per_token, int32_t dtype, int32_t training, void* workspace,
+                                             void* stream);
+
+/* Backward of the shared MLP (omni_mlp_fwd), with the router projection's share of the same products: what autograd does in the reference for
+ * the matmuls of interface.py:23-29 and omni_moe.py:70-71 and the SwiGLU function between them (omni_mlp.py:306-356).
+ *   dy, x [T,H]; gate_weight, up_weight [I,H]; down_weight [H,I]; gate, up, h [T,I] as omni_swiglu_linear_save_fwd left them
+ *   dz : NULL, or [T][2][rp] from omni_router_norm_bwd_padded, with router_weight_x/y [r,H] (num_expert_sqrt = r; 0 without dz)
+ *   dx_addend : NULL, or [T,H] added to d(x) after its rounding (the expert op's d(x)), and the sum rounded again
+ *   dx [T,H], dgate_weight, dup_weight [I,H], ddown_weight [H,I], drouter_weight_x/y [r,H]: outputs, fully overwritten; NULL where not wanted
+ * fp32 sums on the matrix cores, one rounding per output.  bf16 / f16; H and I multiples of 8, at least one token; fp32, and operands of 2 GiB and
+ * more, return OMNI_ERR_UNSUPPORTED with nothing enqueued. */
+OMNI_API size_t omni_mlp_bwd_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t num_expert_sqrt, int32_t dtype);
+OMNI_API int32_t omni_mlp_bwd(const void* dy, const void* x, const void* gate_weight, const void* up_weight, const void* down_weight, const void* gate,
+                              const void* up, const void* h, const void* dz, const void* router_weight_x, const void* router_weight_y,
+                              const void* dx_addend, void* dx, void* dgate_weight, void* dup_weight, void* ddown_weight, void* drouter_weight_x,
+                              void* drouter_weight_y, int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t num_expert_sqrt,
+                              int32_t dtype, void* workspace, void* stream);
 
 /* Two bias-free linear layers sharing their input, written side by side:
  * y[T, 2*out] = [x weight_lo^T | x weight_hi^T].  One GEMM for the router's x and y

@@ -51,8 +51,8 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_bwd_kernel(
     const int my_ix = ok ? my_id / r : -1, my_iy = ok ? my_id - my_ix * r : -1;
     const int n = min(kWave, top_k - j0);
     for (int i = 0; i < n; ++i) {                   // slot order: the sum per column is deterministic
-      const int ix = __shfl(my_ix, i, kWave), iy = __shfl(my_iy, i, kWave);
-      const float ds = __shfl(my_ds, i, kWave);
+      const int ix = __builtin_amdgcn_readlane(my_ix, i), iy = __builtin_amdgcn_readlane(my_iy, i);
+      const float ds = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ds), i));
 #pragma unroll
       for (int c = 0; c < kCols; ++c) {
         ax[c] += (ix == c * kWave + lane) ? ds : 0.f;
@@ -82,16 +82,23 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_bwd_kernel(
 // buffer and per-block column sums, a one-wave-per-column kernel adds those, a third kernel
 // finishes d(z).  Values are rounded to the storage dtype where the reference's torch ops round
 // (d(score), d(l), d(n), d(z)); n and l are recomputed from z and the saved statistics.
-constexpr int kNormTokensPerWave = 8;
+//
+// A token's k slots are walked one after the other (a fixed order of the sums), each slot's id and gradient handed to all lanes by
+// v_readlane; what bounds the pass is that chain, so a wave takes few tokens while there are waves to spare (4096 tokens, 64 keys, k = 16:
+// eight tokens a wave and ds_bpermute exchanges 29 us).
+static inline int norm_tokens_per_wave(int64_t num_tokens) {
+  const int64_t t = num_tokens / (kBwdWavesPerBlock * 512);
+  return (int)(t < 1 ? 1 : t > 8 ? 8 : t);
+}
 
 template <int DT, int R>
 __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kernel(
     const void* __restrict__ dgates, const void* __restrict__ gates, const int32_t* __restrict__ ids,
     const void* __restrict__ z, const float* __restrict__ stats, void* __restrict__ dz, float* __restrict__ partials,
-    int num_tokens, int r, int top_k, int training) {
+    int num_tokens, int r, int top_k, int training, int tokens_per_wave, int dz_half) {
   __shared__ float red[kBwdWavesPerBlock][4][R * kWave];       // per wave: S1x, S2x, S1y, S2y by column
   const int lane = lane_id(), wave = threadIdx.x >> 6;
-  const int first = (blockIdx.x * kBwdWavesPerBlock + wave) * kNormTokensPerWave;
+  const int first = __builtin_amdgcn_readfirstlane((blockIdx.x * kBwdWavesPerBlock + wave) * tokens_per_wave);
   float s1[2][R], s2[2][R];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -106,7 +113,7 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kern
       mean[h][a] = key < r ? stats[(2 * h) * r + key] : 0.f;
       rstd[h][a] = key < r ? stats[(2 * h + 1) * r + key] : 0.f;
     }
-  for (int t = first; t < min(first + kNormTokensPerWave, num_tokens); ++t) {
+  for (int t = first; t < min(first + tokens_per_wave, num_tokens); ++t) {
     // d(l): scatter of the slot gradients, fp32 sums in slot order, one rounding
     float dl[2][R];
 #pragma unroll
@@ -122,8 +129,8 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kern
       const int my_ix = ok ? my_id / r : -1, my_iy = ok ? my_id - my_ix * r : -1;
       const int n = min(kWave, top_k - j0);
       for (int i = 0; i < n; ++i) {
-        const int ix = __shfl(my_ix, i, kWave), iy = __shfl(my_iy, i, kWave);
-        const float ds = __shfl(my_ds, i, kWave);
+        const int ix = __builtin_amdgcn_readlane(my_ix, i), iy = __builtin_amdgcn_readlane(my_iy, i);
+        const float ds = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ds), i));
 #pragma unroll
         for (int a = 0; a < R; ++a) {
           dl[0][a] += (ix == a * kWave + lane) ? ds : 0.f;
@@ -159,12 +166,15 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kern
 #pragma unroll
       for (int a = 0; a < R; ++a) {
         const int key = a * kWave + lane;
-        if (key >= r) continue;
+        if (key >= r) {
+          if (key < dz_half) Elem<DT>::store(dz, (int64_t(t) * 2 + h) * dz_half + key, 0.f);
+          continue;
+        }
         const float p = expf(Elem<DT>::round(l[a] - m - lse));
         const float dn = Elem<DT>::round(dl[h][a] - p * sum_dl);
         s1[h][a] += dn;
         s2[h][a] += dn * nhat[a];
-        Elem<DT>::store(dz, int64_t(t) * 2 * r + h * r + key, training ? dn : dn * rstd[h][a]);
+        Elem<DT>::store(dz, (int64_t(t) * 2 + h) * dz_half + key, training ? dn : dn * rstd[h][a]);
       }
     }
   }
@@ -201,17 +211,22 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_sums
   if (lane == 0) means[idx] = (float)(acc / (double)num_tokens);
 }
 
-// dz = rstd (dn - mean(dn) - nhat mean(dn nhat)), element-wise over [T, 2r]; dn is read from dz
+// dz = rstd (dn - mean(dn) - nhat mean(dn nhat)), element-wise over [T, 2r]; dn is read from dz.  A row of 2r values to a row of `per_block`
+// thread rows, so that no value needs a division.
 template <int DT>
 __global__ __launch_bounds__(256) void router_norm_bwd_finish_kernel(const void* __restrict__ z, const float* __restrict__ stats,
                                                                     const float* __restrict__ means, void* __restrict__ dz,
-                                                                    int64_t num_values, int r) {
-  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < num_values; i += gridDim.x * 256ll) {
-    const int c = (int)(i % (2 * r)), h = c >= r, key = c - h * r;
-    const float mu = stats[(2 * h) * r + key], rs = stats[(2 * h + 1) * r + key];
-    const float nhat = (Elem<DT>::load(z, i) - mu) * rs;
-    const float dn = Elem<DT>::load(dz, i);
-    Elem<DT>::store(dz, i, rs * (dn - means[(2 * h) * r + key] - nhat * means[(2 * h + 1) * r + key]));
+                                                                    int num_tokens, int r, int width, int dz_half) {
+  const int per_block = 256 / width, row = threadIdx.x / width, c0 = threadIdx.x % width;     // width: a power of two up to 256
+  for (int c = c0; c < 2 * r; c += width) {
+    const int h = c >= r, key = c - h * r;
+    const float mu = stats[(2 * h) * r + key], rs = stats[(2 * h + 1) * r + key], m1 = means[(2 * h) * r + key], m2 = means[(2 * h + 1) * r + key];
+    for (int t = blockIdx.x * per_block + row; t < num_tokens; t += gridDim.x * per_block) {
+      const float nhat = (Elem<DT>::load(z, (int64_t)t * 2 * r + c) - mu) * rs;
+      const int64_t at = ((int64_t)t * 2 + h) * dz_half + key;
+      const float dn = Elem<DT>::load(dz, at);
+      Elem<DT>::store(dz, at, rs * (dn - m1 - nhat * m2));
+    }
   }
 }
 
@@ -563,7 +578,7 @@ extern "C" OMNI_API int32_t omni_router_bwd(const void* dscores, const int32_t* 
 
 // workspace of omni_router_norm_bwd: per-block column sums [blocks][4][r] f32 | means [4][r] f32
 static inline int norm_bwd_blocks(int64_t num_tokens) {
-  const int64_t per_block = (int64_t)omni::kBwdWavesPerBlock * omni::kNormTokensPerWave;
+  const int64_t per_block = (int64_t)omni::kBwdWavesPerBlock * omni::norm_tokens_per_wave(num_tokens);
   return (int)((num_tokens + per_block - 1) / per_block);
 }
 
@@ -573,10 +588,9 @@ extern "C" OMNI_API size_t omni_router_norm_bwd_workspace_bytes(int64_t num_toke
   return up256((size_t)norm_bwd_blocks(num_tokens) * 4 * num_expert_sqrt * 4) + up256((size_t)4 * num_expert_sqrt * 4);
 }
 
-extern "C" OMNI_API int32_t omni_router_norm_bwd(const void* dgates, const void* gates, const int32_t* indices, const void* z,
-                                                 const float* stats, void* dz, int64_t num_tokens, int32_t num_expert_sqrt,
-                                                 int32_t num_experts_per_token, int32_t dtype, int32_t training, void* workspace,
-                                                 void* stream) {
+static int32_t router_norm_bwd(const void* dgates, const void* gates, const int32_t* indices, const void* z, const float* stats, void* dz,
+                               int64_t num_tokens, int32_t num_expert_sqrt, int32_t num_experts_per_token, int32_t dtype, int32_t training,
+                               void* workspace, void* stream, int dz_half) {
   using namespace omni;
   const int r = num_expert_sqrt, k = num_experts_per_token;
   if (num_tokens < 0 || num_tokens > INT32_MAX / 4096 || r <= 0 || k < 0) return OMNI_ERR_SHAPE;
@@ -588,24 +602,26 @@ extern "C" OMNI_API int32_t omni_router_norm_bwd(const void* dgates, const void*
   if (training && !workspace) return OMNI_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   const int T = (int)num_tokens, blocks = norm_bwd_blocks(num_tokens);
+  const int per_wave = norm_tokens_per_wave(num_tokens);
+  int width = 32;
+  while (width < 256 && width < 2 * r) width *= 2;
   float* partials = (float*)workspace;
   float* means = training ? (float*)((char*)workspace + up256((size_t)blocks * 4 * r * 4)) : nullptr;
   dim3 block(kBwdWavesPerBlock * kWave);
 #define OMNI_NORM_CASE(DT)                                                                                                    \
   do {                                                                                                                        \
     if (r <= 64) hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 1>), dim3(blocks), block, 0, s, dgates, gates, indices, z,     \
-                                    stats, dz, partials, T, r, k, training);                                                   \
+                                    stats, dz, partials, T, r, k, training, per_wave, dz_half);                                                   \
     else if (r <= 256) hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 4>), dim3(blocks), block, 0, s, dgates, gates, indices,  \
-                                          z, stats, dz, partials, T, r, k, training);                                          \
+                                          z, stats, dz, partials, T, r, k, training, per_wave, dz_half);                                          \
     else hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 16>), dim3(blocks), block, 0, s, dgates, gates, indices, z, stats, dz, \
-                            partials, T, r, k, training);                                                                      \
+                            partials, T, r, k, training, per_wave, dz_half);                                                                      \
     if (training) {                                                                                                           \
       hipLaunchKernelGGL(router_norm_bwd_sums_kernel, dim3((4 * r + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock), block, 0, s,  \
                          partials, means, blocks, r, T);                                                                       \
-      const int64_t values = (int64_t)T * 2 * r;                                                                              \
-      const int64_t want = (values + 255) / 256;                                                                              \
-      hipLaunchKernelGGL(router_norm_bwd_finish_kernel<DT>, dim3((unsigned)(want < 4096 ? want : 4096)), dim3(256), 0, s, z,   \
-                         stats, means, dz, values, r);                                                                         \
+      const int want = (T + 256 / width - 1) / (256 / width);                                                                  \
+      hipLaunchKernelGGL(router_norm_bwd_finish_kernel<DT>, dim3((unsigned)(want < 1024 ? want : 1024)), dim3(256), 0, s, z,   \
+                         stats, means, dz, T, r, width, dz_half);                                                              \
     }                                                                                                                         \
   } while (0)
   if (dtype == OMNI_BF16) OMNI_NORM_CASE(kBF16);
@@ -613,6 +629,21 @@ extern "C" OMNI_API int32_t omni_router_norm_bwd(const void* dgates, const void*
   else OMNI_NORM_CASE(kF32);
 #undef OMNI_NORM_CASE
   return to_code(hipGetLastError());
+}
+
+extern "C" OMNI_API int32_t omni_router_norm_bwd(const void* dgates, const void* gates, const int32_t* indices, const void* z,
+                                                 const float* stats, void* dz, int64_t num_tokens, int32_t num_expert_sqrt,
+                                                 int32_t num_experts_per_token, int32_t dtype, int32_t training, void* workspace,
+                                                 void* stream) {
+  return router_norm_bwd(dgates, gates, indices, z, stats, dz, num_tokens, num_expert_sqrt, num_experts_per_token, dtype, training, workspace, stream, num_expert_sqrt);
+}
+
+extern "C" OMNI_API int32_t omni_router_norm_bwd_padded(const void* dgates, const void* gates, const int32_t* indices, const void* z,
+                                                        const float* stats, void* dz, int64_t num_tokens, int32_t num_expert_sqrt,
+                                                        int32_t num_experts_per_token, int32_t dtype, int32_t training, void* workspace,
+                                                        void* stream) {
+  return router_norm_bwd(dgates, gates, indices, z, stats, dz, num_tokens, num_expert_sqrt, num_experts_per_token, dtype, training, workspace, stream,
+                         (num_expert_sqrt + 7) / 8 * 8);
 }
 
 // workspace: ds [P] f32 | coef [P] f32 | sorted pair ids [P] i32 | sorted token ids [P] i32 | offsets [N+1] i32 |

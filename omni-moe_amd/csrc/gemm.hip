@@ -5,17 +5,18 @@
 //     - the SwiGLU product is formed in the GEMM epilogue, so gate and up never reach HBM
 //   * down projection     y  = h Wd^T (+ expert output)        (interface.py:23-29, omni_moe.py:102)
 //
+// The 16-bit projections go to the tile GEMM (gemm_tiles.hip) whenever their columns come in eights.  Here are
+//   * `gemm_nt_kernel`: single precision, and 16-bit products of odd sizes (global -> registers -> one of two LDS stages with padded rows);
+//   * `gemm_nt_dma_kernel` and `gemm_ksplit_kernel`: the 16-bit router projection, whose epilogue takes column statistics or whose weights are
+//     two matrices, and the gated product of the dense expert algorithm (global -> LDS directly, ring of stages, swizzled rows).
 // Structure: a block of 4 waves (2 x 2) owns a (2*TM*32) x (2*TN*32) tile; each wave owns
 // TM x TN MFMA tiles of 32x32 and K advances 64 at a time.  The largest tile, 256 x 256, runs
-// on 8 waves (2 x 4, two per SIMD) of 128 x 64 instead.  16-bit operands with K % 64 == 0
-// take `gemm_nt_dma_kernel` (global -> LDS directly, ring of stages, swizzled rows); anything
-// else takes `gemm_nt_kernel` (global -> registers -> one of two LDS stages with padded rows).
-// Two more forms of the direct-to-LDS kernel: `gemm_stream_kernel` (the 256 x 256 tile, one block per CU
-// walking its output tiles, on 16x16x32 MFMAs) and `gemm_ksplit_kernel` (fewer 64 x 64 tiles than CUs: a
-// block's waves share out the K tiles).
+// on 8 waves (2 x 4, two per SIMD) of 128 x 64 instead.  `gemm_ksplit_kernel` is for fewer 64 x 64 tiles than CUs: a
+// block's waves share out the K tiles.
 // The weight fragment is the MFMA's first operand, so an accumulator lane holds 4 consecutive
 // output columns of one row; two lanes pair up to store 8 columns (16 bytes) each.
 #include "common.h"
+#include "gemm_tiles.h"
 #include "omni_moe_hip.h"
 
 #include <type_traits>
@@ -74,9 +75,6 @@ struct GemmArgs {           // all element offsets below are scaled by the eleme
   float* part_mean;       // kEpiStats only: [ceil(M/32)][N] mean of each column over
   float* part_m2;         //   rows 32s..32s+31 of the ROUNDED result, and the sum of squared deviations
   const float* gate;      // kEpiGate only: [M, N] fp32 factors; C is then [M, 2N]: round(v) in columns 0..N-1, round(v - round(v)) in N..2N-1
-  uint8_t* save_gate;     // kEpiSwiglu only, or NULL: [M, N] the rounded gate and up projections, kept for a backward pass
-  uint8_t* save_up;       //   (16-byte stores only: N % 8 == 0)
-  int exclusive;          // nothing is meant to run beside this launch: the 256 x 256 tile's grid may be one block per CU that holds it to the end
 };
 
 // Which output tile a block owns.  Blocks go round-robin over the 8 XCDs; each XCD gets
@@ -261,28 +259,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, f32x16_t (&acc)
             const auto s1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
             const int n = nt + pr * 16 + (lane >> 5) * 8;
             if (n < g.N) *(u32x4_t*)(g.c + ((int64_t)m * g.N + n) * 2) = u32x4_t{s0[0], s1[0], s0[1], s1[1]};
-            if constexpr (EPI == kEpiSwiglu) {
-              if (g.save_gate) {                             // the two rounded projections leave the same way
-                uint32_t a[2][2], b[2][2];
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                  const int q4 = 2 * pr + e;
-#pragma unroll
-                  for (int h2 = 0; h2 < 2; ++h2) {
-                    a[e][h2] = pack2<DT>(acc[i][j][q4 * 4 + 2 * h2], acc[i][j][q4 * 4 + 2 * h2 + 1]);
-                    b[e][h2] = pack2<DT>(acc[i][j + TNO][q4 * 4 + 2 * h2], acc[i][j + TNO][q4 * 4 + 2 * h2 + 1]);
-                  }
-                }
-                const auto a0 = __builtin_amdgcn_permlane32_swap(a[0][0], a[1][0], false, false);
-                const auto a1 = __builtin_amdgcn_permlane32_swap(a[0][1], a[1][1], false, false);
-                const auto b0 = __builtin_amdgcn_permlane32_swap(b[0][0], b[1][0], false, false);
-                const auto b1 = __builtin_amdgcn_permlane32_swap(b[0][1], b[1][1], false, false);
-                if (n < g.N) {
-                  *(u32x4_t*)(g.save_gate + ((int64_t)m * g.N + n) * 2) = u32x4_t{a0[0], a1[0], a0[1], a1[1]};
-                  *(u32x4_t*)(g.save_up + ((int64_t)m * g.N + n) * 2) = u32x4_t{b0[0], b1[0], b0[1], b1[1]};
-                }
-              }
-            }
           }
           continue;
         }
@@ -630,337 +606,6 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_nt_dma_kernel(const GemmArgs 
   gemm_epilogue<DT, TM, TN, EPI>(g, acc, m0, n0, wm, wn, lane);
 }
 
-// ---- the 256 x 256 tile as a stream over several output tiles ----------------------------------------
-// One block per CU walks its share of the output tiles (tile index blockIdx, blockIdx + gridDim, ...).  The K tiles of
-// consecutive output tiles form ONE stream through the two LDS stages: while a block multiplies the last K tiles of an
-// output tile, the first K tiles of its next one are already on their way, so only a block's first output tile waits for
-// memory before its first matrix instruction.  Ring loads are buffer loads (scalar base and tile offsets, one 32-bit
-// lane offset per operand).  The grid keeps every CU until the kernel ends, so a kernel on another stream finds no room
-// beside it: the callers use this form where nothing is meant to run concurrently.
-// Needs N a multiple of the tile's columns and K % 64 == 0; a ragged last row tile re-reads the matrix's last row and stores
-// nothing for it.  XCD patches need whole rounds of 256 tiles; other tile counts go in plain order.
-//
-// The wave's 128 x 64 tile is 8 x 4 MFMA tiles of 16 x 16 and K advances 32 per instruction.  Under sustained load the
-// board clocks by power, and on the same operand bits the 16 x 16 x 32 instruction sustains about 15 % more than
-// 32 x 32 x 16 (register-only probes, two waves per SIMD: 2.07 against 1.80 PFLOP/s; this kernel against the same
-// kernel on 32 x 32 x 16: 8192 x 8192 x 2048 207 against 222 us, 32768 x 2 x 8192 x 2048 with SwiGLU 1.66 against
-// 1.76 ms, 4096 x 2 x 4096 x 1024 level).  A lane of accumulator tile (i, j) holds row m = 16 i + lane%16 and the four
-// columns n = 16 j + 4 (lane/16) + 0..3.  The activation fragments are a single set that is refilled row by row (the
-// fragment of row tile i for the next K step is read as soon as row i's four instructions have issued); the weight
-// fragments alternate between two sets.
-__device__ __forceinline__ void tile_coords_of(const GemmArgs& g, int b, int& tile_m, int& tile_n) {
-  if (g.patch_m > 0) {
-    const int per_patch = g.patch_m * g.patch_n;
-    const int xcd = b & 7, idx = b >> 3;
-    const int patch = (idx / per_patch) * 8 + xcd, within = idx % per_patch;
-    const int patches_m = g.tiles_m / g.patch_m;
-    tile_m = (patch % patches_m) * g.patch_m + within % g.patch_m;
-    tile_n = (patch / patches_m) * g.patch_n + within / g.patch_m;
-  } else {
-    tile_m = b % g.tiles_m;
-    tile_n = b / g.tiles_m;
-  }
-}
-
-template <int DT>
-__device__ __forceinline__ f32x4_t mfma16(const u32x4_t a, const u32x4_t b, f32x4_t c) {
-  if constexpr (DT == kBF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-  else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-}
-
-// Epilogue of the streaming kernel (full column tiles, 16-byte stores; rows past M are not stored).  Lanes l and l ^ 16 hold columns 4g..4g+3 and 4g+4..4g+7 of
-// two neighbouring column tiles: one v_permlane16_swap per word leaves every lane with 8 consecutive columns of one
-// of the two tiles, 64 consecutive bytes of a row over the four lanes l, l + 16, l + 32, l + 48.  The store path wants
-// those four in CONSECUTIVE lanes: a store-only microbenchmark moves 14 bytes per cycle and CU when neighbouring lanes
-// write different rows (16 rows x 64 bytes or 8 rows x 128 bytes per instruction alike) and 26-27 when each quad of
-// lanes writes 64 bytes on end, in any order of its four pieces; and while a tile's stores pass through that path the
-// ring loads of the next tile queue behind them.  So every word goes through one ds_bpermute_b32 (lane d takes from
-// lane d / 4 + 16 (d % 4); no LDS memory involved), after which lane d holds 16 bytes of row d / 4.  The residual is
-// fetched in that layout as well, 16 bytes per lane, and added to the rounded product there: the same arithmetic.
-__device__ __forceinline__ u32x4_t to_row_quads(const uint32_t x0, const uint32_t x1, const uint32_t x2, const uint32_t x3, const int from) {
-  return u32x4_t{(uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)x0), (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)x1),
-                 (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)x2), (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)x3)};
-}
-template <int DT> __device__ __forceinline__ float half_lo(const uint32_t w) {
-  if constexpr (DT == kBF16) return bf16_lo(w); else return f16_bits_to_f32((uint16_t)(w & 0xffffu));
-}
-template <int DT> __device__ __forceinline__ float half_hi(const uint32_t w) {
-  if constexpr (DT == kBF16) return bf16_hi(w); else return f16_bits_to_f32((uint16_t)(w >> 16));
-}
-template <int DT, int EPI>
-__device__ __forceinline__ void stream_epilogue(const GemmArgs& g, f32x4_t (&acc)[8][4], const int m0, const int n0, const int wm,
-                                                  const int wn, const int lane) {
-  constexpr int TNO = (EPI == kEpiSwiglu) ? 2 : 4;
-  const int nb = n0 + wn * (TNO * 16);
-  // (not for the SwiGLU form, whose epilogue is bound by its arithmetic: there the exchange costs the layer step 0.4 %)
-  constexpr bool kQuads = EPI != kEpiSwiglu;
-  const int tr = kQuads ? lane >> 2 : lane & 15;       // where the lane's 16 bytes go: row of the 16,
-  const int tg = kQuads ? lane & 3 : lane >> 4;        // ... piece of the row's 64 bytes
-  const int from = (tr + 16 * tg) * 4;                 // ds_bpermute address of the lane that holds them before the exchange
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + wm * 128 + i * 16 + tr;
-    const bool stored = m < g.M;
-#pragma unroll
-    for (int j = 0; j < TNO; j += 2) {
-      uint32_t w[2][2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        float v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          if constexpr (EPI == kEpiSwiglu) {
-            // gate and up are materialised in the storage dtype, silu(gate)*up is formed in fp32 and rounded once (omni_mlp.py:53-61)
-            const float gt = Elem<DT>::round(acc[i][j + t][q]), up = Elem<DT>::round(acc[i][j + t + TNO][q]);
-            v[q] = silu_fast(gt) * up;
-          } else {
-            v[q] = acc[i][j + t][q];
-          }
-        }
-        w[t][0] = pack2<DT>(v[0], v[1]);
-        w[t][1] = pack2<DT>(v[2], v[3]);
-      }
-      // odd 16-lane rows of tile j's words change places with even rows of tile j+1's
-      const auto s0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
-      const auto s1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
-      u32x4_t out = kQuads ? to_row_quads(s0[0], s1[0], s0[1], s1[1], from) : u32x4_t{s0[0], s1[0], s0[1], s1[1]};
-      const int n = nb + (j + (tg & 1)) * 16 + (tg & 2) * 4;
-      const int64_t at = ((int64_t)m * g.N + n) * 2;
-      if constexpr (EPI == kEpiResidual) {
-        const int mr = stored ? m : g.M - 1;             // rows past the matrix are computed but never stored
-        const u32x4_t r = *(const u32x4_t*)(g.res + ((int64_t)mr * g.N + n) * 2);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t o = out[q], rq = r[q];
-          out[q] = pack2<DT>(half_lo<DT>(o) + half_lo<DT>(rq), half_hi<DT>(o) + half_hi<DT>(rq));
-        }
-      }
-      if (stored) *(u32x4_t*)(g.c + at) = out;
-      if constexpr (EPI == kEpiSwiglu) {
-        if (g.save_gate) {                               // the two rounded projections leave the same way (kept for a backward pass)
-          uint32_t a[2][2], b[2][2];
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int h2 = 0; h2 < 2; ++h2) {
-              a[t][h2] = pack2<DT>(acc[i][j + t][2 * h2], acc[i][j + t][2 * h2 + 1]);
-              b[t][h2] = pack2<DT>(acc[i][j + t + TNO][2 * h2], acc[i][j + t + TNO][2 * h2 + 1]);
-            }
-          const auto a0 = __builtin_amdgcn_permlane16_swap(a[0][0], a[1][0], false, false);
-          const auto a1 = __builtin_amdgcn_permlane16_swap(a[0][1], a[1][1], false, false);
-          const auto b0 = __builtin_amdgcn_permlane16_swap(b[0][0], b[1][0], false, false);
-          const auto b1 = __builtin_amdgcn_permlane16_swap(b[0][1], b[1][1], false, false);
-          const u32x4_t ga = {a0[0], a1[0], a0[1], a1[1]}, ub = {b0[0], b1[0], b0[1], b1[1]};
-          if (stored) {
-            *(u32x4_t*)(g.save_gate + at) = ga;
-            *(u32x4_t*)(g.save_up + at) = ub;
-          }
-        }
-      }
-    }
-  }
-}
-
-template <int DT, int EPI>
-__global__ __launch_bounds__(512, 1) void gemm_stream_kernel(const GemmArgs g) {
-  constexpr int TM = 8, TN = 4;                      // MFMA tiles of 16 x 16 per wave: 128 x 64
-  constexpr int BM = 256, BR = 256;
-  constexpr int BN = (EPI == kEpiSwiglu) ? 128 : 256;
-  constexpr int kRow = 128, kStage = (BM + BR) * kRow;
-  extern __shared__ __align__(16) uint8_t lds[];
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
-  const int num_kt = g.K / 64;
-  const int num_tiles = g.tiles_m * g.tiles_n;
-  const uint32_t row_bytes = (uint32_t)g.K * 2;
-
-  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)g.a, 0, 0x7fffffff, 0x00020000);
-  const uint8_t* bsel = (EPI == kEpiSwiglu && (wave >> 2)) ? g.b1 : g.b0;      // waves 0-3 fetch gate rows, 4-7 the up rows
-  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)bsel, 0, 0x7fffffff, 0x00020000);
-  // plain and residual forms: an optional second weight matrix supplies the upper half of the output columns (whole tiles of it)
-  const __amdgpu_buffer_rsrc_t rsrc_hi = __builtin_amdgcn_make_buffer_rsrc((void*)((EPI != kEpiSwiglu && g.b1) ? g.b1 : g.b0), 0, 0x7fffffff, 0x00020000);
-
-  // Load instruction p of a wave fills LDS rows (8p + wave)*8 + lane/8 of a tile; the lane fetches the logical chunk that
-  // belongs at its (swizzled) position, which depends on the wave's parity and the lane only.  For the SwiGLU form rows
-  // 64p .. 64p+31 of the weight tile are gate rows and 64p+32 .. 64p+63 the matching up rows of wave column p.
-  const int sw = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
-  uint32_t a_voff[4];                                  // per load instruction: its row of the tile, clamped to the matrix (set with the cursor)
-  const uint32_t b_voff = (uint32_t)((EPI == kEpiSwiglu ? (wave & 3) * 8 : wave * 8) + (lane >> 3)) * row_bytes + sw * 16;
-  constexpr int kBRowsPerInstr = (EPI == kEpiSwiglu) ? 32 : 64;     // weight rows between consecutive load instructions of a wave
-
-  uint32_t b_voff4[4];                                 // ... and per weight load instruction of the wave
-#pragma unroll
-  for (int q = 0; q < 4; ++q) b_voff4[q] = b_voff + (uint32_t)(q * kBRowsPerInstr) * row_bytes;
-
-  // Fetch cursor: the next K tile of the stream to request.  Everything a load instruction needs beyond its lane offsets is
-  // kept ready in scalar registers and moved on once per K tile (the K loop otherwise spends four scalar instructions
-  // on every matrix instruction, and a wave issues in order): the LDS address of the wave's first row in the cursor's
-  // stage, the byte offset of the K tile within the activation and the weight rows, the weight matrix's descriptor.
-  using LdsPtr = __attribute__((address_space(3))) void*;
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(LdsPtr)lds;
-  int f_tile = blockIdx.x, f_kt = 0;
-  uint32_t f_ldsw = lds_base + (uint32_t)wave * 1024;  // ... of the wave's first row in the cursor's stage
-  int f_flip = kStage;                                 // to the other stage and back
-  uint32_t f_sa = 0, f_sb = 0;
-  int half_pending = 0;                                // the cursor's K tile has its activation half requested, not yet its weights (an int: a bool carried round the loop becomes a lane mask)
-  __amdgpu_buffer_rsrc_t rsrc_w = rsrc_b;              // the second weight matrix for the upper half of the columns (plain and residual forms)
-  auto cursor_coords = [&]() {                         // at a tile's first K tile
-    int tm, tn;
-    tile_coords_of(g, f_tile, tm, tn);
-    f_sa = (uint32_t)(tm * BM) * row_bytes;
-    const bool hi = EPI != kEpiSwiglu && g.b1 != nullptr && tn * BN >= g.N / 2;
-    rsrc_w = hi ? rsrc_hi : rsrc_b;
-    f_sb = (uint32_t)(tn * BN - (hi ? g.N / 2 : 0)) * row_bytes;
-    const int last = g.M - 1 - tm * BM;                // last row of the matrix, counted from the tile's first: a ragged last tile re-reads it
-#pragma unroll
-    for (int q = 0; q < 4; ++q) a_voff[q] = (uint32_t)min(q * 64 + wave * 8 + (lane >> 3), last) * row_bytes + sw * 16;
-  };
-  cursor_coords();
-  auto issue_one = [&](int q) __attribute__((always_inline)) {       // q = 0..3: activation rows, 4..7: weight rows
-    if (q < 4)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (LdsPtr)(uintptr_t)(f_ldsw + q * 8192), 16, a_voff[q], f_sa, 0, 0);
-    else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (LdsPtr)(uintptr_t)(f_ldsw + BM * kRow + (q - 4) * 8192), 16, b_voff4[q - 4], f_sb, 0, 0);
-  };
-  auto cursor_advance = [&]() {                        // after a K tile's second half has been issued
-    f_ldsw += (uint32_t)f_flip;
-    f_flip = -f_flip;
-    if (++f_kt == num_kt) {
-      f_kt = 0;
-      f_tile += gridDim.x;
-      if (f_tile < num_tiles) cursor_coords();
-    } else {
-      f_sa += 128;
-      f_sb += 128;
-    }
-  };
-
-  // fragment reads: lane reads row lane%16 of a 16-row tile, logical chunk 4*kstep + lane/16 (8 K values of the step's 32).
-  // ra[1], rb[1]: the lane's activation / weight fragment row of K step 1 in the stage being multiplied; ra[0], rb[0]: of K step 0
-  // in the OTHER stage (the next K tile's) -- what the first and the second step of a K tile read for the step after them;
-  // the row tile comes as the instruction's immediate offset, and the four change stages once per K tile (c_flip).
-  const int r16 = lane & 15;
-  uint32_t ra[2], rb[2];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const uint32_t off = lds_base + (uint32_t)(r16 * kRow + ((4 * ks + (lane >> 4)) ^ (r16 >> 1)) * 16) + (ks == 0 ? (uint32_t)kStage : 0u);
-    ra[ks] = (uint32_t)((wm * 128) * kRow) + off;
-    rb[ks] = (uint32_t)(BM * kRow + (wn * 64) * kRow) + off;
-  }
-  int c_flip[2] = {-kStage, kStage};                   // next change of ra[ks], rb[ks]
-  using LdsFrag = const __attribute__((address_space(3))) u32x4_t*;
-  u32x4_t af[TM], bf[2][TN];
-  auto read_a = [&](int ks, int i) __attribute__((always_inline)) { af[i] = *(LdsFrag)(uintptr_t)(ra[ks] + i * 16 * kRow); };
-  auto read_b = [&](int ks, int j) __attribute__((always_inline)) { bf[ks][j] = *(LdsFrag)(uintptr_t)(rb[ks] + j * 16 * kRow); };
-
-  f32x4_t acc[TM][TN];
-  auto clear_acc = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[i][j][q] = 0.f;
-  };
-  clear_acc();
-
-  constexpr int kEpiStores = (EPI == kEpiSwiglu) ? 8 : 16;   // store instructions of a wave's epilogue (no memory instruction follows them)
-  // One K step of 32: TM*TN matrix instructions in row order, at most one memory instruction behind each (slot_op).
-  // In the K tile's second step, whose following step reads the other stage, the wave waits after row 0 for its fragment
-  // reads and ring loads and meets the block.
-  constexpr int kSyncRow = 0;
-  // what follows matrix instruction (i, j): 0 nothing, 10+n weight fragment n, 20+n activation fragment n of the following
-  // step, 30+n ring load n of the cursor's K tile (0-3 activation rows, in the second step; 4-7 weight rows, in the first)
-  auto slot_op = [](bool second, int i, int j) constexpr -> int {
-    if (j == 0 && i >= 1 && i <= 4) return 10 + (i - 1);
-    if (j == 1 && i >= 1 && i <= 4) return second ? 30 + (i - 1) : 34 + (i - 1);
-    if (second && j == 1 && i >= 5) return 40 + (i - 5);            // 40-43: the weight rows too, in a tile's last K tile
-    if (second && j == 2 && i == 7) return 43;
-    if (j == 2 && i == 1) return 20;
-    if (j == 3 && i >= 1) return 20 + i;
-    return 0;
-  };
-  // last: the output tile's last K tile; young: memory instructions of the wave issued after the loads this K tile's sync
-  // point waits for (the previous tile's stores, when the K tile is a tile's first)
-  auto kstep = [&](auto ks_tag, auto sync_tag, const int last, const int young) __attribute__((always_inline)) {
-    constexpr int ks = decltype(ks_tag)::value;
-    constexpr bool sync = decltype(sync_tag)::value;
-    constexpr int nks = ks ^ 1;
-    // (scalar registers by force: left alone the compiler keeps these loop-carried flags in vector registers and tests them there)
-    const bool fa = f_tile < num_tiles;
-    const bool hp = half_pending != 0;
-    const bool fl = fa && last;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        acc[i][j] = mfma16<DT>(bf[ks][j], af[i], acc[i][j]);
-        __builtin_amdgcn_sched_barrier(0);
-        const int op = slot_op(sync, i, j);
-        if (op >= 10 && op < 20) read_b(nks, op - 10);
-        if (op >= 20 && op < 30) read_a(nks, op - 20);
-        if (op >= 30 && op < 34) { if (fa) issue_one(op - 30); }
-        if (op >= 34 && op < 40) { if (hp) issue_one(op - 30); }
-        if (op >= 40) { if (fl) issue_one(op - 36); }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if constexpr (sync) {
-        if (i == kSyncRow) {
-          wait_lds_reads();                            // this wave holds every fragment of the K tile
-          // the next K tile has landed.  The counter runs in issue order, loads and stores alike: behind a tile's epilogue
-          // its stores are younger than every load of the next K tile (whose weight rows a tile's last K tile requests
-          // early for that reason) and may stay in flight for another K tile
-          if (young == kEpiStores) wait_vmcnt<kEpiStores>(); else wait_vmcnt<0>();
-          __builtin_amdgcn_s_barrier();                // ... for all waves; this K tile's stage is free
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    }
-  };
-  using I0 = std::integral_constant<int, 0>; using I1 = std::integral_constant<int, 1>;
-  auto k_tile = [&](const int last, const int young) __attribute__((always_inline)) {
-    kstep(I0{}, std::false_type{}, last, 0);           // the weights of the K tile whose activations were requested one step ago
-    if (half_pending) { cursor_advance(); half_pending = 0; }
-    const int fa = f_tile < num_tiles ? 1 : 0;
-    kstep(I1{}, std::true_type{}, last, young);        // the activations of the K tile two ahead go into the freed stage
-    if (last & fa) cursor_advance();                   // ... with its weights, when the epilogue comes next
-    half_pending = fa & (last ^ 1);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) { ra[ks] += (uint32_t)c_flip[ks]; rb[ks] += (uint32_t)c_flip[ks]; c_flip[ks] = -c_flip[ks]; }
-  };
-
-  // ---- prologue: the stream's first two K tiles
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) issue_one(q);
-    cursor_advance();
-  }
-  wait_vmcnt<8>();                                     // the first K tile has landed
-  __builtin_amdgcn_s_barrier();
-#pragma unroll
-  for (int i = 0; i < TM; ++i) af[i] = *(LdsFrag)(uintptr_t)(ra[0] - (uint32_t)kStage + i * 16 * kRow);     // K step 0 of stage 0
-#pragma unroll
-  for (int j = 0; j < TN; ++j) bf[0][j] = *(LdsFrag)(uintptr_t)(rb[0] - (uint32_t)kStage + j * 16 * kRow);
-
-  int young = 0;                                       // stores of the previous tile's epilogue, if their number is known
-  for (int tile = blockIdx.x; tile < num_tiles; tile += gridDim.x) {
-    // (not unrolled, which would include peeling the first K tile off as a second loop body: the compiler then gives the
-    // accumulators different registers in the two bodies and the kernel needs 250 VGPRs instead of 216, which leaves no
-    // room on a SIMD for a wave of the kernels that the layer runs beside this one)
-#pragma clang loop unroll(disable)
-    for (int kt = 0; kt < num_kt; ++kt) k_tile(kt == num_kt - 1 ? 1 : 0, kt == 0 ? young : 0);
-    int tm, tn;
-    tile_coords_of(g, tile, tm, tn);
-    stream_epilogue<DT, EPI>(g, acc, tm * BM, tn * BN, wm, wn, lane);
-    // every row of the wave inside the matrix: each store instruction of the epilogue has been issued
-    young = (g.M - tm * BM - wm * 128 >= 128 && !(EPI == kEpiSwiglu && g.save_gate)) ? kEpiStores : 0;
-    clear_acc();
-  }
-}
-
 // ---- few output tiles, long K: the K tiles of one 64 x 64 output tile dealt out over the block's four waves ----------
 // A product like the router projection at a few thousand tokens (4096 x 128 x 1024) has too few output tiles to fill the
 // GPU and its time is the latency of one block's K loop: with the ring kernel above, 16 rounds of wait - barrier - four
@@ -1089,10 +734,6 @@ struct DmaKernelLds {
   static inline LdsKernel entry{(const void*)gemm_nt_dma_kernel<DT, TM, TN, EPI, BK, NS, NW>, NS * (2 * TM * 32 + (NW / 2) * TN * 32) * BK * 2};
 };
 template <int DT, int EPI>
-struct StreamKernelLds {
-  static inline LdsKernel entry{(const void*)gemm_stream_kernel<DT, EPI>, 2 * 512 * 128};
-};
-template <int DT, int EPI>
 struct KsplitKernelLds {
   static inline LdsKernel entry{(const void*)gemm_ksplit_kernel<DT, EPI>, 4 * 2 * 2 * 64 * 128};
 };
@@ -1113,7 +754,6 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
   g.wide = (DT != kF32) && g.N % 8 == 0 && ((uintptr_t)g.c % 16 == 0);
   g.single = g.N % 4 != 0;
   if (EPI == kEpiGate && !(g.wide && (uintptr_t)g.gate % 16 == 0)) return hipErrorInvalidValue;   // the gate epilogue has the 16-byte form only
-  if (EPI == kEpiSwiglu && g.save_gate && !g.wide) return hipErrorInvalidValue;                  // so has the saving SwiGLU epilogue
   if (blocks % 256 == 0) {
     if (g.tiles_m % 4 == 0 && g.tiles_n % 8 == 0) { g.patch_m = 4; g.patch_n = 8; }
     else if (g.tiles_m % 8 == 0 && g.tiles_n % 4 == 0) { g.patch_m = 8; g.patch_n = 4; }
@@ -1122,25 +762,10 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
   constexpr int kDmaBK = 64;
   constexpr int kFit = (160 * 1024) / ((BM + BR) * kDmaBK * 2);
   constexpr int kDmaStages = kFit > 4 ? 4 : kFit;
-  if constexpr (DT != kF32) if (g.K % kDmaBK == 0) {
+  if constexpr (DT != kF32 && EPI != kEpiSwiglu) if (g.K % kDmaBK == 0) {
     constexpr int kDmaLds = kDmaStages * (BM + BR) * kDmaBK * 2;
     static_assert(kDmaLds <= 160 * 1024, "LDS ring exceeds 160 KiB");
-    if constexpr (TM == 4 && TN == 4 && (EPI == kEpiPlain || EPI == kEpiSwiglu || EPI == kEpiResidual)) {
-      // full column tiles, K tiles enough for the two-stage prologue (buffer loads: operands below 1 Gi elements, 16-byte
-      // aligned).  Nothing meant to run beside it: one block per CU streams through its tiles.  Otherwise the same kernel
-      // with one block per tile, so that CUs come free for the other stream's kernels as blocks retire (two-stream layer
-      // step at 4096 tokens, 1024 x 4096: 123.3 us against 127.2 us with the 32x32x16 kernel below in that place).
-      const bool covers = g.N % BN == 0 && g.K >= 2 * kDmaBK && blocks >= 256 && g.wide &&
-                          (EPI == kEpiSwiglu || !g.b1 || (g.N / 2) % BN == 0) && (int64_t)g.M * g.K < (1ll << 30) &&
-                          (int64_t)g.N * g.K < (1ll << 30) && (uintptr_t)g.a % 16 == 0 && (uintptr_t)g.b0 % 16 == 0 &&
-                          (!g.b1 || (uintptr_t)g.b1 % 16 == 0);
-      if (covers) {
-        if (hipError_t e = StreamKernelLds<DT, EPI>::entry.ensure(); e != hipSuccess) return e;
-        hipLaunchKernelGGL((gemm_stream_kernel<DT, EPI>), dim3(g.exclusive ? 256 : blocks), dim3(512), 2 * 512 * 128, s, g);
-        return hipGetLastError();
-      }
-    }
-    if constexpr (TM == 1 && TN == 1 && EPI != kEpiSwiglu && EPI != kEpiGate) {
+    if constexpr (TM == 1 && TN == 1 && EPI != kEpiGate) {
       // fewer 64 x 64 tiles than CUs and at least two K tiles per wave: the K tiles dealt out over the waves
       if (blocks <= 256 && g.K >= 512) {
         if (hipError_t e = KsplitKernelLds<DT, EPI>::entry.ensure(); e != hipSuccess) return e;
@@ -1178,21 +803,38 @@ static int check_gemm(int64_t M, int64_t N, int64_t K, int elem_bytes) {
 
 static int to_code(hipError_t e) { return e == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)e; }
 
-// C[M,N] = A[M,K] B[N,K]^T (+ res), picking the tile shape from the problem size.
+// The tile GEMM's terms: columns in eights, 16-byte aligned pointers.  *e is then what its launch returned.
+static bool tile_gemm(int dtype, int epilogue, const void* a, const void* b, const void* b2, const void* res, void* c, void* keep_gate, void* keep_up, int64_t M, int64_t N,
+                      int64_t K, void* ws, size_t ws_bytes, bool exclusive, hipStream_t s, hipError_t* e) {
+  if (dtype == OMNI_F32 || N % 8 != 0) return false;
+  for (const void* q : {a, b, b2, res, (const void*)c, (const void*)keep_gate, (const void*)keep_up})
+    if ((uintptr_t)q % 16) return false;
+  TileGroup g;
+  TileProduct& p = g.p[g.count++];
+  p.seg[p.segments++] = TileSegment{(const uint8_t*)a, (const uint8_t*)b, K * 2, K * 2, 0, (int)K};
+  p.M = (int)M; p.N = (int)N; p.ldc = N * 2; p.c = (uint8_t*)c; p.res = (const uint8_t*)res; p.b_up = (const uint8_t*)b2;
+  p.c2 = (uint8_t*)keep_gate; p.c3 = (uint8_t*)keep_up;
+  *e = launch_tile_group(dtype, kNT, epilogue, g, ws, ws_bytes, s, exclusive);
+  return *e != hipErrorInvalidValue;
+}
+
+// C[M,N] = A[M,K] B[N,K]^T (+ res), picking the tile shape from the problem size.  ws: room for a K split (or NULL)
 template <int DT>
 static int gemm_plain(const void* a, const void* b, const void* b_hi, const void* res, void* c, int64_t M, int64_t N, int64_t K, hipStream_t s,
-                      float* part_mean = nullptr, float* part_m2 = nullptr, bool exclusive = true) {
+                      float* part_mean = nullptr, float* part_m2 = nullptr, bool twin = true, bool exclusive = true, void* ws = nullptr, size_t ws_bytes = 0) {
   if (int e = check_gemm(M, N, K, ElemBytes<DT>::value)) return e;
   if (M == 0) return OMNI_OK;
+  hipError_t err;
+  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256), mid = ((M + 127) / 128) * ((N + 127) / 128);
+  // a second weight matrix starts at a multiple of 8 columns there; `twin`: the result is, bit for bit, what two matrices give
+  if (!part_mean && (N % 16 == 0 || !twin) &&
+      tile_gemm(DT, b_hi ? kTileTwo : res ? kTileResidual : kTilePlain, a, b, b_hi, res, c, nullptr, nullptr, M, N, K, ws, ws_bytes, exclusive, s, &err))
+    return to_code(err);
   GemmArgs g{(const uint8_t*)a, (const uint8_t*)b, (const uint8_t*)b_hi, (const uint8_t*)res, (uint8_t*)c, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr};
   g.part_mean = part_mean;
   g.part_m2 = part_m2;
-  g.exclusive = exclusive;
-  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256), mid = ((M + 127) / 128) * ((N + 127) / 128);
-  hipError_t err;
   if (res) {
-    if (big >= 200) err = launch_gemm<DT, 4, 4, kEpiResidual>(g, s);
-    else if (mid >= 200) err = launch_gemm<DT, 2, 2, kEpiResidual>(g, s);
+    if (mid >= 200) err = launch_gemm<DT, 2, 2, kEpiResidual>(g, s);
     else err = launch_gemm<DT, 1, 1, kEpiResidual>(g, s);
   } else if (part_mean) {
     if (big >= 200) err = launch_gemm<DT, 4, 4, kEpiStats>(g, s);
@@ -1208,20 +850,14 @@ static int gemm_plain(const void* a, const void* b, const void* b_hi, const void
 
 template <int DT>
 static int gemm_swiglu(const void* x, const void* wg, const void* wu, void* h, int64_t M, int64_t I, int64_t K, hipStream_t s,
-                       void* save_gate = nullptr, void* save_up = nullptr, bool exclusive = true) {
+                       void* save_gate = nullptr, void* save_up = nullptr, bool exclusive = true, void* ws = nullptr, size_t ws_bytes = 0) {
   if (int e = check_gemm(M, I, K, ElemBytes<DT>::value)) return e;
   if (M == 0) return OMNI_OK;
-  GemmArgs g{(const uint8_t*)x, (const uint8_t*)wg, (const uint8_t*)wu, nullptr, (uint8_t*)h, (int)M, (int)I, (int)K, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr,
-             (uint8_t*)save_gate, (uint8_t*)save_up};
-  g.exclusive = exclusive;
-  if (save_gate) {   // the saving epilogue has the 16-byte form only, in the direct-to-LDS kernel
-    if (DT == kF32 || I % 8 != 0 || K % 64 != 0 || (uintptr_t)h % 16 || (uintptr_t)save_gate % 16 || (uintptr_t)save_up % 16) return OMNI_ERR_UNSUPPORTED;
-  }
-  const int64_t big = ((M + 255) / 256) * ((I + 127) / 128);
   hipError_t err;
-  if (big >= 200) err = launch_gemm<DT, 4, 4, kEpiSwiglu>(g, s);
-  else err = launch_gemm<DT, 2, 2, kEpiSwiglu>(g, s);
-  return to_code(err);
+  if (tile_gemm(DT, kTileSwiglu, x, wg, wu, nullptr, h, save_gate, save_up, M, I, K, ws, ws_bytes, exclusive, s, &err)) return to_code(err);
+  if (save_gate) return OMNI_ERR_UNSUPPORTED;
+  GemmArgs g{(const uint8_t*)x, (const uint8_t*)wg, (const uint8_t*)wu, nullptr, (uint8_t*)h, (int)M, (int)I, (int)K, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr};
+  return to_code(launch_gemm<DT, 2, 2, kEpiSwiglu>(g, s));
 }
 
 }  // namespace omni
@@ -1258,11 +894,50 @@ int omni_gemm_router_projection(const void* x, const void* wx, const void* wy, v
   return OMNI_ERR_DTYPE;
 }
 
+namespace omni {
+// partial sums of whichever of the two projections is split along K (they are not alive together)
+static size_t mlp_sums_bytes(int64_t T, int64_t H, int64_t I, int dtype) {
+  if (dtype == OMNI_F32 || I % 8 || H % 8) return 0;
+  const size_t a = tile_workspace_bytes(kTileSwiglu, T, I, H), b = tile_workspace_bytes(kTileResidual, T, H, I);
+  return a > b ? a : b;
+}
+static size_t mlp_h_bytes(int64_t T, int64_t I, int dtype) { return ((size_t)T * (size_t)I * (dtype == OMNI_F32 ? 4 : 2) + 255) / 256 * 256; }
+
+// The two projections of omni_mlp_fwd, each told whether it has the GPU to itself (the whole-layer call on two streams says no, which keeps
+// them off the form that holds every CU to the end).  `workspace`: omni_mlp_workspace_bytes(), h first.
+template <int DT>
+static int mlp_gate_up(const void* x, const void* wg, const void* wu, int64_t T, int64_t H, int64_t I, void* workspace, hipStream_t s, bool exclusive) {
+  return gemm_swiglu<DT>(x, wg, wu, workspace, T, I, H, s, nullptr, nullptr, exclusive, (char*)workspace + mlp_h_bytes(T, I, DT), mlp_sums_bytes(T, H, I, DT));
+}
+template <int DT>
+static int mlp_down(const void* wd, const void* residual, void* y, int64_t T, int64_t H, int64_t I, void* workspace, hipStream_t s, bool exclusive) {
+  return gemm_plain<DT>(workspace, wd, nullptr, residual, y, T, H, I, s, nullptr, nullptr, false, exclusive, (char*)workspace + mlp_h_bytes(T, I, DT), mlp_sums_bytes(T, H, I, DT));
+}
+int mlp_gate_up_impl(const void* x, const void* wg, const void* wu, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive) {
+  if (!x || !wg || !wu) return OMNI_ERR_NULL;
+  hipStream_t s = (hipStream_t)stream;
+  switch (dtype) {
+    case OMNI_BF16: return mlp_gate_up<kBF16>(x, wg, wu, T, H, I, workspace, s, exclusive);
+    case OMNI_F16: return mlp_gate_up<kF16>(x, wg, wu, T, H, I, workspace, s, exclusive);
+    case OMNI_F32: return mlp_gate_up<kF32>(x, wg, wu, T, H, I, workspace, s, exclusive);
+    default: return OMNI_ERR_DTYPE;
+  }
+}
+int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive) {
+  if (!wd || !y) return OMNI_ERR_NULL;
+  hipStream_t s = (hipStream_t)stream;
+  switch (dtype) {
+    case OMNI_BF16: return mlp_down<kBF16>(wd, residual, y, T, H, I, workspace, s, exclusive);
+    case OMNI_F16: return mlp_down<kF16>(wd, residual, y, T, H, I, workspace, s, exclusive);
+    case OMNI_F32: return mlp_down<kF32>(wd, residual, y, T, H, I, workspace, s, exclusive);
+    default: return OMNI_ERR_DTYPE;
+  }
+}
+}  // namespace omni
+
 extern "C" OMNI_API size_t omni_mlp_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t dtype) {
-  (void)hidden_size;
   if (num_tokens < 0 || intermediate_size < 0) return 0;
-  const size_t es = dtype == OMNI_F32 ? 4 : 2;
-  return (size_t)num_tokens * (size_t)intermediate_size * es;      // h = silu(gate)*up
+  return omni::mlp_h_bytes(num_tokens, intermediate_size, dtype) + omni::mlp_sums_bytes(num_tokens, hidden_size, intermediate_size, dtype);     // h = silu(gate)*up | sums
 }
 
 extern "C" OMNI_API int32_t omni_mlp_fwd(const void* x, const void* gate_weight, const void* up_weight, const void* down_weight,
@@ -1273,32 +948,19 @@ extern "C" OMNI_API int32_t omni_mlp_fwd(const void* x, const void* gate_weight,
   if (num_tokens == 0) return OMNI_OK;
   if (!x || !gate_weight || !up_weight || !down_weight || !y) return OMNI_ERR_NULL;
   if (!workspace) return OMNI_ERR_WORKSPACE;
-  hipStream_t s = (hipStream_t)stream;
   int e;
   if (dtype != OMNI_BF16 && dtype != OMNI_F16 && dtype != OMNI_F32) return OMNI_ERR_DTYPE;
   // both projections are checked before the first one is enqueued: hidden and intermediate size are each the K of one
   const int es = dtype == OMNI_F32 ? 4 : 2;
   if ((e = check_gemm(num_tokens, intermediate_size, hidden_size, es)) || (e = check_gemm(num_tokens, hidden_size, intermediate_size, es)))
     return e;
-  switch (dtype) {
-    case OMNI_BF16:
-      if ((e = gemm_swiglu<kBF16>(x, gate_weight, up_weight, workspace, num_tokens, intermediate_size, hidden_size, s))) return e;
-      return gemm_plain<kBF16>(workspace, down_weight, nullptr, residual, y, num_tokens, hidden_size, intermediate_size, s);
-    case OMNI_F16:
-      if ((e = gemm_swiglu<kF16>(x, gate_weight, up_weight, workspace, num_tokens, intermediate_size, hidden_size, s))) return e;
-      return gemm_plain<kF16>(workspace, down_weight, nullptr, residual, y, num_tokens, hidden_size, intermediate_size, s);
-    case OMNI_F32:
-      if ((e = gemm_swiglu<kF32>(x, gate_weight, up_weight, workspace, num_tokens, intermediate_size, hidden_size, s))) return e;
-      return gemm_plain<kF32>(workspace, down_weight, nullptr, residual, y, num_tokens, hidden_size, intermediate_size, s);
-    default: return OMNI_ERR_DTYPE;
-  }
+  if ((e = mlp_gate_up_impl(x, gate_weight, up_weight, num_tokens, hidden_size, intermediate_size, dtype, workspace, stream, true))) return e;
+  return mlp_down_impl(down_weight, residual, y, num_tokens, hidden_size, intermediate_size, dtype, workspace, stream, true);
 }
 
-// The two projection calls with the caller's word on whether anything runs beside them (the whole-layer call on two
-// streams says no to `exclusive`, which keeps the GEMMs off the streaming form that would hold every CU).
 namespace omni {
-int swiglu_linear_fwd_impl(const void* x, const void* gate_weight, const void* up_weight, void* h, int64_t num_tokens,
-                           int32_t hidden_size, int32_t intermediate_size, int32_t dtype, void* stream, bool exclusive) {
+static int swiglu_linear(const void* x, const void* gate_weight, const void* up_weight, void* h, int64_t num_tokens, int32_t hidden_size,
+                         int32_t intermediate_size, int32_t dtype, void* stream, bool exclusive) {
   if (num_tokens == 0) return OMNI_OK;
   if (!x || !gate_weight || !up_weight || !h) return OMNI_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
@@ -1309,30 +971,18 @@ int swiglu_linear_fwd_impl(const void* x, const void* gate_weight, const void* u
     default: return OMNI_ERR_DTYPE;
   }
 }
-int linear_fwd_impl(const void* x, const void* weight, const void* residual, void* y, int64_t num_tokens, int32_t in_features,
-                    int32_t out_features, int32_t dtype, void* stream, bool exclusive) {
-  if (num_tokens == 0) return OMNI_OK;
-  if (!x || !weight || !y) return OMNI_ERR_NULL;
-  hipStream_t s = (hipStream_t)stream;
-  switch (dtype) {
-    case OMNI_BF16: return gemm_plain<kBF16>(x, weight, nullptr, residual, y, num_tokens, out_features, in_features, s, nullptr, nullptr, exclusive);
-    case OMNI_F16: return gemm_plain<kF16>(x, weight, nullptr, residual, y, num_tokens, out_features, in_features, s, nullptr, nullptr, exclusive);
-    case OMNI_F32: return gemm_plain<kF32>(x, weight, nullptr, residual, y, num_tokens, out_features, in_features, s, nullptr, nullptr, exclusive);
-    default: return OMNI_ERR_DTYPE;
-  }
-}
 }  // namespace omni
 
 extern "C" OMNI_API int32_t omni_swiglu_linear_fwd(const void* x, const void* gate_weight, const void* up_weight, void* h,
                                                    int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size,
                                                    int32_t dtype, void* stream) {
-  return omni::swiglu_linear_fwd_impl(x, gate_weight, up_weight, h, num_tokens, hidden_size, intermediate_size, dtype, stream, true);
+  return omni::swiglu_linear(x, gate_weight, up_weight, h, num_tokens, hidden_size, intermediate_size, dtype, stream, true);
 }
 
 extern "C" OMNI_API int32_t omni_swiglu_linear_fwd_shared(const void* x, const void* gate_weight, const void* up_weight, void* h,
                                                           int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size,
                                                           int32_t dtype, void* stream) {
-  return omni::swiglu_linear_fwd_impl(x, gate_weight, up_weight, h, num_tokens, hidden_size, intermediate_size, dtype, stream, false);
+  return omni::swiglu_linear(x, gate_weight, up_weight, h, num_tokens, hidden_size, intermediate_size, dtype, stream, false);
 }
 
 extern "C" OMNI_API int32_t omni_swiglu_linear_save_fwd(const void* x, const void* gate_weight, const void* up_weight, void* h,
@@ -1352,7 +1002,16 @@ extern "C" OMNI_API int32_t omni_swiglu_linear_save_fwd(const void* x, const voi
 
 extern "C" OMNI_API int32_t omni_linear_fwd(const void* x, const void* weight, const void* residual, void* y, int64_t num_tokens,
                                             int32_t in_features, int32_t out_features, int32_t dtype, void* stream) {
-  return omni::linear_fwd_impl(x, weight, residual, y, num_tokens, in_features, out_features, dtype, stream, true);
+  using namespace omni;
+  if (num_tokens == 0) return OMNI_OK;
+  if (!x || !weight || !y) return OMNI_ERR_NULL;
+  hipStream_t s = (hipStream_t)stream;
+  switch (dtype) {
+    case OMNI_BF16: return gemm_plain<kBF16>(x, weight, nullptr, residual, y, num_tokens, out_features, in_features, s);
+    case OMNI_F16: return gemm_plain<kF16>(x, weight, nullptr, residual, y, num_tokens, out_features, in_features, s);
+    case OMNI_F32: return gemm_plain<kF32>(x, weight, nullptr, residual, y, num_tokens, out_features, in_features, s);
+    default: return OMNI_ERR_DTYPE;
+  }
 }
 
 extern "C" OMNI_API int32_t omni_linear2_fwd(const void* x, const void* weight_lo, const void* weight_hi, void* y,
@@ -1408,6 +1067,12 @@ extern "C" OMNI_API int32_t omni_add_inplace(void* y, const void* addend, int64_
 }
 
 namespace omni {
+template <int DT>
+__device__ __forceinline__ f32x4_t mfma16(const u32x4_t a, const u32x4_t b, f32x4_t c) {
+  if constexpr (DT == kBF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+
 // Matrix-core rate with nothing else going on: every wave keeps 16 accumulator tiles and issues
 // MFMAs on operands it read once (8 KiB of caller data, so that the operand bits are realistic:
 // the sustained clock under the board's power limit depends on how many bits toggle).

@@ -13,13 +13,13 @@ static inline size_t elem_bytes(int dtype) { return dtype == OMNI_F32 ? 4 : 2; }
 int expert_algo_check(int algo, int64_t num_tokens, int hidden_size, int64_t num_experts, int top_k, int dtype);
 // defined beside the select kernels: whether they take num_expert_sqrt keys per half with top_k and this dtype
 bool select_covers(int r, int k, int dtype);
-// defined beside the GEMM kernels: omni_linear_fwd with the caller's word on whether the launch has the GPU to itself
-// (then a GEMM of whole 256-tile rounds may take the form that holds every CU until it ends)
-int linear_fwd_impl(const void* x, const void* weight, const void* residual, void* y, int64_t num_tokens, int32_t in_features,
-                    int32_t out_features, int32_t dtype, void* stream, bool exclusive);
+// defined beside the GEMM kernels: the two projections of omni_mlp_fwd with the caller's word on whether the launch has the GPU to itself
+// (then a GEMM of more tiles than CUs may take the form that holds every CU until it ends); h lies at the workspace's start
+int mlp_gate_up_impl(const void* x, const void* wg, const void* wu, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive);
+int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive);
 }  // namespace omni
 
-// workspace: router workspace | gates [T,k] | ids [T,k] | expert output [T,H] | expert workspace | SwiGLU activations [T,I]
+// workspace: router workspace | gates [T,k] | ids [T,k] | expert output [T,H] | expert workspace | MLP workspace
 extern "C" OMNI_API size_t omni_moe_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size,
                                                     int64_t num_experts, int32_t num_expert_sqrt, int32_t num_experts_per_token,
                                                     int32_t dtype) {
@@ -89,7 +89,7 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   void* experts = w;    w += up256(T * (size_t)hidden_size * es);
   void* expert_ws = w;
   w += up256(omni_expert_workspace_bytes(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype, expert_algo));
-  void* h = w;
+  void* mlp_ws = w;
 
   hipStream_t main_s = (hipStream_t)stream;
   hipStream_t branch = side_stream ? (hipStream_t)side_stream : main_s;
@@ -108,16 +108,14 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   // (CUs come free between the rounds); with more tiles the streaming form wins although it holds every CU (hidden 1024 x
   // intermediate 4096, two streams: 4096 tokens 125.7 against 128.0 us, 6144 tokens 188.9 against 178.5, 8192 tokens 243.5 against 228.7)
   const int64_t gate_up_tiles = ((num_tokens + 255) / 256) * (((int64_t)intermediate_size + 127) / 128);
-  if (!e) e = (alone || gate_up_tiles > 512)
-                  ? omni_swiglu_linear_fwd(x, gate_weight, up_weight, h, num_tokens, hidden_size, intermediate_size, dtype, main_s)
-                  : omni_swiglu_linear_fwd_shared(x, gate_weight, up_weight, h, num_tokens, hidden_size, intermediate_size, dtype, main_s);
+  if (!e) e = mlp_gate_up_impl(x, gate_weight, up_weight, num_tokens, hidden_size, intermediate_size, dtype, mlp_ws, main_s, alone || gate_up_tiles > 512);
   if (!e) e = omni_expert_fwd(x, up_embed, down_embed, gates, ids, experts, num_tokens, hidden_size, num_experts,
                               num_experts_per_token, dtype, expert_algo, expert_ws, branch);
   if (!side_stream) {   // one stream: the add is the down projection's epilogue
-    if (!e) e = linear_fwd_impl(h, down_weight, experts, y, num_tokens, intermediate_size, hidden_size, dtype, main_s, true);
+    if (!e) e = mlp_down_impl(down_weight, experts, y, num_tokens, hidden_size, intermediate_size, dtype, mlp_ws, main_s, true);
     return e;
   }
-  if (!e) e = linear_fwd_impl(h, down_weight, nullptr, y, num_tokens, intermediate_size, hidden_size, dtype, main_s, false);
+  if (!e) e = mlp_down_impl(down_weight, nullptr, y, num_tokens, hidden_size, intermediate_size, dtype, mlp_ws, main_s, false);
   if ((he = hipEventRecord((hipEvent_t)join_event, branch)) != hipSuccess) return e ? e : OMNI_ERR_HIP_BASE + (int)he;
   if ((he = hipStreamWaitEvent(main_s, (hipEvent_t)join_event, 0)) != hipSuccess) return e ? e : OMNI_ERR_HIP_BASE + (int)he;
   if (e) return e;

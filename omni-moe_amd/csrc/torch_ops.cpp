@@ -213,7 +213,7 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     const Tensor x2 = x.view({T, l.H});
     const Tensor e = expert_forward(x2, up, down, r.gates, r.ids, OMNI_EXPERT_ALGO_AUTO);
     Tensor h = at::empty({T, l.I}, x.options()), gate = at::empty({T, l.I}, x.options()), upp = at::empty({T, l.I}, x.options());
-    if (dt != OMNI_F32 && l.I % 8 == 0 && l.H % 64 == 0) {
+    if (dt != OMNI_F32) {                          // (rows of 16 bytes, so both sizes are multiples of 8)
       check(omni_swiglu_linear_save_fwd(ptr(x), ptr(wg), ptr(wu), ptr(h), ptr(gate), ptr(upp), T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_swiglu_linear_save_fwd");
     } else {
       check(omni_linear_fwd(ptr(x), ptr(wg), nullptr, ptr(gate), T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_linear_fwd");
@@ -243,29 +243,46 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     const auto opt = x.options();
     variable_list out(9);
     // experts, then the router stage behind their gates' gradient
-    Tensor dx = at::empty({T, H}, opt);
+    Tensor dx_experts = at::empty({T, H}, opt), dup = at::empty_like(up), ddown = at::empty_like(down), dg = at::empty_like(gates);
     {
-      Tensor dup = at::empty_like(up), ddown = at::empty_like(down), dg = at::empty_like(gates);
       Tensor ws = bytes(omni_expert_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt), x.device());
-      check(omni_expert_bwd(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), ptr(dx), ptr(dup), ptr(ddown), ptr(dg), T, (int32_t)H, N,
+      check(omni_expert_bwd(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), ptr(dx_experts), ptr(dup), ptr(ddown), ptr(dg), T, (int32_t)H, N,
                             (int32_t)k, dt, ptr(ws), st), "omni_expert_bwd");
-      if (need[6]) out[6] = dup;
-      if (need[7]) out[7] = ddown;
-      if (need[0] || need[4] || need[5]) {
-        Tensor dz = at::empty({T, 2 * r}, opt);
-        Tensor nws = bytes(omni_router_norm_bwd_workspace_bytes(T, (int32_t)r), x.device());
-        const uint8_t* z = (const uint8_t*)ptr(rws);
-        check(omni_router_norm_bwd(ptr(dg), ptr(gates), (const int32_t*)ptr(ids), z, (const float*)(z + omni_router_workspace_stats_offset(T, (int32_t)r, dt)), ptr(dz), T,
-                                   (int32_t)r, (int32_t)k, dt, training ? 1 : 0, ptr(nws), st), "omni_router_norm_bwd");
-        if (need[4] || need[5]) {
-          const Tensor dw = at::mm(dz.t(), x);
-          if (need[4]) out[4] = dw.narrow(0, 0, r);
-          if (need[5]) out[5] = dw.narrow(0, r, r);
-        }
-        if (need[0]) dx.addmm_(dz, at::cat({rx, ry}));
+    }
+    if (need[6]) out[6] = dup;
+    if (need[7]) out[7] = ddown;
+    const bool own = dt != OMNI_F32, router = need[0] || need[4] || need[5];        // 16-bit products are the library's own
+    const int64_t rp = own ? (r + 7) / 8 * 8 : r;
+    Tensor dz;
+    if (router) {
+      dz = at::empty({T, 2 * rp}, opt);
+      Tensor nws = bytes(omni_router_norm_bwd_workspace_bytes(T, (int32_t)r), x.device());
+      const uint8_t* z = (const uint8_t*)ptr(rws);
+      const float* stats = (const float*)(z + omni_router_workspace_stats_offset(T, (int32_t)r, dt));
+      check((own ? omni_router_norm_bwd_padded : omni_router_norm_bwd)(ptr(dg), ptr(gates), (const int32_t*)ptr(ids), z, stats, ptr(dz), T, (int32_t)r, (int32_t)k, dt,
+                                                                        training ? 1 : 0, ptr(nws), st), "omni_router_norm_bwd");
+    }
+    if (own) {
+      const Tensor* like[6] = {&x, &wg, &wu, &wd, &rx, &ry};
+      for (int i = 0; i < 6; ++i)
+        if (need[i]) out[i] = at::empty_like(*like[i]);
+      Tensor ws = bytes(omni_mlp_bwd_workspace_bytes(T, (int32_t)H, (int32_t)I, (int32_t)r, dt), x.device());
+      const int32_t code = omni_mlp_bwd(ptr(dy), ptr(x), ptr(wg), ptr(wu), ptr(wd), ptr(gate), ptr(upp), ptr(h), ptr(dz), ptr(rx), ptr(ry), ptr(dx_experts), ptr(out[0]),
+                                        ptr(out[1]), ptr(out[2]), ptr(out[3]), ptr(out[4]), ptr(out[5]), T, (int32_t)H, (int32_t)I, (int32_t)r, dt, ptr(ws), st);
+      if (code != OMNI_ERR_UNSUPPORTED) {
+        check(code, "omni_mlp_bwd");
+        if (need[0]) out[0] = out[0].view(x3.sizes());
+        return out;
       }
     }
-    // shared MLP
+    // single precision, and operands of 2 GiB and more: library products
+    Tensor dx = dx_experts;
+    if (router) {
+      const Tensor zx = dz.narrow(1, 0, r), zy = dz.narrow(1, rp, r);
+      if (need[4]) out[4] = at::mm(zx.t(), x);
+      if (need[5]) out[5] = at::mm(zy.t(), x);
+      if (need[0]) dx.addmm_(zx, rx).addmm_(zy, ry);
+    }
     if (need[3]) out[3] = at::mm(dy.t(), h);
     if (need[0] || need[1] || need[2]) {
       const Tensor dh = at::mm(dy, wd);

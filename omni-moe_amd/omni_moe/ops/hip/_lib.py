@@ -61,6 +61,9 @@ SIGNATURES = {
     "omni_router_workspace_stats_offset": (c_size_t, [c_int64, c_int32, c_int32]),
     "omni_router_norm_bwd_workspace_bytes": (c_size_t, [c_int64, c_int32]),
     "omni_router_norm_bwd": (c_int32, [c_void_p] * 6 + [c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
+    "omni_router_norm_bwd_padded": (c_int32, [c_void_p] * 6 + [c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
+    "omni_mlp_bwd_workspace_bytes": (c_size_t, [c_int64, c_int32, c_int32, c_int32, c_int32]),
+    "omni_mlp_bwd": (c_int32, [c_void_p] * 18 + [c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
 }
 
 _lib = None

@@ -19,7 +19,7 @@ LIB_PATH = os.path.join(HERE, "libomni_moe_hip.so")
 NATIVE_PATH = os.path.join(HERE, "_native.so")
 OBJ_DIR = os.path.join(PKG_ROOT, "build")
 
-SOURCES = ["api.hip", "router.hip", "schedule.hip", "expert.hip", "gemm.hip", "layer.hip", "backward.hip"]
+SOURCES = ["gemm.hip", "gemm_tiles.hip", "router.hip", "expert.hip", "backward.hip", "schedule.hip", "layer.hip", "mlp_bwd.hip", "api.hip"]
 
 # packed-fp32 VALU forms are switched off for all device code of this library
 HIPCC_FLAGS = [
@@ -77,7 +77,7 @@ def _link_native(obj: str, verbose: bool) -> str:
     return NATIVE_PATH
 
 
-def build_library(verbose: bool = False, jobs: int = 4) -> str:
+def build_library(verbose: bool = False, jobs: int = 8) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         native = ex.submit(_compile_native, verbose)

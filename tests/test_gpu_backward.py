@@ -391,3 +391,73 @@ def test_expert_bwd_unused_rows_may_hold_nan(device):
     got = _ops().hip_omni_expert_bwd_func(d[0], d[1], up2.to(device), down2.to(device), d[4], d[5])
     for a, b in zip(got, want):
         assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+# T, H, I, r: one token and the smallest rows; ragged tiles of every shape the products take (64, 128, 256); K tails in every layout;
+# keys that are no multiple of 8; few tiles and long K (d(x) split along K); enough tokens for the 256 x 256 tile
+MLP_BWD_CASES = [(1, 8, 8, 0), (77, 64, 136, 7), (200, 72, 264, 17), (129, 520, 1032, 33), (1000, 512, 2048, 32), (300, 256, 4096, 16), (4100, 1032, 4104, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", MLP_BWD_CASES, ids=lambda c: "T%d-H%d-I%d-r%d" % c)
+def test_mlp_bwd_matches_matmuls(case, dtype, device):
+    """omni_mlp_bwd against the same products in fp32 on the same stored operands.  Both round d(h), d(gate) and d(up) to the storage type; sums in
+    another order move a last bit of some of them, so an output is within one rounding (2^-9 bf16, 2^-12 f16, relative) of the reference in the
+    2-norm, and within a few of the largest value anywhere."""
+    from omni_moe.ops.hip import _lib
+    lib = _lib.load()
+    T, H, I, r = case
+    g = torch.Generator(device=device).manual_seed(T + H)
+    n = lambda *s, std=1.0: torch.empty(*s, device=device).normal_(0, std, generator=g).to(dtype)
+    dy, x, gate, up = n(T, H), n(T, H), n(T, I), n(T, I)
+    wg, wu, wd = n(I, H, std=0.05), n(I, H, std=0.05), n(H, I, std=0.05)
+    h = (torch.nn.functional.silu(gate.float()) * up.float()).to(dtype)
+    rp = (r + 7) // 8 * 8
+    rx, ry, addend = n(max(r, 1), H, std=0.05)[:r], n(max(r, 1), H, std=0.05)[:r], n(T, H)
+    dz = torch.zeros(T, 2, rp, device=device, dtype=dtype)
+    dz[:, :, :r] = n(T, 2, max(r, 1))[:, :, :r]
+    rnd = lambda t: t.to(dtype).float()
+    dh = rnd(dy.float() @ wd.float())
+    gf, sig = gate.float(), torch.sigmoid(gate.float())
+    dup = rnd(dh * gf * sig)
+    dgate = rnd(dh * (gf * sig * (1 - sig) + sig) * up.float())
+    dx = rnd(dgate @ wg.float() + dup @ wu.float() + dz[:, 0, :r].float() @ rx.float() + dz[:, 1, :r].float() @ ry.float()) + addend.float()
+    want = [dx, dgate.t() @ x.float(), dup.t() @ x.float(), dy.float().t() @ h.float()]
+    if r:
+        want += [dz[:, 0, :r].float().t() @ x.float(), dz[:, 1, :r].float().t() @ x.float()]
+    got = [torch.full(w.shape, float("nan"), device=device, dtype=dtype) for w in want]
+    ptrs = [t.data_ptr() for t in got] + [None] * (6 - len(got))
+    dt = _lib.DTYPE_CODE[dtype]
+    ws = torch.empty(lib.omni_mlp_bwd_workspace_bytes(T, H, I, r, dt), device=device, dtype=torch.uint8)
+    print(f"mlp_bwd T={T} H={H} I={I} r={r} {dtype}", flush=True)
+    args = [t.data_ptr() for t in (dy, x, wg, wu, wd, gate, up, h)] + ([dz.data_ptr(), rx.data_ptr(), ry.data_ptr()] if r else [None] * 3)
+    _lib.check(lib.omni_mlp_bwd(*args, addend.data_ptr(), *ptrs, T, H, I, r, dt, ws.data_ptr(), _lib.stream_ptr()), "omni_mlp_bwd")
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for name, a, w in zip(("dx", "dWg", "dWu", "dWd", "dWx", "dWy"), got, want):
+        err = a.float() - w
+        assert (err.norm() <= ulp * w.norm()).item(), (name, (err.norm() / w.norm()).item())
+        assert (err.abs().max() <= 4 * ulp * w.abs().max()).item(), (name, (err.abs().max() / w.abs().max()).item())
+
+
+@pytest.mark.parametrize("training", [True, False], ids=["train", "eval"])
+@pytest.mark.parametrize("case", [(300, 32, 8), (5, 17, 4), (4100, 64, 16), (70, 300, 32)], ids=lambda c: "T%d-r%d-k%d" % c)
+def test_router_norm_bwd_padded(case, training, device):
+    """The padded layout holds exactly what the packed one does, and zeros behind it."""
+    from omni_moe.ops.hip import _lib
+    lib = _lib.load()
+    T, r, k = case
+    g = torch.Generator(device=device).manual_seed(r)
+    dg, gates = (torch.empty(T, k, device=device).uniform_(0.1, 1, generator=g).bfloat16() for _ in range(2))
+    ids = torch.randint(0, r * r, (T, k), device=device, dtype=torch.int32, generator=g)
+    z = torch.empty(T, 2 * r, device=device).normal_(generator=g).bfloat16()
+    stats = torch.rand(4 * r, device=device, generator=g) + 0.5
+    ws = torch.empty(max(lib.omni_router_norm_bwd_workspace_bytes(T, r), 1), device=device, dtype=torch.uint8)
+    rp = (r + 7) // 8 * 8
+    packed = torch.full((T, 2, r), float("nan"), device=device, dtype=torch.bfloat16)
+    padded = torch.full((T, 2, rp), float("nan"), device=device, dtype=torch.bfloat16)
+    for fn, out in ((lib.omni_router_norm_bwd, packed), (lib.omni_router_norm_bwd_padded, padded)):
+        _lib.check(fn(dg.data_ptr(), gates.data_ptr(), ids.data_ptr(), z.data_ptr(), stats.data_ptr(), out.data_ptr(), T, r, k, _lib.OMNI_BF16, int(training),
+                      ws.data_ptr(), _lib.stream_ptr()), "omni_router_norm_bwd")
+    assert torch.isfinite(packed).all()
+    assert torch.equal(padded[:, :, :r], packed)
+    assert (padded[:, :, r:] == 0).all()
