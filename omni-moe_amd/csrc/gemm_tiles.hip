@@ -89,19 +89,25 @@ __device__ __forceinline__ void each_op(F&& f) { each_op_of<Plan, S>(f, std::mak
 __device__ __forceinline__ u32x2_t lds_read_transposed(uint32_t at) {
   return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(uintptr_t)at));
 }
-// 16 bytes per lane from base + off (zeros past `bytes`) to 1 KiB of LDS.  Spelled out, so that the compiler does not take part in counting
+// 16 bytes per lane from base + off + more (zeros past `bytes`; the check counts both offsets) to 1 KiB of LDS.  Spelled out, so that the compiler does not take part in counting
 // it: it would put a wait for ALL outstanding loads in front of every transposing read that follows one, because it cannot tell
 // the two places in LDS apart (4096 x 1024 x 4096, both operands transposed, 256 x 256 tiles: 113 us so, 92 us without).  The kernel
 // does its own waiting.
 template <int kAt>
-__device__ __forceinline__ void load_to_lds(uint64_t base, int bytes, uint32_t lds_base, uint32_t off) {
+__device__ __forceinline__ void load_to_lds(uint64_t base, int bytes, uint32_t lds_base, uint32_t off, int more) {
   const u32x4_t r = {(uint32_t)base, (uint32_t)(base >> 32), (uint32_t)bytes, 0x00020000u};
-  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(off), "s"(r), "n"(kAt) : "memory", "scc");   // (and m0, which nothing else in this file uses)
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_base), "v"(off), "s"(r), "s"(more), "n"(kAt)
+               : "memory", "scc");   // (and m0, which nothing else in this file uses)
 }
 __device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 template <int N> __device__ __forceinline__ void vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// 8-byte and 16-byte fragment reads, epilogue helpers
+// The value, as one that the compiler knows nothing about: what is derived from it is computed where it is needed and not kept in registers
+// around the K loop (which must leave room on a SIMD for waves of the kernels that run beside it)
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
 __device__ __forceinline__ u32x4_t row_quads(const uint32_t x0, const uint32_t x1, const uint32_t x2, const uint32_t x3, const int from) {
   return u32x4_t{(uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)x0), (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)x1),
                  (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)x2), (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)x3)};
@@ -175,13 +181,14 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
   // piece t ^ s(r), s(r) = r % 4 + 4 (r / 8 % 2): the eight rows that 32 lanes of a transposing read take then lie in different
   // banks (rows of 128 bytes, two to the 256 bytes of banks: s(r) = r / 2 % 2 + 2 (r / 8 % 2)).
   auto piece_of = [](int row, int width) -> int { return width >= 128 ? (row & 3) | ((row >> 1) & 4) : ((row >> 1) & 1) | ((row >> 2) & 2); };
-  const int row_chunk = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);        // rows along K: the chunk that a lane loads (NW is even)
-  uint32_t a_off[KG][PA], b_off[KG][PB];
+  // (rows along K: a lane loads chunk lane % 8 ^ (4 wave + lane / 16) % 8 of its rows, whatever the load -- NW is even)
+  constexpr int kOff = kTail ? KG : 1;
+  uint32_t a_off[kOff], b_off[kOff];                           // lane offsets, the same for every load of a step (past a segment's K they differ by group)
   // Everything a load takes beside its lane offset is a scalar that moves on once per ring step: the operands' addresses and what is left of
   // their matrices behind them (nothing, once every ring step has been requested: the loads then fetch nothing, which is cheaper than
   // a branch around each -- a scalar branch among the matrix instructions costs a lone wave as much as one of them).
   uint64_t f_a = 0, f_b = 0;
-  int f_aleft = 0, f_bleft = 0, f_astep = 0, f_bstep = 0;
+  int f_aleft = 0, f_bleft = 0, f_astep = 0, f_bstep = 0, f_amore = 0, f_bmore = 0;      // ..more: from one load of a step to the wave's next
   int f_seg = -1, f_left = 0;                                  // K values of the segment from the cursor on
   int f_half = 0;                                              // kTileTwo: rows of the fetched tile, counted from the wave's first, that are the first matrix's
   constexpr uint32_t kOutside = 0x80000000u;
@@ -197,16 +204,16 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
       if (f_left < 64 * KG) {
 #pragma unroll
         for (int s = 0; s < KG; ++s) {
+          const int lane = opaque(tid & 63), row_chunk = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
           const bool outside = row_chunk * 8 + 64 * s >= f_left;
-#pragma unroll
-          for (int q = 0; q < PA; ++q) if (!AC) a_off[s][q] = outside ? kOutside : a_off[s][q];
-#pragma unroll
-          for (int q = 0; q < PB; ++q) if (!BC) b_off[s][q] = outside ? kOutside : b_off[s][q];
+          if (!AC) a_off[s % kOff] = outside ? kOutside : a_off[s % kOff];
+          if (!BC) b_off[s % kOff] = outside ? kOutside : b_off[s % kOff];
         }
       }
     }
   };
   auto enter_segment = [&](int skip) {                         // at its ring step `skip`
+    const int lane = opaque(tid & 63), row_chunk = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
     const TileSegment& sg = p.seg[f_seg];
     f_left = scalar(sg.K - 64 * KG * skip);
     const int lda = (int)sg.lda, ldb = (int)sg.ldb;
@@ -218,34 +225,29 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
     f_b = scalar64((uint64_t)sg.b + (BC ? (int64_t)fn0 * 2 : (int64_t)fn0 * ldb) + b_in);
     f_bleft = scalar((int)((BC ? (int64_t)sg.K * ldb - (int64_t)fn0 * 2 : (int64_t)min(N - fn0, BN) * ldb) - b_in));
     if constexpr (EPI == kTileTwo) f_half = scalar(N / 2 - fn0 - wave * 8);
-#pragma unroll
-    for (int q = 0; q < PA; ++q) {
-      uint32_t off;
-      if constexpr (AC) {
-        constexpr int W = BM / 8;
-        const int r = (q * NW + wave) * (64 / W) + lane / W;
-        off = (uint32_t)(r * lda) + (uint32_t)((lane % W) ^ (piece_of(r, BM) << 1)) * 16;
-      } else {
-        off = (uint32_t)(((q * NW + wave) * 8 + (lane >> 3)) * lda) + (uint32_t)row_chunk * 16;
-      }
-#pragma unroll
-      for (int s = 0; s < KG; ++s) a_off[s][q] = off;
+    uint32_t a0, b0;
+    if constexpr (AC) {
+      constexpr int W = BM / 8;
+      const int r = wave * (64 / W) + lane / W;
+      a0 = (uint32_t)(r * lda) + (uint32_t)((lane % W) ^ (piece_of(r, BM) << 1)) * 16;
+      f_amore = scalar(NW * (64 / W) * lda);
+    } else {
+      a0 = (uint32_t)((wave * 8 + (lane >> 3)) * lda) + (uint32_t)row_chunk * 16;
+      f_amore = scalar(NW * 8 * lda);
+    }
+    if constexpr (BC) {
+      constexpr int W = BN / 8;
+      const int r = wave * (64 / W) + lane / W;
+      b0 = (uint32_t)(r * ldb) + (uint32_t)((lane % W) ^ (piece_of(r, BN) << 1)) * 16;
+      f_bmore = scalar(NW * (64 / W) * ldb);
+    } else {
+      int r = wave * 8 + (lane >> 3);
+      if constexpr (EPI == kTileSwiglu) r = r % (TN * 8);      // a wave's first TN / 2 column tiles are gate rows, the rest the matching up rows
+      b0 = (uint32_t)(r * ldb) + (uint32_t)row_chunk * 16;
+      f_bmore = scalar((EPI == kTileSwiglu ? TN * 8 : NW * 8) * ldb);
     }
 #pragma unroll
-    for (int q = 0; q < PB; ++q) {
-      uint32_t off;
-      if constexpr (BC) {
-        constexpr int W = BN / 8;
-        const int r = (q * NW + wave) * (64 / W) + lane / W;
-        off = (uint32_t)(r * ldb) + (uint32_t)((lane % W) ^ (piece_of(r, BN) << 1)) * 16;
-      } else {
-        int r = (q * NW + wave) * 8 + (lane >> 3);
-        if constexpr (EPI == kTileSwiglu) r = (r / (TN * 16)) * (TN * 8) + r % (TN * 8);     // a wave's first TN / 2 column tiles are gate rows, the rest the matching up rows
-        off = (uint32_t)(r * ldb) + (uint32_t)row_chunk * 16;
-      }
-#pragma unroll
-      for (int s = 0; s < KG; ++s) b_off[s][q] = off;
-    }
+    for (int s = 0; s < kOff; ++s) { a_off[s] = a0; b_off[s] = b0; }
     mask_tail();
   };
   int tiles = p.steps;                                         // ring steps of one output tile in this block
@@ -270,31 +272,29 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
   uint64_t to_second = 0;
   if constexpr (EPI == kTileSwiglu) to_second = scalar64((uint64_t)p.b_up - (uint64_t)p.seg[0].b);
   if constexpr (EPI == kTileTwo) to_second = scalar64((uint64_t)p.b_up - (uint64_t)p.seg[0].b - (uint64_t)(N / 2) * (uint64_t)p.seg[0].ldb);
-  // the cursor's ring step as its loads take it, group by group (through readfirstlane once more: the compiler does not always see that
+  // the cursor's ring step as its loads take it (through readfirstlane once more: the compiler does not always see that
   // they are the same in every lane)
-  uint64_t c_a[KG], c_b[KG];
-  int c_aleft[KG], c_bleft[KG];
+  uint64_t c_a = 0, c_b = 0;
+  int c_aleft = 0, c_bleft = 0;
   uint32_t c_to = 0;
   auto settle = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int s = 0; s < KG; ++s) {
-      c_a[s] = scalar64(f_a + s * (uint32_t)f_astep);
-      c_b[s] = scalar64(f_b + s * (uint32_t)f_bstep);
-      c_aleft[s] = scalar(max(f_aleft - s * f_astep, 0));
-      c_bleft[s] = scalar(max(f_bleft - s * f_bstep, 0));
-    }
+    c_a = scalar64(f_a);
+    c_b = scalar64(f_b);
+    c_aleft = scalar(max(f_aleft, 0));
+    c_bleft = scalar(max(f_bleft, 0));
     c_to = (uint32_t)scalar((int)(lds_wave + (uint32_t)f_stage));
   };
   // load q of it
   auto issue_one = [&](auto q_tag) __attribute__((always_inline)) {
     constexpr int q = decltype(q_tag)::value, s = q / (PA + PB), o = q % (PA + PB);
     if constexpr (o < PA) {
-      load_to_lds<s * kSub + o * NW * 1024>(c_a[s], c_aleft[s], c_to, a_off[s][o]);
+      load_to_lds<s * kSub + o * NW * 1024>(c_a, c_aleft, c_to, a_off[s % kOff], s * f_astep + o * f_amore);
     } else {
-      uint64_t base = c_b[s];
-      if constexpr (EPI == kTileSwiglu) base += (((o - PA) * NW + wave) * 8 / (TN * 8)) & 1 ? to_second : 0;
-      if constexpr (EPI == kTileTwo) base += (o - PA) * NW * 8 >= f_half ? to_second : 0;     // (the eight rows of a load are of one matrix)
-      load_to_lds<s * kSub + kABytes + (o - PA) * NW * 1024>(base, c_bleft[s], c_to, b_off[s][o - PA]);
+      uint64_t base = c_b;
+      constexpr int b = o - PA, row = b * NW * 8, nth = EPI == kTileSwiglu ? row / (TN * 16) : b;
+      if constexpr (EPI == kTileSwiglu) base += ((row + wave * 8) / (TN * 8)) & 1 ? to_second : 0;
+      if constexpr (EPI == kTileTwo) base += row >= f_half ? to_second : 0;     // (the eight rows of a load are of one matrix)
+      load_to_lds<s * kSub + kABytes + b * NW * 1024>(base, c_bleft, c_to, b_off[s % kOff], s * f_bstep + nth * f_bmore);
     }
   };
   auto advance = [&]() __attribute__((always_inline)) {
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
   // ---- epilogue.  acc[i][j]: row 16 i + r16, columns 16 j + 4 g4 .. + 3.  One bpermute per word puts each row's 64 bytes into four
   // consecutive lanes (the store path wants that: see the streaming GEMM); 16-bit results first trade words between lanes l and
   // l ^ 16, so that a lane holds 8 columns.
-  const int tr = lane >> 2, tg = lane & 3, from = (tr + 16 * tg) * 4;
+  const int lane_e = opaque(lane), tr = lane_e >> 2, tg = lane_e & 3, from = (tr + 16 * tg) * 4;
   const int nb = n0 + wn * (BNO / WN);
   if (p.part) {                                                // partial sums: [split][M][columns] fp32, columns = N (SwiGLU: gate, then up)
     const int64_t cols = EPI == kTileSwiglu ? 2 * (int64_t)N : N;
@@ -752,10 +752,8 @@ static hipError_t launch_tiles(TileGroup& g, float* ws, int splits, bool exclusi
     if constexpr (LAY == kNT && kId == 0) {
       // one stream per CU where there are more tiles than CUs and nothing is meant to run beside the launch; else one block per tile, so
       // that CUs come free for other streams' kernels as blocks retire
-      if (splits == 1 && one.p[0].segments == 1) {
-        const int64_t grid = exclusive && blocks > 256 ? 256 : blocks;
-        return tail ? start_tiles<DT, LAY, kId, EPI, true, true>(one, grid, s) : start_tiles<DT, LAY, kId, EPI, false, true>(one, grid, s);
-      }
+      if (exclusive && blocks > 256 && splits == 1 && one.p[0].segments == 1)
+        return tail ? start_tiles<DT, LAY, kId, EPI, true, true>(one, 256, s) : start_tiles<DT, LAY, kId, EPI, false, true>(one, 256, s);
     }
     e = tail ? start_tiles<DT, LAY, kId, EPI, true, false>(one, blocks, s) : start_tiles<DT, LAY, kId, EPI, false, false>(one, blocks, s);
   }
