@@ -5,6 +5,8 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <type_traits>
+#include <utility>
 
 namespace omni {
 
@@ -98,6 +100,20 @@ __device__ __forceinline__ float xor_lane_f(float v, int lane) {
   return __int_as_float(xor_lane_i<STRIDE>(__float_as_int(v), lane));
 }
 
+// ---- loads into LDS --------------------------------------------------------------
+// 16 bytes per lane from base + off + more (zeros past `bytes`; the check counts both offsets) to 1 KiB of LDS.  Spelled out, so that the compiler does not take part in counting
+// it: it would put a wait for ALL outstanding loads in front of every transposing read that follows one, because it cannot tell
+// the two places in LDS apart (4096 x 1024 x 4096, both operands transposed, 256 x 256 tiles: 113 us so, 92 us without).  The kernels
+// that use it do their own waiting.
+template <int kAt>
+__device__ __forceinline__ void load_to_lds(uint64_t base, int bytes, uint32_t lds_base, uint32_t off, int more) {
+  const u32x4_t r = {(uint32_t)base, (uint32_t)(base >> 32), (uint32_t)bytes, 0x00020000u};
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_base), "v"(off), "s"(r), "s"(more), "n"(kAt)
+               : "memory", "scc");   // (and m0, which nothing else here uses)
+}
+__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+template <int N> __device__ __forceinline__ void vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
 // x*sigmoid(x) in fp32, IEEE division.
 __device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + __expf(-x)); }
 // Same with the hardware reciprocal (1 ulp) and exp2: ~6 instructions.  For results that are
@@ -105,6 +121,10 @@ __device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + __expf(-
 __device__ __forceinline__ float silu_fast(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
 }
+
+// f(0, 1, ...), with the numbers as types: what depends on them is decided at compile time
+template <class F, int... I>
+__device__ __forceinline__ void with_sequence(F& f, std::integer_sequence<int, I...>) { f(std::integral_constant<int, I>{}...); }
 
 // ---- host side ---------------------------------------------------------------
 // A kernel whose dynamic LDS exceeds the 64 KiB default needs its limit raised once per device (the

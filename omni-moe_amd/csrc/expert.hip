@@ -591,7 +591,7 @@ static int expert_dense_dispatch(const void* x, const void* up, const void* down
 //   slice   1 KiB (hidden 4096): 0.59-0.95 with 32 experts per token (a token's pairs fill half of the 64 lanes that
 //                                share out a batch), 1.05-1.38 with 16
 // A skewed router (few live experts) moves every figure towards the split algorithm; the caller who knows says so.
-static int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
+int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
   if (algo != OMNI_EXPERT_ALGO_AUTO) return algo;
   // The dense algorithm is never chosen here: it multiplies every token by every table row, so one non-finite value
   // in a row that nobody selected would reach every token (0 * Inf), where the other algorithms and the reference

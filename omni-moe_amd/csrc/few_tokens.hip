@@ -1,0 +1,392 @@
+// The layer (reference omni_moe/modules/omni_moe.py:60-106) for at most 64 tokens, as in decoding: three launches.
+//
+// What bounds it.  The weights' one trip through memory (25 MB at hidden 1024 x intermediate 4096: 5 us) and, above all, the chain of
+// dependent launches: as six kernels -- projection, select, gate/up, experts, down projection, its partial sums -- the stages
+// took 5-8 us each although none has work for that long (38 us a call for 1 token, 43 us for 48).  So what does not depend on
+// each other shares a launch, by block index:
+//   1. the router's projection | gate and up with their SwiGLU product
+//   2. the router's selection  | the down projection, K split over the grid, as fp32 partial sums
+//   3. the experts, the partial sums and the final add, one block per token.
+// 1 token 38.4 -> 19.5 us a call (kernels 6.5 + 6.7 + 4.3), 48 tokens 42.9 -> 24.0 us (10.8 + 8.4 + 5.3), hidden 1024 x intermediate 4096.
+//
+// Projections.  There is one row tile, so every weight is used once and nothing is gained by staging it through LDS: a lane loads
+// its matrix fragments (8 consecutive K values of a row) straight from memory, all loads of 1024 K values of a block in flight at once.
+// The eight waves of a block share the K range -- a wave takes 64 of K, a 128-byte line of each row, in turn -- and add up
+// through LDS in wave order.  A block has 32 weight rows: 16 gate and the matching 16 up rows, 16 x and 16 y keys, or 32 rows of the
+// down projection; with K split up to eight ways the latter fill the chip too.
+//
+// Experts.  Eight waves share a token's slots, so that all its rows are requested at once, and the block adds their sums in wave order.
+#include "few_tokens.h"
+#include "omni_moe_hip.h"
+#include "rows.h"
+
+#include <type_traits>
+
+namespace omni {
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+
+constexpr int kFewWaves = 8, kFewThreads = kFewWaves * kWave, kUnit = 64 /* of K */, kMostParts = 8;
+
+template <int DT>
+__device__ __forceinline__ f32x4_t mfma(const u32x4_t a, const u32x4_t b, f32x4_t c) {
+  if constexpr (DT == kBF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+template <int DT> __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  if constexpr (DT == kBF16) return pack_bf16(lo, hi); else return pack_f16(lo, hi);
+}
+
+// acc[j][i]: rows 16 i + lane % 16 of `a` ([rows of row_bytes], a_bytes in all, K values a row; TM row tiles, zeros past the matrix) times the 16
+// rows of weight tile j, columns 4 (lane / 16) .. + 3, over the K units u0 + wave, u0 + wave + 8, .. below u1, two at a time.
+// Weights: this lane's row b0 or b1, straight into registers, two units ahead.  Activations: every block reads all of them, from L2, and reads of
+// 64 bytes from each of 16 rows -- what a fragment is -- are slow there (64 tokens, hidden 1024: 15.4 us for launch 1, 10.1 us when an
+// instruction reads 1 KiB on end); so they take whole 128-byte lines of 8 rows into the wave's own `lds` (TM * 4 KiB; position c of row r
+// holds the row's 16-byte piece c ^ (r / 2 % 8), which keeps the fragment reads free of bank conflicts).
+// kTail: K is no multiple of 64 (but of 8); what is past it reads as zero on both sides.
+template <int DT, int TM, bool kTail>
+__device__ __forceinline__ void multiply(f32x4_t (&acc)[2][TM], const uint8_t* a, int row_bytes, int a_bytes, const uint8_t* b0, const uint8_t* b1, int K, int u0, int u1,
+                                         int wave, int lane, uint32_t lds) {
+  const int r16 = lane & 15, g4 = lane >> 4;
+  using Frag = const __attribute__((address_space(3))) u32x4_t*;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i) acc[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  u32x4_t b[2][2][2];                                          // [unit][half of it][weight tile]
+  auto load_weights = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int v = u + q * kFewWaves;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const int k = v * kUnit + ks * 32 + g4 * 8;
+        const bool inside = v < u1 && !(kTail && k >= K);
+        b[q][ks][0] = inside ? *(const u32x4_t*)(b0 + (int64_t)k * 2) : u32x4_t{0, 0, 0, 0};
+        b[q][ks][1] = inside ? *(const u32x4_t*)(b1 + (int64_t)k * 2) : u32x4_t{0, 0, 0, 0};
+      }
+    }
+  };
+  const uint32_t row = (uint32_t)(lane >> 3), from = row * (uint32_t)row_bytes;
+  load_weights(u0 + wave);
+  for (int u = u0 + wave; u < u1; u += 2 * kFewWaves) {
+    auto load_rows = [&](auto n_tag) __attribute__((always_inline)) {
+      constexpr int n = decltype(n_tag)::value, q = n / (2 * TM), part = n % (2 * TM);
+      // rows 8 part + lane / 8: r / 2 % 8 = 4 (part % 2) + lane / 16
+      const int piece = (lane & 7) ^ (4 * (part & 1) + (lane >> 4)), k = (u + q * kFewWaves) * kUnit + piece * 8;
+      const bool inside = u + q * kFewWaves < u1 && !(kTail && k >= K);
+      load_to_lds<n * 1024>((uint64_t)a, a_bytes, lds, inside ? from + (uint32_t)(part * 8 * row_bytes + k * 2) : 0x80000000u, 0);
+    };
+    auto load_all = [&](auto... n) __attribute__((always_inline)) { (load_rows(n), ...); };
+    with_sequence(load_all, std::make_integer_sequence<int, 4 * TM>{});
+    vmcnt<0>();
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4_t w[2][2][2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) w[q][ks][j] = b[q][ks][j];
+    if (u + 2 * kFewWaves < u1) load_weights(u + 2 * kFewWaves);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const u32x4_t f = *(Frag)(uintptr_t)(lds + (uint32_t)((q * TM + i) * 2048 + r16 * 128 + ((4 * ks + g4) ^ (r16 >> 1)) * 16));
+          acc[0][i] = mfma<DT>(w[q][ks][0], f, acc[0][i]);
+          acc[1][i] = mfma<DT>(w[q][ks][1], f, acc[1][i]);
+        }
+    lds_reads_done();                                          // before the next loads overwrite what they read
+  }
+}
+
+// The block's eight sums meet in LDS, each in its wave's own TM * 4 KiB
+template <int TM>
+__device__ __forceinline__ void publish(uint8_t* lds, const f32x4_t (&acc)[2][TM], int wave, int lane) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i) *(f32x4_t*)(lds + wave * TM * 4096 + ((j * TM + i) * kWave + lane) * 16) = acc[j][i];
+  __syncthreads();
+}
+// columns 4 quad .. + 3 of row `row` of weight tile j, all waves
+template <int TM>
+__device__ __forceinline__ f32x4_t gathered(const uint8_t* lds, int j, int row, int quad) {
+  f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < kFewWaves; ++w) {
+    const f32x4_t o = *(const f32x4_t*)(lds + w * TM * 4096 + ((j * TM + row / 16) * kWave + quad * 16 + row % 16) * 16);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] += o[q];
+  }
+  return v;
+}
+
+struct FrontArgs {
+  const uint8_t *x, *wg, *wu, *wx, *wy;
+  uint8_t *h, *z;
+  int T, H, I, r, router_blocks;
+};
+
+// Launch 1: blocks below router_blocks project 16 keys of each half, the others 16 columns of gate and of up.
+template <int DT, int TM, bool kTail>
+__global__ __launch_bounds__(kFewThreads, 2) void few_front_kernel(const FrontArgs g) {
+  extern __shared__ __align__(16) uint8_t lds[];               // TM * 4 KiB a wave
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15;
+  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * TM * 4096;
+  const bool router = (int)blockIdx.x < g.router_blocks;
+  const int n0 = (router ? (int)blockIdx.x : (int)blockIdx.x - g.router_blocks) * 16, rows = router ? g.r : g.I;
+  const int64_t row_bytes = (int64_t)g.H * 2, b_at = min(n0 + r16, rows - 1) * row_bytes;
+  f32x4_t acc[2][TM];
+  multiply<DT, TM, kTail>(acc, g.x, g.H * 2, g.T * g.H * 2, (router ? g.wx : g.wg) + b_at, (router ? g.wy : g.wu) + b_at, g.H, 0, (g.H + kUnit - 1) / kUnit, wave, lane, mine);
+  publish<TM>(lds, acc, wave, lane);
+  for (int i = threadIdx.x; i < TM * 64; i += kFewThreads) {
+    const int row = i >> 2, quad = i & 3, n = n0 + quad * 4;
+    if (row >= g.T || n >= rows) continue;
+    const f32x4_t p = gathered<TM>(lds, 0, row, quad), q = gathered<TM>(lds, 1, row, quad);
+    if (router) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < rows) {
+          Elem<DT>::store(g.z, (int64_t)row * 2 * g.r + n + e, p[e]);
+          Elem<DT>::store(g.z, (int64_t)row * 2 * g.r + g.r + n + e, q[e]);
+        }
+    } else {
+      // gate and up are materialised in the storage dtype, silu(gate) * up is formed in fp32 and rounded once (omni_mlp.py:53-61)
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = silu_fast(Elem<DT>::round(p[e])) * Elem<DT>::round(q[e]);
+      *(u32x2_t*)(g.h + ((int64_t)row * g.I + n) * 2) = u32x2_t{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+    }
+  }
+}
+
+struct MiddleArgs {
+  const uint8_t *h, *wd;
+  float* parts;                      // [splits][T][H]
+  int T, H, I, groups, units;        // groups of 32 output columns; K units to a split
+  int select_blocks, select_regs;    // keys per lane
+  SelectArgs select;
+};
+
+// Launch 2: blocks below select_blocks select for eight tokens each, the others multiply 32 output columns over one of the K splits.
+template <int DT, int TM, bool kTail, bool kSelect, int C>
+__global__ __launch_bounds__(kFewThreads, 2) void few_middle_kernel(const MiddleArgs g) {
+  extern __shared__ __align__(16) uint8_t lds[];               // TM * 4 KiB a wave
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15;
+  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * TM * 4096;
+  if constexpr (kSelect) {
+    if ((int)blockIdx.x < g.select_blocks) {
+      const int first = (int)blockIdx.x * kFewWaves + wave, all = g.select_blocks * kFewWaves;
+      if (g.select_regs <= 1) select_packed<1, C>(g.select, first, all);
+      else if (g.select_regs <= 2) select_packed<2, C>(g.select, first, all);
+      else if (g.select_regs <= 4) select_packed<4, C>(g.select, first, all);
+      else select_packed<8, C>(g.select, first, all);
+      return;
+    }
+  }
+  const int block = (int)blockIdx.x - (kSelect ? g.select_blocks : 0), split = block / g.groups, n0 = (block - split * g.groups) * 32;
+  const int64_t row_bytes = (int64_t)g.I * 2;
+  f32x4_t acc[2][TM];
+  multiply<DT, TM, kTail>(acc, g.h, g.I * 2, g.T * g.I * 2, g.wd + min(n0 + r16, g.H - 1) * row_bytes, g.wd + min(n0 + 16 + r16, g.H - 1) * row_bytes, g.I, split * g.units,
+                          min((split + 1) * g.units, (g.I + kUnit - 1) / kUnit), wave, lane, mine);
+  publish<TM>(lds, acc, wave, lane);
+  for (int i = threadIdx.x; i < TM * 128; i += kFewThreads) {
+    const int row = i >> 3, quad = i & 7, n = n0 + quad * 4;
+    if (row < g.T && n < g.H) *(f32x4_t*)(g.parts + ((int64_t)split * g.T + row) * g.H + n) = gathered<TM>(lds, quad >> 2, row, quad & 3);
+  }
+}
+
+struct BackArgs {
+  const uint8_t *x, *up, *down, *residual;
+  const void* gates;
+  const int32_t* ids;
+  const float* parts;
+  uint8_t* y;
+  int T, H, k, splits;
+  uint32_t N;
+};
+
+// Launch 3, a block per token: y = round(round(sum of the parts) + round(experts)).  NCH 1-KiB pieces of a row; G slots of a wave at once.
+// kExperts false: the MLP alone, residual (or nothing) instead of the experts.
+template <int DT, int NCH, int G, bool kExperts>
+__global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const BackArgs g) {
+  extern __shared__ __align__(16) float sums[];                // [waves][NCH * 512]
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x;
+  constexpr int kRow = NCH * 512;
+  // this thread's first four columns of every part, requested before anything else
+  f32x4_t part[kMostParts];
+  const int64_t plane = (int64_t)g.T * g.H;
+  auto request = [&](int n) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < kMostParts; ++s) part[s] = *(const f32x4_t*)(g.parts + min(s, g.splits - 1) * plane + (int64_t)t * g.H + min(n, g.H - 4));
+  };
+  request(threadIdx.x * 4);
+  const int per = kExperts ? (g.k + kFewWaves - 1) / kFewWaves : 0, active = kExperts ? (g.k + per - 1) / per : 0;
+  if (kExperts && wave < active) {
+    const int64_t row_bytes = (int64_t)g.H * 2;
+    bool live[NCH];
+    u32x4_t xr[NCH];
+    float acc[NCH][8];
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      live[c] = (c * kWave + lane) * 8 < g.H;
+      xr[c] = live[c] ? *(const u32x4_t*)(g.x + t * row_bytes + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[c][i] = 0.f;
+    }
+    const int last = min((wave + 1) * per, g.k);
+    for (int j0 = wave * per; j0 < last; j0 += G) {
+      int64_t at[G];
+      float gate[G];
+      bool ok[G];
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        const int j = min(j0 + i, last - 1), id = g.ids[(int64_t)t * g.k + j];
+        gate[i] = Elem<DT>::load(g.gates, (int64_t)t * g.k + j);
+        ok[i] = j0 + i < last && (uint32_t)id < g.N;           // a slot of another wave, or an id outside the table, contributes nothing
+        at[i] = ok[i] ? id * row_bytes : 0;
+      }
+      u32x4_t u[G][NCH], v[G][NCH];
+#pragma unroll
+      for (int i = 0; i < G; ++i)
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+          u[i][c] = live[c] ? *(const u32x4_t*)(g.up + at[i] + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
+          v[i][c] = live[c] ? *(const u32x4_t*)(g.down + at[i] + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
+        }
+      float s[G];
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        s[i] = 0.f;
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) s[i] = dot16<DT>(xr[c], u[i][c], s[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < G; ++i) s[i] = wave_sum(s[i]);
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        if (!ok[i]) continue;                                  // not even 0 * row: the stand-in row may hold Inf or NaN
+        const float coef = silu_f32(s[i]) * gate[i];
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) axpy16<DT>(coef, v[i][c], acc[c]);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NCH; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *(f32x4_t*)(sums + wave * kRow + (c * kWave + lane) * 8 + 4 * h) = f32x4_t{acc[c][4 * h], acc[c][4 * h + 1], acc[c][4 * h + 2], acc[c][4 * h + 3]};
+  }
+  if (kExperts) __syncthreads();
+  for (int n = threadIdx.x * 4; n < g.H; n += kFewThreads * 4) {
+    if (n != (int)threadIdx.x * 4) request(n);
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < kMostParts; ++s)
+      if (s < g.splits)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] += part[s][q];
+    const int64_t out = ((int64_t)t * g.H + n) * 2;
+    if (kExperts || g.residual) {
+      float e[4] = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (kExperts) {
+        for (int w = 0; w < active; ++w) {
+          const f32x4_t o = *(const f32x4_t*)(sums + w * kRow + n);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) e[q] += o[q];
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) e[q] = Elem<DT>::load(g.residual + out, q);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = Elem<DT>::round(v[q]) + Elem<DT>::round(e[q]);
+    }
+    *(u32x2_t*)(g.y + out) = u32x2_t{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+  }
+}
+
+// K splits of the down projection: as many as fill 256 CUs with blocks of 32 columns while each of a block's waves still has 64 of K
+int few_splits(int64_t H, int64_t I) {
+  const int64_t groups = (H + 31) / 32, units = (I + kUnit - 1) / kUnit;
+  int64_t n = 256 / groups;
+  if (n > units / kFewWaves) n = units / kFewWaves;
+  return n < 1 ? 1 : n > kMostParts ? kMostParts : (int)n;
+}
+
+template <auto kKernel, int kBytes>
+struct FewLds { static inline LdsKernel entry{(const void*)kKernel, kBytes}; };
+template <auto kKernel, int kBytes, class Args>
+hipError_t start(const Args& a, int64_t blocks, hipStream_t s) {
+  if (hipError_t e = FewLds<kKernel, kBytes>::entry.ensure(); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kKernel, dim3((unsigned)blocks), dim3(kFewThreads), kBytes, s, a);
+  return hipGetLastError();
+}
+
+template <int DT, int TM>
+hipError_t launch(const FewTokens& f, hipStream_t s) {
+  const bool layer = f.up != nullptr;
+  const int r = f.select.r;
+  const FrontArgs a{(const uint8_t*)f.x, (const uint8_t*)f.wg, (const uint8_t*)f.wu, (const uint8_t*)f.wx, (const uint8_t*)f.wy, (uint8_t*)f.h, (uint8_t*)f.z,
+                    f.T, f.H, f.I, r, layer ? (r + 15) / 16 : 0};
+  constexpr int kBytes = kFewWaves * TM * 4096;
+  const int64_t front = a.router_blocks + (f.I + 15) / 16;
+  hipError_t e = f.H % kUnit ? start<few_front_kernel<DT, TM, true>, kBytes>(a, front, s) : start<few_front_kernel<DT, TM, false>, kBytes>(a, front, s);
+  if (e != hipSuccess) return e;
+
+  const int units = (f.I + kUnit - 1) / kUnit;
+  MiddleArgs m{(const uint8_t*)f.h, (const uint8_t*)f.wd, f.parts, f.T, f.H, f.I, (f.H + 31) / 32, 0, layer ? (f.T + kFewWaves - 1) / kFewWaves : 0, (r + kWave - 1) / kWave, f.select};
+  int splits = few_splits(f.H, f.I);
+  m.units = (units + splits - 1) / splits;
+  splits = (units + m.units - 1) / m.units;                    // every split has work
+  const int cells = prepare_select(m.select);
+  const int64_t middle = m.select_blocks + (int64_t)m.groups * splits;
+  auto go = [&](auto tail) -> hipError_t {
+    constexpr bool kTail = decltype(tail)::value;
+    if (!layer) return start<few_middle_kernel<DT, TM, kTail, false, 1>, kBytes>(m, middle, s);
+    if (cells <= 1) return start<few_middle_kernel<DT, TM, kTail, true, 1>, kBytes>(m, middle, s);
+    return start<few_middle_kernel<DT, TM, kTail, true, 2>, kBytes>(m, middle, s);
+  };
+  if ((e = f.I % kUnit ? go(std::true_type{}) : go(std::false_type{})) != hipSuccess) return e;
+
+  const BackArgs b{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, (const uint8_t*)f.residual, f.select.gates, f.select.indices, f.parts, (uint8_t*)f.y,
+                   f.T, f.H, f.select.k, splits, (uint32_t)f.N};
+  if (!layer) return start<few_back_kernel<DT, 1, 1, false>, 0>(b, f.T, s);
+  const int nch = (f.H + 511) / 512;
+  if (nch <= 1) return start<few_back_kernel<DT, 1, 4, true>, kFewWaves * 1 * 2048>(b, f.T, s);
+  if (nch <= 2) return start<few_back_kernel<DT, 2, 4, true>, kFewWaves * 2 * 2048>(b, f.T, s);
+  if (nch <= 4) return start<few_back_kernel<DT, 4, 2, true>, kFewWaves * 4 * 2048>(b, f.T, s);
+  return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, f.T, s);
+}
+
+}  // namespace
+
+bool few_tokens_covers(int64_t T, int64_t H, int64_t I, int dtype) {
+  return T > 0 && T <= kFewTokens && dtype != OMNI_F32 && H % 8 == 0 && I % 8 == 0 && H <= (1 << 20) && I <= (1 << 20);   // (32-bit offsets)
+}
+bool few_tokens_covers_layer(int64_t T, int64_t H, int64_t I, int r, int k, int dtype) {
+  // keys and candidates that the joint launch has registers for; rows that a block holds its waves' sums of
+  return few_tokens_covers(T, H, I, dtype) && H <= 4096 && r <= 8 * kWave && k > 0 && num_cells(k, r < k ? r : k) <= 2 * kWave;
+}
+size_t few_tokens_parts_bytes(int64_t T, int64_t H, int64_t I) { return (size_t)few_splits(H, I) * (size_t)T * (size_t)H * 4; }
+
+hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s) {
+  auto go = [&](auto dt) -> hipError_t {
+    constexpr int DT = decltype(dt)::value;
+    if (f.T <= 16) return launch<DT, 1>(f, s);
+    if (f.T <= 32) return launch<DT, 2>(f, s);
+    if (f.T <= 48) return launch<DT, 3>(f, s);
+    return launch<DT, 4>(f, s);
+  };
+  if (dtype == kBF16) return go(std::integral_constant<int, kBF16>{});
+  if (dtype == kF16) return go(std::integral_constant<int, kF16>{});
+  return hipErrorInvalidValue;
+}
+
+}  // namespace omni

@@ -16,6 +16,7 @@
 // The weight fragment is the MFMA's first operand, so an accumulator lane holds 4 consecutive
 // output columns of one row; two lanes pair up to store 8 columns (16 bytes) each.
 #include "common.h"
+#include "few_tokens.h"
 #include "gemm_tiles.h"
 #include "omni_moe_hip.h"
 
@@ -898,8 +899,9 @@ namespace omni {
 // partial sums of whichever of the two projections is split along K (they are not alive together)
 static size_t mlp_sums_bytes(int64_t T, int64_t H, int64_t I, int dtype) {
   if (dtype == OMNI_F32 || I % 8 || H % 8) return 0;
-  const size_t a = tile_workspace_bytes(kTileSwiglu, T, I, H), b = tile_workspace_bytes(kTileResidual, T, H, I);
-  return a > b ? a : b;
+  const size_t few = few_tokens_covers(T, H, I, dtype) ? few_tokens_parts_bytes(T, H, I) : 0;
+  const size_t a = tile_workspace_bytes(kTileSwiglu, T, I, H), b = tile_workspace_bytes(kTileResidual, T, H, I), most = a > b ? a : b;
+  return most > few ? most : few;
 }
 static size_t mlp_h_bytes(int64_t T, int64_t I, int dtype) { return ((size_t)T * (size_t)I * (dtype == OMNI_F32 ? 4 : 2) + 255) / 256 * 256; }
 
@@ -954,6 +956,12 @@ extern "C" OMNI_API int32_t omni_mlp_fwd(const void* x, const void* gate_weight,
   const int es = dtype == OMNI_F32 ? 4 : 2;
   if ((e = check_gemm(num_tokens, intermediate_size, hidden_size, es)) || (e = check_gemm(num_tokens, hidden_size, intermediate_size, es)))
     return e;
+  if (few_tokens_covers(num_tokens, hidden_size, intermediate_size, dtype)) {
+    const FewTokens f{x, gate_weight, up_weight, down_weight, workspace, y, (float*)((char*)workspace + mlp_h_bytes(num_tokens, intermediate_size, dtype)), residual,
+                      (int)num_tokens, hidden_size, intermediate_size};
+    const hipError_t he = launch_few_tokens(dtype, f, (hipStream_t)stream);
+    return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
+  }
   if ((e = mlp_gate_up_impl(x, gate_weight, up_weight, num_tokens, hidden_size, intermediate_size, dtype, workspace, stream, true))) return e;
   return mlp_down_impl(down_weight, residual, y, num_tokens, hidden_size, intermediate_size, dtype, workspace, stream, true);
 }

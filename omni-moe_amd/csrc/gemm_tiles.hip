@@ -75,9 +75,7 @@ struct StepPlan {
   }
 };
 
-// f(0, 1, ...) and f(op), with the numbers as types: what depends on them is decided at compile time
-template <class F, int... I>
-__device__ __forceinline__ void with_sequence(F& f, std::integer_sequence<int, I...>) { f(std::integral_constant<int, I>{}...); }
+// f(op), with the number as a type: what depends on it is decided at compile time
 template <class Plan, int S, class F, int... U>
 __device__ __forceinline__ void each_op_of(F&& f, std::integer_sequence<int, U...>) {
   constexpr Plan plan{};
@@ -89,19 +87,6 @@ __device__ __forceinline__ void each_op(F&& f) { each_op_of<Plan, S>(f, std::mak
 __device__ __forceinline__ u32x2_t lds_read_transposed(uint32_t at) {
   return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(uintptr_t)at));
 }
-// 16 bytes per lane from base + off + more (zeros past `bytes`; the check counts both offsets) to 1 KiB of LDS.  Spelled out, so that the compiler does not take part in counting
-// it: it would put a wait for ALL outstanding loads in front of every transposing read that follows one, because it cannot tell
-// the two places in LDS apart (4096 x 1024 x 4096, both operands transposed, 256 x 256 tiles: 113 us so, 92 us without).  The kernel
-// does its own waiting.
-template <int kAt>
-__device__ __forceinline__ void load_to_lds(uint64_t base, int bytes, uint32_t lds_base, uint32_t off, int more) {
-  const u32x4_t r = {(uint32_t)base, (uint32_t)(base >> 32), (uint32_t)bytes, 0x00020000u};
-  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds_base), "v"(off), "s"(r), "s"(more), "n"(kAt)
-               : "memory", "scc");   // (and m0, which nothing else in this file uses)
-}
-__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-template <int N> __device__ __forceinline__ void vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 // The value, as one that the compiler knows nothing about: what is derived from it is computed where it is needed and not kept in registers
 // around the K loop (which must leave room on a SIMD for waves of the kernels that run beside it)
 __device__ __forceinline__ int opaque(int v) {

@@ -4,6 +4,7 @@
 // (the expert kernel lives on cache bandwidth and no LDS, the down projection on LDS and the
 // matrix cores, so they share CUs); the fork and the join are two events the caller owns.
 #include "common.h"
+#include "few_tokens.h"
 #include "omni_moe_hip.h"
 
 namespace omni {
@@ -11,6 +12,8 @@ static inline size_t up256(size_t v) { return (v + 255) / 256 * 256; }
 static inline size_t elem_bytes(int dtype) { return dtype == OMNI_F32 ? 4 : 2; }
 // defined beside the expert kernels: OMNI_OK when omni_expert_fwd takes `algo` at this shape (decided from the sizes alone)
 int expert_algo_check(int algo, int64_t num_tokens, int hidden_size, int64_t num_experts, int top_k, int dtype);
+// ... and which one OMNI_EXPERT_ALGO_AUTO is there
+int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype);
 // defined beside the select kernels: whether they take num_expert_sqrt keys per half with top_k and this dtype
 bool select_covers(int r, int k, int dtype);
 // defined beside the GEMM kernels: the two projections of omni_mlp_fwd with the caller's word on whether the launch has the GPU to itself
@@ -92,6 +95,26 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   void* mlp_ws = w;
 
   hipStream_t main_s = (hipStream_t)stream;
+  // A few tokens in eval mode: three launches in all, on the caller's stream (few_tokens.hip).  64 is four row
+  // tiles, what a wave has registers and LDS for; there the joint launches take 27 us where the six kernels took 44 (hidden 1024, bf16).
+  if (!training && num_experts <= UINT32_MAX && few_tokens_covers_layer(num_tokens, hidden_size, intermediate_size, num_expert_sqrt, num_experts_per_token, dtype) &&
+      resolve_algo(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) == OMNI_EXPERT_ALGO_GATHER) {
+    if (stats_dtype != OMNI_BF16 && stats_dtype != OMNI_F16 && stats_dtype != OMNI_F32) return OMNI_ERR_DTYPE;
+    if (!gate_weight || !up_weight || !down_weight || !router_weight_x || !router_weight_y || !running_mean_x || !running_var_x || !running_mean_y || !running_var_y)
+      return OMNI_ERR_NULL;
+    FewTokens f{x, gate_weight, up_weight, down_weight, mlp_ws, y, (float*)((char*)mlp_ws + up256(T * (size_t)intermediate_size * es)), nullptr,
+                (int)num_tokens, hidden_size, intermediate_size, router_weight_x, router_weight_y, router_ws};
+    SelectArgs& g = f.select;
+    g.lx = router_ws; g.ly = (const char*)router_ws + (size_t)num_expert_sqrt * es; g.row_stride = 2 * num_expert_sqrt;
+    g.run_mean[0] = running_mean_x; g.run_mean[1] = running_mean_y;
+    g.run_var[0] = running_var_x; g.run_var[1] = running_var_y;
+    g.stat_dt = stats_dtype; g.eps = eps;
+    g.gates = gates; g.indices = ids;
+    g.num_tokens = (int)num_tokens; g.r = num_expert_sqrt; g.k = num_experts_per_token; g.dt = dtype;
+    f.up = up_embed; f.down = down_embed; f.N = num_experts;
+    const hipError_t he = launch_few_tokens(dtype, f, main_s);
+    return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
+  }
   hipStream_t branch = side_stream ? (hipStream_t)side_stream : main_s;
   hipError_t he;
   if (side_stream) {

@@ -1,0 +1,359 @@
+// The router's selection for one wave, as device functions: the select kernels (router.hip; the selection itself is described
+// there) and the launch that selects beside a projection (few_tokens.hip) share them.
+#pragma once
+#include "common.h"
+
+namespace omni {
+
+// Storage dtype handled at run time (one uniform branch per access) to keep the number of
+// kernel instantiations at |R| x |C|.
+__device__ __forceinline__ float load_score(const void* p, int64_t i, int dt) {
+  return dt == kBF16 ? Elem<kBF16>::load(p, i) : dt == kF16 ? Elem<kF16>::load(p, i) : Elem<kF32>::load(p, i);
+}
+__device__ __forceinline__ float round_score(float v, int dt) {
+  return dt == kBF16 ? Elem<kBF16>::round(v) : dt == kF16 ? Elem<kF16>::round(v) : v;
+}
+__device__ __forceinline__ void store_score(void* p, int64_t i, float v, int dt) {
+  if (dt == kBF16) Elem<kBF16>::store(p, i, v);
+  else if (dt == kF16) Elem<kF16>::store(p, i, v);
+  else Elem<kF32>::store(p, i, v);
+}
+
+constexpr int kRouterWaves = 4;
+constexpr int kUnrollMaxR = 2;     // lists of <= 128 items use the unrolled, LDS-free exchanges
+constexpr int kMaxKeys = 1024;        // keys per half that the select kernels hold in registers (16 per lane)
+constexpr int kMaxKeysChunked = 16384; // ... that the chunked kernel walks (16-bit scores, at most 64 candidates per half)
+constexpr float kNegInf = -__builtin_huge_valf();
+
+struct SelectArgs {
+  const void* lx;        // x-half scores of token t at lx[t*row_stride + key]
+  const void* ly;
+  int64_t row_stride;
+  const float* stats;    // NULL, or [4][r] fp32: mean_x, rstd_x, mean_y, rstd_y -> the inputs are raw
+                         // projections; normalise and log-softmax them before selecting
+  const void* run_mean[2];  // instead of stats (eval-mode BatchNorm): the two halves' running_mean / running_var
+  const void* run_var[2];   //   [r] of dtype stat_dt; mean and 1/sqrt(var + eps) are formed here, and block 0
+  float* stats_out;         //   also leaves them at stats_out [4][r] (may be NULL) for a backward pass
+  int stat_dt;
+  float eps;
+  void* scores;          // [T,k] storage dtype, may be NULL
+  void* gates;           // [T,k] storage dtype = exp(score), may be NULL
+  int32_t* indices;      // [T,k]
+  int num_tokens, r, k, kp, dt;
+  uint8_t row_cells[128]; // candidate cells in row a: min(kp, k/(a+1)), filled by select_dispatch
+  int64_t* count_batch[2]; // NULL, or BatchNorm's num_batches_tracked of the two halves: incremented here, behind the
+                           // kernel that read them (train-mode router stage)
+};
+
+__device__ __forceinline__ void count_batch(const SelectArgs& g) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (g.count_batch[0]) *g.count_batch[0] += 1;
+    if (g.count_batch[1]) *g.count_batch[1] += 1;
+  }
+  if (blockIdx.x == 0 && !g.stats && g.run_mean[0] && g.stats_out) {   // eval mode: the statistics a backward pass reads
+    for (int i = threadIdx.x; i < 2 * g.r; i += blockDim.x) {
+      const int half = i >= g.r, key = i - half * g.r;
+      g.stats_out[(2 * half) * g.r + key] = load_score(g.run_mean[half], key, g.stat_dt);
+      g.stats_out[(2 * half + 1) * g.r + key] = __builtin_amdgcn_rsqf(load_score(g.run_var[half], key, g.stat_dt) + g.eps);
+    }
+  }
+}
+
+// BatchNorm (affine-free) of one raw projection value, rounded to the storage dtype as the reference's BatchNorm output is
+__device__ __forceinline__ float normalise_one(float v, const SelectArgs& g, const int half, const int key, const int r, const int dt) {
+  float mean, rstd;
+  if (g.stats) {
+    mean = g.stats[(2 * half) * r + key];
+    rstd = g.stats[(2 * half + 1) * r + key];
+  } else {
+    mean = load_score(g.run_mean[half], key, g.stat_dt);
+    rstd = __builtin_amdgcn_rsqf(load_score(g.run_var[half], key, g.stat_dt) + g.eps);
+  }
+  return round_score((v - mean) * rstd, dt);
+}
+
+// BatchNorm (affine-free) then log-softmax of one half, in place: v holds the raw projection
+// of key a*64+lane (NaN-free -inf padding past r).  Each stage rounds to the storage dtype
+// where the reference's torch ops do (BN output, log-softmax output; omni_moe.py:70-78).
+template <int R>
+__device__ __forceinline__ void normalise_half(float (&v)[R], const SelectArgs& g, const int half, int r, int lane, int dt) {
+  float m = kNegInf;
+#pragma unroll
+  for (int a = 0; a < R; ++a) {
+    const int key = a * kWave + lane;
+    if (key < r) {
+      float mean, rstd;
+      if (g.stats) {
+        mean = g.stats[(2 * half) * r + key];
+        rstd = g.stats[(2 * half + 1) * r + key];
+      } else {                                   // per token and key: the hardware's reciprocal square root (1 ulp), as in stats_out
+        mean = load_score(g.run_mean[half], key, g.stat_dt);
+        rstd = __builtin_amdgcn_rsqf(load_score(g.run_var[half], key, g.stat_dt) + g.eps);
+      }
+      v[a] = round_score((v[a] - mean) * rstd, dt);
+    }
+    m = fmaxf(m, v[a]);
+  }
+  m = wave_max(m);
+  float e = 0.f;
+#pragma unroll
+  for (int a = 0; a < R; ++a) e += (a * kWave + lane < r) ? expf(v[a] - m) : 0.f;
+  const float lse = logf(wave_sum(e));
+#pragma unroll
+  for (int a = 0; a < R; ++a)
+    if (a * kWave + lane < r) v[a] = round_score(v[a] - m - lse, dt);
+}
+
+// This lane's candidate cells: cell index ci = c*64+lane enumerates rows a = 0..kp-1 with
+// min(kp, k/(a+1)) cells each.  Payload (a<<8)|b orders like position a*kp+b.  The row counts
+// come with the arguments: the lanes fetch them all at once (row a in lane a%64) and the uniform
+// loop hands them round by readlane, so it waits for memory once, not once per row.
+template <int R, int C>
+__device__ __forceinline__ void candidate_cells(int (&cell)[C], const SelectArgs& g, const int kp, const int lane) {
+#pragma unroll
+  for (int c = 0; c < C; ++c) cell[c] = -1;
+  // Measured per shape: with 4 or 8 keys and fewer than 8 cells per lane the plain loop, one load per row, is the faster
+  // one by 3-6 % of the kernel (32768 tokens, 256-512 keys per half, k = 32); everywhere else the lanes' loop is, by 1-6 %.
+  if constexpr (R > 2 && C < 8) {
+    for (int a = 0, start = 0; a < kp; ++a) {
+      const int cnt = g.row_cells[a];
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int b = c * kWave + lane - start;
+        cell[c] = (unsigned)b < (unsigned)cnt ? (a << 8) | b : cell[c];
+      }
+      start += cnt;
+    }
+    return;
+  }
+  const int cnt_lo = lane < kp ? g.row_cells[lane] : 0;
+  const int cnt_hi = lane + kWave < kp ? g.row_cells[lane + kWave] : 0;
+  int start = 0;
+  for (int a = 0; a < min(kp, kWave); ++a) {
+    const int cnt = __builtin_amdgcn_readlane(cnt_lo, a);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int b = c * kWave + lane - start;
+      cell[c] = (unsigned)b < (unsigned)cnt ? (a << 8) | b : cell[c];
+    }
+    start += cnt;
+  }
+  for (int a = kWave; a < kp; ++a) {
+    const int cnt = __builtin_amdgcn_readlane(cnt_hi, a - kWave);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int b = c * kWave + lane - start;
+      cell[c] = (unsigned)b < (unsigned)cnt ? (a << 8) | b : cell[c];
+    }
+    start += cnt;
+  }
+}
+
+// ---- 16-bit scores: (score, payload) packed into one ordered 32-bit key ---------------------
+// key = order-preserving image of the 16-bit score << 16 | (0xFFFF - payload): a larger key goes
+// first, equal scores resolve to the lower payload, and a compare-exchange is one max / min.
+// Four times fewer VALU instructions than the (float, int) pairs the fp32 path needs.
+__device__ __forceinline__ uint32_t ord16(uint32_t bits) { return bits ^ ((bits & 0x8000u) ? 0xFFFFu : 0x8000u); }
+__device__ __forceinline__ uint32_t unord16(uint32_t u) { return u ^ ((u & 0x8000u) ? 0x8000u : 0xFFFFu); }
+__device__ __forceinline__ uint32_t make_key(float v, int payload, int dt) {      // v is representable in dt
+  v += 0.0f;                                                                      // -0 -> +0: they compare equal as floats
+  const uint32_t bits = dt == kBF16 ? (uint32_t)f32_to_bf16_bits(v) : (uint32_t)f32_to_f16_bits(v);
+  return (ord16(bits) << 16) | (0xFFFFu - (uint32_t)payload);
+}
+__device__ __forceinline__ float key_score(uint32_t key, int dt) {
+  const uint32_t bits = unord16(key >> 16);
+  return dt == kBF16 ? bf16_bits_to_f32((uint16_t)bits) : f16_bits_to_f32((uint16_t)bits);
+}
+__device__ __forceinline__ int key_payload(uint32_t key) { return (int)(0xFFFFu - (key & 0xFFFFu)); }
+
+template <int R, int SIZE, int STRIDE>
+__device__ __forceinline__ void kstage_ct(uint32_t (&k)[R], const int lane) {
+#pragma unroll
+  for (int a = 0; a < R; ++a) {
+    const uint32_t o = (uint32_t)xor_lane_i<STRIDE>((int)k[a], lane);
+    const bool up = (((a * kWave) | lane) & SIZE) == 0, lower = (lane & STRIDE) == 0;
+    k[a] = (lower == up) ? max(k[a], o) : min(k[a], o);
+  }
+}
+template <int R>
+__device__ __forceinline__ void kstage_rt(uint32_t (&k)[R], const int lane, const int size, const int stride) {
+#pragma unroll
+  for (int a = 0; a < R; ++a) {
+    const uint32_t o = (uint32_t)__shfl_xor((int)k[a], stride, kWave);
+    const bool up = (((a * kWave) | lane) & size) == 0, lower = (lane & stride) == 0;
+    k[a] = (lower == up) ? max(k[a], o) : min(k[a], o);
+  }
+}
+template <int R, int SIZE, int RS>
+__device__ __forceinline__ void kreg_stages(uint32_t (&k)[R]) {
+  if constexpr (RS >= 1) {
+#pragma unroll
+    for (int a = 0; a < R; ++a) {
+      if ((a & RS) == 0) {
+        const int b = a | RS;
+        const bool up = ((a * kWave) & SIZE) == 0;
+        const uint32_t hi = max(k[a], k[b]), lo = min(k[a], k[b]);
+        k[a] = up ? hi : lo;
+        k[b] = up ? lo : hi;
+      }
+    }
+    kreg_stages<R, SIZE, RS / 2>(k);
+  }
+}
+// lane distances STRIDE..1 of the merge for block size SIZE, on one or two lists
+template <int R, int SIZE, int STRIDE>
+__device__ __forceinline__ void kstages_ct(uint32_t (&k0)[R], uint32_t (&k1)[R], const int lane, const bool two) {
+  if constexpr (STRIDE >= 1) {
+    kstage_ct<R, SIZE, STRIDE>(k0, lane);
+    if (two) kstage_ct<R, SIZE, STRIDE>(k1, lane);
+    kstages_ct<R, SIZE, STRIDE / 2>(k0, k1, lane, two);
+  }
+}
+template <int R, int SIZE>
+__device__ __forceinline__ void ksizes(uint32_t (&k0)[R], uint32_t (&k1)[R], const int lane, const bool two) {
+  if constexpr (SIZE <= kWave * R) {
+    if constexpr (SIZE > kWave) {
+      kreg_stages<R, SIZE, SIZE / (2 * kWave)>(k0);
+      if (two) kreg_stages<R, SIZE, SIZE / (2 * kWave)>(k1);
+    }
+    constexpr int kFirst = SIZE > kWave ? kWave / 2 : SIZE / 2;
+    if constexpr (R <= kUnrollMaxR) {
+      kstages_ct<R, SIZE, kFirst>(k0, k1, lane, two);
+    } else {
+#pragma nounroll
+      for (int stride = kFirst; stride >= 1; stride >>= 1) {
+        kstage_rt<R>(k0, lane, SIZE, stride);
+        if (two) kstage_rt<R>(k1, lane, SIZE, stride);
+      }
+    }
+    ksizes<R, SIZE * 2>(k0, k1, lane, two);
+  }
+}
+// sorts the 64*R keys of each list descending (item e = reg*64 + lane)
+template <int R> __device__ __forceinline__ void ksort(uint32_t (&k)[R], const int lane) { ksizes<R, 2>(k, k, lane, false); }
+template <int R> __device__ __forceinline__ void ksort2(uint32_t (&k0)[R], uint32_t (&k1)[R], const int lane) { ksizes<R, 2>(k0, k1, lane, true); }
+
+// The 64 largest keys of each list (64*R keys, item = reg*64 + lane), descending, into register 0 -- all that the
+// candidate stage reads when k' <= 64.  Every register is sorted across the lanes by itself (compile-time lane
+// distances, no LDS), then the registers are merged pairwise: for two descending runs A and B, max(A[i], B[63-i])
+// holds the 64 largest of both as a bitonic sequence, which six more compare-exchange steps put in order.  About a
+// third of the compare-exchanges of a full sort of 512 keys, and none of them through run-time lane distances.
+template <int R>
+__device__ __forceinline__ void ktop64_2(uint32_t (&k0)[R], uint32_t (&k1)[R], const int lane) {
+#pragma unroll
+  for (int a = 0; a < R; ++a) {
+    uint32_t x[1] = {k0[a]}, y[1] = {k1[a]};
+    ksizes<1, 2>(x, y, lane, true);
+    k0[a] = x[0];
+    k1[a] = y[0];
+  }
+#pragma unroll
+  for (int width = R; width > 1; width /= 2) {
+#pragma unroll
+    for (int a = 0; a < width / 2; ++a) {
+      uint32_t x[1] = {max(k0[a], (uint32_t)__shfl((int)k0[a + width / 2], 63 - lane, kWave))};
+      uint32_t y[1] = {max(k1[a], (uint32_t)__shfl((int)k1[a + width / 2], 63 - lane, kWave))};
+      kstages_ct<1, kWave, kWave / 2>(x, y, lane, true);
+      k0[a] = x[0];
+      k1[a] = y[0];
+    }
+  }
+}
+
+template <int R>
+__device__ __forceinline__ uint32_t sorted_key(const uint32_t (&v)[R], int i) {
+  uint32_t r0 = (uint32_t)__shfl((int)v[0], i & 63, kWave);
+  if constexpr (R >= 2) {
+    const uint32_t r1 = (uint32_t)__shfl((int)v[1], i & 63, kWave);
+    r0 = (i >= kWave) ? r1 : r0;
+  }
+  return r0;
+}
+
+// Same selection as router_select_kernel for bf16 / f16 storage, on packed keys: the tokens of wave `wave` of `num_waves`.
+template <int R, int C>
+__device__ __forceinline__ void select_packed(const SelectArgs& g, const int wave, const int num_waves) {
+  const int lane = lane_id();
+  const int r = g.r, k = g.k, kp = g.kp, dt = g.dt;
+
+  float rx[R], ry[R];                             // as in router_select_kernel
+  auto load_raw = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < R; ++a) {
+      const int key = a * kWave + lane;
+      const bool ok = key < r;
+      rx[a] = ok ? load_score(g.lx, int64_t(t) * g.row_stride + key, dt) : kNegInf;
+      ry[a] = ok ? load_score(g.ly, int64_t(t) * g.row_stride + key, dt) : kNegInf;
+    }
+  };
+  constexpr bool kPrefetch = R <= 2;              // beyond that the extra live registers cost a wave per SIMD
+  if (kPrefetch && wave < g.num_tokens) load_raw(wave);
+  int cell[C];
+  candidate_cells<R, C>(cell, g, kp, lane);
+
+  for (int t = wave; t < g.num_tokens; t += num_waves) {
+    float sx[R], sy[R];
+#pragma unroll
+    for (int a = 0; a < R; ++a) {
+      const int key = a * kWave + lane;
+      const bool ok = key < r;
+      sx[a] = kPrefetch ? rx[a] : ok ? load_score(g.lx, int64_t(t) * g.row_stride + key, dt) : kNegInf;
+      sy[a] = kPrefetch ? ry[a] : ok ? load_score(g.ly, int64_t(t) * g.row_stride + key, dt) : kNegInf;
+    }
+    if (kPrefetch && t + num_waves < g.num_tokens) load_raw(t + num_waves);
+    if (g.stats || g.run_mean[0]) {
+      normalise_half<R>(sx, g, 0, r, lane, dt);
+      normalise_half<R>(sy, g, 1, r, lane, dt);
+    }
+    uint32_t kx[R], ky[R];
+#pragma unroll
+    for (int a = 0; a < R; ++a) {
+      const int key = a * kWave + lane;
+      kx[a] = key < r ? make_key(sx[a], key, dt) : 0u;          // 0 sorts behind every real key
+      ky[a] = key < r ? make_key(sy[a], key, dt) : 0u;
+    }
+    if (R > kUnrollMaxR && kp <= kWave) ktop64_2<R>(kx, ky, lane);    // uniform: kp comes with the arguments
+    else ksort2<R>(kx, ky, lane);
+
+    uint32_t ck[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const bool ok = cell[c] >= 0;
+      const int a = ok ? (cell[c] >> 8) : 0, b = ok ? (cell[c] & 255) : 0;
+      const float va = key_score(sorted_key<R>(kx, a), dt), vb = key_score(sorted_key<R>(ky, b), dt);
+      ck[c] = ok ? make_key(round_score(va + vb, dt), cell[c], dt) : 0u;
+    }
+    ksort<C>(ck, lane);
+
+    constexpr int kOut = (C >= 2) ? 2 : 1;          // k <= 128 -> winners live in regs 0..1
+#pragma unroll
+    for (int c = 0; c < kOut; ++c) {
+      const int j = c * kWave + lane;
+      const bool ok = j < k;
+      const int pl = ok ? key_payload(ck[c]) : 0;
+      const int ia = key_payload(sorted_key<R>(kx, pl >> 8)), ib = key_payload(sorted_key<R>(ky, pl & 255));
+      if (ok) {
+        const int64_t o = int64_t(t) * k + j;
+        const float sc = key_score(ck[c], dt);
+        if (g.scores) store_score(g.scores, o, sc, dt);
+        if (g.gates) store_score(g.gates, o, expf(sc), dt);         // gate = P(x key) * P(y key)
+        g.indices[o] = ia * r + ib;
+      }
+    }
+  }
+}
+
+static inline int num_cells(int k, int kp) {
+  int n = 0;
+  for (int a = 0; a < kp; ++a) n += (kp < k / (a + 1)) ? kp : k / (a + 1);
+  return n;
+}
+
+// What select_packed and its kernels want filled in beside the caller's fields; returns the candidate cells per lane
+static inline int prepare_select(SelectArgs& g) {
+  g.kp = g.r < g.k ? g.r : g.k;
+  for (int a = 0; a < 128; ++a) g.row_cells[a] = a < g.kp ? (uint8_t)(g.kp < g.k / (a + 1) ? g.kp : g.k / (a + 1)) : 0;
+  return (num_cells(g.k, g.kp) + kWave - 1) / kWave;            // <= 11 for k <= 128
+}
+
+}  // namespace omni

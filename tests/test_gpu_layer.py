@@ -551,3 +551,53 @@ def test_layer_tiny_token_counts(T, training, device):
         outs.append(layer(x.to(device)))
     torch.testing.assert_close(outs[0].cpu().float(), want.float(), rtol=2e-2, atol=2e-2)
     assert torch.equal(outs[0], outs[1])
+
+
+# T, H, I, N, k: tiles of 16 rows and their remainders; hidden and intermediate sizes that end inside a block's 64 of K or 16 columns, or
+# split K eight ways; 1 to 8 keys per lane, an odd key count, more than 64 candidates, ids beyond the square never chosen
+FEW_TOKEN_CASES = [(1, 1024, 4096, 4096, 16), (16, 200, 312, 1000, 8), (17, 1032, 2056, 700, 32), (33, 256, 1024, 90000, 18), (48, 2048, 1024, 17000, 4),
+                   (49, 4096, 512, 260, 2), (63, 584, 8, 289, 6), (64, 8, 4096, 300000, 32)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", FEW_TOKEN_CASES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
+def test_few_tokens_match_the_operators(case, dtype, device):
+    """At most 64 tokens in eval mode: the joint launches against the router, expert and MLP operators one by one (64-bit MLP), on
+    finite data with a non-finite table row that nobody selects.  Tolerance: one rounding of the storage type per stored value (h, the
+    MLP's and the experts' sums, the total), on the output's scale."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, H, I, N, k = case
+    print(f"few tokens {case} {dtype}", flush=True)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", N, k)).to(device=device, dtype=dtype).eval()
+    g = torch.Generator(device=device).manual_seed(T)
+    for p in layer.parameters():
+        p.normal_(0.0, H ** -0.5, generator=g)
+    layer.down_proj.weight.normal_(0.0, I ** -0.5, generator=g)
+    for norm in (layer.router_norm_x, layer.router_norm_y):
+        norm.running_mean.normal_(0.0, 0.3, generator=g)
+        norm.running_var.uniform_(0.5, 2.0, generator=g)
+    x = torch.randn(1, T, H, device=device, generator=g).to(dtype)
+    gates, ids = layer.route(x[0])
+    unused = torch.ones(N, dtype=torch.bool, device=device)
+    unused[ids.long().flatten()] = False
+    if unused.any():
+        row = int(unused.nonzero()[0])
+        layer.up_embed.weight[row] = float("nan")
+        layer.down_embed.weight[row] = float("inf")
+    got = layer(x)[0]
+    ops = _ops()
+    experts = ops.hip_omni_expert_func(x[0], layer.up_embed.weight, layer.down_embed.weight, gates, ids).double()
+    xd, wg, wu, wd = (t.double() for t in (x[0], layer.gate_proj.weight, layer.up_proj.weight, layer.down_proj.weight))
+    h = (torch.nn.functional.silu((xd @ wg.t()).to(dtype).double()) * (xd @ wu.t()).to(dtype).double()).to(dtype).double()
+    mlp = h @ wd.t()
+    eps = torch.finfo(dtype).eps
+    scale = max(1.0, float((mlp + experts).abs().max()))
+    assert (got.double() - (mlp + experts)).abs().max().item() <= 4 * eps * scale
+    # the MLP operator takes the same launches, with and without a residual
+    alone = ops.hip_omni_mlp_func(x[0], layer.gate_proj.weight, layer.up_proj.weight, layer.down_proj.weight)
+    assert (alone.double() - mlp).abs().max().item() <= 4 * eps * scale
+    both = ops.hip_omni_mlp_func(x[0], layer.gate_proj.weight, layer.up_proj.weight, layer.down_proj.weight, residual=x[0])
+    assert torch.equal(both, (alone.float() + x[0].float()).to(dtype))
+    # ids and gates are those of the router operator: the expert term alone (a zero down projection)
+    layer.down_proj.weight.zero_()
+    assert (layer(x)[0].double() - experts).abs().max().item() <= 4 * eps * max(1.0, float(experts.abs().max()))
