@@ -29,6 +29,8 @@ bool few_tokens_covers(int64_t T, int64_t H, int64_t I, int dtype);
 // ... and with a router of r keys per half and top-k, eval-mode BatchNorm, the gather algorithm's rows
 bool few_tokens_covers_layer(int64_t T, int64_t H, int64_t I, int r, int k, int dtype);
 size_t few_tokens_parts_bytes(int64_t T, int64_t H, int64_t I);
+// rows are fetched 16 bytes at a time: every pointer of `f` (NULL counts as aligned) is
+bool few_tokens_aligned(const FewTokens& f);
 hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s);
 
 }  // namespace omni

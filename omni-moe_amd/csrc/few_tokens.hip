@@ -374,6 +374,11 @@ bool few_tokens_covers_layer(int64_t T, int64_t H, int64_t I, int r, int k, int 
   // keys and candidates that the joint launch has registers for; rows that a block holds its waves' sums of
   return few_tokens_covers(T, H, I, dtype) && H <= 4096 && r <= 8 * kWave && k > 0 && num_cells(k, r < k ? r : k) <= 2 * kWave;
 }
+bool few_tokens_aligned(const FewTokens& f) {
+  for (const void* q : {f.x, f.wg, f.wu, f.wd, (const void*)f.h, (const void*)f.y, (const void*)f.parts, f.residual, f.wx, f.wy, (const void*)f.z, f.up, f.down})
+    if ((uintptr_t)q % 16) return false;
+  return true;
+}
 size_t few_tokens_parts_bytes(int64_t T, int64_t H, int64_t I) { return (size_t)few_splits(H, I) * (size_t)T * (size_t)H * 4; }
 
 hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s) {

@@ -959,8 +959,10 @@ extern "C" OMNI_API int32_t omni_mlp_fwd(const void* x, const void* gate_weight,
   if (few_tokens_covers(num_tokens, hidden_size, intermediate_size, dtype)) {
     const FewTokens f{x, gate_weight, up_weight, down_weight, workspace, y, (float*)((char*)workspace + mlp_h_bytes(num_tokens, intermediate_size, dtype)), residual,
                       (int)num_tokens, hidden_size, intermediate_size};
-    const hipError_t he = launch_few_tokens(dtype, f, (hipStream_t)stream);
-    return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
+    if (few_tokens_aligned(f)) {
+      const hipError_t he = launch_few_tokens(dtype, f, (hipStream_t)stream);
+      return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
+    }
   }
   if ((e = mlp_gate_up_impl(x, gate_weight, up_weight, num_tokens, hidden_size, intermediate_size, dtype, workspace, stream, true))) return e;
   return mlp_down_impl(down_weight, residual, y, num_tokens, hidden_size, intermediate_size, dtype, workspace, stream, true);

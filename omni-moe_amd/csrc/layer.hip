@@ -112,8 +112,10 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
     g.gates = gates; g.indices = ids;
     g.num_tokens = (int)num_tokens; g.r = num_expert_sqrt; g.k = num_experts_per_token; g.dt = dtype;
     f.up = up_embed; f.down = down_embed; f.N = num_experts;
-    const hipError_t he = launch_few_tokens(dtype, f, main_s);
-    return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
+    if (few_tokens_aligned(f)) {
+      const hipError_t he = launch_few_tokens(dtype, f, main_s);
+      return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
+    }
   }
   hipStream_t branch = side_stream ? (hipStream_t)side_stream : main_s;
   hipError_t he;
