@@ -2,8 +2,8 @@
 //
 // Replaces get_scheduling_info's tail part (omni_moe/ops/triton/omni_scheduler.py:48-101),
 // which runs ~12 torch launches including a radix sort and reads two results back to
-// the host (:82, :90).  Here the pairs are sorted by expert id with one counting pass when
-// N <= 4096 (one bin per expert), two passes (low then high half of the id bits) above that.
+// the host (:82, :90).  Here the pairs are sorted by expert id with one counting pass (one bin per
+// expert) when N <= 4096, or N <= 16384 with few pairs, and two passes (low then high half of the id bits) above that.
 // A pass is two kernels:
 //   count:   every block counts the bins of its contiguous tile of the input in LDS and writes
 //            them as one row of hist[tile][bin] (16-bit counters: a tile has fewer than 65536
@@ -33,8 +33,9 @@ constexpr int kSortThreads = 512;
 constexpr int kSortWaves = kSortThreads / kWave;
 constexpr int kSlices = 8;                                // bin slices = XCDs
 constexpr int kMaxBins = 4097;                            // 4096 experts (or id slices) + 1 bin for ids outside [0, N)
+constexpr int kMaxBinsWide = 16385;                       // ... of a single pass over few pairs: what a block's tables leave room for in LDS
 constexpr int kBinChunk = 8;                              // bins per 16-byte load of a histogram row
-constexpr int kMaxWidth = ((kMaxBins + kSlices - 1) / kSlices + kBinChunk - 1) / kBinChunk * kBinChunk;   // bins per slice: 520
+constexpr int slice_width(int bins) { return ((bins + kSlices - 1) / kSlices + kBinChunk - 1) / kBinChunk * kBinChunk; }   // bins per slice
 constexpr int kMaxSortTiles = 1024;
 constexpr int kMaxTile = 63 * 1024;                       // counters are 16 bits wide
 constexpr int kRowBatch = 8;                              // histogram rows a thread has in flight
@@ -51,7 +52,7 @@ struct SortPass {
   uint16_t* hist;           // [tiles][stride] bin counts of every tile
   uint32_t* slice_tot;      // [tiles][8] the same counts summed over each slice
   int64_t num_pairs;
-  int tile;                 // pairs per tile, a multiple of 1024
+  int tile;                 // pairs per tile, a multiple of 512
   int tiles, bins;
   int width, stride;        // bins per slice (a multiple of 8); stride = 8 * width >= bins
   int shift;                // digit = id >> shift ...
@@ -107,8 +108,9 @@ __global__ __launch_bounds__(kSortThreads) void sort_count_kernel(const SortPass
 }
 
 __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(const SortPass a) {
-  __shared__ int32_t tbl[kSortWaves][kMaxWidth];         // per wave and bin: count, then running output position
-  __shared__ int32_t bin_base[kMaxWidth], before_s[kMaxWidth], total_s[kMaxWidth];
+  extern __shared__ int32_t tables[];
+  int32_t* tbl = tables;                                 // [wave][width]: per wave and bin: count, then running output position
+  int32_t *bin_base = tbl + kSortWaves * a.width, *before_s = bin_base + a.width, *total_s = before_s + a.width;
   __shared__ int32_t below_s;                            // pairs in the slices below this one, all tiles
   const int lane = lane_id(), wave = threadIdx.x >> 6;
   const int tile_idx = (int)blockIdx.x / kSlices, slice = (int)blockIdx.x % kSlices;
@@ -127,7 +129,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(const SortPa
   };
   u32x4_t early[kRowBatch];
   load_rows(early, group);
-  for (int d = threadIdx.x; d < kSortWaves * kMaxWidth; d += kSortThreads) (&tbl[0][0])[d] = 0;
+  for (int d = threadIdx.x; d < kSortWaves * a.width; d += kSortThreads) tbl[d] = 0;
   for (int d = threadIdx.x; d < a.width; d += kSortThreads) bin_base[d] = before_s[d] = total_s[d] = 0;
   if (threadIdx.x == 0) below_s = 0;
   __syncthreads();
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(const SortPa
   const int per_wave = a.tile / kSortWaves;
   const int64_t w0 = t0 + (int64_t)wave * per_wave < t1 ? t0 + (int64_t)wave * per_wave : t1;   // this wave's eighth, in order
   const int64_t w1 = w0 + per_wave < t1 ? w0 + per_wave : t1;
-  int32_t* mine = tbl[wave];
+  int32_t* mine = tbl + wave * a.width;
   for (int64_t g0 = w0; g0 < w1; g0 += kGroup * kWave) {
     int32_t key[kGroup];
 #pragma unroll
@@ -222,8 +224,8 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(const SortPa
     int32_t base = bin_base[d];
 #pragma unroll
     for (int w = 0; w < kSortWaves; ++w) {
-      const int32_t c = tbl[w][d];
-      tbl[w][d] = base;
+      const int32_t c = tbl[w * a.width + d];
+      tbl[w * a.width + d] = base;
       base += c;
     }
   }
@@ -294,6 +296,12 @@ static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; 
 
 static inline int ceil_log2(uint64_t v) { int b = 0; while ((1ull << b) < v) ++b; return b; }
 
+// The two kernels' tables in LDS
+static inline int count_lds(int stride) { return stride * 4; }
+static inline int scatter_lds(int width) { return (kSortWaves + 3) * width * 4; }
+static LdsKernel g_count_kernel{(const void*)sort_count_kernel, slice_width(kMaxBinsWide) * kSlices * 4};
+static LdsKernel g_scatter_kernel{(const void*)sort_scatter_kernel, (kSortWaves + 3) * slice_width(kMaxBinsWide) * 4};
+
 // How the sort of P pairs with ids below N is split into passes and tiles.
 struct SortPlan {
   int passes, lo_bits, bins[2], width, stride, tile, tiles;
@@ -301,21 +309,29 @@ struct SortPlan {
 };
 static bool make_plan(int64_t P, int64_t N, SortPlan* pl) {
   const int kb = ceil_log2((uint64_t)N);
-  if (N + 1 <= kMaxBins) { pl->passes = 1; pl->lo_bits = 0; pl->bins[0] = (int)N + 1; pl->bins[1] = 0; }
+  // A wave places an eighth of a tile, 64 items a step: tiles of 8192 pairs are 16 steps; at most 256 tiles (a scatter
+  // block sums its slice of every tile's row), more only where a tile would outgrow its 16-bit counters
+  int64_t tile = 8192;
+  if ((P + tile - 1) / tile > 256) tile = ((P + 255) / 256 + 1023) / 1024 * 1024;
+  if (tile > kMaxTile) tile = kMaxTile;
+  // What the scatter blocks of n tiles read of the histogram in all: n rows each, one block per tile and slice.
+  auto rows_read = [&](int64_t of_tile, int64_t bins) { const int64_t n = (P + of_tile - 1) / of_tile; return n * n * slice_width((int)bins) * kSlices * 2; };
+  // A second pass and the offsets kernel behind it cost about 20 us, as do 64 MB of rows: 32768 pairs over 16384 experts 37 us in two
+  // passes, 21 in one.
+  const bool wide = N + 1 > kMaxBins && N + 1 <= kMaxBinsWide && rows_read(tile, N + 1) <= (64ll << 20);
+  if (N + 1 <= kMaxBins || wide) { pl->passes = 1; pl->lo_bits = 0; pl->bins[0] = (int)N + 1; pl->bins[1] = 0; }
   else {
     pl->passes = 2; pl->lo_bits = kb / 2;
     pl->bins[0] = 1 << pl->lo_bits;
     pl->bins[1] = (int)((N + (1ll << pl->lo_bits) - 1) >> pl->lo_bits) + 1;
   }
   const int maxb = pl->bins[0] > pl->bins[1] ? pl->bins[0] : pl->bins[1];
-  if (maxb > kMaxBins) return false;                       // N > 16 Mi experts
-  pl->width = ((maxb + kSlices - 1) / kSlices + kBinChunk - 1) / kBinChunk * kBinChunk;
+  if (maxb > (wide ? kMaxBinsWide : kMaxBins)) return false;                       // N > 16 Mi experts
+  pl->width = slice_width(maxb);
   pl->stride = pl->width * kSlices;
-  // a wave places an eighth of a tile, 64 items a step: tiles of 8192 pairs are 16 steps; at most 256 tiles (a scatter
-  // block sums its slice of every tile's row), more only where a tile would outgrow its 16-bit counters
-  int64_t tile = 8192;
-  if ((P + tile - 1) / tile > 256) tile = ((P + 255) / 256 + 1023) / 1024 * 1024;
-  if (tile > kMaxTile) tile = kMaxTile;
+  // Few pairs: smaller tiles, for more blocks with fewer steps each, while the rows stay cheap to read (65536 pairs over 4096 experts:
+  // scatter 11.5 -> 8.5 us)
+  while (tile > 2048 && tile <= 8192 && rows_read(tile / 2, maxb) <= (16ll << 20)) tile /= 2;
   if ((P + tile - 1) / tile > kMaxSortTiles) return false;   // more than 64 Mi pairs
   pl->tile = (int)tile;
   pl->tiles = (int)((P + tile - 1) / tile);
@@ -355,6 +371,10 @@ extern "C" OMNI_API int32_t omni_schedule(const int32_t* indices, int32_t* offse
   int32_t* vals_a = (int32_t*)w;
 
   const bool single = pl.passes == 1;
+  if (count_lds(pl.stride) > 65536 || scatter_lds(pl.width) > 65536) {
+    if (hipError_t e = g_count_kernel.ensure(); e != hipSuccess) return OMNI_ERR_HIP_BASE + (int)e;
+    if (hipError_t e = g_scatter_kernel.ensure(); e != hipSuccess) return OMNI_ERR_HIP_BASE + (int)e;
+  }
   if (single || P > 0) {
     for (int pass = 0; pass < pl.passes; ++pass) {
       const bool last = pass == pl.passes - 1;
@@ -380,8 +400,8 @@ extern "C" OMNI_API int32_t omni_schedule(const int32_t* indices, int32_t* offse
       a.inv_shift = 30;
       while ((1ll << (a.inv_shift - 30)) < (int64_t)num_experts_per_token) ++a.inv_shift;
       a.inv_top_k = num_experts_per_token > 0 ? ((1ull << a.inv_shift) + num_experts_per_token - 1) / (uint64_t)num_experts_per_token : 0;
-      hipLaunchKernelGGL(sort_count_kernel, dim3(a.tiles), dim3(kSortThreads), (size_t)a.stride * 4, s, a);
-      hipLaunchKernelGGL(sort_scatter_kernel, dim3(a.tiles * kSlices), dim3(kSortThreads), 0, s, a);
+      hipLaunchKernelGGL(sort_count_kernel, dim3(a.tiles), dim3(kSortThreads), count_lds(a.stride), s, a);
+      hipLaunchKernelGGL(sort_scatter_kernel, dim3(a.tiles * kSlices), dim3(kSortThreads), scatter_lds(a.width), s, a);
     }
   }
   if (!single) {

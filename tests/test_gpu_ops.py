@@ -97,7 +97,10 @@ SCHED_CASES = [(512, 8, 1024, "uniform"), (4096, 16, 4096, "uniform"), (16384, 1
                (4096, 32, 262144, "zipf"), (1000, 6, 5000, "zipf"), (3, 2, 7, "uniform"), (2048, 16, 64, "hot"),
                (32768, 32, 262144, "zipf"), (777, 10, 1048576, "uniform"), (100, 4, 1, "hot"), (5000, 8, 4097, "uniform"),
                # more than 256 tiles of 8192 pairs (tiles grow), and tiles at their 16-bit limit with every pair in one bin
-               (150000, 16, 4096, "uniform"), (1100000, 16, 4096, "hot")]
+               (150000, 16, 4096, "uniform"), (1100000, 16, 4096, "hot"),
+               # one wide pass: just above the narrow one, at its last bin, its tiles of 2048 and 4096 pairs; and just past it in bins and in pairs
+               (64, 2, 4096, "uniform"), (1024, 32, 16384, "uniform"), (2051, 30, 16384, "zipf"), (1024, 32, 16385, "uniform"), (30000, 16, 16000, "uniform"),
+               (9001, 4, 12000, "hot")]
 
 
 def _sched_ids(T, k, N, kind, seed):
