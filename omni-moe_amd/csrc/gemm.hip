@@ -728,6 +728,92 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_ksplit_kernel(const Gemm
   gemm_epilogue<DT, 1, 1, EPI>(g, sum, m0, n0, wave & 1, wave >> 1, lane);
 }
 
+// ---- single precision with few output tiles -----------------------------------------------------------
+// What bounds it: v_mfma_f32_32x32x2 takes 64 cycles, so a CU that has a 128 x 128 tile to itself works 4096 cycles on 32 of K, and a launch
+// of 32 or 64 such tiles leaves the chip idle (512 tokens, hidden 256 x intermediate 1024: gate/up 22.4 us, down projection 26.8 us on 64 x 64
+// tiles, for 4 and 2 us of matrix instructions).  Here a block has 32 x 32 of the output (SwiGLU: of gate and of up) and its four waves deal
+// out the K tiles (32 values, 128-byte rows) as in gemm_ksplit_kernel: a two-stage ring in LDS per wave, no block barrier, the four sums added in
+// wave order: 12.4 and 9.1 us.  Twice the operand traffic of a 64 x 64 tile (32 bytes per cycle and CU), which L2 still carries.
+template <int EPI>
+__global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_small_kernel(const GemmArgs g) {
+  constexpr int TB = EPI == kEpiSwiglu ? 2 : 1, kTile = 32 * 128, kStage = (1 + TB) * kTile, kLoads = 4 * (1 + TB);
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = (int)(blockIdx.x % g.tiles_m) * 32, n0 = (int)(blockIdx.x / g.tiles_m) * 32;
+  const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * 2 * kStage;
+  const int row_bytes = g.K * 4;
+  const uint64_t a = (uint64_t)g.a + (uint64_t)m0 * (uint32_t)row_bytes;
+  const int a_bytes = min(32, g.M - m0) * row_bytes, b_bytes = min(32, g.N - n0) * row_bytes;    // rows past the matrix read as zero
+  // a second matrix: the up weights, or the upper half of the columns (whole blocks of it)
+  uint64_t b[2] = {(uint64_t)g.b0 + (uint64_t)n0 * (uint32_t)row_bytes, 0};
+  if constexpr (EPI == kEpiSwiglu) b[1] = (uint64_t)g.b1 + (uint64_t)n0 * (uint32_t)row_bytes;
+  else if (g.b1 && n0 >= g.N / 2) b[0] = (uint64_t)g.b1 + (uint64_t)(n0 - g.N / 2) * (uint32_t)row_bytes;
+  auto issue = [&](int kt, int stage) __attribute__((always_inline)) {
+    auto one = [&](auto n_tag) __attribute__((always_inline)) {
+      constexpr int n = decltype(n_tag)::value, operand = n / 4, part = n % 4;
+      const int row = part * 8 + (lane >> 3), k = kt * 32 + swizzle<64>(row, lane & 7) * 4;      // position c of a row holds its piece swizzle(c)
+      load_to_lds<n * 1024>(operand == 0 ? a : b[operand == 2], operand == 0 ? a_bytes : b_bytes, ring + (uint32_t)(stage * kStage),
+                            k < g.K ? (uint32_t)(row * row_bytes + k * 4) : 0x80000000u, 0);
+    };
+    auto all = [&](auto... n) __attribute__((always_inline)) { (one(n), ...); };
+    with_sequence(all, std::make_integer_sequence<int, kLoads>{});
+  };
+  f32x16_t acc[TB];
+#pragma unroll
+  for (int j = 0; j < TB; ++j)
+#pragma unroll
+    for (int q = 0; q < 16; ++q) acc[j][q] = 0.f;
+
+  const int rl = lane & 31, num_kt = (g.K + 31) / 32, mine = (num_kt - wave + 3) / 4;
+  if (mine > 0) issue(wave, 0);
+  if (mine > 1) issue(wave + 4, 1);
+  for (int t = 0; t < mine; ++t) {
+    if (t + 1 < mine) wait_vmcnt<kLoads>(); else wait_vmcnt<0>();
+    const uint32_t st = ring + (uint32_t)((t & 1) * kStage + rl * 128);
+    using Frag = const __attribute__((address_space(3))) u32x4_t*;
+    u32x4_t af[4], bf[4][TB];
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl) {
+      const uint32_t at = st + (uint32_t)swizzle<64>(rl, 2 * sl + (lane >> 5)) * 16;
+      af[sl] = *(Frag)(uintptr_t)at;
+#pragma unroll
+      for (int j = 0; j < TB; ++j) bf[sl][j] = *(Frag)(uintptr_t)(at + (1 + j) * kTile);
+    }
+    if (t + 2 < mine) {
+      wait_lds_reads();                                  // the stage is read out (by this wave, its only reader)
+      issue(wave + 4 * (t + 2), t & 1);
+    }
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl)
+#pragma unroll
+      for (int j = 0; j < TB; ++j) acc[j] = mfma32<kF32>(bf[sl][j], af[sl], acc[j]);
+  }
+
+  __syncthreads();                                       // every wave is done with its ring
+  f32x4_t* xch = (f32x4_t*)lds;
+#pragma unroll
+  for (int j = 0; j < TB; ++j)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4)
+      xch[((wave * TB + j) * 4 + q4) * 64 + lane] = f32x4_t{acc[j][q4 * 4], acc[j][q4 * 4 + 1], acc[j][q4 * 4 + 2], acc[j][q4 * 4 + 3]};
+  __syncthreads();
+  if (wave != 0) return;
+  f32x16_t sum[1][TB];
+#pragma unroll
+  for (int j = 0; j < TB; ++j)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      f32x4_t v = xch[(j * 4 + q4) * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) {
+        const f32x4_t o = xch[((w * TB + j) * 4 + q4) * 64 + lane];
+        v[0] += o[0]; v[1] += o[1]; v[2] += o[2]; v[3] += o[3];
+      }
+      sum[0][j][q4 * 4] = v[0]; sum[0][j][q4 * 4 + 1] = v[1]; sum[0][j][q4 * 4 + 2] = v[2]; sum[0][j][q4 * 4 + 3] = v[3];
+    }
+  gemm_epilogue<kF32, 1, TB, EPI>(g, sum, m0, n0, 0, 0, lane);
+}
+
 // One list entry per kernel instantiation that launch_gemm can start (the static members come into being
 // at library load for every instantiation the dispatch below names).
 template <int DT, int TM, int TN, int EPI, int BK, int NS, int NW = 4>
@@ -737,6 +823,11 @@ struct DmaKernelLds {
 template <int DT, int EPI>
 struct KsplitKernelLds {
   static inline LdsKernel entry{(const void*)gemm_ksplit_kernel<DT, EPI>, 4 * 2 * 2 * 64 * 128};
+};
+template <int EPI>
+struct SmallF32Lds {
+  static constexpr int kBytes = 4 * 2 * (EPI == kEpiSwiglu ? 3 : 2) * 32 * 128;
+  static inline LdsKernel entry{(const void*)gemm_f32_small_kernel<EPI>, kBytes};
 };
 template <int DT, int TM, int TN, int EPI>
 struct StagedKernelLds {
@@ -786,6 +877,23 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
       static_assert(kDmaLds == kDmaStages * (2 * TM * 32 + 2 * TN * 32) * kDmaBK * 2, "list entry and launch disagree");
       if (hipError_t e = DmaKernelLds<DT, TM, TN, EPI, kDmaBK, kDmaStages>::entry.ensure(); e != hipSuccess) return e;
       hipLaunchKernelGGL(kern, dim3(blocks), dim3(kGemmThreads), kDmaLds, s, g);
+      return hipGetLastError();
+    }
+  }
+  if constexpr (DT == kF32 && EPI != kEpiGate) {
+    // Cycles of matrix instructions and of what goes round them, per round of 256 blocks: a TM x TN wave tile takes 1024 TM TN for 32 of K, plus
+    // about 900 with one block to a CU and 450 with more (64 x 64 tiles 1700 and 1490, 128 x 128 tiles 5400); a block of 32 x 32 deals the same K out
+    // over four waves.  1000 x 1024 x 4096: 106 us on 64 x 64 tiles, 88 us here; 2500 x 768 x 2304: 97 and 102 us.
+    constexpr int TB = EPI == kEpiSwiglu ? 2 : 1;
+    const int64_t kt = (g.K + 31) / 32, tiles_m = (g.M + 31) / 32, small = tiles_m * ((g.N + 31) / 32);
+    const int64_t tiled = (blocks + 255) / 256 * kt * (1024 * TM * TN + (blocks > 256 ? 450 : 900)), dealt = (small + 255) / 256 * ((kt + 3) / 4 * (1024 * TB + 450) + 2500);
+    const bool aligned = ((uintptr_t)g.a | (uintptr_t)g.b0 | (uintptr_t)g.b1) % 16 == 0;
+    if (dealt < tiled && aligned && small < INT32_MAX && (int64_t)g.K * 128 < INT32_MAX && (EPI == kEpiSwiglu || !g.b1 || g.N % 64 == 0)) {
+      GemmArgs d = g;
+      d.tiles_m = (int)tiles_m;
+      d.tiles_n = (g.N + 31) / 32;
+      if (hipError_t e = SmallF32Lds<EPI>::entry.ensure(); e != hipSuccess) return e;
+      hipLaunchKernelGGL((gemm_f32_small_kernel<EPI>), dim3((unsigned)small), dim3(kGemmThreads), SmallF32Lds<EPI>::kBytes, s, d);
       return hipGetLastError();
     }
   }

@@ -601,3 +601,29 @@ def test_few_tokens_match_the_operators(case, dtype, device):
     # ids and gates are those of the router operator: the expert term alone (a zero down projection)
     layer.down_proj.weight.zero_()
     assert (layer(x)[0].double() - experts).abs().max().item() <= 4 * eps * max(1.0, float(experts.abs().max()))
+
+
+# T, H, I: 32-row and 32-column tiles and their remainders, K of one to five tiles of 32 and with a remainder, more and fewer waves than K tiles
+@pytest.mark.parametrize("case", [(1, 4, 4), (33, 36, 100), (512, 256, 1024), (100, 1028, 68), (640, 160, 96), (65, 128, 132)], ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}")
+def test_small_fp32_products_match_fp64(case, device):
+    """Single precision with few output tiles: the MLP (SwiGLU and residual epilogues) and the router projection's column statistics against 64
+    bits.  Tolerance: sums of K products in 32 bits, sqrt(K) * 2^-24 of the terms' size each, times 8."""
+    T, H, I = case
+    print(f"small fp32 {case}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    x, res = torch.randn(T, H, generator=g), torch.randn(T, H, generator=g)
+    wg, wu, wd = torch.randn(I, H, generator=g) * H ** -0.5, torch.randn(I, H, generator=g) * H ** -0.5, torch.randn(H, I, generator=g) * I ** -0.5
+    want = oracle.mlp_forward(x.double(), wg.double(), wu.double(), wd.double())
+    got = _ops().hip_omni_mlp_func(*(t.to(device) for t in (x, wg, wu, wd)), residual=res.to(device)).cpu().double()
+    assert (got - (want + res.double())).abs().max().item() <= 8 * 2 ** -24 * (H ** 0.5 + I ** 0.5) * max(1.0, float(want.abs().max()))
+    if T == 1:
+        return
+    for r in (32, 30):                                       # the halves' weights begin and end with a block, or inside one
+        wx, wy = torch.randn(r, H, generator=g) * H ** -0.5, torch.randn(r, H, generator=g) * H ** -0.5
+        bufs = _bn_buffers(r, torch.float32, device) + _bn_buffers(r, torch.float32, device)
+        _ops().hip_omni_router_fwd_func(x.to(device), wx.to(device), wy.to(device), *bufs, 4, training=True, momentum=1.0)
+        z = x.double() @ torch.cat([wx, wy]).double().t()
+        mean = torch.cat([bufs[0], bufs[3]]).cpu().double()
+        var = torch.cat([bufs[1], bufs[4]]).cpu().double()
+        torch.testing.assert_close(mean, z.mean(0), rtol=1e-5, atol=8 * 2 ** -24 * H ** 0.5)
+        torch.testing.assert_close(var, z.var(0), rtol=1e-5, atol=8 * 2 ** -24 * H ** 0.5)
