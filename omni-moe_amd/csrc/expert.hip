@@ -34,11 +34,14 @@ constexpr int kTokensPerBlock = 4;   // one wave each
 
 // NCH = 16-byte chunks of a row per lane (row bytes / 1024, rounded up);
 // G   = experts fetched per batch (their 2*G*NCH loads are all in flight at once).
-template <int DT, int NCH, int G>
+// kAdd: the layer's final add as well: y holds the shared MLP's rounded rows (parts = NULL), or the K splits' fp32 sums of them are in
+// parts [splits][tokens][hidden]; both terms are rounded, then their sum.
+struct GatherAdd { const float* parts; int splits; };
+template <int DT, int NCH, int G, bool kAdd = false>
 __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kernel(
     const uint8_t* __restrict__ x, const uint8_t* __restrict__ up, const uint8_t* __restrict__ down,
     const void* __restrict__ gates, const int32_t* __restrict__ ids, uint8_t* __restrict__ y,
-    int num_tokens, int hidden, int top_k, uint32_t num_experts) {
+    int num_tokens, int hidden, int top_k, uint32_t num_experts, GatherAdd add) {
   constexpr int E = Row16<DT>::kElems;
   const int lane = lane_id();
   const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * kTokensPerBlock + (threadIdx.x >> 6));
@@ -108,7 +111,32 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
 
 #pragma unroll
   for (int c = 0; c < NCH; ++c)
-    if (live[c]) *(u32x4_t*)(y + t * row_bytes + off[c]) = pack16<DT>(acc[c]);
+    if (live[c]) {
+      u32x4_t out = pack16<DT>(acc[c]);
+      if constexpr (kAdd) {
+        float e[E], m[E];
+        unpack16<DT>(out, e);
+        if (add.parts) {
+#pragma unroll
+          for (int i = 0; i < E; ++i) m[i] = 0.f;
+          const float* at = add.parts + int64_t(t) * hidden + (c * kWave + lane) * E;
+          for (int s = 0; s < add.splits; ++s, at += int64_t(num_tokens) * hidden)
+#pragma unroll
+            for (int q = 0; q < E; q += 4) {
+              const f32x4_t p = *(const f32x4_t*)(at + q);
+#pragma unroll
+              for (int z = 0; z < 4; ++z) m[q + z] += p[z];
+            }
+          unpack16<DT>(pack16<DT>(m), m);
+        } else {
+          unpack16<DT>(*(const u32x4_t*)(y + t * row_bytes + off[c]), m);
+        }
+#pragma unroll
+        for (int i = 0; i < E; ++i) m[i] += e[i];
+        out = pack16<DT>(m);
+      }
+      *(u32x4_t*)(y + t * row_bytes + off[c]) = out;
+    }
 }
 
 template <int DT, int NCH, int G>
@@ -117,8 +145,27 @@ static hipError_t launch_gather(const void* x, const void* up, const void* down,
   if (T == 0) return hipSuccess;
   dim3 grid((unsigned)((T + kTokensPerBlock - 1) / kTokensPerBlock)), block(kTokensPerBlock * kWave);
   hipLaunchKernelGGL((expert_gather_kernel<DT, NCH, G>), grid, block, 0, s, (const uint8_t*)x, (const uint8_t*)up,
-                     (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N);
+                     (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{nullptr, 0});
   return hipGetLastError();
+}
+
+// The gather algorithm (rows of at most 8 KiB, 16-bit storage) with the layer's final add
+hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, int64_t T, int H,
+                             int k, int64_t N, int dtype, hipStream_t s) {
+  const dim3 grid((unsigned)((T + kTokensPerBlock - 1) / kTokensPerBlock)), block(kTokensPerBlock * kWave);
+  auto go = [&](auto dt, auto nch, auto batch) {
+    hipLaunchKernelGGL((expert_gather_kernel<decltype(dt)::value, decltype(nch)::value, decltype(batch)::value, true>), grid, block, 0, s, (const uint8_t*)x, (const uint8_t*)up,
+                       (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{parts, splits});
+    return hipGetLastError();
+  };
+  auto by_row = [&](auto dt) {
+    const int nch = (H + kWave * 8 - 1) / (kWave * 8);
+    if (nch <= 1) return go(dt, std::integral_constant<int, 1>{}, std::integral_constant<int, 16>{});
+    if (nch <= 2) return go(dt, std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{});
+    if (nch <= 4) return go(dt, std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+    return go(dt, std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{});
+  };
+  return dtype == kBF16 ? by_row(std::integral_constant<int, kBF16>{}) : by_row(std::integral_constant<int, kF16>{});
 }
 
 template <int DT>

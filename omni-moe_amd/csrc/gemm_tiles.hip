@@ -16,6 +16,7 @@
 #include "common.h"
 #include "gemm_tiles.h"
 #include "omni_moe_hip.h"
+#include "select.h"
 
 #include <type_traits>
 #include <utility>
@@ -120,8 +121,9 @@ __device__ __forceinline__ void swiglu_bwd_word(const uint32_t o, const uint32_t
 // only a block's first tile waits for memory before its first matrix instruction.  All of a ring step's loads are then requested in step 1:
 // the epilogue's stores are younger than every load of the next tile's first two ring steps and may stay in flight past its first
 // wait (memory instructions are counted in issue order).
+// (block, blocks): the place in the launch, or in its own part of one that it shares
 template <int DT, int LAY, int WM, int WN, int KG, int TM, int TN, int NS, int EPI, bool kTail, bool kStream, class Group>
-__global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Group g) {
+__device__ __forceinline__ void tiles_block(const Group& g, const int block, const int blocks) {
   constexpr bool AC = LAY == kTN, BC = LAY != kNT;             // the operand's K index is its row
   constexpr int NW = WM * WN * KG, BM = WM * TM * 16, BN = WN * TN * 16, BNO = EPI == kTileSwiglu ? BN / 2 : BN;
   constexpr int kABytes = BM * 128, kSub = (BM + BN) * 128, kStage = KG * kSub;
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
   if constexpr (std::is_same<Group, TileGroup>::value) {
 #pragma unroll
     for (int i = 1; i < kMaxProducts; ++i)
-      if (i < g.count && (int)blockIdx.x >= g.p[i].first) pi = i;
+      if (i < g.count && block >= g.p[i].first) pi = i;
   }
   const TileProduct& p = g.p[pi];
   const int M = p.M, N = p.N;
@@ -157,7 +159,7 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
     n = (w / rows) * BNO;
     return split;
   };
-  int f_tile = (int)blockIdx.x - p.first, fm0, fn0;            // the output tile that is being fetched
+  int f_tile = block - p.first, fm0, fn0;            // the output tile that is being fetched
   const int split = coords(f_tile, fm0, fn0);
 
   // ---- fetch cursor: the next ring step to request
@@ -295,8 +297,8 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
         f_b += KG * (uint32_t)f_bstep; f_bleft -= KG * f_bstep;
         mask_tail();
       }
-    } else if (kStream && f_tile + (int)gridDim.x < all) {
-      f_tile = scalar(f_tile + (int)gridDim.x);
+    } else if (kStream && f_tile + blocks < all) {
+      f_tile = scalar(f_tile + blocks);
       f_steps = tiles;
       coords(f_tile, fm0, fn0);
       enter_segment(0);
@@ -417,7 +419,7 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
   auto all0 = [&](auto... s) __attribute__((always_inline)) { (slot0(s), ...); };
   auto all1 = [&](auto... s) __attribute__((always_inline)) { (slot1(s), ...); };
 #pragma clang loop unroll(disable)
-  for (int tile = (int)blockIdx.x - p.first; tile < all; tile += (int)gridDim.x) {
+  for (int tile = block - p.first; tile < all; tile += blocks) {
   int m0, n0;
   coords(tile, m0, n0);
 #pragma clang loop unroll(disable)
@@ -582,6 +584,11 @@ __global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Gr
   vmcnt<0>();
 }
 
+template <int DT, int LAY, int WM, int WN, int KG, int TM, int TN, int NS, int EPI, bool kTail, bool kStream, class Group>
+__global__ __launch_bounds__(WM* WN* KG * 64, 2) void gemm_tiles_kernel(const Group g) {
+  tiles_block<DT, LAY, WM, WN, KG, TM, TN, NS, EPI, kTail, kStream, Group>(g, (int)blockIdx.x, (int)gridDim.x);
+}
+
 // The partial sums of a split product, added in split order and finished like the epilogue above: 8 columns per lane.
 template <int DT, int EPI>
 __global__ __launch_bounds__(256) void tile_reduce_kernel(const TileProduct p) {
@@ -707,6 +714,79 @@ static hipError_t start_tiles(const Group& g, int64_t blocks, hipStream_t s) {
                      dim3(S::WM * S::WN * S::KG * 64), L::kBytes, s, g);
   return hipGetLastError();
 }
+// ---- launches that two independent stages of the layer share -----------------------------------------
+// Up to a few thousand tokens the router's projection and its selection are 6-8 us launches that leave most of the chip idle, and everything waits for
+// them.  The projection's tiles go in front of the gate/up projection's (same tile shape), the selection beside the down projection's.
+struct TilePair { TileSingle router, mlp; };
+template <int DT, int kId, bool kTail>
+__global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64, 2) void tile_pair_kernel(const TilePair g) {
+  using R = Shape<kId>;
+  using S = Shape<kId, true>;
+  if ((int)blockIdx.x < g.mlp.p[0].first)
+    tiles_block<DT, kNT, R::WM, R::WN, R::KG, R::TM, R::TN, R::NS, kTileTwo, kTail, false, TileSingle>(g.router, (int)blockIdx.x, (int)gridDim.x);
+  else
+    tiles_block<DT, kNT, S::WM, S::WN, S::KG, S::TM, S::TN, S::NS, kTileSwiglu, kTail, false, TileSingle>(g.mlp, (int)blockIdx.x, (int)gridDim.x);
+}
+struct TileSelect {
+  TileSingle mlp;
+  SelectArgs select;
+  int regs, cells;                   // keys and candidates per lane
+};
+template <int DT, int kId>
+__global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64, 2) void tile_select_kernel(const TileSelect g) {
+  using S = Shape<kId>;
+  const int select_blocks = g.mlp.p[0].first;
+  if ((int)blockIdx.x < select_blocks) {
+    constexpr int kWaves = S::WM * S::WN * S::KG;
+    const int first = (int)blockIdx.x * kWaves + (int)(threadIdx.x >> 6), all = select_blocks * kWaves;
+    auto select = [&](auto cells) {
+      constexpr int C = decltype(cells)::value;
+      if (g.regs <= 1) select_packed<1, C>(g.select, first, all);
+      else if (g.regs <= 2) select_packed<2, C>(g.select, first, all);
+      else if (g.regs <= 4) select_packed<4, C>(g.select, first, all);
+      else select_packed<8, C>(g.select, first, all);
+    };
+    if (g.cells <= 1) select(std::integral_constant<int, 1>{});
+    else select(std::integral_constant<int, 2>{});
+    return;
+  }
+  tiles_block<DT, kNT, S::WM, S::WN, S::KG, S::TM, S::TN, S::NS, kTilePlain, false, false, TileSingle>(g.mlp, (int)blockIdx.x, (int)gridDim.x);
+}
+template <int kId, bool kSwiglu>
+constexpr int tile_lds() {
+  using S = Shape<kId, kSwiglu>;
+  return S::NS * S::KG * (S::WM * S::TM * 16 + S::WN * S::TN * 16) * 128;
+}
+template <auto kKernel, int kBytes>
+struct JointLds { static inline LdsKernel entry{(const void*)kKernel, kBytes}; };
+
+// Tiles of one unsplit product of shape kId
+template <int kId, bool kSwiglu>
+static int64_t tile_count(const TileProduct& p) {
+  using S = Shape<kId, kSwiglu>;
+  constexpr int BM = S::WM * S::TM * 16, BN = S::WN * S::TN * 16 / (kSwiglu ? 2 : 1);
+  return (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+}
+template <int DT, int kId>
+static bool start_pair(TilePair& g, hipStream_t s, hipError_t* e) {
+  using S = Shape<kId>;
+  constexpr int kStep = 64 * S::KG, kBytes = tile_lds<kId, true>() > tile_lds<kId, false>() ? tile_lds<kId, true>() : tile_lds<kId, false>();
+  TileProduct &r = g.router.p[0], &m = g.mlp.p[0];
+  const int64_t rb = tile_count<kId, false>(r), mb = tile_count<kId, true>(m), once = kCost[kId].at_once;
+  if (rb + mb > INT32_MAX / 2 || (rb + mb + once - 1) / once != (mb + once - 1) / once) return false;     // (a round more costs what the launch saves)
+  r.steps = m.steps = (r.seg[0].K + kStep - 1) / kStep;
+  m.first = (int)rb;
+  auto go = [&](auto tail) {
+    constexpr bool kTail = decltype(tail)::value;
+    if ((*e = JointLds<tile_pair_kernel<DT, kId, kTail>, kBytes>::entry.ensure()) != hipSuccess) return;
+    hipLaunchKernelGGL((tile_pair_kernel<DT, kId, kTail>), dim3((unsigned)(rb + mb)), dim3(S::WM * S::WN * S::KG * 64), kBytes, s, g);
+    *e = hipGetLastError();
+  };
+  if (r.seg[0].K % kStep) go(std::true_type{});
+  else go(std::false_type{});
+  return true;
+}
+
 template <int DT, int LAY, int kId, int EPI>
 static hipError_t launch_tiles(TileGroup& g, float* ws, int splits, bool exclusive, hipStream_t s) {
   using S = Shape<kId, EPI == kTileSwiglu>;
@@ -809,5 +889,79 @@ hipError_t launch_tile_group(int dtype, int layout, int epilogue, TileGroup& g, 
   if (dtype == kBF16) return go(std::integral_constant<int, kBF16>{});
   if (dtype == kF16) return go(std::integral_constant<int, kF16>{});
   return hipErrorInvalidValue;
+}
+
+static bool in_reach(const TileProduct& p) { return 256 * p.seg[0].lda <= INT32_MAX && 256 * p.seg[0].ldb <= INT32_MAX; }     // as launch_tile_group has it
+
+bool launch_tile_pair(int dtype, const TileProduct& router, const TileProduct& mlp, hipStream_t s, hipError_t* e) {
+  if ((dtype != kBF16 && dtype != kF16) || !in_reach(router) || !in_reach(mlp)) return false;
+  TilePair g;
+  g.router.p[0] = router;
+  g.mlp.p[0] = mlp;
+  const TileSize size{mlp.M, mlp.N};
+  const TileChoice c = choose_tiles(kTileSwiglu, &size, 1, mlp.seg[0].K, false);
+  auto go = [&](auto dt) -> bool {
+    constexpr int DT = decltype(dt)::value;
+    switch (c.shape) {
+      case 0: return start_pair<DT, 0>(g, s, e);
+      case 2: return start_pair<DT, 2>(g, s, e);
+      case 3: return start_pair<DT, 3>(g, s, e);
+      case 4: return start_pair<DT, 4>(g, s, e);
+      default: return false;
+    }
+  };
+  return dtype == kBF16 ? go(std::integral_constant<int, kBF16>{}) : go(std::integral_constant<int, kF16>{});
+}
+
+template <int DT, int kId>
+static hipError_t start_down(TileProduct p, const SelectArgs& select, int splits, float* ws, hipStream_t s, bool* selected, int* parts) {
+  using S = Shape<kId>;
+  constexpr int kStep = 64 * S::KG, kWaves = S::WM * S::WN * S::KG, kBytes = tile_lds<kId, false>();
+  const int total = (p.seg[0].K + kStep - 1) / kStep;
+  p.steps = (total + splits - 1) / splits;
+  p.splits = (total + p.steps - 1) / p.steps;
+  p.part = p.splits > 1 ? ws : nullptr;
+  *parts = p.splits;
+  const int64_t tiles = tile_count<kId, false>(p) * p.splits, once = kCost[kId].at_once;
+  if (tiles > INT32_MAX / 2) return hipErrorInvalidValue;
+  *selected = false;
+  {
+    // the selection takes the places that the last round of tiles leaves free, when they make at most two tokens a wave
+    TileSelect g{TileSingle{{p}}, select, (select.r + kWave - 1) / kWave, 0};
+    g.cells = prepare_select(g.select);
+    const int64_t free = (tiles + once - 1) / once * once - tiles, want = (select.num_tokens + kWaves - 1) / kWaves, blocks = want < free ? want : free;
+    if (total * kStep == p.seg[0].K && g.regs <= 8 && g.cells <= 2 && 2 * blocks * kWaves >= select.num_tokens) {
+      g.mlp.p[0].first = (int)blocks;
+      if (hipError_t e = JointLds<tile_select_kernel<DT, kId>, kBytes>::entry.ensure(); e != hipSuccess) return e;
+      hipLaunchKernelGGL((tile_select_kernel<DT, kId>), dim3((unsigned)(blocks + tiles)), dim3(kWaves * 64), kBytes, s, g);
+      *selected = true;
+      return hipGetLastError();
+    }
+  }
+  const TileSingle one{{p}};
+  return p.seg[0].K % kStep ? start_tiles<DT, kNT, kId, kTilePlain, true, false>(one, tiles, s) : start_tiles<DT, kNT, kId, kTilePlain, false, false>(one, tiles, s);
+}
+
+hipError_t launch_tile_down(int dtype, const TileProduct& p, const SelectArgs& select, void* ws, size_t ws_bytes, hipStream_t s, bool* selected, int* parts) {
+  if ((dtype != kBF16 && dtype != kF16) || !in_reach(p)) return hipErrorInvalidValue;
+  const TileSize size{p.M, p.N};
+  TileChoice c = choose_tiles(kTilePlain, &size, 1, p.seg[0].K, ws != nullptr);
+  if (c.splits > 1 && (size_t)c.splits * (size_t)p.M * (size_t)p.N * 4 > ws_bytes) c = choose_tiles(kTilePlain, &size, 1, p.seg[0].K, false);
+  auto go = [&](auto dt) -> hipError_t {
+    constexpr int DT = decltype(dt)::value;
+    switch (c.shape) {
+      case 0: case 1: {                                        // whole CUs for a tile: nothing beside it
+        *selected = false;
+        *parts = 1;
+        TileGroup g;
+        g.p[g.count++] = p;
+        return launch_choice<DT, kNT, kTilePlain>(g, c, (float*)ws, true, s);
+      }
+      case 2: return start_down<DT, 2>(p, select, c.splits, (float*)ws, s, selected, parts);
+      case 3: return start_down<DT, 3>(p, select, c.splits, (float*)ws, s, selected, parts);
+      default: return start_down<DT, 4>(p, select, c.splits, (float*)ws, s, selected, parts);
+    }
+  };
+  return dtype == kBF16 ? go(std::integral_constant<int, kBF16>{}) : go(std::integral_constant<int, kF16>{});
 }
 }  // namespace omni

@@ -5,7 +5,11 @@
 // matrix cores, so they share CUs); the fork and the join are two events the caller owns.
 #include "common.h"
 #include "few_tokens.h"
+#include "gemm_tiles.h"
 #include "omni_moe_hip.h"
+
+// defined beside the GEMM kernels: z = x [Wx;Wy]^T
+int omni_gemm_router_projection(const void* x, const void* wx, const void* wy, void* z, float* part_mean, float* part_m2, int64_t T, int H, int r, int dtype, void* stream);
 
 namespace omni {
 static inline size_t up256(size_t v) { return (v + 255) / 256 * 256; }
@@ -16,10 +20,43 @@ int expert_algo_check(int algo, int64_t num_tokens, int hidden_size, int64_t num
 int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype);
 // defined beside the select kernels: whether they take num_expert_sqrt keys per half with top_k and this dtype
 bool select_covers(int r, int k, int dtype);
+int launch_router_select(const SelectArgs& g, hipStream_t s);
+// defined beside the expert kernels: the gather algorithm with the final add
+hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, int64_t T, int H,
+                             int k, int64_t N, int dtype, hipStream_t s);
 // defined beside the GEMM kernels: the two projections of omni_mlp_fwd with the caller's word on whether the launch has the GPU to itself
 // (then a GEMM of more tiles than CUs may take the form that holds every CU until it ends); h lies at the workspace's start
 int mlp_gate_up_impl(const void* x, const void* wg, const void* wu, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive);
 int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive);
+// Projection | gate/up, selection | down projection, experts and add; where two stages do not fit one launch, each is its own.
+static int joint_forward(const FewTokens& f, int dtype, size_t parts_bytes, hipStream_t s) {
+  auto code = [](hipError_t e) { return e == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)e; };
+  const int64_t H2 = (int64_t)f.H * 2, I2 = (int64_t)f.I * 2;
+  TileProduct router, mlp, down;
+  router.seg[0] = TileSegment{(const uint8_t*)f.x, (const uint8_t*)f.wx, H2, H2, 0, f.H};
+  router.b_up = (const uint8_t*)f.wy;
+  router.segments = mlp.segments = down.segments = 1;
+  router.M = mlp.M = down.M = f.T;
+  router.N = 2 * f.select.r; router.ldc = 2 * (int64_t)router.N; router.c = (uint8_t*)f.z;
+  mlp.seg[0] = TileSegment{(const uint8_t*)f.x, (const uint8_t*)f.wg, H2, H2, 0, f.H};
+  mlp.b_up = (const uint8_t*)f.wu;
+  mlp.N = f.I; mlp.ldc = I2; mlp.c = (uint8_t*)f.h;
+  down.seg[0] = TileSegment{(const uint8_t*)f.h, (const uint8_t*)f.wd, I2, I2, 0, f.I};
+  down.N = f.H; down.ldc = H2; down.c = (uint8_t*)f.y;
+  hipError_t he = hipSuccess;
+  if (launch_tile_pair(dtype, router, mlp, s, &he)) {
+    if (he != hipSuccess) return code(he);
+  } else {
+    if (int e = omni_gemm_router_projection(f.x, f.wx, f.wy, f.z, nullptr, nullptr, f.T, f.H, f.select.r, dtype, s)) return e;
+    if (int e = mlp_gate_up_impl(f.x, f.wg, f.wu, f.T, f.H, f.I, dtype, f.h, s, true)) return e;
+  }
+  bool selected = false;
+  int parts = 1;
+  if ((he = launch_tile_down(dtype, down, f.select, parts_bytes ? f.parts : nullptr, parts_bytes, s, &selected, &parts)) != hipSuccess) return code(he);
+  if (!selected)
+    if (int e = launch_router_select(f.select, s)) return e;
+  return code(launch_gather_add(f.x, f.up, f.down, f.select.gates, f.select.indices, f.y, parts > 1 ? f.parts : nullptr, parts, f.T, f.H, f.select.k, f.N, dtype, s));
+}
 }  // namespace omni
 
 // workspace: router workspace | gates [T,k] | ids [T,k] | expert output [T,H] | expert workspace | MLP workspace
@@ -95,14 +132,21 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   void* mlp_ws = w;
 
   hipStream_t main_s = (hipStream_t)stream;
-  // A few tokens in eval mode: three launches in all, on the caller's stream (few_tokens.hip).  64 is four row
-  // tiles, what a wave has registers and LDS for; there the joint launches take 27 us where the six kernels took 44 (hidden 1024, bf16).
-  if (!training && num_experts <= UINT32_MAX && few_tokens_covers_layer(num_tokens, hidden_size, intermediate_size, num_expert_sqrt, num_experts_per_token, dtype) &&
+  // Up to a certain size in eval mode the layer is joint launches on the caller's stream: stages that do not depend on each other share one.
+  //   * at most 64 tokens (four row tiles, what a wave has registers and LDS for): few_tokens.hip, three launches; 64 tokens 44 -> 27 us (hidden 1024, bf16).
+  //   * up to 2^33 token x hidden x intermediate (2048 tokens at 1024 x 4096), beyond which gate/up fills the chip for several rounds and two streams are the
+  //     better overlap: projection | gate/up, selection | down projection, experts and add.
+  const size_t h_bytes = up256(T * (size_t)intermediate_size * es);
+  const bool few = few_tokens_covers_layer(num_tokens, hidden_size, intermediate_size, num_expert_sqrt, num_experts_per_token, dtype);
+  const bool joint = dtype != OMNI_F32 && num_experts_per_token > 0 && num_expert_sqrt % 8 == 0 && hidden_size % 8 == 0 && intermediate_size % 8 == 0 &&
+                     (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0;
+  if (!training && num_experts <= UINT32_MAX && (few || joint) &&
       resolve_algo(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) == OMNI_EXPERT_ALGO_GATHER) {
     if (stats_dtype != OMNI_BF16 && stats_dtype != OMNI_F16 && stats_dtype != OMNI_F32) return OMNI_ERR_DTYPE;
     if (!gate_weight || !up_weight || !down_weight || !router_weight_x || !router_weight_y || !running_mean_x || !running_var_x || !running_mean_y || !running_var_y)
       return OMNI_ERR_NULL;
-    FewTokens f{x, gate_weight, up_weight, down_weight, mlp_ws, y, (float*)((char*)mlp_ws + up256(T * (size_t)intermediate_size * es)), nullptr,
+    float* const parts = (float*)((char*)mlp_ws + h_bytes);
+    FewTokens f{x, gate_weight, up_weight, down_weight, mlp_ws, y, parts, nullptr,
                 (int)num_tokens, hidden_size, intermediate_size, router_weight_x, router_weight_y, router_ws};
     SelectArgs& g = f.select;
     g.lx = router_ws; g.ly = (const char*)router_ws + (size_t)num_expert_sqrt * es; g.row_stride = 2 * num_expert_sqrt;
@@ -112,9 +156,12 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
     g.gates = gates; g.indices = ids;
     g.num_tokens = (int)num_tokens; g.r = num_expert_sqrt; g.k = num_experts_per_token; g.dt = dtype;
     f.up = up_embed; f.down = down_embed; f.N = num_experts;
-    if (few_tokens_aligned(f)) {
-      const hipError_t he = launch_few_tokens(dtype, f, main_s);
-      return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
+    if (few_tokens_aligned(f) && num_tokens <= INT32_MAX / 256) {
+      if (few) {
+        const hipError_t he = launch_few_tokens(dtype, f, main_s);
+        return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
+      }
+      return joint_forward(f, dtype, omni_mlp_workspace_bytes(num_tokens, hidden_size, intermediate_size, dtype) - h_bytes, main_s);
     }
   }
   hipStream_t branch = side_stream ? (hipStream_t)side_stream : main_s;

@@ -407,6 +407,9 @@ static int select_dispatch(SelectArgs g, hipStream_t s) {
   return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
 }
 
+// for the layer call, which fills the arguments itself
+int launch_router_select(const SelectArgs& g, hipStream_t s) { return select_dispatch(g, s); }
+
 // ---- BatchNorm1d(affine=False) statistics over the T rows of z [T, C] -------------------
 constexpr int kBnRows = 32;       // rows per partial: one 32-row MFMA tile of the projection GEMM
 

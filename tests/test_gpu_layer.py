@@ -627,3 +627,41 @@ def test_small_fp32_products_match_fp64(case, device):
         var = torch.cat([bufs[1], bufs[4]]).cpu().double()
         torch.testing.assert_close(mean, z.mean(0), rtol=1e-5, atol=8 * 2 ** -24 * H ** 0.5)
         torch.testing.assert_close(var, z.var(0), rtol=1e-5, atol=8 * 2 ** -24 * H ** 0.5)
+
+
+# T, H, I, N, k: past the few-token launches; tile shapes and K splits change with T and H, the selection finds room beside the down projection or not,
+# 2, 4 and 8 keys a lane, a key count that is not a multiple of 8 and one beyond the joint launch's registers (both on launches of their own)
+JOINT_CASES = [(65, 1024, 4096, 4096, 16), (129, 256, 512, 10000, 8), (613, 1024, 4096, 4096, 16), (700, 520, 1048, 65536, 32), (300, 2048, 2056, 262144, 32),
+               (1900, 1024, 4096, 1024, 4), (200, 512, 1536, 900, 6), (90, 256, 1024, 360000, 10)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", JOINT_CASES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
+def test_joint_launches_match_the_operators(case, dtype, device):
+    """Eval mode past 64 tokens: projections, selection and add in joint launches against the operators one by one.  The router's scores may round
+    differently (its sums run in another order), so the expert term is compared where both chose the same experts."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, H, I, N, k = case
+    print(f"joint {case} {dtype}", flush=True)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", N, k)).to(device=device, dtype=dtype).eval()
+    g = torch.Generator(device=device).manual_seed(T)
+    for p in layer.parameters():
+        p.normal_(0.0, H ** -0.5, generator=g)
+    layer.down_proj.weight.normal_(0.0, I ** -0.5, generator=g)
+    for norm in (layer.router_norm_x, layer.router_norm_y):
+        norm.running_mean.normal_(0.0, 0.3, generator=g)
+        norm.running_var.uniform_(0.5, 2.0, generator=g)
+    x = torch.randn(1, T, H, device=device, generator=g).to(dtype)
+    ops = _ops()
+    gates, ids = layer.route(x[0])
+    experts = ops.hip_omni_expert_func(x[0], layer.up_embed.weight, layer.down_embed.weight, gates, ids).double()
+    mlp = ops.hip_omni_mlp_func(x[0], layer.gate_proj.weight, layer.up_proj.weight, layer.down_proj.weight).double()
+    got = layer(x)[0].double()
+    eps = torch.finfo(dtype).eps
+    scale = max(1.0, float((mlp + experts).abs().max()))
+    row = (got - (mlp + experts)).abs().amax(dim=1)
+    assert (row <= 4 * eps * scale).double().mean().item() >= 0.95          # a token with another least expert differs by that expert's share
+    assert row.max().item() <= 0.5 * scale
+    assert torch.equal(layer(x)[0].double(), got)
+    layer.overlap_branches = False
+    assert torch.equal(layer(x)[0].double(), got)
