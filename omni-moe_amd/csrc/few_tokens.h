@@ -31,6 +31,8 @@ bool few_tokens_covers_layer(int64_t T, int64_t H, int64_t I, int r, int k, int 
 size_t few_tokens_parts_bytes(int64_t T, int64_t H, int64_t I);
 // rows are fetched 16 bytes at a time: every pointer of `f` (NULL counts as aligned) is
 bool few_tokens_aligned(const FewTokens& f);
+// launch 3 alone, for any number of tokens (H <= 4096): the experts, and the final add of `splits` parts [splits][T][H] (at most 8) or, with 0, of the rounded rows in y
+hipError_t launch_few_back(int dtype, const FewTokens& f, int splits, hipStream_t s);
 hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s);
 
 }  // namespace omni

@@ -213,6 +213,7 @@ struct BackArgs {
 };
 
 // Launch 3, a block per token: y = round(round(sum of the parts) + round(experts)).  NCH 1-KiB pieces of a row; G slots of a wave at once.
+// splits 0: y holds the rounded sums already.
 // kExperts false: the MLP alone, residual (or nothing) instead of the experts.
 template <int DT, int NCH, int G, bool kExperts>
 __global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const BackArgs g) {
@@ -224,7 +225,8 @@ __global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const BackArgs
   const int64_t plane = (int64_t)g.T * g.H;
   auto request = [&](int n) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < kMostParts; ++s) part[s] = *(const f32x4_t*)(g.parts + min(s, g.splits - 1) * plane + (int64_t)t * g.H + min(n, g.H - 4));
+    for (int s = 0; s < kMostParts; ++s)
+      if (g.splits) part[s] = *(const f32x4_t*)(g.parts + min(s, g.splits - 1) * plane + (int64_t)t * g.H + min(n, g.H - 4));
   };
   request(threadIdx.x * 4);
   const int per = kExperts ? (g.k + kFewWaves - 1) / kFewWaves : 0, active = kExperts ? (g.k + per - 1) / per : 0;
@@ -293,6 +295,10 @@ __global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const BackArgs
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] += part[s][q];
     const int64_t out = ((int64_t)t * g.H + n) * 2;
+    if (kExperts && g.splits == 0) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = Elem<DT>::load(g.y + out, q);
+    }
     if (kExperts || g.residual) {
       float e[4] = {0.f, 0.f, 0.f, 0.f};
       if constexpr (kExperts) {
@@ -329,6 +335,15 @@ hipError_t start(const Args& a, int64_t blocks, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <int DT>
+hipError_t launch_back(const BackArgs& b, hipStream_t s) {
+  const int nch = (b.H + 511) / 512;
+  if (nch <= 1) return start<few_back_kernel<DT, 1, 4, true>, kFewWaves * 1 * 2048>(b, b.T, s);
+  if (nch <= 2) return start<few_back_kernel<DT, 2, 4, true>, kFewWaves * 2 * 2048>(b, b.T, s);
+  if (nch <= 4) return start<few_back_kernel<DT, 4, 2, true>, kFewWaves * 4 * 2048>(b, b.T, s);
+  return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, b.T, s);
+}
+
 template <int DT, int TM>
 hipError_t launch(const FewTokens& f, hipStream_t s) {
   const bool layer = f.up != nullptr;
@@ -358,11 +373,7 @@ hipError_t launch(const FewTokens& f, hipStream_t s) {
   const BackArgs b{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, (const uint8_t*)f.residual, f.select.gates, f.select.indices, f.parts, (uint8_t*)f.y,
                    f.T, f.H, f.select.k, splits, (uint32_t)f.N};
   if (!layer) return start<few_back_kernel<DT, 1, 1, false>, 0>(b, f.T, s);
-  const int nch = (f.H + 511) / 512;
-  if (nch <= 1) return start<few_back_kernel<DT, 1, 4, true>, kFewWaves * 1 * 2048>(b, f.T, s);
-  if (nch <= 2) return start<few_back_kernel<DT, 2, 4, true>, kFewWaves * 2 * 2048>(b, f.T, s);
-  if (nch <= 4) return start<few_back_kernel<DT, 4, 2, true>, kFewWaves * 4 * 2048>(b, f.T, s);
-  return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, f.T, s);
+  return launch_back<DT>(b, s);
 }
 
 }  // namespace
@@ -391,6 +402,14 @@ hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s) {
   };
   if (dtype == kBF16) return go(std::integral_constant<int, kBF16>{});
   if (dtype == kF16) return go(std::integral_constant<int, kF16>{});
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_few_back(int dtype, const FewTokens& f, int splits, hipStream_t s) {
+  const BackArgs b{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, nullptr, f.select.gates, f.select.indices, f.parts, (uint8_t*)f.y,
+                   f.T, f.H, f.select.k, splits, (uint32_t)f.N};
+  if (dtype == kBF16) return launch_back<kBF16>(b, s);
+  if (dtype == kF16) return launch_back<kF16>(b, s);
   return hipErrorInvalidValue;
 }
 

@@ -57,6 +57,7 @@ float tile_estimate_us(int epilogue, int64_t M, int64_t N, int64_t K, bool may_s
 bool launch_tile_pair(int dtype, const TileProduct& router, const TileProduct& mlp, hipStream_t s, hipError_t* e);
 // The down projection (kTilePlain, kNT) and, beside it, the selection, if there is room (*selected).  *parts > 1: its sums are left in ws, [parts][M][N] fp32.
 struct SelectArgs;
+constexpr int kMostDownParts = 8;
 hipError_t launch_tile_down(int dtype, const TileProduct& p, const SelectArgs& select, void* ws, size_t ws_bytes, hipStream_t s, bool* selected, int* parts);
 
 }  // namespace omni

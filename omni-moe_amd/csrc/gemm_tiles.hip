@@ -772,8 +772,8 @@ static bool start_pair(TilePair& g, hipStream_t s, hipError_t* e) {
   using S = Shape<kId>;
   constexpr int kStep = 64 * S::KG, kBytes = tile_lds<kId, true>() > tile_lds<kId, false>() ? tile_lds<kId, true>() : tile_lds<kId, false>();
   TileProduct &r = g.router.p[0], &m = g.mlp.p[0];
-  const int64_t rb = tile_count<kId, false>(r), mb = tile_count<kId, true>(m), once = kCost[kId].at_once;
-  if (rb + mb > INT32_MAX / 2 || (rb + mb + once - 1) / once != (mb + once - 1) / once) return false;     // (a round more costs what the launch saves)
+  const int64_t rb = tile_count<kId, false>(r), mb = tile_count<kId, true>(m);
+  if (rb + mb > INT32_MAX / 2) return false;
   r.steps = m.steps = (r.seg[0].K + kStep - 1) / kStep;
   m.first = (int)rb;
   auto go = [&](auto tail) {
@@ -898,12 +898,21 @@ bool launch_tile_pair(int dtype, const TileProduct& router, const TileProduct& m
   TilePair g;
   g.router.p[0] = router;
   g.mlp.p[0] = mlp;
-  const TileSize size{mlp.M, mlp.N};
-  const TileChoice c = choose_tiles(kTileSwiglu, &size, 1, mlp.seg[0].K, false);
+  // The shape that both products' tiles take least time in, by the figures above, if that is less than a launch for each
+  const TileSize sizes[2] = {{router.M, router.N}, {mlp.M, mlp.N}};
+  const int64_t K = mlp.seg[0].K, kt = (K + 63) / 64;
+  int shape = -1;
+  float best = choose_tiles(kTileTwo, sizes, 1, K, false).us + choose_tiles(kTileSwiglu, sizes + 1, 1, K, true).us;
+  for (int i : {2, 3, 4}) {                                    // (256 x 256: 30.6 us at 1024 tokens, where the two launches take 25.8)
+    const ShapeCost &r = kCost[i], &m = i == 4 ? kSwigluCost : kCost[i];
+    if (r.kg > 1 && K < 512) continue;
+    const int64_t n = ((router.M + r.bm - 1) / r.bm) * ((router.N + r.bn - 1) / r.bn) + ((mlp.M + m.bm - 1) / m.bm) * ((mlp.N + m.bn / 2 - 1) / (m.bn / 2));
+    const float used = n >= m.at_once ? 1.f : (float)n / m.at_once, us = m.fixed + (float)((n + m.at_once - 1) / m.at_once * kt) * (m.idle + (m.full - m.idle) * used);
+    if (us < best) { best = us; shape = i; }
+  }
   auto go = [&](auto dt) -> bool {
     constexpr int DT = decltype(dt)::value;
-    switch (c.shape) {
-      case 0: return start_pair<DT, 0>(g, s, e);
+    switch (shape) {
       case 2: return start_pair<DT, 2>(g, s, e);
       case 3: return start_pair<DT, 3>(g, s, e);
       case 4: return start_pair<DT, 4>(g, s, e);
@@ -918,25 +927,34 @@ static hipError_t start_down(TileProduct p, const SelectArgs& select, int splits
   using S = Shape<kId>;
   constexpr int kStep = 64 * S::KG, kWaves = S::WM * S::WN * S::KG, kBytes = tile_lds<kId, false>();
   const int total = (p.seg[0].K + kStep - 1) / kStep;
-  p.steps = (total + splits - 1) / splits;
-  p.splits = (total + p.steps - 1) / p.steps;
-  p.part = p.splits > 1 ? ws : nullptr;
+  const int64_t once = kCost[kId].at_once, want = (select.num_tokens + kWaves - 1) / kWaves;
+  TileSelect g{TileSingle{}, select, (select.r + kWave - 1) / kWave, 0};
+  g.cells = prepare_select(g.select);
+  const bool joint = total * kStep == p.seg[0].K && g.regs <= 8 && g.cells <= 2;
+  int64_t tiles = 0, blocks = 0;
+  auto split = [&](int n) {
+    p.steps = (total + n - 1) / n;
+    p.splits = (total + p.steps - 1) / p.steps;
+    p.part = p.splits > 1 ? ws : nullptr;
+    tiles = tile_count<kId, false>(p) * p.splits;
+    // the selection takes the places that the last round of tiles leaves free, when they make at most two tokens a wave (of more than 128 keys: one)
+    const int64_t free = (tiles + once - 1) / once * once - tiles;
+    blocks = want < free ? want : free;
+    return joint && (g.regs <= 2 ? 2 : 1) * blocks * kWaves >= select.num_tokens;
+  };
+  // ... for which a product in many splits gives up to a quarter of them (a launch is 5-7 us, a split step 0.2)
+  int n = splits;
+  while (n > 1 && n > splits * 3 / 4 && !split(n)) --n;
+  *selected = split(n);
+  if (!*selected) split(splits);
   *parts = p.splits;
-  const int64_t tiles = tile_count<kId, false>(p) * p.splits, once = kCost[kId].at_once;
   if (tiles > INT32_MAX / 2) return hipErrorInvalidValue;
-  *selected = false;
-  {
-    // the selection takes the places that the last round of tiles leaves free, when they make at most two tokens a wave
-    TileSelect g{TileSingle{{p}}, select, (select.r + kWave - 1) / kWave, 0};
-    g.cells = prepare_select(g.select);
-    const int64_t free = (tiles + once - 1) / once * once - tiles, want = (select.num_tokens + kWaves - 1) / kWaves, blocks = want < free ? want : free;
-    if (total * kStep == p.seg[0].K && g.regs <= 8 && g.cells <= 2 && 2 * blocks * kWaves >= select.num_tokens) {
-      g.mlp.p[0].first = (int)blocks;
-      if (hipError_t e = JointLds<tile_select_kernel<DT, kId>, kBytes>::entry.ensure(); e != hipSuccess) return e;
-      hipLaunchKernelGGL((tile_select_kernel<DT, kId>), dim3((unsigned)(blocks + tiles)), dim3(kWaves * 64), kBytes, s, g);
-      *selected = true;
-      return hipGetLastError();
-    }
+  if (*selected) {
+    g.mlp.p[0] = p;
+    g.mlp.p[0].first = (int)blocks;
+    if (hipError_t e = JointLds<tile_select_kernel<DT, kId>, kBytes>::entry.ensure(); e != hipSuccess) return e;
+    hipLaunchKernelGGL((tile_select_kernel<DT, kId>), dim3((unsigned)(blocks + tiles)), dim3(kWaves * 64), kBytes, s, g);
+    return hipGetLastError();
   }
   const TileSingle one{{p}};
   return p.seg[0].K % kStep ? start_tiles<DT, kNT, kId, kTilePlain, true, false>(one, tiles, s) : start_tiles<DT, kNT, kId, kTilePlain, false, false>(one, tiles, s);
@@ -947,6 +965,7 @@ hipError_t launch_tile_down(int dtype, const TileProduct& p, const SelectArgs& s
   const TileSize size{p.M, p.N};
   TileChoice c = choose_tiles(kTilePlain, &size, 1, p.seg[0].K, ws != nullptr);
   if (c.splits > 1 && (size_t)c.splits * (size_t)p.M * (size_t)p.N * 4 > ws_bytes) c = choose_tiles(kTilePlain, &size, 1, p.seg[0].K, false);
+  if (c.splits > kMostDownParts) c.splits = kMostDownParts;
   auto go = [&](auto dt) -> hipError_t {
     constexpr int DT = decltype(dt)::value;
     switch (c.shape) {
