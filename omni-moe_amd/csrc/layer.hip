@@ -32,7 +32,9 @@ int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int3
 // 10.8 / 11, 613 tokens 14.3 / 11.0 (hidden 1024, top-16).
 constexpr int kBlockPerToken = 384;
 // Projection | gate/up, selection | down projection, experts and add; where two stages do not fit one launch, each is its own.
-static int joint_forward(const FewTokens& f, int dtype, size_t parts_bytes, hipStream_t s) {
+// statistics (training): projects z and leaves its column statistics, which f.select reads.
+template <class Statistics>
+static int joint_forward(const FewTokens& f, int dtype, size_t parts_bytes, hipStream_t s, bool training, Statistics&& statistics) {
   auto code = [](hipError_t e) { return e == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)e; };
   const int64_t H2 = (int64_t)f.H * 2, I2 = (int64_t)f.I * 2;
   TileProduct router, mlp, down;
@@ -47,7 +49,10 @@ static int joint_forward(const FewTokens& f, int dtype, size_t parts_bytes, hipS
   down.seg[0] = TileSegment{(const uint8_t*)f.h, (const uint8_t*)f.wd, I2, I2, 0, f.I};
   down.N = f.H; down.ldc = H2; down.c = (uint8_t*)f.y;
   hipError_t he = hipSuccess;
-  if (launch_tile_pair(dtype, router, mlp, s, &he)) {
+  if (training) {
+    if (int e = statistics()) return e;
+    if (int e = mlp_gate_up_impl(f.x, f.wg, f.wu, f.T, f.H, f.I, dtype, f.h, s, true)) return e;
+  } else if (launch_tile_pair(dtype, router, mlp, s, &he)) {
     if (he != hipSuccess) return code(he);
   } else {
     if (int e = omni_gemm_router_projection(f.x, f.wx, f.wy, f.z, nullptr, nullptr, f.T, f.H, f.select.r, dtype, s)) return e;
@@ -136,15 +141,16 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   void* mlp_ws = w;
 
   hipStream_t main_s = (hipStream_t)stream;
-  // Up to a certain size in eval mode the layer is joint launches on the caller's stream: stages that do not depend on each other share one.
-  //   * at most 64 tokens (four row tiles, what a wave has registers and LDS for): few_tokens.hip, three launches; 64 tokens 44 -> 27 us (hidden 1024, bf16).
+  // Up to a certain size the layer is joint launches on the caller's stream: stages that do not depend on each other share one.
+  //   * at most 64 tokens in eval mode (four row tiles, what a wave has registers and LDS for): few_tokens.hip, three launches; 64 tokens 44 -> 27 us (hidden 1024, bf16).
   //   * up to 2^33 token x hidden x intermediate (2048 tokens at 1024 x 4096), beyond which gate/up fills the chip for several rounds and two streams are the
   //     better overlap: projection | gate/up, selection | down projection, experts and add.
   const size_t h_bytes = up256(T * (size_t)intermediate_size * es);
   const bool few = few_tokens_covers_layer(num_tokens, hidden_size, intermediate_size, num_expert_sqrt, num_experts_per_token, dtype);
   const bool joint = dtype != OMNI_F32 && num_experts_per_token > 0 && num_expert_sqrt % 8 == 0 && hidden_size % 8 == 0 && intermediate_size % 8 == 0 &&
                      (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0;
-  if (!training && num_experts <= UINT32_MAX && (few || joint) &&
+  // (batch statistics: the projection and their merge stay launches of their own; a cumulative average, momentum < 0, is counted by the select kernel)
+  if ((training ? joint && momentum >= 0.f : few || joint) && num_experts <= UINT32_MAX &&
       resolve_algo(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) == OMNI_EXPERT_ALGO_GATHER) {
     if (stats_dtype != OMNI_BF16 && stats_dtype != OMNI_F16 && stats_dtype != OMNI_F32) return OMNI_ERR_DTYPE;
     if (!gate_weight || !up_weight || !down_weight || !router_weight_x || !router_weight_y || !running_mean_x || !running_var_x || !running_mean_y || !running_var_y)
@@ -154,18 +160,27 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
                 (int)num_tokens, hidden_size, intermediate_size, router_weight_x, router_weight_y, router_ws};
     SelectArgs& g = f.select;
     g.lx = router_ws; g.ly = (const char*)router_ws + (size_t)num_expert_sqrt * es; g.row_stride = 2 * num_expert_sqrt;
-    g.run_mean[0] = running_mean_x; g.run_mean[1] = running_mean_y;
-    g.run_var[0] = running_var_x; g.run_var[1] = running_var_y;
-    g.stat_dt = stats_dtype; g.eps = eps;
+    if (training) {
+      g.stats = (const float*)((const char*)router_ws + omni_router_workspace_stats_offset(num_tokens, num_expert_sqrt, dtype));
+    } else {
+      g.run_mean[0] = running_mean_x; g.run_mean[1] = running_mean_y;
+      g.run_var[0] = running_var_x; g.run_var[1] = running_var_y;
+      g.stat_dt = stats_dtype; g.eps = eps;
+    }
     g.gates = gates; g.indices = ids;
     g.num_tokens = (int)num_tokens; g.r = num_expert_sqrt; g.k = num_experts_per_token; g.dt = dtype;
     f.up = up_embed; f.down = down_embed; f.N = num_experts;
     if (few_tokens_aligned(f) && num_tokens <= INT32_MAX / 256) {
-      if (few) {
+      if (few && !training) {
         const hipError_t he = launch_few_tokens(dtype, f, main_s);
         return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
       }
-      return joint_forward(f, dtype, omni_mlp_workspace_bytes(num_tokens, hidden_size, intermediate_size, dtype) - h_bytes, main_s);
+      return joint_forward(f, dtype, omni_mlp_workspace_bytes(num_tokens, hidden_size, intermediate_size, dtype) - h_bytes, main_s, training != 0, [&]() -> int {
+        // without a selection (k = 0) omni_router_fwd projects, merges the statistics, moves the running buffers and counts the batch
+        return omni_router_fwd(x, router_weight_x, router_weight_y, running_mean_x, running_var_x, num_batches_tracked_x, running_mean_y, running_var_y,
+                               num_batches_tracked_y, 1, momentum, eps, nullptr, nullptr, nullptr, num_tokens, hidden_size, num_expert_sqrt, 0, dtype, stats_dtype,
+                               router_ws, main_s);
+      });
     }
   }
   hipStream_t branch = side_stream ? (hipStream_t)side_stream : main_s;

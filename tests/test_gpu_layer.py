@@ -665,3 +665,14 @@ def test_joint_launches_match_the_operators(case, dtype, device):
     assert torch.equal(layer(x)[0].double(), got)
     layer.overlap_branches = False
     assert torch.equal(layer(x)[0].double(), got)
+    # batch statistics: the router stage alone on equal buffers leaves the same buffers and chooses the same experts
+    layer.train()
+    before = [b.clone() for b in layer.buffers()]
+    gates, ids = layer.route(x[0])
+    after = [b.clone() for b in layer.buffers()]
+    for b, v in zip(layer.buffers(), before):
+        b.copy_(v)
+    got = layer(x)[0].double()
+    assert all(torch.equal(a, b) for a, b in zip(after, layer.buffers()))
+    experts = ops.hip_omni_expert_func(x[0], layer.up_embed.weight, layer.down_embed.weight, gates, ids).double()
+    assert (got - (mlp + experts)).abs().max().item() <= 4 * eps * max(1.0, float((mlp + experts).abs().max()))
