@@ -305,7 +305,7 @@ def main():
         r = layer.num_expert_sqrt
         # the gate/up projection as the two-stream layer step runs it (one block per tile: 512 blocks that leave room for the side branch as they retire) ...
         m, b = time_launches(torch, lambda: hip.hip_swiglu_linear_func(xf, layer.gate_proj.weight, layer.up_proj.weight, shared=True))
-        kernels.append(mfma_entry("gemm_stream_kernel<swiglu>, one block per tile (gate/up projection + SwiGLU, as in the two-stream layer step), c4", 4 * T * H * I, m, b, TRAFFIC_BYTES["gateup_c4"], sustained))
+        kernels.append(mfma_entry("gemm_tiles_kernel<swiglu>, one block per tile (gate/up projection + SwiGLU, as in the two-stream layer step), c4", 4 * T * H * I, m, b, TRAFFIC_BYTES["gateup_c4"], sustained))
         # ... and as every caller gets it that has the GPU to itself (operator calls, the one-stream layer): one block per CU streaming through its tiles
         m_s, b_s = time_launches(torch, lambda: hip.hip_swiglu_linear_func(xf, layer.gate_proj.weight, layer.up_proj.weight))
         kernels[-1]["streaming_form_alone_ms"] = m_s
@@ -487,13 +487,13 @@ def main():
         del layer5.overlap_max_work
         xf5 = x5
         m_gu, b_gu = time_launches(torch, lambda: hip.hip_swiglu_linear_func(xf5, layer5.gate_proj.weight, layer5.up_proj.weight), n=5, reps=5, warmup=2)
-        e_gu = mfma_entry("gemm_stream_kernel<swiglu> (gate/up projection + SwiGLU), config 5 (32768 x 2 x 8192 x 2048)", 4 * T5 * H5 * I5, m_gu, b_gu, None, sustained)
+        e_gu = mfma_entry("gemm_tiles_kernel<swiglu> (gate/up projection + SwiGLU), config 5 (32768 x 2 x 8192 x 2048)", 4 * T5 * H5 * I5, m_gu, b_gu, None, sustained)
         h5 = hip.hip_swiglu_linear_func(xf5, layer5.gate_proj.weight, layer5.up_proj.weight)
         m_d, b_d = time_launches(torch, lambda: hip.hip_linear_func(h5, layer5.down_proj.weight), n=5, reps=5, warmup=2)
-        e_d = mfma_entry("gemm_stream_kernel<plain> (down projection), config 5 (32768 x 2048 x 8192)", 2 * T5 * H5 * I5, m_d, b_d, None, sustained)
+        e_d = mfma_entry("gemm_tiles_kernel<plain> (down projection), config 5 (32768 x 2048 x 8192)", 2 * T5 * H5 * I5, m_d, b_d, None, sustained)
         wcat5 = torch.cat([wx5, wy5], 0)
         m_r, b_r = time_launches(torch, lambda: hip.hip_linear_func(xf5, wcat5), n=5, reps=5, warmup=2)
-        e_r = mfma_entry("gemm_stream_kernel<plain> (router projection, both halves: 32768 x 1024 x 2048; arithmetic intensity 669 flop/B), config 5",
+        e_r = mfma_entry("gemm_tiles_kernel<plain> (router projection, both halves: 32768 x 1024 x 2048; arithmetic intensity 669 flop/B), config 5",
                          4 * T5 * H5 * r5, m_r, b_r, None, sustained)
         m_lib, _ = time_launches(torch, lambda: torch.matmul(xf5, wcat5.t()), n=5, reps=3, warmup=2)
         e_r["library_gemm_same_flops_ms"] = m_lib
