@@ -111,6 +111,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(const SortPa
   extern __shared__ int32_t tables[];
   int32_t* tbl = tables;                                 // [wave][width]: per wave and bin: count, then running output position
   int32_t *bin_base = tbl + kSortWaves * a.width, *before_s = bin_base + a.width, *total_s = before_s + a.width;
+  __shared__ int32_t wave_total_s[kSortWaves];
   __shared__ int32_t below_s;                            // pairs in the slices below this one, all tiles
   const int lane = lane_id(), wave = threadIdx.x >> 6;
   const int tile_idx = (int)blockIdx.x / kSlices, slice = (int)blockIdx.x % kSlices;
@@ -197,9 +198,9 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(const SortPa
   }
   __syncthreads();
 
-  // exclusive scan of the slice's totals (wave 0, a run of consecutive bins per lane): every bin's first position
-  if (wave == 0) {
-    const int per = (a.width + kWave - 1) / kWave, b0 = lane * per;
+  // exclusive scan of the slice's totals (a run of consecutive bins per thread): every bin's first position
+  {
+    const int per = (a.width + kSortThreads - 1) / kSortThreads, b0 = (int)threadIdx.x * per;
     int32_t sum = 0;
     for (int i = 0; i < per; ++i) sum += b0 + i < a.width ? total_s[b0 + i] : 0;
     int32_t inc = sum;
@@ -208,7 +209,11 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(const SortPa
       const int32_t o = __shfl_up(inc, d, kWave);
       if (lane >= d) inc += o;
     }
+    if (lane == kWave - 1) wave_total_s[wave] = inc;
+    __syncthreads();
     int32_t excl = below_s + inc - sum;
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) excl += w < wave ? wave_total_s[w] : 0;
     for (int i = 0; i < per; ++i) {
       const int b = b0 + i;
       if (b < a.width) {
@@ -317,7 +322,7 @@ static bool make_plan(int64_t P, int64_t N, SortPlan* pl) {
   // What the scatter blocks of n tiles read of the histogram in all: n rows each, one block per tile and slice.
   auto rows_read = [&](int64_t of_tile, int64_t bins) { const int64_t n = (P + of_tile - 1) / of_tile; return n * n * slice_width((int)bins) * kSlices * 2; };
   // A second pass and the offsets kernel behind it cost about 20 us, as do 64 MB of rows: 32768 pairs over 16384 experts 37 us in two
-  // passes, 21 in one.
+  // passes, 18 in one.
   const bool wide = N + 1 > kMaxBins && N + 1 <= kMaxBinsWide && rows_read(tile, N + 1) <= (64ll << 20);
   if (N + 1 <= kMaxBins || wide) { pl->passes = 1; pl->lo_bits = 0; pl->bins[0] = (int)N + 1; pl->bins[1] = 0; }
   else {
