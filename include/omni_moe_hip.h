@@ -337,7 +337,8 @@ OMNI_API int32_t omni_router_fwd(const void* x, const void* weight_x, const void
  *   side_stream : NULL, or a second stream on which the router + expert branch is enqueued while the
  *                 MLP branch runs on `stream`; then fork_event and join_event must be two events of
  *                 the caller (hipEvent_t, timing disabled is fine); `stream` waits for the branch before
- *                 the final add, so after the call `stream` alone orders all later work.
+ *                 the final add, so after the call `stream` alone orders all later work.  16-bit calls of
+ *                 up to 2^33 tokens x H x I run joint launches on `stream` whether or not one is given.
  *   workspace   : omni_moe_workspace_bytes() bytes; must stay untouched until the work has run. */
 OMNI_API size_t omni_moe_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size,
                                          int64_t num_experts, int32_t num_expert_sqrt, int32_t num_experts_per_token,
