@@ -850,11 +850,14 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
     if (g.tiles_m % 4 == 0 && g.tiles_n % 8 == 0) { g.patch_m = 4; g.patch_n = 8; }
     else if (g.tiles_m % 8 == 0 && g.tiles_n % 4 == 0) { g.patch_m = 8; g.patch_n = 4; }
   }
+  // Loads straight to LDS take 16-byte pieces from 16-byte boundaries; operands that begin anywhere else (views into a flat buffer) are staged
+  // through registers.
+  const bool aligned = ((uintptr_t)g.a | (uintptr_t)g.b0 | (uintptr_t)g.b1) % 16 == 0;
   // 128-byte LDS rows (64-byte rows halve the fetch rate); as many ring stages as 160 KiB hold, up to 4
   constexpr int kDmaBK = 64;
   constexpr int kFit = (160 * 1024) / ((BM + BR) * kDmaBK * 2);
   constexpr int kDmaStages = kFit > 4 ? 4 : kFit;
-  if constexpr (DT != kF32 && EPI != kEpiSwiglu) if (g.K % kDmaBK == 0) {
+  if constexpr (DT != kF32 && EPI != kEpiSwiglu) if (g.K % kDmaBK == 0 && aligned) {
     constexpr int kDmaLds = kDmaStages * (BM + BR) * kDmaBK * 2;
     static_assert(kDmaLds <= 160 * 1024, "LDS ring exceeds 160 KiB");
     if constexpr (TM == 1 && TN == 1 && EPI != kEpiGate) {
@@ -887,7 +890,6 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
     constexpr int TB = EPI == kEpiSwiglu ? 2 : 1;
     const int64_t kt = (g.K + 31) / 32, tiles_m = (g.M + 31) / 32, small = tiles_m * ((g.N + 31) / 32);
     const int64_t tiled = (blocks + 255) / 256 * kt * (1024 * TM * TN + (blocks > 256 ? 450 : 900)), dealt = (small + 255) / 256 * ((kt + 3) / 4 * (1024 * TB + 450) + 2500);
-    const bool aligned = ((uintptr_t)g.a | (uintptr_t)g.b0 | (uintptr_t)g.b1) % 16 == 0;
     if (dealt < tiled && aligned && small < INT32_MAX && (int64_t)g.K * 128 < INT32_MAX && (EPI == kEpiSwiglu || !g.b1 || g.N % 64 == 0)) {
       GemmArgs d = g;
       d.tiles_m = (int)tiles_m;
@@ -897,7 +899,7 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
       return hipGetLastError();
     }
   }
-  auto kern = gemm_nt_kernel<DT, TM, TN, EPI>;       // any K % 8 == 0: staged through registers
+  auto kern = gemm_nt_kernel<DT, TM, TN, EPI>;       // any K % 8 == 0, any address: staged through registers
   if (hipError_t e = StagedKernelLds<DT, TM, TN, EPI>::entry.ensure(); e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(kGemmThreads), kLds, s, g);
   return hipGetLastError();

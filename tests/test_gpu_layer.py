@@ -434,6 +434,38 @@ def test_linear_matches_matmul(case, dtype, device):
     assert torch.equal(got_r, (got.float() + res.float()).to(dtype))
 
 
+def _elsewhere(t, device):
+    """t's values, contiguous, from one element past a 16-byte boundary on: a parameter that is a view into a flat buffer."""
+    flat = torch.empty(t.numel() + 1, device=device, dtype=t.dtype)
+    out = flat[1:].view(t.shape)
+    out.copy_(t)
+    assert out.is_contiguous() and out.data_ptr() % 16 == t.element_size()
+    return out
+
+
+# few 64 x 64 tiles and long K, more of them than CUs, 128 x 128 and 256 x 256 tiles, each with K in whole tiles of 64
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("case", [(130, 72, 640), (1100, 1024, 128), (3300, 1024, 512), (4100, 4096, 128)], ids=lambda c: f"M{c[0]}-N{c[1]}-K{c[2]}")
+def test_linear_takes_operands_at_any_address(case, dtype, device):
+    """Each operand in turn, and all of them, one element past a 16-byte boundary: one rounding of an fp32 sum, as test_linear_matches_matmul states it,
+    and with a residual a second one."""
+    M, N, K = case
+    g = torch.Generator(device=device).manual_seed(M + K)
+    x = torch.randn(M, K, device=device, generator=g).to(dtype)
+    w = (torch.randn(N, K, device=device, generator=g) * 0.05).to(dtype)
+    res = torch.randn(M, N, device=device, generator=g).to(dtype)
+    print(f"linear off the boundary M={M} N={N} K={K} {dtype}", flush=True)
+    want = x.double() @ w.double().t()
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -23}[dtype]
+    noise = 1e-4 if dtype != torch.float32 else 8 * 2.0 ** -24 * K ** 0.5
+    for which in ((0,), (1,), (2,), (0, 1, 2)):
+        xo, wo, ro = (_elsewhere(t, device) if i in which else t for i, t in enumerate((x, w, res)))
+        got = _ops().hip_linear_func(xo, wo)
+        assert ((got.double() - want).abs() <= ulp * want.abs() * 1.01 + noise * want.abs().max()).all(), which
+        both = _ops().hip_linear_func(xo, wo, residual=ro).double() - (want + res.double())
+        assert (both.abs() <= ulp * (want.abs() + (want + res.double()).abs()) * 1.01 + noise * want.abs().max()).all(), which
+
+
 # (M, columns per weight matrix, K): streaming kernel (second matrix = whole tiles), K tiles dealt out over the waves, ring kernel, staged kernel
 LINEAR2_CASES = [(8192, 512, 256), (16384, 256, 128), (1000, 52, 512), (3000, 200, 192), (300, 36, 40)]
 
