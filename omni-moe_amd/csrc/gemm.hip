@@ -965,8 +965,13 @@ static int gemm_swiglu(const void* x, const void* wg, const void* wu, void* h, i
   if (int e = check_gemm(M, I, K, ElemBytes<DT>::value)) return e;
   if (M == 0) return OMNI_OK;
   hipError_t err;
+  if (save_gate && (DT == kF32 || I % 8 || ((uintptr_t)h | (uintptr_t)save_gate | (uintptr_t)save_up) % 16)) return OMNI_ERR_UNSUPPORTED;
   if (tile_gemm(DT, kTileSwiglu, x, wg, wu, nullptr, h, save_gate, save_up, M, I, K, ws, ws_bytes, exclusive, s, &err)) return to_code(err);
-  if (save_gate) return OMNI_ERR_UNSUPPORTED;
+  if (save_gate) {     // operands at any other address, or out of the tile GEMM's reach: the two projections by themselves, and their product
+    if (int e = gemm_plain<DT>(x, wg, nullptr, nullptr, save_gate, M, I, K, s)) return e;
+    if (int e = gemm_plain<DT>(x, wu, nullptr, nullptr, save_up, M, I, K, s)) return e;
+    return omni_swiglu_fwd(save_gate, save_up, h, M * I, DT, s);
+  }
   GemmArgs g{(const uint8_t*)x, (const uint8_t*)wg, (const uint8_t*)wu, nullptr, (uint8_t*)h, (int)M, (int)I, (int)K, 0, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr};
   return to_code(launch_gemm<DT, 2, 2, kEpiSwiglu>(g, s));
 }

@@ -213,7 +213,7 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     const Tensor x2 = x.view({T, l.H});
     const Tensor e = expert_forward(x2, up, down, r.gates, r.ids, OMNI_EXPERT_ALGO_AUTO);
     Tensor h = at::empty({T, l.I}, x.options()), gate = at::empty({T, l.I}, x.options()), upp = at::empty({T, l.I}, x.options());
-    if (dt != OMNI_F32) {                          // (rows of 16 bytes, so both sizes are multiples of 8)
+    if (dt != OMNI_F32) {                          // (rows of 16 bytes, so both sizes are multiples of 8; operands at any address)
       check(omni_swiglu_linear_save_fwd(ptr(x), ptr(wg), ptr(wu), ptr(h), ptr(gate), ptr(upp), T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_swiglu_linear_save_fwd");
     } else {
       check(omni_linear_fwd(ptr(x), ptr(wg), nullptr, ptr(gate), T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_linear_fwd");

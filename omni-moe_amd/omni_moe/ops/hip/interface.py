@@ -376,7 +376,7 @@ def hip_swiglu_bwd_func(dout, gate, up):
 
 
 def _swiglu_linear_save_covers(x, gate_weight) -> bool:
-    """Shapes the saving form of the fused gate/up GEMM takes (omni_swiglu_linear_save_fwd)."""
+    """Shapes the saving form of the fused gate/up GEMM takes (omni_swiglu_linear_save_fwd), at any address of x and the weights."""
     return x.dtype in (torch.bfloat16, torch.float16) and gate_weight.size(0) % 8 == 0 and x.size(1) % 8 == 0
 
 

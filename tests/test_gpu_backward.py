@@ -199,6 +199,47 @@ def test_swiglu_linear_save_keeps_gate_and_up(shape, dtype, device):
                                                    T, H, I - 4, _lib.DTYPE_CODE[dtype], None) == _lib.ERR_UNSUPPORTED
 
 
+def _elsewhere(t, device):
+    """t's values, contiguous, from one element past a 16-byte boundary on: a view into a flat buffer."""
+    flat = torch.empty(t.numel() + 1, device=device, dtype=t.dtype)
+    out = flat[1:].view(t.shape)
+    out.copy_(t)
+    assert out.is_contiguous() and out.data_ptr() % 16 == t.element_size()
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", [(192, 128, 256), (77, 72, 136), (2100, 512, 1024)], ids=lambda s: "T%d-H%d-I%d" % s)
+def test_swiglu_linear_save_takes_operands_at_any_address(shape, dtype, device):
+    """x or a weight matrix off a 16-byte boundary: gate and up are one rounding of an fp32 sum, h is the SwiGLU operator's product of those two; the
+    differentiable MLP operator takes such operands too.  Outputs have to be aligned."""
+    from omni_moe.ops.hip import _lib
+    T, H, I = shape
+    g = torch.Generator(device=device).manual_seed(12)
+    x = torch.randn(T, H, device=device, generator=g).to(dtype)
+    wg, wu = ((torch.randn(I, H, device=device, generator=g) * H ** -0.5).to(dtype) for _ in range(2))
+    wd = (torch.randn(H, I, device=device, generator=g) * I ** -0.5).to(dtype)
+    dy = torch.randn(T, H, device=device, generator=g).to(dtype)
+    hip, lib, dt = _ops(), _lib.load(), _lib.DTYPE_CODE[dtype]
+    want = [x.double() @ w.double().t() for w in (wg, wu)]
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    print(f"saving gate/up off the boundary {shape} {dtype}", flush=True)
+    for which in ((0,), (1,), (2,), (0, 1, 2)):
+        a = [_elsewhere(t, device) if i in which else t for i, t in enumerate((x, wg, wu))]
+        h, gate, up = (torch.full((T, I), float("nan"), device=device, dtype=dtype) for _ in range(3))
+        _lib.check(lib.omni_swiglu_linear_save_fwd(*(t.data_ptr() for t in (*a, h, gate, up)), T, H, I, dt, _lib.stream_ptr()), "omni_swiglu_linear_save_fwd")
+        for got, w in zip((gate, up), want):
+            assert ((got.double() - w).abs() <= ulp * w.abs() * 1.01 + 1e-4 * w.abs().max()).all(), which
+        assert torch.equal(h, hip.hip_swiglu_func(gate, up)), which
+        assert lib.omni_swiglu_linear_save_fwd(*(t.data_ptr() for t in (*a, _elsewhere(h, device), gate, up)), T, H, I, dt, _lib.stream_ptr()) == _lib.ERR_UNSUPPORTED
+    leaves = [_elsewhere(t, device).requires_grad_() for t in (x, wg, wu, wd)]
+    hip.hip_omni_mlp_func(*leaves).backward(dy)
+    cl = [t.double().cpu().requires_grad_() for t in (x, wg, wu, wd)]
+    oracle.mlp_forward(*cl).backward(dy.double().cpu())
+    for leaf, c, what in zip(leaves, cl, ("dx", "dgate_weight", "dup_weight", "ddown_weight")):
+        _close(leaf.grad, c.grad, dtype, what)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 def test_mlp_func_autograd(dtype, device):
     """The differentiable MLP op (three GEMMs around the SwiGLU function) against fp64 autograd; its forward
@@ -281,6 +322,66 @@ def test_layer_backward_matches_oracle_autograd(training, device):
     _close(dx_in.grad, cx.grad, tol, "dx")
     for n in names:
         _close(getattr(layer, n).weight.grad, cw[n].grad, tol, f"d{n}")
+
+
+def _layer_reference(layer, x, dy, training):
+    """Output and gradients of the layer in 64 bits (autograd of the reference's composition, omni_moe.py:64-104), for a layer that selects every expert
+    (top-k = keys squared), so that no rounding can change the choice."""
+    names = ("gate_proj", "up_proj", "down_proj", "router_gate_x", "router_gate_y", "up_embed", "down_embed")
+    cw = {n: getattr(layer, n).weight.detach().double().requires_grad_() for n in names}
+    cx = x.detach().double().requires_grad_()
+    xf = cx.view(-1, cx.size(-1))
+    assert layer.top_k == layer.num_expert_sqrt ** 2 == layer.num_experts
+
+    def half(weight, norm):
+        z = xf @ weight.t()
+        mean, var = (z.mean(0), z.var(0, unbiased=False)) if training else (norm.running_mean.double(), norm.running_var.double())
+        return torch.log_softmax((z - mean) / torch.sqrt(var + norm.eps), -1)
+
+    lx, ly = half(cw["router_gate_x"], layer.router_norm_x), half(cw["router_gate_y"], layer.router_norm_y)
+    gates = torch.exp((lx.unsqueeze(2) + ly.unsqueeze(1)).flatten(1))                          # [T, N]: expert ix * r + iy
+    y = (torch.nn.functional.silu(xf @ cw["gate_proj"].t()) * (xf @ cw["up_proj"].t())) @ cw["down_proj"].t()
+    y = y + (torch.nn.functional.silu(xf @ cw["up_embed"].t()) * gates) @ cw["down_embed"]
+    y.backward(dy.double().view_as(y))
+    return y.detach().view_as(cx), {"x": cx.grad, **{n: cw[n].grad for n in names}}
+
+
+LAYER_NODE_CASES = [  # T, H, I; what lies off a 16-byte boundary
+    (300, 128, 256, ("x",)), (300, 128, 256, ("gate_proj",)), (300, 128, 256, ("up_proj",)), (300, 128, 256, ("down_proj",)), (300, 72, 264, ("x", "weights"))]
+
+
+@pytest.mark.parametrize("training", [True, False], ids=["train", "eval"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", LAYER_NODE_CASES, ids=lambda c: "T%d-H%d-I%d-%s" % (*c[:3], "+".join(c[3]) or "aligned"))
+def test_layer_16_bit_gradients(case, dtype, training, device):
+    """The 16-bit layer's differentiable node: output and every gradient against 64 bits.  Each is a sum over many values that were rounded to the
+    storage type a handful of times (projections, normalisation, scores, gates and their gradients): _tol of the largest value, five of its roundings."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, H, I, off = case
+    print(f"layer node T={T} H={H} I={I} {dtype} training={training} off the boundary: {off}", flush=True)
+    g = torch.Generator(device=device).manual_seed(T + H)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", 16, 16)).to(device=device, dtype=dtype).train(training)
+    with torch.no_grad():
+        for n, p in layer.named_parameters():
+            p.normal_(0.0, p.size(1) ** -0.5, generator=g)
+            if n.split(".")[0] in off or "weights" in off:
+                p.data = _elsewhere(p, device)
+        for norm in (layer.router_norm_x, layer.router_norm_y):
+            norm.running_mean.normal_(0.0, 0.3, generator=g)
+            norm.running_var.uniform_(0.5, 2.0, generator=g)
+    x = torch.randn(1, T, H, device=device, generator=g).to(dtype)
+    x = (_elsewhere(x, device) if "x" in off else x).requires_grad_()
+    dy = torch.randn(1, T, H, device=device, generator=g).to(dtype)
+    want_y, want = _layer_reference(layer, x, dy, training)
+    y = layer(x)
+    y.backward(dy)
+    got = {"x": x.grad, **{n: getattr(layer, n).weight.grad for n in want if n != "x"}}
+    for n, a, w in [("y", y.detach(), want_y)] + [(n, got[n], want[n]) for n in want]:
+        assert a.dtype == dtype and a.shape == w.shape
+        err = (a.double() - w).abs().max().item() / w.abs().max().item()
+        print(f"   {n}: {err:.2e}")
+        assert err <= _tol(dtype), (n, err)
+    assert layer.router_norm_x.num_batches_tracked.item() == int(training)
 
 
 def test_layer_trains_bf16(device):
