@@ -285,8 +285,8 @@ OMNI_API int32_t omni_router_norm_bwd_padded(const void* dgates, const void* gat
  *   dz : NULL, or [T][2][rp] from omni_router_norm_bwd_padded, with router_weight_x/y [r,H] (num_expert_sqrt = r; 0 without dz)
  *   dx_addend : NULL, or [T,H] added to d(x) after its rounding (the expert op's d(x)), and the sum rounded again
  *   dx [T,H], dgate_weight, dup_weight [I,H], ddown_weight [H,I], drouter_weight_x/y [r,H]: outputs, fully overwritten; NULL where not wanted
- * fp32 sums on the matrix cores, one rounding per output.  bf16 / f16; H and I multiples of 8, at least one token; fp32, and operands of 2 GiB and
- * more, return OMNI_ERR_UNSUPPORTED with nothing enqueued. */
+ * fp32 sums on the matrix cores, one rounding per output.  bf16 / f16; H and I multiples of 8, at least one token; fp32, pointers that are not
+ * 16-byte aligned and operands of 2 GiB and more return OMNI_ERR_UNSUPPORTED with nothing enqueued. */
 OMNI_API size_t omni_mlp_bwd_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t num_expert_sqrt, int32_t dtype);
 OMNI_API int32_t omni_mlp_bwd(const void* dy, const void* x, const void* gate_weight, const void* up_weight, const void* down_weight, const void* gate,
                               const void* up, const void* h, const void* dz, const void* router_weight_x, const void* router_weight_y,

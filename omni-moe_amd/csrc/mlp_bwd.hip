@@ -41,7 +41,11 @@ extern "C" OMNI_API int32_t omni_mlp_bwd(const void* dy, const void* x, const vo
   if (!dy || !x || !gate_weight || !up_weight || !down_weight || !gate || !up || !h) return OMNI_ERR_NULL;
   if (dz ? (r == 0 || !router_weight_x || !router_weight_y) : (drouter_weight_x || drouter_weight_y)) return OMNI_ERR_NULL;
   if (!workspace) return OMNI_ERR_WORKSPACE;
-  // every operand within reach of the kernel's 31-bit offsets (2 GiB), before anything is enqueued
+  // What the tile GEMM asks of its operands, before anything is enqueued: 16-byte aligned (dy, for one, may be a view that autograd cut out of a flat
+  // gradient at any offset), and within reach of 31-bit offsets (2 GiB)
+  for (const void* q : {dy, x, gate_weight, up_weight, down_weight, gate, up, h, dz, router_weight_x, router_weight_y, dx_addend, (const void*)dx, (const void*)dgate_weight,
+                        (const void*)dup_weight, (const void*)ddown_weight, (const void*)drouter_weight_x, (const void*)drouter_weight_y, (const void*)workspace})
+    if ((uintptr_t)q % 16) return OMNI_ERR_UNSUPPORTED;
   if (T * (I > H ? I : H) * 2 > INT32_MAX || H * I * 2 > INT32_MAX || T * 4 * ((r + 7) / 8 * 8) > INT32_MAX) return OMNI_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
   uint8_t* dgate = (uint8_t*)workspace;

@@ -275,7 +275,7 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
         return out;
       }
     }
-    // single precision, and operands of 2 GiB and more: library products
+    // single precision, operands off a 16-byte boundary, and operands of 2 GiB and more: library products
     Tensor dx = dx_experts;
     if (router) {
       const Tensor zx = dz.narrow(1, 0, r), zy = dz.narrow(1, rp, r);

@@ -97,6 +97,17 @@ def test_argument_errors_need_no_gpu():
         assert lib.omni_init() >= 1000           # a HIP error (no device), not a crash
 
 
+def test_mlp_bwd_refuses_unaligned_pointers():
+    """Each pointer of omni_mlp_bwd in turn two bytes past a 16-byte boundary: refused before anything is enqueued."""
+    lib = _lib().load()
+    call = lambda ptrs, ws=4096: lib.omni_mlp_bwd(*ptrs, 64, 64, 64, 8, 0, ws, None)
+    for i in range(18):
+        ptrs = [4096] * 18
+        ptrs[i] += 2
+        assert call(ptrs) == -5, i
+    assert call([4096] * 18, ws=4098) == -5
+
+
 def test_schedule_token_id_division_is_exact():
     """The schedule writes sorted_token_ids = pair_id // top_k as (pair_id * ceil(2^s / top_k)) >> s with
     s = 30 + ceil(log2(top_k)) (schedule.hip); the entry points admit pair ids below 2^30.  Within that bound the

@@ -347,7 +347,8 @@ def _layer_reference(layer, x, dy, training):
 
 
 LAYER_NODE_CASES = [  # T, H, I; what lies off a 16-byte boundary
-    (300, 128, 256, ("x",)), (300, 128, 256, ("gate_proj",)), (300, 128, 256, ("up_proj",)), (300, 128, 256, ("down_proj",)), (300, 72, 264, ("x", "weights"))]
+    (300, 128, 256, ("x",)), (300, 128, 256, ("gate_proj",)), (300, 128, 256, ("up_proj",)), (300, 128, 256, ("down_proj",)), (300, 128, 256, ("router_gate_x",)),
+    (300, 128, 256, ("dy",)), (300, 72, 264, ("x", "weights", "dy"))]
 
 
 @pytest.mark.parametrize("training", [True, False], ids=["train", "eval"])
@@ -374,7 +375,14 @@ def test_layer_16_bit_gradients(case, dtype, training, device):
     dy = torch.randn(1, T, H, device=device, generator=g).to(dtype)
     want_y, want = _layer_reference(layer, x, dy, training)
     y = layer(x)
-    y.backward(dy)
+    if "dy" in off:                                               # the layer's part of a flat gradient, behind one element of another tensor's
+        seen = []
+        y.register_hook(lambda t: seen.append(t.data_ptr() % 16))
+        one = torch.zeros(1, device=device, dtype=dtype)
+        torch.cat([one, y.flatten()]).backward(torch.cat([one, dy.flatten()]))
+        assert seen == [2]
+    else:
+        y.backward(dy)
     got = {"x": x.grad, **{n: getattr(layer, n).weight.grad for n in want if n != "x"}}
     for n, a, w in [("y", y.detach(), want_y)] + [(n, got[n], want[n]) for n in want]:
         assert a.dtype == dtype and a.shape == w.shape
