@@ -27,8 +27,6 @@ namespace omni {
 
 constexpr int kBwdWavesPerBlock = 4;
 
-__device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
-
 // ---- router ------------------------------------------------------------------------------------
 // One wave per token; lane l accumulates columns l, l+64, ... of both halves (r <= 64 * kCols).
 template <int DT, int kCols>

@@ -114,7 +114,8 @@ __device__ __forceinline__ void load_to_lds(uint64_t base, int bytes, uint32_t l
 __device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 template <int N> __device__ __forceinline__ void vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// x*sigmoid(x) in fp32, IEEE division.
+// sigmoid(x), x*sigmoid(x) in fp32, IEEE division.
+__device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
 __device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + __expf(-x)); }
 // Same with the hardware reciprocal (1 ulp) and exp2: ~6 instructions.  For results that are
 // rounded to a 16-bit type straight away.

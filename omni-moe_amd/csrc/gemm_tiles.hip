@@ -105,7 +105,7 @@ __device__ __forceinline__ void swiglu_bwd_word(const uint32_t o, const uint32_t
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const float d = e ? hi16<DT>(o) : lo16<DT>(o), gt = e ? hi16<DT>(gq) : lo16<DT>(gq), upv = e ? hi16<DT>(uq) : lo16<DT>(uq);
-    const float sig = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gt * -1.4426950408889634f)), silu = gt * sig;
+    const float sig = sigmoid_f32(gt), silu = gt * sig;
     g2[e] = d * (silu * (1.0f - sig) + sig) * upv;
     u2[e] = d * silu;
   }
