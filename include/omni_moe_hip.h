@@ -194,7 +194,8 @@ OMNI_API int32_t omni_swiglu_linear_fwd_shared(const void* x, const void* gate_w
  *   gate_out, up_out [T,I]: x Wg^T and x Wu^T rounded to the storage dtype; h [T,I] their SwiGLU product.
  * bf16 / f16 only, intermediate_size a multiple of 8, 16-byte aligned h, gate_out and up_out; anything else returns
  * OMNI_ERR_UNSUPPORTED (use omni_linear_fwd twice and omni_swiglu_fwd).  hidden_size a multiple of 8 (else OMNI_ERR_SHAPE).
- * x and the weights at any address: one launch where they are 16-byte aligned, three where one of them is not. */
+ * x and the weights at any address: one launch where they are 16-byte aligned and hidden_size is a multiple of 64; otherwise h is omni_swiglu_fwd of
+ * the two projections, in a launch of its own. */
 OMNI_API int32_t omni_swiglu_linear_save_fwd(const void* x, const void* gate_weight, const void* up_weight, void* h,
                                              void* gate_out, void* up_out, int64_t num_tokens, int32_t hidden_size,
                                              int32_t intermediate_size, int32_t dtype, void* stream);

@@ -240,6 +240,21 @@ def test_swiglu_linear_save_takes_operands_at_any_address(shape, dtype, device):
         _close(leaf.grad, c.grad, dtype, what)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_swiglu_linear_save_divides_at_odd_hidden_sizes(dtype, device):
+    """Hidden sizes that are no multiple of 64: h is bit for bit the SwiGLU operator's product of the kept gate and up, as the differentiable MLP operator
+    forms it there (2 million values, of which the hardware reciprocal moves about 30 in f16)."""
+    from omni_moe.ops.hip.interface import OmniSwiGLULinearFunc
+    T, H, I = 2000, 520, 1048
+    g = torch.Generator(device=device).manual_seed(13)
+    x = torch.randn(T, H, device=device, generator=g).to(dtype).requires_grad_()
+    wg, wu = ((torch.randn(I, H, device=device, generator=g) * 2 * H ** -0.5).to(dtype) for _ in range(2))
+    h = OmniSwiGLULinearFunc.apply(x, wg, wu)
+    *_, gate, up = h.grad_fn.saved_tensors
+    want = _ops().hip_swiglu_func(gate, up)
+    assert torch.equal(h.detach(), want), (h.detach() != want).sum().item()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 def test_mlp_func_autograd(dtype, device):
     """The differentiable MLP op (three GEMMs around the SwiGLU function) against fp64 autograd; its forward
