@@ -10,6 +10,7 @@
 // it raises the errors that the operator contract names.
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/extension.h>
 
@@ -57,11 +58,24 @@ void* stream_of(const at::Device& dev) { return (void*)c10::hip::getCurrentHIPSt
 void* ptr(const Tensor& t) { return t.defined() && t.numel() ? t.data_ptr() : nullptr; }
 Tensor bytes(size_t n, const at::Device& dev) { return at::empty({(int64_t)(n ? n : 1)}, at::TensorOptions().dtype(at::kByte).device(dev)); }
 
-void check(int32_t code, const char* what) {
+// A HIP error keeps the type that the Python path raises for it, from the autograd engine's threads too: torch translates what derives from PyTorchError.
+PyObject* hip_error_type = nullptr;               // OmniHipError, handed over at load
+struct HipError : torch::PyTorchError {
+  using PyTorchError::PyTorchError;
+  PyObject* python_type() override { return hip_error_type ? hip_error_type : PyExc_RuntimeError; }
+};
+struct TopkError : torch::PyTorchError {
+  using PyTorchError::PyTorchError;
+  PyObject* python_type() override { return PyExc_AssertionError; }      // the reference asserts (utils.py:81-104)
+};
+
+void check(int32_t code, const std::string& what) {
   if (code == OMNI_OK) return;
-  const std::string text = std::string(what) + ": " + omni_error_string(code) + " (code " + std::to_string(code) + ")";
-  if (code < 0) TORCH_CHECK_VALUE(false, text);
-  TORCH_CHECK(false, text);
+  const std::string text = what + ": " + omni_error_string(code);
+  if (code == OMNI_ERR_TOPK) throw TopkError(text);
+  const std::string full = text + " (code " + std::to_string(code) + ")";
+  if (code < 0) TORCH_CHECK_VALUE(false, full);
+  throw HipError(full);
 }
 
 bool records(std::initializer_list<const Tensor*> ts) {
@@ -400,6 +414,8 @@ py::object layer_forward(py::handle self, const Tensor& x, const py::dict& algos
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("hip_error_type", [](py::object type) { hip_error_type = type.release().ptr(); });
+  m.def("check", &check);
   m.def("expert", &expert);
   m.def("router_select", &router_select);
   m.def("router_stage", &router_stage);

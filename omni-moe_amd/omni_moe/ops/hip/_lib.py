@@ -103,6 +103,7 @@ def native():
         spec = importlib.util.spec_from_file_location("_native", path)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        module.hip_error_type(OmniHipError)
         _native = module
     return _native
 

@@ -143,6 +143,21 @@ def test_ops_fail_loudly_without_gpu():
         hip.hip_omni_expert_func(torch.zeros(4, 8), torch.zeros(16, 8), torch.zeros(16, 8), torch.zeros(4, 2), torch.zeros(4, 2, dtype=torch.int32))
 
 
+def test_native_path_raises_the_types_of_the_python_path():
+    """What the native host path raises for a library code, and what _lib.check raises for it: the same type and text."""
+    lib = _lib()
+    native = lib.native()
+    native.check(0, "call")
+    for code in (-1, -2, -3, -4, -5, -6, -7, 1002, 1700):
+        with pytest.raises(Exception) as a:
+            lib.check(code, "call")
+        with pytest.raises(Exception) as b:
+            native.check(code, "call")
+        assert type(a.value) is type(b.value), code
+        assert str(b.value).splitlines()[0] == str(a.value), code
+    assert issubclass(lib.OmniHipError, RuntimeError) and type(b.value) is lib.OmniHipError
+
+
 def test_reference_import_paths():
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
     from omni_moe.ops.triton import triton_omni_expert_func, triton_omni_mlp_func, triton_omni_router_func  # noqa: F401
