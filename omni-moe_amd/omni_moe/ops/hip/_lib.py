@@ -2,14 +2,15 @@
 
 The library is loaded after ``import torch`` so that its HIP symbols bind to the HIP
 runtime torch has already loaded (same soname), which makes torch's streams and device
-pointers valid inside it.  There is no fallback: if the library is missing or a call
-is made without a GPU, an exception is raised.
+pointers valid inside it.  There is no fallback from its kernels: if the library is missing
+or a call is made without a GPU, an exception is raised.
 """
 from __future__ import annotations
 
 import ctypes
 import importlib.util
 import os
+import warnings
 from ctypes import c_char_p, c_float, c_int32, c_int64, c_size_t, c_void_p
 
 import torch  # noqa: F401  (must precede loading the library)
@@ -89,21 +90,32 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 _native = None
 
 
+class WithoutNative:
+    """Stands in for a host path that does not load: every entry answers None, as that one does to a call it does not take."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def native():
-    """The torch host path (csrc/torch_ops.cpp), loaded once; it links the library above."""
+    """The torch host path (csrc/torch_ops.cpp), loaded once; it links the library above.  If it does not load (missing, or built against another torch)
+    the operators go through Python to the same kernels, and say so once."""
     global _native
     if _native is None:
         load()
-        path = os.path.join(_HERE, "_native.so")
-        if not os.path.exists(path):
-            raise OmniHipError(f"{path} is missing: build it with `python -m omni_moe.ops.hip.build`")
-        spec = importlib.util.spec_from_file_location("_native", path)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        module.hip_error_type(OmniHipError)
+        try:
+            spec = importlib.util.spec_from_file_location("_native", NATIVE_PATH)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            module.hip_error_type(OmniHipError)
+        except ImportError as e:
+            warnings.warn(f"{NATIVE_PATH} does not load ({e}): operator calls take more host time; build it with `python -m omni_moe.ops.hip.build`",
+                          RuntimeWarning, stacklevel=3)
+            module = WithoutNative()
         _native = module
     return _native
 

@@ -158,6 +158,20 @@ def test_native_path_raises_the_types_of_the_python_path():
     assert issubclass(lib.OmniHipError, RuntimeError) and type(b.value) is lib.OmniHipError
 
 
+def test_host_path_that_does_not_load_leaves_the_python_path(tmp_path, monkeypatch):
+    """Missing, or not a library that this interpreter can load: one warning, and every entry answers None from then on."""
+    lib = _lib()
+    broken = tmp_path / "_native.so"
+    broken.write_bytes(b"not a library")
+    for path in (tmp_path / "missing.so", broken):
+        monkeypatch.setattr(lib, "NATIVE_PATH", str(path))
+        monkeypatch.setattr(lib, "_native", None)
+        with pytest.warns(RuntimeWarning, match="does not load"):
+            native = lib.native()
+        assert native.layer_forward(None, None, {}) is None and native.mlp(1, 2, 3, 4, None) is None
+        assert lib.native() is native
+
+
 def test_reference_import_paths():
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
     from omni_moe.ops.triton import triton_omni_expert_func, triton_omni_mlp_func, triton_omni_router_func  # noqa: F401

@@ -393,6 +393,29 @@ def test_layer_takes_noncontiguous_weights(device):
     assert torch.equal(layer(x), want)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_layer_without_the_native_host_path(dtype, device, monkeypatch):
+    """The Python path behind the native one reaches the same kernels: equal bits in both norm modes, and gradients for every parameter."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    from omni_moe.ops.hip import _lib
+    torch.manual_seed(6)
+    layer = OmniMoE(OmniMoEConfig(128, 256, "silu", 256, 8)).to(device=device, dtype=dtype)
+    fresh = {n: b.clone() for n, b in layer.named_buffers()}
+    x = torch.randn(1, 300, 128, device=device).to(dtype)
+
+    def both_modes():
+        for n, b in layer.named_buffers():
+            b.copy_(fresh[n])
+        return [layer.train(mode)(x) for mode in (True, False)]
+
+    want = both_modes()
+    monkeypatch.setattr(_lib, "_native", _lib.WithoutNative())
+    assert all(torch.equal(a, b) for a, b in zip(want, both_modes()))
+    with torch.enable_grad():
+        layer(x).float().square().sum().backward()
+    assert all(p.grad is not None and torch.isfinite(p.grad).all() for p in layer.parameters())
+
+
 def test_add_inplace(device):
     hip = _ops()
     for dtype in (torch.bfloat16, torch.float16, torch.float32):
