@@ -147,8 +147,9 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   //     better overlap: projection | gate/up, selection | down projection, experts and add.
   const size_t h_bytes = up256(T * (size_t)intermediate_size * es);
   const bool few = few_tokens_covers_layer(num_tokens, hidden_size, intermediate_size, num_expert_sqrt, num_experts_per_token, dtype);
+  //     (rows within reach of the tile kernels' 31-bit offsets, as few_tokens_covers bounds them; the two launches of the general path have no such bound)
   const bool joint = dtype != OMNI_F32 && num_experts_per_token > 0 && num_expert_sqrt % 8 == 0 && hidden_size % 8 == 0 && intermediate_size % 8 == 0 &&
-                     (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0;
+                     intermediate_size <= (1 << 20) && (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0;
   // (batch statistics: the projection and their merge stay launches of their own; a cumulative average, momentum < 0, is counted by the select kernel)
   if ((training ? joint && momentum >= 0.f : few || joint) && num_experts <= UINT32_MAX &&
       resolve_algo(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) == OMNI_EXPERT_ALGO_GATHER) {

@@ -731,3 +731,22 @@ def test_joint_launches_match_the_operators(case, dtype, device):
     assert all(torch.equal(a, b) for a, b in zip(after, layer.buffers()))
     experts = ops.hip_omni_expert_func(x[0], layer.up_embed.weight, layer.down_embed.weight, gates, ids).double()
     assert (got - (mlp + experts)).abs().max().item() <= 4 * eps * max(1.0, float((mlp + experts).abs().max()))
+
+
+def test_layer_with_rows_beyond_the_tile_kernels_reach(device):
+    """An intermediate size whose rows put 256 of them beyond 2 GiB: no joint launch, and the result of the operators one by one (MLP in 64 bits)."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, H, I, N, k = 65, 8, 4194312, 64, 2
+    print(f"layer T={T} H={H} I={I}", flush=True)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", N, k)).to(device=device, dtype=torch.bfloat16).eval()
+    g = torch.Generator(device=device).manual_seed(7)
+    for p in layer.parameters():
+        p.normal_(0.0, p.size(1) ** -0.5, generator=g)
+    x = torch.randn(1, T, H, device=device, generator=g).bfloat16()
+    got = layer(x)[0].double()
+    experts = _ops().hip_omni_expert_func(x[0], layer.up_embed.weight, layer.down_embed.weight, *layer.route(x[0])).double()
+    xd, wg, wu, wd = (t.double() for t in (x[0], layer.gate_proj.weight, layer.up_proj.weight, layer.down_proj.weight))
+    h = (torch.nn.functional.silu((xd @ wg.t()).bfloat16().double()) * (xd @ wu.t()).bfloat16().double()).bfloat16().double()
+    want = h @ wd.t() + experts
+    # h rounds alike but for last bits here and there; the sum of 4 million products runs in 32 bits, over partial sums of one wave each
+    assert (got - want).abs().max().item() <= 4 * 2.0 ** -7 * max(1.0, want.abs().max().item())
