@@ -2,15 +2,18 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--sections a,b,...]
 
-Prints ONE JSON line.  A step = one forward of the OmniMoE layer over one batch of synthetic,
-HBM-resident input: benchmark config 4, the README shape (1 x 4096 tokens, hidden 1024,
-intermediate 4096, 4096 experts = 64 x 64 keys, top-16, bf16, train-mode BatchNorm).
+Prints ONE JSON line of at most 4 KiB (a reader may keep only so much of a line); --details FILE
+writes everything that was measured.  A step = one forward of the OmniMoE layer over one batch of
+synthetic, HBM-resident input: the README shape (1 x 4096 tokens, hidden 1024, intermediate 4096,
+4096 experts = 64 x 64 keys, top-16, bf16, train-mode BatchNorm), called config 4 below.
 All timing uses HIP events recorded on the stream the kernels run on (torch's current stream;
 the library enqueues there).
 
+In the line:
   value          whole-layer tokens/s over the K timed steps (one event pair around all K)
   step_ms        the same step timed one at a time with a freshly cloned input per repeat, as the
                  reference's harness does (tests/testing.py:152-212): median and best
+  grad_enabled_forward   the same call with autograd recording
   roofline       the kernel that takes the largest share of a step (gate/up MFMA GEMM); its
                  duration is the average over back-to-back launches between one event pair, so
                  that it matches what a kernel trace shows
@@ -18,14 +21,16 @@ the library enqueues there).
                          cache-resident: fraction of HBM peak from the bytes that really cross the fabric
   roofline_expert_hbm    the expert op at benchmark config 5's shape (2 GiB tables): HBM-resident, so
                          algorithmic bytes are HBM bytes
-  kernels        per-launch figures for every stage
   layer_c5       the whole layer at benchmark config 5 (32768 tokens, hidden 2048, intermediate 8192, 262144
                  experts, top-32, Zipf-skewed keys): step time, tokens/s and its three MFMA GEMMs
+  cpu_baseline   the oracle (the reference's PyTorch layer restated with torch CPU ops) on the
+                 host cores, same workload
+Only among the details:
+  kernels        per-launch figures for every stage, with what each counts and where its byte figures come from
+  mfma_probe     what the matrix cores sustain on register operands
   ref_grid       the shapes of the reference's own operator benchmarks (tests/test_router.py:103-110,
                  tests/test_expert.py:181-187, tests/test_mlp.py:144-150), each beside the same operator
                  composed from torch library ops on this GPU
-  cpu_baseline   the oracle (the reference's PyTorch layer restated with torch CPU ops) on the
-                 host cores, same workload
 
 Sections (default: all): layer, kernels, expert_c3, expert_c5, layer_c5, ref_grid, probe, train, cpu.
 """
@@ -148,6 +153,34 @@ def mfma_entry(name, flops, ms, best, traffic=None, sustained=None):
     return d
 
 
+#: What the printed line holds: keys of the full result, each whole (None) or the named parts of it.
+LINE = {**{k: None for k in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling", "vs_baseline", "dtype",
+                             "data", "config")},
+        "step_ms": ("median_single", "best_single", "repeats"), "grad_enabled_forward": ("ms_per_step", "tokens_per_s"),
+        **{k: ("kernel", "bound", "achieved", "peak", "unit", "frac", "kernel_ms", "traffic", "frac_of_sustained", "frac_compulsory", "library_gemm_same_flops_ms")
+           for k in ("roofline", "roofline_expert", "roofline_expert_hbm")},
+        "layer_c5": ("ms_per_step", "tokens_per_s", "frac_of_mfma_peak"), "cpu_baseline": None}
+LINE_BYTES = 4096
+
+
+def short(v):
+    """Floats to seven figures: more than a timing has, and half the text."""
+    if isinstance(v, dict):
+        return {k: short(x) for k, x in v.items()}
+    return float(f"{v:.7g}") if isinstance(v, float) else v
+
+
+def headline(out):
+    """The printed line: the entries of LINE that were measured."""
+    line = {}
+    for key, parts in LINE.items():
+        if key in out:
+            line[key] = short(out[key] if parts is None else {p: out[key][p] for p in parts if p in out[key]})
+    text = json.dumps(line)
+    assert len(text) <= LINE_BYTES, len(text)
+    return text
+
+
 def cpu_model():
     try:
         for line in open("/proc/cpuinfo"):
@@ -165,6 +198,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=100,
                     help="untimed steps; the first ~100 steps after the GPU has idled run about 7 %% slower (clocks ramp up)")
     ap.add_argument("--sections", default=",".join(SECTIONS), help="comma-separated subset of: " + ", ".join(SECTIONS))
+    ap.add_argument("--details", metavar="FILE", help="also write every figure measured to FILE, as JSON")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-kernels", action="store_true", help="only the layer steps (profiling runs)")
     ap.add_argument("--calibration-copy", action="store_true",
@@ -206,8 +240,8 @@ def main():
         "value": None, "unit": "tokens/s", "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": None, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "bf16", "data": "synthetic",
-        "config": {"workload": "BASELINE.json configs[3] (benchmark config 4, the README shape): full OmniMoE layer forward, 1x4096 tokens, hidden 1024, intermediate 4096, "
-                               "4096 experts (64x64), top-16, silu, train-mode BatchNorm, seed 3"},
+        "config": {"model": f"OmniMoE layer forward: hidden {H}, intermediate {I}, {N} experts (64x64 keys), top-{k}, silu, train-mode BatchNorm, seed {seed}",
+                   "global_batch": 1, "seq_len": T, "parallelism": "one GPU"},
     }
 
     for _ in range(a.warmup):
@@ -243,12 +277,12 @@ def main():
                           "protocol": "single: fresh cloned input, synchronise, events around one call (reference tests/testing.py:152-212); "
                                       "back_to_back: the K timed steps between one event pair"}
         # the layer exactly as the reference's README calls it: grad enabled, parameters requiring grad
-        # (the differentiable composition of the operators, not the single fused call)
+        # (one differentiable node, not the single fused call)
         with torch.enable_grad():
             g_med, g_best = time_launches(torch, lambda: layer(dx), n=20, reps=5, warmup=3)
         out["grad_enabled_forward"] = {"ms_per_step": g_med, "ms_per_step_best": g_best, "tokens_per_s": T / (g_med * 1e-3),
-                                       "note": "moe(x) with autograd recording (README quick start): router stage, expert op and MLP op as "
-                                               "differentiable nodes; the gate/up GEMM also stores gate and up for the backward pass"}
+                                       "note": "moe(x) with autograd recording (README quick start), as one differentiable node; the gate/up GEMM "
+                                               "also stores gate and up for the backward pass"}
 
         # correctness spot check against the oracle (outside the timed region): eval mode on both
         # sides so that the repeated train-mode steps above do not matter
@@ -318,9 +352,9 @@ def main():
         m_lib, b_lib = time_launches(torch, lambda: torch.matmul(h, layer.down_proj.weight.t()))
         del wcat
         m, b = time_launches(torch, lambda: hip.hip_linear_func(h, layer.down_proj.weight, e_out))
-        kernels.append(mfma_entry("gemm_nt_dma_kernel<residual> (down projection + experts add), c4", 2 * T * H * I, m, b, TRAFFIC_BYTES["down_c4"], sustained32))
+        kernels.append(mfma_entry("gemm_tiles_kernel<residual> (down projection + experts add), c4", 2 * T * H * I, m, b, TRAFFIC_BYTES["down_c4"], sustained))
         m, b = time_launches(torch, lambda: hip.hip_linear_func(h, layer.down_proj.weight))
-        kernels.append(mfma_entry("gemm_nt_dma_kernel<plain> (down projection alone, as on the two-stream path), c4", 2 * T * H * I, m, b, TRAFFIC_BYTES["down_plain_c4"], sustained32))
+        kernels.append(mfma_entry("gemm_tiles_kernel<plain> (down projection alone, as on the two-stream path), c4", 2 * T * H * I, m, b, TRAFFIC_BYTES["down_plain_c4"], sustained))
         kernels[-1]["library_gemm_same_flops_ms"] = m_lib
         m, b = time_launches(torch, lambda: hip.hip_add_inplace_func(y0, e_out))
         kernels.append(hbm_entry("add_inplace_kernel (join of the two branches), c4", m, b, 3 * T * H * 2, resident_in_hbm=False,
@@ -505,7 +539,7 @@ def main():
         e_d["library_gemm_same_flops_ms"] = m_lib
         m_rt, b_rt = time_launches(torch, router_stage_call(torch, _lib, layer5, xf5, False), n=5, reps=5, warmup=2)
         kernels += [e_gu, e_d, e_r]
-        out["layer_c5"] = {"workload": "BASELINE.json configs[4] (benchmark config 5): full OmniMoE layer forward, 8x4096 tokens, hidden 2048, intermediate 8192, "
+        out["layer_c5"] = {"workload": "benchmark config 5: full OmniMoE layer forward, 8x4096 tokens, hidden 2048, intermediate 8192, "
                                        "262144 experts (512x512), top-32, eval-mode BatchNorm whose buffers carry the Zipf(1.1) key bias, seed 4",
                            "ms_per_step": per_algo["auto"]["ms_per_step"], "tokens_per_s": per_algo["auto"]["tokens_per_s"],
                            "with_expert_algo_gather": per_algo["gather"], "on_two_streams": {"ms_per_step": m2, "ms_per_step_best": b2},
@@ -593,7 +627,10 @@ def main():
                                "host_logical_cpus": os.cpu_count(), "cpu_model": cpu_model(),
                                "sample": f"{reps} forwards of the whole workload (4096 tokens) in {dt:.1f} s, bf16 torch CPU ops on "
                                          f"{torch.get_num_threads()} threads (oracle restatement of OmniMoE_Torch.forward)"}
-    print(json.dumps(out))
+    if a.details:
+        with open(a.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(headline(out))
 
 
 if __name__ == "__main__":
