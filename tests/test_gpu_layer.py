@@ -20,6 +20,15 @@ def _ops():
     return hip
 
 
+def _elsewhere(t, device):
+    """t's values, contiguous, from one element past a 16-byte boundary on: a parameter that is a view into a flat buffer."""
+    flat = torch.empty(t.numel() + 1, device=device, dtype=t.dtype)
+    out = flat[1:].view(t.shape)
+    out.copy_(t)
+    assert out.is_contiguous() and out.data_ptr() % 16 == t.element_size()
+    return out
+
+
 # the first four are the reference's benchmark grid (tests/test_mlp.py:144-150): intermediate 1024 .. 65536
 MLP_CASES = [(1024, 1024, 1024), (1024, 1024, 4096), (1024, 1024, 16384), (1024, 1024, 65536), (4096, 1024, 4096), (4100, 1024, 4096),
              (333, 256, 1000), (128, 64, 128), (512, 2048, 8192), (5, 8, 8),
@@ -332,20 +341,50 @@ def test_layer_expert_term_visible_auto_split(two_streams, dtype, training, devi
     torch.testing.assert_close(y.cpu().float()[same], want_y.view(-1, H).float()[same], rtol=tol, atol=tol * (e_scale + m_scale))
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
-def test_layer_two_streams_equals_one_stream(dtype, device):
+def _waits_for_side_stream(layer, x):
+    """Whether the call forks to the layer's side stream and joins it: what stands on that stream beforehand must then end before the call's work does."""
+    layer(x)                                                 # whatever a first call allocates and loads
+    side = layer._branch_resources(x.device)[0]
+    torch.cuda.synchronize()
+    before, after = torch.cuda.Event(), torch.cuda.Event()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(20_000_000)                        # (far longer than the call and its host work)
+        before.record()
+    layer(x)
+    after.record()
+    after.synchronize()
+    waited = before.query()
+    torch.cuda.synchronize()
+    return waited
+
+
+# T, H, I.  16 bits: up to 2^33 token x hidden x intermediate the calls are joint launches on one stream whatever the switches say; beyond it, and in
+# single precision and for operands off a 16-byte boundary at any size, they are the two schedules that the switches choose between.
+STREAM_CASES = [(torch.bfloat16, (300, 256, 512), True, False), (torch.bfloat16, (300, 256, 512), False, True), (torch.float32, (300, 256, 512), True, True),
+                (torch.bfloat16, (2100, 1024, 4096), True, True), (torch.float16, (2100, 1024, 4096), True, True)]
+
+
+@pytest.mark.parametrize("algo", ["gather", "split"])
+@pytest.mark.parametrize("case", STREAM_CASES, ids=lambda c: f"{str(c[0])[6:]}-T{c[1][0]}-H{c[1][1]}-I{c[1][2]}-{'aligned' if c[2] else 'off-boundary'}")
+def test_layer_two_streams_equals_one_stream(case, algo, device):
     """The two-stream schedule (router+experts beside the MLP, joined by omni_add_inplace) and the
     one-stream schedule (add fused into the down projection) give bit-identical output, call after call."""
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    dtype, (T, H, I), aligned, forks = case
     torch.manual_seed(0)
-    layer = OmniMoE(OmniMoEConfig(256, 512, "silu", 1024, 8)).to(device=device, dtype=dtype).eval()
-    layer.overlap_min_work = 0                    # two streams whatever the size
-    x = torch.randn(3, 100, 256, device=device).to(dtype)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", 1024, 8)).to(device=device, dtype=dtype).eval()
+    layer.expert_algo = algo
+    layer.overlap_min_work = 0                    # two streams at any size that has them
+    x = torch.randn(3, T // 3, H, device=device).to(dtype)
+    if not aligned:
+        x = _elsewhere(x, device)
     layer.overlap_branches = False
     ref = layer(x)
+    assert not _waits_for_side_stream(layer, x)
     layer.overlap_branches = True
     for _ in range(5):
         assert torch.equal(layer(x), ref)
+    assert _waits_for_side_stream(layer, x) == (forks or algo == "split")           # (the split algorithm has no joint launches)
     # and next to other work on the caller's stream
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
@@ -362,10 +401,10 @@ def test_layer_copies_and_saves_like_a_plain_module(device, tmp_path):
     import copy
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
     torch.manual_seed(3)
-    cfg = OmniMoEConfig(256, 512, "silu", 1024, 8)
+    cfg = OmniMoEConfig(1024, 4096, "silu", 1024, 8)
     layer = OmniMoE(cfg).to(device=device, dtype=torch.bfloat16).eval()
-    layer.overlap_min_work = 0
-    x = torch.randn(2, 200, 256, device=device).bfloat16()
+    x = torch.randn(2, 1100, 1024, device=device).bfloat16()             # beyond the joint launches: two streams
+    assert _waits_for_side_stream(layer, x)
     want = layer(x)
     twin = copy.deepcopy(layer)
     assert torch.equal(twin(x), want)
@@ -375,7 +414,6 @@ def test_layer_copies_and_saves_like_a_plain_module(device, tmp_path):
     assert torch.equal(loaded(x), want)
     fresh = OmniMoE(cfg).to(device=device, dtype=torch.bfloat16).eval()
     fresh.load_state_dict(layer.state_dict())
-    fresh.overlap_min_work = 0
     assert torch.equal(fresh(x), want)
     assert not any(isinstance(v, (torch.cuda.Stream, torch.cuda.Event)) for v in vars(layer).values())
 
@@ -457,15 +495,6 @@ def test_linear_matches_matmul(case, dtype, device):
     assert torch.equal(got_r, (got.float() + res.float()).to(dtype))
 
 
-def _elsewhere(t, device):
-    """t's values, contiguous, from one element past a 16-byte boundary on: a parameter that is a view into a flat buffer."""
-    flat = torch.empty(t.numel() + 1, device=device, dtype=t.dtype)
-    out = flat[1:].view(t.shape)
-    out.copy_(t)
-    assert out.is_contiguous() and out.data_ptr() % 16 == t.element_size()
-    return out
-
-
 # few 64 x 64 tiles and long K, more of them than CUs, 128 x 128 and 256 x 256 tiles, each with K in whole tiles of 64
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
 @pytest.mark.parametrize("case", [(130, 72, 640), (1100, 1024, 128), (3300, 1024, 512), (4100, 4096, 128)], ids=lambda c: f"M{c[0]}-N{c[1]}-K{c[2]}")
@@ -515,16 +544,20 @@ def test_linear_two_weight_matrices_equals_one(case, device):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("shape", [(150, 256, 512), (1100, 1024, 4096)], ids=["joint", "schedules"])
 @pytest.mark.parametrize("overlap", [True, False], ids=["two-streams", "one-stream"])
-def test_layer_is_graph_capturable(overlap, device):
+def test_layer_is_graph_capturable(overlap, shape, device):
     """The library only launches kernels and records/waits events, so a whole layer forward (fork and join
-    included) can be captured into a HIP graph; every replay, with eager work in between, equals the eager result."""
+    included) can be captured into a HIP graph; every replay, with eager work in between, equals the eager result.
+    The smaller shape is joint launches on one stream whatever the switches say."""
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
     torch.manual_seed(1)
-    layer = OmniMoE(OmniMoEConfig(256, 512, "silu", 1024, 8)).to(device=device, dtype=torch.bfloat16).eval()
+    T, H, I = shape
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", 1024, 8)).to(device=device, dtype=torch.bfloat16).eval()
     layer.overlap_branches = overlap
     layer.overlap_min_work = 0
-    x = torch.randn(2, 150, 256, device=device).bfloat16()
+    x = torch.randn(2, T, H, device=device).bfloat16()
+    assert _waits_for_side_stream(layer, x) == (overlap and T > 150)
     want = layer(x).clone()
     warm = torch.cuda.Stream()
     warm.wait_stream(torch.cuda.current_stream())
@@ -570,11 +603,13 @@ def test_layer_cumulative_batch_norm(device):
         layer(x.to(device))
 
 
+@pytest.mark.parametrize("aligned", [True, False], ids=["joint", "schedules"])
 @pytest.mark.parametrize("training", [True, False], ids=["train", "eval"])
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 31, 33, 65])
-def test_layer_tiny_token_counts(T, training, device):
+def test_layer_tiny_token_counts(T, training, aligned, device):
     """A handful of tokens (one wave, one partial strip, a single BatchNorm sample in training), on one and on two
-    streams: same tolerance as the big cases, and both schedules bit-identical."""
+    streams: same tolerance as the big cases, and both schedules bit-identical.  Aligned input of these sizes is joint launches either way;
+    input off a 16-byte boundary takes the two schedules."""
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
     H, I, N, k = 128, 256, 256, 8
     x, w = oracle.make_layer_inputs(T, T, H, I, N)
@@ -603,7 +638,10 @@ def test_layer_tiny_token_counts(T, training, device):
         layer = layer.to(device=device, dtype=torch.bfloat16).train(training)
         layer.overlap_branches = overlap
         layer.overlap_min_work = 0
-        outs.append(layer(x.to(device)))
+        xd = x.to(device) if aligned else _elsewhere(x, device)
+        outs.append(layer(xd))
+        if not training:
+            assert _waits_for_side_stream(layer, xd) == (overlap and not aligned)
     torch.testing.assert_close(outs[0].cpu().float(), want.float(), rtol=2e-2, atol=2e-2)
     assert torch.equal(outs[0], outs[1])
 
