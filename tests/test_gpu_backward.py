@@ -361,22 +361,25 @@ def _layer_reference(layer, x, dy, training):
     return y.detach().view_as(cx), {"x": cx.grad, **{n: cw[n].grad for n in names}}
 
 
-LAYER_NODE_CASES = [  # T, H, I; what lies off a 16-byte boundary
-    (300, 128, 256, ("x",)), (300, 128, 256, ("gate_proj",)), (300, 128, 256, ("up_proj",)), (300, 128, 256, ("down_proj",)), (300, 128, 256, ("router_gate_x",)),
-    (300, 128, 256, ("dy",)), (300, 72, 264, ("x", "weights", "dy"))]
+# T, H, I, keys a half (d(z) is padded to eights); what lies off a 16-byte boundary.  Not fewer than 17 tokens: batch statistics of two leave each key
+# +1 and -1 whatever the scores, so the router's gradient is zero but for rounding (4e-2 of itself, measured), and of a few it is a difference of that kind.
+LAYER_NODE_CASES = [
+    (300, 128, 256, 4, ()), (1000, 512, 2048, 8, ()), (65, 1032, 520, 10, ()), (17, 64, 128, 4, ()), (2100, 256, 1024, 6, ()),
+    (300, 128, 256, 4, ("x",)), (300, 128, 256, 4, ("gate_proj",)), (300, 128, 256, 4, ("up_proj",)), (300, 128, 256, 4, ("down_proj",)),
+    (300, 128, 256, 4, ("router_gate_x",)), (300, 128, 256, 4, ("dy",)), (300, 72, 264, 4, ("x", "weights", "dy"))]
 
 
 @pytest.mark.parametrize("training", [True, False], ids=["train", "eval"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("case", LAYER_NODE_CASES, ids=lambda c: "T%d-H%d-I%d-%s" % (*c[:3], "+".join(c[3]) or "aligned"))
+@pytest.mark.parametrize("case", LAYER_NODE_CASES, ids=lambda c: "T%d-H%d-I%d-r%d-%s" % (*c[:4], "+".join(c[4]) or "aligned"))
 def test_layer_16_bit_gradients(case, dtype, training, device):
     """The 16-bit layer's differentiable node: output and every gradient against 64 bits.  Each is a sum over many values that were rounded to the
     storage type a handful of times (projections, normalisation, scores, gates and their gradients): _tol of the largest value, five of its roundings."""
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
-    T, H, I, off = case
-    print(f"layer node T={T} H={H} I={I} {dtype} training={training} off the boundary: {off}", flush=True)
+    T, H, I, r, off = case
+    print(f"layer node T={T} H={H} I={I} r={r} {dtype} training={training} off the boundary: {off}", flush=True)
     g = torch.Generator(device=device).manual_seed(T + H)
-    layer = OmniMoE(OmniMoEConfig(H, I, "silu", 16, 16)).to(device=device, dtype=dtype).train(training)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", r * r, r * r)).to(device=device, dtype=dtype).train(training)
     with torch.no_grad():
         for n, p in layer.named_parameters():
             p.normal_(0.0, p.size(1) ** -0.5, generator=g)
@@ -405,6 +408,30 @@ def test_layer_16_bit_gradients(case, dtype, training, device):
         print(f"   {n}: {err:.2e}")
         assert err <= _tol(dtype), (n, err)
     assert layer.router_norm_x.num_batches_tracked.item() == int(training)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_layer_gradients_only_where_wanted(dtype, device):
+    """The layer's node with any one of its inputs wanted, and with all but one: what is wanted has the bits of the full backward, the rest stays None."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    torch.manual_seed(8)
+    layer = OmniMoE(OmniMoEConfig(128, 256, "silu", 100, 6)).to(device=device, dtype=dtype).eval()
+    x, dy = (torch.randn(1, 200, 128, device=device).to(dtype) for _ in range(2))
+    leaves = {"x": x, **dict(layer.named_parameters())}
+
+    def gradients(wanted):
+        for n, t in leaves.items():
+            t.grad = None
+            t.requires_grad_(n in wanted)
+        layer(x).backward(dy)
+        return {n: t.grad for n, t in leaves.items()}
+
+    full = gradients(set(leaves))
+    for n in leaves:
+        for wanted in ({n}, set(leaves) - {n}):
+            for m, grad in gradients(wanted).items():
+                assert (grad is None) == (m not in wanted), (wanted, m)
+                assert grad is None or torch.equal(grad, full[m]), (wanted, m)
 
 
 def test_layer_trains_bf16(device):
