@@ -3,14 +3,16 @@
 Same constructor, attribute / ``state_dict`` names and ``forward(hidden_states, **kwargs)``
 as the reference's ``OmniMoE`` (omni_moe/modules/omni_moe.py:14-106); the forward is ONE call
 into the gfx950 library (``omni_moe_fwd``): router (projection, BatchNorm, log-softmax,
-Cartesian top-k, exp) and fused experts on a side stream, the shared SwiGLU MLP on the
-caller's stream, joined by the final add (``overlap_branches = False``: everything on the
-caller's stream, the add fused into the down projection).
+Cartesian top-k, exp), fused experts, the shared SwiGLU MLP and the final add.  Small 16-bit
+calls are a few joint launches on the caller's stream; beyond them the router and the
+experts run on a side stream beside the MLP (``overlap_branches`` below).
 
-When autograd is recording and the input or a parameter requires grad, ``forward`` instead
-composes differentiable operators in the reference's order (omni_moe.py:64-104: the router
-stage -- Linear, BatchNorm1d, log_softmax, router op, exp -- as one node, the expert op, the
-MLP op, add), so the layer trains; call it under ``torch.no_grad()`` for the fused path.
+When autograd is recording and the input or a parameter requires grad, the whole layer is one
+differentiable node (``csrc/torch_ops.cpp``) that keeps what its backward needs.  Subclasses, and
+calls that the native host path does not take, compose differentiable operators instead, in the
+reference's order (omni_moe.py:64-104: the router stage -- Linear, BatchNorm1d, log_softmax,
+router op, exp -- as one node, the expert op, the MLP op, add).  Call it under
+``torch.no_grad()`` for the fused path.
 """
 import math
 import threading
@@ -95,8 +97,10 @@ class OmniMoE(nn.Module):
     # two HIP streams (both at the default priority) and joins them at the final add: the expert
     # kernel (cache bandwidth, no LDS) shares CUs with the projections (LDS and MFMA).  Set to False
     # to keep everything on one stream, with the add as the down projection's epilogue.
+    # 16-bit calls of up to 2^33 tokens x hidden x intermediate are joint launches on one stream whatever these switches say, wherever those
+    # cover the call (the gather algorithm, key counts in eights or at most 64 tokens, 16-byte aligned operands, a fixed momentum in training).
     overlap_branches = True
-    # The fork and join cost about 50 us of host time per call, so below this much work (tokens x hidden x
+    # For the others: the fork and join cost about 50 us of host time per call, so below this much work (tokens x hidden x
     # intermediate; 2048 x 1024 x 4096 measured level on an MI355X) the call would be host-bound: one stream then.
     overlap_min_work = 2 ** 33
     # ... and from this much work on, one stream is the faster schedule again: the chip is power-limited under the GEMMs, so

@@ -6,8 +6,10 @@ work is done by hand-written gfx950 kernels behind the C ABI in
 ``include/omni_moe_hip.h``.  Like the reference's operators they are differentiable: when
 autograd is recording and an input requires grad, the router, expert and MLP operators go
 through ``torch.autograd.Function`` wrappers (``OmniRouterFunc``, ``OmniExpertFunc``,
-``OmniSwiGLUFunc``, ``OmniLinearFunc``) whose backward passes are HIP kernels too (GEMM
-gradients are library matmuls, as in the reference).  Otherwise no graph is built.
+``OmniSwiGLUFunc``, ``OmniSwiGLULinearFunc``, ``OmniLinearFunc``, ``OmniRouterStageFunc``) whose
+backward passes are HIP kernels too (their GEMM gradients are library matmuls, as in the
+reference; the layer's own node, in ``csrc/torch_ops.cpp``, has those of 16-bit operands from
+``omni_mlp_bwd``).  Otherwise no graph is built.
 
 The operators that a model calls step after step first offer the call to the native host path (``_lib.native()``,
 ``csrc/torch_ops.cpp``), which takes contiguous tensors of matching shapes on one GPU and answers None to anything else:
