@@ -30,13 +30,13 @@ int mlp_gate_up_impl(const void* x, const void* wg, const void* wu, int64_t T, i
 int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive);
 // The experts with a block per token up to here, with a wave per token beyond: 65 tokens (8 parts) 5.5 against 13.5 us, 256 tokens 6.8 / 11.8, 400 tokens
 // 10.8 / 11, 613 tokens 14.3 / 11.0 (hidden 1024, top-16).  The whole layer, block against wave, at 65 / 256 / 384 / 512 / 640 tokens:
-//   hidden  256, top-16   20 / 22    20 / 22    20 / 22     20 / 22      23 / 22 us
-//   hidden 1024, top-2    21 / 26    25 / 27    29 / 28     38 / 36      42 / 39
-//   hidden 1024, top-16   24 / 31    27 / 31    32 / 32     42 / 42      47 / 44
-//   hidden 1024, top-32   26 / 39    31 / 40    35 / 40     45 / 49      50 / 52
-//   hidden 2048, top-16   32 / 43    41 / 48    47 / 49     69 / 70      70 / 70
-//   hidden 4096, top-16   40 / 70    66 / 79    72 / 80    103 / 107
-//   hidden 4096, top-4    35 / 41    44 / 48    51 / 51     67 / 67      66 / 63
+//   hidden  256, top-16   20 / 21    19 / 21    20 / 21     20 / 21      23 / 21 us
+//   hidden 1024, top-2    21 / 26    25 / 27    29 / 28     37 / 36      42 / 38
+//   hidden 1024, top-16   23 / 31    27 / 31    32 / 32     42 / 41      47 / 44
+//   hidden 1024, top-32   26 / 39    31 / 40    35 / 40     44 / 48      50 / 51
+//   hidden 2048, top-16   32 / 43    41 / 47    47 / 49     69 / 71      69 / 69
+//   hidden 4096, top-16   40 / 69    67 / 79    73 / 80    103 / 107
+//   hidden 4096, top-4    35 / 40    44 / 48    51 / 51     69 / 69      67 / 63
 // so the two cross between 320 and 640 tokens everywhere, and at 384 either is within 3 % or the block ahead.
 constexpr int kBlockPerToken = 384;
 // Projection | gate/up, selection | down projection, experts and add; where two stages do not fit one launch, each is its own.
@@ -155,7 +155,7 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   //     better overlap: projection | gate/up, selection | down projection, experts and add.  The bound is this rule's own: a side stream that is given
   //     does not move it (OmniMoE.overlap_min_work, the least work that OmniMoE gives one for, is the same number so that the two schedules meet).
   //     Key counts in eights: the projection's tiles take the two halves' weights eight rows at a time.  Others keep the six launches below (100 x 100 keys
-  //     against 104 x 104, hidden 1024 x 4096: 43 / 27 us at 65 tokens, 60 / 44 at 613, 63 / 64 at 1024, 96 / 92 at 2000).
+  //     against 104 x 104, hidden 1024 x 4096: 43 / 27 us at 65 tokens, 59 / 44 at 613, 63 / 64 at 1024, 94 / 93 at 2000).
   const size_t h_bytes = up256(T * (size_t)intermediate_size * es);
   const bool few = few_tokens_covers_layer(num_tokens, hidden_size, intermediate_size, num_expert_sqrt, num_experts_per_token, dtype);
   //     (rows within reach of the tile kernels' 31-bit offsets, as few_tokens_covers bounds them; the two launches of the general path have no such bound)
