@@ -69,13 +69,14 @@ struct TopkError : torch::PyTorchError {
   PyObject* python_type() override { return PyExc_AssertionError; }      // the reference asserts (utils.py:81-104)
 };
 
-void check(int32_t code, const std::string& what) {
-  if (code == OMNI_OK) return;
-  const std::string text = what + ": " + omni_error_string(code);
+[[noreturn]] void raise(int32_t code, const char* what) {
+  const std::string text = std::string(what) + ": " + omni_error_string(code), full = text + " (code " + std::to_string(code) + ")";
   if (code == OMNI_ERR_TOPK) throw TopkError(text);
-  const std::string full = text + " (code " + std::to_string(code) + ")";
-  if (code < 0) TORCH_CHECK_VALUE(false, full);
-  throw HipError(full);
+  if (code >= 0) throw HipError(full);
+  C10_THROW_ERROR(ValueError, full);
+}
+inline void check(int32_t code, const char* what) {
+  if (code != OMNI_OK) raise(code, what);
 }
 
 bool records(std::initializer_list<const Tensor*> ts) {
@@ -415,7 +416,7 @@ py::object layer_forward(py::handle self, const Tensor& x, const py::dict& algos
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("hip_error_type", [](py::object type) { hip_error_type = type.release().ptr(); });
-  m.def("check", &check);
+  m.def("check", [](int32_t code, const std::string& what) { check(code, what.c_str()); });
   m.def("expert", &expert);
   m.def("router_select", &router_select);
   m.def("router_stage", &router_stage);
