@@ -7,7 +7,9 @@
 // come out of LDS through the transposing read ds_read_b64_tr_b16 (within 16 lanes, lane i names 8 bytes, 4 elements, of row i / 4 of
 // a 4 x 16 block and receives column i of it; two of them give a lane the 8 consecutive K values of v_mfma_f32_16x16x32).
 //
-// What bounds it.  The 256 x 256 tile: the matrix pipelines under the board's power limit, as in the streaming forward GEMM.  The
+// What bounds it.  The 256 x 256 tile at K = 2048 and more: the matrix pipelines under the board's power limit (gate/up at 32768 x 2 8192 x 2048: busy 70 % of
+// the cycles at 1.90 GHz, 1.40 PFLOP/s); at K = 1024 the 16 ring steps between its fill and its epilogue (4096 x 2 4096 x 1024: 51 % at 2.08 GHz, 1.11
+// PFLOP/s with a block to a tile, 58 % and 1.23 streamed; d(h) with the SwiGLU backward as epilogue 28 %, 0.62).  The
 // 128 x 128 tile: the path from L2 into LDS, which carries 64 bytes per cycle and CU -- what that tile asks for at full matrix rate --
 // and, with one block to a CU, the chain of reads and waits between two barriers.  So a block's waves keep 64 x 64 of the tile each (LDS
 // serves 256 bytes a cycle, and smaller wave tiles read more per product) and, alone on its CU, a block has two groups of four waves
