@@ -386,6 +386,34 @@ def test_expert_dense_refusals_and_bad_ids(device):
     assert torch.count_nonzero(y0).item() == 0             # k = 0 -> zeros
 
 
+# the dense algorithm's gated product on 64 x 64, 128 x 128 and 256 x 256 tiles
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", [(300, 64, 64, 4), (4096, 256, 2048, 8), (8200, 128, 2048, 16)], ids=lambda c: f"T{c[0]}-H{c[1]}-N{c[2]}-k{c[3]}")
+def test_expert_takes_operands_at_any_address(case, dtype, device):
+    """Every operand one element past a 16-byte boundary: the bits of the aligned call where the same kernel runs; the dense algorithm, whose product then
+    is staged through registers, to the 16 significant bits of its coefficients as in test_expert_dense_algorithm."""
+    T, H, N, k = case
+
+    def elsewhere(t):
+        flat = torch.empty(t.numel() + 1, device=device, dtype=t.dtype)
+        flat[1:].view(t.shape).copy_(t)
+        return flat[1:].view(t.shape)
+
+    d = [t.to(device) for t in _expert_inputs(T, H, N, k, dtype, "ref", seed=T + H)]
+    off = [elsewhere(t) for t in d]
+    assert all(t.is_contiguous() and t.data_ptr() % 16 == t.element_size() for t in off)
+    print(f"experts off the boundary T={T} H={H} N={N} k={k} {dtype}", flush=True)
+    want = _ops().hip_omni_expert_func(*d, algo="gather")
+    for algo in ("gather", "segment") + (("split",) if H >= 256 else ()):
+        assert torch.equal(_ops().hip_omni_expert_func(*off, algo=algo), _ops().hip_omni_expert_func(*d, algo=algo)), algo
+    got = _ops().hip_omni_expert_func(*off, algo="dense").float()
+    assert (got - want.float()).abs().max().item() <= 1e-2 * max(want.float().abs().max().item(), 1e-6)
+    assert (got != want.float()).float().mean().item() < 0.05
+    dy = torch.randn(T, H, device=device, generator=torch.Generator(device=device).manual_seed(1)).to(dtype)
+    for a, b in zip(_ops().hip_omni_expert_bwd_func(elsewhere(dy), *off), _ops().hip_omni_expert_bwd_func(dy, *d)):
+        assert torch.equal(a, b)
+
+
 def test_expert_split_bad_ids(device):
     g = torch.Generator().manual_seed(12)
     T, H, N, k = 2100, 1024, 512, 8
