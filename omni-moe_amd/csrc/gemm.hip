@@ -5,10 +5,11 @@
 //     - the SwiGLU product is formed in the GEMM epilogue, so gate and up never reach HBM
 //   * down projection     y  = h Wd^T (+ expert output)        (interface.py:23-29, omni_moe.py:102)
 //
-// The 16-bit projections go to the tile GEMM (gemm_tiles.hip) whenever their columns come in eights.  Here are
-//   * `gemm_nt_kernel`: single precision, and 16-bit products of odd sizes (global -> registers -> one of two LDS stages with padded rows);
-//   * `gemm_nt_dma_kernel` and `gemm_ksplit_kernel`: the 16-bit router projection, whose epilogue takes column statistics or whose weights are
-//     two matrices, and the gated product of the dense expert algorithm (global -> LDS directly, ring of stages, swizzled rows).
+// The 16-bit projections go to the tile GEMM (gemm_tiles.hip) whenever their columns come in eights and every operand is 16-byte aligned.  Here are
+//   * `gemm_nt_kernel`: single precision, and 16-bit products whose K is no multiple of 64 or whose operands lie at any other address (global ->
+//     registers -> one of two LDS stages with padded rows);
+//   * `gemm_nt_dma_kernel` and `gemm_ksplit_kernel`: the 16-bit router projection with column statistics, the gated product of the dense expert
+//     algorithm, and aligned products whose columns do not come in eights (global -> LDS directly, ring of stages, swizzled rows).
 // Structure: a block of 4 waves (2 x 2) owns a (2*TM*32) x (2*TN*32) tile; each wave owns
 // TM x TN MFMA tiles of 32x32 and K advances 64 at a time.  The largest tile, 256 x 256, runs
 // on 8 waves (2 x 4, two per SIMD) of 128 x 64 instead.  `gemm_ksplit_kernel` is for fewer 64 x 64 tiles than CUs: a
@@ -870,7 +871,7 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
     }
     if constexpr (TM == 4 && TN == 4) {
       // the 256 x 256 block tile on 8 waves of 128 x 64, two per SIMD: one wave's barrier and load waits are the other's
-      // issue slots (gate/up projection at 4096 x 4096 x 1024: 66.7 against 69.1 us), at 6 fragment reads per 8 MFMAs
+      // issue slots (66.7 against 69.1 us for the 4096-token gate/up projection when that ran here), at 6 fragment reads per 8 MFMAs
       auto kern8 = gemm_nt_dma_kernel<DT, 4, 2, EPI, kDmaBK, kDmaStages, 8>;
       if (hipError_t e = DmaKernelLds<DT, 4, 2, EPI, kDmaBK, kDmaStages, 8>::entry.ensure(); e != hipSuccess) return e;
       hipLaunchKernelGGL(kern8, dim3(blocks), dim3(512), kDmaLds, s, g);

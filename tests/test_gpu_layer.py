@@ -9,8 +9,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(autouse=True)
 def _inference():
-    """These tests cover the fused forward; with autograd recording the module composes the
-    differentiable operators instead (tests/test_gpu_backward.py)."""
+    """These tests cover the fused forward; with autograd recording the module is one
+    differentiable node instead (tests/test_gpu_backward.py)."""
     with torch.no_grad():
         yield
 
