@@ -357,9 +357,13 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_weight
 #pragma unroll
     for (int i = 0; i < E; ++i) au[c][i] = av[c][i] = 0.f;
   }
-  // ends the run [run_first, run_last) of expert e and clears the accumulators
+  // Ends the run [run_first, run_last) of expert e and clears the accumulators.  A run inside the chunk is its expert's whole segment; only the
+  // chunk's first and last run need a look at the pairs beyond it, and those ids are fetched ahead (the segment's offsets, asked for at each
+  // flush, were a wait for memory per run; with them gone and the indices of 64 pairs fetched at once, 32768 pairs over 16384 experts, hidden
+  // 1024: 24.7 -> 23.2 us).
+  const int before = first > 0 ? ids[sorted_pair_ids[first - 1]] : -1, after = last < valid ? ids[sorted_pair_ids[last]] : -1;
   auto flush = [&](int e, int run_first, int run_last) {
-    const bool whole = offsets[e] == run_first && offsets[e + 1] == run_last;
+    const bool whole = (run_first != first || before != e) && (run_last != last || after != e);
     if (whole) {
 #pragma unroll
       for (int c = 0; c < NCH; ++c)
@@ -386,40 +390,42 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_weight
       for (int i = 0; i < E; ++i) au[c][i] = av[c][i] = 0.f;
   };
 
-  int run_e = __builtin_amdgcn_readfirstlane(ids[sorted_pair_ids[first]]), run_first = first;
-  for (int p0 = first; p0 < last; p0 += G) {          // list order = (expert, pair) order: a fixed summation order
-    int64_t tok[G];
-    int ee[G];
-    float cs[G], cc[G];
+  int run_e = -1, run_first = first;
+  for (int p64 = first; p64 < last; p64 += kWave) {   // list order = (expert, pair) order: a fixed summation order
+    // lane i holds what belongs to pair p64 + i: the chain pair -> id is walked once for 64 pairs, and the rows of every batch can be asked for at once
+    const int mine = min(p64 + lane, last - 1), my_pid = sorted_pair_ids[mine], my_tok = sorted_token_ids[mine];
+    const int my_e = ids[my_pid];
+    const float my_ds = ds[my_pid], my_coef = coef[my_pid];
+    const int end = min(p64 + kWave, last);
+    if (run_e < 0) run_e = __builtin_amdgcn_readlane(my_e, 0);
+    for (int p0 = p64; p0 < end; p0 += G) {
+      u32x4_t xr[G][NCH], dyr[G][NCH];
 #pragma unroll
-    for (int i = 0; i < G; ++i) {
-      const int p = min(p0 + i, last - 1);
-      const int pid = sorted_pair_ids[p];
-      tok[i] = sorted_token_ids[p];
-      ee[i] = __builtin_amdgcn_readfirstlane(ids[pid]);
-      cs[i] = ds[pid];
-      cc[i] = coef[pid];
-    }
-    u32x4_t xr[G][NCH], dyr[G][NCH];
+      for (int i = 0; i < G; ++i) {
+        const int64_t at = __builtin_amdgcn_readlane(my_tok, min(p0 + i, end - 1) - p64) * row_bytes;
 #pragma unroll
-    for (int i = 0; i < G; ++i)
-#pragma unroll
-      for (int c = 0; c < NCH; ++c) {
-        xr[i][c] = live[c] ? *(const u32x4_t*)(x + tok[i] * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
-        dyr[i][c] = live[c] ? *(const u32x4_t*)(dy + tok[i] * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
+        for (int c = 0; c < NCH; ++c) {
+          xr[i][c] = live[c] ? *(const u32x4_t*)(x + at + off[c]) : u32x4_t{0, 0, 0, 0};
+          dyr[i][c] = live[c] ? *(const u32x4_t*)(dy + at + off[c]) : u32x4_t{0, 0, 0, 0};
+        }
       }
 #pragma unroll
-    for (int i = 0; i < G; ++i) {
-      if (p0 + i >= last) break;
-      if (ee[i] != run_e) {
-        flush(run_e, run_first, p0 + i);
-        run_e = ee[i];
-        run_first = p0 + i;
-      }
+      for (int i = 0; i < G; ++i) {
+        const int p = p0 + i;
+        if (p >= end) break;
+        const int e = __builtin_amdgcn_readlane(my_e, p - p64);
+        const float cs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ds), p - p64));
+        const float cc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_coef), p - p64));
+        if (e != run_e) {
+          flush(run_e, run_first, p);
+          run_e = e;
+          run_first = p;
+        }
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) {
-        axpy16<DT>(cs[i], xr[i][c], au[c]);
-        axpy16<DT>(cc[i], dyr[i][c], av[c]);
+        for (int c = 0; c < NCH; ++c) {
+          axpy16<DT>(cs, xr[i][c], au[c]);
+          axpy16<DT>(cc, dyr[i][c], av[c]);
+        }
       }
     }
   }
