@@ -151,6 +151,12 @@ OMNI_API int32_t omni_expert_fwd(const void* x, const void* up_weight, const voi
                         int64_t num_tokens, int32_t hidden_size, int64_t num_experts,
                         int32_t num_experts_per_token, int32_t dtype, int32_t algo,
                         void* workspace, void* stream);
+/* omni_expert_fwd which also leaves <x[t], up_weight[indices[t,j]]> of every pair in scores [T,k] f32 (NULL: omni_expert_fwd), for
+ * omni_expert_bwd_scores; algorithms AUTO, GATHER and SPLIT.  The score of an id outside [0,N) is unspecified. */
+OMNI_API int32_t omni_expert_fwd_scores(const void* x, const void* up_weight, const void* down_weight, const void* routing_weights,
+                                        const int32_t* indices, void* y, float* scores, int64_t num_tokens, int32_t hidden_size,
+                                        int64_t num_experts, int32_t num_experts_per_token, int32_t dtype, int32_t algo,
+                                        void* workspace, void* stream);
 
 /* Shared SwiGLU MLP  y = (silu(x Wg^T) * (x Wu^T)) Wd^T  [+ residual].
  * Replaces triton_omni_mlp_func (interface.py:7-29: three torch.matmul around the SwiGLU
@@ -260,6 +266,12 @@ OMNI_API int32_t omni_expert_bwd(const void* dy, const void* x, const void* up_w
                                  void* ddown_weight, void* drouting_weights, int64_t num_tokens, int32_t hidden_size,
                                  int64_t num_experts, int32_t num_experts_per_token, int32_t dtype, void* workspace,
                                  void* stream);
+/* omni_expert_bwd with the pair scores of the same forward pass (omni_expert_fwd_scores; NULL: recomputed). */
+OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x, const void* up_weight, const void* down_weight,
+                                        const void* routing_weights, const int32_t* indices, const float* scores, void* dx,
+                                        void* dup_weight, void* ddown_weight, void* drouting_weights, int64_t num_tokens,
+                                        int32_t hidden_size, int64_t num_experts, int32_t num_experts_per_token, int32_t dtype,
+                                        void* workspace, void* stream);
 
 /* Element-wise SwiGLU for the training path, which keeps gate and up:
  *   omni_swiglu_fwd: out = silu(gate) * up, fp32 product, one rounding

@@ -12,16 +12,18 @@
 // reference accumulates dx, dU and dV with atomics in the storage dtype), so gradients are
 // run-to-run identical.
 //
-// Expert backward in two passes.  Token pass: one wave owns one token, keeps x_t, dy_t and the
-// fp32 dx accumulator in registers, fetches each selected up and down row once, recomputes s
-// (nothing is saved by the forward), writes dg and, to an fp32 workspace, ds and the forward
-// coefficient silu(s) g of every pair.  Weight pass: the pairs are grouped by expert with the
+// Expert backward in two passes.  Token pass: forms dx and dg and, in an fp32 workspace, ds and the forward coefficient silu(s) g of
+// every pair, in the organisation that the forward takes at the sizes: gather (one wave owns one token, keeps x_t, dy_t and the fp32 dx
+// accumulator in registers and fetches each selected up and down row once) or split (the rows in eight column slices, one to an XCD).
+// s comes from the forward where that kept it, else it is recomputed.  Weight pass: the pairs are grouped by expert with the
 // stable schedule of the forward path; one wave owns one expert, walks its segment and gathers
 // the x and dy rows of the segment's tokens, so every dU/dV row is written exactly once
 // (zeros for experts nobody selected).
 #include "common.h"
+#include "expert_split.h"
 #include "omni_moe_hip.h"
 #include "rows.h"
+#include "schedule.h"
 
 namespace omni {
 
@@ -229,16 +231,47 @@ __global__ __launch_bounds__(256) void router_norm_bwd_finish_kernel(const void*
 }
 
 // ---- experts, token pass -----------------------------------------------------------------------
+// Both organisations are bound as the forward's are: gather by the rows' trip over the fabric, split by the vector-memory path on rows that an XCD's
+// L2 holds; split needs the sums over the slices in between, so the forward keeps its <x, U> (4 bytes a pair) and only <dy, V> is formed here.
+// The sort of the pairs, which only the weight pass needs, runs beside: the token pass comes in two launches whose first blocks sort, the count
+// pass beside the first and the scatter pass beside the second.  All blocks have the sort's threads.
+// Sort and token pass, hidden 1024, bf16: 4096 tokens x 16 over 4096 experts 13 + 40 us (gather) -> 11 + 17.5, 1024 x 32 over 16384 18 + 30 -> 7.5 + 15.5.
+constexpr int kTokenWaves = kSortWaves;
+enum : int { kSortNone = 0, kSortCount = 1, kSortScatter = 2 };
+struct SortShare { SortPass pass; int kind, blocks; };          // blocks: a multiple of 8, so that block % 8 names the slice of the others too
+__device__ __forceinline__ bool sort_share(const SortShare& s, uint8_t* lds) {       // false: the block is not one of them
+  if ((int)blockIdx.x >= s.blocks) return false;
+  if (s.kind == kSortScatter) sort_scatter_block(s.pass, (int)blockIdx.x, (int32_t*)lds);
+  else if ((int)blockIdx.x < s.pass.tiles) sort_count_block(s.pass, (int)blockIdx.x, (int32_t*)lds);
+  return true;
+}
+
+struct TokenPass {
+  const uint8_t *x, *dy, *up, *down;
+  const void* gates;
+  const int32_t* ids;
+  const float* scores;               // NULL: recompute
+  uint8_t* dx;
+  void* dgates;
+  float *ds, *coef;                  // [tokens][top_k]
+  float *partial_a, *partial_s;      // split: [8][tokens][top_k]
+  int first, last, num_tokens, hidden, top_k;      // gather: the tokens of this launch
+  uint32_t num_experts;
+};
+struct PairGrad { float dg, ds, coef; };
+__device__ __forceinline__ PairGrad pair_grad(float s, float a, float g) {
+  const float sig = sigmoid_f32(s), silu = s * sig, dsilu = sig + silu * (1.0f - sig);
+  return {a * silu, a * g * dsilu, silu * g};
+}
+
 template <int DT, int NCH, int G>
-__global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_token_kernel(
-    const uint8_t* __restrict__ x, const uint8_t* __restrict__ dy, const uint8_t* __restrict__ up,
-    const uint8_t* __restrict__ down, const void* __restrict__ gates, const int32_t* __restrict__ ids,
-    uint8_t* __restrict__ dx, void* __restrict__ dgates, float* __restrict__ ds_out, float* __restrict__ coef_out,
-    int num_tokens, int hidden, int top_k, uint32_t num_experts) {
+__global__ __launch_bounds__(kSortThreads, 2) void expert_bwd_token_kernel(const TokenPass p, const SortShare sort) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  if (sort_share(sort, lds)) return;
   constexpr int E = Row16<DT>::kElems;
-  const int lane = lane_id();
-  const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * kBwdWavesPerBlock + (threadIdx.x >> 6));
-  if (t >= num_tokens) return;
+  const int lane = lane_id(), hidden = p.hidden, top_k = p.top_k;
+  const int t = __builtin_amdgcn_readfirstlane(p.first + ((int)blockIdx.x - sort.blocks) * kTokenWaves + (int)(threadIdx.x >> 6));
+  if (t >= p.last) return;
   const int64_t row_bytes = int64_t(hidden) * (16 / E);
 
   bool live[NCH];
@@ -249,8 +282,8 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_token_
   for (int c = 0; c < NCH; ++c) {
     live[c] = (c * kWave + lane) * E < hidden;
     off[c] = int64_t(c * kWave + lane) * 16;
-    xr[c] = live[c] ? *(const u32x4_t*)(x + t * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
-    dyr[c] = live[c] ? *(const u32x4_t*)(dy + t * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
+    xr[c] = live[c] ? *(const u32x4_t*)(p.x + t * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
+    dyr[c] = live[c] ? *(const u32x4_t*)(p.dy + t * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < E; ++i) acc[c][i] = 0.f;
   }
@@ -263,9 +296,9 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_token_
 #pragma unroll
     for (int i = 0; i < G; ++i) {
       const int j = min(j0 + i, top_k - 1);
-      const int id = ids[base + j];
-      const float gate = Elem<DT>::load(gates, base + j);
-      const bool ok = (j0 + i < top_k) && (uint32_t)id < num_experts;   // as the forward: such a pair contributes nothing
+      const int id = p.ids[base + j];
+      const float gate = Elem<DT>::load(p.gates, base + j);
+      const bool ok = (j0 + i < top_k) && (uint32_t)id < p.num_experts;   // as the forward: such a pair contributes nothing
       e[i] = ok ? id : 0;
       g[i] = ok ? gate : 0.f;
       live_slot[i] = ok;
@@ -275,12 +308,12 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_token_
     for (int i = 0; i < G; ++i)
 #pragma unroll
       for (int c = 0; c < NCH; ++c)
-        ur[i][c] = live[c] ? *(const u32x4_t*)(up + e[i] * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
+        ur[i][c] = live[c] ? *(const u32x4_t*)(p.up + e[i] * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < G; ++i)
 #pragma unroll
       for (int c = 0; c < NCH; ++c)
-        vr[i][c] = live[c] ? *(const u32x4_t*)(down + e[i] * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
+        vr[i][c] = live[c] ? *(const u32x4_t*)(p.down + e[i] * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
 
     float s[G], a[G];
 #pragma unroll
@@ -299,28 +332,65 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_token_
       s[i] = wave_sum(s[i]);
       a[i] = wave_sum(a[i]);
     }
+    // every lane forms the gradients of all of the batch's pairs; lane i keeps pair i's
+    PairGrad mine{0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < G; ++i) {
-      const float sig = sigmoid_f32(s[i]);
-      const float silu = s[i] * sig;
-      const float dsilu = sig + silu * (1.0f - sig);
-      const float dg = live_slot[i] ? a[i] * silu : 0.f;
-      const float ds = live_slot[i] ? a[i] * g[i] * dsilu : 0.f;
-      const float coef = live_slot[i] ? silu * g[i] : 0.f;
-      if (lane == 0 && j0 + i < top_k) {
-        Elem<DT>::store(dgates, base + j0 + i, dg);
-        ds_out[base + j0 + i] = ds;
-        coef_out[base + j0 + i] = coef;
-      }
+      PairGrad q = pair_grad(s[i], a[i], g[i]);
+      if (!live_slot[i]) q = PairGrad{0.f, 0.f, 0.f};
+      if (lane == i) mine = q;
       if (live_slot[i]) {                       // not even 0 * row: the stand-in row may hold Inf or NaN
 #pragma unroll
-        for (int c = 0; c < NCH; ++c) axpy16<DT>(ds, ur[i][c], acc[c]);
+        for (int c = 0; c < NCH; ++c) axpy16<DT>(q.ds, ur[i][c], acc[c]);
       }
+    }
+    if (lane < G && j0 + lane < top_k) {
+      Elem<DT>::store(p.dgates, base + j0 + lane, mine.dg);
+      p.ds[base + j0 + lane] = mine.ds;
+      p.coef[base + j0 + lane] = mine.coef;
     }
   }
 #pragma unroll
   for (int c = 0; c < NCH; ++c)
-    if (live[c]) *(u32x4_t*)(dx + t * row_bytes + off[c]) = pack16<DT>(acc[c]);
+    if (live[c]) *(u32x4_t*)(p.dx + t * row_bytes + off[c]) = pack16<DT>(acc[c]);
+}
+
+// Split: partial <dy, V> (and, where the forward kept no scores, <x, U>) of every pair and slice ...
+template <int DT, int LPR, bool SMALL>
+__global__ __launch_bounds__(kSortThreads) void expert_bwd_dots_kernel(const TokenPass p, const SortShare sort) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  if (sort_share(sort, lds)) return;
+  const int block = (int)blockIdx.x - sort.blocks;
+  split_dots_block<DT, LPR, SMALL, kTokenWaves>(p.dy, p.down, p.ids, p.partial_a, p.num_tokens, p.hidden, p.top_k, p.num_experts, 0, block);
+  if (!p.scores) split_dots_block<DT, LPR, SMALL, kTokenWaves>(p.x, p.up, p.ids, p.partial_s, p.num_tokens, p.hidden, p.top_k, p.num_experts, 0, block);
+}
+
+// ... then the slice of dx = sum of ds U, with ds from the sums over the slices; slice 0 leaves dg, ds and the coefficients
+template <int DT, int LPR, bool SMALL>
+__global__ __launch_bounds__(kSortThreads) void expert_bwd_accumulate_kernel(const TokenPass p, const SortShare sort) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  if (sort_share(sort, lds)) return;
+  using Off = typename SplitOff<SMALL>::type;
+  const int block = (int)blockIdx.x - sort.blocks;
+  split_accumulate_block<DT, LPR, SMALL, kTokenWaves, true>(p.up, p.ids, p.dx, p.num_tokens, p.hidden, p.top_k, p.num_experts, 0, block, [&](int t, Off pair, int j, bool ok) {
+    PairGrad q{0.f, 0.f, 0.f};
+    if (ok) {
+      auto sum = [&](const float* partial) {
+        float v = 0.f;
+#pragma unroll
+        for (int sl = 0; sl < kSlices; ++sl) v += partial[(Off(sl) * p.num_tokens + t) * p.top_k + j];
+        return v;
+      };
+      const float a = sum(p.partial_a), s = p.scores ? p.scores[pair] : sum(p.partial_s);
+      q = pair_grad(s, a, Elem<DT>::load(p.gates, pair));
+    }
+    if (block % kSlices == 0) {
+      Elem<DT>::store(p.dgates, pair, q.dg);
+      p.ds[pair] = q.ds;
+      p.coef[pair] = q.coef;
+    }
+    return q.ds;
+  });
 }
 
 // ---- experts, weight pass ----------------------------------------------------------------------
@@ -524,26 +594,72 @@ static inline int weight_chunk(size_t pairs) {
   return (int)(c < 16 ? 16 : c);
 }
 
-template <int DT, int NCH, int G>
-static hipError_t launch_expert_bwd(const void* dy, const void* x, const void* up, const void* down, const void* gates,
-                                    const int32_t* ids, void* dx, void* dup, void* ddown, void* dgates, float* ds, float* coef,
-                                    const int32_t* offsets, const int32_t* pair_ids, const int32_t* token_ids, float* partials,
-                                    int64_t T, int H, int64_t N, int k, hipStream_t s) {
-  dim3 block(kBwdWavesPerBlock * kWave);
-  if (T > 0) {
-    dim3 grid((unsigned)((T + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock));
-    hipLaunchKernelGGL((expert_bwd_token_kernel<DT, NCH, G>), grid, block, 0, s, (const uint8_t*)x, (const uint8_t*)dy,
-                       (const uint8_t*)up, (const uint8_t*)down, gates, ids, (uint8_t*)dx, dgates, ds, coef, (int)T, H, k,
-                       (uint32_t)N);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+// What a launch of the token pass takes in LDS: the tables of the sort beside it
+template <auto kKernel>
+struct TokenLds { static inline LdsKernel entry{(const void*)kKernel, (kSortWaves + 3) * slice_width(kMaxBinsWide) * 4}; };
+template <auto kKernel>
+static hipError_t start_token(const TokenPass& p, const SortPass* sort, int kind, int64_t blocks, hipStream_t s) {
+  SortShare share{};
+  int bytes = 0;
+  if (kind != kSortNone) {
+    share = SortShare{*sort, kind, kind == kSortCount ? (sort->tiles + kSlices - 1) / kSlices * kSlices : sort->tiles * kBinSlices};
+    bytes = kind == kSortCount ? count_lds(sort->stride) : scatter_lds(sort->width);
+    if (bytes > 65536)
+      if (hipError_t e = TokenLds<kKernel>::entry.ensure(); e != hipSuccess) return e;
   }
+  if (share.blocks + blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(kKernel, dim3((unsigned)(share.blocks + blocks)), dim3(kSortThreads), bytes, s, p, share);
+  return hipGetLastError();
+}
+template <int DT, int LPR, bool SMALL>
+static hipError_t launch_token_split(const TokenPass& p, const SortPass* sort, hipStream_t s) {
+  constexpr int kPerBlock = kTokenWaves * (kWave / LPR);
+  const int64_t blocks = (int64_t)((p.num_tokens + kPerBlock - 1) / kPerBlock) * kSlices;
+  if (hipError_t e = start_token<expert_bwd_dots_kernel<DT, LPR, SMALL>>(p, sort, sort ? kSortCount : kSortNone, blocks, s); e != hipSuccess) return e;
+  // (32-bit offsets in the accumulate pass from 512-byte slices on, as in the forward)
+  return start_token<expert_bwd_accumulate_kernel<DT, LPR, SMALL && (LPR >= 32)>>(p, sort, sort ? kSortScatter : kSortNone, blocks, s);
+}
+template <int DT>
+static hipError_t launch_token_split_by_row(const TokenPass& p, const SortPass* sort, int lanes_per_row, hipStream_t s) {
+  const bool small = split_offsets_small(p.num_tokens, p.hidden, p.top_k, p.num_experts, 1, DT == kF32 ? 4 : 2);
+  switch (lanes_per_row) {
+    case 8: return small ? launch_token_split<DT, 8, true>(p, sort, s) : launch_token_split<DT, 8, false>(p, sort, s);
+    case 16: return small ? launch_token_split<DT, 16, true>(p, sort, s) : launch_token_split<DT, 16, false>(p, sort, s);
+    case 32: return small ? launch_token_split<DT, 32, true>(p, sort, s) : launch_token_split<DT, 32, false>(p, sort, s);
+    case 64: return small ? launch_token_split<DT, 64, true>(p, sort, s) : launch_token_split<DT, 64, false>(p, sort, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+// Gather: the scatter pass has all tokens beside it, from 4096 tokens on (two rounds of waves) the count pass half of them
+template <int DT, int NCH, int G>
+static hipError_t launch_token_gather(TokenPass p, const SortPass* sort, hipStream_t s) {
+  constexpr auto kKernel = expert_bwd_token_kernel<DT, NCH, G>;
+  const int early = sort && p.num_tokens >= 4096 ? p.num_tokens / 2 : 0;
+  auto blocks = [](int tokens) -> int64_t { return (tokens + kTokenWaves - 1) / kTokenWaves; };
+  p.first = 0;
+  p.last = early;
+  if (sort)
+    if (hipError_t e = start_token<kKernel>(p, sort, kSortCount, blocks(early), s); e != hipSuccess) return e;
+  p.first = early;
+  p.last = p.num_tokens;
+  return start_token<kKernel>(p, sort, sort ? kSortScatter : kSortNone, blocks(p.num_tokens - early), s);
+}
+
+template <int DT, int NCH, int G>
+static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, int lanes_per_row, void* dup, void* ddown, const int32_t* offsets, const int32_t* pair_ids,
+                                    const int32_t* token_ids, float* partials, hipStream_t s) {
+  const int64_t T = p.num_tokens, N = p.num_experts;
+  const int H = p.hidden, k = p.top_k;
+  const hipError_t te = lanes_per_row ? launch_token_split_by_row<DT>(p, sort, lanes_per_row, s) : launch_token_gather<DT, NCH, G>(p, sort, s);
+  if (te != hipSuccess) return te;
+  dim3 block(kBwdWavesPerBlock * kWave);
   const size_t P = (size_t)T * (size_t)k;
   const int chunk = weight_chunk(P);
   const int num_chunks = (int)((P + chunk - 1) / chunk);
   if (num_chunks > 0) {
     dim3 grid((unsigned)((num_chunks + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock));
-    hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, NCH, G>), grid, block, 0, s, (const uint8_t*)x, (const uint8_t*)dy, ds, coef,
-                       ids, offsets, pair_ids, token_ids, (uint8_t*)dup, (uint8_t*)ddown, partials, N, H, chunk, num_chunks);
+    hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, NCH, G>), grid, block, 0, s, p.x, p.dy, p.ds, p.coef,
+                       p.ids, offsets, pair_ids, token_ids, (uint8_t*)dup, (uint8_t*)ddown, partials, N, H, chunk, num_chunks);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   dim3 grid((unsigned)((N + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock));
@@ -650,16 +766,26 @@ extern "C" OMNI_API int32_t omni_router_norm_bwd_padded(const void* dgates, cons
                          (num_expert_sqrt + 7) / 8 * 8);
 }
 
+namespace omni {
+int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype);       // defined beside the expert kernels: what AUTO runs
+// Lanes per row slice where the token pass takes the split organisation -- where the forward does -- else 0.
+static int bwd_split_lanes(int64_t T, int H, int64_t N, int k, int dtype) {
+  if (resolve_algo(OMNI_EXPERT_ALGO_AUTO, T, H, N, k, dtype) != OMNI_EXPERT_ALGO_SPLIT) return 0;
+  const int lanes = split_lanes_per_row(H, dtype == OMNI_F32 ? 4 : 2);
+  return lanes >= 8 ? lanes : 0;
+}
+}  // namespace omni
+
 // workspace: ds [P] f32 | coef [P] f32 | sorted pair ids [P] i32 | sorted token ids [P] i32 | offsets [N+1] i32 |
-//            partial rows [chunks][2][2][H] f32 | schedule workspace
+//            partial rows [chunks][2][2][H] f32 | split: partial <dy, V>, partial <x, U> [8][P] f32 each | schedule workspace
 extern "C" OMNI_API size_t omni_expert_bwd_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int64_t num_experts,
                                                            int32_t num_experts_per_token, int32_t dtype) {
   using namespace omni;
-  (void)dtype;
   if (num_tokens < 0 || num_experts <= 0 || num_experts_per_token < 0 || hidden_size <= 0) return 0;
   const size_t P = (size_t)num_tokens * (size_t)num_experts_per_token;
   const size_t chunks = (P + weight_chunk(P) - 1) / weight_chunk(P);
   return 4 * up256(P * 4) + up256(((size_t)num_experts + 1) * 4) + up256(chunks * 4 * (size_t)hidden_size * 4) +
+         (bwd_split_lanes(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) ? 2 * up256(kSlices * P * 4) : 0) +
          omni_schedule_workspace_bytes(num_tokens, num_experts_per_token, num_experts);
 }
 
@@ -668,6 +794,14 @@ extern "C" OMNI_API int32_t omni_expert_bwd(const void* dy, const void* x, const
                                             void* ddown_weight, void* drouting_weights, int64_t num_tokens, int32_t hidden_size,
                                             int64_t num_experts, int32_t num_experts_per_token, int32_t dtype, void* workspace,
                                             void* stream) {
+  return omni_expert_bwd_scores(dy, x, up_weight, down_weight, routing_weights, indices, nullptr, dx, dup_weight, ddown_weight, drouting_weights, num_tokens, hidden_size,
+                                num_experts, num_experts_per_token, dtype, workspace, stream);
+}
+
+extern "C" OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x, const void* up_weight, const void* down_weight, const void* routing_weights,
+                                                   const int32_t* indices, const float* scores, void* dx, void* dup_weight, void* ddown_weight, void* drouting_weights,
+                                                   int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_experts_per_token, int32_t dtype,
+                                                   void* workspace, void* stream) {
   using namespace omni;
   if (num_tokens < 0 || hidden_size <= 0 || num_experts <= 0 || num_experts_per_token < 0) return OMNI_ERR_SHAPE;
   if (num_tokens > INT32_MAX / 2 || num_experts > INT32_MAX / 2 ||
@@ -694,14 +828,22 @@ extern "C" OMNI_API int32_t omni_expert_bwd(const void* dy, const void* x, const
     const size_t chunks = (P + weight_chunk(P) - 1) / weight_chunk(P);
     w += up256(chunks * 4 * (size_t)hidden_size * 4);
   }
+  const int lanes = bwd_split_lanes(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype);
+  float *partial_a = nullptr, *partial_s = nullptr;
+  if (lanes) {
+    partial_a = (float*)w;             w += up256(kSlices * P * 4);
+    partial_s = (float*)w;             w += up256(kSlices * P * 4);
+  }
   hipStream_t s = (hipStream_t)stream;
-  if (int e = omni_schedule(indices, offsets, pair_ids, token_ids, num_tokens, num_experts_per_token, num_experts, w, stream)) return e;
-  const int64_t T = num_tokens, N = num_experts;
-  const int H = hidden_size, k = num_experts_per_token;
+  // one counting pass: beside the token pass; two: on their own, in front of it
+  SortPass pass;
+  const bool beside = schedule_single_pass(indices, offsets, pair_ids, token_ids, num_tokens, num_experts_per_token, num_experts, w, &pass);
+  if (!beside)
+    if (int e = omni_schedule(indices, offsets, pair_ids, token_ids, num_tokens, num_experts_per_token, num_experts, w, stream)) return e;
+  const TokenPass p{(const uint8_t*)x, (const uint8_t*)dy, (const uint8_t*)up_weight, (const uint8_t*)down_weight, routing_weights, indices, scores, (uint8_t*)dx,
+                    drouting_weights, ds, coef, partial_a, partial_s, 0, (int)num_tokens, (int)num_tokens, hidden_size, num_experts_per_token, (uint32_t)num_experts};
   hipError_t err;
-#define OMNI_BWD_ARGS                                                                                                   \
-  dy, x, up_weight, down_weight, routing_weights, indices, dx, dup_weight, ddown_weight, drouting_weights, ds, coef, offsets, \
-      pair_ids, token_ids, partials, T, H, N, k, s
+#define OMNI_BWD_ARGS p, beside ? &pass : nullptr, lanes, dup_weight, ddown_weight, offsets, pair_ids, token_ids, partials, s
 #define OMNI_BWD_CASE(DT)                                                      \
   do {                                                                         \
     if (nch <= 1) err = launch_expert_bwd<DT, 1, 8>(OMNI_BWD_ARGS);            \

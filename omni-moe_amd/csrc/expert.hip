@@ -22,6 +22,7 @@
 // it moves the same rows plus the schedule and a [T,k] fp32 coefficient buffer, and exists so
 // that the two organisations can be measured side by side.
 #include "common.h"
+#include "expert_split.h"
 #include "omni_moe_hip.h"
 #include "rows.h"
 
@@ -36,7 +37,8 @@ constexpr int kTokensPerBlock = 4;   // one wave each
 // G   = experts fetched per batch (their 2*G*NCH loads are all in flight at once).
 // kAdd: the layer's final add as well: y holds the shared MLP's rounded rows (parts = NULL), or the K splits' fp32 sums of them are in
 // parts [splits][tokens][hidden]; both terms are rounded, then their sum.
-struct GatherAdd { const float* parts; int splits; };
+// scores: NULL, or [tokens][top_k] where <x, u> of every pair goes, for a backward pass.
+struct GatherAdd { const float* parts; int splits; float* scores; };
 template <int DT, int NCH, int G, bool kAdd = false>
 __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kernel(
     const uint8_t* __restrict__ x, const uint8_t* __restrict__ up, const uint8_t* __restrict__ down,
@@ -100,6 +102,12 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
     }
 #pragma unroll
     for (int i = 0; i < G; ++i) s[i] = wave_sum(s[i]);
+    if (!kAdd && add.scores) {
+      float mine = 0.f;
+#pragma unroll
+      for (int i = 0; i < G; ++i) mine = lane == i ? s[i] : mine;
+      if (lane < G && j0 + lane < top_k) add.scores[int64_t(t) * top_k + j0 + lane] = mine;
+    }
 #pragma unroll
     for (int i = 0; i < G; ++i) {
       if (!live_slot[i]) continue;                  // not even 0 * row: the stand-in row may hold Inf or NaN
@@ -141,11 +149,11 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
 
 template <int DT, int NCH, int G>
 static hipError_t launch_gather(const void* x, const void* up, const void* down, const void* gates,
-                                const int32_t* ids, void* y, int64_t T, int H, int k, int64_t N, hipStream_t s) {
+                                const int32_t* ids, void* y, float* scores, int64_t T, int H, int k, int64_t N, hipStream_t s) {
   if (T == 0) return hipSuccess;
   dim3 grid((unsigned)((T + kTokensPerBlock - 1) / kTokensPerBlock)), block(kTokensPerBlock * kWave);
   hipLaunchKernelGGL((expert_gather_kernel<DT, NCH, G>), grid, block, 0, s, (const uint8_t*)x, (const uint8_t*)up,
-                     (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{nullptr, 0});
+                     (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{nullptr, 0, scores});
   return hipGetLastError();
 }
 
@@ -155,7 +163,7 @@ hipError_t launch_gather_add(const void* x, const void* up, const void* down, co
   const dim3 grid((unsigned)((T + kTokensPerBlock - 1) / kTokensPerBlock)), block(kTokensPerBlock * kWave);
   auto go = [&](auto dt, auto nch, auto batch) {
     hipLaunchKernelGGL((expert_gather_kernel<decltype(dt)::value, decltype(nch)::value, decltype(batch)::value, true>), grid, block, 0, s, (const uint8_t*)x, (const uint8_t*)up,
-                       (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{parts, splits});
+                       (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{parts, splits, nullptr});
     return hipGetLastError();
   };
   auto by_row = [&](auto dt) {
@@ -170,15 +178,15 @@ hipError_t launch_gather_add(const void* x, const void* up, const void* down, co
 
 template <int DT>
 static int expert_gather_dispatch(const void* x, const void* up, const void* down, const void* gates,
-                                  const int32_t* ids, void* y, int64_t T, int H, int k, int64_t N, hipStream_t s) {
+                                  const int32_t* ids, void* y, int64_t T, int H, int k, int64_t N, hipStream_t s, float* scores = nullptr) {
   constexpr int E = Row16<DT>::kElems;
   if (H % E != 0) return OMNI_ERR_SHAPE;              // rows must be 16-byte multiples
   const int nch = (H + kWave * E - 1) / (kWave * E);
   hipError_t err;
-  if (nch <= 1) err = launch_gather<DT, 1, 16>(x, up, down, gates, ids, y, T, H, k, N, s);
-  else if (nch <= 2) err = launch_gather<DT, 2, 8>(x, up, down, gates, ids, y, T, H, k, N, s);
-  else if (nch <= 4) err = launch_gather<DT, 4, 4>(x, up, down, gates, ids, y, T, H, k, N, s);
-  else if (nch <= 8) err = launch_gather<DT, 8, 2>(x, up, down, gates, ids, y, T, H, k, N, s);
+  if (nch <= 1) err = launch_gather<DT, 1, 16>(x, up, down, gates, ids, y, scores, T, H, k, N, s);
+  else if (nch <= 2) err = launch_gather<DT, 2, 8>(x, up, down, gates, ids, y, scores, T, H, k, N, s);
+  else if (nch <= 4) err = launch_gather<DT, 4, 4>(x, up, down, gates, ids, y, scores, T, H, k, N, s);
+  else if (nch <= 8) err = launch_gather<DT, 8, 2>(x, up, down, gates, ids, y, scores, T, H, k, N, s);
   else return OMNI_ERR_UNSUPPORTED;
   return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
 }
@@ -334,170 +342,38 @@ static int expert_segment_dispatch(const void* x, const void* up, const void* do
 //      y[t, slice] = sum_j coefficient_j * down[id_j, slice].
 // A row slice is LPR lanes of 16 bytes (64 / LPR pairs per wave at a time).  Fixed summation
 // order, no atomics; results agree with the gather algorithm to fp32 rounding of the dot product.
-constexpr int kSlices = 8;
-
-// Sum over the LPR lanes of a group of LPR values per lane, scattered: lane `sub` of the group
-// ends up with the total of value `sub`.  Every step halves what a lane keeps (LPR - 1 exchanges
-// in all, against LPR * log2(LPR) for one tree per value).
-template <int LPR, int N = LPR>
-__device__ __forceinline__ float reduce_scatter_group(float (&v)[N], const int lane) {
-  if constexpr (N == 1) {
-    return v[0];
-  } else {
-    constexpr int S = N / 2;                   // lane distance of this step = half of what is left
-    const bool upper = lane & S;
-    float keep[S];
-#pragma unroll
-    for (int e = 0; e < S; ++e) keep[e] = (upper ? v[e + S] : v[e]) + xor_lane_f<S>(upper ? v[e] : v[e + S], lane);
-    return reduce_scatter_group<LPR, S>(keep, lane);
-  }
-}
-
-// A wave owns GP = 64 / LPR tokens, one per lane group; the group's LPR lanes cover the token's
-// row slice, 16 bytes each.  Pairs go in batches of LPR: LPR partial dot products per lane,
-// then one reduce-scatter leaves pair `sub` of the batch in lane `sub`.
-// SMALL: every table, x, y and the partial sums stay below 4 GiB, ids and row lengths below 2^24 (split_offsets_small):
-// a row's byte offset is then one full-rate v_mad_u32_u24 on 32-bit lane offsets instead of a 64-bit multiply-add and two
-// 32-bit multiplies at a quarter of the rate -- address arithmetic was more than half of the vector instructions' time here.
-template <bool SMALL> struct SplitOff { using type = int64_t; };
-template <> struct SplitOff<true> { using type = uint32_t; };
-template <bool SMALL>
-__device__ __forceinline__ typename SplitOff<SMALL>::type split_mul(uint32_t a, typename SplitOff<SMALL>::type b) {
-  if constexpr (SMALL) return __umul24(a, b); else return (int64_t)a * b;
-}
-
 template <int DT, int LPR, bool SMALL>
 __global__ __launch_bounds__(kTokensPerBlock* kWave) void expert_split_dots_kernel(
     const uint8_t* __restrict__ x, const uint8_t* __restrict__ up, const int32_t* __restrict__ ids,
     float* __restrict__ partial, int num_tokens, int hidden, int top_k, uint32_t num_experts, int col_block) {
-  using Off = typename SplitOff<SMALL>::type;
-  constexpr int E = Row16<DT>::kElems, GP = kWave / LPR;
-  constexpr int LD = LPR < 8 ? LPR : 8;                          // row loads in flight at a time
-  const int lane = lane_id(), sub = lane % LPR, grp = lane / LPR;
-  const int slice = blockIdx.x % kSlices;
-  const int t = ((int)(blockIdx.x / kSlices) * kTokensPerBlock + (threadIdx.x >> 6)) * GP + grp;
-  const bool live = t < num_tokens;
-  const int tt = live ? t : 0;
-  const Off row_bytes = Off(hidden) * (16 / E);
-  // this lane's 16 bytes inside a row (rows wider than 8 slices of 64 lanes go in column blocks of 8 slices, one launch each)
-  const Off col = (Off(col_block) * kSlices + slice) * LPR * 16 + sub * 16;
-  const u32x4_t xr = *(const u32x4_t*)(x + (split_mul<SMALL>((uint32_t)tt, row_bytes) + col));
-  const Off base = split_mul<SMALL>((uint32_t)tt, (Off)top_k);
-  for (int jb = 0; jb < top_k; jb += LPR) {
-    // lane `sub` of a group fetches the id of pair `sub` of the batch; the group reads the ids from its lanes
-    const int my_id = ids[base + min(jb + sub, top_k - 1)];
-    float d[LPR];
-#pragma unroll
-    for (int e0 = 0; e0 < LPR; e0 += LD) {
-      u32x4_t ur[LD];
-#pragma unroll
-      for (int e = 0; e < LD; ++e) {
-        const int id = __shfl(my_id, grp * LPR + e0 + e, kWave);
-        ur[e] = *(const u32x4_t*)(up + (split_mul<SMALL>((uint32_t)id < num_experts ? (uint32_t)id : 0u, row_bytes) + col));
-      }
-#pragma unroll
-      for (int e = 0; e < LD; ++e) d[e0 + e] = dot16<DT>(xr, ur[e], 0.f);
-    }
-    const float total = reduce_scatter_group<LPR>(d, lane);
-    const int j = jb + sub;
-    if (live && j < top_k) {
-      const bool ok = (uint32_t)my_id < num_experts;
-      partial[((Off(col_block) * kSlices + slice) * num_tokens + t) * top_k + j] = ok ? total : 0.f;
-    }
-  }
+  split_dots_block<DT, LPR, SMALL, kTokensPerBlock>(x, up, ids, partial, num_tokens, hidden, top_k, num_experts, col_block, (int)blockIdx.x);
 }
 
-// Same ownership.  Lane `sub` of a group forms the coefficient of pair `sub` of a batch (sum of
-// the 8 slice partials in slice order, silu, gate); the group then walks the batch, every lane
-// fetching its 16 bytes of the down row and the pair's coefficient from the lane that holds it.
+// The coefficient of a pair: the sum of the 8 slice partials in slice order, silu, gate.
 // WIDE: rows of several column blocks (col_block of col_blocks); otherwise both are compile-time constants, which keeps
 // the eight partial-sum loads of the common case one unrolled group that the compiler places behind the row requests.
-template <int DT, int LPR, bool WIDE, bool SMALL>
+// kScores: the dot products go to `scores` as well, for a backward pass (the kernel without them is 3 % faster at 16384 tokens x 16, hidden 1024).
+template <int DT, int LPR, bool WIDE, bool SMALL, bool kScores>
 __global__ __launch_bounds__(kTokensPerBlock* kWave) void expert_split_accumulate_kernel(
     const uint8_t* __restrict__ down, const void* __restrict__ gates, const int32_t* __restrict__ ids,
-    const float* __restrict__ partial, uint8_t* __restrict__ y, int num_tokens, int hidden, int top_k, uint32_t num_experts,
+    const float* __restrict__ partial, uint8_t* __restrict__ y, float* __restrict__ scores, int num_tokens, int hidden, int top_k, uint32_t num_experts,
     int col_block_arg, int col_blocks_arg) {
   using Off = typename SplitOff<SMALL>::type;
   const int col_block = WIDE ? col_block_arg : 0, col_blocks = WIDE ? col_blocks_arg : 1;
-  constexpr int E = Row16<DT>::kElems, GP = kWave / LPR;
-  constexpr int LD = LPR < 8 ? LPR : 8;
-  const int lane = lane_id(), sub = lane % LPR, grp = lane / LPR;
-  const int slice = blockIdx.x % kSlices;
-  const int t = ((int)(blockIdx.x / kSlices) * kTokensPerBlock + (threadIdx.x >> 6)) * GP + grp;
-  const bool live = t < num_tokens;
-  const int tt = live ? t : 0;
-  const Off row_bytes = Off(hidden) * (16 / E);
-  const Off col = (Off(col_block) * kSlices + slice) * LPR * 16 + sub * 16;
-  const Off base = split_mul<SMALL>((uint32_t)tt, (Off)top_k);
-  float acc[E];
+  split_accumulate_block<DT, LPR, SMALL, kTokensPerBlock, false>(down, ids, y, num_tokens, hidden, top_k, num_experts, col_block, (int)blockIdx.x, [&](int t, Off pair, int j, bool) {
+    float sdot = 0.f;
+    for (int cb = 0; cb < col_blocks; ++cb) {                  // slice order, column block by column block
 #pragma unroll
-  for (int i = 0; i < E; ++i) acc[i] = 0.f;
-  for (int jb = 0; jb < top_k; jb += LPR) {
-    const int j = jb + sub;
-    int my_id = -1;                                               // -1: a padded slot or an id outside the table
-    if (j < top_k) {
-      const int id = ids[base + j];
-      if ((uint32_t)id < num_experts) my_id = id;
+      for (int sl = 0; sl < kSlices; ++sl) sdot += partial[((Off(cb) * kSlices + sl) * num_tokens + t) * top_k + j];
     }
-    // the down rows only need the ids: the first LD of them are requested ahead of the partial sums the coefficients
-    // wait for; every row that has been added makes room for the request of a later one (LD row registers in all)
-    u32x4_t vr[LD];
-    bool used[LD];
-    auto request = [&](int slot, int e) {
-      const int id = __shfl(my_id, grp * LPR + e, kWave);         // from the lane of this group that holds pair e
-      used[slot] = id >= 0;
-      vr[slot] = *(const u32x4_t*)(down + (split_mul<SMALL>(used[slot] ? (uint32_t)id : 0u, row_bytes) + col));
-    };
-#pragma unroll
-    for (int e = 0; e < LD; ++e) request(e, e);
-    float coef = 0.f;
-    if (my_id >= 0) {
-      float sdot = 0.f;
-      for (int cb = 0; cb < col_blocks; ++cb) {                  // slice order, column block by column block
-#pragma unroll
-        for (int sl = 0; sl < kSlices; ++sl) sdot += partial[((Off(cb) * kSlices + sl) * num_tokens + tt) * top_k + j];
-      }
-      coef = silu_f32(sdot) * Elem<DT>::load(gates, base + j);
-    }
-#pragma unroll
-    for (int e = 0; e < LPR; ++e) {
-      const float cf = __shfl(coef, grp * LPR + e, kWave);
-      if (used[e % LD]) axpy16<DT>(cf, vr[e % LD], acc);          // not even 0 * row: the stand-in row may hold Inf or NaN
-      if (e + LD < LPR) request(e % LD, e + LD);
-    }
-  }
-  if (live) *(u32x4_t*)(y + (split_mul<SMALL>((uint32_t)t, row_bytes) + col)) = pack16<DT>(acc);
-}
-
-// lanes per row slice, or 0 when the row does not cut into 8 slices of 4..64 lanes
-static inline int split_lanes_per_row(int hidden, int elem_bytes) {
-  const int64_t slice_bytes = (int64_t)hidden * elem_bytes / kSlices;
-  if ((int64_t)hidden * elem_bytes % (kSlices * 16) != 0) return 0;
-  const int lpr = (int)(slice_bytes / 16);
-  return (lpr == 4 || lpr == 8 || lpr == 16 || lpr == 32 || lpr == 64) ? lpr : 0;
-}
-// Rows beyond 8 KiB (8 slices of 64 lanes): the smallest number of column blocks, each 8 slices of a power-of-two number of
-// lanes, that the row cuts into; 0 if there is none (up to 64 blocks: rows of 512 KiB).  1 for rows that split_lanes_per_row takes.
-constexpr int kMaxColBlocks = 64;
-static inline int split_col_blocks(int hidden, int elem_bytes, int* lanes_per_row) {
-  for (int b = 1; b <= kMaxColBlocks; ++b) {
-    if (hidden % b != 0) continue;
-    const int lpr = split_lanes_per_row(hidden / b, elem_bytes);
-    if (lpr) { *lanes_per_row = lpr; return b; }
-  }
-  return 0;
-}
-
-// every byte offset into x, y, the tables and the partial sums fits 32 bits, and the factors of its products 24
-static inline bool split_offsets_small(int64_t T, int H, int k, int64_t N, int col_blocks, int elem_bytes) {
-  const int64_t row = (int64_t)H * elem_bytes, lim = (int64_t)1 << 32, f24 = (int64_t)1 << 24;
-  return row < f24 && N < f24 && T < f24 && k < f24 && N * row < lim && T * row < lim && T * k < lim &&
-         (int64_t)kSlices * col_blocks * T * k * 4 < lim;
+    if (kScores && blockIdx.x % kSlices == 0 && col_block == 0) scores[pair] = sdot;
+    return silu_f32(sdot) * Elem<DT>::load(gates, pair);
+  });
 }
 
 template <int DT, int LPR, bool SMALL>
 static hipError_t launch_split_as(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids,
-                                  float* partial, void* y, int64_t T, int H, int k, int64_t N, int col_blocks, hipStream_t s) {
+                                  float* partial, void* y, float* scores, int64_t T, int H, int k, int64_t N, int col_blocks, hipStream_t s) {
   constexpr int kPerBlock = kTokensPerBlock * (kWave / LPR);       // tokens per block
   // measured (bf16, same box): the dots pass gains 1-3 % from 32-bit offsets at every slice length; the accumulate pass gains
   // 3 % at 512-byte slices and LOSES 4-8 % at 256-byte ones (the compiler's schedule of its row window changes with them)
@@ -506,28 +382,33 @@ static hipError_t launch_split_as(const void* x, const void* up, const void* dow
   for (int cb = 0; cb < col_blocks; ++cb)                            // all partial dot products first: a coefficient needs the whole row
     hipLaunchKernelGGL((expert_split_dots_kernel<DT, LPR, SMALL>), dim3(blocks), dim3(kTokensPerBlock * kWave), 0, s, (const uint8_t*)x,
                        (const uint8_t*)up, ids, partial, (int)T, H, k, (uint32_t)N, cb);
+  auto accumulate = [&](auto kernel, int cb) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kTokensPerBlock * kWave), 0, s, (const uint8_t*)down, gates, ids, partial, (uint8_t*)y, scores, (int)T, H, k, (uint32_t)N, cb,
+                       col_blocks);
+  };
   if (col_blocks == 1) {
-    hipLaunchKernelGGL((expert_split_accumulate_kernel<DT, LPR, false, kAccSmall>), dim3(blocks), dim3(kTokensPerBlock * kWave), 0, s,
-                       (const uint8_t*)down, gates, ids, partial, (uint8_t*)y, (int)T, H, k, (uint32_t)N, 0, 1);
+    if (scores) accumulate(expert_split_accumulate_kernel<DT, LPR, false, kAccSmall, true>, 0);
+    else accumulate(expert_split_accumulate_kernel<DT, LPR, false, kAccSmall, false>, 0);
     return hipGetLastError();
   }
-  for (int cb = 0; cb < col_blocks; ++cb)
-    hipLaunchKernelGGL((expert_split_accumulate_kernel<DT, LPR, true, kAccSmall>), dim3(blocks), dim3(kTokensPerBlock * kWave), 0, s,
-                       (const uint8_t*)down, gates, ids, partial, (uint8_t*)y, (int)T, H, k, (uint32_t)N, cb, col_blocks);
+  for (int cb = 0; cb < col_blocks; ++cb) {
+    if (scores) accumulate(expert_split_accumulate_kernel<DT, LPR, true, kAccSmall, true>, cb);
+    else accumulate(expert_split_accumulate_kernel<DT, LPR, true, kAccSmall, false>, cb);
+  }
   return hipGetLastError();
 }
 template <int DT, int LPR>
 static hipError_t launch_split(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids,
-                               float* partial, void* y, int64_t T, int H, int k, int64_t N, int col_blocks, hipStream_t s) {
+                               float* partial, void* y, float* scores, int64_t T, int H, int k, int64_t N, int col_blocks, hipStream_t s) {
   if (split_offsets_small(T, H, k, N, col_blocks, DT == kF32 ? 4 : 2))
-    return launch_split_as<DT, LPR, true>(x, up, down, gates, ids, partial, y, T, H, k, N, col_blocks, s);
-  return launch_split_as<DT, LPR, false>(x, up, down, gates, ids, partial, y, T, H, k, N, col_blocks, s);
+    return launch_split_as<DT, LPR, true>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
+  return launch_split_as<DT, LPR, false>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
 }
 
 // workspace: partial dot products [8 * column blocks][T][k] f32
 template <int DT>
 static int expert_split_dispatch(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids,
-                                 void* y, int64_t T, int H, int k, int64_t N, void* workspace, hipStream_t s) {
+                                 void* y, float* scores, int64_t T, int H, int k, int64_t N, void* workspace, hipStream_t s) {
   int lpr = 0;
   const int col_blocks = split_col_blocks(H, DT == kF32 ? 4 : 2, &lpr);
   if (col_blocks == 0 || k > 2 * kWave) return OMNI_ERR_UNSUPPORTED;
@@ -536,11 +417,11 @@ static int expert_split_dispatch(const void* x, const void* up, const void* down
   if (!workspace) return OMNI_ERR_WORKSPACE;
   float* partial = (float*)workspace;
   hipError_t err;
-  if (lpr == 4) err = launch_split<DT, 4>(x, up, down, gates, ids, partial, y, T, H, k, N, col_blocks, s);
-  else if (lpr == 8) err = launch_split<DT, 8>(x, up, down, gates, ids, partial, y, T, H, k, N, col_blocks, s);
-  else if (lpr == 16) err = launch_split<DT, 16>(x, up, down, gates, ids, partial, y, T, H, k, N, col_blocks, s);
-  else if (lpr == 32) err = launch_split<DT, 32>(x, up, down, gates, ids, partial, y, T, H, k, N, col_blocks, s);
-  else err = launch_split<DT, 64>(x, up, down, gates, ids, partial, y, T, H, k, N, col_blocks, s);
+  if (lpr == 4) err = launch_split<DT, 4>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
+  else if (lpr == 8) err = launch_split<DT, 8>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
+  else if (lpr == 16) err = launch_split<DT, 16>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
+  else if (lpr == 32) err = launch_split<DT, 32>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
+  else err = launch_split<DT, 64>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
   return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
 }
 
@@ -698,6 +579,13 @@ extern "C" OMNI_API int32_t omni_expert_fwd(const void* x, const void* up_weight
                                int64_t num_tokens, int32_t hidden_size, int64_t num_experts,
                                int32_t num_experts_per_token, int32_t dtype, int32_t algo,
                                void* workspace, void* stream) {
+  return omni_expert_fwd_scores(x, up_weight, down_weight, routing_weights, indices, y, nullptr, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype, algo,
+                                workspace, stream);
+}
+
+extern "C" OMNI_API int32_t omni_expert_fwd_scores(const void* x, const void* up_weight, const void* down_weight, const void* routing_weights, const int32_t* indices, void* y,
+                                                   float* scores, int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_experts_per_token, int32_t dtype,
+                                                   int32_t algo, void* workspace, void* stream) {
   using namespace omni;
   if (num_tokens < 0 || hidden_size <= 0 || num_experts <= 0 || num_experts_per_token < 0) return OMNI_ERR_SHAPE;
   if (num_tokens > INT32_MAX / 2 || num_experts > UINT32_MAX) return OMNI_ERR_SHAPE;
@@ -705,6 +593,7 @@ extern "C" OMNI_API int32_t omni_expert_fwd(const void* x, const void* up_weight
   if (num_tokens > 0 && num_experts_per_token > 0 && (!routing_weights || !indices)) return OMNI_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
   algo = resolve_algo(algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype);
+  if (scores && algo != OMNI_EXPERT_ALGO_GATHER && algo != OMNI_EXPERT_ALGO_SPLIT) return OMNI_ERR_UNSUPPORTED;
   if (algo == OMNI_EXPERT_ALGO_SEGMENT) {
     switch (dtype) {
       case OMNI_BF16: return expert_segment_dispatch<kBF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, workspace, s);
@@ -715,9 +604,9 @@ extern "C" OMNI_API int32_t omni_expert_fwd(const void* x, const void* up_weight
   }
   if (algo == OMNI_EXPERT_ALGO_SPLIT) {
     switch (dtype) {
-      case OMNI_BF16: return expert_split_dispatch<kBF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, workspace, s);
-      case OMNI_F16: return expert_split_dispatch<kF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, workspace, s);
-      case OMNI_F32: return expert_split_dispatch<kF32>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, workspace, s);
+      case OMNI_BF16: return expert_split_dispatch<kBF16>(x, up_weight, down_weight, routing_weights, indices, y, scores, num_tokens, hidden_size, num_experts_per_token, num_experts, workspace, s);
+      case OMNI_F16: return expert_split_dispatch<kF16>(x, up_weight, down_weight, routing_weights, indices, y, scores, num_tokens, hidden_size, num_experts_per_token, num_experts, workspace, s);
+      case OMNI_F32: return expert_split_dispatch<kF32>(x, up_weight, down_weight, routing_weights, indices, y, scores, num_tokens, hidden_size, num_experts_per_token, num_experts, workspace, s);
       default: return OMNI_ERR_DTYPE;
     }
   }
@@ -730,9 +619,9 @@ extern "C" OMNI_API int32_t omni_expert_fwd(const void* x, const void* up_weight
   }
   if (algo != OMNI_EXPERT_ALGO_GATHER) return OMNI_ERR_UNSUPPORTED;
   switch (dtype) {
-    case OMNI_BF16: return expert_gather_dispatch<kBF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s);
-    case OMNI_F16: return expert_gather_dispatch<kF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s);
-    case OMNI_F32: return expert_gather_dispatch<kF32>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s);
+    case OMNI_BF16: return expert_gather_dispatch<kBF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores);
+    case OMNI_F16: return expert_gather_dispatch<kF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores);
+    case OMNI_F32: return expert_gather_dispatch<kF32>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores);
     default: return OMNI_ERR_DTYPE;
   }
 }

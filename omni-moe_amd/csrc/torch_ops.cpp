@@ -87,24 +87,26 @@ bool records(std::initializer_list<const Tensor*> ts) {
 }
 
 // ---- expert op -------------------------------------------------------------------------------------
-Tensor expert_forward(const Tensor& x, const Tensor& up, const Tensor& down, const Tensor& gates, const Tensor& ids, int algo) {
+// scores: NULL, or where the pair scores that a backward pass takes over are put
+Tensor expert_forward(const Tensor& x, const Tensor& up, const Tensor& down, const Tensor& gates, const Tensor& ids, int algo, Tensor* scores = nullptr) {
   const int64_t T = x.size(0), H = x.size(1), N = up.size(0), k = ids.size(1);
   const int dt = dtype_code(x.scalar_type());
   Tensor y = at::empty_like(x);
   const size_t need = omni_expert_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt, algo);
   Tensor ws = need ? bytes(need, x.device()) : Tensor();
-  check(omni_expert_fwd(ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), ptr(y), T, (int32_t)H, N, (int32_t)k, dt, algo, ptr(ws),
-                        stream_of(x.device())), "omni_expert_fwd");
+  if (scores) *scores = at::empty({T, k}, x.options().dtype(at::kFloat));
+  check(omni_expert_fwd_scores(ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), ptr(y), scores ? (float*)ptr(*scores) : nullptr, T, (int32_t)H, N, (int32_t)k,
+                               dt, algo, ptr(ws), stream_of(x.device())), "omni_expert_fwd");
   return y;
 }
 
 struct ExpertFn : public torch::autograd::Function<ExpertFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& up, const Tensor& down, const Tensor& gates, const Tensor& ids) {
-    Tensor y = expert_forward(x, up, down, gates, ids, OMNI_EXPERT_ALGO_AUTO);
-    ctx->save_for_backward({x, up, down, gates, ids});
+    Tensor scores;
+    Tensor y = expert_forward(x, up, down, gates, ids, OMNI_EXPERT_ALGO_AUTO, &scores);
+    ctx->save_for_backward({x, up, down, gates, ids, scores});
     return y;
   }
-  // only the inputs were saved: the backward recomputes the pair scores
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
     const Tensor &x = s[0], &up = s[1], &down = s[2], &gates = s[3], &ids = s[4];
@@ -115,8 +117,8 @@ struct ExpertFn : public torch::autograd::Function<ExpertFn> {
     const int dt = dtype_code(x.scalar_type());
     Tensor dx = at::empty_like(x), dup = at::empty_like(up), ddown = at::empty_like(down), dg = at::empty_like(gates);
     Tensor ws = bytes(omni_expert_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt), x.device());
-    check(omni_expert_bwd(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), ptr(dx), ptr(dup), ptr(ddown), ptr(dg), T, (int32_t)H, N,
-                          (int32_t)k, dt, ptr(ws), stream_of(x.device())), "omni_expert_bwd");
+    check(omni_expert_bwd_scores(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), (const float*)ptr(s[5]), ptr(dx), ptr(dup), ptr(ddown), ptr(dg), T,
+                                 (int32_t)H, N, (int32_t)k, dt, ptr(ws), stream_of(x.device())), "omni_expert_bwd");
     return {dx, dup, ddown, dg, Tensor()};
   }
 };
@@ -216,8 +218,8 @@ struct Layer {
   int64_t H = 0, I = 0, N = 0, r = 0, k = 0;
 };
 
-// One differentiable node for the whole layer (reference omni_moe.py:64-104).  Kept for the backward pass: the input, the gates
-// and ids, the router's workspace (z and the statistics), the rounded gate and up projections and their SwiGLU product.
+// One differentiable node for the whole layer (reference omni_moe.py:64-104).  Kept for the backward pass: the input, the gates,
+// ids and pair scores, the router's workspace (z and the statistics), the rounded gate and up projections and their SwiGLU product.
 struct LayerFn : public torch::autograd::Function<LayerFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& wg, const Tensor& wu, const Tensor& wd, const Tensor& rx, const Tensor& ry,
                         const Tensor& up, const Tensor& down, const Layer& l) {
@@ -226,7 +228,8 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     void* s = stream_of(x.device());
     const RouterOut r = router_forward(x, T, l.H, rx, ry, l.norms, l.k);
     const Tensor x2 = x.view({T, l.H});
-    const Tensor e = expert_forward(x2, up, down, r.gates, r.ids, OMNI_EXPERT_ALGO_AUTO);
+    Tensor scores;
+    const Tensor e = expert_forward(x2, up, down, r.gates, r.ids, OMNI_EXPERT_ALGO_AUTO, &scores);
     Tensor h = at::empty({T, l.I}, x.options()), gate = at::empty({T, l.I}, x.options()), upp = at::empty({T, l.I}, x.options());
     if (dt != OMNI_F32) {                          // (rows of 16 bytes, so both sizes are multiples of 8; operands at any address)
       check(omni_swiglu_linear_save_fwd(ptr(x), ptr(wg), ptr(wu), ptr(h), ptr(gate), ptr(upp), T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_swiglu_linear_save_fwd");
@@ -237,7 +240,7 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     }
     Tensor y = at::empty_like(x);
     check(omni_linear_fwd(ptr(h), ptr(wd), ptr(e), ptr(y), T, (int32_t)l.I, (int32_t)l.H, dt, s), "omni_linear_fwd");
-    ctx->save_for_backward({x, wg, wu, wd, rx, ry, up, down, r.gates, r.ids, r.ws, gate, upp, h});
+    ctx->save_for_backward({x, wg, wu, wd, rx, ry, up, down, r.gates, r.ids, r.ws, gate, upp, h, scores});
     ctx->saved_data["training"] = l.norms.training;
     return y;
   }
@@ -261,8 +264,8 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     Tensor dx_experts = at::empty({T, H}, opt), dup = at::empty_like(up), ddown = at::empty_like(down), dg = at::empty_like(gates);
     {
       Tensor ws = bytes(omni_expert_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt), x.device());
-      check(omni_expert_bwd(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), ptr(dx_experts), ptr(dup), ptr(ddown), ptr(dg), T, (int32_t)H, N,
-                            (int32_t)k, dt, ptr(ws), st), "omni_expert_bwd");
+      check(omni_expert_bwd_scores(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), (const float*)ptr(s[14]), ptr(dx_experts), ptr(dup), ptr(ddown),
+                                   ptr(dg), T, (int32_t)H, N, (int32_t)k, dt, ptr(ws), st), "omni_expert_bwd");
     }
     if (need[6]) out[6] = dup;
     if (need[7]) out[7] = ddown;

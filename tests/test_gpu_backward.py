@@ -136,6 +136,49 @@ def test_expert_bwd_skewed_and_bad_ids(device):
     assert not dg.cpu()[~ok].any()
 
 
+# T, hidden bytes, N, k: the split token pass at every slice length (128 bytes to 1 KiB), ragged tokens, its sort in one pass (4096 bins, more) and in two;
+# the gather token pass with half of its tokens beside the count pass
+EXPERT_BWD_SPLIT_CASES = [(4100, 1024, 2050, 32), (1030, 2048, 4099, 32), (1025, 4096, 20000, 32), (1031, 8192, 600, 32), (4101, 512, 300, 6)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("case", EXPERT_BWD_SPLIT_CASES, ids=lambda c: "T%d-B%d-N%d-k%d" % c)
+def test_expert_bwd_split_matches_fp64(case, dtype, device):
+    """Many pairs: with the forward's pair scores (autograd) and without (the operator), against 64 bits, to the tolerance of the other cases."""
+    T, row, N, k = case
+    H = row // torch.empty(0, dtype=dtype).element_size()
+    print(f"expert bwd split T={T} H={H} N={N} k={k} {dtype}", flush=True)
+    g = torch.Generator(device=device).manual_seed(T + H)
+    n = lambda *s, std=1.0: torch.empty(*s, device=device).normal_(0, std, generator=g).to(dtype)
+    x, dy, up, down = n(T, H), n(T, H), n(N, H, std=0.05), n(N, H, std=0.05)
+    gates = torch.softmax(n(T, k).float(), -1).to(dtype)
+    ids = torch.randint(0, N, (T, k), device=device, dtype=torch.int32, generator=g)
+    ids[::3, 1] = ids[::3, 0]
+    ids[::5, 4] = N + 3
+    ids[1::7, 5] = -1
+    ids[:, 3] = 7                                                       # a segment over many chunks
+    want = [torch.zeros(t.shape, device=device, dtype=torch.float64) for t in (x, up, down, gates)]
+    for a in range(0, T, 64):
+        xs, ys, gs, e = x[a:a + 64].double(), dy[a:a + 64].double(), gates[a:a + 64].double(), ids[a:a + 64].long()
+        ok = ((e >= 0) & (e < N)).double()
+        e = e.clamp(0, N - 1)
+        u, v = up[e].double(), down[e].double()
+        s, p = (xs[:, None] * u).sum(-1), (ys[:, None] * v).sum(-1)
+        sig = torch.sigmoid(s)
+        silu = s * sig
+        ds, cf = p * gs * (sig + silu * (1 - sig)) * ok, silu * gs * ok
+        want[0][a:a + 64] = (ds[..., None] * u).sum(1)
+        want[1].index_add_(0, e.flatten(), (ds[..., None] * xs[:, None]).flatten(0, 1))
+        want[2].index_add_(0, e.flatten(), (cf[..., None] * ys[:, None]).flatten(0, 1))
+        want[3][a:a + 64] = p * silu * ok
+    leaves = [t.detach().clone().requires_grad_() for t in (x, up, down, gates)]
+    _ops().hip_omni_expert_func(*leaves, ids).backward(dy)
+    op = _ops().hip_omni_expert_bwd_func(dy, x, up, down, gates, ids)
+    for leaf, got, ref, what in zip(leaves, op, want, ("dx", "dup", "ddown", "dgates")):
+        _close(leaf.grad, ref, dtype, what)
+        _close(got, ref, dtype, what)
+
+
 def test_expert_func_autograd(device):
     T, H, N, k = 128, 256, 64, 8
     x, up, down, gates, ids = oracle.make_expert_inputs(13, T, H, N, k, dtype=torch.float32, w_std=0.05)
