@@ -124,12 +124,10 @@ OMNI_API int32_t omni_schedule_noalloc(const int32_t* indices, int32_t* offsets,
  *               of partial dot products (H*sizeof(elem)/8 must be 64..1024 bytes, a power of two; wider rows are
  *               taken in up to 64 column blocks of that form, one pair of launches per block, [8 * blocks][T][k] floats).
  *               Rows beyond 8 KiB exist for SPLIT only, and AUTO is SPLIT for them.
- *               AUTO chooses between GATHER and SPLIT from a measured grid, by the length of the row slice
- *               each lane group streams (H*sizeof(elem)/8), the bytes of both tables and the pair count
- *               T*k: GATHER below 32768 pairs, for tables of at most 3 MiB, for slices under 128 bytes
- *               and for k > 128; SPLIT for 128-byte slices up to 32 MiB of tables from 131072 pairs, for
- *               256-byte slices up to 128 MiB (from 65536 pairs, or from 16 MiB of tables), for longer
- *               slices up to 256 MiB of tables or from 262144 pairs (and 2k >= lanes per row), and for
+ *               AUTO chooses between GATHER and SPLIT from a measured grid, by the bytes of a row, of a
+ *               table and of the rows that all pairs name (T*k rows): GATHER for few pairs (less than 32 to
+ *               64 MiB of rows), tables beyond 16 MiB (rows under 1 KiB) to 256 MiB, rows under 512 bytes
+ *               and k > 128; SPLIT elsewhere, and for
  *               rows beyond 8 KiB.  SEGMENT is the expert-centric organisation:
  *               omni_schedule, a pass over the sorted pairs for the coefficients, a token pass
  *               for the sum; kept so that the organisations can be measured side by side.

@@ -256,6 +256,7 @@ struct TokenPass {
   float *ds, *coef;                  // [tokens][top_k]
   float *partial_a, *partial_s;      // split: [8][tokens][top_k]
   int first, last, num_tokens, hidden, top_k;      // gather: the tokens of this launch
+  int lanes, slices;                 // split: 16-byte lanes of a row slice, and slices; 0, 0: gather
   uint32_t num_experts;
 };
 struct PairGrad { float dg, ds, coef; };
@@ -270,7 +271,7 @@ __global__ __launch_bounds__(kSortThreads, 2) void expert_bwd_token_kernel(const
   if (sort_share(sort, lds)) return;
   constexpr int E = Row16<DT>::kElems;
   const int lane = lane_id(), hidden = p.hidden, top_k = p.top_k;
-  const int t = __builtin_amdgcn_readfirstlane(p.first + ((int)blockIdx.x - sort.blocks) * kTokenWaves + (int)(threadIdx.x >> 6));
+  const int t = __builtin_amdgcn_readfirstlane(p.first + ((int)blockIdx.x - sort.blocks) * (int)(blockDim.x / kWave) + (int)(threadIdx.x >> 6));
   if (t >= p.last) return;
   const int64_t row_bytes = int64_t(hidden) * (16 / E);
 
@@ -356,41 +357,59 @@ __global__ __launch_bounds__(kSortThreads, 2) void expert_bwd_token_kernel(const
 }
 
 // Split: partial <dy, V> (and, where the forward kept no scores, <x, U>) of every pair and slice ...
-template <int DT, int LPR, bool SMALL>
+template <int DT, int LPR, int S, bool RAGGED, bool SMALL>
 __global__ __launch_bounds__(kSortThreads) void expert_bwd_dots_kernel(const TokenPass p, const SortShare sort) {
   extern __shared__ __align__(16) uint8_t lds[];
   if (sort_share(sort, lds)) return;
   const int block = (int)blockIdx.x - sort.blocks;
-  split_dots_block<DT, LPR, SMALL, kTokenWaves>(p.dy, p.down, p.ids, p.partial_a, p.num_tokens, p.hidden, p.top_k, p.num_experts, 0, block);
-  if (!p.scores) split_dots_block<DT, LPR, SMALL, kTokenWaves>(p.x, p.up, p.ids, p.partial_s, p.num_tokens, p.hidden, p.top_k, p.num_experts, 0, block);
+  split_dots_block<DT, LPR, S, RAGGED, SMALL, kTokenWaves>(p.dy, p.down, p.ids, p.partial_a, p.num_tokens, p.hidden, p.top_k, p.num_experts, p.lanes, 0, block);
+  if (!p.scores) split_dots_block<DT, LPR, S, RAGGED, SMALL, kTokenWaves>(p.x, p.up, p.ids, p.partial_s, p.num_tokens, p.hidden, p.top_k, p.num_experts, p.lanes, 0, block);
 }
 
 // ... then the slice of dx = sum of ds U, with ds from the sums over the slices; slice 0 leaves dg, ds and the coefficients
-template <int DT, int LPR, bool SMALL>
+template <int DT, int S, class Off>
+struct SplitPairGrad {
+  const TokenPass& p;
+  bool writes, there, use;
+  float part_a[S], part_s[S], gate;
+  Off at;
+  __device__ __forceinline__ void request(bool there_, int t, Off pair, int j, bool inside) {
+    there = there_;
+    use = there && inside;
+    at = pair;
+#pragma unroll
+    for (int sl = 0; sl < S; ++sl) part_a[sl] = p.partial_a[(Off(sl) * p.num_tokens + t) * p.top_k + j];
+    if (p.scores) part_s[0] = p.scores[pair];
+    else
+#pragma unroll
+      for (int sl = 0; sl < S; ++sl) part_s[sl] = p.partial_s[(Off(sl) * p.num_tokens + t) * p.top_k + j];
+    gate = Elem<DT>::load(p.gates, pair);
+  }
+  __device__ __forceinline__ float value() {
+    float a = part_a[0], s = part_s[0];
+#pragma unroll
+    for (int sl = 1; sl < S; ++sl) a += part_a[sl];
+    if (!p.scores)
+#pragma unroll
+      for (int sl = 1; sl < S; ++sl) s += part_s[sl];
+    PairGrad q = pair_grad(s, a, gate);
+    if (!use) q = PairGrad{0.f, 0.f, 0.f};
+    if (there && writes) {
+      Elem<DT>::store(p.dgates, at, q.dg);
+      p.ds[at] = q.ds;
+      p.coef[at] = q.coef;
+    }
+    return q.ds;
+  }
+};
+template <int DT, int LPR, int S, bool RAGGED, bool SMALL>
 __global__ __launch_bounds__(kSortThreads) void expert_bwd_accumulate_kernel(const TokenPass p, const SortShare sort) {
   extern __shared__ __align__(16) uint8_t lds[];
   if (sort_share(sort, lds)) return;
   using Off = typename SplitOff<SMALL>::type;
   const int block = (int)blockIdx.x - sort.blocks;
-  split_accumulate_block<DT, LPR, SMALL, kTokenWaves, true>(p.up, p.ids, p.dx, p.num_tokens, p.hidden, p.top_k, p.num_experts, 0, block, [&](int t, Off pair, int j, bool ok) {
-    PairGrad q{0.f, 0.f, 0.f};
-    if (ok) {
-      auto sum = [&](const float* partial) {
-        float v = 0.f;
-#pragma unroll
-        for (int sl = 0; sl < kSlices; ++sl) v += partial[(Off(sl) * p.num_tokens + t) * p.top_k + j];
-        return v;
-      };
-      const float a = sum(p.partial_a), s = p.scores ? p.scores[pair] : sum(p.partial_s);
-      q = pair_grad(s, a, Elem<DT>::load(p.gates, pair));
-    }
-    if (block % kSlices == 0) {
-      Elem<DT>::store(p.dgates, pair, q.dg);
-      p.ds[pair] = q.ds;
-      p.coef[pair] = q.coef;
-    }
-    return q.ds;
-  });
+  SplitPairGrad<DT, S, Off> pair{p, block % S == 0};
+  split_accumulate_block<DT, LPR, S, RAGGED, SMALL, kTokenWaves>(p.up, p.ids, p.dx, p.num_tokens, p.hidden, p.top_k, p.num_experts, p.lanes, 0, block, pair);
 }
 
 // ---- experts, weight pass ----------------------------------------------------------------------
@@ -598,59 +617,60 @@ static inline int weight_chunk(size_t pairs) {
 template <auto kKernel>
 struct TokenLds { static inline LdsKernel entry{(const void*)kKernel, (kSortWaves + 3) * slice_width(kMaxBinsWide) * 4}; };
 template <auto kKernel>
-static hipError_t start_token(const TokenPass& p, const SortPass* sort, int kind, int64_t blocks, hipStream_t s) {
+static hipError_t start_token(const TokenPass& p, const SortPass* sort, int kind, int64_t blocks, hipStream_t s, int threads = kSortThreads) {
   SortShare share{};
   int bytes = 0;
   if (kind != kSortNone) {
-    share = SortShare{*sort, kind, kind == kSortCount ? (sort->tiles + kSlices - 1) / kSlices * kSlices : sort->tiles * kBinSlices};
+    share = SortShare{*sort, kind, kind == kSortCount ? (sort->tiles + kXcds - 1) / kXcds * kXcds : sort->tiles * kBinSlices};
     bytes = kind == kSortCount ? count_lds(sort->stride) : scatter_lds(sort->width);
     if (bytes > 65536)
       if (hipError_t e = TokenLds<kKernel>::entry.ensure(); e != hipSuccess) return e;
   }
   if (share.blocks + blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(kKernel, dim3((unsigned)(share.blocks + blocks)), dim3(kSortThreads), bytes, s, p, share);
+  hipLaunchKernelGGL(kKernel, dim3((unsigned)(share.blocks + blocks)), dim3(threads), bytes, s, p, share);
   return hipGetLastError();
 }
-template <int DT, int LPR, bool SMALL>
-static hipError_t launch_token_split(const TokenPass& p, const SortPass* sort, hipStream_t s) {
-  constexpr int kPerBlock = kTokenWaves * (kWave / LPR);
-  const int64_t blocks = (int64_t)((p.num_tokens + kPerBlock - 1) / kPerBlock) * kSlices;
-  if (hipError_t e = start_token<expert_bwd_dots_kernel<DT, LPR, SMALL>>(p, sort, sort ? kSortCount : kSortNone, blocks, s); e != hipSuccess) return e;
-  // (32-bit offsets in the accumulate pass from 512-byte slices on, as in the forward)
-  return start_token<expert_bwd_accumulate_kernel<DT, LPR, SMALL && (LPR >= 32)>>(p, sort, sort ? kSortScatter : kSortNone, blocks, s);
-}
 template <int DT>
-static hipError_t launch_token_split_by_row(const TokenPass& p, const SortPass* sort, int lanes_per_row, hipStream_t s) {
-  const bool small = split_offsets_small(p.num_tokens, p.hidden, p.top_k, p.num_experts, 1, DT == kF32 ? 4 : 2);
-  switch (lanes_per_row) {
-    case 8: return small ? launch_token_split<DT, 8, true>(p, sort, s) : launch_token_split<DT, 8, false>(p, sort, s);
-    case 16: return small ? launch_token_split<DT, 16, true>(p, sort, s) : launch_token_split<DT, 16, false>(p, sort, s);
-    case 32: return small ? launch_token_split<DT, 32, true>(p, sort, s) : launch_token_split<DT, 32, false>(p, sort, s);
-    case 64: return small ? launch_token_split<DT, 64, true>(p, sort, s) : launch_token_split<DT, 64, false>(p, sort, s);
-    default: return hipErrorInvalidValue;
-  }
+static hipError_t launch_token_split(const TokenPass& p, const SortPass* sort, hipStream_t s) {
+  const bool small = split_offsets_small(p.up, p.down, p.num_tokens, p.hidden, p.top_k, p.num_experts, 1, DT == kF32 ? 4 : 2);
+  return split_dispatch(p.lanes, p.slices, [&](auto group, auto s_tag, auto ragged) {
+    constexpr int LPR = decltype(group)::value, S = decltype(s_tag)::value;
+    constexpr bool RAGGED = decltype(ragged)::value;
+    const int64_t blocks = split_blocks(p.num_tokens, kTokenWaves * (kWave / LPR), S);
+    const int count = sort ? kSortCount : kSortNone, scatter = sort ? kSortScatter : kSortNone;
+    if constexpr (LPR < 8) {
+      return hipErrorInvalidValue;
+    } else {
+      const hipError_t e = small ? start_token<expert_bwd_dots_kernel<DT, LPR, S, RAGGED, true>>(p, sort, count, blocks, s)
+                                 : start_token<expert_bwd_dots_kernel<DT, LPR, S, RAGGED, false>>(p, sort, count, blocks, s);
+      if (e != hipSuccess) return e;
+      return small ? start_token<expert_bwd_accumulate_kernel<DT, LPR, S, RAGGED, true>>(p, sort, scatter, blocks, s)
+                   : start_token<expert_bwd_accumulate_kernel<DT, LPR, S, RAGGED, false>>(p, sort, scatter, blocks, s);
+    }
+  });
 }
-// Gather: the scatter pass has all tokens beside it, from 4096 tokens on (two rounds of waves) the count pass half of them
+// Gather: the scatter pass has all tokens beside it, from 4096 tokens on (two rounds of waves) the count pass half of them; with nothing to share, blocks of
+// four waves, two to a CU (23578 tokens x 6, hidden 1024: 2 % of the whole backward)
 template <int DT, int NCH, int G>
 static hipError_t launch_token_gather(TokenPass p, const SortPass* sort, hipStream_t s) {
   constexpr auto kKernel = expert_bwd_token_kernel<DT, NCH, G>;
-  const int early = sort && p.num_tokens >= 4096 ? p.num_tokens / 2 : 0;
-  auto blocks = [](int tokens) -> int64_t { return (tokens + kTokenWaves - 1) / kTokenWaves; };
+  auto blocks = [](int tokens, int waves) -> int64_t { return (tokens + waves - 1) / waves; };
   p.first = 0;
-  p.last = early;
-  if (sort)
-    if (hipError_t e = start_token<kKernel>(p, sort, kSortCount, blocks(early), s); e != hipSuccess) return e;
-  p.first = early;
   p.last = p.num_tokens;
-  return start_token<kKernel>(p, sort, sort ? kSortScatter : kSortNone, blocks(p.num_tokens - early), s);
+  if (!sort) return start_token<kKernel>(p, nullptr, kSortNone, blocks(p.num_tokens, kBwdWavesPerBlock), s, kBwdWavesPerBlock * kWave);
+  p.last = p.num_tokens >= 4096 ? p.num_tokens / 2 : 0;
+  if (hipError_t e = start_token<kKernel>(p, sort, kSortCount, blocks(p.last, kTokenWaves), s); e != hipSuccess) return e;
+  p.first = p.last;
+  p.last = p.num_tokens;
+  return start_token<kKernel>(p, sort, kSortScatter, blocks(p.last - p.first, kTokenWaves), s);
 }
 
 template <int DT, int NCH, int G>
-static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, int lanes_per_row, void* dup, void* ddown, const int32_t* offsets, const int32_t* pair_ids,
+static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, void* dup, void* ddown, const int32_t* offsets, const int32_t* pair_ids,
                                     const int32_t* token_ids, float* partials, hipStream_t s) {
   const int64_t T = p.num_tokens, N = p.num_experts;
   const int H = p.hidden, k = p.top_k;
-  const hipError_t te = lanes_per_row ? launch_token_split_by_row<DT>(p, sort, lanes_per_row, s) : launch_token_gather<DT, NCH, G>(p, sort, s);
+  const hipError_t te = p.lanes ? launch_token_split<DT>(p, sort, s) : launch_token_gather<DT, NCH, G>(p, sort, s);
   if (te != hipSuccess) return te;
   dim3 block(kBwdWavesPerBlock * kWave);
   const size_t P = (size_t)T * (size_t)k;
@@ -768,11 +788,11 @@ extern "C" OMNI_API int32_t omni_router_norm_bwd_padded(const void* dgates, cons
 
 namespace omni {
 int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype);       // defined beside the expert kernels: what AUTO runs
-// Lanes per row slice where the token pass takes the split organisation -- where the forward does -- else 0.
-static int bwd_split_lanes(int64_t T, int H, int64_t N, int k, int dtype) {
+// Slices where the token pass takes the split organisation -- where the forward does -- else 0
+static int bwd_split_slices(int64_t T, int H, int64_t N, int k, int dtype) {
   if (resolve_algo(OMNI_EXPERT_ALGO_AUTO, T, H, N, k, dtype) != OMNI_EXPERT_ALGO_SPLIT) return 0;
-  const int lanes = split_lanes_per_row(H, dtype == OMNI_F32 ? 4 : 2);
-  return lanes >= 8 ? lanes : 0;
+  const int es = dtype == OMNI_F32 ? 4 : 2, slices = (int64_t)H * es <= 8192 ? split_slices(H, N, es) : 0;
+  return slices && split_lanes_per_row(H, es, slices) >= 5 ? slices : 0;       // (no kernels for groups of four lanes)
 }
 }  // namespace omni
 
@@ -785,7 +805,7 @@ extern "C" OMNI_API size_t omni_expert_bwd_workspace_bytes(int64_t num_tokens, i
   const size_t P = (size_t)num_tokens * (size_t)num_experts_per_token;
   const size_t chunks = (P + weight_chunk(P) - 1) / weight_chunk(P);
   return 4 * up256(P * 4) + up256(((size_t)num_experts + 1) * 4) + up256(chunks * 4 * (size_t)hidden_size * 4) +
-         (bwd_split_lanes(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) ? 2 * up256(kSlices * P * 4) : 0) +
+         (bwd_split_slices(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) ? 2 * up256(kSlices * P * 4) : 0) +
          omni_schedule_workspace_bytes(num_tokens, num_experts_per_token, num_experts);
 }
 
@@ -828,7 +848,8 @@ extern "C" OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x
     const size_t chunks = (P + weight_chunk(P) - 1) / weight_chunk(P);
     w += up256(chunks * 4 * (size_t)hidden_size * 4);
   }
-  const int lanes = bwd_split_lanes(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype);
+  const int slices = bwd_split_slices(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype);
+  const int lanes = slices ? split_lanes_per_row(hidden_size, dtype == OMNI_F32 ? 4 : 2, slices) : 0;
   float *partial_a = nullptr, *partial_s = nullptr;
   if (lanes) {
     partial_a = (float*)w;             w += up256(kSlices * P * 4);
@@ -841,9 +862,10 @@ extern "C" OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x
   if (!beside)
     if (int e = omni_schedule(indices, offsets, pair_ids, token_ids, num_tokens, num_experts_per_token, num_experts, w, stream)) return e;
   const TokenPass p{(const uint8_t*)x, (const uint8_t*)dy, (const uint8_t*)up_weight, (const uint8_t*)down_weight, routing_weights, indices, scores, (uint8_t*)dx,
-                    drouting_weights, ds, coef, partial_a, partial_s, 0, (int)num_tokens, (int)num_tokens, hidden_size, num_experts_per_token, (uint32_t)num_experts};
+                    drouting_weights, ds, coef, partial_a, partial_s, 0, (int)num_tokens, (int)num_tokens, hidden_size, num_experts_per_token,
+                    lanes, slices, (uint32_t)num_experts};
   hipError_t err;
-#define OMNI_BWD_ARGS p, beside ? &pass : nullptr, lanes, dup_weight, ddown_weight, offsets, pair_ids, token_ids, partials, s
+#define OMNI_BWD_ARGS p, beside ? &pass : nullptr, dup_weight, ddown_weight, offsets, pair_ids, token_ids, partials, s
 #define OMNI_BWD_CASE(DT)                                                      \
   do {                                                                         \
     if (nch <= 1) err = launch_expert_bwd<DT, 1, 8>(OMNI_BWD_ARGS);            \

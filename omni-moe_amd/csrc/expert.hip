@@ -342,86 +342,104 @@ static int expert_segment_dispatch(const void* x, const void* up, const void* do
 //      y[t, slice] = sum_j coefficient_j * down[id_j, slice].
 // A row slice is LPR lanes of 16 bytes (64 / LPR pairs per wave at a time).  Fixed summation
 // order, no atomics; results agree with the gather algorithm to fp32 rounding of the dot product.
-template <int DT, int LPR, bool SMALL>
+template <int DT, int LPR, int S, bool RAGGED, bool SMALL>
 __global__ __launch_bounds__(kTokensPerBlock* kWave) void expert_split_dots_kernel(
     const uint8_t* __restrict__ x, const uint8_t* __restrict__ up, const int32_t* __restrict__ ids,
-    float* __restrict__ partial, int num_tokens, int hidden, int top_k, uint32_t num_experts, int col_block) {
-  split_dots_block<DT, LPR, SMALL, kTokensPerBlock>(x, up, ids, partial, num_tokens, hidden, top_k, num_experts, col_block, (int)blockIdx.x);
+    float* __restrict__ partial, int num_tokens, int hidden, int top_k, uint32_t num_experts, int lanes, int col_block) {
+  split_dots_block<DT, LPR, S, RAGGED, SMALL, kTokensPerBlock>(x, up, ids, partial, num_tokens, hidden, top_k, num_experts, lanes, col_block, (int)blockIdx.x);
 }
 
-// The coefficient of a pair: the sum of the 8 slice partials in slice order, silu, gate.
-// WIDE: rows of several column blocks (col_block of col_blocks); otherwise both are compile-time constants, which keeps
-// the eight partial-sum loads of the common case one unrolled group that the compiler places behind the row requests.
-// kScores: the dot products go to `scores` as well, for a backward pass (the kernel without them is 3 % faster at 16384 tokens x 16, hidden 1024).
-template <int DT, int LPR, bool WIDE, bool SMALL, bool kScores>
+// The coefficient of a pair: the sum of the 8 slice partials in slice order (WIDE: column block by column block), silu, gate.
+// kScores: the dot products go to `scores` as well, for a backward pass.
+template <int DT, int S, bool WIDE, bool kScores, class Off>
+struct SplitCoefficient {
+  const void* gates;
+  const float* partial;
+  float* scores;
+  int num_tokens, top_k, col_blocks;
+  bool writes;                                                   // the block that leaves the scores
+  float part[S], gate;
+  bool use;
+  Off at;
+  __device__ __forceinline__ void request(bool there, int t, Off pair, int j, bool inside) {
+    use = there && inside;
+    at = pair;
+#pragma unroll
+    for (int sl = 0; sl < S; ++sl) part[sl] = partial[(Off(sl) * num_tokens + t) * top_k + j];
+    gate = Elem<DT>::load(gates, pair);
+    if constexpr (WIDE) {
+      float sum = 0.f;
+#pragma unroll
+      for (int sl = 0; sl < S; ++sl) sum += part[sl];
+      for (int cb = 1; cb < col_blocks; ++cb)
+#pragma unroll
+        for (int sl = 0; sl < S; ++sl) sum += partial[((Off(cb) * S + sl) * num_tokens + t) * top_k + j];
+      part[0] = sum;
+    }
+  }
+  __device__ __forceinline__ float value() {
+    float s = part[0];
+    if constexpr (!WIDE)
+#pragma unroll
+      for (int sl = 1; sl < S; ++sl) s += part[sl];
+    if (kScores && use && writes) scores[at] = s;
+    return use ? silu_f32(s) * gate : 0.f;
+  }
+};
+template <int DT, int LPR, int S, bool RAGGED, bool WIDE, bool SMALL, bool kScores>
 __global__ __launch_bounds__(kTokensPerBlock* kWave) void expert_split_accumulate_kernel(
     const uint8_t* __restrict__ down, const void* __restrict__ gates, const int32_t* __restrict__ ids,
     const float* __restrict__ partial, uint8_t* __restrict__ y, float* __restrict__ scores, int num_tokens, int hidden, int top_k, uint32_t num_experts,
-    int col_block_arg, int col_blocks_arg) {
+    int lanes, int col_block_arg, int col_blocks_arg) {
   using Off = typename SplitOff<SMALL>::type;
-  const int col_block = WIDE ? col_block_arg : 0, col_blocks = WIDE ? col_blocks_arg : 1;
-  split_accumulate_block<DT, LPR, SMALL, kTokensPerBlock, false>(down, ids, y, num_tokens, hidden, top_k, num_experts, col_block, (int)blockIdx.x, [&](int t, Off pair, int j, bool) {
-    float sdot = 0.f;
-    for (int cb = 0; cb < col_blocks; ++cb) {                  // slice order, column block by column block
-#pragma unroll
-      for (int sl = 0; sl < kSlices; ++sl) sdot += partial[((Off(cb) * kSlices + sl) * num_tokens + t) * top_k + j];
-    }
-    if (kScores && blockIdx.x % kSlices == 0 && col_block == 0) scores[pair] = sdot;
-    return silu_f32(sdot) * Elem<DT>::load(gates, pair);
-  });
+  const int col_block = WIDE ? col_block_arg : 0;
+  SplitCoefficient<DT, S, WIDE, kScores, Off> pair{gates, partial, scores, num_tokens, top_k, col_blocks_arg, blockIdx.x % S == 0 && col_block == 0};
+  split_accumulate_block<DT, LPR, S, RAGGED, SMALL, kTokensPerBlock>(down, ids, y, num_tokens, hidden, top_k, num_experts, lanes, col_block, (int)blockIdx.x, pair);
 }
 
-template <int DT, int LPR, bool SMALL>
+template <int DT, int LPR, int S, bool RAGGED, bool SMALL>
 static hipError_t launch_split_as(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids,
-                                  float* partial, void* y, float* scores, int64_t T, int H, int k, int64_t N, int col_blocks, hipStream_t s) {
+                                  float* partial, void* y, float* scores, int64_t T, int H, int k, int64_t N, int lanes, int col_blocks, hipStream_t s) {
   constexpr int kPerBlock = kTokensPerBlock * (kWave / LPR);       // tokens per block
-  // measured (bf16, same box): the dots pass gains 1-3 % from 32-bit offsets at every slice length; the accumulate pass gains
-  // 3 % at 512-byte slices and LOSES 4-8 % at 256-byte ones (the compiler's schedule of its row window changes with them)
-  constexpr bool kAccSmall = SMALL && LPR >= 32;
-  const unsigned blocks = (unsigned)((T + kPerBlock - 1) / kPerBlock) * kSlices;
+  const unsigned blocks = (unsigned)split_blocks(T, kPerBlock, S);
   for (int cb = 0; cb < col_blocks; ++cb)                            // all partial dot products first: a coefficient needs the whole row
-    hipLaunchKernelGGL((expert_split_dots_kernel<DT, LPR, SMALL>), dim3(blocks), dim3(kTokensPerBlock * kWave), 0, s, (const uint8_t*)x,
-                       (const uint8_t*)up, ids, partial, (int)T, H, k, (uint32_t)N, cb);
+    hipLaunchKernelGGL((expert_split_dots_kernel<DT, LPR, S, RAGGED, SMALL>), dim3(blocks), dim3(kTokensPerBlock * kWave), 0, s, (const uint8_t*)x,
+                       (const uint8_t*)up, ids, partial, (int)T, H, k, (uint32_t)N, lanes, cb);
   auto accumulate = [&](auto kernel, int cb) {
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kTokensPerBlock * kWave), 0, s, (const uint8_t*)down, gates, ids, partial, (uint8_t*)y, scores, (int)T, H, k, (uint32_t)N, cb,
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kTokensPerBlock * kWave), 0, s, (const uint8_t*)down, gates, ids, partial, (uint8_t*)y, scores, (int)T, H, k, (uint32_t)N, lanes, cb,
                        col_blocks);
   };
   if (col_blocks == 1) {
-    if (scores) accumulate(expert_split_accumulate_kernel<DT, LPR, false, kAccSmall, true>, 0);
-    else accumulate(expert_split_accumulate_kernel<DT, LPR, false, kAccSmall, false>, 0);
+    if (scores) accumulate(expert_split_accumulate_kernel<DT, LPR, S, RAGGED, false, SMALL, true>, 0);
+    else accumulate(expert_split_accumulate_kernel<DT, LPR, S, RAGGED, false, SMALL, false>, 0);
     return hipGetLastError();
   }
-  for (int cb = 0; cb < col_blocks; ++cb) {
-    if (scores) accumulate(expert_split_accumulate_kernel<DT, LPR, true, kAccSmall, true>, cb);
-    else accumulate(expert_split_accumulate_kernel<DT, LPR, true, kAccSmall, false>, cb);
-  }
+  if constexpr (S == kSlices && !RAGGED)                             // rows of several column blocks are cut into eight slices each
+    for (int cb = 0; cb < col_blocks; ++cb) {
+      if (scores) accumulate(expert_split_accumulate_kernel<DT, LPR, S, false, true, SMALL, true>, cb);
+      else accumulate(expert_split_accumulate_kernel<DT, LPR, S, false, true, SMALL, false>, cb);
+    }
   return hipGetLastError();
 }
-template <int DT, int LPR>
-static hipError_t launch_split(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids,
-                               float* partial, void* y, float* scores, int64_t T, int H, int k, int64_t N, int col_blocks, hipStream_t s) {
-  if (split_offsets_small(T, H, k, N, col_blocks, DT == kF32 ? 4 : 2))
-    return launch_split_as<DT, LPR, true>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
-  return launch_split_as<DT, LPR, false>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
-}
 
-// workspace: partial dot products [8 * column blocks][T][k] f32
+// workspace: partial dot products [slices * column blocks][T][k] f32
 template <int DT>
 static int expert_split_dispatch(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids,
                                  void* y, float* scores, int64_t T, int H, int k, int64_t N, void* workspace, hipStream_t s) {
-  int lpr = 0;
-  const int col_blocks = split_col_blocks(H, DT == kF32 ? 4 : 2, &lpr);
-  if (col_blocks == 0 || k > 2 * kWave) return OMNI_ERR_UNSUPPORTED;
+  constexpr int es = DT == kF32 ? 4 : 2;
+  const SplitCut cut = split_cut(H, N, es);
+  if (cut.col_blocks == 0 || k > 2 * kWave) return OMNI_ERR_UNSUPPORTED;
   if (T == 0) return OMNI_OK;
   if (k == 0) return expert_gather_dispatch<DT>(x, up, down, gates, ids, y, T, H, k, N, s);   // writes zeros
   if (!workspace) return OMNI_ERR_WORKSPACE;
   float* partial = (float*)workspace;
-  hipError_t err;
-  if (lpr == 4) err = launch_split<DT, 4>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
-  else if (lpr == 8) err = launch_split<DT, 8>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
-  else if (lpr == 16) err = launch_split<DT, 16>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
-  else if (lpr == 32) err = launch_split<DT, 32>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
-  else err = launch_split<DT, 64>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, col_blocks, s);
+  const bool small = split_offsets_small(up, down, T, H, k, N, cut.col_blocks, es);
+  const hipError_t err = split_dispatch(cut.lanes, cut.slices, [&](auto group, auto s_tag, auto ragged) {
+    constexpr int LPR = decltype(group)::value, S = decltype(s_tag)::value;
+    constexpr bool RAGGED = decltype(ragged)::value;
+    return small ? launch_split_as<DT, LPR, S, RAGGED, true>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, cut.lanes, cut.col_blocks, s)
+                 : launch_split_as<DT, LPR, S, RAGGED, false>(x, up, down, gates, ids, partial, y, scores, T, H, k, N, cut.lanes, cut.col_blocks, s);
+  });
   return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
 }
 
@@ -506,18 +524,19 @@ static int expert_dense_dispatch(const void* x, const void* up, const void* down
   return omni_linear_fwd(coef, vt2, nullptr, y, T, (int32_t)(2 * N), H, dtype, s);
 }
 
-// What OMNI_EXPERT_ALGO_AUTO runs, from the sizes alone.  The split algorithm gives every XCD an eighth of each table row,
-// so it pays while an XCD's share of the tables stays near its caches (its 4 MiB L2 and its part of the memory-side cache)
-// and a row slice is long enough to fetch well; whole-row gathering wins on short rows, on tables far beyond the caches
-// and with few pairs (the split algorithm's second launch: at 32768 pairs it wins from 512-byte slices on, or from 16 MiB
-// of tables on with 256-byte slices).  Measured with ids uniform over the experts, bf16, 4096 /
-// 16384 / 32768 tokens x 16 / 16 / 32 experts per token, time of split over time of gather:
-//   slice  64 B (hidden  256): 1.3-3.4 at every table size                        -> gather
-//   slice 128 B (hidden  512): 0.72-0.91 up to 32 MiB of tables from 262144 pairs on, 1.02-1.6 beyond
-//   slice 256 B (hidden 1024): 0.49-0.67 up to 64 MiB, 0.95-1.01 at 256 MiB, 1.03-1.14 beyond
-//   slice 512 B (hidden 2048): 0.37-0.77 up to 128 MiB, 0.9 at 256 MiB; beyond, 0.89-0.99 from 262144 pairs on and 1.04-1.16 with 65536
-//   slice   1 KiB (hidden 4096): 0.59-0.95 with 32 experts per token (a token's pairs fill half of the 64 lanes that
-//                                share out a batch), 1.05-1.38 with 16
+// What OMNI_EXPERT_ALGO_AUTO runs, from the sizes alone.  The split algorithm gives every XCD a part of each table row, so it pays while that part of the
+// tables stays near its caches (its 4 MiB L2 and its part of the memory-side cache) and where the rows that are moved outweigh its second launch; whole-row
+// gathering wins with few pairs and on tables far beyond the caches.  Time of split (the better number of slices) over time of gather, bf16, ids uniform
+// over the experts; "moved" is pairs x row bytes, a table N x row bytes:
+//   rows 512 B   16384 x 16 and 4096 x 32 tokens: 0.57-0.70 up to 8 MB a table, 0.81-0.91 at 32 MB, 1.0-1.4 at 128 MB; 4096 x 2 to 4096 x 8: 0.65-0.92;
+//                2048 x 16 1.0, 1024 x 32 1.1, fewer pairs 1.3-1.5
+//   rows 1 KiB   0.41-0.82 up to 16 MB, 0.88-0.97 at 64 MB, 0.9-1.1 at 256 MB; 2048 x 8 1.0-1.1, 1024 x 16 1.0-1.3
+//   rows 1.5 KiB 0.43-0.85 up to 24 MB, 0.86-0.96 at 96 MB, 0.9-1.03 at 384 MB; 1024 x 16 0.75-1.05; 2048 x 16 over a table of 1.5 MB 1.02
+//   rows 2 KiB   0.39-0.81 up to 32 MB, 0.89-0.95 at 128 MB, at 512 MB 0.92-0.95 from 262144 pairs on and 0.94-1.05 with fewer; 2048 x 8 0.74-1.08,
+//                1024 x 16 0.64-0.98, 16384 x 4 0.75-1.0, 4096 x 4 0.9-1.1, 4096 x 2 1.1-1.2
+//   rows 2.5 KiB 0.43-0.87 up to 40 MB, 0.89-0.98 at 160 MB, 0.91-1.03 at 640 MB
+//   rows 4 KiB   0.36-0.78 up to 64 MB, 0.94-0.99 at 256 MB, 0.88-1.0 at 1 GB; 512 x 16 0.56-0.88; 16384 x 8 1.0 at 256 MB; 16384 x 4 0.71-0.89, 1.1 from 256 MB on
+//   rows 8 KiB   0.36-0.86 up to 128 MB, 0.87-1.0 at 512 MB
 // A skewed router (few live experts) moves every figure towards the split algorithm; the caller who knows says so.
 int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
   if (algo != OMNI_EXPERT_ALGO_AUTO) return algo;
@@ -527,15 +546,27 @@ int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
   // with N <= 16 k: 63 us against 67.5 us gather at 16384 tokens, hidden 1024, N = 256, k = 16; 95 against 70 at N = 512).
   const int es = dtype == OMNI_F32 ? 4 : 2;
   // rows beyond 8 KiB do not fit the gather kernel's registers: the split kernels take them in column blocks
-  if ((int64_t)H * es > 8192) return OMNI_EXPERT_ALGO_SPLIT;
-  const int64_t tables = 2 * N * (int64_t)H * es, pairs = T * (int64_t)k;
-  const int lpr = split_lanes_per_row(H, es);           // 16-byte lanes per row slice: 4 .. 64, or 0
-  if (lpr < 8 || k > 2 * kWave || tables <= (3ll << 20) || pairs < 32768) return OMNI_EXPERT_ALGO_GATHER;
-  bool split;
-  if (lpr == 8) split = tables <= (32ll << 20) && pairs >= 131072;
-  else if (lpr == 16) split = tables <= (128ll << 20) && (pairs >= 65536 || tables >= (16ll << 20));
-  else split = (tables <= (256ll << 20) || pairs >= 262144) && 2 * k >= lpr;
-  return split ? OMNI_EXPERT_ALGO_SPLIT : OMNI_EXPERT_ALGO_GATHER;
+  const int64_t row = (int64_t)H * es, table = N * row, pairs = T * (int64_t)k, moved = pairs * row, MiB = 1 << 20;
+  if (row > 8192) return OMNI_EXPERT_ALGO_SPLIT;
+  if (row < 512 || k > 2 * kWave || split_slices(H, N, es) == 0) return OMNI_EXPERT_ALGO_GATHER;
+  const bool enough = moved >= 64 * MiB ? k >= 4 : moved >= 32 * MiB ? k >= 8 && table > 2 * MiB && (k >= 16 || table <= 64 * MiB) : row <= 1024 && T >= 4096;
+  const bool near = row < 1024 ? table <= 16 * MiB : row < 1536 ? table <= 64 * MiB : row < 2048 ? table <= 128 * MiB
+                  : k >= 16 ? table <= 256 * MiB || pairs >= 262144 : table <= 64 * MiB;
+  return enough && near ? OMNI_EXPERT_ALGO_SPLIT : OMNI_EXPERT_ALGO_GATHER;
+}
+
+// Whether the whole layer may take its joint launches (layer.hip), whose last kernel gathers the experts and adds: where the experts alone would be a little
+// faster split, the launches that the layer saves outweigh it.  Up to where that was measured.
+bool joint_launches_gather(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
+  if (algo != OMNI_EXPERT_ALGO_AUTO) return algo == OMNI_EXPERT_ALGO_GATHER;
+  const int es = dtype == OMNI_F32 ? 4 : 2;
+  const int64_t row = (int64_t)H * es, tables = 2 * N * row, pairs = T * (int64_t)k;
+  if (row > 8192) return false;
+  const int lanes = split_lanes_per_row(H, es, kSlices);
+  if (lanes < 8 || (lanes & (lanes - 1)) || k > 2 * kWave || tables <= (3ll << 20) || pairs < 32768) return true;
+  if (lanes == 8) return !(tables <= (32ll << 20) && pairs >= 131072);
+  if (lanes == 16) return !(tables <= (128ll << 20) && (pairs >= 65536 || tables >= (16ll << 20)));
+  return !((tables <= (256ll << 20) || pairs >= 262144) && 2 * k >= lanes);
 }
 
 // OMNI_OK when omni_expert_fwd takes `algo` for these sizes (what the whole-layer call checks before it enqueues anything).
@@ -562,8 +593,7 @@ extern "C" OMNI_API size_t omni_expert_workspace_bytes(int64_t num_tokens, int32
   if (num_tokens < 0 || num_experts <= 0 || num_experts_per_token < 0) return 0;
   algo = omni::resolve_algo(algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype);
   if (algo == OMNI_EXPERT_ALGO_SPLIT) {
-    int lpr = 0;
-    const int col_blocks = omni::split_col_blocks(hidden_size, dtype == OMNI_F32 ? 4 : 2, &lpr);
+    const int col_blocks = omni::split_cut(hidden_size, num_experts, dtype == OMNI_F32 ? 4 : 2).col_blocks;
     return omni::align256((size_t)omni::kSlices * (size_t)(col_blocks ? col_blocks : 1) * (size_t)num_tokens * (size_t)num_experts_per_token * 4);
   }
   if (algo == OMNI_EXPERT_ALGO_DENSE)
@@ -592,6 +622,8 @@ extern "C" OMNI_API int32_t omni_expert_fwd_scores(const void* x, const void* up
   if (num_tokens > 0 && (!x || !up_weight || !down_weight || !y)) return OMNI_ERR_NULL;
   if (num_tokens > 0 && num_experts_per_token > 0 && (!routing_weights || !indices)) return OMNI_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
+  int lanes = 0;
+  if (algo == OMNI_EXPERT_ALGO_SPLIT && split_col_blocks(hidden_size, dtype == OMNI_F32 ? 4 : 2, &lanes) == 0) return OMNI_ERR_UNSUPPORTED;
   algo = resolve_algo(algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype);
   if (scores && algo != OMNI_EXPERT_ALGO_GATHER && algo != OMNI_EXPERT_ALGO_SPLIT) return OMNI_ERR_UNSUPPORTED;
   if (algo == OMNI_EXPERT_ALGO_SEGMENT) {

@@ -16,8 +16,8 @@ static inline size_t up256(size_t v) { return (v + 255) / 256 * 256; }
 static inline size_t elem_bytes(int dtype) { return dtype == OMNI_F32 ? 4 : 2; }
 // defined beside the expert kernels: OMNI_OK when omni_expert_fwd takes `algo` at this shape (decided from the sizes alone)
 int expert_algo_check(int algo, int64_t num_tokens, int hidden_size, int64_t num_experts, int top_k, int dtype);
-// ... and which one OMNI_EXPERT_ALGO_AUTO is there
-int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype);
+// ... and whether the joint launches may gather the experts there
+bool joint_launches_gather(int algo, int64_t T, int H, int64_t N, int k, int dtype);
 // defined beside the select kernels: whether they take num_expert_sqrt keys per half with top_k and this dtype
 bool select_covers(int r, int k, int dtype);
 int launch_router_select(const SelectArgs& g, hipStream_t s);
@@ -163,7 +163,7 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
                      intermediate_size <= (1 << 20) && (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0;
   // (batch statistics: the projection and their merge stay launches of their own; a cumulative average, momentum < 0, is counted by the select kernel)
   if ((training ? joint && momentum >= 0.f : few || joint) && num_experts <= UINT32_MAX &&
-      resolve_algo(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) == OMNI_EXPERT_ALGO_GATHER) {
+      joint_launches_gather(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype)) {
     if (stats_dtype != OMNI_BF16 && stats_dtype != OMNI_F16 && stats_dtype != OMNI_F32) return OMNI_ERR_DTYPE;
     if (!gate_weight || !up_weight || !down_weight || !router_weight_x || !router_weight_y || !running_mean_x || !running_var_x || !running_mean_y || !running_var_y)
       return OMNI_ERR_NULL;

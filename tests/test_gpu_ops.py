@@ -278,6 +278,40 @@ def test_expert_split_algorithm(case, device):
     assert (got.float() - ref).abs().max().item() <= (1e-2 if dtype != torch.float32 else 1e-5) * scale
 
 
+# AUTO's split algorithm: four slices of 10, 8, 24, 40, 33 and 64 lanes, eight of 32 and 64; top-k below, at and beyond a batch of 16; ragged tokens
+EXPERT_AUTO_SPLIT_CASES = [(4100, 320, 500, 2, torch.bfloat16), (4097, 256, 900, 6, torch.float16), (2050, 768, 3000, 16, torch.bfloat16),
+                           (1100, 1280, 900, 34, torch.bfloat16), (1030, 1056, 12000, 18, torch.bfloat16), (1003, 2048, 700, 12, torch.float16),
+                           (1100, 2048, 8000, 16, torch.bfloat16), (600, 4096, 70, 16, torch.bfloat16), (4099, 160, 300, 4, torch.float32),
+                           (1001, 512, 300, 128, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("case", EXPERT_AUTO_SPLIT_CASES, ids=lambda c: f"T{c[0]}-H{c[1]}-N{c[2]}-k{c[3]}-{str(c[4]).split('.')[-1]}")
+def test_expert_auto_split_equals_gather(case, device):
+    """Sizes that AUTO gives to the split algorithm, against the gather algorithm: the same sums in another fp32 order, so equal up to one rounding to the storage
+    type of a result near a rounding boundary.  Bad ids, and the tables at any address (then 64-bit offsets and other loads, the same arithmetic)."""
+    from omni_moe.ops.hip import _lib
+    T, H, N, k, dtype = case
+    print(f"expert auto split T={T} H={H} N={N} k={k} {dtype}", flush=True)
+    assert _lib.load().omni_expert_workspace_bytes(T, H, N, k, _lib.DTYPE_CODE[dtype], _lib.ALGO_AUTO) > 0, "AUTO should pick the split algorithm here"
+    g = torch.Generator(device=device).manual_seed(T)
+    n = lambda *s, std=1.0: torch.empty(*s, device=device).normal_(0, std, generator=g).to(dtype)
+    x, up, down, gates = n(T, H), n(N, H, std=0.05), n(N, H, std=0.05), torch.softmax(n(T, k).float(), -1).to(dtype)
+    ids = torch.randint(0, N, (T, k), device=device, dtype=torch.int32, generator=g)
+    ids[::7, 1] = N
+    ids[3::11, 0] = -5
+    ref = _ops().hip_omni_expert_func(x, up, down, gates, ids, algo="gather")
+    got = _ops().hip_omni_expert_func(x, up, down, gates, ids)
+    ulp = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 1e-5}[dtype]      # neighbours differ by up to 2^-7 (2^-10) of the value
+    diff = (got.float() - ref.float()).abs()
+    assert (diff <= 1.01 * ulp * ref.float().abs() + 1e-6 * ref.float().abs().max()).all()
+    moved = []
+    for t in (up, down):
+        flat = torch.empty(t.numel() + 1, device=device, dtype=dtype)
+        flat[1:] = t.flatten()
+        moved.append(flat[1:].view(t.shape))
+    assert torch.equal(got, _ops().hip_omni_expert_func(x, *moved, gates, ids))
+
+
 def test_expert_split_tables_beyond_4gib(device):
     """Tables of 4 GiB each: the split kernels then take their 64-bit row offsets (below that size they use 32-bit ones).
     Rows built on the device, ids from both ends of the tables; checked against the oracle on the rows that are used."""
