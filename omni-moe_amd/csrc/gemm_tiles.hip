@@ -741,12 +741,19 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
   if ((int)blockIdx.x < select_blocks) {
     constexpr int kWaves = S::WM * S::WN * S::KG;
     const int first = (int)blockIdx.x * kWaves + (int)(threadIdx.x >> 6), all = select_blocks * kWaves;
+    const float* stats = g.select.stats;
+    if (g.select.part_mean) {                                  // batch statistics: the block merges them first
+      extern __shared__ __align__(16) uint8_t lds[];
+      merge_statistics(g.select, (float*)lds, kWaves * kWave);
+      count_batch(g.select);
+      stats = (const float*)lds;
+    }
     auto select = [&](auto cells) {
       constexpr int C = decltype(cells)::value;
-      if (g.regs <= 1) select_packed<1, C>(g.select, first, all);
-      else if (g.regs <= 2) select_packed<2, C>(g.select, first, all);
-      else if (g.regs <= 4) select_packed<4, C>(g.select, first, all);
-      else select_packed<8, C>(g.select, first, all);
+      if (g.regs <= 1) select_packed<1, C>(g.select, first, all, stats);
+      else if (g.regs <= 2) select_packed<2, C>(g.select, first, all, stats);
+      else if (g.regs <= 4) select_packed<4, C>(g.select, first, all, stats);
+      else select_packed<8, C>(g.select, first, all, stats);
     };
     if (g.cells <= 1) select(std::integral_constant<int, 1>{});
     else select(std::integral_constant<int, 2>{});
@@ -757,6 +764,7 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
 template <int kId, bool kSwiglu>
 constexpr int tile_lds() {
   using S = Shape<kId, kSwiglu>;
+  static_assert(S::NS * S::KG * (S::WM * S::TM * 16 + S::WN * S::TN * 16) * 128 >= 4 * merge_lds_floats(kMergeKeys, S::WM * S::WN * S::KG * 64), "a block that selects merges statistics there");
   return S::NS * S::KG * (S::WM * S::TM * 16 + S::WN * S::TN * 16) * 128;
 }
 template <auto kKernel, int kBytes>

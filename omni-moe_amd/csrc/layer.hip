@@ -40,7 +40,7 @@ int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int3
 // so the two cross between 320 and 640 tokens everywhere, and at 384 either is within 3 % or the block ahead.
 constexpr int kBlockPerToken = 384;
 // Projection | gate/up, selection | down projection, experts and add; where two stages do not fit one launch, each is its own.
-// statistics (training): projects z and leaves its column statistics, which f.select reads.
+// statistics (training): projects z and leaves its column statistics, which f.select merges or reads.
 template <class Statistics>
 static int joint_forward(const FewTokens& f, int dtype, size_t parts_bytes, hipStream_t s, bool training, Statistics&& statistics) {
   auto code = [](hipError_t e) { return e == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)e; };
@@ -172,8 +172,17 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
                 (int)num_tokens, hidden_size, intermediate_size, router_weight_x, router_weight_y, router_ws};
     SelectArgs& g = f.select;
     g.lx = router_ws; g.ly = (const char*)router_ws + (size_t)num_expert_sqrt * es; g.row_stride = 2 * num_expert_sqrt;
-    if (training) {
-      g.stats = (const float*)((const char*)router_ws + omni_router_workspace_stats_offset(num_tokens, num_expert_sqrt, dtype));
+    const bool merge = training && merge_here(num_tokens, num_expert_sqrt);
+    const size_t strips = ((size_t)num_tokens + kBnRows - 1) / kBnRows;
+    float* const stats = (float*)((char*)router_ws + omni_router_workspace_stats_offset(num_tokens, num_expert_sqrt, dtype));
+    float* const part_mean = (float*)((char*)stats + up256((size_t)4 * num_expert_sqrt * 4));       // as omni_router_fwd lays its workspace out
+    float* const part_m2 = (float*)((char*)part_mean + up256(strips * 2 * num_expert_sqrt * 4));
+    if (merge) {
+      g.part_mean = part_mean; g.part_m2 = part_m2; g.strips = (int)strips; g.momentum = momentum; g.stats_out = stats;
+      g.count_batch[0] = num_batches_tracked_x; g.count_batch[1] = num_batches_tracked_y;
+    }
+    if (training && !merge) {
+      g.stats = stats;
     } else {
       g.run_mean[0] = running_mean_x; g.run_mean[1] = running_mean_y;
       g.run_var[0] = running_var_x; g.run_var[1] = running_var_y;
@@ -188,6 +197,7 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
         return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
       }
       return joint_forward(f, dtype, omni_mlp_workspace_bytes(num_tokens, hidden_size, intermediate_size, dtype) - h_bytes, main_s, training != 0, [&]() -> int {
+        if (merge) return omni_gemm_router_projection(x, router_weight_x, router_weight_y, router_ws, part_mean, part_m2, num_tokens, hidden_size, num_expert_sqrt, dtype, main_s);
         // without a selection (k = 0) omni_router_fwd projects, merges the statistics, moves the running buffers and counts the batch
         return omni_router_fwd(x, router_weight_x, router_weight_y, running_mean_x, running_var_x, num_batches_tracked_x, running_mean_y, running_var_y,
                                num_batches_tracked_y, 1, momentum, eps, nullptr, nullptr, nullptr, num_tokens, hidden_size, num_expert_sqrt, 0, dtype, stats_dtype,

@@ -206,6 +206,8 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
   };
   constexpr bool kPrefetch = R <= 2;              // beyond that the extra live registers cost a wave per SIMD
   if (kPrefetch && wave < g.num_tokens) load_raw(wave);
+  const float* stats = g.stats;
+  const NormKeys<R> norm(g, stats, lane);
   int cell[C];
   candidate_cells<R, C>(cell, g, kp, lane);
 
@@ -221,9 +223,9 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
       px[a] = py[a] = key;
     }
     if (kPrefetch && t + num_waves < g.num_tokens) load_raw(t + num_waves);
-    if (g.stats || g.run_mean[0]) {
-      normalise_half<R>(sx, g, 0, r, lane, dt);
-      normalise_half<R>(sy, g, 1, r, lane, dt);
+    if (stats || g.run_mean[0]) {
+      normalise_half<R>(sx, g, norm, stats, 0, r, lane, dt);
+      normalise_half<R>(sy, g, norm, stats, 1, r, lane, dt);
     }
     bitonic_sort2<R>(sx, px, sy, py, lane);
 
@@ -259,7 +261,7 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
 template <int R, int C>
 __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_packed_kernel(const SelectArgs g) {
   count_batch(g);
-  select_packed<R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves);
+  select_packed<R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats);
 }
 
 // More keys per half than a wave's registers hold (r > 1024): 16-bit scores, k' <= 64.  The row is walked in chunks of
@@ -407,12 +409,7 @@ static int select_dispatch(SelectArgs g, hipStream_t s) {
   return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
 }
 
-// for the layer call, which fills the arguments itself
-int launch_router_select(const SelectArgs& g, hipStream_t s) { return select_dispatch(g, s); }
-
 // ---- BatchNorm1d(affine=False) statistics over the T rows of z [T, C] -------------------
-constexpr int kBnRows = 32;       // rows per partial: one 32-row MFMA tile of the projection GEMM
-
 struct BnFinalArgs {
   const float* part_mean;   // [strips][2r] (training)
   const float* part_m2;
@@ -425,8 +422,7 @@ struct BnFinalArgs {
   float momentum, eps;               // momentum < 0: cumulative moving average, factor 1 / (batches tracked so far + 1)
 };
 
-// One wave per column: merges the strip partials (mean = sum n_s mean_s / n,
-// M2 = sum M2_s + n_s (mean_s - mean)^2, in double), writes mean and 1/sqrt(var+eps), and in
+// One wave per column: merges the strip partials, writes mean and 1/sqrt(var+eps), and in
 // training moves the running buffers (unbiased variance) as nn.BatchNorm1d does.  In eval
 // the running buffers provide mean and variance.
 __global__ __launch_bounds__(256) void bn_finalize_kernel(const BnFinalArgs g) {
@@ -442,30 +438,22 @@ __global__ __launch_bounds__(256) void bn_finalize_kernel(const BnFinalArgs g) {
     // the running buffers (and the batch count) are requested first: their latency passes beside the strips'
     const float rm = load_score(g.running_mean[half], key, g.stat_dt), rv = load_score(g.running_var[half], key, g.stat_dt);
     const float f = g.momentum >= 0.f ? g.momentum : 1.0f / (float)(*g.num_batches_tracked[half] + 1);
-    // one pass over the strips, both sums in double: M2 = sum (M2_s + n_s mean_s^2) - n mu^2 (double carries 29 bits more than
-    // the fp32 result keeps, so the difference stays exact to fp32 while mean^2 / variance < 2^29)
-    double wsum = 0., q = 0.;
-    for (int s = lane; s < g.strips; s += kWave) {
-      const double ns = (double)min(kBnRows, g.num_rows - s * kBnRows), ms = (double)g.part_mean[int64_t(s) * 2 * g.r + col];
-      wsum += ns * ms;
-      q += (double)g.part_m2[int64_t(s) * 2 * g.r + col] + ns * ms * ms;
-    }
-    double sum2[2] = {wsum, q};
+    ColumnSums c{0., 0.};
+    for (int strip = lane; strip < g.strips; strip += kWave) add_strip(c, g.part_mean, g.part_m2, strip, 2 * g.r, col, g.num_rows);
+    double sum2[2] = {c.weighted, c.squares};
 #pragma unroll
     for (int m = kWave / 2; m >= 1; m >>= 1) {
       const double o0 = __shfl_xor(sum2[0], m, kWave), o1 = __shfl_xor(sum2[1], m, kWave);
       sum2[0] += o0;
       sum2[1] += o1;
     }
-    const double n = (double)g.num_rows, mu = sum2[0] / n;
-    const double m2 = fmax(sum2[1] - n * mu * mu, 0.);
-    mean = (float)mu;
-    var = (float)(m2 / n);                                   // biased: normalises the batch
+    const ColumnStats v = column_stats(ColumnSums{sum2[0], sum2[1]}, g.num_rows);
+    mean = v.mean;
+    var = v.var;
     if (lane == 0) {
-      const float unbiased = (float)(m2 / (n > 1. ? n - 1. : 1.));
       // nn.BatchNorm1d(momentum=None): the factor f is 1 / num_batches_tracked AFTER this batch has been counted
       store_score(g.running_mean[half], key, (1.f - f) * rm + f * mean, g.stat_dt);
-      store_score(g.running_var[half], key, (1.f - f) * rv + f * unbiased, g.stat_dt);
+      store_score(g.running_var[half], key, (1.f - f) * rv + f * v.unbiased, g.stat_dt);
     }
   } else {
     mean = load_score(g.running_mean[half], key, g.stat_dt);
@@ -473,8 +461,22 @@ __global__ __launch_bounds__(256) void bn_finalize_kernel(const BnFinalArgs g) {
   }
   if (lane == 0) {
     g.stats[(2 * half) * g.r + key] = mean;
-    g.stats[(2 * half + 1) * g.r + key] = 1.0f / sqrtf(var + g.eps);
+    g.stats[(2 * half + 1) * g.r + key] = rstd_of(var, g.eps);
   }
+}
+
+// The selection for the layer call, which fills the arguments itself; with column statistics in them the launch that merges those in front of it
+int launch_router_select(const SelectArgs& args, hipStream_t s) {
+  SelectArgs g = args;
+  if (g.part_mean) {
+    const BnFinalArgs b{g.part_mean, g.part_m2, g.stats_out, {(void*)g.run_mean[0], (void*)g.run_mean[1]}, {(void*)g.run_var[0], (void*)g.run_var[1]},
+                        {g.count_batch[0], g.count_batch[1]}, g.num_tokens, g.r, g.strips, 1, g.stat_dt, 0, g.momentum, g.eps};
+    hipLaunchKernelGGL(bn_finalize_kernel, dim3((2 * g.r + 3) / 4), dim3(256), 0, s, b);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return OMNI_ERR_HIP_BASE + (int)e;
+    g.stats = g.stats_out;
+    g.part_mean = g.part_m2 = nullptr;
+  }
+  return select_dispatch(g, s);
 }
 
 static inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }

@@ -43,14 +43,79 @@ struct SelectArgs {
   uint8_t row_cells[128]; // candidate cells in row a: min(kp, k/(a+1)), filled by select_dispatch
   int64_t* count_batch[2]; // NULL, or BatchNorm's num_batches_tracked of the two halves: incremented here, behind the
                            // kernel that read them (train-mode router stage)
+  const float* part_mean;  // NULL, or the projection's column statistics [strips][2r] of every 32 rows (training; joint launches): each block merges them
+  const float* part_m2;    //   itself (merge_statistics); block 0 moves run_mean / run_var with `momentum` and leaves the result at stats_out
+  int strips;
+  float momentum;          // < 0: cumulative average, factor 1 / (batches tracked so far + 1)
 };
+constexpr int kMergeKeys = 128;    // keys per half up to which a block merges batch statistics itself
+constexpr int kBnRows = 32;       // rows per strip: one 32-row MFMA tile of the projection GEMM
 
+// One column's batch statistics from its strips' sums (mean = sum n_s mean_s / n, M2 = sum M2_s + n_s mean_s^2 - n mean^2, in double: 29 bits more than
+// the fp32 result keeps, so the difference stays exact to fp32 while mean^2 / variance < 2^29).
+struct ColumnSums { double weighted, squares; };
+__device__ __forceinline__ void add_strip(ColumnSums& c, const float* part_mean, const float* part_m2, int strip, int cols, int col, int num_rows) {
+  const double ns = (double)min(kBnRows, num_rows - strip * kBnRows), ms = (double)part_mean[int64_t(strip) * cols + col];
+  c.weighted += ns * ms;
+  c.squares += (double)part_m2[int64_t(strip) * cols + col] + ns * ms * ms;
+}
+struct ColumnStats { float mean, var, unbiased; };             // var: biased, normalises the batch
+__device__ __forceinline__ ColumnStats column_stats(const ColumnSums& c, int num_rows) {
+  const double n = (double)num_rows, mu = c.weighted / n, m2 = fmax(c.squares - n * mu * mu, 0.);
+  return {(float)mu, (float)(m2 / n), (float)(m2 / (n > 1. ? n - 1. : 1.))};
+}
+__device__ __forceinline__ float rstd_of(float var, float eps) { return 1.0f / sqrtf(var + eps); }
+
+// Batch statistics for a block of `threads` that selects beside another kernel's tiles: every such block merges all columns (2r of them, a few dozen strips each),
+// which the tiles hide, where a merge of its own is a 4-5 us launch between projection and selection.  (A selection by itself is better off behind that
+// launch: 4096 tokens, 64 keys, blocks of 16 waves that merge first 13 us, against 4.5 + 8.8.)  lds: merge_lds_floats(r, threads) floats, 16-byte aligned; the first 4r hold mean_x, rstd_x,
+// mean_y, rstd_y afterwards.
+__device__ __host__ constexpr int merge_lds_floats(int r, int threads) { return (4 * r + 3) / 4 * 4 + 4 * threads; }
+__device__ __forceinline__ void merge_statistics(const SelectArgs& g, float* lds, const int threads) {
+  const int cols = 2 * g.r, tid = threadIdx.x, parts = max(threads / cols, 1);
+  ColumnSums* sums = (ColumnSums*)(lds + (4 * g.r + 3) / 4 * 4);
+  for (int c0 = 0; c0 < cols; c0 += threads) {                  // (one round up to threads / 2 keys)
+    const int part = tid / cols, col = c0 + (parts > 1 ? tid - part * cols : tid);
+    if (part < parts && col < cols) {
+      ColumnSums c{0., 0.};
+      for (int strip = part; strip < g.strips; strip += parts) add_strip(c, g.part_mean, g.part_m2, strip, cols, col, g.num_tokens);
+      sums[tid] = c;
+    }
+    __syncthreads();
+    const int mine = c0 + tid;
+    if (tid < min(cols - c0, threads)) {
+      ColumnSums c = sums[tid];
+      for (int q = 1; q < parts; ++q) {
+        c.weighted += sums[q * cols + tid].weighted;
+        c.squares += sums[q * cols + tid].squares;
+      }
+      const ColumnStats v = column_stats(c, g.num_tokens);
+      const int half = mine >= g.r, key = mine - half * g.r;
+      const float rstd = rstd_of(v.var, g.eps);
+      lds[(2 * half) * g.r + key] = v.mean;
+      lds[(2 * half + 1) * g.r + key] = rstd;
+      if (blockIdx.x == 0) {
+        const float f = g.momentum >= 0.f ? g.momentum : 1.0f / (float)(*g.count_batch[half] + 1);
+        const float rm = load_score(g.run_mean[half], key, g.stat_dt), rv = load_score(g.run_var[half], key, g.stat_dt);
+        store_score((void*)g.run_mean[half], key, (1.f - f) * rm + f * v.mean, g.stat_dt);
+        store_score((void*)g.run_var[half], key, (1.f - f) * rv + f * v.unbiased, g.stat_dt);
+        if (g.stats_out) {
+          g.stats_out[(2 * half) * g.r + key] = v.mean;
+          g.stats_out[(2 * half + 1) * g.r + key] = rstd;
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// (behind merge_statistics, which reads the counts)
 __device__ __forceinline__ void count_batch(const SelectArgs& g) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (g.count_batch[0]) *g.count_batch[0] += 1;
     if (g.count_batch[1]) *g.count_batch[1] += 1;
   }
-  if (blockIdx.x == 0 && !g.stats && g.run_mean[0] && g.stats_out) {   // eval mode: the statistics a backward pass reads
+  if (blockIdx.x == 0 && !g.stats && !g.part_mean && g.run_mean[0] && g.stats_out) {   // eval mode: the statistics a backward pass reads
     for (int i = threadIdx.x; i < 2 * g.r; i += blockDim.x) {
       const int half = i >= g.r, key = i - half * g.r;
       g.stats_out[(2 * half) * g.r + key] = load_score(g.run_mean[half], key, g.stat_dt);
@@ -72,24 +137,45 @@ __device__ __forceinline__ float normalise_one(float v, const SelectArgs& g, con
   return round_score((v - mean) * rstd, dt);
 }
 
+// Mean and 1/sqrt(var + eps) of this lane's keys: g.stats, or (eval mode) the running buffers with the hardware's reciprocal square root (1 ulp), as in
+// stats_out, or a block's own merge (merged: the LDS that merge_statistics filled).  Held for all of a wave's tokens up to 8 keys a lane.
+template <int R>
+struct NormKeys {
+  static constexpr bool kHeld = R <= 8;
+  float mean[2][kHeld ? R : 1], rstd[2][kHeld ? R : 1];
+  __device__ __forceinline__ static void one(const SelectArgs& g, const float* stats, int half, int key, float& mean, float& rstd) {
+    if (stats) {
+      mean = stats[(2 * half) * g.r + key];
+      rstd = stats[(2 * half + 1) * g.r + key];
+    } else {
+      mean = load_score(g.run_mean[half], key, g.stat_dt);
+      rstd = __builtin_amdgcn_rsqf(load_score(g.run_var[half], key, g.stat_dt) + g.eps);
+    }
+  }
+  __device__ __forceinline__ NormKeys(const SelectArgs& g, const float* stats, int lane) {
+    if constexpr (kHeld) {
+      if (!stats && !g.run_mean[0]) return;
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int a = 0; a < R; ++a) one(g, stats, half, min(a * kWave + lane, g.r - 1), mean[half][a], rstd[half][a]);
+    }
+  }
+};
+
 // BatchNorm (affine-free) then log-softmax of one half, in place: v holds the raw projection
 // of key a*64+lane (NaN-free -inf padding past r).  Each stage rounds to the storage dtype
 // where the reference's torch ops do (BN output, log-softmax output; omni_moe.py:70-78).
 template <int R>
-__device__ __forceinline__ void normalise_half(float (&v)[R], const SelectArgs& g, const int half, int r, int lane, int dt) {
+__device__ __forceinline__ void normalise_half(float (&v)[R], const SelectArgs& g, const NormKeys<R>& norm, const float* stats, const int half, int r, int lane, int dt) {
   float m = kNegInf;
 #pragma unroll
   for (int a = 0; a < R; ++a) {
     const int key = a * kWave + lane;
     if (key < r) {
       float mean, rstd;
-      if (g.stats) {
-        mean = g.stats[(2 * half) * r + key];
-        rstd = g.stats[(2 * half + 1) * r + key];
-      } else {                                   // per token and key: the hardware's reciprocal square root (1 ulp), as in stats_out
-        mean = load_score(g.run_mean[half], key, g.stat_dt);
-        rstd = __builtin_amdgcn_rsqf(load_score(g.run_var[half], key, g.stat_dt) + g.eps);
-      }
+      if constexpr (NormKeys<R>::kHeld) { mean = norm.mean[half][a]; rstd = norm.rstd[half][a]; }
+      else NormKeys<R>::one(g, stats, half, key, mean, rstd);
       v[a] = round_score((v[a] - mean) * rstd, dt);
     }
     m = fmaxf(m, v[a]);
@@ -270,9 +356,10 @@ __device__ __forceinline__ uint32_t sorted_key(const uint32_t (&v)[R], int i) {
   return r0;
 }
 
-// Same selection as router_select_kernel for bf16 / f16 storage, on packed keys: the tokens of wave `wave` of `num_waves`.
+// Same selection as router_select_kernel for bf16 / f16 storage, on packed keys: the tokens of wave `wave` of `num_waves`.  stats: g.stats, or what the
+// block merged.
 template <int R, int C>
-__device__ __forceinline__ void select_packed(const SelectArgs& g, const int wave, const int num_waves) {
+__device__ __forceinline__ void select_packed(const SelectArgs& g, const int wave, const int num_waves, const float* stats) {
   const int lane = lane_id();
   const int r = g.r, k = g.k, kp = g.kp, dt = g.dt;
 
@@ -288,6 +375,7 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
   };
   constexpr bool kPrefetch = R <= 2;              // beyond that the extra live registers cost a wave per SIMD
   if (kPrefetch && wave < g.num_tokens) load_raw(wave);
+  const NormKeys<R> norm(g, stats, lane);
   int cell[C];
   candidate_cells<R, C>(cell, g, kp, lane);
 
@@ -301,9 +389,9 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
       sy[a] = kPrefetch ? ry[a] : ok ? load_score(g.ly, int64_t(t) * g.row_stride + key, dt) : kNegInf;
     }
     if (kPrefetch && t + num_waves < g.num_tokens) load_raw(t + num_waves);
-    if (g.stats || g.run_mean[0]) {
-      normalise_half<R>(sx, g, 0, r, lane, dt);
-      normalise_half<R>(sy, g, 1, r, lane, dt);
+    if (stats || g.run_mean[0]) {
+      normalise_half<R>(sx, g, norm, stats, 0, r, lane, dt);
+      normalise_half<R>(sy, g, norm, stats, 1, r, lane, dt);
     }
     uint32_t kx[R], ky[R];
 #pragma unroll
@@ -348,6 +436,9 @@ static inline int num_cells(int k, int kp) {
   for (int a = 0; a < kp; ++a) n += (kp < k / (a + 1)) ? kp : k / (a + 1);
   return n;
 }
+
+// Whether a joint launch's blocks merge the batch statistics: up to 128 KiB of them to a block
+static inline bool merge_here(int64_t num_tokens, int r) { return r <= kMergeKeys && (num_tokens + kBnRows - 1) / kBnRows * 2 * r <= 16384; }
 
 // What select_packed and its kernels want filled in beside the caller's fields; returns the candidate cells per lane
 static inline int prepare_select(SelectArgs& g) {

@@ -788,3 +788,35 @@ def test_layer_with_rows_beyond_the_tile_kernels_reach(device):
     want = h @ wd.t() + experts
     # h rounds alike but for last bits here and there; the sum of 4 million products runs in 32 bits, over partial sums of one wave each
     assert (got - want).abs().max().item() <= 4 * 2.0 ** -7 * max(1.0, want.abs().max().item())
+
+
+# one strip, ragged strips, the most strips a block merges at 64 keys and one more, 8 to 128 keys; 136 keys: the merge's own launch
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("case", [(2, 8), (33, 64), (700, 104), (2048, 128), (4096, 64), (4100, 64), (300, 136)], ids=lambda c: "T%d-r%d" % c)
+def test_joint_batch_statistics_equal_the_router_stage(case, dtype, device):
+    """A small layer merges the batch statistics inside its joint launches: buffers and counts as the router stage (which launches the merge) leaves them on the
+    same input, to the last bit of an fp32 result (double sums in another order) rounded to the buffers' type."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    from omni_moe.ops import hip
+    T, r = case
+    H, I, k = 64, 128, 8
+    print(f"joint statistics T={T} r={r} {dtype}", flush=True)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", r * r, k)).to(device=device, dtype=dtype)
+    g = torch.Generator(device=device).manual_seed(T + r)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, 0.05, generator=g)
+        for n in (layer.router_norm_x, layer.router_norm_y):
+            n.running_mean.normal_(0.0, 0.3, generator=g)
+            n.running_var.uniform_(0.5, 1.5, generator=g)
+        x = torch.empty(1, T, H, device=device, dtype=dtype).normal_(0.0, 1.0, generator=g)
+        stats = [b.clone() for n in (layer.router_norm_x, layer.router_norm_y) for b in (n.running_mean, n.running_var, n.num_batches_tracked)]
+        hip.hip_omni_router_fwd_func(x[0], layer.router_gate_x.weight, layer.router_gate_y.weight, *stats, k, training=True)
+        layer(x)
+    got = [b for n in (layer.router_norm_x, layer.router_norm_y) for b in (n.running_mean, n.running_var, n.num_batches_tracked)]
+    ulp = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -22}[dtype]      # neighbours of the buffers' type
+    for a, b in zip(got, stats):
+        if a.dtype == torch.int64:
+            assert torch.equal(a, b)
+        else:
+            assert ((a.float() - b.float()).abs() <= 1.01 * ulp * b.float().abs() + 1e-6).all()     # 1e-6: where the two terms of the moving average cancel
