@@ -346,6 +346,49 @@ __device__ __forceinline__ void ktop64_2(uint32_t (&k0)[R], uint32_t (&k1)[R], c
   }
 }
 
+// The same for the kp <= 32 largest alone, from the few keys that can be among them: of 64 lanes' largest keys the kp-th is a bound that kp keys reach, so
+// every key below it is out; what is left (for scores in no particular order about 42 of 512 keys at kp = 32) goes through LDS into one register and is
+// sorted there.  Two sorts of 64 keys instead of R and the merges: 32768 tokens, 2 x 512 keys, k = 32: 211 -> 165 us.  More than 64 left, or fewer than kp lanes with a key: all of them, as above.
+constexpr int kPruneTop = 32, kPruneWaves = 8;
+template <int R>
+__device__ __forceinline__ void ktop_pruned_2(uint32_t (&k0)[R], uint32_t (&k1)[R], const int kp, const int lane) {
+  __shared__ uint32_t pool[kPruneWaves][2][kWave];
+  uint32_t (*mine)[kWave] = pool[(threadIdx.x >> 6) % kPruneWaves];
+  uint32_t m0[1] = {k0[0]}, m1[1] = {k1[0]};
+#pragma unroll
+  for (int a = 1; a < R; ++a) {
+    m0[0] = max(m0[0], k0[a]);
+    m1[0] = max(m1[0], k1[a]);
+  }
+  ksizes<1, 2>(m0, m1, lane, true);
+  const uint32_t t0 = (uint32_t)__builtin_amdgcn_readlane((int)m0[0], kp - 1), t1 = (uint32_t)__builtin_amdgcn_readlane((int)m1[0], kp - 1);
+  int n0 = 0, n1 = 0;
+#pragma unroll
+  for (int a = 0; a < R; ++a) {
+    n0 += __popcll(__ballot(k0[a] >= t0));
+    n1 += __popcll(__ballot(k1[a] >= t1));
+  }
+  if (t0 == 0u || t1 == 0u || n0 > kWave || n1 > kWave) {
+    ktop64_2<R>(k0, k1, lane);
+    return;
+  }
+  int at0 = 0, at1 = 0;
+#pragma unroll
+  for (int a = 0; a < R; ++a) {
+    const uint64_t b0 = __ballot(k0[a] >= t0), b1 = __ballot(k1[a] >= t1);
+    if (k0[a] >= t0) mine[0][at0 + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b0 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b0, 0u))] = k0[a];
+    if (k1[a] >= t1) mine[1][at1 + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b1 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b1, 0u))] = k1[a];
+    at0 += __popcll(b0);
+    at1 += __popcll(b1);
+  }
+  __builtin_amdgcn_wave_barrier();                              // a wave's LDS instructions take effect in order
+  uint32_t x[1] = {lane < n0 ? mine[0][lane] : 0u}, y[1] = {lane < n1 ? mine[1][lane] : 0u};
+  __builtin_amdgcn_wave_barrier();
+  ksizes<1, 2>(x, y, lane, true);
+  k0[0] = x[0];
+  k1[0] = y[0];
+}
+
 template <int R>
 __device__ __forceinline__ uint32_t sorted_key(const uint32_t (&v)[R], int i) {
   uint32_t r0 = (uint32_t)__shfl((int)v[0], i & 63, kWave);
@@ -400,8 +443,13 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
       kx[a] = key < r ? make_key(sx[a], key, dt) : 0u;          // 0 sorts behind every real key
       ky[a] = key < r ? make_key(sy[a], key, dt) : 0u;
     }
-    if (R > kUnrollMaxR && kp <= kWave) ktop64_2<R>(kx, ky, lane);    // uniform: kp comes with the arguments
-    else ksort2<R>(kx, ky, lane);
+    if constexpr (R > kUnrollMaxR) {                             // uniform: kp comes with the arguments
+      if (kp <= kPruneTop) ktop_pruned_2<R>(kx, ky, kp, lane);
+      else if (kp <= kWave) ktop64_2<R>(kx, ky, lane);
+      else ksort2<R>(kx, ky, lane);
+    } else {
+      ksort2<R>(kx, ky, lane);
+    }
 
     uint32_t ck[C];
 #pragma unroll

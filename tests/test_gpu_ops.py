@@ -92,6 +92,28 @@ def test_router_select_contract(device):
     assert torch.equal(s1, s2) and torch.equal(i1, i2)
 
 
+# keys per half beyond 128: two to eight to a lane.  "lanes": the best keys sit in four lanes (more than 64 reach the bound that the lanes' best give, the full
+# sort takes over); "ties": a handful of values
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("kind", ["random", "lanes", "ties", "descending"])
+@pytest.mark.parametrize("r,k", [(129, 2), (200, 16), (256, 32), (300, 34), (512, 32), (512, 30)])
+def test_router_select_many_keys_bit_exact(r, k, kind, dtype, device):
+    T = 67
+    g = torch.Generator().manual_seed(r + k)
+    s = torch.randn(2, T, r, generator=g)
+    if kind == "lanes":
+        s = s + 8.0 * ((torch.arange(r) % 64) < 4)
+    elif kind == "ties":
+        s = torch.randint(0, 5, (2, T, r), generator=g).float()
+    elif kind == "descending":
+        s = -torch.arange(r).float().expand(2, T, r) * 0.05
+    lx, ly = (torch.log_softmax(h, -1).to(dtype) for h in s)
+    print(f"router select r={r} k={k} {kind} {dtype}", flush=True)
+    got_s, got_i = _ops().hip_omni_router_func(lx.to(device), ly.to(device), r, k)
+    want_s, want_i = oracle.router_select(lx, ly, r, k)
+    assert torch.equal(got_i.cpu(), want_i) and torch.equal(got_s.cpu(), want_s)
+
+
 # ---------------------------------------------------------------- schedule
 SCHED_CASES = [(512, 8, 1024, "uniform"), (4096, 16, 4096, "uniform"), (16384, 16, 4096, "uniform"),
                (4096, 32, 262144, "zipf"), (1000, 6, 5000, "zipf"), (3, 2, 7, "uniform"), (2048, 16, 64, "hot"),
