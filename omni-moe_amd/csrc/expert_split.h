@@ -216,12 +216,12 @@ static inline int split_lanes_per_row(int hidden, int elem_bytes, int slices) {
 // keeps a larger part of the table's rows in its 4 MiB L2.  Time with four over eight, bf16, 4096 to 32768 tokens x 16 or 32, ids uniform:
 //   rows  512 B, 1 KiB, 1.5 KiB, 2.5 KiB: 0.2-0.6, 0.4-0.9, 0.7-0.9, 0.8-1.0 at tables of 0.5 to 640 MB (2.5 KiB x 40 MB: 1.0-1.07)
 //   rows  2 KiB: 0.84-1.04 up to 16 MB, 1.1-1.35 at 32 MB, 0.85-0.99 from 128 MB on
-//   rows  4 KiB: 0.88-1.01 up to 16 MB, 1.1-1.5 at 32 and 64 MB, 0.94-1.04 from 256 MB on
+//   rows  4 KiB: 0.88-1.01 up to 16 MB, 1.1-1.5 at 32 and 64 MB, 0.94-1.04 from 256 MB on; 1 GB with the ids of a router that keeps to 3700 rows 1.05-1.1
 //   rows  8 KiB: eight slices of 64 lanes
 static inline int split_slices(int hidden, int64_t num_experts, int elem_bytes) {
   const int64_t row = (int64_t)hidden * elem_bytes, table = num_experts * row;
   const int four = split_lanes_per_row(hidden, elem_bytes, 4);
-  if (four >= 5 && (row < 2048 || table <= (24ll << 20) || table >= (128ll << 20))) return 4;
+  if (four >= 5 && (row < 2048 || table <= (24ll << 20) || (row < 4096 && table >= (128ll << 20)))) return 4;
   return split_lanes_per_row(hidden, elem_bytes, kSlices) ? kSlices : four >= 5 ? 4 : 0;
 }
 // Rows beyond 8 KiB: the smallest number of column blocks, each 8 slices of a power-of-two number of lanes, that the row cuts into; 0 if there is none (up

@@ -183,10 +183,10 @@ __global__ __launch_bounds__(kFewThreads, 2) void few_middle_kernel(const Middle
   if constexpr (kSelect) {
     if ((int)blockIdx.x < g.select_blocks) {
       const int first = (int)blockIdx.x * kFewWaves + wave, all = g.select_blocks * kFewWaves;
-      if (g.select_regs <= 1) select_packed<1, C>(g.select, first, all, g.select.stats);
-      else if (g.select_regs <= 2) select_packed<2, C>(g.select, first, all, g.select.stats);
-      else if (g.select_regs <= 4) select_packed<4, C>(g.select, first, all, g.select.stats);
-      else select_packed<8, C>(g.select, first, all, g.select.stats);
+      if (g.select_regs <= 1) select_packed<DT, 1, C>(g.select, first, all, g.select.stats);
+      else if (g.select_regs <= 2) select_packed<DT, 2, C>(g.select, first, all, g.select.stats);
+      else if (g.select_regs <= 4) select_packed<DT, 4, C>(g.select, first, all, g.select.stats);
+      else select_packed<DT, 8, C>(g.select, first, all, g.select.stats);
       return;
     }
   }

@@ -750,10 +750,10 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
     }
     auto select = [&](auto cells) {
       constexpr int C = decltype(cells)::value;
-      if (g.regs <= 1) select_packed<1, C>(g.select, first, all, stats);
-      else if (g.regs <= 2) select_packed<2, C>(g.select, first, all, stats);
-      else if (g.regs <= 4) select_packed<4, C>(g.select, first, all, stats);
-      else select_packed<8, C>(g.select, first, all, stats);
+      if (g.regs <= 1) select_packed<DT, 1, C>(g.select, first, all, stats);
+      else if (g.regs <= 2) select_packed<DT, 2, C>(g.select, first, all, stats);
+      else if (g.regs <= 4) select_packed<DT, 4, C>(g.select, first, all, stats);
+      else select_packed<DT, 8, C>(g.select, first, all, stats);
     };
     if (g.cells <= 1) select(std::integral_constant<int, 1>{});
     else select(std::integral_constant<int, 2>{});

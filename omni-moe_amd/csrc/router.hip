@@ -192,7 +192,8 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
   const int lane = lane_id();
   const int wave = blockIdx.x * kRouterWaves + (threadIdx.x >> 6);
   const int num_waves = gridDim.x * kRouterWaves;
-  const int r = g.r, k = g.k, kp = g.kp, dt = g.dt;
+  using S = Elem<kF32>;                           // (16-bit scores travel packed)
+  const int r = g.r, k = g.k, kp = g.kp;
 
   float rx[R], ry[R];                             // raw scores of the token about to be selected
   auto load_raw = [&](int t) __attribute__((always_inline)) {
@@ -200,8 +201,8 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
     for (int a = 0; a < R; ++a) {
       const int key = a * kWave + lane;
       const bool ok = key < r;
-      rx[a] = ok ? load_score(g.lx, int64_t(t) * g.row_stride + key, dt) : kNegInf;
-      ry[a] = ok ? load_score(g.ly, int64_t(t) * g.row_stride + key, dt) : kNegInf;
+      rx[a] = ok ? S::load(g.lx, int64_t(t) * g.row_stride + key) : kNegInf;
+      ry[a] = ok ? S::load(g.ly, int64_t(t) * g.row_stride + key) : kNegInf;
     }
   };
   constexpr bool kPrefetch = R <= 2;              // beyond that the extra live registers cost a wave per SIMD
@@ -218,14 +219,14 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
     for (int a = 0; a < R; ++a) {
       const int key = a * kWave + lane;
       const bool ok = key < r;
-      sx[a] = kPrefetch ? rx[a] : ok ? load_score(g.lx, int64_t(t) * g.row_stride + key, dt) : kNegInf;
-      sy[a] = kPrefetch ? ry[a] : ok ? load_score(g.ly, int64_t(t) * g.row_stride + key, dt) : kNegInf;
+      sx[a] = kPrefetch ? rx[a] : ok ? S::load(g.lx, int64_t(t) * g.row_stride + key) : kNegInf;
+      sy[a] = kPrefetch ? ry[a] : ok ? S::load(g.ly, int64_t(t) * g.row_stride + key) : kNegInf;
       px[a] = py[a] = key;
     }
     if (kPrefetch && t + num_waves < g.num_tokens) load_raw(t + num_waves);
     if (stats || g.run_mean[0]) {
-      normalise_half<R>(sx, g, norm, stats, 0, r, lane, dt);
-      normalise_half<R>(sy, g, norm, stats, 1, r, lane, dt);
+      normalise_half<kF32, R>(sx, g, norm, stats, 0, r, lane);
+      normalise_half<kF32, R>(sy, g, norm, stats, 1, r, lane);
     }
     bitonic_sort2<R>(sx, px, sy, py, lane);
 
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
       const bool ok = cell[c] >= 0;
       const int a = ok ? (cell[c] >> 8) : 0, b = ok ? (cell[c] & 255) : 0;
       const float va = sorted_item<R>(sx, a), vb = sorted_item<R>(sy, b);
-      cs[c] = ok ? round_score(va + vb, dt) : kNegInf;
+      cs[c] = ok ? va + vb : kNegInf;
       cp[c] = ok ? cell[c] : (0x40000000 | (c * kWave + lane));
     }
     bitonic_sort<C>(cs, cp, lane);
@@ -250,32 +251,32 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
       const int ia = sorted_item<R>(px, a), ib = sorted_item<R>(py, b);
       if (ok) {
         const int64_t o = int64_t(t) * k + j;
-        if (g.scores) store_score(g.scores, o, cs[c], dt);
-        if (g.gates) store_score(g.gates, o, expf(cs[c]), dt);      // gate = P(x key) * P(y key)
+        if (g.scores) S::store(g.scores, o, cs[c]);
+        if (g.gates) S::store(g.gates, o, expf(cs[c]));      // gate = P(x key) * P(y key)
         g.indices[o] = ia * r + ib;
       }
     }
   }
 }
 
-template <int R, int C>
+template <int DT, int R, int C>
 __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_packed_kernel(const SelectArgs g) {
   count_batch(g);
-  select_packed<R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats);
+  select_packed<DT, R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats);
 }
 
 // More keys per half than a wave's registers hold (r > 1024): 16-bit scores, k' <= 64.  The row is walked in chunks of
 // 512 keys per half: each chunk's 64 best (ktop64_2) are merged into the running 64 best by the same max(A[i], B[63-i])
 // step.  With the BatchNorm + log-softmax front the row is read three times (maximum, sum of exponentials, keys), each
 // time with the arithmetic and the per-lane summation order of normalise_half, so a row gives the bits it would give there.
-template <int C>
+template <int DT, int C>
 __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_chunked_kernel(const SelectArgs g) {
   constexpr int RC = 8, kChunk = RC * kWave;
   count_batch(g);
   const int lane = lane_id();
   const int wave = blockIdx.x * kRouterWaves + (threadIdx.x >> 6);
   const int num_waves = gridDim.x * kRouterWaves;
-  const int r = g.r, k = g.k, kp = g.kp, dt = g.dt;
+  const int r = g.r, k = g.k, kp = g.kp;
   const int chunks = (r + kChunk - 1) / kChunk;
   const bool norm = g.stats || g.run_mean[0];
   int cell[C];
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_chunked_ker
 #pragma unroll
           for (int a = 0; a < RC; ++a) {
             const int key = c * kChunk + a * kWave + lane;
-            if (key < r) m = fmaxf(m, normalise_one(load_score(src, row + key, dt), g, half, key, r, dt));
+            if (key < r) m = fmaxf(m, normalise_one<DT>(Elem<DT>::load(src, row + key), g, half, key, r));
           }
         m = wave_max(m);
         float e = 0.f;
@@ -300,7 +301,7 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_chunked_ker
 #pragma unroll
           for (int a = 0; a < RC; ++a) {
             const int key = c * kChunk + a * kWave + lane;
-            e += key < r ? expf(normalise_one(load_score(src, row + key, dt), g, half, key, r, dt) - m) : 0.f;
+            e += key < r ? expf(normalise_one<DT>(Elem<DT>::load(src, row + key), g, half, key, r) - m) : 0.f;
           }
         mx[half] = m;
         lse[half] = logf(wave_sum(e));
@@ -313,13 +314,13 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_chunked_ker
       for (int a = 0; a < RC; ++a) {
         const int key = c * kChunk + a * kWave + lane;
         const bool ok = key < r;
-        float vx = ok ? load_score(g.lx, row + key, dt) : 0.f, vy = ok ? load_score(g.ly, row + key, dt) : 0.f;
+        float vx = ok ? Elem<DT>::load(g.lx, row + key) : 0.f, vy = ok ? Elem<DT>::load(g.ly, row + key) : 0.f;
         if (norm && ok) {
-          vx = round_score(normalise_one(vx, g, 0, key, r, dt) - mx[0] - lse[0], dt);
-          vy = round_score(normalise_one(vy, g, 1, key, r, dt) - mx[1] - lse[1], dt);
+          vx = Elem<DT>::round(normalise_one<DT>(vx, g, 0, key, r) - mx[0] - lse[0]);
+          vy = Elem<DT>::round(normalise_one<DT>(vy, g, 1, key, r) - mx[1] - lse[1]);
         }
-        kx[a] = ok ? make_key(vx, key, dt) : 0u;    // 0 sorts behind every real key
-        ky[a] = ok ? make_key(vy, key, dt) : 0u;
+        kx[a] = ok ? make_key<DT>(vx, key) : 0u;    // 0 sorts behind every real key
+        ky[a] = ok ? make_key<DT>(vy, key) : 0u;
       }
       ktop64_2<RC>(kx, ky, lane);
       uint32_t x[1] = {max(bx, (uint32_t)__shfl((int)kx[0], 63 - lane, kWave))};
@@ -335,8 +336,8 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_chunked_ker
     for (int c = 0; c < C; ++c) {
       const bool ok = cell[c] >= 0;
       const int a = ok ? (cell[c] >> 8) : 0, b = ok ? (cell[c] & 255) : 0;
-      const float va = key_score(sorted_key<1>(sx, a), dt), vb = key_score(sorted_key<1>(sy, b), dt);
-      ck[c] = ok ? make_key(round_score(va + vb, dt), cell[c], dt) : 0u;
+      const float va = key_score<DT>(sorted_key<1>(sx, a)), vb = key_score<DT>(sorted_key<1>(sy, b));
+      ck[c] = ok ? make_key<DT>(Elem<DT>::round(va + vb), cell[c]) : 0u;
     }
     ksort<C>(ck, lane);
 
@@ -349,9 +350,9 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_chunked_ker
       const int ia = key_payload(sorted_key<1>(sx, pl >> 8)), ib = key_payload(sorted_key<1>(sy, pl & 255));
       if (ok) {
         const int64_t o = int64_t(t) * k + j;
-        const float sc = key_score(ck[c], dt);
-        if (g.scores) store_score(g.scores, o, sc, dt);
-        if (g.gates) store_score(g.gates, o, expf(sc), dt);
+        const float sc = key_score<DT>(ck[c]);
+        if (g.scores) Elem<DT>::store(g.scores, o, sc);
+        if (g.gates) Elem<DT>::store(g.gates, o, expf(sc));
         g.indices[o] = ia * r + ib;
       }
     }
@@ -362,7 +363,8 @@ template <int C>
 static hipError_t launch_select_chunked(const SelectArgs& g, hipStream_t s) {
   int64_t blocks = ((int64_t)g.num_tokens + kRouterWaves - 1) / kRouterWaves;
   if (blocks > 256 * 16) blocks = 256 * 16;
-  hipLaunchKernelGGL((router_select_chunked_kernel<C>), dim3((unsigned)blocks), dim3(kRouterWaves * kWave), 0, s, g);
+  if (g.dt == kBF16) hipLaunchKernelGGL((router_select_chunked_kernel<kBF16, C>), dim3((unsigned)blocks), dim3(kRouterWaves * kWave), 0, s, g);
+  else hipLaunchKernelGGL((router_select_chunked_kernel<kF16, C>), dim3((unsigned)blocks), dim3(kRouterWaves * kWave), 0, s, g);
   return hipGetLastError();
 }
 
@@ -378,8 +380,10 @@ static hipError_t launch_select(const SelectArgs& g, hipStream_t s) {
   if (blocks > 256 * 16) blocks = 256 * 16;     // waves loop over tokens beyond that
   if (g.dt == kF32)
     hipLaunchKernelGGL((router_select_kernel<R, C>), dim3((unsigned)blocks), dim3(kRouterWaves * kWave), 0, s, g);
+  else if (g.dt == kBF16)
+    hipLaunchKernelGGL((router_select_packed_kernel<kBF16, R, C>), dim3((unsigned)blocks), dim3(kRouterWaves * kWave), 0, s, g);
   else
-    hipLaunchKernelGGL((router_select_packed_kernel<R, C>), dim3((unsigned)blocks), dim3(kRouterWaves * kWave), 0, s, g);
+    hipLaunchKernelGGL((router_select_packed_kernel<kF16, R, C>), dim3((unsigned)blocks), dim3(kRouterWaves * kWave), 0, s, g);
   return hipGetLastError();
 }
 

@@ -5,13 +5,10 @@
 
 namespace omni {
 
-// Storage dtype handled at run time (one uniform branch per access) to keep the number of
-// kernel instantiations at |R| x |C|.
+// Storage dtype handled at run time, one uniform branch per access: for the norms' buffers, whose dtype is their own.  (The scores' dtype is a template
+// parameter: with a branch to every load and rounding a token was 142 branches to 817 vector instructions, and its loads waited for one another.)
 __device__ __forceinline__ float load_score(const void* p, int64_t i, int dt) {
   return dt == kBF16 ? Elem<kBF16>::load(p, i) : dt == kF16 ? Elem<kF16>::load(p, i) : Elem<kF32>::load(p, i);
-}
-__device__ __forceinline__ float round_score(float v, int dt) {
-  return dt == kBF16 ? Elem<kBF16>::round(v) : dt == kF16 ? Elem<kF16>::round(v) : v;
 }
 __device__ __forceinline__ void store_score(void* p, int64_t i, float v, int dt) {
   if (dt == kBF16) Elem<kBF16>::store(p, i, v);
@@ -125,7 +122,8 @@ __device__ __forceinline__ void count_batch(const SelectArgs& g) {
 }
 
 // BatchNorm (affine-free) of one raw projection value, rounded to the storage dtype as the reference's BatchNorm output is
-__device__ __forceinline__ float normalise_one(float v, const SelectArgs& g, const int half, const int key, const int r, const int dt) {
+template <int DT>
+__device__ __forceinline__ float normalise_one(float v, const SelectArgs& g, const int half, const int key, const int r) {
   float mean, rstd;
   if (g.stats) {
     mean = g.stats[(2 * half) * r + key];
@@ -134,7 +132,7 @@ __device__ __forceinline__ float normalise_one(float v, const SelectArgs& g, con
     mean = load_score(g.run_mean[half], key, g.stat_dt);
     rstd = __builtin_amdgcn_rsqf(load_score(g.run_var[half], key, g.stat_dt) + g.eps);
   }
-  return round_score((v - mean) * rstd, dt);
+  return Elem<DT>::round((v - mean) * rstd);
 }
 
 // Mean and 1/sqrt(var + eps) of this lane's keys: g.stats, or (eval mode) the running buffers with the hardware's reciprocal square root (1 ulp), as in
@@ -152,13 +150,31 @@ struct NormKeys {
       rstd = __builtin_amdgcn_rsqf(load_score(g.run_var[half], key, g.stat_dt) + g.eps);
     }
   }
+  template <class Mean, class Rstd>
+  __device__ __forceinline__ void fill(const SelectArgs& g, int lane, Mean&& mean_of, Rstd&& rstd_of) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int a = 0; a < R; ++a) {
+        const int key = min(a * kWave + lane, g.r - 1);
+        mean[half][a] = mean_of(half, key);
+        rstd[half][a] = rstd_of(half, key);
+      }
+  }
   __device__ __forceinline__ NormKeys(const SelectArgs& g, const float* stats, int lane) {
     if constexpr (kHeld) {
-      if (!stats && !g.run_mean[0]) return;
-#pragma unroll
-      for (int half = 0; half < 2; ++half)
-#pragma unroll
-        for (int a = 0; a < R; ++a) one(g, stats, half, min(a * kWave + lane, g.r - 1), mean[half][a], rstd[half][a]);
+      if (stats) {
+        fill(g, lane, [&](int half, int key) { return stats[(2 * half) * g.r + key]; }, [&](int half, int key) { return stats[(2 * half + 1) * g.r + key]; });
+      } else if (g.run_mean[0]) {
+        auto buffers = [&](auto dt) {
+          using B = Elem<decltype(dt)::value>;
+          fill(g, lane, [&](int half, int key) { return B::load(g.run_mean[half], key); },
+               [&](int half, int key) { return __builtin_amdgcn_rsqf(B::load(g.run_var[half], key) + g.eps); });
+        };
+        if (g.stat_dt == kBF16) buffers(std::integral_constant<int, kBF16>{});
+        else if (g.stat_dt == kF16) buffers(std::integral_constant<int, kF16>{});
+        else buffers(std::integral_constant<int, kF32>{});
+      }
     }
   }
 };
@@ -166,8 +182,8 @@ struct NormKeys {
 // BatchNorm (affine-free) then log-softmax of one half, in place: v holds the raw projection
 // of key a*64+lane (NaN-free -inf padding past r).  Each stage rounds to the storage dtype
 // where the reference's torch ops do (BN output, log-softmax output; omni_moe.py:70-78).
-template <int R>
-__device__ __forceinline__ void normalise_half(float (&v)[R], const SelectArgs& g, const NormKeys<R>& norm, const float* stats, const int half, int r, int lane, int dt) {
+template <int DT, int R>
+__device__ __forceinline__ void normalise_half(float (&v)[R], const SelectArgs& g, const NormKeys<R>& norm, const float* stats, const int half, int r, int lane) {
   float m = kNegInf;
 #pragma unroll
   for (int a = 0; a < R; ++a) {
@@ -176,7 +192,7 @@ __device__ __forceinline__ void normalise_half(float (&v)[R], const SelectArgs& 
       float mean, rstd;
       if constexpr (NormKeys<R>::kHeld) { mean = norm.mean[half][a]; rstd = norm.rstd[half][a]; }
       else NormKeys<R>::one(g, stats, half, key, mean, rstd);
-      v[a] = round_score((v[a] - mean) * rstd, dt);
+      v[a] = Elem<DT>::round((v[a] - mean) * rstd);
     }
     m = fmaxf(m, v[a]);
   }
@@ -187,7 +203,7 @@ __device__ __forceinline__ void normalise_half(float (&v)[R], const SelectArgs& 
   const float lse = logf(wave_sum(e));
 #pragma unroll
   for (int a = 0; a < R; ++a)
-    if (a * kWave + lane < r) v[a] = round_score(v[a] - m - lse, dt);
+    if (a * kWave + lane < r) v[a] = Elem<DT>::round(v[a] - m - lse);
 }
 
 // This lane's candidate cells: cell index ci = c*64+lane enumerates rows a = 0..kp-1 with
@@ -241,14 +257,16 @@ __device__ __forceinline__ void candidate_cells(int (&cell)[C], const SelectArgs
 // Four times fewer VALU instructions than the (float, int) pairs the fp32 path needs.
 __device__ __forceinline__ uint32_t ord16(uint32_t bits) { return bits ^ ((bits & 0x8000u) ? 0xFFFFu : 0x8000u); }
 __device__ __forceinline__ uint32_t unord16(uint32_t u) { return u ^ ((u & 0x8000u) ? 0x8000u : 0xFFFFu); }
-__device__ __forceinline__ uint32_t make_key(float v, int payload, int dt) {      // v is representable in dt
+template <int DT>
+__device__ __forceinline__ uint32_t make_key(float v, int payload) {              // v is representable in DT
   v += 0.0f;                                                                      // -0 -> +0: they compare equal as floats
-  const uint32_t bits = dt == kBF16 ? (uint32_t)f32_to_bf16_bits(v) : (uint32_t)f32_to_f16_bits(v);
+  const uint32_t bits = DT == kBF16 ? __float_as_uint(v) >> 16 : (uint32_t)f32_to_f16_bits(v);
   return (ord16(bits) << 16) | (0xFFFFu - (uint32_t)payload);
 }
-__device__ __forceinline__ float key_score(uint32_t key, int dt) {
+template <int DT>
+__device__ __forceinline__ float key_score(uint32_t key) {
   const uint32_t bits = unord16(key >> 16);
-  return dt == kBF16 ? bf16_bits_to_f32((uint16_t)bits) : f16_bits_to_f32((uint16_t)bits);
+  return DT == kBF16 ? bf16_bits_to_f32((uint16_t)bits) : f16_bits_to_f32((uint16_t)bits);
 }
 __device__ __forceinline__ int key_payload(uint32_t key) { return (int)(0xFFFFu - (key & 0xFFFFu)); }
 
@@ -401,10 +419,10 @@ __device__ __forceinline__ uint32_t sorted_key(const uint32_t (&v)[R], int i) {
 
 // Same selection as router_select_kernel for bf16 / f16 storage, on packed keys: the tokens of wave `wave` of `num_waves`.  stats: g.stats, or what the
 // block merged.
-template <int R, int C>
+template <int DT, int R, int C>
 __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wave, const int num_waves, const float* stats) {
   const int lane = lane_id();
-  const int r = g.r, k = g.k, kp = g.kp, dt = g.dt;
+  const int r = g.r, k = g.k, kp = g.kp;
 
   float rx[R], ry[R];                             // as in router_select_kernel
   auto load_raw = [&](int t) __attribute__((always_inline)) {
@@ -412,8 +430,8 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
     for (int a = 0; a < R; ++a) {
       const int key = a * kWave + lane;
       const bool ok = key < r;
-      rx[a] = ok ? load_score(g.lx, int64_t(t) * g.row_stride + key, dt) : kNegInf;
-      ry[a] = ok ? load_score(g.ly, int64_t(t) * g.row_stride + key, dt) : kNegInf;
+      rx[a] = ok ? Elem<DT>::load(g.lx, int64_t(t) * g.row_stride + key) : kNegInf;
+      ry[a] = ok ? Elem<DT>::load(g.ly, int64_t(t) * g.row_stride + key) : kNegInf;
     }
   };
   constexpr bool kPrefetch = R <= 2;              // beyond that the extra live registers cost a wave per SIMD
@@ -428,20 +446,20 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
     for (int a = 0; a < R; ++a) {
       const int key = a * kWave + lane;
       const bool ok = key < r;
-      sx[a] = kPrefetch ? rx[a] : ok ? load_score(g.lx, int64_t(t) * g.row_stride + key, dt) : kNegInf;
-      sy[a] = kPrefetch ? ry[a] : ok ? load_score(g.ly, int64_t(t) * g.row_stride + key, dt) : kNegInf;
+      sx[a] = kPrefetch ? rx[a] : ok ? Elem<DT>::load(g.lx, int64_t(t) * g.row_stride + key) : kNegInf;
+      sy[a] = kPrefetch ? ry[a] : ok ? Elem<DT>::load(g.ly, int64_t(t) * g.row_stride + key) : kNegInf;
     }
     if (kPrefetch && t + num_waves < g.num_tokens) load_raw(t + num_waves);
     if (stats || g.run_mean[0]) {
-      normalise_half<R>(sx, g, norm, stats, 0, r, lane, dt);
-      normalise_half<R>(sy, g, norm, stats, 1, r, lane, dt);
+      normalise_half<DT, R>(sx, g, norm, stats, 0, r, lane);
+      normalise_half<DT, R>(sy, g, norm, stats, 1, r, lane);
     }
     uint32_t kx[R], ky[R];
 #pragma unroll
     for (int a = 0; a < R; ++a) {
       const int key = a * kWave + lane;
-      kx[a] = key < r ? make_key(sx[a], key, dt) : 0u;          // 0 sorts behind every real key
-      ky[a] = key < r ? make_key(sy[a], key, dt) : 0u;
+      kx[a] = key < r ? make_key<DT>(sx[a], key) : 0u;          // 0 sorts behind every real key
+      ky[a] = key < r ? make_key<DT>(sy[a], key) : 0u;
     }
     if constexpr (R > kUnrollMaxR) {                             // uniform: kp comes with the arguments
       if (kp <= kPruneTop) ktop_pruned_2<R>(kx, ky, kp, lane);
@@ -456,8 +474,8 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
     for (int c = 0; c < C; ++c) {
       const bool ok = cell[c] >= 0;
       const int a = ok ? (cell[c] >> 8) : 0, b = ok ? (cell[c] & 255) : 0;
-      const float va = key_score(sorted_key<R>(kx, a), dt), vb = key_score(sorted_key<R>(ky, b), dt);
-      ck[c] = ok ? make_key(round_score(va + vb, dt), cell[c], dt) : 0u;
+      const float va = key_score<DT>(sorted_key<R>(kx, a)), vb = key_score<DT>(sorted_key<R>(ky, b));
+      ck[c] = ok ? make_key<DT>(Elem<DT>::round(va + vb), cell[c]) : 0u;
     }
     ksort<C>(ck, lane);
 
@@ -470,9 +488,9 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
       const int ia = key_payload(sorted_key<R>(kx, pl >> 8)), ib = key_payload(sorted_key<R>(ky, pl & 255));
       if (ok) {
         const int64_t o = int64_t(t) * k + j;
-        const float sc = key_score(ck[c], dt);
-        if (g.scores) store_score(g.scores, o, sc, dt);
-        if (g.gates) store_score(g.gates, o, expf(sc), dt);         // gate = P(x key) * P(y key)
+        const float sc = key_score<DT>(ck[c]);
+        if (g.scores) Elem<DT>::store(g.scores, o, sc);
+        if (g.gates) Elem<DT>::store(g.gates, o, expf(sc));         // gate = P(x key) * P(y key)
         g.indices[o] = ia * r + ib;
       }
     }
