@@ -157,7 +157,7 @@ static hipError_t launch_gather(const void* x, const void* up, const void* down,
   return hipGetLastError();
 }
 
-// The gather algorithm (rows of at most 8 KiB, 16-bit storage) with the layer's final add
+// The gather algorithm (rows of at most 8 KiB) with the layer's final add
 hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, int64_t T, int H,
                              int k, int64_t N, int dtype, hipStream_t s) {
   const dim3 grid((unsigned)((T + kTokensPerBlock - 1) / kTokensPerBlock)), block(kTokensPerBlock * kWave);
@@ -167,13 +167,14 @@ hipError_t launch_gather_add(const void* x, const void* up, const void* down, co
     return hipGetLastError();
   };
   auto by_row = [&](auto dt) {
-    const int nch = (H + kWave * 8 - 1) / (kWave * 8);
+    constexpr int E = Row16<decltype(dt)::value>::kElems;
+    const int nch = (H + kWave * E - 1) / (kWave * E);
     if (nch <= 1) return go(dt, std::integral_constant<int, 1>{}, std::integral_constant<int, 16>{});
     if (nch <= 2) return go(dt, std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{});
     if (nch <= 4) return go(dt, std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
     return go(dt, std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{});
   };
-  return dtype == kBF16 ? by_row(std::integral_constant<int, kBF16>{}) : by_row(std::integral_constant<int, kF16>{});
+  return dtype == kBF16 ? by_row(std::integral_constant<int, kBF16>{}) : dtype == kF16 ? by_row(std::integral_constant<int, kF16>{}) : by_row(std::integral_constant<int, kF32>{});
 }
 
 template <int DT>

@@ -20,6 +20,7 @@
 #include "few_tokens.h"
 #include "gemm_tiles.h"
 #include "omni_moe_hip.h"
+#include "select.h"
 
 #include <type_traits>
 
@@ -736,11 +737,10 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_ksplit_kernel(const Gemm
 // out the K tiles (32 values, 128-byte rows) as in gemm_ksplit_kernel: a two-stage ring in LDS per wave, no block barrier, the four sums added in
 // wave order: 12.4 and 9.1 us.  Twice the operand traffic of a 64 x 64 tile (32 bytes per cycle and CU), which L2 still carries.
 template <int EPI>
-__global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_small_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gemm_f32_small_block(const GemmArgs& g, const int block, uint8_t* lds) {
   constexpr int TB = EPI == kEpiSwiglu ? 2 : 1, kTile = 32 * 128, kStage = (1 + TB) * kTile, kLoads = 4 * (1 + TB);
-  extern __shared__ __align__(16) uint8_t lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int m0 = (int)(blockIdx.x % g.tiles_m) * 32, n0 = (int)(blockIdx.x / g.tiles_m) * 32;
+  const int m0 = block % g.tiles_m * 32, n0 = block / g.tiles_m * 32;
   const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * 2 * kStage;
   const int row_bytes = g.K * 4;
   const uint64_t a = (uint64_t)g.a + (uint64_t)m0 * (uint32_t)row_bytes;
@@ -814,6 +814,38 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_small_kernel(const G
     }
   gemm_epilogue<kF32, 1, TB, EPI>(g, sum, m0, n0, 0, 0, lane);
 }
+template <int EPI>
+__global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_small_kernel(const GemmArgs g) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  gemm_f32_small_block<EPI>(g, (int)blockIdx.x, lds);
+}
+
+// A layer of such products in single precision: stages that do not depend on each other share a launch, as in 16 bits (gemm_tiles.hip).  Six dependent launches
+// of 4 to 12 us are four: projection | gate/up (the projection's blocks first: half as long), then selection | down projection.
+struct F32Front { GemmArgs router, mlp; int router_blocks; };
+template <int EPI>                    // of the projection: kEpiStats or kEpiPlain
+__global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_front_kernel(const F32Front g) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  if ((int)blockIdx.x < g.router_blocks) gemm_f32_small_block<EPI>(g.router, (int)blockIdx.x, lds);
+  else gemm_f32_small_block<kEpiSwiglu>(g.mlp, (int)blockIdx.x - g.router_blocks, lds);
+}
+struct F32Down { GemmArgs down; SelectArgs select; int select_blocks; };
+template <int R, int C>
+__global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_select_kernel(const F32Down g) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  if ((int)blockIdx.x >= g.select_blocks) {
+    gemm_f32_small_block<kEpiPlain>(g.down, (int)blockIdx.x - g.select_blocks, lds);
+    return;
+  }
+  const float* stats = g.select.stats;
+  if (g.select.part_mean) {                                    // batch statistics: the block merges them first
+    merge_statistics(g.select, (float*)lds, kGemmThreads);
+    count_batch(g.select);
+    stats = (const float*)lds;
+  }
+  constexpr int kWaves = kGemmThreads / kWave;
+  select_pairs<R, C>(g.select, (int)blockIdx.x * kWaves + (int)(threadIdx.x >> 6), g.select_blocks * kWaves, stats);
+}
 
 // One list entry per kernel instantiation that launch_gemm can start (the static members come into being
 // at library load for every instantiation the dispatch below names).
@@ -830,10 +862,35 @@ struct SmallF32Lds {
   static constexpr int kBytes = 4 * 2 * (EPI == kEpiSwiglu ? 3 : 2) * 32 * 128;
   static inline LdsKernel entry{(const void*)gemm_f32_small_kernel<EPI>, kBytes};
 };
+template <auto kKernel, int kBytes>
+struct F32JointLds { static inline LdsKernel entry{(const void*)kKernel, kBytes}; };
 template <int DT, int TM, int TN, int EPI>
 struct StagedKernelLds {
   static inline LdsKernel entry{(const void*)gemm_nt_kernel<DT, TM, TN, EPI>, 2 * (2 * TM * 32 + 2 * TN * 32) * kRowBytes};
 };
+
+// Blocks of gemm_f32_small_kernel where that takes fewer cycles than TM x TN tiles, else 0.
+// Cycles of matrix instructions and of what goes round them, per round of 256 blocks: a TM x TN wave tile takes 1024 TM TN for 32 of K, plus
+// about 900 with one block to a CU and 450 with more (64 x 64 tiles 1700 and 1490, 128 x 128 tiles 5400); a block of 32 x 32 deals the same K out
+// over four waves.  1000 x 1024 x 4096: 106 us on 64 x 64 tiles, 88 us here; 2500 x 768 x 2304: 97 and 102 us.
+template <int TM, int TN, int EPI>
+static int64_t f32_small_blocks(GemmArgs& g) {
+  constexpr int BM = 2 * TM * 32, BN = EPI == kEpiSwiglu ? TN * 32 : 2 * TN * 32, TB = EPI == kEpiSwiglu ? 2 : 1;
+  const int64_t blocks = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
+  const int64_t kt = (g.K + 31) / 32, tiles_m = (g.M + 31) / 32, small = tiles_m * ((g.N + 31) / 32);
+  const int64_t tiled = (blocks + 255) / 256 * kt * (1024 * TM * TN + (blocks > 256 ? 450 : 900)), dealt = (small + 255) / 256 * ((kt + 3) / 4 * (1024 * TB + 450) + 2500);
+  if (dealt >= tiled || small >= INT32_MAX / 4 || (int64_t)g.K * 128 >= INT32_MAX || (EPI != kEpiSwiglu && g.b1 && g.N % 64 != 0)) return 0;
+  g.tiles_m = (int)tiles_m;
+  g.tiles_n = (g.N + 31) / 32;
+  return small;
+}
+template <int EPI>
+static int64_t f32_small_blocks_of(GemmArgs& g) {              // ... against the tiles that gemm_plain and gemm_swiglu choose
+  g.single = g.N % 4 != 0;
+  if (EPI == kEpiSwiglu) return f32_small_blocks<2, 2, EPI>(g);
+  const int64_t big = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256), mid = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+  return big >= 200 ? f32_small_blocks<4, 4, EPI>(g) : mid >= 200 ? f32_small_blocks<2, 2, EPI>(g) : f32_small_blocks<1, 1, EPI>(g);
+}
 
 template <int DT, int TM, int TN, int EPI>
 static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
@@ -885,16 +942,8 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
     }
   }
   if constexpr (DT == kF32 && EPI != kEpiGate) {
-    // Cycles of matrix instructions and of what goes round them, per round of 256 blocks: a TM x TN wave tile takes 1024 TM TN for 32 of K, plus
-    // about 900 with one block to a CU and 450 with more (64 x 64 tiles 1700 and 1490, 128 x 128 tiles 5400); a block of 32 x 32 deals the same K out
-    // over four waves.  1000 x 1024 x 4096: 106 us on 64 x 64 tiles, 88 us here; 2500 x 768 x 2304: 97 and 102 us.
-    constexpr int TB = EPI == kEpiSwiglu ? 2 : 1;
-    const int64_t kt = (g.K + 31) / 32, tiles_m = (g.M + 31) / 32, small = tiles_m * ((g.N + 31) / 32);
-    const int64_t tiled = (blocks + 255) / 256 * kt * (1024 * TM * TN + (blocks > 256 ? 450 : 900)), dealt = (small + 255) / 256 * ((kt + 3) / 4 * (1024 * TB + 450) + 2500);
-    if (dealt < tiled && aligned && small < INT32_MAX && (int64_t)g.K * 128 < INT32_MAX && (EPI == kEpiSwiglu || !g.b1 || g.N % 64 == 0)) {
-      GemmArgs d = g;
-      d.tiles_m = (int)tiles_m;
-      d.tiles_n = (g.N + 31) / 32;
+    GemmArgs d = g;
+    if (const int64_t small = f32_small_blocks<TM, TN, EPI>(d); small && aligned) {
       if (hipError_t e = SmallF32Lds<EPI>::entry.ensure(); e != hipSuccess) return e;
       hipLaunchKernelGGL((gemm_f32_small_kernel<EPI>), dim3((unsigned)small), dim3(kGemmThreads), SmallF32Lds<EPI>::kBytes, s, d);
       return hipGetLastError();
@@ -1018,6 +1067,49 @@ int omni_gemm_router_projection(const void* x, const void* wx, const void* wy, v
   if (dtype == OMNI_F32) return gemm_plain<kF32>(x, wx, wy, nullptr, z, T, 2 * (int64_t)r, H, s, part_mean, part_m2);
   return OMNI_ERR_DTYPE;
 }
+
+namespace omni {
+// The layer's projection, gate/up, selection and down projection in single precision as two launches (see gemm_f32_front_kernel), y then holding the shared MLP's
+// rows; false, with nothing enqueued, where one of the products is not of the kind.  The operands are 16-byte aligned.
+bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, const void* wg, const void* wu, const void* wd, void* h, void* y, int64_t T, int64_t H, int64_t I,
+                      const SelectArgs& args, bool statistics, hipStream_t s, hipError_t* e) {
+  if (check_gemm(T, I, H, 4) || check_gemm(T, H, I, 4)) return false;
+  GemmArgs router{}, mlp{}, down{};
+  router.a = mlp.a = (const uint8_t*)x;
+  router.b0 = (const uint8_t*)wx; router.b1 = (const uint8_t*)wy; router.c = (uint8_t*)z;
+  mlp.b0 = (const uint8_t*)wg; mlp.b1 = (const uint8_t*)wu; mlp.c = (uint8_t*)h;
+  down.a = (const uint8_t*)h; down.b0 = (const uint8_t*)wd; down.c = (uint8_t*)y;
+  router.M = mlp.M = down.M = (int)T;
+  router.N = 2 * args.r; router.K = mlp.K = (int)H; mlp.N = down.K = (int)I; down.N = (int)H;
+  if (statistics) { router.part_mean = (float*)args.part_mean; router.part_m2 = (float*)args.part_m2; }
+  F32Down d{down, args, 0};
+  const int cells = prepare_select(d.select), regs = (args.r + kWave - 1) / kWave;
+  const int64_t rb = f32_small_blocks_of<kEpiPlain>(router), mb = f32_small_blocks_of<kEpiSwiglu>(mlp), db = f32_small_blocks_of<kEpiPlain>(d.down);
+  if (!rb || !mb || !db || regs > 4 || cells > 2) return false;
+  const F32Front f{router, mlp, (int)rb};
+  constexpr int kFront = SmallF32Lds<kEpiSwiglu>::kBytes, kDown = SmallF32Lds<kEpiPlain>::kBytes;
+  static_assert(kDown >= 4 * merge_lds_floats(kMergeKeys, kGemmThreads), "a block that selects merges statistics there");
+  auto start = [&](auto kernel, LdsKernel& entry, int bytes, int64_t blocks, const auto& a) {
+    if ((*e = entry.ensure()) != hipSuccess) return;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kGemmThreads), bytes, s, a);
+    *e = hipGetLastError();
+  };
+  if (statistics) start(gemm_f32_front_kernel<kEpiStats>, F32JointLds<gemm_f32_front_kernel<kEpiStats>, kFront>::entry, kFront, rb + mb, f);
+  else start(gemm_f32_front_kernel<kEpiPlain>, F32JointLds<gemm_f32_front_kernel<kEpiPlain>, kFront>::entry, kFront, rb + mb, f);
+  if (*e != hipSuccess) return true;
+  constexpr int kWaves = kGemmThreads / kWave;
+  d.select_blocks = (int)((T + kWaves - 1) / kWaves < 1024 ? (T + kWaves - 1) / kWaves : 1024);
+  auto by_cells = [&](auto r_tag) {
+    constexpr int R = decltype(r_tag)::value;
+    if (cells <= 1) start(gemm_f32_select_kernel<R, 1>, F32JointLds<gemm_f32_select_kernel<R, 1>, kDown>::entry, kDown, d.select_blocks + db, d);
+    else start(gemm_f32_select_kernel<R, 2>, F32JointLds<gemm_f32_select_kernel<R, 2>, kDown>::entry, kDown, d.select_blocks + db, d);
+  };
+  if (regs <= 1) by_cells(std::integral_constant<int, 1>{});
+  else if (regs <= 2) by_cells(std::integral_constant<int, 2>{});
+  else by_cells(std::integral_constant<int, 4>{});
+  return true;
+}
+}  // namespace omni
 
 namespace omni {
 // partial sums of whichever of the two projections is split along K (they are not alive together)

@@ -25,238 +25,10 @@ int omni_gemm_router_projection(const void* x, const void* wx, const void* wy, v
 
 namespace omni {
 
-// strict "a goes before b": higher score first, then lower payload
-__device__ __forceinline__ bool goes_before(float sa, int pa, float sb, int pb) {
-  return (sa > sb) || (sa == sb && pa < pb);
-}
-
-// Compare-exchange step with a compile-time lane distance, fully unrolled (small R only).
-template <int R, int SIZE, int STRIDE>
-__device__ __forceinline__ void lane_stage_ct(float (&s)[R], int (&p)[R], const int lane) {
-#pragma unroll
-  for (int a = 0; a < R; ++a) {
-    const float os = xor_lane_f<STRIDE>(s[a], lane);
-    const int op = xor_lane_i<STRIDE>(p[a], lane);
-    const bool up = (((a * kWave) | lane) & SIZE) == 0;
-    const bool lower = (lane & STRIDE) == 0;
-    const bool take_other = (lower == up) != goes_before(s[a], p[a], os, op);
-    s[a] = take_other ? os : s[a];
-    p[a] = take_other ? op : p[a];
-  }
-}
-// strides STRIDE, STRIDE/2, ..., 1 of the merge for block size SIZE, on NL lists in lockstep
-template <int R, int SIZE, int STRIDE>
-__device__ __forceinline__ void lane_stages_ct(float (&s0)[R], int (&p0)[R], float (&s1)[R], int (&p1)[R], const int lane, const bool two) {
-  if constexpr (STRIDE >= 1) {
-    lane_stage_ct<R, SIZE, STRIDE>(s0, p0, lane);
-    if (two) lane_stage_ct<R, SIZE, STRIDE>(s1, p1, lane);
-    lane_stages_ct<R, SIZE, STRIDE / 2>(s0, p0, s1, p1, lane, two);
-  }
-}
-template <int R, int SIZE>
-__device__ __forceinline__ void small_sizes_ct(float (&s0)[R], int (&p0)[R], float (&s1)[R], int (&p1)[R], const int lane, const bool two) {
-  if constexpr (SIZE <= kWave) {
-    lane_stages_ct<R, SIZE, SIZE / 2>(s0, p0, s1, p1, lane, two);
-    small_sizes_ct<R, SIZE * 2>(s0, p0, s1, p1, lane, two);
-  }
-}
-
-// One compare-exchange step between lanes `stride` apart (stride < 64), all R registers.
-template <int R>
-__device__ __forceinline__ void lane_stage(float (&s)[R], int (&p)[R], const int lane, const int size, const int stride) {
-#pragma unroll
-  for (int a = 0; a < R; ++a) {
-    const float os = __shfl_xor(s[a], stride, kWave);
-    const int op = __shfl_xor(p[a], stride, kWave);
-    const bool up = (((a * kWave) | lane) & size) == 0;
-    const bool lower = (lane & stride) == 0;
-    const bool take_other = (lower == up) != goes_before(s[a], p[a], os, op);
-    s[a] = take_other ? os : s[a];
-    p[a] = take_other ? op : p[a];
-  }
-}
-
-// One compare-exchange step between registers RS apart (element stride 64*RS).
-template <int R, int SIZE, int RS>
-__device__ __forceinline__ void reg_stage(float (&s)[R], int (&p)[R]) {
-#pragma unroll
-  for (int a = 0; a < R; ++a) {
-    if ((a & RS) == 0) {
-      const int b = a | RS;
-      const bool up = ((a * kWave) & SIZE) == 0;
-      const bool swap = goes_before(s[a], p[a], s[b], p[b]) != up;
-      const float ts = swap ? s[b] : s[a];
-      const int tp = swap ? p[b] : p[a];
-      s[b] = swap ? s[a] : s[b];
-      p[b] = swap ? p[a] : p[b];
-      s[a] = ts;
-      p[a] = tp;
-    }
-  }
-}
-
-template <int R, int SIZE, int RS>
-__device__ __forceinline__ void reg_stages_down(float (&s)[R], int (&p)[R]) {
-  if constexpr (RS >= 1) {
-    reg_stage<R, SIZE, RS>(s, p);
-    reg_stages_down<R, SIZE, RS / 2>(s, p);
-  }
-}
-
-// Merge steps for block size SIZE (> 64) and the sizes above it, up to 64*R.
-
-template <int R, int SIZE>
-__device__ __forceinline__ void big_sizes(float (&s)[R], int (&p)[R], const int lane) {
-  if constexpr (SIZE <= kWave * R) {
-    reg_stages_down<R, SIZE, SIZE / (2 * kWave)>(s, p);
-    if constexpr (R <= kUnrollMaxR) {
-      lane_stages_ct<R, SIZE, kWave / 2>(s, p, s, p, lane, false);
-    } else {
-#pragma nounroll
-      for (int stride = kWave / 2; stride >= 1; stride >>= 1) lane_stage<R>(s, p, lane, SIZE, stride);
-    }
-    big_sizes<R, SIZE * 2>(s, p, lane);
-  }
-}
-
-// Sorts the 64*R (score, payload) items held as item e = reg*64 + lane with a bitonic
-// network.  Steps between lanes run as rolled loops (the shuffle distance is a run-time
-// value); steps between registers are unrolled so that register indices are constants.
-template <int R>
-__device__ __forceinline__ void bitonic_sort(float (&s)[R], int (&p)[R], const int lane) {
-  if constexpr (R <= kUnrollMaxR) {
-    small_sizes_ct<R, 2>(s, p, s, p, lane, false);
-  } else {
-#pragma nounroll
-    for (int size = 2; size <= kWave; size <<= 1) {
-#pragma nounroll
-      for (int stride = size >> 1; stride >= 1; stride >>= 1) lane_stage<R>(s, p, lane, size, stride);
-    }
-  }
-  big_sizes<R, 2 * kWave>(s, p, lane);
-}
-
-// Two independent lists sorted in lockstep: the two dependency chains interleave, which
-// hides most of the cross-lane exchange latency.
-template <int R, int SIZE>
-__device__ __forceinline__ void big_sizes2(float (&s0)[R], int (&p0)[R], float (&s1)[R], int (&p1)[R], const int lane) {
-  if constexpr (SIZE <= kWave * R) {
-    reg_stages_down<R, SIZE, SIZE / (2 * kWave)>(s0, p0);
-    reg_stages_down<R, SIZE, SIZE / (2 * kWave)>(s1, p1);
-    if constexpr (R <= kUnrollMaxR) {
-      lane_stages_ct<R, SIZE, kWave / 2>(s0, p0, s1, p1, lane, true);
-    } else {
-#pragma nounroll
-      for (int stride = kWave / 2; stride >= 1; stride >>= 1) {
-        lane_stage<R>(s0, p0, lane, SIZE, stride);
-        lane_stage<R>(s1, p1, lane, SIZE, stride);
-      }
-    }
-    big_sizes2<R, SIZE * 2>(s0, p0, s1, p1, lane);
-  }
-}
-template <int R>
-__device__ __forceinline__ void bitonic_sort2(float (&s0)[R], int (&p0)[R], float (&s1)[R], int (&p1)[R], const int lane) {
-  if constexpr (R <= kUnrollMaxR) {
-    small_sizes_ct<R, 2>(s0, p0, s1, p1, lane, true);
-  } else {
-#pragma nounroll
-    for (int size = 2; size <= kWave; size <<= 1) {
-#pragma nounroll
-      for (int stride = size >> 1; stride >= 1; stride >>= 1) {
-        lane_stage<R>(s0, p0, lane, size, stride);
-        lane_stage<R>(s1, p1, lane, size, stride);
-      }
-    }
-  }
-  big_sizes2<R, 2 * kWave>(s0, p0, s1, p1, lane);
-}
-
-// value of sorted item `i` (i < 128) of a list held as item = reg*64+lane
-template <int R, typename T>
-__device__ __forceinline__ T sorted_item(const T (&v)[R], int i) {
-  T r0 = __shfl(v[0], i & 63, kWave);
-  if constexpr (R >= 2) {
-    T r1 = __shfl(v[1], i & 63, kWave);
-    r0 = (i >= kWave) ? r1 : r0;
-  }
-  return r0;
-}
-
-// R = half keys per lane (r <= 64*R); C = candidate cells per lane.  With few keys per lane a wave requests
-// the raw scores of its first token before anything else and those of its next token as soon as the current
-// token's are consumed.
 template <int R, int C>
 __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(const SelectArgs g) {
   count_batch(g);
-  const int lane = lane_id();
-  const int wave = blockIdx.x * kRouterWaves + (threadIdx.x >> 6);
-  const int num_waves = gridDim.x * kRouterWaves;
-  using S = Elem<kF32>;                           // (16-bit scores travel packed)
-  const int r = g.r, k = g.k, kp = g.kp;
-
-  float rx[R], ry[R];                             // raw scores of the token about to be selected
-  auto load_raw = [&](int t) __attribute__((always_inline)) {
-#pragma unroll
-    for (int a = 0; a < R; ++a) {
-      const int key = a * kWave + lane;
-      const bool ok = key < r;
-      rx[a] = ok ? S::load(g.lx, int64_t(t) * g.row_stride + key) : kNegInf;
-      ry[a] = ok ? S::load(g.ly, int64_t(t) * g.row_stride + key) : kNegInf;
-    }
-  };
-  constexpr bool kPrefetch = R <= 2;              // beyond that the extra live registers cost a wave per SIMD
-  if (kPrefetch && wave < g.num_tokens) load_raw(wave);
-  const float* stats = g.stats;
-  const NormKeys<R> norm(g, stats, lane);
-  int cell[C];
-  candidate_cells<R, C>(cell, g, kp, lane);
-
-  for (int t = wave; t < g.num_tokens; t += num_waves) {
-    float sx[R], sy[R];
-    int px[R], py[R];
-#pragma unroll
-    for (int a = 0; a < R; ++a) {
-      const int key = a * kWave + lane;
-      const bool ok = key < r;
-      sx[a] = kPrefetch ? rx[a] : ok ? S::load(g.lx, int64_t(t) * g.row_stride + key) : kNegInf;
-      sy[a] = kPrefetch ? ry[a] : ok ? S::load(g.ly, int64_t(t) * g.row_stride + key) : kNegInf;
-      px[a] = py[a] = key;
-    }
-    if (kPrefetch && t + num_waves < g.num_tokens) load_raw(t + num_waves);
-    if (stats || g.run_mean[0]) {
-      normalise_half<kF32, R>(sx, g, norm, stats, 0, r, lane);
-      normalise_half<kF32, R>(sy, g, norm, stats, 1, r, lane);
-    }
-    bitonic_sort2<R>(sx, px, sy, py, lane);
-
-    float cs[C];
-    int cp[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      const bool ok = cell[c] >= 0;
-      const int a = ok ? (cell[c] >> 8) : 0, b = ok ? (cell[c] & 255) : 0;
-      const float va = sorted_item<R>(sx, a), vb = sorted_item<R>(sy, b);
-      cs[c] = ok ? va + vb : kNegInf;
-      cp[c] = ok ? cell[c] : (0x40000000 | (c * kWave + lane));
-    }
-    bitonic_sort<C>(cs, cp, lane);
-
-    constexpr int kOut = (C >= 2) ? 2 : 1;          // k <= 128 -> winners live in regs 0..1
-#pragma unroll
-    for (int c = 0; c < kOut; ++c) {
-      const int j = c * kWave + lane;
-      const bool ok = j < k;
-      const int a = ok ? (cp[c] >> 8) & 255 : 0, b = ok ? (cp[c] & 255) : 0;
-      const int ia = sorted_item<R>(px, a), ib = sorted_item<R>(py, b);
-      if (ok) {
-        const int64_t o = int64_t(t) * k + j;
-        if (g.scores) S::store(g.scores, o, cs[c]);
-        if (g.gates) S::store(g.gates, o, expf(cs[c]));      // gate = P(x key) * P(y key)
-        g.indices[o] = ia * r + ib;
-      }
-    }
-  }
+  select_pairs<R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats);
 }
 
 template <int DT, int R, int C>
