@@ -39,15 +39,20 @@ constexpr int kTokensPerBlock = 4;   // one wave each
 // parts [splits][tokens][hidden]; both terms are rounded, then their sum.
 // scores: NULL, or [tokens][top_k] where <x, u> of every pair goes, for a backward pass.
 struct GatherAdd { const float* parts; int splits; float* scores; };
-template <int DT, int NCH, int G, bool kAdd = false>
+// W waves share a token's slots, each a run of them, and add up in wave order: with fewer tokens than the chip holds waves a token's batches of G slots are
+// a chain of waits.
+template <int DT, int NCH, int G, bool kAdd = false, int W = 1>
 __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kernel(
     const uint8_t* __restrict__ x, const uint8_t* __restrict__ up, const uint8_t* __restrict__ down,
     const void* __restrict__ gates, const int32_t* __restrict__ ids, uint8_t* __restrict__ y,
     int num_tokens, int hidden, int top_k, uint32_t num_experts, GatherAdd add) {
   constexpr int E = Row16<DT>::kElems;
   const int lane = lane_id();
-  const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * kTokensPerBlock + (threadIdx.x >> 6));
-  if (t >= num_tokens) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), share = wave % W;
+  const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * (kTokensPerBlock / W) + wave / W);
+  if (W == 1 && t >= num_tokens) return;
+  const int per = W == 1 ? top_k : (top_k + W - 1) / W;
+  const int first = share * per, last = t >= num_tokens ? first : min(first + per, top_k);
   const int64_t row_bytes = int64_t(hidden) * (16 / E);
 
   bool live[NCH];
@@ -56,8 +61,7 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
   float acc[NCH][E];
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
-    const int first = (c * kWave + lane) * E;
-    live[c] = first < hidden;
+    live[c] = (c * kWave + lane) * E < hidden && (W == 1 || t < num_tokens);
     off[c] = int64_t(c * kWave + lane) * 16;
     xr[c] = live[c] ? *(const u32x4_t*)(x + t * row_bytes + off[c]) : u32x4_t{0, 0, 0, 0};
 #pragma unroll
@@ -65,17 +69,17 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
   }
 
   const int32_t* my_ids = ids + int64_t(t) * top_k;
-  for (int j0 = 0; j0 < top_k; j0 += G) {
+  for (int j0 = first; j0 < last; j0 += G) {
     int e[G];
     float g[G];
     bool live_slot[G];
 #pragma unroll
     for (int i = 0; i < G; ++i) {
-      const int j = min(j0 + i, top_k - 1);          // always a valid slot: no branch around the loads
+      const int j = min(j0 + i, last - 1);          // always a valid slot: no branch around the loads
       const int id = my_ids[j];
       const float gate = Elem<DT>::load(gates, int64_t(t) * top_k + j);
-      // a slot past k, or an id outside the table, contributes nothing
-      const bool ok = (j0 + i < top_k) && (uint32_t)id < num_experts;
+      // a slot of another wave or past k, or an id outside the table, contributes nothing
+      const bool ok = (j0 + i < last) && (uint32_t)id < num_experts;
       e[i] = ok ? id : 0;
       g[i] = ok ? gate : 0.f;
       live_slot[i] = ok;
@@ -106,7 +110,7 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
       float mine = 0.f;
 #pragma unroll
       for (int i = 0; i < G; ++i) mine = lane == i ? s[i] : mine;
-      if (lane < G && j0 + lane < top_k) add.scores[int64_t(t) * top_k + j0 + lane] = mine;
+      if (lane < G && j0 + lane < last) add.scores[int64_t(t) * top_k + j0 + lane] = mine;
     }
 #pragma unroll
     for (int i = 0; i < G; ++i) {
@@ -117,6 +121,26 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
     }
   }
 
+  if constexpr (W > 1) {
+    __shared__ __align__(16) float sums[kTokensPerBlock][NCH * kWave * E];
+    if (share > 0)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+#pragma unroll
+        for (int q = 0; q < E; q += 4) *(f32x4_t*)(&sums[wave][(c * kWave + lane) * E + q]) = f32x4_t{acc[c][q], acc[c][q + 1], acc[c][q + 2], acc[c][q + 3]};
+    __syncthreads();
+    if (share > 0 || t >= num_tokens) return;
+#pragma unroll
+    for (int w = 1; w < W; ++w)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+#pragma unroll
+        for (int q = 0; q < E; q += 4) {
+          const f32x4_t o = *(const f32x4_t*)(&sums[wave + w][(c * kWave + lane) * E + q]);
+#pragma unroll
+          for (int z = 0; z < 4; ++z) acc[c][q + z] += o[z];
+        }
+  }
 #pragma unroll
   for (int c = 0; c < NCH; ++c)
     if (live[c]) {
@@ -147,24 +171,49 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
     }
 }
 
+// Waves to a token: while the chip has room for them (2048 at these register counts) and a token's slots are several batches.  Time with 2 and 4 over 1,
+// bf16, 4096 experts (65536: the same within 5 %), at 200 / 400 / 613 / 1000 / 1500 tokens:
+//   two batches   hidden 256 k 32, 1024 k 16, 2048 k 8:   2: 0.64-0.72 / 0.64-0.74 / 0.81-0.95 / 0.81-0.94 / 0.8-1.03   4: 0.6-0.7 / 0.72-0.82 / 0.86-1.09 / 1.04-1.08
+//   four and more hidden 1024 k 32, 2048 k 16 and 32, 4096: 2: 0.60-0.66 / 0.74-0.84 / 0.83-0.97 / 0.88-1.03 / 1.0   4: 0.40-0.58 / 0.63-0.84 / 0.78-1.0 / 0.87-1.08 / 1.0
+//   one batch: 1.0-1.25 and 1.0-1.8
+// Not where the gather algorithm is asked for by name: its sums are those of the segment algorithm, slot by slot.
+static inline int gather_waves(int64_t T, int k, int batch) {
+  const int batches = (k + batch - 1) / batch;
+  return batches < 2 || T > 1024 ? 1 : batches >= 4 && T <= 512 ? 4 : 2;
+}
 template <int DT, int NCH, int G>
 static hipError_t launch_gather(const void* x, const void* up, const void* down, const void* gates,
-                                const int32_t* ids, void* y, float* scores, int64_t T, int H, int k, int64_t N, hipStream_t s) {
+                                const int32_t* ids, void* y, float* scores, bool shared, int64_t T, int H, int k, int64_t N, hipStream_t s) {
   if (T == 0) return hipSuccess;
-  dim3 grid((unsigned)((T + kTokensPerBlock - 1) / kTokensPerBlock)), block(kTokensPerBlock * kWave);
-  hipLaunchKernelGGL((expert_gather_kernel<DT, NCH, G>), grid, block, 0, s, (const uint8_t*)x, (const uint8_t*)up,
-                     (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{nullptr, 0, scores});
-  return hipGetLastError();
+  auto go = [&](auto waves) {
+    constexpr int W = decltype(waves)::value, kTokens = kTokensPerBlock / W;
+    hipLaunchKernelGGL((expert_gather_kernel<DT, NCH, G, false, W>), dim3((unsigned)((T + kTokens - 1) / kTokens)), dim3(kTokensPerBlock * kWave), 0, s, (const uint8_t*)x,
+                       (const uint8_t*)up, (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{nullptr, 0, scores});
+    return hipGetLastError();
+  };
+  switch (shared ? gather_waves(T, k, G) : 1) {
+    case 4: return go(std::integral_constant<int, 4>{});
+    case 2: return go(std::integral_constant<int, 2>{});
+    default: return go(std::integral_constant<int, 1>{});
+  }
 }
 
 // The gather algorithm (rows of at most 8 KiB) with the layer's final add
 hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, int64_t T, int H,
                              int k, int64_t N, int dtype, hipStream_t s) {
-  const dim3 grid((unsigned)((T + kTokensPerBlock - 1) / kTokensPerBlock)), block(kTokensPerBlock * kWave);
-  auto go = [&](auto dt, auto nch, auto batch) {
-    hipLaunchKernelGGL((expert_gather_kernel<decltype(dt)::value, decltype(nch)::value, decltype(batch)::value, true>), grid, block, 0, s, (const uint8_t*)x, (const uint8_t*)up,
-                       (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N, GatherAdd{parts, splits, nullptr});
+  auto launch = [&](auto dt, auto nch, auto batch, auto waves) {
+    constexpr int W = decltype(waves)::value, kTokens = kTokensPerBlock / W;
+    hipLaunchKernelGGL((expert_gather_kernel<decltype(dt)::value, decltype(nch)::value, decltype(batch)::value, true, W>), dim3((unsigned)((T + kTokens - 1) / kTokens)),
+                       dim3(kTokensPerBlock * kWave), 0, s, (const uint8_t*)x, (const uint8_t*)up, (const uint8_t*)down, gates, ids, (uint8_t*)y, (int)T, H, k, (uint32_t)N,
+                       GatherAdd{parts, splits, nullptr});
     return hipGetLastError();
+  };
+  auto go = [&](auto dt, auto nch, auto batch) {
+    switch (gather_waves(T, k, decltype(batch)::value)) {
+      case 4: return launch(dt, nch, batch, std::integral_constant<int, 4>{});
+      case 2: return launch(dt, nch, batch, std::integral_constant<int, 2>{});
+      default: return launch(dt, nch, batch, std::integral_constant<int, 1>{});
+    }
   };
   auto by_row = [&](auto dt) {
     constexpr int E = Row16<decltype(dt)::value>::kElems;
@@ -179,15 +228,15 @@ hipError_t launch_gather_add(const void* x, const void* up, const void* down, co
 
 template <int DT>
 static int expert_gather_dispatch(const void* x, const void* up, const void* down, const void* gates,
-                                  const int32_t* ids, void* y, int64_t T, int H, int k, int64_t N, hipStream_t s, float* scores = nullptr) {
+                                  const int32_t* ids, void* y, int64_t T, int H, int k, int64_t N, hipStream_t s, float* scores = nullptr, bool shared = false) {
   constexpr int E = Row16<DT>::kElems;
   if (H % E != 0) return OMNI_ERR_SHAPE;              // rows must be 16-byte multiples
   const int nch = (H + kWave * E - 1) / (kWave * E);
   hipError_t err;
-  if (nch <= 1) err = launch_gather<DT, 1, 16>(x, up, down, gates, ids, y, scores, T, H, k, N, s);
-  else if (nch <= 2) err = launch_gather<DT, 2, 8>(x, up, down, gates, ids, y, scores, T, H, k, N, s);
-  else if (nch <= 4) err = launch_gather<DT, 4, 4>(x, up, down, gates, ids, y, scores, T, H, k, N, s);
-  else if (nch <= 8) err = launch_gather<DT, 8, 2>(x, up, down, gates, ids, y, scores, T, H, k, N, s);
+  if (nch <= 1) err = launch_gather<DT, 1, 16>(x, up, down, gates, ids, y, scores, shared, T, H, k, N, s);
+  else if (nch <= 2) err = launch_gather<DT, 2, 8>(x, up, down, gates, ids, y, scores, shared, T, H, k, N, s);
+  else if (nch <= 4) err = launch_gather<DT, 4, 4>(x, up, down, gates, ids, y, scores, shared, T, H, k, N, s);
+  else if (nch <= 8) err = launch_gather<DT, 8, 2>(x, up, down, gates, ids, y, scores, shared, T, H, k, N, s);
   else return OMNI_ERR_UNSUPPORTED;
   return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
 }
@@ -625,6 +674,7 @@ extern "C" OMNI_API int32_t omni_expert_fwd_scores(const void* x, const void* up
   hipStream_t s = (hipStream_t)stream;
   int lanes = 0;
   if (algo == OMNI_EXPERT_ALGO_SPLIT && split_col_blocks(hidden_size, dtype == OMNI_F32 ? 4 : 2, &lanes) == 0) return OMNI_ERR_UNSUPPORTED;
+  const bool shared = algo == OMNI_EXPERT_ALGO_AUTO;
   algo = resolve_algo(algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype);
   if (scores && algo != OMNI_EXPERT_ALGO_GATHER && algo != OMNI_EXPERT_ALGO_SPLIT) return OMNI_ERR_UNSUPPORTED;
   if (algo == OMNI_EXPERT_ALGO_SEGMENT) {
@@ -652,9 +702,9 @@ extern "C" OMNI_API int32_t omni_expert_fwd_scores(const void* x, const void* up
   }
   if (algo != OMNI_EXPERT_ALGO_GATHER) return OMNI_ERR_UNSUPPORTED;
   switch (dtype) {
-    case OMNI_BF16: return expert_gather_dispatch<kBF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores);
-    case OMNI_F16: return expert_gather_dispatch<kF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores);
-    case OMNI_F32: return expert_gather_dispatch<kF32>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores);
+    case OMNI_BF16: return expert_gather_dispatch<kBF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores, shared);
+    case OMNI_F16: return expert_gather_dispatch<kF16>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores, shared);
+    case OMNI_F32: return expert_gather_dispatch<kF32>(x, up_weight, down_weight, routing_weights, indices, y, num_tokens, hidden_size, num_experts_per_token, num_experts, s, scores, shared);
     default: return OMNI_ERR_DTYPE;
   }
 }

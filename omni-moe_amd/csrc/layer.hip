@@ -31,17 +31,15 @@ bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, co
 // (then a GEMM of more tiles than CUs may take the form that holds every CU until it ends); h lies at the workspace's start
 int mlp_gate_up_impl(const void* x, const void* wg, const void* wu, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive);
 int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive);
-// The experts with a block per token up to here, with a wave per token beyond: 65 tokens (8 parts) 5.5 against 13.5 us, 256 tokens 6.8 / 11.8, 400 tokens
-// 10.8 / 11, 613 tokens 14.3 / 11.0 (hidden 1024, top-16).  The whole layer, block against wave, at 65 / 256 / 384 / 512 / 640 tokens:
-//   hidden  256, top-16   20 / 21    19 / 21    20 / 21     20 / 21      23 / 21 us
-//   hidden 1024, top-2    21 / 26    25 / 27    29 / 28     37 / 36      42 / 38
-//   hidden 1024, top-16   23 / 31    27 / 31    32 / 32     42 / 41      47 / 44
-//   hidden 1024, top-32   26 / 39    31 / 40    35 / 40     44 / 48      50 / 51
-//   hidden 2048, top-16   32 / 43    41 / 47    47 / 49     69 / 71      69 / 69
-//   hidden 4096, top-16   40 / 69    67 / 79    73 / 80    103 / 107
-//   hidden 4096, top-4    35 / 40    44 / 48    51 / 51     69 / 69      67 / 63
-// so the two cross between 320 and 640 tokens everywhere, and at 384 either is within 3 % or the block ahead.
-constexpr int kBlockPerToken = 384;
+// The experts with a block of eight waves per token up to here, with one to four waves per token (gather_waves) beyond.  The whole layer, block against waves, at
+// 65 / 128 / 256 / 320 / 384 tokens, bf16:
+//   hidden  256, top-16   20 / 20     20 / 20     20 / 20     20 / 20     20 / 20 us
+//   hidden 1024, top-2    20 / 25     21 / 25     25 / 27     29 / 28     29 / 28
+//   hidden 1024, top-16   21 / 26     22 / 26     27 / 28     31 / 30     32 / 30
+//   hidden 1024, top-32   23 / 27     25 / 29     28 / 30     33 / 32     34 / 33
+//   hidden 2048, top-16   27 / 30     28 / 31     40 / 41     45 / 44     46 / 45
+//   hidden 4096, top-4    51 / 67     55 / 70     87 / 92
+constexpr int kBlockPerToken = 256;
 // Projection | gate/up, selection | down projection, experts and add; where two stages do not fit one launch, each is its own.
 // statistics (training): projects z and leaves its column statistics, which f.select merges or reads.
 template <class Statistics>
