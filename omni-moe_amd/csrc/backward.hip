@@ -637,7 +637,7 @@ static hipError_t launch_token_split(const TokenPass& p, const SortPass* sort, h
     constexpr int LPR = decltype(group)::value, S = decltype(s_tag)::value;
     constexpr bool RAGGED = decltype(ragged)::value;
     const int64_t blocks = split_blocks(p.num_tokens, kTokenWaves * (kWave / LPR), S);
-    const int count = sort ? kSortCount : kSortNone, scatter = sort ? kSortScatter : kSortNone;
+    const int count = sort && sort->tiles > 1 ? kSortCount : kSortNone, scatter = sort ? kSortScatter : kSortNone;
     if constexpr (LPR < 8) {
       return hipErrorInvalidValue;
     } else {
@@ -658,8 +658,9 @@ static hipError_t launch_token_gather(TokenPass p, const SortPass* sort, hipStre
   p.first = 0;
   p.last = p.num_tokens;
   if (!sort) return start_token<kKernel>(p, nullptr, kSortNone, blocks(p.num_tokens, kBwdWavesPerBlock), s, kBwdWavesPerBlock * kWave);
-  p.last = p.num_tokens >= 4096 ? p.num_tokens / 2 : 0;
-  if (hipError_t e = start_token<kKernel>(p, sort, kSortCount, blocks(p.last, kTokenWaves), s); e != hipSuccess) return e;
+  p.last = p.num_tokens >= 4096 && sort->tiles > 1 ? p.num_tokens / 2 : 0;
+  if (sort->tiles > 1)
+    if (hipError_t e = start_token<kKernel>(p, sort, kSortCount, blocks(p.last, kTokenWaves), s); e != hipSuccess) return e;
   p.first = p.last;
   p.last = p.num_tokens;
   return start_token<kKernel>(p, sort, kSortScatter, blocks(p.last - p.first, kTokenWaves), s);

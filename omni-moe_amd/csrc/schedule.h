@@ -84,6 +84,7 @@ __device__ __forceinline__ void sort_count_block(const SortPass& a, const int bl
 }
 
 // A block of the scatter kernel: tile block / 8, slice block % 8.  tables: [(waves + 3) * width] in LDS.
+// Of a sort of one tile every block counts all pairs for itself, so no count kernel runs in front of it.
 __device__ __forceinline__ void sort_scatter_block(const SortPass& a, const int block, int32_t* tables) {
   int32_t* tbl = tables;                                 // [wave][width]: per wave and bin: count, then running output position
   int32_t *bin_base = tbl + kSortWaves * a.width, *before_s = bin_base + a.width, *total_s = before_s + a.width;
@@ -96,7 +97,7 @@ __device__ __forceinline__ void sort_scatter_block(const SortPass& a, const int 
   // 16-byte load per row) of the rows t / C, t / C + G, ..; the first batch of loads flies while the tile is counted.
   const int C = a.width / kBinChunk, G = kSortThreads / C;
   const int chunk = threadIdx.x % C, group = threadIdx.x / C;
-  const bool summing = group < G;
+  const bool one = a.tiles == 1, summing = group < G && !one;
   auto load_rows = [&](u32x4_t (&row)[kRowBatch], int first) {
 #pragma unroll
     for (int j = 0; j < kRowBatch; ++j) {
@@ -117,6 +118,7 @@ __device__ __forceinline__ void sort_scatter_block(const SortPass& a, const int 
   const int64_t w0 = t0 + (int64_t)wave * per_wave < t1 ? t0 + (int64_t)wave * per_wave : t1;   // this wave's eighth, in order
   const int64_t w1 = w0 + per_wave < t1 ? w0 + per_wave : t1;
   int32_t* mine = tbl + wave * a.width;
+  int32_t lower = 0;                                     // this lane's pairs in the slices below
   for (int64_t g0 = w0; g0 < w1; g0 += kGroup * kWave) {
     int32_t key[kGroup];
 #pragma unroll
@@ -127,20 +129,33 @@ __device__ __forceinline__ void sort_scatter_block(const SortPass& a, const int 
 #pragma unroll
     for (int u = 0; u < kGroup; ++u) {
       const int d = sort_digit(a, key[u]) - lo;
-      if (g0 + u * kWave + lane < w1 && (uint32_t)d < (uint32_t)a.width) atomicAdd(&mine[d], 1);
+      const bool in = g0 + u * kWave + lane < w1;
+      if (in && (uint32_t)d < (uint32_t)a.width) atomicAdd(&mine[d], 1);
+      lower += in && d < 0 ? 1 : 0;
     }
   }
 
   // what the slices below this one hold, over all tiles
   {
-    int32_t part = 0;
-    for (int e = threadIdx.x; e < a.tiles * kBinSlices; e += kSortThreads)
-      part += (e % kBinSlices) < slice ? (int32_t)a.slice_tot[e] : 0;
+    int32_t part = lower;
+    if (!one) {
+      part = 0;
+      for (int e = threadIdx.x; e < a.tiles * kBinSlices; e += kSortThreads)
+        part += (e % kBinSlices) < slice ? (int32_t)a.slice_tot[e] : 0;
+    }
     part = wave_sum_i32(part);
     if (lane == 0 && part) atomicAdd(&below_s, part);
   }
   // this slice of the histogram rows: what earlier tiles put into each bin, and each bin's total
-  {
+  if (one) {
+    __syncthreads();                                       // the waves' counts are complete
+    for (int d = threadIdx.x; d < a.width; d += kSortThreads) {
+      int32_t sum = 0;
+#pragma unroll
+      for (int w = 0; w < kSortWaves; ++w) sum += tbl[w * a.width + d];
+      total_s[d] = sum;
+    }
+  } else {
     int32_t before[kBinChunk], rest[kBinChunk];
 #pragma unroll
     for (int i = 0; i < kBinChunk; ++i) before[i] = rest[i] = 0;
@@ -269,8 +284,8 @@ struct SortPlan {
   int passes, lo_bits, bins[2], width, stride, tile, tiles;
   size_t hist_entries;
 };
-// The arguments of a schedule that one counting pass does, for a launch of its own or one that it shares: tiles blocks of sort_count_block, then
-// tiles * 8 of sort_scatter_block, all of kSortThreads threads.  False where it takes two passes.
+// The arguments of a schedule that one counting pass does, for a launch of its own or one that it shares: tiles blocks of sort_count_block (none for
+// one tile), then tiles * 8 of sort_scatter_block, all of kSortThreads threads.  False where it takes two passes.
 bool schedule_single_pass(const int32_t* indices, int32_t* offsets, int32_t* sorted_pair_ids, int32_t* sorted_token_ids, int64_t num_tokens, int num_experts_per_token,
                           int64_t num_experts, void* workspace, SortPass* a);
 

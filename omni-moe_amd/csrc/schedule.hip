@@ -5,7 +5,7 @@
 // the host (:82, :90).  Here the pairs are sorted by expert id with one counting pass (one bin per
 // expert) when N <= 4096, or N <= 16384 with few pairs, and two passes (low then high half of the id bits) above that.
 // A pass is two kernels:
-//   count:   every block counts the bins of its contiguous tile of the input in LDS and writes
+//   count:   (where there is more than one tile) every block counts the bins of its contiguous tile of the input in LDS and writes
 //            them as one row of hist[tile][bin] (16-bit counters: a tile has fewer than 65536
 //            pairs), plus the row's sum over each of the 8 bin slices;
 //   scatter: the bins are cut into 8 slices and a block places the pairs of ONE tile that fall
@@ -27,6 +27,8 @@
 #include "common.h"
 #include "omni_moe_hip.h"
 #include "schedule.h"
+
+#include <algorithm>
 
 namespace omni {
 
@@ -59,6 +61,11 @@ static inline int ceil_log2(uint64_t v) { int b = 0; while ((1ull << b) < v) ++b
 static LdsKernel g_count_kernel{(const void*)sort_count_kernel, slice_width(kMaxBinsWide) * kBinSlices * 4};
 static LdsKernel g_scatter_kernel{(const void*)sort_scatter_kernel, (kSortWaves + 3) * slice_width(kMaxBinsWide) * 4};
 
+// Up to so many pairs are one tile: every scatter block counts them all, and the count kernel's launch goes, for longer chains of steps in the scatter
+// blocks.  One pass, 512 / 4096 / 8192 pairs over 1024 experts 9.0 / 9.2 / 9.4 -> 5.5 / 6.6 / 9.5 us, 8192 over 16384 15.0 -> 11.9; beside the expert
+// backward's token pass (8000 pairs, hidden 512) 3.6 + 8.1 us in two launches -> 11.6 in one.  Two passes: 8000 pairs 22.6 -> 24.5, so half as many.
+constexpr int kOneTile = 8192;
+
 static bool make_plan(int64_t P, int64_t N, SortPlan* pl) {
   const int kb = ceil_log2((uint64_t)N);
   // A wave places an eighth of a tile, 64 items a step: tiles of 8192 pairs are 16 steps; at most 256 tiles (a scatter
@@ -89,6 +96,10 @@ static bool make_plan(int64_t P, int64_t N, SortPlan* pl) {
   pl->tiles = (int)((P + tile - 1) / tile);
   if (pl->tiles < 1) pl->tiles = 1;
   pl->hist_entries = (size_t)pl->stride * pl->tiles;
+  if (P <= (pl->passes == 1 ? kOneTile : kOneTile / 2)) {
+    pl->tile = (int)std::max<int64_t>((P + kSortThreads - 1) / kSortThreads, 1) * kSortThreads;
+    pl->tiles = 1;
+  }
   return true;
 }
 
@@ -171,7 +182,7 @@ extern "C" OMNI_API int32_t omni_schedule(const int32_t* indices, int32_t* offse
       a.vals_out = last ? sorted_pair_ids : vals_a;
       a.tok_out = last ? sorted_token_ids : nullptr;
       a.offsets_out = single ? offsets : nullptr;          // one bin per expert: the bins' first positions ARE the offsets
-      hipLaunchKernelGGL(sort_count_kernel, dim3(a.tiles), dim3(kSortThreads), count_lds(a.stride), s, a);
+      if (a.tiles > 1) hipLaunchKernelGGL(sort_count_kernel, dim3(a.tiles), dim3(kSortThreads), count_lds(a.stride), s, a);
       hipLaunchKernelGGL(sort_scatter_kernel, dim3(a.tiles * kBinSlices), dim3(kSortThreads), scatter_lds(a.width), s, a);
     }
   }

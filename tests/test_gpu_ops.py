@@ -122,7 +122,10 @@ SCHED_CASES = [(512, 8, 1024, "uniform"), (4096, 16, 4096, "uniform"), (16384, 1
                (150000, 16, 4096, "uniform"), (1100000, 16, 4096, "hot"),
                # one wide pass: just above the narrow one, at its last bin, its tiles of 2048 and 4096 pairs; and just past it in bins and in pairs
                (64, 2, 4096, "uniform"), (1024, 32, 16384, "uniform"), (2051, 30, 16384, "zipf"), (1024, 32, 16385, "uniform"), (30000, 16, 16000, "uniform"),
-               (9001, 4, 12000, "hot")]
+               (9001, 4, 12000, "hot"),
+               # one tile (up to 8192 pairs, 4096 in two passes; no count kernel): one step of one wave, a partial step, the last size and one past it
+               (16, 4, 1000, "uniform"), (33, 6, 4096, "hot"), (512, 16, 1024, "zipf"), (512, 16, 16384, "uniform"), (512, 8, 262144, "uniform"), (513, 8, 262144, "zipf"),
+               (1366, 6, 16384, "zipf")]
 
 
 def _sched_ids(T, k, N, kind, seed):
