@@ -14,6 +14,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 
@@ -87,23 +88,22 @@ bool records(std::initializer_list<const Tensor*> ts) {
 }
 
 // ---- expert op -------------------------------------------------------------------------------------
-// scores: NULL, or where the pair scores that a backward pass takes over are put
-Tensor expert_forward(const Tensor& x, const Tensor& up, const Tensor& down, const Tensor& gates, const Tensor& ids, int algo, Tensor* scores = nullptr) {
-  const int64_t T = x.size(0), H = x.size(1), N = up.size(0), k = ids.size(1);
+// x: T rows; gates, ids: [T, k]; scores: NULL, or where the pair scores that a backward pass takes over are put
+Tensor expert_forward(const Tensor& x, int64_t T, const Tensor& up, const Tensor& down, const void* gates, const void* ids, int64_t k, int algo, void* scores) {
+  const int64_t H = up.size(1), N = up.size(0);
   const int dt = dtype_code(x.scalar_type());
   Tensor y = at::empty_like(x);
   const size_t need = omni_expert_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt, algo);
   Tensor ws = need ? bytes(need, x.device()) : Tensor();
-  if (scores) *scores = at::empty({T, k}, x.options().dtype(at::kFloat));
-  check(omni_expert_fwd_scores(ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), ptr(y), scores ? (float*)ptr(*scores) : nullptr, T, (int32_t)H, N, (int32_t)k,
+  check(omni_expert_fwd_scores(ptr(x), ptr(up), ptr(down), gates, (const int32_t*)ids, ptr(y), (float*)scores, T, (int32_t)H, N, (int32_t)k,
                                dt, algo, ptr(ws), stream_of(x.device())), "omni_expert_fwd");
   return y;
 }
 
 struct ExpertFn : public torch::autograd::Function<ExpertFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& up, const Tensor& down, const Tensor& gates, const Tensor& ids) {
-    Tensor scores;
-    Tensor y = expert_forward(x, up, down, gates, ids, OMNI_EXPERT_ALGO_AUTO, &scores);
+    Tensor scores = at::empty(ids.sizes(), x.options().dtype(at::kFloat));
+    Tensor y = expert_forward(x, x.size(0), up, down, ptr(gates), ptr(ids), ids.size(1), OMNI_EXPERT_ALGO_AUTO, ptr(scores));
     ctx->save_for_backward({x, up, down, gates, ids, scores});
     return y;
   }
@@ -133,7 +133,7 @@ py::object expert(const Tensor& x, const Tensor& up, const Tensor& down, const T
   {
     py::gil_scoped_release nogil;
     const c10::DeviceGuard guard(x.device());
-    y = grad ? ExpertFn::apply(x, up, down, gates, ids) : expert_forward(x, up, down, gates, ids, algo);
+    y = grad ? ExpertFn::apply(x, up, down, gates, ids) : expert_forward(x, x.size(0), up, down, ptr(gates), ptr(ids), ids.size(1), algo, nullptr);
   }
   return py::cast(y);
 }
@@ -168,15 +168,11 @@ struct Norms {
   }
 };
 
-struct RouterOut { Tensor gates, ids, ws; };
-RouterOut router_forward(const Tensor& x, int64_t T, int64_t H, const Tensor& wx, const Tensor& wy, const Norms& n, int64_t k) {
+void router_forward(const Tensor& x, int64_t T, int64_t H, const Tensor& wx, const Tensor& wy, const Norms& n, int64_t k, void* gates, void* ids, void* ws) {
   const int64_t r = wx.size(0);
-  const int dt = dtype_code(x.scalar_type());
-  RouterOut o{at::empty({T, k}, x.options()), at::empty({T, k}, x.options().dtype(at::kInt)), bytes(omni_router_workspace_bytes(T, (int32_t)r, dt), x.device())};
   check(omni_router_fwd(ptr(x), ptr(wx), ptr(wy), ptr(n.rmx), ptr(n.rvx), (int64_t*)ptr(n.nbx), ptr(n.rmy), ptr(n.rvy), (int64_t*)ptr(n.nby), n.training ? 1 : 0,
-                        (float)n.momentum, (float)n.eps, ptr(o.gates), (int32_t*)ptr(o.ids), nullptr, T, (int32_t)H, (int32_t)r, (int32_t)k, dt,
-                        dtype_code(n.rmx.scalar_type()), ptr(o.ws), stream_of(x.device())), "omni_router_fwd");
-  return o;
+                        (float)n.momentum, (float)n.eps, gates, (int32_t*)ids, nullptr, T, (int32_t)H, (int32_t)r, (int32_t)k, dtype_code(x.scalar_type()),
+                        dtype_code(n.rmx.scalar_type()), ws, stream_of(x.device())), "omni_router_fwd");
 }
 
 py::object router_stage(const Tensor& x, const Tensor& wx, const Tensor& wy, const Tensor& rmx, const Tensor& rvx, const c10::optional<Tensor>& nbx,
@@ -187,9 +183,12 @@ py::object router_stage(const Tensor& x, const Tensor& wx, const Tensor& wy, con
   if (k < 0 || k > r * r || k > 128 || k % 2 || !n.fits(x, r, x.size(0)) || records({&x, &wx, &wy}) || !prepare(x.device())) return py::none();
   py::gil_scoped_release nogil;
   const c10::DeviceGuard guard(x.device());
-  RouterOut o = router_forward(x, x.size(0), x.size(1), wx, wy, n, k);
+  const int64_t T = x.size(0);
+  Tensor gates = at::empty({T, k}, x.options()), ids = at::empty({T, k}, x.options().dtype(at::kInt));
+  Tensor ws = bytes(omni_router_workspace_bytes(T, (int32_t)r, dtype_code(x.scalar_type())), x.device());
+  router_forward(x, T, x.size(1), wx, wy, n, k, ptr(gates), ptr(ids), ptr(ws));
   py::gil_scoped_acquire gil;
-  return py::make_tuple(o.gates, o.ids);
+  return py::make_tuple(gates, ids);
 }
 
 // ---- shared MLP ------------------------------------------------------------------------------------
@@ -218,92 +217,117 @@ struct Layer {
   int64_t H = 0, I = 0, N = 0, r = 0, k = 0;
 };
 
-// One differentiable node for the whole layer (reference omni_moe.py:64-104).  Kept for the backward pass: the input, the gates,
-// ids and pair scores, the router's workspace (z and the statistics), the rounded gate and up projections and their SwiGLU product.
+// What the forward pass leaves for the backward one, in ONE allocation (as are the backward pass's temporaries): a step of 1000 tokens with
+// hidden 512 is bound by the host, and two dozen allocations and fifteen saved tensors cost it a fifth of its time (195-205 -> 160-168 us).
+struct Slab {
+  size_t size = 0;
+  size_t add(size_t n) {
+    const size_t at = size;
+    size += (n + 255) / 256 * 256;
+    return at;
+  }
+};
+struct Kept {                                       // gates and ids, the router's workspace (z and the statistics), pair scores, rounded gate and up projections, their SwiGLU product
+  Slab s;
+  size_t gates, ids, router, scores, gate, up, h;
+  Kept(int64_t T, int64_t I, int64_t r, int64_t k, int dt) {
+    const size_t es = dt == OMNI_F32 ? 4 : 2, pairs = (size_t)(T * k), wide = (size_t)(T * I) * es;
+    gates = s.add(pairs * es); ids = s.add(pairs * 4); router = s.add(omni_router_workspace_bytes(T, (int32_t)r, dt)); scores = s.add(pairs * 4);
+    gate = s.add(wide); up = s.add(wide); h = s.add(wide);
+  }
+};
+// [rows, cols] of dtype `like`, `at` bytes into the slab
+Tensor part(const Tensor& slab, size_t at, int64_t rows, int64_t cols, const Tensor& like) {
+  return slab.narrow(0, (int64_t)at, rows * cols * like.element_size()).view(like.scalar_type()).view({rows, cols});
+}
+
+// One differentiable node for the whole layer (reference omni_moe.py:64-104).
 struct LayerFn : public torch::autograd::Function<LayerFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& wg, const Tensor& wu, const Tensor& wd, const Tensor& rx, const Tensor& ry,
                         const Tensor& up, const Tensor& down, const Layer& l) {
     const int64_t T = x.numel() / l.H;
     const int dt = dtype_code(x.scalar_type());
     void* s = stream_of(x.device());
-    const RouterOut r = router_forward(x, T, l.H, rx, ry, l.norms, l.k);
-    const Tensor x2 = x.view({T, l.H});
-    Tensor scores;
-    const Tensor e = expert_forward(x2, up, down, r.gates, r.ids, OMNI_EXPERT_ALGO_AUTO, &scores);
-    Tensor h = at::empty({T, l.I}, x.options()), gate = at::empty({T, l.I}, x.options()), upp = at::empty({T, l.I}, x.options());
+    const Kept at(T, l.I, l.r, l.k, dt);
+    const Tensor kept = bytes(at.s.size, x.device());
+    uint8_t* k = (uint8_t*)ptr(kept);
+    router_forward(x, T, l.H, rx, ry, l.norms, l.k, k + at.gates, k + at.ids, k + at.router);
+    const Tensor e = expert_forward(x, T, up, down, k + at.gates, k + at.ids, l.k, OMNI_EXPERT_ALGO_AUTO, k + at.scores);
     if (dt != OMNI_F32) {                          // (rows of 16 bytes, so both sizes are multiples of 8; operands at any address)
-      check(omni_swiglu_linear_save_fwd(ptr(x), ptr(wg), ptr(wu), ptr(h), ptr(gate), ptr(upp), T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_swiglu_linear_save_fwd");
+      check(omni_swiglu_linear_save_fwd(ptr(x), ptr(wg), ptr(wu), k + at.h, k + at.gate, k + at.up, T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_swiglu_linear_save_fwd");
     } else {
-      check(omni_linear_fwd(ptr(x), ptr(wg), nullptr, ptr(gate), T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_linear_fwd");
-      check(omni_linear_fwd(ptr(x), ptr(wu), nullptr, ptr(upp), T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_linear_fwd");
-      check(omni_swiglu_fwd(ptr(gate), ptr(upp), ptr(h), T * l.I, dt, s), "omni_swiglu_fwd");
+      check(omni_linear_fwd(ptr(x), ptr(wg), nullptr, k + at.gate, T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_linear_fwd");
+      check(omni_linear_fwd(ptr(x), ptr(wu), nullptr, k + at.up, T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_linear_fwd");
+      check(omni_swiglu_fwd(k + at.gate, k + at.up, k + at.h, T * l.I, dt, s), "omni_swiglu_fwd");
     }
     Tensor y = at::empty_like(x);
-    check(omni_linear_fwd(ptr(h), ptr(wd), ptr(e), ptr(y), T, (int32_t)l.I, (int32_t)l.H, dt, s), "omni_linear_fwd");
-    ctx->save_for_backward({x, wg, wu, wd, rx, ry, up, down, r.gates, r.ids, r.ws, gate, upp, h, scores});
+    check(omni_linear_fwd(k + at.h, ptr(wd), ptr(e), ptr(y), T, (int32_t)l.I, (int32_t)l.H, dt, s), "omni_linear_fwd");
+    ctx->save_for_backward({x, wg, wu, wd, rx, ry, up, down, kept});
     ctx->saved_data["training"] = l.norms.training;
+    ctx->saved_data["top_k"] = l.k;
     return y;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
-    const Tensor &x3 = s[0], &wg = s[1], &wu = s[2], &wd = s[3], &rx = s[4], &ry = s[5], &up = s[6], &down = s[7], &gates = s[8], &ids = s[9], &rws = s[10], &gate = s[11],
-                 &upp = s[12], &h = s[13];
+    const Tensor &x3 = s[0], &wg = s[1], &wu = s[2], &wd = s[3], &rx = s[4], &ry = s[5], &up = s[6], &down = s[7], &kept = s[8];
     if (!grads[0].defined()) return variable_list(9);
     const c10::DeviceGuard guard(x3.device());
-    const int64_t H = wg.size(1), I = wg.size(0), N = up.size(0), r = rx.size(0), k = ids.size(1), T = x3.numel() / H;
+    const int64_t H = wg.size(1), I = wg.size(0), N = up.size(0), r = rx.size(0), k = ctx->saved_data["top_k"].toInt(), T = x3.numel() / H;
     const bool training = ctx->saved_data["training"].toBool();
     const int dt = dtype_code(x3.scalar_type());
     void* st = stream_of(x3.device());
-    const Tensor x = x3.view({T, H}), dy = grads[0].contiguous().view({T, H});
+    const Tensor dy = grads[0].contiguous();
     bool need[8];
     for (int i = 0; i < 8; ++i) need[i] = ctx->needs_input_grad(i);
-    const auto opt = x.options();
     variable_list out(9);
-    // experts, then the router stage behind their gates' gradient
-    Tensor dx_experts = at::empty({T, H}, opt), dup = at::empty_like(up), ddown = at::empty_like(down), dg = at::empty_like(gates);
-    {
-      Tensor ws = bytes(omni_expert_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt), x.device());
-      check(omni_expert_bwd_scores(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), (const float*)ptr(s[14]), ptr(dx_experts), ptr(dup), ptr(ddown),
-                                   ptr(dg), T, (int32_t)H, N, (int32_t)k, dt, ptr(ws), st), "omni_expert_bwd");
-    }
-    if (need[6]) out[6] = dup;
-    if (need[7]) out[7] = ddown;
     const bool own = dt != OMNI_F32, router = need[0] || need[4] || need[5];        // 16-bit products are the library's own
     const int64_t rp = own ? (r + 7) / 8 * 8 : r;
-    Tensor dz;
+    const Kept at(T, I, r, k, dt);
+    const uint8_t* saved = (const uint8_t*)ptr(kept);
+    // temporaries: the experts' d(x), d(gates), d(z), and one workspace for three stages that follow one another on the stream
+    Slab t;
+    const size_t es = own ? 2 : 4, dx_at = t.add((size_t)(T * H) * es), dg_at = t.add((size_t)(T * k) * es), dz_at = t.add(router ? (size_t)(T * 2 * rp) * es : 0);
+    const size_t ws_at = t.add(std::max({omni_expert_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt), router ? omni_router_norm_bwd_workspace_bytes(T, (int32_t)r) : 0,
+                                         own ? omni_mlp_bwd_workspace_bytes(T, (int32_t)H, (int32_t)I, (int32_t)r, dt) : 0}));
+    const Tensor temp = bytes(t.size, x3.device());
+    uint8_t* w = (uint8_t*)ptr(temp);
+    // experts, then the router stage behind their gates' gradient
+    Tensor dup = at::empty_like(up), ddown = at::empty_like(down);
+    check(omni_expert_bwd_scores(ptr(dy), ptr(x3), ptr(up), ptr(down), saved + at.gates, (const int32_t*)(saved + at.ids), (const float*)(saved + at.scores), w + dx_at, ptr(dup),
+                                 ptr(ddown), w + dg_at, T, (int32_t)H, N, (int32_t)k, dt, w + ws_at, st), "omni_expert_bwd");
+    if (need[6]) out[6] = dup;
+    if (need[7]) out[7] = ddown;
     if (router) {
-      dz = at::empty({T, 2 * rp}, opt);
-      Tensor nws = bytes(omni_router_norm_bwd_workspace_bytes(T, (int32_t)r), x.device());
-      const uint8_t* z = (const uint8_t*)ptr(rws);
+      const uint8_t* z = saved + at.router;
       const float* stats = (const float*)(z + omni_router_workspace_stats_offset(T, (int32_t)r, dt));
-      check((own ? omni_router_norm_bwd_padded : omni_router_norm_bwd)(ptr(dg), ptr(gates), (const int32_t*)ptr(ids), z, stats, ptr(dz), T, (int32_t)r, (int32_t)k, dt,
-                                                                        training ? 1 : 0, ptr(nws), st), "omni_router_norm_bwd");
+      check((own ? omni_router_norm_bwd_padded : omni_router_norm_bwd)(w + dg_at, saved + at.gates, (const int32_t*)(saved + at.ids), z, stats, w + dz_at, T, (int32_t)r,
+                                                                        (int32_t)k, dt, training ? 1 : 0, w + ws_at, st), "omni_router_norm_bwd");
     }
     if (own) {
-      const Tensor* like[6] = {&x, &wg, &wu, &wd, &rx, &ry};
+      const Tensor* like[6] = {&x3, &wg, &wu, &wd, &rx, &ry};
       for (int i = 0; i < 6; ++i)
         if (need[i]) out[i] = at::empty_like(*like[i]);
-      Tensor ws = bytes(omni_mlp_bwd_workspace_bytes(T, (int32_t)H, (int32_t)I, (int32_t)r, dt), x.device());
-      const int32_t code = omni_mlp_bwd(ptr(dy), ptr(x), ptr(wg), ptr(wu), ptr(wd), ptr(gate), ptr(upp), ptr(h), ptr(dz), ptr(rx), ptr(ry), ptr(dx_experts), ptr(out[0]),
-                                        ptr(out[1]), ptr(out[2]), ptr(out[3]), ptr(out[4]), ptr(out[5]), T, (int32_t)H, (int32_t)I, (int32_t)r, dt, ptr(ws), st);
+      const int32_t code = omni_mlp_bwd(ptr(dy), ptr(x3), ptr(wg), ptr(wu), ptr(wd), saved + at.gate, saved + at.up, saved + at.h, router ? w + dz_at : nullptr, ptr(rx),
+                                        ptr(ry), w + dx_at, ptr(out[0]), ptr(out[1]), ptr(out[2]), ptr(out[3]), ptr(out[4]), ptr(out[5]), T, (int32_t)H, (int32_t)I,
+                                        (int32_t)r, dt, w + ws_at, st);
       if (code != OMNI_ERR_UNSUPPORTED) {
         check(code, "omni_mlp_bwd");
-        if (need[0]) out[0] = out[0].view(x3.sizes());
         return out;
       }
     }
     // single precision, operands off a 16-byte boundary, and operands of 2 GiB and more: library products
-    Tensor dx = dx_experts;
+    const Tensor x = x3.view({T, H}), dy2 = dy.view({T, H}), gate = part(kept, at.gate, T, I, x3), upp = part(kept, at.up, T, I, x3);
+    Tensor dx = part(temp, dx_at, T, H, x3);
     if (router) {
-      const Tensor zx = dz.narrow(1, 0, r), zy = dz.narrow(1, rp, r);
+      const Tensor dz = part(temp, dz_at, T, 2 * rp, x3), zx = dz.narrow(1, 0, r), zy = dz.narrow(1, rp, r);
       if (need[4]) out[4] = at::mm(zx.t(), x);
       if (need[5]) out[5] = at::mm(zy.t(), x);
-      if (need[0]) dx.addmm_(zx, rx).addmm_(zy, ry);
+      if (need[0]) dx = at::addmm(dx, zx, rx).addmm_(zy, ry);                       // (a tensor of its own)
     }
-    if (need[3]) out[3] = at::mm(dy.t(), h);
+    if (need[3]) out[3] = at::mm(dy2.t(), part(kept, at.h, T, I, x3));
     if (need[0] || need[1] || need[2]) {
-      const Tensor dh = at::mm(dy, wd);
+      const Tensor dh = at::mm(dy2, wd);
       Tensor dgate = at::empty_like(gate), dupp = at::empty_like(upp);
       check(omni_swiglu_bwd(ptr(dh), ptr(gate), ptr(upp), ptr(dgate), ptr(dupp), T * I, dt, st), "omni_swiglu_bwd");
       if (need[1]) out[1] = at::mm(dgate.t(), x);

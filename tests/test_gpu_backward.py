@@ -477,6 +477,23 @@ def test_layer_gradients_only_where_wanted(dtype, device):
                 assert grad is None or torch.equal(grad, full[m]), (wanted, m)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_layer_saved_tensors_through_hooks(dtype, device):
+    """What the layer's node keeps may be moved away by saved-tensor hooks and come back elsewhere, and is left whole for a second backward pass."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    torch.manual_seed(9)
+    layer = OmniMoE(OmniMoEConfig(128, 256, "silu", 100, 6)).to(device=device, dtype=dtype).eval()
+    x, dy = (torch.randn(1, 77, 128, device=device).to(dtype) for _ in range(2))
+    leaves = [x.requires_grad_(), *layer.parameters()]
+    y = layer(x)
+    first = torch.autograd.grad(y, leaves, dy, retain_graph=True)
+    second = torch.autograd.grad(y, leaves, dy)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(device)):
+        moved = torch.autograd.grad(layer(x), leaves, dy)
+    for a, b, c in zip(first, second, moved):
+        assert torch.equal(a, b) and torch.equal(a, c)
+
+
 def test_layer_trains_bf16(device):
     """A few SGD steps on a bf16 layer through the HIP forward and backward reduce a regression loss; the
     no_grad forward of the same weights takes the fused path and agrees with the composed one."""
