@@ -34,6 +34,8 @@ constexpr int kBK = 64;                       // K elements per LDS stage
 constexpr int kRowBytes = kBK * 2 + 16;       // padded LDS row
 constexpr int kGemmThreads = 256;
 
+constexpr int ksplit_lds(int tm) { return 4 * (tm == 1 ? 3 : 2) * (32 * tm + 64) * 128; }    // gemm_ksplit_kernel's four rings
+
 enum : int { kEpiPlain = 0, kEpiSwiglu = 1, kEpiResidual = 2, kEpiStats = 3, kEpiGate = 4 };   // kEpiStats: plain + column statistics; kEpiGate: silu(acc) * gate, as a pair of 16-bit values
 
 template <int DT> struct ElemBytes { static constexpr int value = (DT == kF32) ? 4 : 2; };
@@ -609,56 +611,60 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_nt_dma_kernel(const GemmArgs 
   gemm_epilogue<DT, TM, TN, EPI>(g, acc, m0, n0, wm, wn, lane);
 }
 
-// ---- few output tiles, long K: the K tiles of one 64 x 64 output tile dealt out over the block's four waves ----------
+// ---- few output tiles, long K: the K tiles of one 32 TM x 64 output tile dealt out over the block's four waves ----------
 // A product like the router projection at a few thousand tokens (4096 x 128 x 1024) has too few output tiles to fill the
 // GPU and its time is the latency of one block's K loop: with the ring kernel above, 16 rounds of wait - barrier - four
-// MFMAs.  Here every wave multiplies the whole 64 x 64 tile (2 x 2 MFMA tiles) over ITS K tiles (kt = wave, wave + 4,
-// ...) through a two-stage LDS ring of its own, so the K loop is a quarter as long, has four independent accumulators
+// MFMAs.  Here every wave multiplies the whole tile (TM x 2 MFMA tiles) over ITS K tiles (kt = wave, wave + 4,
+// ...) through an LDS ring of its own, so the K loop is a quarter as long, has independent accumulators
 // to keep the matrix pipeline fed, and meets no block barrier: a wave waits only for its own loads.  The four partial
 // tiles then meet in LDS (summed in wave order, so the result does not depend on timing), and wave w finishes MFMA tile
-// (w % 2, w / 2) with the common epilogue.  Needs K % 64 == 0; worth it while there are fewer tiles than CUs.
-template <int DT, int EPI>
+// (w % TM, w / TM) with the common epilogue.  Needs K % 64 == 0; worth it while there are fewer tiles than CUs.
+// TM = 1 where that makes at most 256 blocks and nothing runs beside the launch: every CU may have one, which loads three quarters as much, with three
+// stages in flight instead of two (router stage of 1000 / 2048 / 4096 tokens, hidden 1024, 64 keys: 16.3 / 16.8 / 19.3 -> 15.6 / 16.3 / 18.5 us).  Beside gate/up,
+// whose tiles take 128 KiB of LDS of a CU, blocks of both kinds wait for one another: the 4096-token layer on two streams 118 -> 130 us.
+template <int DT, int EPI, int TM>
 __global__ __launch_bounds__(kGemmThreads, 1) void gemm_ksplit_kernel(const GemmArgs g) {
-  constexpr int kRow = 128, kTile = 64 * kRow;          // one operand's 64 rows of a K tile
-  constexpr int kStage = 2 * kTile, kRing = 2 * kStage; // per wave: two stages of [activations | weights]
+  constexpr int kRow = 128, kATile = 32 * TM * kRow, kBTile = 64 * kRow, PA = 4 * TM, PB = 8;      // a K tile of each operand, in 1-KiB loads
+  constexpr int NS = TM == 1 ? 3 : 2, kStage = kATile + kBTile, kRing = NS * kStage;              // per wave: stages of [activations | weights]
+  static_assert(4 * kRing == ksplit_lds(TM), "launch and kernel disagree");
   extern __shared__ __align__(16) uint8_t lds[];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tile_m = blockIdx.x % g.tiles_m, tile_n = blockIdx.x / g.tiles_m;
-  const int m0 = tile_m * 64, n0 = tile_n * 64;
+  const int m0 = tile_m * 32 * TM, n0 = tile_n * 64;
   uint8_t* ring = lds + wave * kRing;
 
-  // load instruction p (0..7) fills rows 8p + lane/8 of an operand tile; the lane fetches the logical chunk that belongs at
+  // load instruction p fills rows 8p + lane/8 of an operand tile; the lane fetches the logical chunk that belongs at
   // its (swizzled) position
-  const uint8_t* a_src[8];
-  const uint8_t* b_src[8];
+  const uint8_t* a_src[PA];
+  const uint8_t* b_src[PB];
 #pragma unroll
-  for (int p = 0; p < 8; ++p) {
+  for (int p = 0; p < PA; ++p) {
+    const int rl = p * 8 + (lane >> 3), row = min(m0 + rl, g.M - 1);      // clamp: tail rows and columns are never stored
+    a_src[p] = g.a + ((int64_t)row * g.K + swizzle<64>(rl, lane & 7) * 8) * 2;
+  }
+#pragma unroll
+  for (int p = 0; p < PB; ++p) {
     const int rl = p * 8 + (lane >> 3);
-    const int c = swizzle<64>(rl, lane & 7);
-    int row = m0 + rl;
-    row = row < g.M ? row : g.M - 1;                    // clamp: tail rows and columns are never stored
-    a_src[p] = g.a + ((int64_t)row * g.K + c * 8) * 2;
-    int col = n0 + rl;
-    col = col < g.N ? col : g.N - 1;
+    int col = min(n0 + rl, g.N - 1);
     const uint8_t* base = g.b0;
     if constexpr (EPI == kEpiPlain || EPI == kEpiStats) {
       if (g.b1 && col >= g.N / 2) { base = g.b1; col -= g.N / 2; }
     }
-    b_src[p] = base + ((int64_t)col * g.K + c * 8) * 2;
+    b_src[p] = base + ((int64_t)col * g.K + swizzle<64>(rl, lane & 7) * 8) * 2;
   }
   auto issue_tile = [&](int kt, int stage) __attribute__((always_inline)) {
     uint8_t* st = ring + stage * kStage;
     const int koff = kt * kRow;
 #pragma unroll
-    for (int p = 0; p < 8; ++p)
+    for (int p = 0; p < PA; ++p)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(a_src[p] + koff),
                                        (__attribute__((address_space(3))) void*)(st + p * 1024), 16, 0, 0);
 #pragma unroll
-    for (int p = 0; p < 8; ++p)
+    for (int p = 0; p < PB; ++p)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(b_src[p] + koff),
-                                       (__attribute__((address_space(3))) void*)(st + kTile + p * 1024), 16, 0, 0);
+                                       (__attribute__((address_space(3))) void*)(st + kATile + p * 1024), 16, 0, 0);
   };
 
   // fragment reads: lane reads row lane%32 (+32 i), logical chunk 2*slab + lane/32
@@ -667,9 +673,9 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_ksplit_kernel(const Gemm
 #pragma unroll
   for (int sl = 0; sl < 4; ++sl) off_slab[sl] = rl * kRow + swizzle<64>(rl, 2 * sl + (lane >> 5)) * 16;
 
-  f32x16_t acc[2][2];
+  f32x16_t acc[TM][2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -677,57 +683,65 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_ksplit_kernel(const Gemm
 
   const int num_kt = g.K / 64;
   const int mine = (num_kt - wave + 3) / 4;             // K tiles wave, wave + 4, ...
-  if (mine > 0) issue_tile(wave, 0);
-  if (mine > 1) issue_tile(wave + 4, 1);
+#pragma unroll
+  for (int t = 0; t < NS; ++t)
+    if (mine > t) issue_tile(wave + 4 * t, t);
+  int stage = 0;
   for (int t = 0; t < mine; ++t) {
-    if (t + 1 < mine) wait_vmcnt<16>(); else wait_vmcnt<0>();     // this tile has landed; the next one may be in flight
-    const uint8_t* st = ring + (t & 1) * kStage;
-    u32x4_t af[2][2], bf[2][2];
+    // this tile has landed; the next ones may be in flight
+    const int younger = min(mine - 1 - t, NS - 1);
+    if (NS > 2 && younger > 1) wait_vmcnt<2 * (PA + PB)>();
+    else if (younger > 0) wait_vmcnt<PA + PB>();
+    else wait_vmcnt<0>();
+    const uint8_t* st = ring + stage * kStage;
+    u32x4_t af[2][TM], bf[2][2];
     auto read_slab = [&](int sl) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) af[sl & 1][i] = *(const u32x4_t*)(st + off_slab[sl] + i * 32 * kRow);
+      for (int i = 0; i < TM; ++i) af[sl & 1][i] = *(const u32x4_t*)(st + off_slab[sl] + i * 32 * kRow);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) bf[sl & 1][j] = *(const u32x4_t*)(st + kTile + off_slab[sl] + j * 32 * kRow);
+      for (int j = 0; j < 2; ++j) bf[sl & 1][j] = *(const u32x4_t*)(st + kATile + off_slab[sl] + j * 32 * kRow);
     };
     read_slab(0);
 #pragma unroll
     for (int sl = 0; sl < 4; ++sl) {
       if (sl + 1 < 4) read_slab(sl + 1);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = mfma32<DT>(bf[sl & 1][j], af[sl & 1][i], acc[i][j]);
     }
-    if (t + 2 < mine) {
+    if (t + NS < mine) {
       wait_lds_reads();                                  // the stage is read out (by this wave, its only reader)
-      issue_tile(wave + 4 * (t + 2), t & 1);
+      issue_tile(wave + 4 * (t + NS), stage);
     }
+    stage = stage + 1 == NS ? 0 : stage + 1;
   }
 
   // ---- the four partial tiles meet in LDS: [wave][MFMA tile][column group][lane] 16 bytes each
   __syncthreads();                                       // every wave is done with its ring
   f32x4_t* xch = (f32x4_t*)lds;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4)
-        xch[((wave * 4 + (j * 2 + i)) * 4 + q4) * 64 + lane] =
+        xch[((wave * 2 * TM + (j * TM + i)) * 4 + q4) * 64 + lane] =
             f32x4_t{acc[i][j][q4 * 4], acc[i][j][q4 * 4 + 1], acc[i][j][q4 * 4 + 2], acc[i][j][q4 * 4 + 3]};
   __syncthreads();
+  if (wave >= 2 * TM) return;
   f32x16_t sum[1][1];
 #pragma unroll
   for (int q4 = 0; q4 < 4; ++q4) {
-    f32x4_t v = xch[((0 * 4 + wave) * 4 + q4) * 64 + lane];
+    f32x4_t v = xch[(wave * 4 + q4) * 64 + lane];
 #pragma unroll
     for (int w = 1; w < 4; ++w) {
-      const f32x4_t o = xch[((w * 4 + wave) * 4 + q4) * 64 + lane];
+      const f32x4_t o = xch[((w * 2 * TM + wave) * 4 + q4) * 64 + lane];
       v[0] += o[0]; v[1] += o[1]; v[2] += o[2]; v[3] += o[3];
     }
     sum[0][0][q4 * 4] = v[0]; sum[0][0][q4 * 4 + 1] = v[1]; sum[0][0][q4 * 4 + 2] = v[2]; sum[0][0][q4 * 4 + 3] = v[3];
   }
-  gemm_epilogue<DT, 1, 1, EPI>(g, sum, m0, n0, wave & 1, wave >> 1, lane);
+  gemm_epilogue<DT, 1, 1, EPI>(g, sum, m0, n0, wave % TM, wave / TM, lane);
 }
 
 // ---- single precision with few output tiles -----------------------------------------------------------
@@ -853,9 +867,9 @@ template <int DT, int TM, int TN, int EPI, int BK, int NS, int NW = 4>
 struct DmaKernelLds {
   static inline LdsKernel entry{(const void*)gemm_nt_dma_kernel<DT, TM, TN, EPI, BK, NS, NW>, NS * (2 * TM * 32 + (NW / 2) * TN * 32) * BK * 2};
 };
-template <int DT, int EPI>
+template <int DT, int EPI, int TM>
 struct KsplitKernelLds {
-  static inline LdsKernel entry{(const void*)gemm_ksplit_kernel<DT, EPI>, 4 * 2 * 2 * 64 * 128};
+  static inline LdsKernel entry{(const void*)gemm_ksplit_kernel<DT, EPI, TM>, ksplit_lds(TM)};
 };
 template <int EPI>
 struct SmallF32Lds {
@@ -893,7 +907,7 @@ static int64_t f32_small_blocks_of(GemmArgs& g) {              // ... against th
 }
 
 template <int DT, int TM, int TN, int EPI>
-static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
+static hipError_t launch_gemm(GemmArgs g, hipStream_t s, bool exclusive = false) {
   constexpr int BM = 2 * TM * 32, BR = 2 * TN * 32, BN = (EPI == kEpiSwiglu) ? BR / 2 : BR;
   constexpr int kLds = 2 * (BM + BR) * kRowBytes;
   g.tiles_m = (g.M + BM - 1) / BM;
@@ -921,8 +935,15 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s) {
     if constexpr (TM == 1 && TN == 1 && EPI != kEpiGate) {
       // fewer 64 x 64 tiles than CUs and at least two K tiles per wave: the K tiles dealt out over the waves
       if (blocks <= 256 && g.K >= 512) {
-        if (hipError_t e = KsplitKernelLds<DT, EPI>::entry.ensure(); e != hipSuccess) return e;
-        hipLaunchKernelGGL((gemm_ksplit_kernel<DT, EPI>), dim3(blocks), dim3(kGemmThreads), 4 * 2 * 2 * 64 * 128, s, g);
+        const int tiles32 = (g.M + 31) / 32, blocks32 = tiles32 * g.tiles_n;
+        if (exclusive && blocks32 <= 256) {
+          g.tiles_m = tiles32;
+          if (hipError_t e = KsplitKernelLds<DT, EPI, 1>::entry.ensure(); e != hipSuccess) return e;
+          hipLaunchKernelGGL((gemm_ksplit_kernel<DT, EPI, 1>), dim3(blocks32), dim3(kGemmThreads), ksplit_lds(1), s, g);
+          return hipGetLastError();
+        }
+        if (hipError_t e = KsplitKernelLds<DT, EPI, 2>::entry.ensure(); e != hipSuccess) return e;
+        hipLaunchKernelGGL((gemm_ksplit_kernel<DT, EPI, 2>), dim3(blocks), dim3(kGemmThreads), ksplit_lds(2), s, g);
         return hipGetLastError();
       }
     }
@@ -1000,7 +1021,7 @@ static int gemm_plain(const void* a, const void* b, const void* b_hi, const void
   } else if (part_mean) {
     if (big >= 200) err = launch_gemm<DT, 4, 4, kEpiStats>(g, s);
     else if (mid >= 200) err = launch_gemm<DT, 2, 2, kEpiStats>(g, s);
-    else err = launch_gemm<DT, 1, 1, kEpiStats>(g, s);
+    else err = launch_gemm<DT, 1, 1, kEpiStats>(g, s, exclusive);
   } else {
     if (big >= 200) err = launch_gemm<DT, 4, 4, kEpiPlain>(g, s);
     else if (mid >= 200) err = launch_gemm<DT, 2, 2, kEpiPlain>(g, s);
@@ -1059,11 +1080,11 @@ int omni_gemm_gated(const void* x, const void* w, const float* gate, void* c, in
 }
 
 int omni_gemm_router_projection(const void* x, const void* wx, const void* wy, void* z, float* part_mean, float* part_m2,
-                                int64_t T, int H, int r, int dtype, void* stream) {
+                                int64_t T, int H, int r, int dtype, void* stream, bool exclusive) {
   using namespace omni;
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == OMNI_BF16) return gemm_plain<kBF16>(x, wx, wy, nullptr, z, T, 2 * (int64_t)r, H, s, part_mean, part_m2);
-  if (dtype == OMNI_F16) return gemm_plain<kF16>(x, wx, wy, nullptr, z, T, 2 * (int64_t)r, H, s, part_mean, part_m2);
+  if (dtype == OMNI_BF16) return gemm_plain<kBF16>(x, wx, wy, nullptr, z, T, 2 * (int64_t)r, H, s, part_mean, part_m2, true, exclusive || !part_mean);
+  if (dtype == OMNI_F16) return gemm_plain<kF16>(x, wx, wy, nullptr, z, T, 2 * (int64_t)r, H, s, part_mean, part_m2, true, exclusive || !part_mean);
   if (dtype == OMNI_F32) return gemm_plain<kF32>(x, wx, wy, nullptr, z, T, 2 * (int64_t)r, H, s, part_mean, part_m2);
   return OMNI_ERR_DTYPE;
 }

@@ -21,7 +21,7 @@
 // defined beside the GEMM kernels: z = x [Wx;Wy]^T, optionally with per-32-row column
 // partial statistics (mean, M2) [ceil(T/32)][2r] of the rounded z
 int omni_gemm_router_projection(const void* x, const void* wx, const void* wy, void* z, float* part_mean, float* part_m2,
-                                int64_t T, int H, int r, int dtype, void* stream);
+                                int64_t T, int H, int r, int dtype, void* stream, bool exclusive = true);
 
 namespace omni {
 
@@ -294,14 +294,15 @@ extern "C" OMNI_API size_t omni_router_workspace_stats_offset(int64_t num_tokens
   return align256((size_t)num_tokens * 2 * (size_t)num_expert_sqrt * es);
 }
 
-extern "C" OMNI_API int32_t omni_router_fwd(const void* x, const void* weight_x, const void* weight_y,
-                                            void* running_mean_x, void* running_var_x, int64_t* num_batches_tracked_x,
-                                            void* running_mean_y, void* running_var_y, int64_t* num_batches_tracked_y,
-                                            int32_t training, float momentum, float eps, void* gates, int32_t* indices,
-                                            void* scores, int64_t num_tokens, int32_t hidden_size, int32_t num_expert_sqrt,
-                                            int32_t num_experts_per_token, int32_t dtype, int32_t stats_dtype,
-                                            void* workspace, void* stream) {
-  using namespace omni;
+namespace omni {
+// exclusive: nothing is meant to run beside the call
+int router_fwd(const void* x, const void* weight_x, const void* weight_y,
+               void* running_mean_x, void* running_var_x, int64_t* num_batches_tracked_x,
+               void* running_mean_y, void* running_var_y, int64_t* num_batches_tracked_y,
+               int32_t training, float momentum, float eps, void* gates, int32_t* indices,
+               void* scores, int64_t num_tokens, int32_t hidden_size, int32_t num_expert_sqrt,
+               int32_t num_experts_per_token, int32_t dtype, int32_t stats_dtype,
+               void* workspace, void* stream, bool exclusive) {
   const int r = num_expert_sqrt, k = num_experts_per_token;
   if (num_tokens < 0 || num_tokens > INT32_MAX / 256 || r <= 0 || hidden_size <= 0) return OMNI_ERR_SHAPE;
   if (k < 0 || (int64_t)k > (int64_t)r * r || k > 128 || (k & 1)) return OMNI_ERR_TOPK;
@@ -327,7 +328,7 @@ extern "C" OMNI_API int32_t omni_router_fwd(const void* x, const void* weight_x,
   // z = x [Wx;Wy]^T on the matrix cores
   // (in training its epilogue also leaves the per-32-row column statistics)
   if (int e = omni_gemm_router_projection(x, weight_x, weight_y, z, training ? part_mean : nullptr, training ? part_m2 : nullptr,
-                                          num_tokens, hidden_size, r, dtype, stream)) return e;
+                                          num_tokens, hidden_size, r, dtype, stream, exclusive)) return e;
   // Training: one more launch merges the partial statistics and moves the running buffers.  In eval mode the
   // select kernel reads the running buffers itself (and leaves mean and 1/sqrt(var + eps) in `stats`).
   if (training || k == 0) {
@@ -352,4 +353,16 @@ extern "C" OMNI_API int32_t omni_router_fwd(const void* x, const void* weight_x,
     g.stats_out = stats; g.stat_dt = stats_dtype; g.eps = eps;
   }
   return select_dispatch(g, s);
+}
+}  // namespace omni
+
+extern "C" OMNI_API int32_t omni_router_fwd(const void* x, const void* weight_x, const void* weight_y,
+                                            void* running_mean_x, void* running_var_x, int64_t* num_batches_tracked_x,
+                                            void* running_mean_y, void* running_var_y, int64_t* num_batches_tracked_y,
+                                            int32_t training, float momentum, float eps, void* gates, int32_t* indices,
+                                            void* scores, int64_t num_tokens, int32_t hidden_size, int32_t num_expert_sqrt,
+                                            int32_t num_experts_per_token, int32_t dtype, int32_t stats_dtype,
+                                            void* workspace, void* stream) {
+  return omni::router_fwd(x, weight_x, weight_y, running_mean_x, running_var_x, num_batches_tracked_x, running_mean_y, running_var_y, num_batches_tracked_y, training, momentum, eps,
+                          gates, indices, scores, num_tokens, hidden_size, num_expert_sqrt, num_experts_per_token, dtype, stats_dtype, workspace, stream, true);
 }

@@ -569,3 +569,32 @@ def test_expert_unused_rows_may_hold_nan(algo, device):
     up2[0], down2[0] = float("nan"), float("inf")
     got = _ops().hip_omni_expert_func(d[0], up2.to(device), down2.to(device), d[3], d[4], algo=algo)
     assert torch.isfinite(got).all() and torch.equal(got, want)
+
+
+# ---------------------------------------------------------------- router projection with column statistics
+@pytest.mark.parametrize("case", [(2, 1024, 64), (31, 512, 32), (33, 576, 20), (1000, 512, 32), (4096, 1024, 64), (4097, 1024, 64), (8193, 512, 16), (95, 2048, 130)],
+                         ids=lambda c: "T%d-H%d-r%d" % c)
+def test_router_projection_and_statistics(case, device):
+    """z and its batch statistics as a training-mode router stage leaves them, in blocks of 32 and of 64 rows: full and partial strips, K tiles that the waves share
+    evenly or not, the last size that is in 32-row blocks and the next.  z is a sum of H products of bf16 values in fp32 (error below H 2^-24 of the sum of magnitudes,
+    here under 2^-10) rounded once (2^-8); the statistics are those of the stored z, in fp32."""
+    from omni_moe.ops.hip import _lib
+    lib = _lib.load()
+    T, H, r = case
+    g = torch.Generator(device=device).manual_seed(T + r)
+    x = torch.empty(T, H, device=device).normal_(generator=g).bfloat16()
+    w = torch.empty(2, r, H, device=device).normal_(0, H ** -0.5, generator=g).bfloat16()
+    run = [torch.zeros(r, device=device), torch.ones(r, device=device), torch.zeros((), device=device, dtype=torch.long)] * 2
+    gates, ids = torch.empty(T, 2, device=device, dtype=torch.bfloat16), torch.empty(T, 2, device=device, dtype=torch.int32)
+    ws = torch.empty(lib.omni_router_workspace_bytes(T, r, _lib.OMNI_BF16), device=device, dtype=torch.uint8)
+    run = [t.clone() for t in run]
+    _lib.check(lib.omni_router_fwd(x.data_ptr(), w[0].data_ptr(), w[1].data_ptr(), *(t.data_ptr() for t in run), 1, 0.1, 1e-5, gates.data_ptr(), ids.data_ptr(), None, T, H, r, 2,
+                                   _lib.OMNI_BF16, _lib.OMNI_F32, ws.data_ptr(), _lib.stream_ptr()), "omni_router_fwd")
+    z = ws[:T * 2 * r * 2].view(torch.bfloat16).view(T, 2 * r).double()
+    want = x.double() @ w.double().reshape(2 * r, H).t()
+    assert ((z - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -10).all()
+    at = lib.omni_router_workspace_stats_offset(T, r, _lib.OMNI_BF16)
+    stats = ws[at:at + 16 * r].view(torch.float32).view(2, 2, r).double()
+    mean, var = z.mean(0).view(2, r), z.var(0, unbiased=False).view(2, r)
+    assert ((stats[:, 0] - mean).abs() <= 1e-5 * (1 + mean.abs())).all()
+    assert ((stats[:, 1] * torch.sqrt(var + 1e-5) - 1).abs() <= 1e-4).all()
