@@ -484,12 +484,10 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
     }
     return;
   }
-  // What the epilogue reads (the residual, or gate and up) is requested row tiles ahead, from inside the matrix whatever the lane: a wait for each
-  // piece in turn made the SwiGLU backward of 4096 x 4096 x 1024 take 28 us on top of 32.  Gate and up three ahead, in the registers that the fragments
-  // had (12 KiB of them in flight per wave instead of 4: 58.2 -> 55.0 us); the residual one (three: 4096 x 1024 x 4096 37.7 -> 43.8).
+  // What the epilogue reads (the residual, or gate and up) is requested one row tile ahead, from inside the matrix whatever the lane: a wait for each
+  // piece in turn made the SwiGLU backward of 4096 x 4096 x 1024 take 28 us on top of 32.
   constexpr int kJ = (EPI == kTileSwiglu ? TN / 2 : TN) / 2, kSide = EPI == kTileSwigluBwd ? 2 : EPI == kTileResidual ? 1 : 0;
-  constexpr int kAhead = EPI == kTileSwigluBwd && KG == 1 ? 3 : 1, kBufs = kAhead + 1;
-  u32x4_t side[kBufs][kJ][kSide ? kSide : 1];
+  u32x4_t side[2][kJ][kSide ? kSide : 1];
   auto place = [&](int i, int jp, int& m, int& n) { m = m0 + (wm * TM + i) * 16 + tr; n = nb + (2 * jp + (tg & 1)) * 16 + (tg & 2) * 4; };
   auto request = [&](int i) {
     if constexpr (kSide > 0) {
@@ -498,21 +496,16 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
         int m, n;
         place(i, jp, m, n);
         const int64_t at = (int64_t)min(m, M - 1) * p.ldc + (int64_t)min(n, N - 8) * 2;
-        side[i % kBufs][jp][0] = *(const u32x4_t*)((EPI == kTileResidual ? p.res : p.gate) + at);
-        if constexpr (kSide == 2) side[i % kBufs][jp][kSide - 1] = *(const u32x4_t*)(p.up + at);
+        side[i & 1][jp][0] = *(const u32x4_t*)((EPI == kTileResidual ? p.res : p.gate) + at);
+        if constexpr (kSide == 2) side[i & 1][jp][kSide - 1] = *(const u32x4_t*)(p.up + at);
       }
     }
   };
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     if (KG == 2 && i / (TM / 2) != kg) continue;
-    auto here = [i](int t) { return t < TM && (KG == 1 || t / (TM / 2) == i / (TM / 2)); };      // the group's row tiles
-    if (i == 0 || (KG == 2 && i == TM / 2)) {
-#pragma unroll
-      for (int a = 0; a < kAhead; ++a)
-        if (here(i + a)) request(i + a);
-    }
-    if (here(i + kAhead)) request(i + kAhead);
+    if (i == 0 || (KG == 2 && i == TM / 2)) request(i);
+    if (i + 1 < TM && (KG == 1 || (i + 1) / (TM / 2) == i / (TM / 2))) request(i + 1);
 #pragma unroll
     for (int jp = 0; jp < kJ; ++jp) {
       const int j = 2 * jp;
@@ -540,7 +533,7 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
         u32x4_t dg, du;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const uint32_t oq = out[q], gq = side[i % kBufs][jp][0][q], uq = side[i % kBufs][jp][kSide - 1][q];
+          const uint32_t oq = out[q], gq = side[i & 1][jp][0][q], uq = side[i & 1][jp][kSide - 1][q];
           uint32_t a, b;
           swiglu_bwd_word<DT>(oq, gq, uq, a, b);
           dg[q] = a; du[q] = b;
@@ -553,7 +546,7 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
         if constexpr (EPI == kTileResidual) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const uint32_t o = out[q], rq = side[i % kBufs][jp][0][q];
+            const uint32_t o = out[q], rq = side[i & 1][jp][0][q];
             out[q] = pack16x2<DT>(lo16<DT>(o) + lo16<DT>(rq), hi16<DT>(o) + hi16<DT>(rq));
           }
         }
