@@ -9,10 +9,11 @@
 //
 // What bounds it.  The 256 x 256 tile at K = 2048 and more: the matrix pipelines under the board's power limit (gate/up at 32768 x 2 8192 x 2048: busy 70 % of
 // the cycles at 1.90 GHz, 1.40 PFLOP/s); at K = 1024 the 16 ring steps between its fill and its epilogue (4096 x 2 4096 x 1024: 51 % at 2.08 GHz, 1.11
-// PFLOP/s with a block to a tile, 58 % and 1.23 streamed; d(h) with the SwiGLU backward as epilogue 28 %, 0.62).  The
+// PFLOP/s with a block to a tile, 58 % and 1.23 streamed; d(h) with the SwiGLU backward as epilogue 57 us, 0.60 PFLOP/s, half of them its 134 MB).  The
 // 128 x 128 tile: the path from L2 into LDS, which carries 64 bytes per cycle and CU -- what that tile asks for at full matrix rate --
 // and, with one block to a CU, the chain of reads and waits between two barriers.  So a block's waves keep 64 x 64 of the tile each (LDS
-// serves 256 bytes a cycle, and smaller wave tiles read more per product) and, alone on its CU, a block has two groups of four waves
+// serves 256 bytes a cycle, and smaller wave tiles read more per product) and, alone on its CU, a block has four ring stages in flight (two groups of four
+// waves with two stages each instead: 4096 x 1024 x 4096 36.4 -> 39.2 us, x 8192 75 -> 94); the 64 x 64 tile has two groups of waves
 // that take every other K tile and add up at the end: one barrier for two K tiles and a second wave to issue while the first waits.
 // Splitting K over the grid costs a pass over fp32 partial sums (summed in split order: results do not depend on timing).
 #include "common.h"

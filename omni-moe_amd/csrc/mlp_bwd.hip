@@ -3,7 +3,7 @@
 //   d(gate), d(up) [T,I]  from  d(h) = dy Wd, the SwiGLU backward as its epilogue: d(h) itself never reaches memory
 //   dWg, dWu, dWd, dWx, dWy  in one launch: each has too few tiles to fill the chip alone
 //   d(x) = dgate Wg + dup Wu + dz_x Wx + dz_y Wy  (+ the experts' d(x)) as one sum in fp32
-// At 4096 tokens x 1024 x 4096 with 64 keys a half, bf16: 58 + 105 + 76 us of kernels (traced) where the library's nine products, the element-wise SwiGLU
+// At 4096 tokens x 1024 x 4096 with 64 keys a half, bf16: 57 + 101 + 76 us of kernels (traced) where the library's nine products, the element-wise SwiGLU
 // kernel and the additions took 350.
 #include "common.h"
 #include "gemm_tiles.h"
