@@ -7,7 +7,7 @@
 //   1. the router's projection | gate and up with their SwiGLU product
 //   2. the router's selection  | the down projection, K split over the grid, as fp32 partial sums
 //   3. the experts, the partial sums and the final add, one block per token.
-// 1 token 38.4 -> 19.5 us a call (kernels 6.5 + 6.7 + 4.3), 48 tokens 42.9 -> 24.0 us (10.8 + 8.4 + 5.3), hidden 1024 x intermediate 4096.
+// 1 token 38.4 -> 18.1 us a call (kernels 6.5 + 5.0 + 4.6), 48 tokens 42.9 -> 21.9 us (9.4 + 6.6 + 5.4), hidden 1024 x intermediate 4096.
 //
 // Projections.  There is one row tile, so every weight is used once and nothing is gained by staging it through LDS: a lane loads
 // its matrix fragments (8 consecutive K values of a row) straight from memory, all loads of 1024 K values of a block in flight at once.
@@ -40,13 +40,13 @@ template <int DT> __device__ __forceinline__ uint32_t pack2(float lo, float hi) 
 }
 
 // acc[j][i]: rows 16 i + lane % 16 of `a` ([rows of row_bytes], a_bytes in all, K values a row; TM row tiles, zeros past the matrix) times the 16
-// rows of weight tile j, columns 4 (lane / 16) .. + 3, over the K units u0 + wave, u0 + wave + 8, .. below u1, two at a time.
-// Weights: this lane's row b0 or b1, straight into registers, two units ahead.  Activations: every block reads all of them, from L2, and reads of
+// rows of weight tile j, columns 4 (lane / 16) .. + 3, over the K units u0 + wave, u0 + wave + 8, .. below u1, Q at a time.
+// Weights: this lane's row b0 or b1, straight into registers, Q units ahead.  Activations: every block reads all of them, from L2, and reads of
 // 64 bytes from each of 16 rows -- what a fragment is -- are slow there (64 tokens, hidden 1024: 15.4 us for launch 1, 10.1 us when an
-// instruction reads 1 KiB on end); so they take whole 128-byte lines of 8 rows into the wave's own `lds` (TM * 4 KiB; position c of row r
+// instruction reads 1 KiB on end); so they take whole 128-byte lines of 8 rows into the wave's own `lds` (Q * TM * 2 KiB; position c of row r
 // holds the row's 16-byte piece c ^ (r / 2 % 8), which keeps the fragment reads free of bank conflicts).
 // kTail: K is no multiple of 64 (but of 8); what is past it reads as zero on both sides.
-template <int DT, int TM, bool kTail>
+template <int DT, int TM, int Q, bool kTail>
 __device__ __forceinline__ void multiply(f32x4_t (&acc)[2][TM], const uint8_t* a, int row_bytes, int a_bytes, const uint8_t* b0, const uint8_t* b1, int K, int u0, int u1,
                                          int wave, int lane, uint32_t lds) {
   const int r16 = lane & 15, g4 = lane >> 4;
@@ -55,10 +55,10 @@ __device__ __forceinline__ void multiply(f32x4_t (&acc)[2][TM], const uint8_t* a
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < TM; ++i) acc[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  u32x4_t b[2][2][2];                                          // [unit][half of it][weight tile]
+  u32x4_t b[Q][2][2];                                          // [unit][half of it][weight tile]
   auto load_weights = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < Q; ++q) {
       const int v = u + q * kFewWaves;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
@@ -71,7 +71,7 @@ __device__ __forceinline__ void multiply(f32x4_t (&acc)[2][TM], const uint8_t* a
   };
   const uint32_t row = (uint32_t)(lane >> 3), from = row * (uint32_t)row_bytes;
   load_weights(u0 + wave);
-  for (int u = u0 + wave; u < u1; u += 2 * kFewWaves) {
+  for (int u = u0 + wave; u < u1; u += Q * kFewWaves) {
     auto load_rows = [&](auto n_tag) __attribute__((always_inline)) {
       constexpr int n = decltype(n_tag)::value, q = n / (2 * TM), part = n % (2 * TM);
       // rows 8 part + lane / 8: r / 2 % 8 = 4 (part % 2) + lane / 16
@@ -80,19 +80,19 @@ __device__ __forceinline__ void multiply(f32x4_t (&acc)[2][TM], const uint8_t* a
       load_to_lds<n * 1024>((uint64_t)a, a_bytes, lds, inside ? from + (uint32_t)(part * 8 * row_bytes + k * 2) : 0x80000000u, 0);
     };
     auto load_all = [&](auto... n) __attribute__((always_inline)) { (load_rows(n), ...); };
-    with_sequence(load_all, std::make_integer_sequence<int, 4 * TM>{});
+    with_sequence(load_all, std::make_integer_sequence<int, 2 * Q * TM>{});
     vmcnt<0>();
     __builtin_amdgcn_sched_barrier(0);
-    u32x4_t w[2][2][2];
+    u32x4_t w[Q][2][2];
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < Q; ++q)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
         for (int j = 0; j < 2; ++j) w[q][ks][j] = b[q][ks][j];
-    if (u + 2 * kFewWaves < u1) load_weights(u + 2 * kFewWaves);
+    if (u + Q * kFewWaves < u1) load_weights(u + Q * kFewWaves);
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < Q; ++q)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -105,22 +105,22 @@ __device__ __forceinline__ void multiply(f32x4_t (&acc)[2][TM], const uint8_t* a
   }
 }
 
-// The block's eight sums meet in LDS, each in its wave's own TM * 4 KiB
-template <int TM>
+// The block's eight sums meet in LDS, each at the start of its wave's own Q * TM * 2 KiB
+template <int TM, int Q>
 __device__ __forceinline__ void publish(uint8_t* lds, const f32x4_t (&acc)[2][TM], int wave, int lane) {
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int i = 0; i < TM; ++i) *(f32x4_t*)(lds + wave * TM * 4096 + ((j * TM + i) * kWave + lane) * 16) = acc[j][i];
+    for (int i = 0; i < TM; ++i) *(f32x4_t*)(lds + wave * Q * TM * 2048 + ((j * TM + i) * kWave + lane) * 16) = acc[j][i];
   __syncthreads();
 }
 // columns 4 quad .. + 3 of row `row` of weight tile j, all waves
-template <int TM>
+template <int TM, int Q>
 __device__ __forceinline__ f32x4_t gathered(const uint8_t* lds, int j, int row, int quad) {
   f32x4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int w = 0; w < kFewWaves; ++w) {
-    const f32x4_t o = *(const f32x4_t*)(lds + w * TM * 4096 + ((j * TM + row / 16) * kWave + quad * 16 + row % 16) * 16);
+    const f32x4_t o = *(const f32x4_t*)(lds + w * Q * TM * 2048 + ((j * TM + row / 16) * kWave + quad * 16 + row % 16) * 16);
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] += o[q];
   }
@@ -134,21 +134,21 @@ struct FrontArgs {
 };
 
 // Launch 1: blocks below router_blocks project 16 keys of each half, the others 16 columns of gate and of up.
-template <int DT, int TM, bool kTail>
-__global__ __launch_bounds__(kFewThreads, 2) void few_front_kernel(const FrontArgs g) {
-  extern __shared__ __align__(16) uint8_t lds[];               // TM * 4 KiB a wave
+template <int DT, int TM, int Q, bool kTail>
+__global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_front_kernel(const FrontArgs g) {
+  extern __shared__ __align__(16) uint8_t lds[];               // Q * TM * 2 KiB a wave
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15;
-  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * TM * 4096;
+  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * Q * TM * 2048;
   const bool router = (int)blockIdx.x < g.router_blocks;
   const int n0 = (router ? (int)blockIdx.x : (int)blockIdx.x - g.router_blocks) * 16, rows = router ? g.r : g.I;
   const int64_t row_bytes = (int64_t)g.H * 2, b_at = min(n0 + r16, rows - 1) * row_bytes;
   f32x4_t acc[2][TM];
-  multiply<DT, TM, kTail>(acc, g.x, g.H * 2, g.T * g.H * 2, (router ? g.wx : g.wg) + b_at, (router ? g.wy : g.wu) + b_at, g.H, 0, (g.H + kUnit - 1) / kUnit, wave, lane, mine);
-  publish<TM>(lds, acc, wave, lane);
+  multiply<DT, TM, Q, kTail>(acc, g.x, g.H * 2, g.T * g.H * 2, (router ? g.wx : g.wg) + b_at, (router ? g.wy : g.wu) + b_at, g.H, 0, (g.H + kUnit - 1) / kUnit, wave, lane, mine);
+  publish<TM, Q>(lds, acc, wave, lane);
   for (int i = threadIdx.x; i < TM * 64; i += kFewThreads) {
     const int row = i >> 2, quad = i & 3, n = n0 + quad * 4;
     if (row >= g.T || n >= rows) continue;
-    const f32x4_t p = gathered<TM>(lds, 0, row, quad), q = gathered<TM>(lds, 1, row, quad);
+    const f32x4_t p = gathered<TM, Q>(lds, 0, row, quad), q = gathered<TM, Q>(lds, 1, row, quad);
     if (router) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -175,11 +175,11 @@ struct MiddleArgs {
 };
 
 // Launch 2: blocks below select_blocks select for eight tokens each, the others multiply 32 output columns over one of the K splits.
-template <int DT, int TM, bool kTail, bool kSelect, int C>
-__global__ __launch_bounds__(kFewThreads, 2) void few_middle_kernel(const MiddleArgs g) {
-  extern __shared__ __align__(16) uint8_t lds[];               // TM * 4 KiB a wave
+template <int DT, int TM, int Q, bool kTail, bool kSelect, int C>
+__global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel(const MiddleArgs g) {
+  extern __shared__ __align__(16) uint8_t lds[];               // Q * TM * 2 KiB a wave
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15;
-  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * TM * 4096;
+  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * Q * TM * 2048;
   if constexpr (kSelect) {
     if ((int)blockIdx.x < g.select_blocks) {
       const int first = (int)blockIdx.x * kFewWaves + wave, all = g.select_blocks * kFewWaves;
@@ -193,12 +193,12 @@ __global__ __launch_bounds__(kFewThreads, 2) void few_middle_kernel(const Middle
   const int block = (int)blockIdx.x - (kSelect ? g.select_blocks : 0), split = block / g.groups, n0 = (block - split * g.groups) * 32;
   const int64_t row_bytes = (int64_t)g.I * 2;
   f32x4_t acc[2][TM];
-  multiply<DT, TM, kTail>(acc, g.h, g.I * 2, g.T * g.I * 2, g.wd + min(n0 + r16, g.H - 1) * row_bytes, g.wd + min(n0 + 16 + r16, g.H - 1) * row_bytes, g.I, split * g.units,
+  multiply<DT, TM, Q, kTail>(acc, g.h, g.I * 2, g.T * g.I * 2, g.wd + min(n0 + r16, g.H - 1) * row_bytes, g.wd + min(n0 + 16 + r16, g.H - 1) * row_bytes, g.I, split * g.units,
                           min((split + 1) * g.units, (g.I + kUnit - 1) / kUnit), wave, lane, mine);
-  publish<TM>(lds, acc, wave, lane);
+  publish<TM, Q>(lds, acc, wave, lane);
   for (int i = threadIdx.x; i < TM * 128; i += kFewThreads) {
     const int row = i >> 3, quad = i & 7, n = n0 + quad * 4;
-    if (row < g.T && n < g.H) *(f32x4_t*)(g.parts + ((int64_t)split * g.T + row) * g.H + n) = gathered<TM>(lds, quad >> 2, row, quad & 3);
+    if (row < g.T && n < g.H) *(f32x4_t*)(g.parts + ((int64_t)split * g.T + row) * g.H + n) = gathered<TM, Q>(lds, quad >> 2, row, quad & 3);
   }
 }
 
@@ -350,9 +350,21 @@ hipError_t launch(const FewTokens& f, hipStream_t s) {
   const int r = f.select.r;
   const FrontArgs a{(const uint8_t*)f.x, (const uint8_t*)f.wg, (const uint8_t*)f.wu, (const uint8_t*)f.wx, (const uint8_t*)f.wy, (uint8_t*)f.h, (uint8_t*)f.z,
                     f.T, f.H, f.I, r, layer ? (r + 15) / 16 : 0};
-  constexpr int kBytes = kFewWaves * TM * 4096;
   const int64_t front = a.router_blocks + (f.I + 15) / 16;
-  hipError_t e = f.H % kUnit ? start<few_front_kernel<DT, TM, true>, kBytes>(a, front, s) : start<few_front_kernel<DT, TM, false>, kBytes>(a, front, s);
+  // From 33 tokens on, two K units of a wave in LDS at once are more than half of a CU's: one block to a CU, and blocks beyond 256 wait for a whole round.
+  // One unit at a time then (in turn over three sets of inputs, hidden 1024 x intermediate 4096: 33 tokens 23.5 -> 21.3 us, 48 24.1 -> 21.9, 64 26.2 -> 22.9;
+  // 48 tokens, 2048 x 8192 49.9 -> 43.9).  Where the first launch has no more blocks than CUs both units stay in flight.
+  constexpr bool kWide = TM >= 3;
+  auto units_at_once = [&](bool one, auto&& go) -> hipError_t {
+    if constexpr (kWide) {
+      if (one) return go(std::integral_constant<int, 1>{});
+    }
+    return go(std::integral_constant<int, 2>{});
+  };
+  hipError_t e = units_at_once(front > 256, [&](auto q) -> hipError_t {
+    constexpr int Q = decltype(q)::value, kBytes = kFewWaves * Q * TM * 2048;
+    return f.H % kUnit ? start<few_front_kernel<DT, TM, Q, true>, kBytes>(a, front, s) : start<few_front_kernel<DT, TM, Q, false>, kBytes>(a, front, s);
+  });
   if (e != hipSuccess) return e;
 
   const int units = (f.I + kUnit - 1) / kUnit;
@@ -362,13 +374,17 @@ hipError_t launch(const FewTokens& f, hipStream_t s) {
   splits = (units + m.units - 1) / m.units;                    // every split has work
   const int cells = prepare_select(m.select);
   const int64_t middle = m.select_blocks + (int64_t)m.groups * splits;
-  auto go = [&](auto tail) -> hipError_t {
-    constexpr bool kTail = decltype(tail)::value;
-    if (!layer) return start<few_middle_kernel<DT, TM, kTail, false, 1>, kBytes>(m, middle, s);
-    if (cells <= 1) return start<few_middle_kernel<DT, TM, kTail, true, 1>, kBytes>(m, middle, s);
-    return start<few_middle_kernel<DT, TM, kTail, true, 2>, kBytes>(m, middle, s);
-  };
-  if ((e = f.I % kUnit ? go(std::true_type{}) : go(std::false_type{})) != hipSuccess) return e;
+  e = units_at_once(middle > 256 || m.units <= kFewWaves, [&](auto q) -> hipError_t {           // (a wave may have one unit only)
+    constexpr int Q = decltype(q)::value, kBytes = kFewWaves * Q * TM * 2048;
+    auto go = [&](auto tail) -> hipError_t {
+      constexpr bool kTail = decltype(tail)::value;
+      if (!layer) return start<few_middle_kernel<DT, TM, Q, kTail, false, 1>, kBytes>(m, middle, s);
+      if (cells <= 1) return start<few_middle_kernel<DT, TM, Q, kTail, true, 1>, kBytes>(m, middle, s);
+      return start<few_middle_kernel<DT, TM, Q, kTail, true, 2>, kBytes>(m, middle, s);
+    };
+    return f.I % kUnit ? go(std::true_type{}) : go(std::false_type{});
+  });
+  if (e != hipSuccess) return e;
 
   const BackArgs b{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, (const uint8_t*)f.residual, f.select.gates, f.select.indices, f.parts, (uint8_t*)f.y,
                    f.T, f.H, f.select.k, splits, (uint32_t)f.N};

@@ -649,7 +649,9 @@ def test_layer_tiny_token_counts(T, training, aligned, device):
 # T, H, I, N, k: tiles of 16 rows and their remainders; hidden and intermediate sizes that end inside a block's 64 of K or 16 columns, or
 # split K eight ways; 1 to 8 keys per lane, an odd key count, more than 64 candidates, ids beyond the square never chosen
 FEW_TOKEN_CASES = [(1, 1024, 4096, 4096, 16), (16, 200, 312, 1000, 8), (17, 1032, 2056, 700, 32), (33, 256, 1024, 90000, 18), (48, 2048, 1024, 17000, 4),
-                   (49, 4096, 512, 260, 2), (63, 584, 8, 289, 6), (64, 8, 4096, 300000, 32)]
+                   (49, 4096, 512, 260, 2), (63, 584, 8, 289, 6), (64, 8, 4096, 300000, 32),
+                   # more than 256 blocks in the first launch (one K unit in LDS at a time) and just not, in the second (splits of one unit a wave or of several)
+                   (33, 1024, 4104, 4096, 16), (48, 1032, 4032, 256, 8), (48, 1032, 4048, 256, 8), (64, 2048, 8200, 1000, 4)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
