@@ -748,14 +748,17 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_ksplit_kernel(const Gemm
 // What bounds it: v_mfma_f32_32x32x2 takes 64 cycles, so a CU that has a 128 x 128 tile to itself works 4096 cycles on 32 of K, and a launch
 // of 32 or 64 such tiles leaves the chip idle (512 tokens, hidden 256 x intermediate 1024: gate/up 22.4 us, down projection 26.8 us on 64 x 64
 // tiles, for 4 and 2 us of matrix instructions).  Here a block has 32 x 32 of the output (SwiGLU: of gate and of up) and its four waves deal
-// out the K tiles (32 values, 128-byte rows) as in gemm_ksplit_kernel: a two-stage ring in LDS per wave, no block barrier, the four sums added in
+// out the K tiles (32 values, 128-byte rows) as in gemm_ksplit_kernel: a ring in LDS per wave, no block barrier, the four sums added in
 // wave order: 12.4 and 9.1 us.  Twice the operand traffic of a 64 x 64 tile (32 bytes per cycle and CU), which L2 still carries.
-template <int EPI>
+// NS: ring stages.  A K tile's fragments are all read before its matrix instructions, so one stage still has the next tile's loads in flight during them; two
+// start a block faster but take 96 KiB (SwiGLU; else 64), one block to a CU: one where the launch has more blocks than fit the CUs that way
+// (the layer at 512 x 256 x 1024 29.8 -> 25.9 us, 1000 x 256 x 1024 43.3 -> 38.2, 300 x 1024 x 4096 116 -> 106; the MLP at 512 x 256 x 1024 17.8 -> 16.0).
+template <int EPI, int NS>
 __device__ __forceinline__ void gemm_f32_small_block(const GemmArgs& g, const int block, uint8_t* lds) {
   constexpr int TB = EPI == kEpiSwiglu ? 2 : 1, kTile = 32 * 128, kStage = (1 + TB) * kTile, kLoads = 4 * (1 + TB);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m0 = block % g.tiles_m * 32, n0 = block / g.tiles_m * 32;
-  const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * 2 * kStage;
+  const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * NS * kStage;
   const int row_bytes = g.K * 4;
   const uint64_t a = (uint64_t)g.a + (uint64_t)m0 * (uint32_t)row_bytes;
   const int a_bytes = min(32, g.M - m0) * row_bytes, b_bytes = min(32, g.N - n0) * row_bytes;    // rows past the matrix read as zero
@@ -781,10 +784,10 @@ __device__ __forceinline__ void gemm_f32_small_block(const GemmArgs& g, const in
 
   const int rl = lane & 31, num_kt = (g.K + 31) / 32, mine = (num_kt - wave + 3) / 4;
   if (mine > 0) issue(wave, 0);
-  if (mine > 1) issue(wave + 4, 1);
+  if (NS == 2 && mine > 1) issue(wave + 4, 1);
   for (int t = 0; t < mine; ++t) {
-    if (t + 1 < mine) wait_vmcnt<kLoads>(); else wait_vmcnt<0>();
-    const uint32_t st = ring + (uint32_t)((t & 1) * kStage + rl * 128);
+    if (NS == 2 && t + 1 < mine) wait_vmcnt<kLoads>(); else wait_vmcnt<0>();
+    const uint32_t st = ring + (uint32_t)(t % NS * kStage + rl * 128);
     using Frag = const __attribute__((address_space(3))) u32x4_t*;
     u32x4_t af[4], bf[4][TB];
 #pragma unroll
@@ -794,9 +797,9 @@ __device__ __forceinline__ void gemm_f32_small_block(const GemmArgs& g, const in
 #pragma unroll
       for (int j = 0; j < TB; ++j) bf[sl][j] = *(Frag)(uintptr_t)(at + (1 + j) * kTile);
     }
-    if (t + 2 < mine) {
+    if (t + NS < mine) {
       wait_lds_reads();                                  // the stage is read out (by this wave, its only reader)
-      issue(wave + 4 * (t + 2), t & 1);
+      issue(wave + 4 * (t + NS), t % NS);
     }
 #pragma unroll
     for (int sl = 0; sl < 4; ++sl)
@@ -828,27 +831,27 @@ __device__ __forceinline__ void gemm_f32_small_block(const GemmArgs& g, const in
     }
   gemm_epilogue<kF32, 1, TB, EPI>(g, sum, m0, n0, 0, 0, lane);
 }
-template <int EPI>
+template <int EPI, int NS>
 __global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_small_kernel(const GemmArgs g) {
   extern __shared__ __align__(16) uint8_t lds[];
-  gemm_f32_small_block<EPI>(g, (int)blockIdx.x, lds);
+  gemm_f32_small_block<EPI, NS>(g, (int)blockIdx.x, lds);
 }
 
 // A layer of such products in single precision: stages that do not depend on each other share a launch, as in 16 bits (gemm_tiles.hip).  Six dependent launches
 // of 4 to 12 us are four: projection | gate/up (the projection's blocks first: half as long), then selection | down projection.
 struct F32Front { GemmArgs router, mlp; int router_blocks; };
-template <int EPI>                    // of the projection: kEpiStats or kEpiPlain
+template <int EPI, int NS>            // of the projection: kEpiStats or kEpiPlain
 __global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_front_kernel(const F32Front g) {
   extern __shared__ __align__(16) uint8_t lds[];
-  if ((int)blockIdx.x < g.router_blocks) gemm_f32_small_block<EPI>(g.router, (int)blockIdx.x, lds);
-  else gemm_f32_small_block<kEpiSwiglu>(g.mlp, (int)blockIdx.x - g.router_blocks, lds);
+  if ((int)blockIdx.x < g.router_blocks) gemm_f32_small_block<EPI, NS>(g.router, (int)blockIdx.x, lds);
+  else gemm_f32_small_block<kEpiSwiglu, NS>(g.mlp, (int)blockIdx.x - g.router_blocks, lds);
 }
 struct F32Down { GemmArgs down; SelectArgs select; int select_blocks; };
 template <int R, int C>
 __global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_select_kernel(const F32Down g) {
   extern __shared__ __align__(16) uint8_t lds[];
   if ((int)blockIdx.x >= g.select_blocks) {
-    gemm_f32_small_block<kEpiPlain>(g.down, (int)blockIdx.x - g.select_blocks, lds);
+    gemm_f32_small_block<kEpiPlain, 2>(g.down, (int)blockIdx.x - g.select_blocks, lds);
     return;
   }
   const float* stats = g.select.stats;
@@ -871,10 +874,10 @@ template <int DT, int EPI, int TM>
 struct KsplitKernelLds {
   static inline LdsKernel entry{(const void*)gemm_ksplit_kernel<DT, EPI, TM>, ksplit_lds(TM)};
 };
-template <int EPI>
+template <int EPI, int NS>
 struct SmallF32Lds {
-  static constexpr int kBytes = 4 * 2 * (EPI == kEpiSwiglu ? 3 : 2) * 32 * 128;
-  static inline LdsKernel entry{(const void*)gemm_f32_small_kernel<EPI>, kBytes};
+  static constexpr int kBytes = 4 * NS * (EPI == kEpiSwiglu ? 3 : 2) * 32 * 128;
+  static inline LdsKernel entry{(const void*)gemm_f32_small_kernel<EPI, NS>, kBytes};
 };
 template <auto kKernel, int kBytes>
 struct F32JointLds { static inline LdsKernel entry{(const void*)kKernel, kBytes}; };
@@ -965,9 +968,15 @@ static hipError_t launch_gemm(GemmArgs g, hipStream_t s, bool exclusive = false)
   if constexpr (DT == kF32 && EPI != kEpiGate) {
     GemmArgs d = g;
     if (const int64_t small = f32_small_blocks<TM, TN, EPI>(d); small && aligned) {
-      if (hipError_t e = SmallF32Lds<EPI>::entry.ensure(); e != hipSuccess) return e;
-      hipLaunchKernelGGL((gemm_f32_small_kernel<EPI>), dim3((unsigned)small), dim3(kGemmThreads), SmallF32Lds<EPI>::kBytes, s, d);
-      return hipGetLastError();
+      auto go = [&](auto ns) -> hipError_t {
+        constexpr int NS = decltype(ns)::value;
+        using L = SmallF32Lds<EPI, NS>;
+        if (hipError_t e = L::entry.ensure(); e != hipSuccess) return e;
+        hipLaunchKernelGGL((gemm_f32_small_kernel<EPI, NS>), dim3((unsigned)small), dim3(kGemmThreads), L::kBytes, s, d);
+        return hipGetLastError();
+      };
+      if (small > (EPI == kEpiSwiglu ? 256 : 512)) return go(std::integral_constant<int, 1>{});
+      return go(std::integral_constant<int, 2>{});
     }
   }
   auto kern = gemm_nt_kernel<DT, TM, TN, EPI>;       // any K % 8 == 0, any address: staged through registers
@@ -1108,15 +1117,20 @@ bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, co
   const int64_t rb = f32_small_blocks_of<kEpiPlain>(router), mb = f32_small_blocks_of<kEpiSwiglu>(mlp), db = f32_small_blocks_of<kEpiPlain>(d.down);
   if (!rb || !mb || !db || regs > 4 || cells > 2) return false;
   const F32Front f{router, mlp, (int)rb};
-  constexpr int kFront = SmallF32Lds<kEpiSwiglu>::kBytes, kDown = SmallF32Lds<kEpiPlain>::kBytes;
+  constexpr int kDown = SmallF32Lds<kEpiPlain, 2>::kBytes;
   static_assert(kDown >= 4 * merge_lds_floats(kMergeKeys, kGemmThreads), "a block that selects merges statistics there");
   auto start = [&](auto kernel, LdsKernel& entry, int bytes, int64_t blocks, const auto& a) {
     if ((*e = entry.ensure()) != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kGemmThreads), bytes, s, a);
     *e = hipGetLastError();
   };
-  if (statistics) start(gemm_f32_front_kernel<kEpiStats>, F32JointLds<gemm_f32_front_kernel<kEpiStats>, kFront>::entry, kFront, rb + mb, f);
-  else start(gemm_f32_front_kernel<kEpiPlain>, F32JointLds<gemm_f32_front_kernel<kEpiPlain>, kFront>::entry, kFront, rb + mb, f);
+  auto front = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value, kFront = SmallF32Lds<kEpiSwiglu, NS>::kBytes;
+    if (statistics) start(gemm_f32_front_kernel<kEpiStats, NS>, F32JointLds<gemm_f32_front_kernel<kEpiStats, NS>, kFront>::entry, kFront, rb + mb, f);
+    else start(gemm_f32_front_kernel<kEpiPlain, NS>, F32JointLds<gemm_f32_front_kernel<kEpiPlain, NS>, kFront>::entry, kFront, rb + mb, f);
+  };
+  if (rb + mb > 256) front(std::integral_constant<int, 1>{});
+  else front(std::integral_constant<int, 2>{});
   if (*e != hipSuccess) return true;
   constexpr int kWaves = kGemmThreads / kWave;
   d.select_blocks = (int)((T + kWaves - 1) / kWaves < 1024 ? (T + kWaves - 1) / kWaves : 1024);

@@ -699,7 +699,9 @@ def test_few_tokens_match_the_operators(case, dtype, device):
 
 
 # T, H, I: 32-row and 32-column tiles and their remainders, K of one to five tiles of 32 and with a remainder, more and fewer waves than K tiles
-@pytest.mark.parametrize("case", [(1, 4, 4), (33, 36, 100), (512, 256, 1024), (100, 1028, 68), (640, 160, 96), (65, 128, 132)], ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}")
+@pytest.mark.parametrize("case", [(1, 4, 4), (33, 36, 100), (512, 256, 1024), (100, 1028, 68), (640, 160, 96), (65, 128, 132),
+                   # 256 and 288 blocks of the SwiGLU product (two ring stages, one), 512 and 544 of the down projection
+                   (256, 160, 1024), (257, 160, 1024), (257, 32, 1024), (512, 1024, 544), (513, 1024, 544)], ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}")
 def test_small_fp32_products_match_fp64(case, device):
     """Single precision with few output tiles: the MLP (SwiGLU and residual epilogues) and the router projection's column statistics against 64
     bits.  Tolerance: sums of K products in 32 bits, sqrt(K) * 2^-24 of the terms' size each, times 8."""
