@@ -176,7 +176,8 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave, 2) void expert_gather_kerne
 //   two batches   hidden 256 k 32, 1024 k 16, 2048 k 8:   2: 0.64-0.72 / 0.64-0.74 / 0.81-0.95 / 0.81-0.94 / 0.8-1.03   4: 0.6-0.7 / 0.72-0.82 / 0.86-1.09 / 1.04-1.08
 //   four and more hidden 1024 k 32, 2048 k 16 and 32, 4096: 2: 0.60-0.66 / 0.74-0.84 / 0.83-0.97 / 0.88-1.03 / 1.0   4: 0.40-0.58 / 0.63-0.84 / 0.78-1.0 / 0.87-1.08 / 1.0
 //   one batch: 1.0-1.25 and 1.0-1.8
-// Not where the gather algorithm is asked for by name: its sums are those of the segment algorithm, slot by slot.
+// Only where AUTO leads here (`shared` of the launches).  Asked for by name the gather algorithm's sums are those of the segment algorithm, slot by slot, and
+// so they are where the layer ends with this kernel.
 static inline int gather_waves(int64_t T, int k, int batch) {
   const int batches = (k + batch - 1) / batch;
   return batches < 2 || T > 1024 ? 1 : batches >= 4 && T <= 512 ? 4 : 2;
@@ -199,8 +200,8 @@ static hipError_t launch_gather(const void* x, const void* up, const void* down,
 }
 
 // The gather algorithm (rows of at most 8 KiB) with the layer's final add
-hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, int64_t T, int H,
-                             int k, int64_t N, int dtype, hipStream_t s) {
+hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, bool shared, int64_t T,
+                             int H, int k, int64_t N, int dtype, hipStream_t s) {
   auto launch = [&](auto dt, auto nch, auto batch, auto waves) {
     constexpr int W = decltype(waves)::value, kTokens = kTokensPerBlock / W;
     hipLaunchKernelGGL((expert_gather_kernel<decltype(dt)::value, decltype(nch)::value, decltype(batch)::value, true, W>), dim3((unsigned)((T + kTokens - 1) / kTokens)),
@@ -209,7 +210,7 @@ hipError_t launch_gather_add(const void* x, const void* up, const void* down, co
     return hipGetLastError();
   };
   auto go = [&](auto dt, auto nch, auto batch) {
-    switch (gather_waves(T, k, decltype(batch)::value)) {
+    switch (shared ? gather_waves(T, k, decltype(batch)::value) : 1) {
       case 4: return launch(dt, nch, batch, std::integral_constant<int, 4>{});
       case 2: return launch(dt, nch, batch, std::integral_constant<int, 2>{});
       default: return launch(dt, nch, batch, std::integral_constant<int, 1>{});

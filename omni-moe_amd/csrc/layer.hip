@@ -29,9 +29,9 @@ int router_fwd(const void* x, const void* weight_x, const void* weight_y,
                void* scores, int64_t num_tokens, int32_t hidden_size, int32_t num_expert_sqrt,
                int32_t num_experts_per_token, int32_t dtype, int32_t stats_dtype,
                void* workspace, void* stream, bool exclusive);
-// defined beside the expert kernels: the gather algorithm with the final add
-hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, int64_t T, int H,
-                             int k, int64_t N, int dtype, hipStream_t s);
+// defined beside the expert kernels: the gather algorithm with the final add (shared: AUTO's, whose waves may share a token's slots)
+hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, bool shared, int64_t T,
+                             int H, int k, int64_t N, int dtype, hipStream_t s);
 // defined beside the GEMM kernels: a small single-precision layer up to the experts, as two launches
 bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, const void* wg, const void* wu, const void* wd, void* h, void* y, int64_t T, int64_t H, int64_t I,
                       const SelectArgs& args, bool statistics, hipStream_t s, hipError_t* e);
@@ -49,9 +49,10 @@ int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int3
 //   hidden 4096, top-4    51 / 67     55 / 70     87 / 92
 constexpr int kBlockPerToken = 256;
 // Projection | gate/up, selection | down projection, experts and add; where two stages do not fit one launch, each is its own.
-// statistics (training): projects z and leaves its column statistics, which f.select merges or reads.
+// shared: launch_gather_add's (a block per token always shares its slots).  statistics (training): projects z and leaves its column statistics, which f.select
+// merges or reads.
 template <class Statistics>
-static int joint_forward(const FewTokens& f, int dtype, size_t parts_bytes, hipStream_t s, bool training, Statistics&& statistics) {
+static int joint_forward(const FewTokens& f, int dtype, size_t parts_bytes, hipStream_t s, bool shared, bool training, Statistics&& statistics) {
   auto code = [](hipError_t e) { return e == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)e; };
   const int64_t H2 = (int64_t)f.H * 2, I2 = (int64_t)f.I * 2;
   TileProduct router, mlp, down;
@@ -81,7 +82,7 @@ static int joint_forward(const FewTokens& f, int dtype, size_t parts_bytes, hipS
   if (!selected)
     if (int e = launch_router_select(f.select, s)) return e;
   if (f.T <= kBlockPerToken) return code(launch_few_back(dtype, f, parts > 1 ? parts : 0, s));
-  return code(launch_gather_add(f.x, f.up, f.down, f.select.gates, f.select.indices, f.y, parts > 1 ? f.parts : nullptr, parts, f.T, f.H, f.select.k, f.N, dtype, s));
+  return code(launch_gather_add(f.x, f.up, f.down, f.select.gates, f.select.indices, f.y, parts > 1 ? f.parts : nullptr, parts, shared, f.T, f.H, f.select.k, f.N, dtype, s));
 }
 }  // namespace omni
 
@@ -204,19 +205,20 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
     g.gates = gates; g.indices = ids;
     g.num_tokens = (int)num_tokens; g.r = num_expert_sqrt; g.k = num_experts_per_token; g.dt = dtype;
     f.up = up_embed; f.down = down_embed; f.N = num_experts;
+    const bool shared = expert_algo == OMNI_EXPERT_ALGO_AUTO;
     if (few_tokens_aligned(f) && num_tokens <= INT32_MAX / 256) {
       if (dtype == OMNI_F32) {
         hipError_t he = hipSuccess;
         if (launch_f32_joint(x, router_weight_x, router_weight_y, router_ws, gate_weight, up_weight, down_weight, mlp_ws, y, num_tokens, hidden_size, intermediate_size, g, training != 0,
                              main_s, &he)) {
-          if (he == hipSuccess) he = launch_gather_add(x, up_embed, down_embed, gates, ids, y, nullptr, 0, num_tokens, hidden_size, num_experts_per_token, num_experts, dtype, main_s);
+          if (he == hipSuccess) he = launch_gather_add(x, up_embed, down_embed, gates, ids, y, nullptr, 0, shared, num_tokens, hidden_size, num_experts_per_token, num_experts, dtype, main_s);
           return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
         }
       } else if (few && !training) {
         const hipError_t he = launch_few_tokens(dtype, f, main_s);
         return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
       }
-      if (dtype != OMNI_F32) return joint_forward(f, dtype, omni_mlp_workspace_bytes(num_tokens, hidden_size, intermediate_size, dtype) - h_bytes, main_s, training != 0, [&]() -> int {
+      if (dtype != OMNI_F32) return joint_forward(f, dtype, omni_mlp_workspace_bytes(num_tokens, hidden_size, intermediate_size, dtype) - h_bytes, main_s, shared, training != 0, [&]() -> int {
         if (merge) return omni_gemm_router_projection(x, router_weight_x, router_weight_y, router_ws, part_mean, part_m2, num_tokens, hidden_size, num_expert_sqrt, dtype, main_s);
         // without a selection (k = 0) omni_router_fwd projects, merges the statistics, moves the running buffers and counts the batch
         return omni_router_fwd(x, router_weight_x, router_weight_y, running_mean_x, running_var_x, num_batches_tracked_x, running_mean_y, running_var_y,

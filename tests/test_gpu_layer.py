@@ -794,6 +794,32 @@ def test_layer_with_rows_beyond_the_tile_kernels_reach(device):
     assert (got - want).abs().max().item() <= 4 * 2.0 ** -7 * max(1.0, want.abs().max().item())
 
 
+# T, H, I, N, k
+GATHER_BY_NAME_CASES = [(300, 1024, 2048, 1024, 32), (1000, 512, 1024, 4096, 34), (512, 2048, 2048, 1024, 16), (257, 1024, 1024, 1024, 8)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("case", GATHER_BY_NAME_CASES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
+def test_layer_gather_by_name_is_the_operator(case, dtype, device):
+    """The gather algorithm by name adds a token's slots one after the other, in the joint launches' last kernel as in the operator.  An MLP of zeros leaves the
+    experts' rows alone in the output; batch statistics, where the joint launches choose the router stage's experts with its gates."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, H, I, N, k = case
+    print(f"gather by name {case} {dtype}", flush=True)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", N, k)).to(device=device, dtype=dtype)
+    layer.expert_algo = "gather"
+    g = torch.Generator(device=device).manual_seed(T)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, H ** -0.5, generator=g)
+        layer.down_proj.weight.zero_()
+        x = torch.randn(1, T, H, device=device, generator=g).to(dtype)
+        gates, ids = layer.route(x[0])
+        got = layer(x)[0]
+    want = _ops().hip_omni_expert_func(x[0], layer.up_embed.weight, layer.down_embed.weight, gates, ids, algo="gather")
+    assert torch.equal(got, want)
+
+
 # one strip, ragged strips, the most strips a block merges at 64 keys and one more, 8 to 128 keys; 136 keys: the merge's own launch
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
 @pytest.mark.parametrize("case", [(2, 8), (33, 64), (700, 104), (2048, 128), (4096, 64), (4100, 64), (300, 136)], ids=lambda c: "T%d-r%d" % c)
