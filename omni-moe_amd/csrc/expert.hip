@@ -242,6 +242,11 @@ static int expert_gather_dispatch(const void* x, const void* up, const void* dow
   return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
 }
 
+// The gather algorithm alone, for a layer whose schedules must agree on it
+int expert_gather_f32(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, bool shared, int64_t T, int H, int k, int64_t N, hipStream_t s) {
+  return expert_gather_dispatch<kF32>(x, up, down, gates, ids, y, T, H, k, N, s, nullptr, shared);
+}
+
 // ---- expert-centric variant -------------------------------------------------------------------
 constexpr int kPairsPerWave = 16;
 

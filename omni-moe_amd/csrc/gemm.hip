@@ -1099,11 +1099,19 @@ int omni_gemm_router_projection(const void* x, const void* wx, const void* wy, v
 }
 
 namespace omni {
+// Whether the three products of a single-precision layer are all of gemm_f32_small_kernel's kind and the selection fits beside them: from the sizes alone
+bool f32_joint_covers(int64_t T, int64_t H, int64_t I, int r, int k) {
+  if (check_gemm(T, I, H, 4) || check_gemm(T, H, I, 4) || check_gemm(T, 2 * (int64_t)r, H, 4) || r % 32) return false;       // (r: the halves' weights meet at a tile's border)
+  GemmArgs router{}, mlp{}, down{};
+  router.M = mlp.M = down.M = (int)T;
+  router.N = 2 * r; router.K = mlp.K = (int)H; mlp.N = down.K = (int)I; down.N = (int)H;
+  return r <= 4 * kWave && num_cells(k, r < k ? r : k) <= 2 * kWave && f32_small_blocks_of<kEpiPlain>(router) && f32_small_blocks_of<kEpiSwiglu>(mlp) &&
+         f32_small_blocks_of<kEpiPlain>(down);
+}
 // The layer's projection, gate/up, selection and down projection in single precision as two launches (see gemm_f32_front_kernel), y then holding the shared MLP's
-// rows; false, with nothing enqueued, where one of the products is not of the kind.  The operands are 16-byte aligned.
-bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, const void* wg, const void* wu, const void* wd, void* h, void* y, int64_t T, int64_t H, int64_t I,
-                      const SelectArgs& args, bool statistics, hipStream_t s, hipError_t* e) {
-  if (check_gemm(T, I, H, 4) || check_gemm(T, H, I, 4)) return false;
+// rows: sizes that f32_joint_covers takes, operands 16-byte aligned.
+hipError_t launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, const void* wg, const void* wu, const void* wd, void* h, void* y, int64_t T, int64_t H, int64_t I,
+                            const SelectArgs& args, bool statistics, hipStream_t s) {
   GemmArgs router{}, mlp{}, down{};
   router.a = mlp.a = (const uint8_t*)x;
   router.b0 = (const uint8_t*)wx; router.b1 = (const uint8_t*)wy; router.c = (uint8_t*)z;
@@ -1115,14 +1123,15 @@ bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, co
   F32Down d{down, args, 0};
   const int cells = prepare_select(d.select), regs = (args.r + kWave - 1) / kWave;
   const int64_t rb = f32_small_blocks_of<kEpiPlain>(router), mb = f32_small_blocks_of<kEpiSwiglu>(mlp), db = f32_small_blocks_of<kEpiPlain>(d.down);
-  if (!rb || !mb || !db || regs > 4 || cells > 2) return false;
+  if (!rb || !mb || !db || regs > 4 || cells > 2) return hipErrorInvalidValue;
+  hipError_t e = hipSuccess;
   const F32Front f{router, mlp, (int)rb};
   constexpr int kDown = SmallF32Lds<kEpiPlain, 2>::kBytes;
   static_assert(kDown >= 4 * merge_lds_floats(kMergeKeys, kGemmThreads), "a block that selects merges statistics there");
   auto start = [&](auto kernel, LdsKernel& entry, int bytes, int64_t blocks, const auto& a) {
-    if ((*e = entry.ensure()) != hipSuccess) return;
+    if ((e = entry.ensure()) != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kGemmThreads), bytes, s, a);
-    *e = hipGetLastError();
+    e = hipGetLastError();
   };
   auto front = [&](auto ns) {
     constexpr int NS = decltype(ns)::value, kFront = SmallF32Lds<kEpiSwiglu, NS>::kBytes;
@@ -1131,7 +1140,7 @@ bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, co
   };
   if (rb + mb > 256) front(std::integral_constant<int, 1>{});
   else front(std::integral_constant<int, 2>{});
-  if (*e != hipSuccess) return true;
+  if (e != hipSuccess) return e;
   constexpr int kWaves = kGemmThreads / kWave;
   d.select_blocks = (int)((T + kWaves - 1) / kWaves < 1024 ? (T + kWaves - 1) / kWaves : 1024);
   auto by_cells = [&](auto r_tag) {
@@ -1142,7 +1151,7 @@ bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, co
   if (regs <= 1) by_cells(std::integral_constant<int, 1>{});
   else if (regs <= 2) by_cells(std::integral_constant<int, 2>{});
   else by_cells(std::integral_constant<int, 4>{});
-  return true;
+  return e;
 }
 }  // namespace omni
 

@@ -32,9 +32,13 @@ int router_fwd(const void* x, const void* weight_x, const void* weight_y,
 // defined beside the expert kernels: the gather algorithm with the final add (shared: AUTO's, whose waves may share a token's slots)
 hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, bool shared, int64_t T,
                              int H, int k, int64_t N, int dtype, hipStream_t s);
-// defined beside the GEMM kernels: a small single-precision layer up to the experts, as two launches
-bool launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, const void* wg, const void* wu, const void* wd, void* h, void* y, int64_t T, int64_t H, int64_t I,
-                      const SelectArgs& args, bool statistics, hipStream_t s, hipError_t* e);
+// ... and alone
+int expert_gather_f32(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, bool shared, int64_t T, int H, int k, int64_t N,
+                      hipStream_t s);
+// defined beside the GEMM kernels: a small single-precision layer up to the experts, as two launches, and whether they cover its sizes
+bool f32_joint_covers(int64_t T, int64_t H, int64_t I, int r, int k);
+hipError_t launch_f32_joint(const void* x, const void* wx, const void* wy, void* z, const void* wg, const void* wu, const void* wd, void* h, void* y, int64_t T, int64_t H, int64_t I,
+                            const SelectArgs& args, bool statistics, hipStream_t s);
 // defined beside the GEMM kernels: the two projections of omni_mlp_fwd with the caller's word on whether the launch has the GPU to itself
 // (then a GEMM of more tiles than CUs may take the form that holds every CU until it ends); h lies at the workspace's start
 int mlp_gate_up_impl(const void* x, const void* wg, const void* wu, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive);
@@ -172,12 +176,15 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   const bool joint = dtype != OMNI_F32 && num_experts_per_token > 0 && num_expert_sqrt % 8 == 0 && hidden_size % 8 == 0 && intermediate_size % 8 == 0 &&
                      intermediate_size <= (1 << 20) && (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0;
   // (batch statistics: the projection and their merge stay launches of their own; a cumulative average, momentum < 0, is counted by the select kernel)
-  //   * single precision where every product has few output tiles (launch_f32_joint): the same bound; the general path gives the same bits, so a side
-  //     stream that is given is used
-  const bool joint_f32 = dtype == OMNI_F32 && !side_stream && num_experts_per_token > 0 && (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0 &&
-                         (!training || (momentum >= 0.f && merge_here(num_tokens, num_expert_sqrt)));
-  if ((joint_f32 || (training ? joint && momentum >= 0.f : few || joint)) && num_experts <= UINT32_MAX &&
-      joint_launches_gather(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype)) {
+  //   * single precision where every product has few output tiles (f32_joint_covers): the same bound.  A side stream that is given is used, and the two
+  //     schedules give the same bits: the sizes alone say how the experts' sums run, on either.
+  const bool gathers = joint_launches_gather(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) && num_experts <= UINT32_MAX;
+  const bool shared = expert_algo == OMNI_EXPERT_ALGO_AUTO;
+  const bool f32_sizes = dtype == OMNI_F32 && gathers && num_experts_per_token > 0 && (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0 &&
+                         num_tokens <= INT32_MAX / 256 && (!training || (momentum >= 0.f && merge_here(num_tokens, num_expert_sqrt))) &&
+                         f32_joint_covers(num_tokens, hidden_size, intermediate_size, num_expert_sqrt, num_experts_per_token);
+  const bool joint_f32 = f32_sizes && !side_stream;
+  if (joint_f32 || (gathers && (training ? joint && momentum >= 0.f : few || joint))) {
     if (stats_dtype != OMNI_BF16 && stats_dtype != OMNI_F16 && stats_dtype != OMNI_F32) return OMNI_ERR_DTYPE;
     if (!gate_weight || !up_weight || !down_weight || !router_weight_x || !router_weight_y || !running_mean_x || !running_var_x || !running_mean_y || !running_var_y)
       return OMNI_ERR_NULL;
@@ -205,20 +212,17 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
     g.gates = gates; g.indices = ids;
     g.num_tokens = (int)num_tokens; g.r = num_expert_sqrt; g.k = num_experts_per_token; g.dt = dtype;
     f.up = up_embed; f.down = down_embed; f.N = num_experts;
-    const bool shared = expert_algo == OMNI_EXPERT_ALGO_AUTO;
     if (few_tokens_aligned(f) && num_tokens <= INT32_MAX / 256) {
       if (dtype == OMNI_F32) {
-        hipError_t he = hipSuccess;
-        if (launch_f32_joint(x, router_weight_x, router_weight_y, router_ws, gate_weight, up_weight, down_weight, mlp_ws, y, num_tokens, hidden_size, intermediate_size, g, training != 0,
-                             main_s, &he)) {
-          if (he == hipSuccess) he = launch_gather_add(x, up_embed, down_embed, gates, ids, y, nullptr, 0, shared, num_tokens, hidden_size, num_experts_per_token, num_experts, dtype, main_s);
-          return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
-        }
+        hipError_t he = launch_f32_joint(x, router_weight_x, router_weight_y, router_ws, gate_weight, up_weight, down_weight, mlp_ws, y, num_tokens, hidden_size, intermediate_size, g,
+                                         training != 0, main_s);
+        if (he == hipSuccess) he = launch_gather_add(x, up_embed, down_embed, gates, ids, y, nullptr, 0, shared, num_tokens, hidden_size, num_experts_per_token, num_experts, dtype, main_s);
+        return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
       } else if (few && !training) {
         const hipError_t he = launch_few_tokens(dtype, f, main_s);
         return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
       }
-      if (dtype != OMNI_F32) return joint_forward(f, dtype, omni_mlp_workspace_bytes(num_tokens, hidden_size, intermediate_size, dtype) - h_bytes, main_s, shared, training != 0, [&]() -> int {
+      return joint_forward(f, dtype, omni_mlp_workspace_bytes(num_tokens, hidden_size, intermediate_size, dtype) - h_bytes, main_s, shared, training != 0, [&]() -> int {
         if (merge) return omni_gemm_router_projection(x, router_weight_x, router_weight_y, router_ws, part_mean, part_m2, num_tokens, hidden_size, num_expert_sqrt, dtype, main_s);
         // without a selection (k = 0) omni_router_fwd projects, merges the statistics, moves the running buffers and counts the batch
         return omni_router_fwd(x, router_weight_x, router_weight_y, running_mean_x, running_var_x, num_batches_tracked_x, running_mean_y, running_var_y,
@@ -243,8 +247,9 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   // intermediate 4096, two streams: 4096 tokens 125.7 against 128.0 us, 6144 tokens 188.9 against 178.5, 8192 tokens 243.5 against 228.7)
   const int64_t gate_up_tiles = ((num_tokens + 255) / 256) * (((int64_t)intermediate_size + 127) / 128);
   if (!e) e = mlp_gate_up_impl(x, gate_weight, up_weight, num_tokens, hidden_size, intermediate_size, dtype, mlp_ws, main_s, alone || gate_up_tiles > 512);
-  if (!e) e = omni_expert_fwd(x, up_embed, down_embed, gates, ids, experts, num_tokens, hidden_size, num_experts,
-                              num_experts_per_token, dtype, expert_algo, expert_ws, branch);
+  if (!e) e = f32_sizes ? expert_gather_f32(x, up_embed, down_embed, gates, ids, experts, shared, num_tokens, hidden_size, num_experts_per_token, num_experts, branch)
+                        : omni_expert_fwd(x, up_embed, down_embed, gates, ids, experts, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype, expert_algo,
+                                          expert_ws, branch);
   if (!side_stream) {   // one stream: the add is the down projection's epilogue
     if (!e) e = mlp_down_impl(down_weight, experts, y, num_tokens, hidden_size, intermediate_size, dtype, mlp_ws, main_s, true);
     return e;

@@ -395,6 +395,37 @@ def test_layer_two_streams_equals_one_stream(case, algo, device):
     assert torch.equal(out, layer(x * 2))
 
 
+# T, H, I, N, k in single precision: sizes of the joint launches at which the experts alone would be split, or would share a token's slots between four or two waves
+F32_STREAM_CASES = [(1100, 256, 1024, 4096, 32), (512, 512, 1024, 4096, 32), (300, 256, 512, 1024, 32), (1000, 512, 1024, 1024, 16)]
+
+
+@pytest.mark.parametrize("training", [False, True], ids=["eval", "train"])
+@pytest.mark.parametrize("aligned", [True, False], ids=["aligned", "off-boundary"])
+@pytest.mark.parametrize("algo", ["auto", "gather"])
+@pytest.mark.parametrize("case", F32_STREAM_CASES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
+def test_layer_fp32_two_streams_equals_one_stream(case, algo, aligned, training, device):
+    """In single precision a small layer has joint launches on one stream and the two schedules on two: the experts' sums must run in one order on either, so the
+    output is the same to the bit."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, H, I, N, k = case
+    print(f"fp32 streams {case} {algo} aligned={aligned} training={training}", flush=True)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", N, k)).to(device=device).train(training)
+    g = torch.Generator(device=device).manual_seed(T)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, H ** -0.5, generator=g)
+        x = torch.randn(1, T, H, device=device, generator=g)
+        if not aligned:
+            x = _elsewhere(x, device)
+        layer.expert_algo = algo
+        layer.overlap_min_work = 0
+        layer.overlap_branches = False
+        ref = layer(x)
+        layer.overlap_branches = True
+        assert _waits_for_side_stream(layer, x)
+        assert torch.equal(layer(x), ref)
+
+
 def test_layer_copies_and_saves_like_a_plain_module(device, tmp_path):
     """After a two-stream forward (side stream and events in use) a layer is still a plain nn.Module:
     copy.deepcopy, torch.save / torch.load and a state_dict round trip give layers with identical output."""
