@@ -52,7 +52,7 @@ extern "C" {
 #define OMNI_EXPERT_ALGO_AUTO 0
 #define OMNI_EXPERT_ALGO_GATHER 1   /* token-resident gather, no schedule needed */
 #define OMNI_EXPERT_ALGO_SEGMENT 2  /* expert-centric segments from omni_schedule */
-#define OMNI_EXPERT_ALGO_SPLIT 3    /* hidden dimension cut into 8 slices, one per XCD: table slices stay in that XCD's L2 */
+#define OMNI_EXPERT_ALGO_SPLIT 3    /* hidden dimension cut into 4 or 8 slices, for two XCDs or one each: table slices stay in their L2s */
 #define OMNI_EXPERT_ALGO_DENSE 4    /* few experts, hundreds of tokens each: two MFMA GEMMs over all experts (the reference's group regime) */
 
 OMNI_API int32_t omni_abi_version(void);
@@ -119,15 +119,15 @@ OMNI_API int32_t omni_schedule_noalloc(const int32_t* indices, int32_t* offsets,
  *   as in the reference); y [T,H] dtype `dtype`, fully overwritten.
  * H*sizeof(elem) must be a multiple of 16.  Sums are fp32, one rounding at the end.
  *   algo      : OMNI_EXPERT_ALGO_*.  GATHER: one wave per token fetches whole rows.  SPLIT: the hidden
- *               dimension in 8 slices, slice s handled by the blocks that run on XCD s, so that
- *               each XCD's L2 holds its eighth of both tables; two launches and [8][T][k] floats
- *               of partial dot products (H*sizeof(elem)/8 must be 64..1024 bytes, a power of two; wider rows are
+ *               dimension in 4 or 8 slices, each handled by the blocks that run on two XCDs or one, so that
+ *               an XCD's L2 holds its slice of both tables; two launches and a float of partial dot product per
+ *               pair and slice (by name: H*sizeof(elem)/8 must be 64..1024 bytes, a power of two; wider rows are
  *               taken in up to 64 column blocks of that form, one pair of launches per block, [8 * blocks][T][k] floats).
  *               Rows beyond 8 KiB exist for SPLIT only, and AUTO is SPLIT for them.
- *               AUTO chooses between GATHER and SPLIT from a measured grid, by the bytes of a row, of a
- *               table and of the rows that all pairs name (T*k rows): GATHER for few pairs (less than 32 to
- *               64 MiB of rows), tables beyond 16 MiB (rows under 1 KiB) to 256 MiB, rows under 512 bytes
- *               and k > 128; SPLIT elsewhere, and for
+ *               AUTO chooses between GATHER and SPLIT from a measured grid, by the tokens (rows of up to 1 KiB), the
+ *               bytes of a row, of a table and of the rows that all pairs name (T*k rows): GATHER for few tokens (up to
+ *               1024, or 4096 over larger tables) or pairs (less than 32 to 64 MiB of rows), for tables beyond 16 to
+ *               256 MiB, rows under 512 bytes and k > 128; SPLIT elsewhere -- more tokens never turn it back -- and for
  *               rows beyond 8 KiB.  SEGMENT is the expert-centric organisation:
  *               omni_schedule, a pass over the sorted pairs for the coefficients, a token pass
  *               for the sum; kept so that the organisations can be measured side by side.

@@ -789,9 +789,10 @@ extern "C" OMNI_API int32_t omni_router_norm_bwd_padded(const void* dgates, cons
 
 namespace omni {
 int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype);       // defined beside the expert kernels: what AUTO runs
-// Slices where the token pass takes the split organisation -- where the forward does -- else 0
+// Slices where the token pass takes the split organisation, else 0: where the forward does, but for sorts of one tile, beside which the gather organisation is
+// one launch less (whole backward, bf16, rows of 512 B to 1 KiB, 1100 and 2048 tokens x 2 and 4, split over gather: 1.09-1.18 up to 8192 pairs, 0.97-1.02 at 8800)
 static int bwd_split_slices(int64_t T, int H, int64_t N, int k, int dtype) {
-  if (resolve_algo(OMNI_EXPERT_ALGO_AUTO, T, H, N, k, dtype) != OMNI_EXPERT_ALGO_SPLIT) return 0;
+  if (T * (int64_t)k <= 8192 || resolve_algo(OMNI_EXPERT_ALGO_AUTO, T, H, N, k, dtype) != OMNI_EXPERT_ALGO_SPLIT) return 0;
   const int es = dtype == OMNI_F32 ? 4 : 2, slices = (int64_t)H * es <= 8192 ? split_slices(H, N, es) : 0;
   return slices && split_lanes_per_row(H, es, slices) >= 5 ? slices : 0;       // (no kernels for groups of four lanes)
 }

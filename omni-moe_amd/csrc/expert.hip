@@ -581,18 +581,21 @@ static int expert_dense_dispatch(const void* x, const void* up, const void* down
 }
 
 // What OMNI_EXPERT_ALGO_AUTO runs, from the sizes alone.  The split algorithm gives every XCD a part of each table row, so it pays while that part of the
-// tables stays near its caches (its 4 MiB L2 and its part of the memory-side cache) and where the rows that are moved outweigh its second launch; whole-row
-// gathering wins with few pairs and on tables far beyond the caches.  Time of split (the better number of slices) over time of gather, bf16, ids uniform
-// over the experts; "moved" is pairs x row bytes, a table N x row bytes:
-//   rows 512 B   16384 x 16 and 4096 x 32 tokens: 0.57-0.70 up to 8 MB a table, 0.81-0.91 at 32 MB, 1.0-1.4 at 128 MB; 4096 x 2 to 4096 x 8: 0.65-0.92;
-//                2048 x 16 1.0, 1024 x 32 1.1, fewer pairs 1.3-1.5
-//   rows 1 KiB   0.41-0.82 up to 16 MB, 0.88-0.97 at 64 MB, 0.9-1.1 at 256 MB; 2048 x 8 1.0-1.1, 1024 x 16 1.0-1.3
-//   rows 1.5 KiB 0.43-0.85 up to 24 MB, 0.86-0.96 at 96 MB, 0.9-1.03 at 384 MB; 1024 x 16 0.75-1.05; 2048 x 16 over a table of 1.5 MB 1.02
-//   rows 2 KiB   0.39-0.81 up to 32 MB, 0.89-0.95 at 128 MB, at 512 MB 0.92-0.95 from 262144 pairs on and 0.94-1.05 with fewer; 2048 x 8 0.74-1.08,
-//                1024 x 16 0.64-0.98, 16384 x 4 0.75-1.0, 4096 x 4 0.9-1.1, 4096 x 2 1.1-1.2
-//   rows 2.5 KiB 0.43-0.87 up to 40 MB, 0.89-0.98 at 160 MB, 0.91-1.03 at 640 MB
-//   rows 4 KiB   0.36-0.78 up to 64 MB, 0.94-0.99 at 256 MB, 0.88-1.0 at 1 GB; 512 x 16 0.56-0.88; 16384 x 8 1.0 at 256 MB; 16384 x 4 0.71-0.89, 1.1 from 256 MB on
-//   rows 8 KiB   0.36-0.86 up to 128 MB, 0.87-1.0 at 512 MB
+// tables stays near its caches (its 4 MiB L2 and its part of the memory-side cache) and where what the gather algorithm moves outweighs its second launch.
+// Rows up to 1 KiB the gather kernel fetches with half of its lanes or less, so there the number of tokens decides (1024: its waves share a token's slots up to
+// there); longer rows go by the bytes that all pairs name ("moved": pairs x row bytes).  A row that is no power of two leaves lanes of a slice idle (`whole`), few
+// pairs to a token leave part of a batch of 8 empty, and a table of at most 2 MiB ("little") every L2 holds whole.  More tokens never turn it back to gather.
+// Time of split over time of gather, bf16, ids uniform over the experts, tables of 1 to 256 MB each ("table": N x row bytes):
+//   rows 512 B    k <= 8: 0.92-1.09 at 1024 tokens, 0.71-0.97 at 1536 to 3000, 0.59-0.88 at 4096, 0.31-0.79 at 32768 and 65536
+//                 k 12 to 32 up to 16 MB: 0.80-1.08 at 1536 to 3000, 0.67-0.93 at 4096, 0.51-0.97 beyond; above 16 MB 0.85-1.3
+//   rows 1 KiB    k <= 4: 0.71-0.94 at 4096, 0.61-0.91 beyond; k >= 6 up to 64 MB 0.50-0.98, above 0.95-1.13; 1536 to 3000 tokens 0.69-0.98 up to 16 MB, 0.82-1.13 above
+//   640 to 896 B  0.65-1.09 up to 16 MB (k 10 1.16); above k 2 0.69-0.92, k 4 0.85-1.11, k 6 and 8 1.04-1.5
+//   1.1 to 1.4 KiB  k 2 0.94-1.31; moved >= 64 MB up to 16 MB 0.70-1.0, at 64 MB 1.05-1.3
+//   rows 1.5 KiB  moved >= 64 MB: k >= 4 0.49-1.06 up to 64 MB; 32 to 64 MB: k >= 8 0.65-0.95 at 4 and 16 MB, 0.95-1.02 at 64; k 2 0.91-1.26
+//   rows 2 KiB    moved >= 64 MB: 0.42-0.95 from 4 to 64 MB, k 4 to 8 over a little table 0.94-1.09, 128 and 256 MB 0.93-1.10; 32 to 64 MB: k 6 0.86-0.94, k 8 0.74-0.95 up to 32 MB
+//   rows 2.5 and 3 KiB  k 4 0.93-1.72, k 6 0.71-1.04 from 4 to 64 MB; little tables: k 6 1.06-1.23, k 8 and 12 1.0-1.24 (their backward 0.85-0.92), 16 0.88-1.0, 32 0.83-0.96
+//   rows 4 and 8 KiB    moved >= 64 MB: k >= 4 0.34-1.07 from 4 to 64 MB; little tables: k 4 1.2-1.6, k 6 0.93-1.29, k 8 and 12 0.88-1.24, 16 and 32 0.72-1.03; 256 MB: k < 16 0.91-1.16, k >= 16 0.72-1.03
+// (the rule's choice takes 0.7 % more than the better of the two on average, over 10 % at 2 % of the 3032 points of these rows)
 // A skewed router (few live experts) moves every figure towards the split algorithm; the caller who knows says so.
 int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
   if (algo != OMNI_EXPERT_ALGO_AUTO) return algo;
@@ -605,9 +608,17 @@ int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
   const int64_t row = (int64_t)H * es, table = N * row, pairs = T * (int64_t)k, moved = pairs * row, MiB = 1 << 20;
   if (row > 8192) return OMNI_EXPERT_ALGO_SPLIT;
   if (row < 512 || k > 2 * kWave || split_slices(H, N, es) == 0) return OMNI_EXPERT_ALGO_GATHER;
-  const bool enough = moved >= 64 * MiB ? k >= 4 : moved >= 32 * MiB ? k >= 8 && table > 2 * MiB && (k >= 16 || table <= 64 * MiB) : row <= 1024 && T >= 4096;
-  const bool near = row < 1024 ? table <= 16 * MiB : row < 1536 ? table <= 64 * MiB : row < 2048 ? table <= 128 * MiB
-                  : k >= 16 ? table <= 256 * MiB || pairs >= 262144 : table <= 64 * MiB;
+  const bool whole = (row & (row - 1)) == 0, little = table <= 2 * MiB;
+  bool enough, near;
+  if (row <= 1024) {
+    enough = T >= 4096 || moved >= 64 * MiB || (moved >= 32 * MiB && !little && k >= 16) || (T > 1024 && (table <= (row == 1024 ? 16 : 4) * MiB || (row == 512 && k <= 8)));
+    near = table <= (row == 1024 ? 64 : 16) * MiB || k <= (row == 1024 ? 4 : row == 512 ? 8 : 2);
+  } else {
+    const int least = row <= 2048 || (whole && !little) ? 4 : little ? 8 : 6;
+    const bool half = row > 2048 && row < 2560;                  // little more than half of a slice's lanes
+    enough = moved >= 64 * MiB ? k >= least : moved >= 32 * MiB && !little && (k >= 16 || (k >= 6 && N <= 16384));
+    near = table <= (row < 1536 ? 16 : row < 2048 ? 128 : half ? 32 : k >= 16 ? 256 : 64) * MiB || (row >= 2048 && !half && k >= 16 && pairs >= 262144);
+  }
   return enough && near ? OMNI_EXPERT_ALGO_SPLIT : OMNI_EXPERT_ALGO_GATHER;
 }
 

@@ -97,6 +97,18 @@ def test_argument_errors_need_no_gpu():
         assert lib.omni_init() >= 1000           # a HIP error (no device), not a crash
 
 
+@pytest.mark.parametrize("row", [512, 640, 1024, 1280, 1536, 2048, 2304, 2560, 4096, 8192])
+def test_auto_keeps_the_split_algorithm_as_tokens_grow(row):
+    """What AUTO runs shows in the workspace it asks for (the gather algorithm needs none).  Once it splits it does so for every larger number of tokens."""
+    lib = _lib().load()
+    for dtype, size in ((0, 2), (2, 4)):
+        for experts in (64, 256, 900, 1024, 4096, 10000, 16384, 65536, 262144):
+            for k in (2, 4, 6, 8, 12, 16, 32, 64, 128):
+                tokens = [2 ** n + d for n in range(6, 18) for d in (0, 2 ** (n - 1))]
+                split = [lib.omni_expert_workspace_bytes(t, row // size, experts, k, dtype, 0) > 0 for t in tokens]
+                assert split == sorted(split), (dtype, experts, k, [t for t, s in zip(tokens, split) if s])
+
+
 def test_mlp_bwd_refuses_unaligned_pointers():
     """Each pointer of omni_mlp_bwd in turn two bytes past a 16-byte boundary: refused before anything is enqueued."""
     lib = _lib().load()

@@ -137,8 +137,10 @@ def test_expert_bwd_skewed_and_bad_ids(device):
 
 
 # T, hidden bytes, N, k: the split token pass at every slice length (128 bytes to 1 KiB), ragged tokens, its sort in one pass (4096 bins, more) and in two;
-# the gather token pass with half of its tokens beside the count pass
-EXPERT_BWD_SPLIT_CASES = [(4100, 1024, 2050, 32), (1030, 2048, 4099, 32), (1025, 4096, 20000, 32), (1031, 8192, 600, 32), (4101, 512, 300, 6)]
+# at 7800 pairs a forward that splits and a backward that gathers (one tile to sort), at 8400 both split; the gather token pass with half of its tokens beside the
+# count pass
+EXPERT_BWD_SPLIT_CASES = [(4100, 1024, 2050, 32), (1030, 2048, 4099, 32), (1025, 4096, 20000, 32), (1031, 8192, 600, 32), (4101, 512, 300, 6),
+                          (1300, 512, 3000, 6), (1400, 1024, 4000, 6), (4101, 2048, 300, 6)]
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)

@@ -303,11 +303,12 @@ def test_expert_split_algorithm(case, device):
     assert (got.float() - ref).abs().max().item() <= (1e-2 if dtype != torch.float32 else 1e-5) * scale
 
 
-# AUTO's split algorithm: four slices of 10, 8, 24, 40, 33 and 64 lanes, eight of 32 and 64; top-k below, at and beyond a batch of 16; ragged tokens
+# AUTO's split algorithm: four slices of 10, 8, 24, 40, 33 and 64 lanes, eight of 32 and 64; top-k below, at and beyond a batch of 16; ragged tokens;
+# short rows from 1025 tokens on, over tables beyond every cache too
 EXPERT_AUTO_SPLIT_CASES = [(4100, 320, 500, 2, torch.bfloat16), (4097, 256, 900, 6, torch.float16), (2050, 768, 3000, 16, torch.bfloat16),
                            (1100, 1280, 900, 34, torch.bfloat16), (1030, 1056, 12000, 18, torch.bfloat16), (1003, 2048, 700, 12, torch.float16),
                            (1100, 2048, 8000, 16, torch.bfloat16), (600, 4096, 70, 16, torch.bfloat16), (4099, 160, 300, 4, torch.float32),
-                           (1001, 512, 300, 128, torch.bfloat16)]
+                           (1001, 512, 300, 128, torch.bfloat16), (1025, 256, 70000, 8, torch.bfloat16), (1100, 448, 2000, 34, torch.float16), (4097, 512, 150000, 4, torch.bfloat16)]
 
 
 @pytest.mark.parametrize("case", EXPERT_AUTO_SPLIT_CASES, ids=lambda c: f"T{c[0]}-H{c[1]}-N{c[2]}-k{c[3]}-{str(c[4]).split('.')[-1]}")
