@@ -264,7 +264,10 @@ OMNI_API int32_t omni_expert_bwd(const void* dy, const void* x, const void* up_w
                                  void* ddown_weight, void* drouting_weights, int64_t num_tokens, int32_t hidden_size,
                                  int64_t num_experts, int32_t num_experts_per_token, int32_t dtype, void* workspace,
                                  void* stream);
-/* omni_expert_bwd with the pair scores of the same forward pass (omni_expert_fwd_scores; NULL: recomputed). */
+/* omni_expert_bwd with the pair scores of the same forward pass (omni_expert_fwd_scores; NULL: recomputed).
+ * omni_expert_bwd_reads_scores: 1 where they are read (the split token pass), 0 where a forward pass need not leave them. */
+OMNI_API int32_t omni_expert_bwd_reads_scores(int64_t num_tokens, int32_t hidden_size, int64_t num_experts,
+                                              int32_t num_experts_per_token, int32_t dtype);
 OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x, const void* up_weight, const void* down_weight,
                                         const void* routing_weights, const int32_t* indices, const float* scores, void* dx,
                                         void* dup_weight, void* ddown_weight, void* drouting_weights, int64_t num_tokens,

@@ -15,7 +15,7 @@
 // Expert backward in two passes.  Token pass: forms dx and dg and, in an fp32 workspace, ds and the forward coefficient silu(s) g of
 // every pair, in the organisation that the forward takes at the sizes: gather (one wave owns one token, keeps x_t, dy_t and the fp32 dx
 // accumulator in registers and fetches each selected up and down row once) or split (the rows in eight column slices, one to an XCD).
-// s comes from the forward where that kept it, else it is recomputed.  Weight pass: the pairs are grouped by expert with the
+// split takes s from the forward where that kept it; gather, which has the up rows in hand for dx, and split without it form it again.  Weight pass: the pairs are grouped by expert with the
 // stable schedule of the forward path; one wave owns one expert, walks its segment and gathers
 // the x and dy rows of the segment's tokens, so every dU/dV row is written exactly once
 // (zeros for experts nobody selected).
@@ -250,11 +250,11 @@ struct TokenPass {
   const uint8_t *x, *dy, *up, *down;
   const void* gates;
   const int32_t* ids;
-  const float* scores;               // NULL: recompute
+  const float* scores;               // split: NULL: recompute
   uint8_t* dx;
   void* dgates;
   float *ds, *coef;                  // [tokens][top_k]
-  float *partial_a, *partial_s;      // split: [8][tokens][top_k]
+  float *partial_a, *partial_s;      // split: [slices][tokens][top_k], partial_s without scores only
   int first, last, num_tokens, hidden, top_k;      // gather: the tokens of this launch
   int lanes, slices;                 // split: 16-byte lanes of a row slice, and slices; 0, 0: gather
   uint32_t num_experts;
@@ -799,16 +799,21 @@ static int bwd_split_slices(int64_t T, int H, int64_t N, int k, int dtype) {
 }  // namespace omni
 
 // workspace: ds [P] f32 | coef [P] f32 | sorted pair ids [P] i32 | sorted token ids [P] i32 | offsets [N+1] i32 |
-//            partial rows [chunks][2][2][H] f32 | split: partial <dy, V>, partial <x, U> [8][P] f32 each | schedule workspace
+//            partial rows [chunks][2][2][H] f32 | split: partial <dy, V>, partial <x, U> (without scores) [slices][P] f32 each | schedule workspace
 extern "C" OMNI_API size_t omni_expert_bwd_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int64_t num_experts,
                                                            int32_t num_experts_per_token, int32_t dtype) {
   using namespace omni;
   if (num_tokens < 0 || num_experts <= 0 || num_experts_per_token < 0 || hidden_size <= 0) return 0;
   const size_t P = (size_t)num_tokens * (size_t)num_experts_per_token;
   const size_t chunks = (P + weight_chunk(P) - 1) / weight_chunk(P);
-  return 4 * up256(P * 4) + up256(((size_t)num_experts + 1) * 4) + up256(chunks * 4 * (size_t)hidden_size * 4) +
-         (bwd_split_slices(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) ? 2 * up256(kSlices * P * 4) : 0) +
+  const size_t slices = (size_t)bwd_split_slices(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype);
+  return 4 * up256(P * 4) + up256(((size_t)num_experts + 1) * 4) + up256(chunks * 4 * (size_t)hidden_size * 4) + 2 * up256(slices * P * 4) +
          omni_schedule_workspace_bytes(num_tokens, num_experts_per_token, num_experts);
+}
+
+extern "C" OMNI_API int32_t omni_expert_bwd_reads_scores(int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_experts_per_token, int32_t dtype) {
+  if (num_tokens < 0 || num_experts <= 0 || num_experts_per_token < 0 || hidden_size <= 0) return 0;
+  return omni::bwd_split_slices(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) ? 1 : 0;
 }
 
 extern "C" OMNI_API int32_t omni_expert_bwd(const void* dy, const void* x, const void* up_weight, const void* down_weight,
@@ -854,8 +859,8 @@ extern "C" OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x
   const int lanes = slices ? split_lanes_per_row(hidden_size, dtype == OMNI_F32 ? 4 : 2, slices) : 0;
   float *partial_a = nullptr, *partial_s = nullptr;
   if (lanes) {
-    partial_a = (float*)w;             w += up256(kSlices * P * 4);
-    partial_s = (float*)w;             w += up256(kSlices * P * 4);
+    partial_a = (float*)w;             w += up256(slices * P * 4);
+    partial_s = (float*)w;             w += up256(slices * P * 4);
   }
   hipStream_t s = (hipStream_t)stream;
   // one counting pass: beside the token pass; two: on their own, in front of it

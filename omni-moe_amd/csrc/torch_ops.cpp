@@ -102,9 +102,13 @@ Tensor expert_forward(const Tensor& x, int64_t T, const Tensor& up, const Tensor
 
 struct ExpertFn : public torch::autograd::Function<ExpertFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& up, const Tensor& down, const Tensor& gates, const Tensor& ids) {
-    Tensor scores = at::empty(ids.sizes(), x.options().dtype(at::kFloat));
+    Tensor scores;                                 // kept where the backward pass reads them
+    if (omni_expert_bwd_reads_scores(x.size(0), (int32_t)x.size(1), up.size(0), (int32_t)ids.size(1), dtype_code(x.scalar_type())))
+      scores = at::empty(ids.sizes(), x.options().dtype(at::kFloat));
     Tensor y = expert_forward(x, x.size(0), up, down, ptr(gates), ptr(ids), ids.size(1), OMNI_EXPERT_ALGO_AUTO, ptr(scores));
-    ctx->save_for_backward({x, up, down, gates, ids, scores});
+    variable_list kept{x, up, down, gates, ids};
+    if (scores.defined()) kept.push_back(scores);
+    ctx->save_for_backward(kept);
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -117,7 +121,7 @@ struct ExpertFn : public torch::autograd::Function<ExpertFn> {
     const int dt = dtype_code(x.scalar_type());
     Tensor dx = at::empty_like(x), dup = at::empty_like(up), ddown = at::empty_like(down), dg = at::empty_like(gates);
     Tensor ws = bytes(omni_expert_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt), x.device());
-    check(omni_expert_bwd_scores(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), (const float*)ptr(s[5]), ptr(dx), ptr(dup), ptr(ddown), ptr(dg), T,
+    check(omni_expert_bwd_scores(ptr(dy), ptr(x), ptr(up), ptr(down), ptr(gates), (const int32_t*)ptr(ids), s.size() > 5 ? (const float*)ptr(s[5]) : nullptr, ptr(dx), ptr(dup), ptr(ddown), ptr(dg), T,
                                  (int32_t)H, N, (int32_t)k, dt, ptr(ws), stream_of(x.device())), "omni_expert_bwd");
     return {dx, dup, ddown, dg, Tensor()};
   }
@@ -227,12 +231,13 @@ struct Slab {
     return at;
   }
 };
-struct Kept {                                       // gates and ids, the router's workspace (z and the statistics), pair scores, rounded gate and up projections, their SwiGLU product
+struct Kept {     // gates and ids, the router's workspace (z and the statistics), pair scores where the backward pass reads them, rounded gate and up projections, their SwiGLU product
   Slab s;
   size_t gates, ids, router, scores, gate, up, h;
-  Kept(int64_t T, int64_t I, int64_t r, int64_t k, int dt) {
+  bool scored;
+  Kept(int64_t T, int64_t H, int64_t I, int64_t N, int64_t r, int64_t k, int dt) : scored(omni_expert_bwd_reads_scores(T, (int32_t)H, N, (int32_t)k, dt) != 0) {
     const size_t es = dt == OMNI_F32 ? 4 : 2, pairs = (size_t)(T * k), wide = (size_t)(T * I) * es;
-    gates = s.add(pairs * es); ids = s.add(pairs * 4); router = s.add(omni_router_workspace_bytes(T, (int32_t)r, dt)); scores = s.add(pairs * 4);
+    gates = s.add(pairs * es); ids = s.add(pairs * 4); router = s.add(omni_router_workspace_bytes(T, (int32_t)r, dt)); scores = s.add(scored ? pairs * 4 : 0);
     gate = s.add(wide); up = s.add(wide); h = s.add(wide);
   }
 };
@@ -248,11 +253,11 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     const int64_t T = x.numel() / l.H;
     const int dt = dtype_code(x.scalar_type());
     void* s = stream_of(x.device());
-    const Kept at(T, l.I, l.r, l.k, dt);
+    const Kept at(T, l.H, l.I, l.N, l.r, l.k, dt);
     const Tensor kept = bytes(at.s.size, x.device());
     uint8_t* k = (uint8_t*)ptr(kept);
     router_forward(x, T, l.H, rx, ry, l.norms, l.k, k + at.gates, k + at.ids, k + at.router);
-    const Tensor e = expert_forward(x, T, up, down, k + at.gates, k + at.ids, l.k, OMNI_EXPERT_ALGO_AUTO, k + at.scores);
+    const Tensor e = expert_forward(x, T, up, down, k + at.gates, k + at.ids, l.k, OMNI_EXPERT_ALGO_AUTO, at.scored ? k + at.scores : nullptr);
     if (dt != OMNI_F32) {                          // (rows of 16 bytes, so both sizes are multiples of 8; operands at any address)
       check(omni_swiglu_linear_save_fwd(ptr(x), ptr(wg), ptr(wu), k + at.h, k + at.gate, k + at.up, T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_swiglu_linear_save_fwd");
     } else {
@@ -283,7 +288,7 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     variable_list out(9);
     const bool own = dt != OMNI_F32, router = need[0] || need[4] || need[5];        // 16-bit products are the library's own
     const int64_t rp = own ? (r + 7) / 8 * 8 : r;
-    const Kept at(T, I, r, k, dt);
+    const Kept at(T, H, I, N, r, k, dt);
     const uint8_t* saved = (const uint8_t*)ptr(kept);
     // temporaries: the experts' d(x), d(gates), d(z), and one workspace for three stages that follow one another on the stream
     Slab t;
@@ -294,7 +299,7 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     uint8_t* w = (uint8_t*)ptr(temp);
     // experts, then the router stage behind their gates' gradient
     Tensor dup = at::empty_like(up), ddown = at::empty_like(down);
-    check(omni_expert_bwd_scores(ptr(dy), ptr(x3), ptr(up), ptr(down), saved + at.gates, (const int32_t*)(saved + at.ids), (const float*)(saved + at.scores), w + dx_at, ptr(dup),
+    check(omni_expert_bwd_scores(ptr(dy), ptr(x3), ptr(up), ptr(down), saved + at.gates, (const int32_t*)(saved + at.ids), at.scored ? (const float*)(saved + at.scores) : nullptr, w + dx_at, ptr(dup),
                                  ptr(ddown), w + dg_at, T, (int32_t)H, N, (int32_t)k, dt, w + ws_at, st), "omni_expert_bwd");
     if (need[6]) out[6] = dup;
     if (need[7]) out[7] = ddown;

@@ -58,6 +58,7 @@ SIGNATURES = {
     "omni_router_bwd": (c_int32, [c_void_p] * 4 + [c_int64, c_int32, c_int32, c_int32, c_void_p]),
     "omni_expert_bwd_workspace_bytes": (c_size_t, [c_int64, c_int32, c_int64, c_int32, c_int32]),
     "omni_expert_bwd": (c_int32, [c_void_p] * 10 + [c_int64, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p]),
+    "omni_expert_bwd_reads_scores": (c_int32, [c_int64, c_int32, c_int64, c_int32, c_int32]),
     "omni_expert_bwd_scores": (c_int32, [c_void_p] * 11 + [c_int64, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p]),
     "omni_swiglu_fwd": (c_int32, [c_void_p] * 3 + [c_int64, c_int32, c_void_p]),
     "omni_swiglu_bwd": (c_int32, [c_void_p] * 5 + [c_int64, c_int32, c_void_p]),

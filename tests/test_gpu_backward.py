@@ -138,21 +138,40 @@ def test_expert_bwd_skewed_and_bad_ids(device):
 
 # T, hidden bytes, N, k: the split token pass at every slice length (128 bytes to 1 KiB), ragged tokens, its sort in one pass (4096 bins, more) and in two;
 # at 7800 pairs a forward that splits and a backward that gathers (one tile to sort), at 8400 both split; the gather token pass with half of its tokens beside the
-# count pass
+# count pass; slices of 10, 13, 21, 24, 33, 40 and 48 lanes (four) and of 18 and 48 (eight)
 EXPERT_BWD_SPLIT_CASES = [(4100, 1024, 2050, 32), (1030, 2048, 4099, 32), (1025, 4096, 20000, 32), (1031, 8192, 600, 32), (4101, 512, 300, 6),
-                          (1300, 512, 3000, 6), (1400, 1024, 4000, 6), (4101, 2048, 300, 6)]
+                          (1300, 512, 3000, 6), (1400, 1024, 4000, 6), (4101, 2048, 300, 6), (1100, 640, 2000, 10), (4100, 832, 500, 16), (2050, 1344, 2000, 16),
+                          (4100, 1536, 3000, 16), (1030, 2112, 12000, 18), (1100, 2560, 900, 34), (1300, 3072, 2000, 34), (1030, 2304, 13000, 18), (1040, 6144, 1200, 32)]
+EXPERT_BWD_GATHERS = [(1300, 512, 3000, 6), (4101, 2048, 300, 6)]
+
+
+def _expert_bwd_splits(T, H, N, k, dtype):
+    from omni_moe.ops.hip import _lib
+    return bool(_lib.load().omni_expert_bwd_reads_scores(T, H, N, k, _lib.DTYPE_CODE[dtype]))
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
 @pytest.mark.parametrize("case", EXPERT_BWD_SPLIT_CASES, ids=lambda c: "T%d-B%d-N%d-k%d" % c)
 def test_expert_bwd_split_matches_fp64(case, dtype, device):
     """Many pairs: with the forward's pair scores (autograd) and without (the operator), against 64 bits, to the tolerance of the other cases."""
+    _check_expert_bwd(case, dtype, device)
+
+
+# tables off a 16-byte boundary: 64-bit addresses instead of buffer loads, whole slices and ragged ones
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("case", [(4100, 1024, 2050, 32), (4100, 1536, 3000, 16), (1030, 2112, 12000, 18), (1031, 8192, 600, 32)], ids=lambda c: "T%d-B%d-N%d-k%d" % c)
+def test_expert_bwd_split_takes_tables_at_any_address(case, dtype, device):
+    _check_expert_bwd(case, dtype, device, place=lambda t: _elsewhere(t, device))
+
+
+def _check_expert_bwd(case, dtype, device, place=lambda t: t):
     T, row, N, k = case
     H = row // torch.empty(0, dtype=dtype).element_size()
+    assert _expert_bwd_splits(T, H, N, k, dtype) == (case not in EXPERT_BWD_GATHERS)
     print(f"expert bwd split T={T} H={H} N={N} k={k} {dtype}", flush=True)
     g = torch.Generator(device=device).manual_seed(T + H)
     n = lambda *s, std=1.0: torch.empty(*s, device=device).normal_(0, std, generator=g).to(dtype)
-    x, dy, up, down = n(T, H), n(T, H), n(N, H, std=0.05), n(N, H, std=0.05)
+    x, dy, up, down = n(T, H), n(T, H), place(n(N, H, std=0.05)), place(n(N, H, std=0.05))
     gates = torch.softmax(n(T, k).float(), -1).to(dtype)
     ids = torch.randint(0, N, (T, k), device=device, dtype=torch.int32, generator=g)
     ids[::3, 1] = ids[::3, 0]
@@ -173,7 +192,7 @@ def test_expert_bwd_split_matches_fp64(case, dtype, device):
         want[1].index_add_(0, e.flatten(), (ds[..., None] * xs[:, None]).flatten(0, 1))
         want[2].index_add_(0, e.flatten(), (cf[..., None] * ys[:, None]).flatten(0, 1))
         want[3][a:a + 64] = p * silu * ok
-    leaves = [t.detach().clone().requires_grad_() for t in (x, up, down, gates)]
+    leaves = [t.detach().requires_grad_() for t in (x, up, down, gates)]
     _ops().hip_omni_expert_func(*leaves, ids).backward(dy)
     op = _ops().hip_omni_expert_bwd_func(dy, x, up, down, gates, ids)
     for leaf, got, ref, what in zip(leaves, op, want, ("dx", "dup", "ddown", "dgates")):
@@ -494,6 +513,33 @@ def test_layer_saved_tensors_through_hooks(dtype, device):
         moved = torch.autograd.grad(layer(x), leaves, dy)
     for a, b, c in zip(first, second, moved):
         assert torch.equal(a, b) and torch.equal(a, c)
+
+
+# T, H, N, k: a backward pass that gathers, one that splits
+@pytest.mark.parametrize("case", [(1000, 512, 1024, 8), (4100, 512, 2050, 16)], ids=["gather", "split"])
+def test_pair_scores_are_kept_where_the_backward_reads_them(case, device):
+    """The forward's <x, U> are four bytes a pair until the backward pass: the operator and the layer keep them for the split token pass alone."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    from omni_moe.ops.hip import _lib
+    T, H, N, k = case
+    I, dtype = 1024, torch.bfloat16
+    splits = _expert_bwd_splits(T, H, N, k, dtype)
+    assert splits == (T > 4096)
+    torch.manual_seed(3)
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", N, k)).to(device=device, dtype=dtype)
+    x = torch.randn(1, T, H, device=device).to(dtype)
+    gates, ids = layer.route(x[0])
+    saved = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t) or t, lambda t: t):
+        _ops().hip_omni_expert_func(x[0].detach().requires_grad_(), layer.up_embed.weight, layer.down_embed.weight, gates, ids)
+    assert [t.shape for t in saved if t.dtype == torch.float32] == ([ids.shape] if splits else [])
+    saved.clear()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t) or t, lambda t: t):
+        layer(x.requires_grad_())
+    kept = sum(t.numel() for t in saved if t.dtype == torch.uint8)
+    others = T * k * (2 + 4) + _lib.load().omni_router_workspace_bytes(T, layer.num_expert_sqrt, _lib.DTYPE_CODE[dtype]) + 3 * T * I * 2
+    padding = 7 * 256                                                    # of seven parts to 256 bytes each
+    assert others <= kept - (T * k * 4 if splits else 0) <= others + padding
 
 
 def test_layer_trains_bf16(device):
