@@ -851,17 +851,19 @@ def test_layer_gather_by_name_is_the_operator(case, dtype, device):
     assert torch.equal(got, want)
 
 
-# one strip, ragged strips, the most strips a block merges at 64 keys and one more, 8 to 128 keys; 136 keys: the merge's own launch
+# one strip, ragged strips, the most strips a block merges at 64 keys and one more, 8 to 128 keys; 136 keys: the merge's own launch; top-56 and up: a selection that
+# does not fit beside the down projection's tiles, behind the merge's own launch
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
-@pytest.mark.parametrize("case", [(2, 8), (33, 64), (700, 104), (2048, 128), (4096, 64), (4100, 64), (300, 136)], ids=lambda c: "T%d-r%d" % c)
+@pytest.mark.parametrize("case", [(2, 8), (33, 64), (700, 104), (2048, 128), (4096, 64), (4100, 64), (300, 136), (700, 64, 64), (2048, 24, 56), (3, 16, 128)],
+                         ids=lambda c: ("T%d-r%d" if len(c) == 2 else "T%d-r%d-k%d") % c)
 def test_joint_batch_statistics_equal_the_router_stage(case, dtype, device):
     """A small layer merges the batch statistics inside its joint launches: buffers and counts as the router stage (which launches the merge) leaves them on the
     same input, to the last bit of an fp32 result (double sums in another order) rounded to the buffers' type."""
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
     from omni_moe.ops import hip
-    T, r = case
-    H, I, k = 64, 128, 8
-    print(f"joint statistics T={T} r={r} {dtype}", flush=True)
+    T, r, k = (*case, 8)[:3]
+    H, I = 64, 128
+    print(f"joint statistics T={T} r={r} k={k} {dtype}", flush=True)
     layer = OmniMoE(OmniMoEConfig(H, I, "silu", r * r, k)).to(device=device, dtype=dtype)
     g = torch.Generator(device=device).manual_seed(T + r)
     with torch.no_grad():
@@ -872,8 +874,13 @@ def test_joint_batch_statistics_equal_the_router_stage(case, dtype, device):
             n.running_var.uniform_(0.5, 1.5, generator=g)
         x = torch.empty(1, T, H, device=device, dtype=dtype).normal_(0.0, 1.0, generator=g)
         stats = [b.clone() for n in (layer.router_norm_x, layer.router_norm_y) for b in (n.running_mean, n.running_var, n.num_batches_tracked)]
-        hip.hip_omni_router_fwd_func(x[0], layer.router_gate_x.weight, layer.router_gate_y.weight, *stats, k, training=True)
-        layer(x)
+        gates, ids = hip.hip_omni_router_fwd_func(x[0], layer.router_gate_x.weight, layer.router_gate_y.weight, *stats, k, training=True)
+        y = layer(x)
+        if k > 8 and dtype != torch.float32:                               # both merge in a launch of its own: the same choice, to the bit
+            experts = hip.hip_omni_expert_func(x[0], layer.up_embed.weight, layer.down_embed.weight, gates, ids)
+            want = hip.hip_omni_mlp_func(x[0], layer.gate_proj.weight, layer.up_proj.weight, layer.down_proj.weight).float() + experts.float()
+            # sums of the same terms in another order, a rounding at each of three places
+            assert ((y[0].float() - want).abs() <= 4 * {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype] * want.abs().max()).all()
     got = [b for n in (layer.router_norm_x, layer.router_norm_y) for b in (n.running_mean, n.running_var, n.num_batches_tracked)]
     ulp = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -22}[dtype]      # neighbours of the buffers' type
     for a, b in zip(got, stats):
