@@ -388,15 +388,16 @@ static int expert_segment_dispatch(const void* x, const void* up, const void* do
 // ---- hidden-split variant ("split" algorithm) ------------------------------------------------
 // For tables that fit the chip's caches but not one XCD's 4 MiB L2 (16 MiB at N = 4096,
 // H = 1024): the hidden dimension is cut into 8 slices and slice s is only ever touched by
-// blocks with blockIdx % 8 == s, which the dispatcher places on XCD s.  An XCD then needs
-// N * H/8 elements of each table -- 1 MiB each in that example -- and serves every table row
+// blocks with blockIdx % 8 == s, which the dispatcher places on XCD s -- or into 4, each for
+// the blocks of two XCDs (split_slices).  With 8 an XCD then needs
+// N * H/8 elements of each table -- 1 MiB each in that example, 2 with 4 -- and serves every table row
 // from its own L2 instead of pulling three quarters of them over the fabric.  The price is a
-// cross-slice reduction of the pair scores, which is tiny ([8][T][k] floats):
+// cross-slice reduction of the pair scores ([slices][T][k] floats):
 //   A. block (token group, slice): partial dot products <x[t, slice], up[id, slice]> for the k pairs
 //      of each of its tokens -> partial[slice][t][j];
 //   B. block (token group, slice): coefficient silu(sum over slices, in slice order) * gate, then
 //      y[t, slice] = sum_j coefficient_j * down[id_j, slice].
-// A row slice is LPR lanes of 16 bytes (64 / LPR pairs per wave at a time).  Fixed summation
+// A row slice is up to LPR lanes of 16 bytes, LPR a power of two (64 / LPR tokens to a wave).  Fixed summation
 // order, no atomics; results agree with the gather algorithm to fp32 rounding of the dot product.
 template <int DT, int LPR, int S, bool RAGGED, bool SMALL>
 __global__ __launch_bounds__(kTokensPerBlock* kWave) void expert_split_dots_kernel(
@@ -405,7 +406,7 @@ __global__ __launch_bounds__(kTokensPerBlock* kWave) void expert_split_dots_kern
   split_dots_block<DT, LPR, S, RAGGED, SMALL, kTokensPerBlock>(x, up, ids, partial, num_tokens, hidden, top_k, num_experts, lanes, col_block, (int)blockIdx.x);
 }
 
-// The coefficient of a pair: the sum of the 8 slice partials in slice order (WIDE: column block by column block), silu, gate.
+// The coefficient of a pair: the sum of the slice partials in slice order (WIDE: column block by column block), silu, gate.
 // kScores: the dot products go to `scores` as well, for a backward pass.
 template <int DT, int S, bool WIDE, bool kScores, class Off>
 struct SplitCoefficient {
@@ -622,8 +623,13 @@ int resolve_algo(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
   return enough && near ? OMNI_EXPERT_ALGO_SPLIT : OMNI_EXPERT_ALGO_GATHER;
 }
 
-// Whether the whole layer may take its joint launches (layer.hip), whose last kernel gathers the experts and adds: where the experts alone would be a little
-// faster split, the launches that the layer saves outweigh it.  Up to where that was measured.
+// Whether the whole layer may take its joint launches (layer.hip), whose last kernel gathers the experts and adds, or its stages one by one with what resolve_algo
+// says: the joint launches for few pairs, for little tables and for rows that are no power of two or under 1 KiB.  Time of the layer with split by name over its time
+// by this rule, bf16, one stream, where the rule gathers and resolve_algo says split:
+//   hidden  256   8192 tokens x 8 0.80, 16384 x 16 0.85, 32768 x 32 0.77 over 4096 experts, 4096 x 32 over 1024 0.83
+//   hidden  512   4096 x 8 over 1024 0.93          hidden  768   4096 x 8 and 2048 x 16 1.0, 4096 x 32 0.90 over 4096, 4096 x 16 over 65536 1.04
+//   hidden 1024   2000 x 16 0.97, 1000 x 32 0.91   hidden 1280   2600 x 16 0.87, 1600 x 32 0.89
+//   hidden 2048   1000 x 16 0.90 over 4096, 500 x 32 over 16384 1.01
 bool joint_launches_gather(int algo, int64_t T, int H, int64_t N, int k, int dtype) {
   if (algo != OMNI_EXPERT_ALGO_AUTO) return algo == OMNI_EXPERT_ALGO_GATHER;
   const int es = dtype == OMNI_F32 ? 4 : 2;

@@ -838,7 +838,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_small_kernel(const G
 }
 
 // A layer of such products in single precision: stages that do not depend on each other share a launch, as in 16 bits (gemm_tiles.hip).  Six dependent launches
-// of 4 to 12 us are four: projection | gate/up (the projection's blocks first: half as long), then selection | down projection.
+// of 4 to 12 us are three: projection | gate/up (the projection's blocks first: half as long), then selection | down projection; the third gathers the experts and adds (expert.hip).
 struct F32Front { GemmArgs router, mlp; int router_blocks; };
 template <int EPI, int NS>            // of the projection: kEpiStats or kEpiPlain
 __global__ __launch_bounds__(kGemmThreads, 1) void gemm_f32_front_kernel(const F32Front g) {

@@ -175,7 +175,8 @@ extern "C" OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_we
   //     (rows within reach of the tile kernels' 31-bit offsets, as few_tokens_covers bounds them; the two launches of the general path have no such bound)
   const bool joint = dtype != OMNI_F32 && num_experts_per_token > 0 && num_expert_sqrt % 8 == 0 && hidden_size % 8 == 0 && intermediate_size % 8 == 0 &&
                      intermediate_size <= (1 << 20) && (double)num_tokens * hidden_size * intermediate_size <= 8589934592.0;
-  // (batch statistics: the projection and their merge stay launches of their own; a cumulative average, momentum < 0, is counted by the select kernel)
+  // (batch statistics: the projection is a launch of its own, and the selecting blocks merge them up to where merge_here says, else a launch in front; a
+  // cumulative average, momentum < 0, takes the general path)
   //   * single precision where every product has few output tiles (f32_joint_covers): the same bound.  A side stream that is given is used, and the two
   //     schedules give the same bits: the sizes alone say how the experts' sums run, on either.
   const bool gathers = joint_launches_gather(expert_algo, num_tokens, hidden_size, num_experts, num_experts_per_token, dtype) && num_experts <= UINT32_MAX;
