@@ -109,7 +109,7 @@ template <int LPR> struct SplitRows<LPR, false> {
   }
 };
 
-// Partial dot products <a[t, slice], table[id, slice]> of the k pairs of a block's tokens -> partial[slice][t][j].  block % 8 is the slice, WAVES the block's
+// Partial dot products <a[t, slice], table[id, slice]> of the k pairs of a block's tokens -> partial[slice][t][j].  block % 8 names the slice (SplitPlace), WAVES the block's
 // waves.  (rows wider than 8 slices of 64 lanes go in column blocks of 8 slices, one launch each)
 template <int DT, int LPR, int S, bool RAGGED, bool SMALL, int WAVES>
 __device__ __forceinline__ void split_dots_block(const uint8_t* __restrict__ x, const uint8_t* __restrict__ up, const int32_t* __restrict__ ids,
@@ -264,15 +264,20 @@ template <class Go>
 static inline hipError_t split_dispatch(int lanes, int slices, Go&& go) {
   auto by_slices = [&](auto group) -> hipError_t {
     constexpr int LPR = decltype(group)::value;
-    auto by_lanes = [&](auto s) -> hipError_t { return lanes == LPR ? go(group, s, std::false_type{}) : go(group, s, std::true_type{}); };
+    auto by_lanes = [&](auto s) -> hipError_t {
+      if constexpr (LPR > 4) {                                   // (no slice has fewer lanes: split_lanes_per_row)
+        if (lanes != LPR) return go(group, s, std::true_type{});
+      }
+      return go(group, s, std::false_type{});
+    };
     if (slices == 4) {
       if constexpr (LPR >= 8) return by_lanes(std::integral_constant<int, 4>{});
       else return hipErrorInvalidValue;
     }
     return slices == kSlices ? by_lanes(std::integral_constant<int, kSlices>{}) : hipErrorInvalidValue;
   };
-  if (lanes <= 0 || lanes > 64) return hipErrorInvalidValue;
-  if (lanes <= 4) return by_slices(std::integral_constant<int, 4>{});
+  if (lanes < 4 || lanes > 64) return hipErrorInvalidValue;
+  if (lanes == 4) return by_slices(std::integral_constant<int, 4>{});
   if (lanes <= 8) return by_slices(std::integral_constant<int, 8>{});
   if (lanes <= 16) return by_slices(std::integral_constant<int, 16>{});
   if (lanes <= 32) return by_slices(std::integral_constant<int, 32>{});
