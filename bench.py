@@ -51,11 +51,11 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16, published
 # Bytes that cross the fabric per launch (FETCH_SIZE + WRITE_SIZE of rocprofv3 --pmc, each scaled by a plain copy of
 # known size); counters cannot be read in-process, so these are the figures of the committed summaries named here.
 TRAFFIC_SOURCE = ("profiles/bench_layer_c4_hbm_counters.txt, profiles/expert_c5_hbm_counters.txt; measured on the kernels as of the commit "
-                  "'Profiles regenerated on the tile GEMM and the joint launches' (expert op at config 5: 'Expert split passes: 32-bit row offsets') -- a "
+                  "'Split expert passes: no ragged kernels for groups of four lanes, which no cut produces' -- a "
                   "later change to a kernel's memory access pattern needs a new counter run")
-TRAFFIC_BYTES = {"expert_c3": 180.6e6, "expert_c4": 57.8e6, "expert_gather_c3": 898.9e6, "gateup_c4": 134.4e6, "down_c4": 117.6e6,
-                 "down_plain_c4": 109.2e6, "schedule_c3": 12.4e6, "expert_segment_c3": 928.3e6, "expert_bwd_c3": 2159.5e6,
-                 "expert_c5_routed": 1029.1e6, "expert_c5_routed_split": 724.9e6, "expert_c5_uniform": 8848.6e6}
+TRAFFIC_BYTES = {"expert_c3": 132.4e6, "expert_c4": 58.3e6, "expert_gather_c3": 899.2e6, "gateup_c4": 134.4e6, "down_c4": 117.6e6,
+                 "down_plain_c4": 109.2e6, "schedule_c3": 12.4e6, "expert_segment_c3": 927.1e6, "expert_bwd_c3": 1527.8e6,
+                 "expert_c5_routed": 1030.3e6, "expert_c5_routed_split": 731.5e6, "expert_c5_uniform": 8846.5e6}
 SECTIONS = ("layer", "kernels", "expert_c3", "expert_c5", "layer_c5", "ref_grid", "probe", "train", "cpu")
 
 
@@ -387,7 +387,7 @@ def main():
         m, b = time_launches(torch, lambda: hip.hip_omni_expert_func(x3, up3, down3, g3, i3))
         e3 = hbm_entry("expert op (split algorithm: expert_split_dots_kernel + expert_split_accumulate_kernel), c3 (T=16384)", m, b,
                        expert_alg_bytes(T3, H, k), TRAFFIC_BYTES["expert_c3"], expert_min_bytes(T3, H, N, k),
-                       note="the 16 MiB tables are cache-resident (each XCD's L2 holds the eighth of them its blocks use): the kernel is bound by "
+                       note="the 16 MiB tables are cache-resident (each XCD's L2 holds the quarter of them its blocks use): the kernel is bound by "
                             "the vector-memory path (L2 hits), so the fraction of HBM peak counts only the bytes that cross the fabric")
         kernels.append(e3)
         out["roofline_expert"] = e3
@@ -403,8 +403,8 @@ def main():
         kernels.append(hbm_entry("expert op, expert-centric 'segment' algorithm (schedule + scores pass + token pass), c3", m, b,
                                  expert_alg_bytes(T3, H, k), TRAFFIC_BYTES["expert_segment_c3"], expert_min_bytes(T3, H, N, k),
                                  note="for comparison; same results as the gather algorithm"))
-        # the reference's group regime (omni_scheduler.py:58: tokens x k / experts > 256): same tokens, 256 experts; AUTO takes
-        # the dense algorithm (two MFMA GEMMs over all experts), timed beside the gather algorithm on the same inputs
+        # the reference's group regime (omni_scheduler.py:58: tokens x k / experts > 256): same tokens, 256 experts; the
+        # dense algorithm by name (two MFMA GEMMs over all experts), timed beside the gather algorithm on the same inputs
         Ng = 256
         xg_c, upg_c, downg_c, gg_c, ig_c = oracle.make_expert_inputs(2, T3, H, Ng, k)
         xg, upg, downg, gg, ig = (t.to(dev) for t in (xg_c, upg_c, downg_c, gg_c, ig_c))
