@@ -121,7 +121,7 @@ OMNI_API int32_t omni_schedule_noalloc(const int32_t* indices, int32_t* offsets,
  *   algo      : OMNI_EXPERT_ALGO_*.  GATHER: one wave per token fetches whole rows.  SPLIT: the hidden
  *               dimension in 4 or 8 slices, each handled by the blocks that run on two XCDs or one, so that
  *               an XCD's L2 holds its slice of both tables; two launches and a float of partial dot product per
- *               pair and slice (by name: H*sizeof(elem)/8 must be 64..1024 bytes, a power of two; wider rows are
+ *               pair and slice (by name: H*sizeof(elem)/8 must be 64..1024 bytes, a power of two -- AUTO takes any slice of 5 to 64 times 16 bytes too; wider rows are
  *               taken in up to 64 column blocks of that form, one pair of launches per block, [8 * blocks][T][k] floats).
  *               Rows beyond 8 KiB exist for SPLIT only, and AUTO is SPLIT for them.
  *               AUTO chooses between GATHER and SPLIT from a measured grid, by the tokens (rows of up to 1 KiB), the
