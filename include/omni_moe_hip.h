@@ -293,6 +293,16 @@ OMNI_API int32_t omni_router_norm_bwd_padded(const void* dgates, const void* gat
                                              int32_t num_experts_per_token, int32_t dtype, int32_t training, void* workspace,
                                              void* stream);
 
+/* omni_expert_bwd_scores, and behind its token pass omni_router_norm_bwd (padded 0) or omni_router_norm_bwd_padded (1) from its d(gates), as one call whose
+ * stages share launches where they do not depend on each other.  gates, dgates: routing_weights and drouting_weights of the former.
+ *   workspace : omni_expert_router_bwd_workspace_bytes() bytes */
+OMNI_API size_t omni_expert_router_bwd_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_expert_sqrt,
+                                                       int32_t num_experts_per_token, int32_t dtype);
+OMNI_API int32_t omni_expert_router_bwd(const void* dy, const void* x, const void* up_weight, const void* down_weight, const void* gates, const int32_t* indices,
+                                        const float* scores, const void* z, const float* stats, void* dx, void* dup_weight, void* ddown_weight, void* dgates,
+                                        void* dz, int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_expert_sqrt,
+                                        int32_t num_experts_per_token, int32_t dtype, int32_t training, int32_t padded, void* workspace, void* stream);
+
 /* Backward of the shared MLP (omni_mlp_fwd), with the router projection's share of the same products: what autograd does in the reference for
  * the matmuls of interface.py:23-29 and omni_moe.py:70-71 and the SwiGLU function between them (omni_mlp.py:306-356).
  *   dy, x [T,H]; gate_weight, up_weight [I,H]; down_weight [H,I]; gate, up, h [T,I] as omni_swiglu_linear_save_fwd left them

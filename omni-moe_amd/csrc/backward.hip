@@ -86,19 +86,32 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_bwd_kernel(
 // A token's k slots are walked one after the other (a fixed order of the sums), each slot's id and gradient handed to all lanes by
 // v_readlane; what bounds the pass is that chain, so a wave takes few tokens while there are waves to spare (4096 tokens, 64 keys, k = 16:
 // eight tokens a wave and ds_bpermute exchanges 29 us).
+// Two launches in training: the blocks that finish d(z) add the column sums of their 64 columns themselves, 512 bytes from each block of the first launch, of
+// which there are few (4096 tokens: 256).  Reads nothing that the experts' weight pass leaves, so the layer's backward puts the first
+// launch beside that pass's fix-up (expert_bwd_weight_fixup_kernel).
 static inline int norm_tokens_per_wave(int64_t num_tokens) {
   const int64_t t = num_tokens / (kBwdWavesPerBlock * 512);
   return (int)(t < 1 ? 1 : t > 8 ? 8 : t);
 }
+struct RouterPass {
+  const void *dgates, *gates;
+  const int32_t* ids;
+  const void* z;
+  const float* stats;
+  void* dz;
+  float* partials;                   // training: column sums [block][S1x, S2x, S1y, S2y][r]
+  int num_tokens, r, top_k, training, tokens_per_wave, dz_half;
+};
+// waves of a block: eight, or four where a lane has more than four columns of each half (the sums' LDS).  Sixteen put them on half as many CUs: fix-up and
+// router's first launch 13.9 us at 4096 tokens, eight 12.2
+constexpr int norm_waves(int cols) { return cols <= 4 ? 8 : kBwdWavesPerBlock; }
 
 template <int DT, int R>
-__global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kernel(
-    const void* __restrict__ dgates, const void* __restrict__ gates, const int32_t* __restrict__ ids,
-    const void* __restrict__ z, const float* __restrict__ stats, void* __restrict__ dz, float* __restrict__ partials,
-    int num_tokens, int r, int top_k, int training, int tokens_per_wave, int dz_half) {
-  __shared__ float red[kBwdWavesPerBlock][4][R * kWave];       // per wave: S1x, S2x, S1y, S2y by column
-  const int lane = lane_id(), wave = threadIdx.x >> 6;
-  const int first = __builtin_amdgcn_readfirstlane((blockIdx.x * kBwdWavesPerBlock + wave) * tokens_per_wave);
+__device__ __forceinline__ void router_norm_bwd_block(const RouterPass& p, const int block) {
+  constexpr int W = norm_waves(R);
+  __shared__ float red[W][4][R * kWave];                       // per wave: S1x, S2x, S1y, S2y by column
+  const int lane = lane_id(), wave = threadIdx.x >> 6, r = p.r;
+  const int first = __builtin_amdgcn_readfirstlane((block * W + wave) * p.tokens_per_wave);
   float s1[2][R], s2[2][R];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -110,24 +123,51 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kern
 #pragma unroll
     for (int a = 0; a < R; ++a) {
       const int key = a * kWave + lane;
-      mean[h][a] = key < r ? stats[(2 * h) * r + key] : 0.f;
-      rstd[h][a] = key < r ? stats[(2 * h + 1) * r + key] : 0.f;
+      mean[h][a] = key < r ? p.stats[(2 * h) * r + key] : 0.f;
+      rstd[h][a] = key < r ? p.stats[(2 * h + 1) * r + key] : 0.f;
     }
-  for (int t = first; t < min(first + tokens_per_wave, num_tokens); ++t) {
+  // What a token's sums start from, requested ahead of the one before it: the chain of slots then waits for memory once
+  float zv[2][R], my_dg, my_gate;
+  int my_slot;
+  auto request = [&](int t) __attribute__((always_inline)) {
+    const int j = min(lane, p.top_k - 1);
+    const int64_t base = int64_t(t) * p.top_k;
+    my_slot = p.top_k ? p.ids[base + j] : -1;
+    my_dg = p.top_k ? Elem<DT>::load(p.dgates, base + j) : 0.f;
+    my_gate = p.top_k ? Elem<DT>::load(p.gates, base + j) : 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int a = 0; a < R; ++a) zv[h][a] = Elem<DT>::load(p.z, int64_t(t) * 2 * r + h * r + min(a * kWave + lane, r - 1));
+  };
+  const int last = min(first + p.tokens_per_wave, p.num_tokens);
+  if (first < last) request(first);
+  for (int t = first; t < last; ++t) {
+    float zt[2][R];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int a = 0; a < R; ++a) zt[h][a] = zv[h][a];
+    int slot = my_slot;
+    float dg = my_dg, gate = my_gate;
+    if (t + 1 < last) request(t + 1);
     // d(l): scatter of the slot gradients, fp32 sums in slot order, one rounding
     float dl[2][R];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int a = 0; a < R; ++a) dl[h][a] = 0.f;
-    const int64_t base = int64_t(t) * top_k;
-    for (int j0 = 0; j0 < top_k; j0 += kWave) {
-      const int j = j0 + lane;
-      const int my_id = j < top_k ? ids[base + j] : -1;
-      const float my_ds = j < top_k ? Elem<DT>::round(Elem<DT>::load(dgates, base + j) * Elem<DT>::load(gates, base + j)) : 0.f;
-      const bool ok = (uint32_t)my_id < (uint32_t)r * (uint32_t)r;
-      const int my_ix = ok ? my_id / r : -1, my_iy = ok ? my_id - my_ix * r : -1;
-      const int n = min(kWave, top_k - j0);
+    for (int j0 = 0; j0 < p.top_k; j0 += kWave) {
+      if (j0 > 0) {                                             // k <= 128: a second round
+        const int64_t at = int64_t(t) * p.top_k + min(j0 + lane, p.top_k - 1);
+        slot = p.ids[at];
+        dg = Elem<DT>::load(p.dgates, at);
+        gate = Elem<DT>::load(p.gates, at);
+      }
+      const float my_ds = Elem<DT>::round(dg * gate);
+      const bool ok = j0 + lane < p.top_k && (uint32_t)slot < (uint32_t)r * (uint32_t)r;
+      const int my_ix = ok ? slot / r : -1, my_iy = ok ? slot - my_ix * r : -1;
+      const int n = min(kWave, p.top_k - j0);
       for (int i = 0; i < n; ++i) {
         const int ix = __builtin_amdgcn_readlane(my_ix, i), iy = __builtin_amdgcn_readlane(my_iy, i);
         const float ds = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ds), i));
@@ -146,8 +186,7 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kern
 #pragma unroll
       for (int a = 0; a < R; ++a) {
         const int key = a * kWave + lane;
-        const float zv = key < r ? Elem<DT>::load(z, int64_t(t) * 2 * r + h * r + key) : 0.f;
-        nhat[a] = (zv - mean[h][a]) * rstd[h][a];
+        nhat[a] = (zt[h][a] - mean[h][a]) * rstd[h][a];
         l[a] = key < r ? Elem<DT>::round(nhat[a]) : -INFINITY;
         m = fmaxf(m, l[a]);
       }
@@ -167,18 +206,18 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kern
       for (int a = 0; a < R; ++a) {
         const int key = a * kWave + lane;
         if (key >= r) {
-          if (key < dz_half) Elem<DT>::store(dz, (int64_t(t) * 2 + h) * dz_half + key, 0.f);
+          if (key < p.dz_half) Elem<DT>::store(p.dz, (int64_t(t) * 2 + h) * p.dz_half + key, 0.f);
           continue;
         }
-        const float p = expf(Elem<DT>::round(l[a] - m - lse));
-        const float dn = Elem<DT>::round(dl[h][a] - p * sum_dl);
+        const float prob = expf(Elem<DT>::round(l[a] - m - lse));
+        const float dn = Elem<DT>::round(dl[h][a] - prob * sum_dl);
         s1[h][a] += dn;
         s2[h][a] += dn * nhat[a];
-        Elem<DT>::store(dz, (int64_t(t) * 2 + h) * dz_half + key, training ? dn : dn * rstd[h][a]);
+        Elem<DT>::store(p.dz, (int64_t(t) * 2 + h) * p.dz_half + key, p.training ? dn : dn * rstd[h][a]);
       }
     }
   }
-  if (!training) return;
+  if (!p.training) return;
   // column sums of the block: waves in order through LDS, then one row of partials per block
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -188,44 +227,68 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_kern
       red[wave][2 * h + 1][a * kWave + lane] = s2[h][a];
     }
   __syncthreads();
-  for (int i = threadIdx.x; i < 4 * R * kWave; i += kBwdWavesPerBlock * kWave) {
+  for (int i = threadIdx.x; i < 4 * R * kWave; i += W * kWave) {
     const int q = i / (R * kWave), col = i % (R * kWave);
     if (col >= r) continue;
     float acc = 0.f;
 #pragma unroll
-    for (int w = 0; w < kBwdWavesPerBlock; ++w) acc += red[w][q][col];
-    partials[(int64_t(blockIdx.x) * 4 + q) * r + col] = acc;     // [block][S1x, S2x, S1y, S2y][r]
+    for (int w = 0; w < W; ++w) acc += red[w][q][col];
+    p.partials[(int64_t(block) * 4 + q) * r + col] = acc;
   }
 }
-
-// means[q][col] = sum over blocks of partials / T; one wave per (q, col)
-__global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_norm_bwd_sums_kernel(
-    const float* __restrict__ partials, float* __restrict__ means, int blocks, int r, int num_tokens) {
-  const int lane = lane_id();
-  const int idx = blockIdx.x * kBwdWavesPerBlock + (threadIdx.x >> 6);      // q * r + col
-  if (idx >= 4 * r) return;
-  double acc = 0.;
-  for (int b = lane; b < blocks; b += kWave) acc += (double)partials[int64_t(b) * 4 * r + idx];
-#pragma unroll
-  for (int m = kWave / 2; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, kWave);
-  if (lane == 0) means[idx] = (float)(acc / (double)num_tokens);
+template <int DT, int R>
+__global__ __launch_bounds__(norm_waves(R)* kWave) void router_norm_bwd_kernel(const RouterPass p) {
+  router_norm_bwd_block<DT, R>(p, (int)blockIdx.x);
 }
 
-// dz = rstd (dn - mean(dn) - nhat mean(dn nhat)), element-wise over [T, 2r]; dn is read from dz.  A row of 2r values to a row of `per_block`
-// thread rows, so that no value needs a division.
+// dz = rstd (dn - mean(dn) - nhat mean(dn nhat)); dn is read from dz.  Blocks alternate between the groups of 64 columns of a half; a block adds its columns'
+// sums over the `rows` partials in double, sixteen waves side by side, while its first tokens' values are on their way.
+constexpr int kFinishWaves = 16, kFinishRows = 4;               // tokens that a wave has in flight
 template <int DT>
-__global__ __launch_bounds__(256) void router_norm_bwd_finish_kernel(const void* __restrict__ z, const float* __restrict__ stats,
-                                                                    const float* __restrict__ means, void* __restrict__ dz,
-                                                                    int num_tokens, int r, int width, int dz_half) {
-  const int per_block = 256 / width, row = threadIdx.x / width, c0 = threadIdx.x % width;     // width: a power of two up to 256
-  for (int c = c0; c < 2 * r; c += width) {
-    const int h = c >= r, key = c - h * r;
-    const float mu = stats[(2 * h) * r + key], rs = stats[(2 * h + 1) * r + key], m1 = means[(2 * h) * r + key], m2 = means[(2 * h + 1) * r + key];
-    for (int t = blockIdx.x * per_block + row; t < num_tokens; t += gridDim.x * per_block) {
-      const float nhat = (Elem<DT>::load(z, (int64_t)t * 2 * r + c) - mu) * rs;
-      const int64_t at = ((int64_t)t * 2 + h) * dz_half + key;
-      const float dn = Elem<DT>::load(dz, at);
-      Elem<DT>::store(dz, at, rs * (dn - m1 - nhat * m2));
+__global__ __launch_bounds__(kFinishWaves* kWave) void router_norm_bwd_finish_kernel(const RouterPass p, const int rows) {
+  __shared__ double sums[2][kFinishWaves][kWave];
+  __shared__ float means[2][kWave];
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = p.r, per_half = (r + kWave - 1) / kWave, groups = 2 * per_half;
+  const int group = (int)blockIdx.x % groups, part = (int)blockIdx.x / groups, parts = (int)gridDim.x / groups;
+  const int h = group / per_half, col = (group - h * per_half) * kWave + lane, key = min(col, r - 1);
+  const bool live = col < r;
+  float zv[kFinishRows], dn[kFinishRows];
+  auto at = [&](int t) __attribute__((always_inline)) { return ((int64_t)t * 2 + h) * p.dz_half + key; };
+  auto request = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kFinishRows; ++i) {
+      const int t = min(t0 + i * kFinishWaves, p.num_tokens - 1);
+      zv[i] = Elem<DT>::load(p.z, ((int64_t)t * 2 + h) * r + key);
+      dn[i] = Elem<DT>::load(p.dz, at(t));
+    }
+  };
+  constexpr int kStep = kFinishWaves * kFinishRows;
+  request(part * kStep + wave);
+  const float mu = p.stats[(2 * h) * r + key], rs = p.stats[(2 * h + 1) * r + key];
+  double a1 = 0., a2 = 0.;
+#pragma unroll 4
+  for (int b = wave; b < rows; b += kFinishWaves) {
+    const float* row = p.partials + ((int64_t)b * 4 + 2 * h) * r + key;
+    a1 += (double)row[0];
+    a2 += (double)row[r];
+  }
+  sums[0][wave][lane] = a1;
+  sums[1][wave][lane] = a2;
+  __syncthreads();
+  if (wave < 2) {
+    double acc = 0.;
+#pragma unroll
+    for (int w = 0; w < kFinishWaves; ++w) acc += sums[wave][w][lane];
+    means[wave][lane] = (float)(acc / (double)p.num_tokens);
+  }
+  __syncthreads();
+  const float m1 = means[0][lane], m2 = means[1][lane];
+  for (int t0 = part * kStep + wave; t0 < p.num_tokens; t0 += parts * kStep) {
+    if (t0 != part * kStep + wave) request(t0);
+#pragma unroll
+    for (int i = 0; i < kFinishRows; ++i) {
+      const int t = t0 + i * kFinishWaves;
+      if (live && t < p.num_tokens) Elem<DT>::store(p.dz, at(t), rs * (dn[i] - m1 - (zv[i] - mu) * rs * m2));
     }
   }
 }
@@ -524,13 +587,22 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_weight
 // One wave per expert: zero rows for an expert nobody selected; for a segment that crosses a chunk
 // border the sum of its partial rows, first chunk to last.  A segment inside one chunk was
 // stored by the pass above.
-template <int DT, int NCH>
-__global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void expert_bwd_weight_fixup_kernel(
+// R > 0: the launch's first `router_blocks` blocks are the router's (R columns of a half to a lane), which only needs the token pass in front of it: a layer's
+// backward of 4096 tokens x 1024, 64 keys, k = 16 took 7.4 us for the fix-up and 8.2 + 5.0 + 4.1 for the router's three launches behind it; both in one launch
+// 12.2, and 7.0 to finish (1000 tokens x 512, k = 8: 3.8 + 4.9 + 3.6 + 2.8 -> 4.6 + 5.5).
+template <int DT, int NCH, int R>
+__global__ __launch_bounds__((R ? norm_waves(R) : kBwdWavesPerBlock) * kWave) void expert_bwd_weight_fixup_kernel(
     const int32_t* __restrict__ offsets, const float* __restrict__ partials, uint8_t* __restrict__ dup,
-    uint8_t* __restrict__ ddown, int64_t num_experts, int hidden, int chunk) {
-  constexpr int E = Row16<DT>::kElems;
+    uint8_t* __restrict__ ddown, int64_t num_experts, int hidden, int chunk, const RouterPass router, const int router_blocks) {
+  constexpr int E = Row16<DT>::kElems, W = R ? norm_waves(R) : kBwdWavesPerBlock;
+  if constexpr (R > 0) {
+    if ((int)blockIdx.x < router_blocks) {
+      router_norm_bwd_block<DT, R>(router, (int)blockIdx.x);
+      return;
+    }
+  }
   const int lane = lane_id();
-  const int64_t e = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kBwdWavesPerBlock + (threadIdx.x >> 6)));
+  const int64_t e = __builtin_amdgcn_readfirstlane((int)(((int)blockIdx.x - router_blocks) * W + (int)(threadIdx.x >> 6)));
   if (e >= num_experts) return;
   const int begin = offsets[e], end = offsets[e + 1];
   const int c0 = begin / chunk, c1 = end > begin ? (end - 1) / chunk : c0;
@@ -666,9 +738,31 @@ static hipError_t launch_token_gather(TokenPass p, const SortPass* sort, hipStre
   return start_token<kKernel>(p, sort, kSortScatter, blocks(p.last - p.first, kTokenWaves), s);
 }
 
+// The router's share of a backward pass: blocks of its first launch, and its launches
+static int norm_blocks(int64_t num_tokens, int r) {
+  const int64_t per_block = (int64_t)norm_waves((r + kWave - 1) / kWave) * norm_tokens_per_wave(num_tokens);
+  return (int)((num_tokens + per_block - 1) / per_block);
+}
+template <int DT>
+static hipError_t launch_norm_first(const RouterPass& p, hipStream_t s) {
+  const unsigned blocks = (unsigned)norm_blocks(p.num_tokens, p.r);
+  if (p.r <= kWave) hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 1>), dim3(blocks), dim3(norm_waves(1) * kWave), 0, s, p);
+  else if (p.r <= 4 * kWave) hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 4>), dim3(blocks), dim3(norm_waves(4) * kWave), 0, s, p);
+  else hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 16>), dim3(blocks), dim3(norm_waves(16) * kWave), 0, s, p);
+  return hipGetLastError();
+}
+template <int DT>
+static hipError_t launch_norm_finish(const RouterPass& p, hipStream_t s) {
+  if (!p.training) return hipSuccess;
+  // a CU's block for every group of columns, or fewer where 64 tokens to a block are all
+  const int groups = 2 * ((p.r + kWave - 1) / kWave), want = (p.num_tokens + kFinishWaves * kFinishRows - 1) / (kFinishWaves * kFinishRows), most = groups < 256 ? 256 / groups : 1;
+  hipLaunchKernelGGL(router_norm_bwd_finish_kernel<DT>, dim3((unsigned)(groups * (want < most ? want : most))), dim3(kFinishWaves * kWave), 0, s, p, norm_blocks(p.num_tokens, p.r));
+  return hipGetLastError();
+}
+
 template <int DT, int NCH, int G>
 static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, void* dup, void* ddown, const int32_t* offsets, const int32_t* pair_ids,
-                                    const int32_t* token_ids, float* partials, hipStream_t s) {
+                                    const int32_t* token_ids, float* partials, const RouterPass* router, hipStream_t s) {
   const int64_t T = p.num_tokens, N = p.num_experts;
   const int H = p.hidden, k = p.top_k;
   const hipError_t te = p.lanes ? launch_token_split<DT>(p, sort, s) : launch_token_gather<DT, NCH, G>(p, sort, s);
@@ -683,10 +777,25 @@ static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, vo
                        p.ids, offsets, pair_ids, token_ids, (uint8_t*)dup, (uint8_t*)ddown, partials, N, H, chunk, num_chunks);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
-  dim3 grid((unsigned)((N + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock));
-  hipLaunchKernelGGL((expert_bwd_weight_fixup_kernel<DT, NCH>), grid, block, 0, s, offsets, partials, (uint8_t*)dup,
-                     (uint8_t*)ddown, N, H, chunk);
-  return hipGetLastError();
+  // Rows of up to 4 KiB (16-bit 2048 columns), and up to four columns of a half to a lane: the router's first launch beside the fix-up
+  const bool beside = router && NCH <= 4 && router->r <= 4 * kWave;
+  auto fixup = [&](auto cols, int router_blocks) {
+    constexpr int R = decltype(cols)::value, W = R ? norm_waves(R) : kBwdWavesPerBlock;
+    hipLaunchKernelGGL((expert_bwd_weight_fixup_kernel<DT, NCH, R>), dim3((unsigned)(router_blocks + (N + W - 1) / W)), dim3(W * kWave), 0, s, offsets, partials, (uint8_t*)dup,
+                       (uint8_t*)ddown, N, H, chunk, router ? *router : RouterPass{}, router_blocks);
+    return hipGetLastError();
+  };
+  hipError_t e;
+  if constexpr (NCH <= 4) {
+    if (beside) e = router->r <= kWave ? fixup(std::integral_constant<int, 1>{}, norm_blocks(T, router->r)) : fixup(std::integral_constant<int, 4>{}, norm_blocks(T, router->r));
+    else e = fixup(std::integral_constant<int, 0>{}, 0);
+  } else {
+    e = fixup(std::integral_constant<int, 0>{}, 0);
+  }
+  if (e != hipSuccess || !router) return e;
+  if (!beside)
+    if ((e = launch_norm_first<DT>(*router, s)) != hipSuccess) return e;
+  return launch_norm_finish<DT>(*router, s);
 }
 
 }  // namespace omni
@@ -717,23 +826,17 @@ extern "C" OMNI_API int32_t omni_router_bwd(const void* dscores, const int32_t* 
   return to_code(hipGetLastError());
 }
 
-// workspace of omni_router_norm_bwd: per-block column sums [blocks][4][r] f32 | means [4][r] f32
-static inline int norm_bwd_blocks(int64_t num_tokens) {
-  const int64_t per_block = (int64_t)omni::kBwdWavesPerBlock * omni::norm_tokens_per_wave(num_tokens);
-  return (int)((num_tokens + per_block - 1) / per_block);
-}
-
+// workspace of omni_router_norm_bwd: per-block column sums [blocks][4][r] f32
 extern "C" OMNI_API size_t omni_router_norm_bwd_workspace_bytes(int64_t num_tokens, int32_t num_expert_sqrt) {
   using namespace omni;
   if (num_tokens < 0 || num_expert_sqrt <= 0) return 0;
-  return up256((size_t)norm_bwd_blocks(num_tokens) * 4 * num_expert_sqrt * 4) + up256((size_t)4 * num_expert_sqrt * 4);
+  return up256((size_t)norm_blocks(num_tokens, num_expert_sqrt) * 4 * num_expert_sqrt * 4);
 }
 
-static int32_t router_norm_bwd(const void* dgates, const void* gates, const int32_t* indices, const void* z, const float* stats, void* dz,
-                               int64_t num_tokens, int32_t num_expert_sqrt, int32_t num_experts_per_token, int32_t dtype, int32_t training,
-                               void* workspace, void* stream, int dz_half) {
+// Checks the arguments and fills p; num_tokens 0: nothing to do
+static int32_t router_pass(omni::RouterPass& p, const void* dgates, const void* gates, const int32_t* indices, const void* z, const float* stats, void* dz, int64_t num_tokens,
+                           int r, int k, int32_t dtype, int32_t training, void* workspace, bool padded) {
   using namespace omni;
-  const int r = num_expert_sqrt, k = num_experts_per_token;
   if (num_tokens < 0 || num_tokens > INT32_MAX / 4096 || r <= 0 || k < 0) return OMNI_ERR_SHAPE;
   if (r > 1024) return OMNI_ERR_UNSUPPORTED;
   if (k > 128) return OMNI_ERR_TOPK;
@@ -741,50 +844,39 @@ static int32_t router_norm_bwd(const void* dgates, const void* gates, const int3
   if (num_tokens == 0) return OMNI_OK;
   if (!z || !stats || !dz || (k > 0 && (!dgates || !gates || !indices))) return OMNI_ERR_NULL;
   if (training && !workspace) return OMNI_ERR_WORKSPACE;
+  p = RouterPass{dgates, gates, indices, z, stats, dz, (float*)workspace, (int)num_tokens, r, k, training, norm_tokens_per_wave(num_tokens), padded ? (r + 7) / 8 * 8 : r};
+  return OMNI_OK;
+}
+static int32_t router_norm_bwd(const void* dgates, const void* gates, const int32_t* indices, const void* z, const float* stats, void* dz,
+                               int64_t num_tokens, int32_t num_expert_sqrt, int32_t num_experts_per_token, int32_t dtype, int32_t training,
+                               void* workspace, void* stream, bool padded) {
+  using namespace omni;
+  RouterPass p;
+  if (int e = router_pass(p, dgates, gates, indices, z, stats, dz, num_tokens, num_expert_sqrt, num_experts_per_token, dtype, training, workspace, padded)) return e;
+  if (num_tokens == 0) return OMNI_OK;
   hipStream_t s = (hipStream_t)stream;
-  const int T = (int)num_tokens, blocks = norm_bwd_blocks(num_tokens);
-  const int per_wave = norm_tokens_per_wave(num_tokens);
-  int width = 32;
-  while (width < 256 && width < 2 * r) width *= 2;
-  float* partials = (float*)workspace;
-  float* means = training ? (float*)((char*)workspace + up256((size_t)blocks * 4 * r * 4)) : nullptr;
-  dim3 block(kBwdWavesPerBlock * kWave);
-#define OMNI_NORM_CASE(DT)                                                                                                    \
-  do {                                                                                                                        \
-    if (r <= 64) hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 1>), dim3(blocks), block, 0, s, dgates, gates, indices, z,     \
-                                    stats, dz, partials, T, r, k, training, per_wave, dz_half);                                                   \
-    else if (r <= 256) hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 4>), dim3(blocks), block, 0, s, dgates, gates, indices,  \
-                                          z, stats, dz, partials, T, r, k, training, per_wave, dz_half);                                          \
-    else hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 16>), dim3(blocks), block, 0, s, dgates, gates, indices, z, stats, dz, \
-                            partials, T, r, k, training, per_wave, dz_half);                                                                      \
-    if (training) {                                                                                                           \
-      hipLaunchKernelGGL(router_norm_bwd_sums_kernel, dim3((4 * r + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock), block, 0, s,  \
-                         partials, means, blocks, r, T);                                                                       \
-      const int want = (T + 256 / width - 1) / (256 / width);                                                                  \
-      hipLaunchKernelGGL(router_norm_bwd_finish_kernel<DT>, dim3((unsigned)(want < 1024 ? want : 1024)), dim3(256), 0, s, z,   \
-                         stats, means, dz, T, r, width, dz_half);                                                              \
-    }                                                                                                                         \
-  } while (0)
-  if (dtype == OMNI_BF16) OMNI_NORM_CASE(kBF16);
-  else if (dtype == OMNI_F16) OMNI_NORM_CASE(kF16);
-  else OMNI_NORM_CASE(kF32);
-#undef OMNI_NORM_CASE
-  return to_code(hipGetLastError());
+  auto go = [&](auto dt) {
+    constexpr int DT = decltype(dt)::value;
+    const hipError_t e = launch_norm_first<DT>(p, s);
+    return to_code(e != hipSuccess ? e : launch_norm_finish<DT>(p, s));
+  };
+  if (dtype == OMNI_BF16) return go(std::integral_constant<int, kBF16>{});
+  if (dtype == OMNI_F16) return go(std::integral_constant<int, kF16>{});
+  return go(std::integral_constant<int, kF32>{});
 }
 
 extern "C" OMNI_API int32_t omni_router_norm_bwd(const void* dgates, const void* gates, const int32_t* indices, const void* z,
                                                  const float* stats, void* dz, int64_t num_tokens, int32_t num_expert_sqrt,
                                                  int32_t num_experts_per_token, int32_t dtype, int32_t training, void* workspace,
                                                  void* stream) {
-  return router_norm_bwd(dgates, gates, indices, z, stats, dz, num_tokens, num_expert_sqrt, num_experts_per_token, dtype, training, workspace, stream, num_expert_sqrt);
+  return router_norm_bwd(dgates, gates, indices, z, stats, dz, num_tokens, num_expert_sqrt, num_experts_per_token, dtype, training, workspace, stream, false);
 }
 
 extern "C" OMNI_API int32_t omni_router_norm_bwd_padded(const void* dgates, const void* gates, const int32_t* indices, const void* z,
                                                         const float* stats, void* dz, int64_t num_tokens, int32_t num_expert_sqrt,
                                                         int32_t num_experts_per_token, int32_t dtype, int32_t training, void* workspace,
                                                         void* stream) {
-  return router_norm_bwd(dgates, gates, indices, z, stats, dz, num_tokens, num_expert_sqrt, num_experts_per_token, dtype, training, workspace, stream,
-                         (num_expert_sqrt + 7) / 8 * 8);
+  return router_norm_bwd(dgates, gates, indices, z, stats, dz, num_tokens, num_expert_sqrt, num_experts_per_token, dtype, training, workspace, stream, true);
 }
 
 namespace omni {
@@ -825,10 +917,11 @@ extern "C" OMNI_API int32_t omni_expert_bwd(const void* dy, const void* x, const
                                 num_experts, num_experts_per_token, dtype, workspace, stream);
 }
 
-extern "C" OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x, const void* up_weight, const void* down_weight, const void* routing_weights,
-                                                   const int32_t* indices, const float* scores, void* dx, void* dup_weight, void* ddown_weight, void* drouting_weights,
-                                                   int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_experts_per_token, int32_t dtype,
-                                                   void* workspace, void* stream) {
+// router: NULL, or the router's share, enqueued behind the token pass
+static int32_t expert_bwd(const void* dy, const void* x, const void* up_weight, const void* down_weight, const void* routing_weights,
+                          const int32_t* indices, const float* scores, void* dx, void* dup_weight, void* ddown_weight, void* drouting_weights,
+                          int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_experts_per_token, int32_t dtype,
+                          void* workspace, void* stream, const omni::RouterPass* router) {
   using namespace omni;
   if (num_tokens < 0 || hidden_size <= 0 || num_experts <= 0 || num_experts_per_token < 0) return OMNI_ERR_SHAPE;
   if (num_tokens > INT32_MAX / 2 || num_experts > INT32_MAX / 2 ||
@@ -872,7 +965,7 @@ extern "C" OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x
                     drouting_weights, ds, coef, partial_a, partial_s, 0, (int)num_tokens, (int)num_tokens, hidden_size, num_experts_per_token,
                     lanes, slices, (uint32_t)num_experts};
   hipError_t err;
-#define OMNI_BWD_ARGS p, beside ? &pass : nullptr, dup_weight, ddown_weight, offsets, pair_ids, token_ids, partials, s
+#define OMNI_BWD_ARGS p, beside ? &pass : nullptr, dup_weight, ddown_weight, offsets, pair_ids, token_ids, partials, router, s
 #define OMNI_BWD_CASE(DT)                                                      \
   do {                                                                         \
     if (nch <= 1) err = launch_expert_bwd<DT, 1, 8>(OMNI_BWD_ARGS);            \
@@ -886,6 +979,32 @@ extern "C" OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x
 #undef OMNI_BWD_ARGS
 #undef OMNI_BWD_CASE
   return to_code(err);
+}
+
+extern "C" OMNI_API int32_t omni_expert_bwd_scores(const void* dy, const void* x, const void* up_weight, const void* down_weight, const void* routing_weights,
+                                                   const int32_t* indices, const float* scores, void* dx, void* dup_weight, void* ddown_weight, void* drouting_weights,
+                                                   int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_experts_per_token, int32_t dtype,
+                                                   void* workspace, void* stream) {
+  return expert_bwd(dy, x, up_weight, down_weight, routing_weights, indices, scores, dx, dup_weight, ddown_weight, drouting_weights, num_tokens, hidden_size, num_experts,
+                    num_experts_per_token, dtype, workspace, stream, nullptr);
+}
+
+extern "C" OMNI_API size_t omni_expert_router_bwd_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_expert_sqrt,
+                                                                  int32_t num_experts_per_token, int32_t dtype) {
+  return omni::up256(omni_expert_bwd_workspace_bytes(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype)) +
+         omni_router_norm_bwd_workspace_bytes(num_tokens, num_expert_sqrt);
+}
+extern "C" OMNI_API int32_t omni_expert_router_bwd(const void* dy, const void* x, const void* up_weight, const void* down_weight, const void* gates, const int32_t* indices,
+                                                   const float* scores, const void* z, const float* stats, void* dx, void* dup_weight, void* ddown_weight, void* dgates,
+                                                   void* dz, int64_t num_tokens, int32_t hidden_size, int64_t num_experts, int32_t num_expert_sqrt,
+                                                   int32_t num_experts_per_token, int32_t dtype, int32_t training, int32_t padded, void* workspace, void* stream) {
+  using namespace omni;
+  if (!workspace) return OMNI_ERR_WORKSPACE;
+  RouterPass p;
+  void* const sums = (char*)workspace + up256(omni_expert_bwd_workspace_bytes(num_tokens, hidden_size, num_experts, num_experts_per_token, dtype));
+  if (int e = router_pass(p, dgates, gates, indices, z, stats, dz, num_tokens, num_expert_sqrt, num_experts_per_token, dtype, training, sums, padded != 0)) return e;
+  return expert_bwd(dy, x, up_weight, down_weight, gates, indices, scores, dx, dup_weight, ddown_weight, dgates, num_tokens, hidden_size, num_experts, num_experts_per_token,
+                    dtype, workspace, stream, num_tokens ? &p : nullptr);
 }
 
 static int32_t swiglu_launch(bool bwd, const void* dout, const void* gate, const void* up, void* out0, void* out1,

@@ -290,25 +290,29 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
     const int64_t rp = own ? (r + 7) / 8 * 8 : r;
     const Kept at(T, H, I, N, r, k, dt);
     const uint8_t* saved = (const uint8_t*)ptr(kept);
-    // temporaries: the experts' d(x), d(gates), d(z), and one workspace for three stages that follow one another on the stream
+    // temporaries: the experts' d(x), d(gates), d(z), and one workspace for two stages that follow one another on the stream
     Slab t;
     const size_t es = own ? 2 : 4, dx_at = t.add((size_t)(T * H) * es), dg_at = t.add((size_t)(T * k) * es), dz_at = t.add(router ? (size_t)(T * 2 * rp) * es : 0);
-    const size_t ws_at = t.add(std::max({omni_expert_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt), router ? omni_router_norm_bwd_workspace_bytes(T, (int32_t)r) : 0,
-                                         own ? omni_mlp_bwd_workspace_bytes(T, (int32_t)H, (int32_t)I, (int32_t)r, dt) : 0}));
+    const size_t ws_at = t.add(std::max(router ? omni_expert_router_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)r, (int32_t)k, dt)
+                                               : omni_expert_bwd_workspace_bytes(T, (int32_t)H, N, (int32_t)k, dt),
+                                        own ? omni_mlp_bwd_workspace_bytes(T, (int32_t)H, (int32_t)I, (int32_t)r, dt) : 0));
     const Tensor temp = bytes(t.size, x3.device());
     uint8_t* w = (uint8_t*)ptr(temp);
-    // experts, then the router stage behind their gates' gradient
+    // experts, and the router stage behind their gates' gradient
     Tensor dup = at::empty_like(up), ddown = at::empty_like(down);
-    check(omni_expert_bwd_scores(ptr(dy), ptr(x3), ptr(up), ptr(down), saved + at.gates, (const int32_t*)(saved + at.ids), at.scored ? (const float*)(saved + at.scores) : nullptr, w + dx_at, ptr(dup),
-                                 ptr(ddown), w + dg_at, T, (int32_t)H, N, (int32_t)k, dt, w + ws_at, st), "omni_expert_bwd");
-    if (need[6]) out[6] = dup;
-    if (need[7]) out[7] = ddown;
+    const float* scores = at.scored ? (const float*)(saved + at.scores) : nullptr;
+    const int32_t* ids = (const int32_t*)(saved + at.ids);
     if (router) {
       const uint8_t* z = saved + at.router;
-      const float* stats = (const float*)(z + omni_router_workspace_stats_offset(T, (int32_t)r, dt));
-      check((own ? omni_router_norm_bwd_padded : omni_router_norm_bwd)(w + dg_at, saved + at.gates, (const int32_t*)(saved + at.ids), z, stats, w + dz_at, T, (int32_t)r,
-                                                                        (int32_t)k, dt, training ? 1 : 0, w + ws_at, st), "omni_router_norm_bwd");
+      check(omni_expert_router_bwd(ptr(dy), ptr(x3), ptr(up), ptr(down), saved + at.gates, ids, scores, z, (const float*)(z + omni_router_workspace_stats_offset(T, (int32_t)r, dt)),
+                                   w + dx_at, ptr(dup), ptr(ddown), w + dg_at, w + dz_at, T, (int32_t)H, N, (int32_t)r, (int32_t)k, dt, training ? 1 : 0, own ? 1 : 0, w + ws_at, st),
+            "omni_expert_router_bwd");
+    } else {
+      check(omni_expert_bwd_scores(ptr(dy), ptr(x3), ptr(up), ptr(down), saved + at.gates, ids, scores, w + dx_at, ptr(dup), ptr(ddown), w + dg_at, T, (int32_t)H, N, (int32_t)k, dt,
+                                   w + ws_at, st), "omni_expert_bwd");
     }
+    if (need[6]) out[6] = dup;
+    if (need[7]) out[7] = ddown;
     if (own) {
       const Tensor* like[6] = {&x3, &wg, &wu, &wd, &rx, &ry};
       for (int i = 0; i < 6; ++i)

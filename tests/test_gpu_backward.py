@@ -750,3 +750,42 @@ def test_router_norm_bwd_padded(case, training, device):
     assert torch.isfinite(packed).all()
     assert torch.equal(padded[:, :, :r], packed)
     assert (padded[:, :, r:] == 0).all()
+
+
+@pytest.mark.parametrize("training", [True, False], ids=["train", "eval"])
+@pytest.mark.parametrize("case", [(1, 64, 64, 8, 8, "bf16"), (300, 256, 1024, 32, 8, "f16"), (1037, 1024, 289, 17, 16, "bf16"), (4133, 512, 4225, 65, 4, "bf16"), (130, 64, 65536, 256, 32, "f32"),
+                                  (100, 256, 66049, 257, 16, "bf16"), (70, 4096, 64, 8, 6, "bf16"), (40, 64, 20000, 130, 128, "f32")], ids=lambda c: "T%d-H%d-N%d-r%d-k%d-%s" % c)
+def test_expert_router_bwd_is_the_two_operators(case, training, device):
+    """The launches that the experts' and the router's backward share give every bit that each gives alone, in the packed and the padded layout: edges of the
+    blocks' tokens and of 64 columns, more than 64 slots, and the sizes (257 keys, rows beyond 4 KiB) at which nothing is shared."""
+    from omni_moe.ops.hip import _lib
+    lib = _lib.load()
+    T, H, N, r, k, name = case
+    dtype = dict(bf16=torch.bfloat16, f16=torch.float16, f32=torch.float32)[name]
+    dt = _lib.DTYPE_CODE[dtype]
+    g = torch.Generator(device=device).manual_seed(T + r)
+
+    def normal(*shape, std=1.0):
+        return torch.empty(*shape, device=device).normal_(0, std, generator=g).to(dtype)
+    dy, x, up, down, z = normal(T, H), normal(T, H), normal(N, H, std=0.05), normal(N, H, std=0.05), normal(T, 2 * r)
+    gates = torch.empty(T, k, device=device).uniform_(0.1, 1, generator=g).to(dtype)
+    ids = torch.randint(0, r * r, (T, k), device=device, dtype=torch.int32, generator=g)
+    stats = torch.rand(4 * r, device=device, generator=g) + 0.5
+    stream = _lib.stream_ptr()
+    nan = float("nan")
+    for padded in (0, 1):
+        rp = (r + 7) // 8 * 8 if padded else r
+        outs = [[torch.full(s, nan, device=device, dtype=dtype) for s in ((T, H), (N, H), (N, H), (T, k), (T, 2, rp))] for _ in range(2)]
+        dx, du, dv, dg, dz = outs[0]
+        ws = torch.empty(max(lib.omni_expert_bwd_workspace_bytes(T, H, N, k, dt), lib.omni_router_norm_bwd_workspace_bytes(T, r)), device=device, dtype=torch.uint8)
+        _lib.check(lib.omni_expert_bwd(dy.data_ptr(), x.data_ptr(), up.data_ptr(), down.data_ptr(), gates.data_ptr(), ids.data_ptr(), dx.data_ptr(), du.data_ptr(), dv.data_ptr(),
+                                       dg.data_ptr(), T, H, N, k, dt, ws.data_ptr(), stream), "omni_expert_bwd")
+        _lib.check((lib.omni_router_norm_bwd_padded if padded else lib.omni_router_norm_bwd)(dg.data_ptr(), gates.data_ptr(), ids.data_ptr(), z.data_ptr(), stats.data_ptr(),
+                   dz.data_ptr(), T, r, k, dt, int(training), ws.data_ptr(), stream), "omni_router_norm_bwd")
+        dx, du, dv, dg, dz = outs[1]
+        ws = torch.empty(lib.omni_expert_router_bwd_workspace_bytes(T, H, N, r, k, dt), device=device, dtype=torch.uint8)
+        _lib.check(lib.omni_expert_router_bwd(dy.data_ptr(), x.data_ptr(), up.data_ptr(), down.data_ptr(), gates.data_ptr(), ids.data_ptr(), None, z.data_ptr(), stats.data_ptr(),
+                                              dx.data_ptr(), du.data_ptr(), dv.data_ptr(), dg.data_ptr(), dz.data_ptr(), T, H, N, r, k, dt, int(training), padded, ws.data_ptr(),
+                                              stream), "omni_expert_router_bwd")
+        for a, b, what in zip(outs[0], outs[1], ("dx", "dup", "ddown", "dgates", "dz")):
+            assert torch.isfinite(a).all() and torch.equal(a, b), (padded, what)
