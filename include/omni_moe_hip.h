@@ -399,6 +399,26 @@ OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_weight, const
                                    int32_t training, float momentum, float eps, void* workspace, void* stream,
                                    void* side_stream, void* fork_event, void* join_event, int32_t expert_algo);
 
+/* omni_moe_fwd for a differentiable call: the same result, and what the layer's backward pass reads stays with the caller.
+ *   router_workspace : omni_router_workspace_bytes() bytes, as omni_router_fwd leaves it (z, and the statistics at
+ *                      omni_router_workspace_stats_offset())
+ *   gates, indices   : [T,k]; scores: NULL, or [T,k] fp32 for the pair scores (where omni_expert_bwd_reads_scores())
+ *   gate, up, h      : [T,I], the rounded projections and their SwiGLU product
+ *   workspace        : omni_moe_save_workspace_bytes() bytes; free again once the work has run.
+ * The expert algorithm is AUTO's; ids beyond the tables add nothing and are no error.  Replaces OmniMoE.forward under autograd (omni_moe.py:60-106). */
+OMNI_API size_t omni_moe_save_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int64_t num_experts,
+                                              int32_t num_experts_per_token, int32_t dtype);
+OMNI_API int32_t omni_moe_save_fwd(const void* x, const void* gate_weight, const void* up_weight, const void* down_weight,
+                                   const void* router_weight_x, const void* router_weight_y,
+                                   void* running_mean_x, void* running_var_x, int64_t* num_batches_tracked_x,
+                                   void* running_mean_y, void* running_var_y, int64_t* num_batches_tracked_y,
+                                   const void* up_embed, const void* down_embed, void* y,
+                                   void* router_workspace, void* gates, int32_t* indices, float* scores, void* gate, void* up, void* h,
+                                   int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int64_t num_experts,
+                                   int32_t num_expert_sqrt, int32_t num_experts_per_token, int32_t dtype, int32_t stats_dtype,
+                                   int32_t training, float momentum, float eps, void* workspace, void* stream,
+                                   void* side_stream, void* fork_event, void* join_event);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1157,7 +1157,7 @@ hipError_t launch_f32_joint(const void* x, const void* wx, const void* wy, void*
 
 namespace omni {
 // partial sums of whichever of the two projections is split along K (they are not alive together)
-static size_t mlp_sums_bytes(int64_t T, int64_t H, int64_t I, int dtype) {
+size_t mlp_sums_bytes(int64_t T, int64_t H, int64_t I, int dtype) {
   if (dtype == OMNI_F32 || I % 8 || H % 8) return 0;
   const size_t few = few_tokens_covers(T, H, I, dtype) ? few_tokens_parts_bytes(T, H, I) : 0;
   const size_t a = tile_workspace_bytes(kTileSwiglu, T, I, H), b = tile_workspace_bytes(kTileResidual, T, H, I), most = a > b ? a : b;
@@ -1166,32 +1166,27 @@ static size_t mlp_sums_bytes(int64_t T, int64_t H, int64_t I, int dtype) {
 static size_t mlp_h_bytes(int64_t T, int64_t I, int dtype) { return ((size_t)T * (size_t)I * (dtype == OMNI_F32 ? 4 : 2) + 255) / 256 * 256; }
 
 // The two projections of omni_mlp_fwd, each told whether it has the GPU to itself (the whole-layer call on two streams says no, which keeps
-// them off the form that holds every CU to the end).  `workspace`: omni_mlp_workspace_bytes(), h first.
-template <int DT>
-static int mlp_gate_up(const void* x, const void* wg, const void* wu, int64_t T, int64_t H, int64_t I, void* workspace, hipStream_t s, bool exclusive) {
-  return gemm_swiglu<DT>(x, wg, wu, workspace, T, I, H, s, nullptr, nullptr, exclusive, (char*)workspace + mlp_h_bytes(T, I, DT), mlp_sums_bytes(T, H, I, DT));
-}
-template <int DT>
-static int mlp_down(const void* wd, const void* residual, void* y, int64_t T, int64_t H, int64_t I, void* workspace, hipStream_t s, bool exclusive) {
-  return gemm_plain<DT>(workspace, wd, nullptr, residual, y, T, H, I, s, nullptr, nullptr, false, exclusive, (char*)workspace + mlp_h_bytes(T, I, DT), mlp_sums_bytes(T, H, I, DT));
-}
-int mlp_gate_up_impl(const void* x, const void* wg, const void* wu, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive) {
+// them off the form that holds every CU to the end).  sums: mlp_sums_bytes(); gate, up: NULL, or where the rounded projections go as well (16-bit types).
+int mlp_gate_up_impl(const void* x, const void* wg, const void* wu, void* h, void* gate, void* up, int64_t T, int32_t H, int32_t I, int32_t dtype, void* sums, void* stream,
+                     bool exclusive) {
   if (!x || !wg || !wu) return OMNI_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
+  const size_t n = mlp_sums_bytes(T, H, I, dtype);
   switch (dtype) {
-    case OMNI_BF16: return mlp_gate_up<kBF16>(x, wg, wu, T, H, I, workspace, s, exclusive);
-    case OMNI_F16: return mlp_gate_up<kF16>(x, wg, wu, T, H, I, workspace, s, exclusive);
-    case OMNI_F32: return mlp_gate_up<kF32>(x, wg, wu, T, H, I, workspace, s, exclusive);
+    case OMNI_BF16: return gemm_swiglu<kBF16>(x, wg, wu, h, T, I, H, s, gate, up, exclusive, sums, n);
+    case OMNI_F16: return gemm_swiglu<kF16>(x, wg, wu, h, T, I, H, s, gate, up, exclusive, sums, n);
+    case OMNI_F32: return gemm_swiglu<kF32>(x, wg, wu, h, T, I, H, s, gate, up, exclusive, sums, n);
     default: return OMNI_ERR_DTYPE;
   }
 }
-int mlp_down_impl(const void* wd, const void* residual, void* y, int64_t T, int32_t H, int32_t I, int32_t dtype, void* workspace, void* stream, bool exclusive) {
+int mlp_down_impl(const void* h, const void* wd, const void* residual, void* y, int64_t T, int32_t H, int32_t I, int32_t dtype, void* sums, void* stream, bool exclusive) {
   if (!wd || !y) return OMNI_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
+  const size_t n = mlp_sums_bytes(T, H, I, dtype);
   switch (dtype) {
-    case OMNI_BF16: return mlp_down<kBF16>(wd, residual, y, T, H, I, workspace, s, exclusive);
-    case OMNI_F16: return mlp_down<kF16>(wd, residual, y, T, H, I, workspace, s, exclusive);
-    case OMNI_F32: return mlp_down<kF32>(wd, residual, y, T, H, I, workspace, s, exclusive);
+    case OMNI_BF16: return gemm_plain<kBF16>(h, wd, nullptr, residual, y, T, H, I, s, nullptr, nullptr, false, exclusive, sums, n);
+    case OMNI_F16: return gemm_plain<kF16>(h, wd, nullptr, residual, y, T, H, I, s, nullptr, nullptr, false, exclusive, sums, n);
+    case OMNI_F32: return gemm_plain<kF32>(h, wd, nullptr, residual, y, T, H, I, s, nullptr, nullptr, false, exclusive, sums, n);
     default: return OMNI_ERR_DTYPE;
   }
 }
@@ -1224,8 +1219,9 @@ extern "C" OMNI_API int32_t omni_mlp_fwd(const void* x, const void* gate_weight,
       return he == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)he;
     }
   }
-  if ((e = mlp_gate_up_impl(x, gate_weight, up_weight, num_tokens, hidden_size, intermediate_size, dtype, workspace, stream, true))) return e;
-  return mlp_down_impl(down_weight, residual, y, num_tokens, hidden_size, intermediate_size, dtype, workspace, stream, true);
+  void* const sums = (char*)workspace + mlp_h_bytes(num_tokens, intermediate_size, dtype);
+  if ((e = mlp_gate_up_impl(x, gate_weight, up_weight, workspace, nullptr, nullptr, num_tokens, hidden_size, intermediate_size, dtype, sums, stream, true))) return e;
+  return mlp_down_impl(workspace, down_weight, residual, y, num_tokens, hidden_size, intermediate_size, dtype, sums, stream, true);
 }
 
 namespace omni {

@@ -746,9 +746,9 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
     if (g.select.part_mean) {                                  // batch statistics: the block merges them first
       extern __shared__ __align__(16) uint8_t lds[];
       merge_statistics(g.select, (float*)lds, kWaves * kWave);
-      count_batch(g.select);
       stats = (const float*)lds;
     }
+    count_batch(g.select);
     auto select = [&](auto cells) {
       constexpr int C = decltype(cells)::value;
       if (g.regs <= 1) select_packed<DT, 1, C>(g.select, first, all, stats);

@@ -219,6 +219,7 @@ struct Layer {
   Tensor wg, wu, wd, rx, ry, up, down;
   Norms norms;
   int64_t H = 0, I = 0, N = 0, r = 0, k = 0;
+  void *side = nullptr, *fork = nullptr, *join = nullptr;      // the second stream and its events, where the call takes one
 };
 
 // What the forward pass leaves for the backward one, in ONE allocation (as are the backward pass's temporaries): a step of 1000 tokens with
@@ -252,21 +253,17 @@ struct LayerFn : public torch::autograd::Function<LayerFn> {
                         const Tensor& up, const Tensor& down, const Layer& l) {
     const int64_t T = x.numel() / l.H;
     const int dt = dtype_code(x.scalar_type());
-    void* s = stream_of(x.device());
     const Kept at(T, l.H, l.I, l.N, l.r, l.k, dt);
     const Tensor kept = bytes(at.s.size, x.device());
     uint8_t* k = (uint8_t*)ptr(kept);
-    router_forward(x, T, l.H, rx, ry, l.norms, l.k, k + at.gates, k + at.ids, k + at.router);
-    const Tensor e = expert_forward(x, T, up, down, k + at.gates, k + at.ids, l.k, OMNI_EXPERT_ALGO_AUTO, at.scored ? k + at.scores : nullptr);
-    if (dt != OMNI_F32) {                          // (rows of 16 bytes, so both sizes are multiples of 8; operands at any address)
-      check(omni_swiglu_linear_save_fwd(ptr(x), ptr(wg), ptr(wu), k + at.h, k + at.gate, k + at.up, T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_swiglu_linear_save_fwd");
-    } else {
-      check(omni_linear_fwd(ptr(x), ptr(wg), nullptr, k + at.gate, T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_linear_fwd");
-      check(omni_linear_fwd(ptr(x), ptr(wu), nullptr, k + at.up, T, (int32_t)l.H, (int32_t)l.I, dt, s), "omni_linear_fwd");
-      check(omni_swiglu_fwd(k + at.gate, k + at.up, k + at.h, T * l.I, dt, s), "omni_swiglu_fwd");
-    }
-    Tensor y = at::empty_like(x);
-    check(omni_linear_fwd(k + at.h, ptr(wd), ptr(e), ptr(y), T, (int32_t)l.I, (int32_t)l.H, dt, s), "omni_linear_fwd");
+    // given back at the end of the call: the current stream waits for a side branch, as below
+    const Tensor ws = bytes(omni_moe_save_workspace_bytes(T, (int32_t)l.H, (int32_t)l.I, l.N, (int32_t)l.k, dt), x.device());
+    Tensor y = at::empty(x.sizes(), x.options());
+    const Norms& b = l.norms;
+    check(omni_moe_save_fwd(ptr(x), ptr(wg), ptr(wu), ptr(wd), ptr(rx), ptr(ry), ptr(b.rmx), ptr(b.rvx), (int64_t*)ptr(b.nbx), ptr(b.rmy), ptr(b.rvy), (int64_t*)ptr(b.nby), ptr(up),
+                            ptr(down), ptr(y), k + at.router, k + at.gates, (int32_t*)(k + at.ids), at.scored ? (float*)(k + at.scores) : nullptr, k + at.gate, k + at.up, k + at.h, T,
+                            (int32_t)l.H, (int32_t)l.I, l.N, (int32_t)l.r, (int32_t)l.k, dt, dtype_code(b.rmx.scalar_type()), b.training ? 1 : 0, (float)b.momentum, (float)b.eps,
+                            ptr(ws), stream_of(x.device()), l.side, l.fork, l.join), "omni_moe_save_fwd");
     ctx->save_for_backward({x, wg, wu, wd, rx, ry, up, down, kept});
     ctx->saved_data["training"] = l.norms.training;
     ctx->saved_data["top_k"] = l.k;
@@ -408,6 +405,15 @@ py::object layer_forward(py::handle self, const Tensor& x, const py::dict& algos
   if (x.size(2) != l.H || T == 0 || !is(l.wg, {l.I, l.H}) || !is(l.wu, {l.I, l.H}) || !is(l.wd, {l.H, l.I}) || !is(l.rx, {l.r, l.H}) || !is(l.ry, {l.r, l.H}) ||
       !is(l.up, {l.N, l.H}) || !is(l.down, {l.N, l.H}) || l.k < 0 || l.k > l.r * l.r || l.k > 128 || l.k % 2 || !b.fits(x, l.r, T) || !prepare(x.device()))
     return py::none();
+  const py::object overlap = py::reinterpret_steal<py::object>(PyObject_GetAttr(self.ptr(), n.overlap)), low = py::reinterpret_steal<py::object>(PyObject_GetAttr(self.ptr(), n.min_work)),
+                   high = py::reinterpret_steal<py::object>(PyObject_GetAttr(self.ptr(), n.max_work)), name = py::reinterpret_steal<py::object>(PyObject_GetAttr(self.ptr(), n.algo));
+  if (!overlap || !low || !high || !name) throw py::error_already_set();
+  const double work = (double)T * (double)l.H * (double)l.I;
+  if (PyObject_IsTrue(overlap.ptr()) == 1 && low.cast<double>() < work && work < high.cast<double>()) {
+    const py::tuple res = self.attr(py::handle(n.resources))(py::cast(x.device()));
+    auto handle = [](py::handle o, PyObject* attr) { return (void*)(uintptr_t)o.attr(py::handle(attr)).cast<uint64_t>(); };
+    l.side = handle(res[0], n.cuda_stream); l.fork = handle(res[1], n.cuda_event); l.join = handle(res[2], n.cuda_event);
+  }
   if (records({&x, &l.wg, &l.wu, &l.wd, &l.rx, &l.ry, &l.up, &l.down})) {
     Tensor y;
     {
@@ -417,19 +423,9 @@ py::object layer_forward(py::handle self, const Tensor& x, const py::dict& algos
     }
     return py::cast(y);
   }
-  const py::object overlap = py::reinterpret_steal<py::object>(PyObject_GetAttr(self.ptr(), n.overlap)), low = py::reinterpret_steal<py::object>(PyObject_GetAttr(self.ptr(), n.min_work)),
-                   high = py::reinterpret_steal<py::object>(PyObject_GetAttr(self.ptr(), n.max_work)), name = py::reinterpret_steal<py::object>(PyObject_GetAttr(self.ptr(), n.algo));
-  if (!overlap || !low || !high || !name) throw py::error_already_set();
   PyObject* algo_code = PyDict_GetItemWithError(algos.ptr(), name.ptr());
   if (!algo_code) { PyErr_Clear(); return py::none(); }
   const int algo = (int)PyLong_AsLong(algo_code);
-  const double work = (double)T * (double)l.H * (double)l.I;
-  void *side = nullptr, *fork = nullptr, *join = nullptr;
-  if (PyObject_IsTrue(overlap.ptr()) == 1 && low.cast<double>() < work && work < high.cast<double>()) {
-    const py::tuple res = self.attr(py::handle(n.resources))(py::cast(x.device()));
-    auto handle = [](py::handle o, PyObject* attr) { return (void*)(uintptr_t)o.attr(py::handle(attr)).cast<uint64_t>(); };
-    side = handle(res[0], n.cuda_stream); fork = handle(res[1], n.cuda_event); join = handle(res[2], n.cuda_event);
-  }
   Tensor y;
   {
     py::gil_scoped_release nogil;
@@ -442,7 +438,7 @@ py::object layer_forward(py::handle self, const Tensor& x, const py::dict& algos
     Tensor ws = bytes(omni_moe_workspace_bytes_algo(T, (int32_t)l.H, (int32_t)l.I, l.N, (int32_t)l.r, (int32_t)l.k, dt, algo), x.device());
     check(omni_moe_fwd_algo(ptr(x), ptr(l.wg), ptr(l.wu), ptr(l.wd), ptr(l.rx), ptr(l.ry), ptr(b.rmx), ptr(b.rvx), (int64_t*)ptr(b.nbx), ptr(b.rmy), ptr(b.rvy),
                             (int64_t*)ptr(b.nby), ptr(l.up), ptr(l.down), ptr(y), T, (int32_t)l.H, (int32_t)l.I, l.N, (int32_t)l.r, (int32_t)l.k, dt,
-                            dtype_code(b.rmx.scalar_type()), b.training ? 1 : 0, (float)b.momentum, (float)b.eps, ptr(ws), stream_of(x.device()), side, fork, join, algo),
+                            dtype_code(b.rmx.scalar_type()), b.training ? 1 : 0, (float)b.momentum, (float)b.eps, ptr(ws), stream_of(x.device()), l.side, l.fork, l.join, algo),
           "omni_moe_fwd_algo");
   }
   return py::cast(y);
