@@ -19,7 +19,7 @@ LIB_PATH = os.path.join(HERE, "libomni_moe_hip.so")
 NATIVE_PATH = os.path.join(HERE, "_native.so")
 OBJ_DIR = os.path.join(PKG_ROOT, "build")
 
-SOURCES = ["gemm.hip", "gemm_tiles.hip", "router.hip", "expert.hip", "backward.hip", "schedule.hip", "layer.hip", "few_tokens.hip", "mlp_bwd.hip", "api.hip"]
+SOURCES = ["gemm.hip", "gemm_tiles.hip", "gemm_tiles_bf16.hip", "gemm_tiles_f16.hip", "router.hip", "expert.hip", "backward.hip", "schedule.hip", "layer.hip", "few_tokens.hip", "mlp_bwd.hip", "api.hip"]
 
 # packed-fp32 VALU forms are switched off for all device code of this library
 HIPCC_FLAGS = [
