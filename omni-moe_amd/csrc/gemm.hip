@@ -16,6 +16,7 @@
 // block's waves share out the K tiles.
 // The weight fragment is the MFMA's first operand, so an accumulator lane holds 4 consecutive
 // output columns of one row; two lanes pair up to store 8 columns (16 bytes) each.
+#include <algorithm>
 #include "common.h"
 #include "few_tokens.h"
 #include "gemm_tiles.h"
@@ -1160,8 +1161,7 @@ namespace omni {
 size_t mlp_sums_bytes(int64_t T, int64_t H, int64_t I, int dtype) {
   if (dtype == OMNI_F32 || I % 8 || H % 8) return 0;
   const size_t few = few_tokens_covers(T, H, I, dtype) ? few_tokens_parts_bytes(T, H, I) : 0;
-  const size_t a = tile_workspace_bytes(kTileSwiglu, T, I, H), b = tile_workspace_bytes(kTileResidual, T, H, I), most = a > b ? a : b;
-  return most > few ? most : few;
+  return std::max({few, tile_workspace_bytes(kTileSwiglu, T, I, H), tile_workspace_bytes(kTileResidual, T, H, I), tile_down_workspace_bytes(T, H, I)});
 }
 static size_t mlp_h_bytes(int64_t T, int64_t I, int dtype) { return ((size_t)T * (size_t)I * (dtype == OMNI_F32 ? 4 : 2) + 255) / 256 * 256; }
 

@@ -49,8 +49,6 @@ struct TileSingle {
 hipError_t launch_tile_group(int dtype, int layout, int epilogue, TileGroup& g, void* ws, size_t ws_bytes, hipStream_t s, bool exclusive = true);
 // What launch_tile_group wants for one product; K: the sum of its segments, each rounded up to 64
 size_t tile_workspace_bytes(int epilogue, int64_t M, int64_t N, int64_t K);
-// What it expects one product to take
-float tile_estimate_us(int epilogue, int64_t M, int64_t N, int64_t K, bool may_split);
 
 // The layer's joint launches.  The router's projection (kTileTwo) in front of the gate/up projection (kTileSwiglu, nothing kept), both kNT over the same
 // K; false, and nothing launched, where its tiles would cost a round of their own or the operands are out of reach.
@@ -58,6 +56,7 @@ bool launch_tile_pair(int dtype, const TileProduct& router, const TileProduct& m
 // The down projection (kTilePlain, kNT) and, beside it, the selection, if there is room (*selected).  *parts > 1: its sums are left in ws, [parts][M][N] fp32.
 struct SelectArgs;
 constexpr int kMostDownParts = 8;
+size_t tile_down_workspace_bytes(int64_t M, int64_t N, int64_t K);               // (what it wants in ws)
 hipError_t launch_tile_down(int dtype, const TileProduct& p, const SelectArgs& select, void* ws, size_t ws_bytes, hipStream_t s, bool* selected, int* parts);
 
 }  // namespace omni

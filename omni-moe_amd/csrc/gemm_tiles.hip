@@ -3,11 +3,23 @@
 
 namespace omni {
 
-// The fastest shape and K split by the figures above.  K is split for a product on its own only, where every part keeps 256 of K, and the 64 x 64
+// (joint: those that share their launch with the layer's router)
+constexpr unsigned kAnyShape = (1u << kShapes) - 1, kJointShapes = 1u << 1 | 1u << 2 | 1u << 3 | 1u << 4 | 1u << 7 | 1u << 8;
+
+// Microseconds that a launch of n blocks of one shape takes for 64 of K.  Where two blocks share a CU, the CUs with two set the time however few they are
+// (gate/up of 613 x 1024 x 4096 on 128 x 128 tiles, 320 blocks: 19.7 us; 450 rows, 256 blocks: 16.4; 1000 rows, 512 blocks: 21.4).
+static float step_us(const ShapeCost& c, int64_t n) {
+  constexpr int kCus = 256;
+  const int64_t rounds = (n + c.at_once - 1) / c.at_once;
+  const float used = n >= c.at_once ? 1.f : n > kCus ? 0.86f + 0.14f * (float)(n - kCus) / (c.at_once - kCus) : (float)n / c.at_once;
+  return (float)rounds * (c.idle + (c.full - c.idle) * used);
+}
+// The fastest shape and K split by those figures.  K is split for a product on its own only, where every part keeps 256 of K, and the 64 x 64
 // shape (whose two groups also split K) is for K >= 512: shorter sums stay in one order whatever the shape.
-static TileChoice choose_tiles(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split) {
+static TileChoice choose_of(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes) {
   TileChoice best;
   for (int i = 0; i < kShapes; ++i) {
+    if (!(shapes >> i & 1)) continue;
     const ShapeCost& c = i == 4 && epilogue == kTileSwiglu ? kSwigluCost : kCost[i];
     if (c.kg > 1 && K < 512) continue;
     const int bn = epilogue == kTileSwiglu ? c.bn / 2 : c.bn;
@@ -16,26 +28,47 @@ static TileChoice choose_tiles(int epilogue, const TileSize* sizes, int count, i
     const int64_t kt = (K + 63) / 64;
     for (int s = 1; s <= (may_split && count == 1 ? kMostSplits : 1); ++s) {
       if (s > 1 && kt / s < 4) break;
-      const int64_t n = tiles * s, rounds = (n + c.at_once - 1) / c.at_once;
-      const float used = n >= c.at_once ? 1.f : (float)n / c.at_once;
-      float us = c.fixed + (float)(rounds * ((kt + s - 1) / s)) * (c.idle + (c.full - c.idle) * used);
+      float us = c.fixed + (float)((kt + s - 1) / s) * step_us(c, tiles * s);
       if (s > 1) us += kReduceUs + (float)s * (float)sizes[0].M * (float)(epilogue == kTileSwiglu ? 2 * sizes[0].N : sizes[0].N) * 4.f * (1.f / kPartsOut + 1.f / kPartsIn);
       if (us < best.us) best = TileChoice{i, s, us};
     }
   }
   return best;
 }
+// A call asks for its workspace and then for its launches, a program for the same sizes over and over, and a choice takes 0.6 us: a layer of one token,
+// bound by the host, asked eight times.  Each thread keeps the last few products' choices, which nothing but the sizes goes into.
+static TileChoice choose_tiles(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes = kAnyShape) {
+  if (count != 1) return choose_of(epilogue, sizes, count, K, may_split, shapes);
+  struct Kept { int64_t M, N, K; uint64_t how; TileChoice choice; };
+  constexpr int kKept = 16;
+  static thread_local Kept kept[kKept];                        // (M = 0: none)
+  static thread_local int oldest = 0;
+  const uint64_t how = (uint64_t)shapes << 8 | (uint64_t)epilogue << 1 | (may_split ? 1 : 0);
+  for (const Kept& k : kept)
+    if (k.M == sizes->M && k.N == sizes->N && k.K == K && k.how == how) return k.choice;
+  Kept& k = kept[oldest];
+  oldest = (oldest + 1) % kKept;
+  k = Kept{sizes->M, sizes->N, K, how, choose_of(epilogue, sizes, count, K, may_split, shapes)};
+  return k.choice;
+}
+
+// The layer's down projection: a shape that takes the selection beside it, unless another one gains more than the selection's own launch costs
+static TileChoice choose_down(const TileSize& size, int64_t K, bool may_split) {
+  constexpr float kSelectUs = 6.f;
+  const TileChoice any = choose_tiles(kTilePlain, &size, 1, K, may_split), joint = choose_tiles(kTilePlain, &size, 1, K, may_split, kJointShapes);
+  return joint.us <= any.us + kSelectUs ? joint : any;
+}
+static size_t parts_bytes(const TileChoice& c, int64_t M, int64_t columns) { return c.splits > 1 ? (size_t)c.splits * (size_t)M * (size_t)columns * 4 : 0; }
 
 size_t tile_workspace_bytes(int epilogue, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const TileSize size{M, N};
   const TileChoice c = choose_tiles(epilogue, &size, 1, K, true);
-  return c.splits > 1 ? (size_t)c.splits * (size_t)M * (size_t)(epilogue == kTileSwiglu ? 2 * N : N) * 4 : 0;
+  return parts_bytes(c, M, epilogue == kTileSwiglu ? 2 * N : N);
 }
-
-float tile_estimate_us(int epilogue, int64_t M, int64_t N, int64_t K, bool may_split) {
-  const TileSize size{M, N};
-  return choose_tiles(epilogue, &size, 1, K, may_split).us;
+size_t tile_down_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return parts_bytes(choose_down(TileSize{M, N}, K, true), M, N);
 }
 
 hipError_t launch_tile_group(int dtype, int layout, int epilogue, TileGroup& g, void* ws, size_t ws_bytes, hipStream_t s, bool exclusive) {
@@ -55,7 +88,7 @@ hipError_t launch_tile_group(int dtype, int layout, int epilogue, TileGroup& g, 
     K = k > K ? k : K;
   }
   TileChoice c = choose_tiles(epilogue, sizes, g.count, K, ws != nullptr);
-  if (c.splits > 1 && (size_t)c.splits * (size_t)g.p[0].M * (size_t)(epilogue == kTileSwiglu ? 2 * g.p[0].N : g.p[0].N) * 4 > ws_bytes)
+  if (parts_bytes(c, g.p[0].M, epilogue == kTileSwiglu ? 2 * (int64_t)g.p[0].N : g.p[0].N) > ws_bytes)
     c = choose_tiles(epilogue, sizes, g.count, K, false);
   if (dtype == kBF16) return tile_group_of<kBF16>(layout, epilogue, g, c, (float*)ws, exclusive, s);
   if (dtype == kF16) return tile_group_of<kF16>(layout, epilogue, g, c, (float*)ws, exclusive, s);
@@ -74,11 +107,12 @@ bool launch_tile_pair(int dtype, const TileProduct& router, const TileProduct& m
   const int64_t K = mlp.seg[0].K, kt = (K + 63) / 64;
   int shape = -1;
   float best = choose_tiles(kTileTwo, sizes, 1, K, false).us + choose_tiles(kTileSwiglu, sizes + 1, 1, K, true).us;
-  for (int i : {2, 3, 4}) {                                    // (256 x 256: 30.6 us at 1024 tokens, where the two launches take 25.8)
+  for (int i = 0; i < kShapes; ++i) {
+    if (!(kJointShapes >> i & 1)) continue;                    // (256 x 256: 30.6 us at 1024 tokens, where the two launches take 25.8)
     const ShapeCost &r = kCost[i], &m = i == 4 ? kSwigluCost : kCost[i];
     if (r.kg > 1 && K < 512) continue;
     const int64_t n = ((router.M + r.bm - 1) / r.bm) * ((router.N + r.bn - 1) / r.bn) + ((mlp.M + m.bm - 1) / m.bm) * ((mlp.N + m.bn / 2 - 1) / (m.bn / 2));
-    const float used = n >= m.at_once ? 1.f : (float)n / m.at_once, us = m.fixed + (float)((n + m.at_once - 1) / m.at_once * kt) * (m.idle + (m.full - m.idle) * used);
+    const float us = m.fixed + (float)kt * step_us(m, n);
     if (us < best) { best = us; shape = i; }
   }
   return dtype == kBF16 ? tile_pair_of<kBF16>(shape, g, s, e) : tile_pair_of<kF16>(shape, g, s, e);
@@ -87,8 +121,8 @@ bool launch_tile_pair(int dtype, const TileProduct& router, const TileProduct& m
 hipError_t launch_tile_down(int dtype, const TileProduct& p, const SelectArgs& select, void* ws, size_t ws_bytes, hipStream_t s, bool* selected, int* parts) {
   if ((dtype != kBF16 && dtype != kF16) || !in_reach(p)) return hipErrorInvalidValue;
   const TileSize size{p.M, p.N};
-  TileChoice c = choose_tiles(kTilePlain, &size, 1, p.seg[0].K, ws != nullptr);
-  if (c.splits > 1 && (size_t)c.splits * (size_t)p.M * (size_t)p.N * 4 > ws_bytes) c = choose_tiles(kTilePlain, &size, 1, p.seg[0].K, false);
+  TileChoice c = choose_down(size, p.seg[0].K, ws != nullptr);
+  if (parts_bytes(c, p.M, p.N) > ws_bytes) c = choose_down(size, p.seg[0].K, false);
   if (c.splits > kMostDownParts) c.splits = kMostDownParts;
   return dtype == kBF16 ? tile_down_of<kBF16>(p, select, c, (float*)ws, s, selected, parts) : tile_down_of<kF16>(p, select, c, (float*)ws, s, selected, parts);
 }

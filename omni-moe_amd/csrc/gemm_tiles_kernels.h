@@ -117,6 +117,16 @@ __device__ __forceinline__ void swiglu_bwd_word(const uint32_t o, const uint32_t
   du = pack16x2<DT>(u2[0], u2[1]);
 }
 
+// Rows of A that a stage holds: as many as the waves' loads bring in (all of them load alike), and a power of two where A's rows run along M
+// (the pieces of such a row change places by XOR).
+template <int LAY>
+constexpr int staged_rows(int rows, int waves) {
+  if (LAY != kTN) return (rows + 8 * waves - 1) / (8 * waves) * (8 * waves);
+  int up = 1;
+  while (up < rows) up *= 2;
+  return up;
+}
+
 // A block is KG groups of WM x WN waves; a wave owns TM x TN matrix tiles of 16 x 16.  The ring advances 64 * KG of K a step through NS stages;
 // group g multiplies the g-th 64 of each.  kTail: some segment's K is not a multiple of the ring step, and an operand's rows run along K.
 //
@@ -130,9 +140,10 @@ template <int DT, int LAY, int WM, int WN, int KG, int TM, int TN, int NS, int E
 __device__ __forceinline__ void tiles_block(const Group& g, const int block, const int blocks) {
   constexpr bool AC = LAY == kTN, BC = LAY != kNT;             // the operand's K index is its row
   constexpr int NW = WM * WN * KG, BM = WM * TM * 16, BN = WN * TN * 16, BNO = EPI == kTileSwiglu ? BN / 2 : BN;
-  constexpr int kABytes = BM * 128, kSub = (BM + BN) * 128, kStage = KG * kSub;
-  constexpr int PA = BM / 8 / NW, PB = BN / 8 / NW, LPT = KG * (PA + PB);     // 1 KiB load instructions per wave and ring step
-  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "the waves share the loads evenly");
+  constexpr int LM = staged_rows<LAY>(BM, NW);                 // A's rows in a stage, those behind the tile's unread
+  constexpr int kABytes = LM * 128, kSub = (LM + BN) * 128, kStage = KG * kSub;
+  constexpr int PA = LM / 8 / NW, PB = BN / 8 / NW, LPT = KG * (PA + PB);     // 1 KiB load instructions per wave and ring step
+  static_assert(LM % (8 * NW) == 0 && BN % (8 * NW) == 0, "the waves share the loads evenly");
   static_assert(TN % (EPI == kTileSwiglu ? 4 : 2) == 0 && TM % KG == 0, "the epilogue takes column tiles in pairs");
   constexpr int RA = AC ? 2 : 1, RB = BC ? 2 : 1;              // LDS reads per fragment
   using LdsPtr = __attribute__((address_space(3))) void*;
@@ -218,9 +229,9 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
     if constexpr (EPI == kTileTwo) f_half = scalar(N / 2 - fn0 - wave * 8);
     uint32_t a0, b0;
     if constexpr (AC) {
-      constexpr int W = BM / 8;
-      const int r = wave * (64 / W) + lane / W;
-      a0 = (uint32_t)(r * lda) + (uint32_t)((lane % W) ^ (piece_of(r, BM) << 1)) * 16;
+      constexpr int W = LM / 8;
+      const int r = wave * (64 / W) + lane / W, chunk = (lane % W) ^ (piece_of(r, LM) << 1);
+      a0 = BM < LM && chunk >= BM / 8 ? kOutside : (uint32_t)(r * lda) + (uint32_t)chunk * 16;
       f_amore = scalar(NW * (64 / W) * lda);
     } else {
       a0 = (uint32_t)((wave * 8 + (lane >> 3)) * lda) + (uint32_t)row_chunk * 16;
@@ -315,13 +326,13 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
 
   // ---- fragment reads.  Lane (r16 = lane % 16, g4 = lane / 16) takes the K values 32 ks + 8 g4 .. + 7 of row r16 of a 16-row tile.
   const int r16 = lane & 15, g4 = lane >> 4;
-  constexpr int kRowA = AC ? BM * 2 : 128, kRowB = BC ? BN * 2 : 128;
+  constexpr int kRowA = AC ? LM * 2 : 128, kRowB = BC ? BN * 2 : 128;
   uint32_t a_addr[AC ? TM : 2], b_addr[BC ? TN : 2];
   const uint32_t tr_row = (uint32_t)(8 * g4 + (r16 >> 2)), tr_in = (uint32_t)(r16 & 3) * 8;       // (piece_of() of the row is the same in every K step and part)
   const uint32_t my_base = lds_base + (uint32_t)kg * kSub;
   if constexpr (AC) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) a_addr[i] = my_base + tr_row * kRowA + (uint32_t)((wm * TM + i) ^ piece_of((int)tr_row, BM)) * 32 + tr_in;
+    for (int i = 0; i < TM; ++i) a_addr[i] = my_base + tr_row * kRowA + (uint32_t)((wm * TM + i) ^ piece_of((int)tr_row, LM)) * 32 + tr_in;
   } else {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) a_addr[ks] = my_base + (uint32_t)(wm * TM * 16 + r16) * 128 + (uint32_t)((4 * ks + g4) ^ (r16 >> 1)) * 16;
@@ -667,12 +678,22 @@ template <bool kSwiglu> struct Shape<2, kSwiglu> { enum { WM = 2, WN = 2, KG = 1
 template <bool kSwiglu> struct Shape<3, kSwiglu> { enum { WM = 2, WN = 2, KG = 1, TM = 4, TN = 4, NS = 4 }; };      // 128 x 128, one block to a CU
 template <> struct Shape<4, false> { enum { WM = 2, WN = 2, KG = 2, TM = 2, TN = 2, NS = 4 }; };                    // 64 x 64, two K groups, one block to a CU
 template <> struct Shape<4, true> { enum { WM = 2, WN = 2, KG = 2, TM = 2, TN = 4, NS = 3 }; };                     // (SwiGLU: 64 x 128, so that a wave holds two column tiles of gate)
-constexpr int kShapes = 5;
+// Lower tiles, for row counts that leave the last round of the ones above half empty
+template <bool kSwiglu> struct Shape<5, kSwiglu> { enum { WM = 2, WN = 4, KG = 1, TM = 7, TN = 4, NS = 2 }; };      // 224 x 256, one block to a CU
+template <bool kSwiglu> struct Shape<6, kSwiglu> { enum { WM = 2, WN = 4, KG = 1, TM = 6, TN = 4, NS = 2 }; };      // 192 x 256, one block to a CU
+template <bool kSwiglu> struct Shape<7, kSwiglu> { enum { WM = 4, WN = 2, KG = 1, TM = 3, TN = 4, NS = 3 }; };      // 192 x 128, one block to a CU
+template <bool kSwiglu> struct Shape<8, kSwiglu> { enum { WM = 2, WN = 2, KG = 1, TM = 3, TN = 4, NS = 4 }; };      // 96 x 128, one block to a CU
+constexpr int kShapes = 9;
 // ... and what a launch of n blocks takes, in microseconds per 64 of K and round of `at_once` blocks: idle + (full - idle) times the share of
-// the chip in use.  Measured on 256 x 256 x 4096 (few blocks) and 4096 x 4096 x 4096 (all CUs busy), bf16; about 4 us more for a launch.
+// the chip in use.  Measured on 256 x 256 x 4096 (few blocks) and 4096 x 4096 x 4096 (all CUs busy), the lower tiles and the 64 x 64 one over 57 products of
+// 300 to 12000 rows, bf16, where the rule's choice takes 0.4 % more than the best shape on average and 9 % at most; about 4 us more for a launch.
+// The lower tiles took, the best of the others / now: gate/up of 3000 x 1024 x 4096 (256 tiles of 256 columns a round) 49.5 / 45.4 us, 613 x 1024 x 4096
+// 17.4 / 15.2; down of 3000 x 4096 x 1024 31.9 / 29.4, 12000 x 1536 x 512 23.7 / 19.6; five weight gradients of 4096 tokens x 1024 x 4096 (200 tiles of
+// 256 rows, 236 of 224) 118 / 107.
 struct ShapeCost { int bm, bn, kg, at_once; float idle, full, fixed; };
-constexpr ShapeCost kCost[kShapes] = {{256, 256, 1, 256, 1.10f, 1.55f, 5.f}, {256, 128, 1, 256, 0.66f, 0.92f, 4.5f}, {128, 128, 1, 512, 0.50f, 0.97f, 4.f},
-                                      {128, 128, 1, 256, 0.44f, 0.57f, 4.f}, {64, 64, 2, 256, 0.20f, 0.235f, 4.f}};
+constexpr ShapeCost kCost[kShapes] = {{256, 256, 1, 256, 1.10f, 1.55f, 5.f}, {256, 128, 1, 256, 0.66f, 0.92f, 4.5f}, {128, 128, 1, 512, 0.50f, 1.00f, 4.f},
+                                      {128, 128, 1, 256, 0.44f, 0.57f, 4.f}, {64, 64, 2, 256, 0.16f, 0.235f, 4.f}, {224, 256, 1, 256, 1.04f, 1.44f, 5.f},
+                                      {192, 256, 1, 256, 0.92f, 1.26f, 5.f}, {192, 128, 1, 256, 0.52f, 0.70f, 4.5f}, {96, 128, 1, 256, 0.36f, 0.47f, 4.f}};
 constexpr ShapeCost kSwigluCost = {64, 128, 2, 256, 0.26f, 0.37f, 4.f};
 // A split writes its fp32 sums and a second kernel adds them: its launch, and the two trips
 constexpr float kReduceUs = 3.3f, kPartsOut = 8e6f, kPartsIn = 5e6f;      // us, bytes per us
@@ -683,7 +704,7 @@ struct TileSize { int64_t M, N; };
 template <int DT, int LAY, int kId, int EPI, bool kTail, bool kStream, class Group>
 struct TilesLds {
   using S = Shape<kId, EPI == kTileSwiglu>;
-  static constexpr int kBytes = S::NS * S::KG * (S::WM * S::TM * 16 + S::WN * S::TN * 16) * 128;
+  static constexpr int kBytes = S::NS * S::KG * (staged_rows<LAY>(S::WM * S::TM * 16, S::WM * S::WN * S::KG) + S::WN * S::TN * 16) * 128;
   static inline LdsKernel entry{(const void*)gemm_tiles_kernel<DT, LAY, S::WM, S::WN, S::KG, S::TM, S::TN, S::NS, EPI, kTail, kStream, Group>, kBytes};
 };
 template <int DT, int LAY, int kId, int EPI, bool kTail, bool kStream, class Group>
@@ -743,8 +764,9 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
 template <int kId, bool kSwiglu>
 constexpr int tile_lds() {
   using S = Shape<kId, kSwiglu>;
-  static_assert(S::NS * S::KG * (S::WM * S::TM * 16 + S::WN * S::TN * 16) * 128 >= 4 * merge_lds_floats(kMergeKeys, S::WM * S::WN * S::KG * 64), "a block that selects merges statistics there");
-  return S::NS * S::KG * (S::WM * S::TM * 16 + S::WN * S::TN * 16) * 128;
+  constexpr int kBytes = S::NS * S::KG * (staged_rows<kNT>(S::WM * S::TM * 16, S::WM * S::WN * S::KG) + S::WN * S::TN * 16) * 128;
+  static_assert(kBytes >= 4 * merge_lds_floats(kMergeKeys, S::WM * S::WN * S::KG * 64), "a block that selects merges statistics there");
+  return kBytes;
 }
 template <auto kKernel, int kBytes>
 struct JointLds { static inline LdsKernel entry{(const void*)kKernel, kBytes}; };
@@ -803,7 +825,7 @@ static hipError_t launch_tiles(TileGroup& g, float* ws, int splits, bool exclusi
   } else {
     if (g.count != 1) return hipErrorInvalidValue;
     const TileSingle one{{g.p[0]}};
-    if constexpr (LAY == kNT && kId == 0) {
+    if constexpr (LAY == kNT && (kId == 0 || kId == 5 || kId == 6)) {
       // one stream per CU where there are more tiles than CUs and nothing is meant to run beside the launch; else one block per tile, so
       // that CUs come free for other streams' kernels as blocks retire
       if (exclusive && blocks > 256 && splits == 1 && one.p[0].segments == 1)
@@ -828,7 +850,11 @@ static hipError_t launch_choice(TileGroup& g, const TileChoice& c, float* ws, bo
     case 1: return launch_tiles<DT, LAY, 1, EPI>(g, ws, c.splits, exclusive, s);
     case 2: return launch_tiles<DT, LAY, 2, EPI>(g, ws, c.splits, exclusive, s);
     case 3: return launch_tiles<DT, LAY, 3, EPI>(g, ws, c.splits, exclusive, s);
-    default: return launch_tiles<DT, LAY, 4, EPI>(g, ws, c.splits, exclusive, s);
+    case 4: return launch_tiles<DT, LAY, 4, EPI>(g, ws, c.splits, exclusive, s);
+    case 5: return launch_tiles<DT, LAY, 5, EPI>(g, ws, c.splits, exclusive, s);
+    case 6: return launch_tiles<DT, LAY, 6, EPI>(g, ws, c.splits, exclusive, s);
+    case 7: return launch_tiles<DT, LAY, 7, EPI>(g, ws, c.splits, exclusive, s);
+    default: return launch_tiles<DT, LAY, 8, EPI>(g, ws, c.splits, exclusive, s);
   }
 }
 
@@ -886,25 +912,31 @@ hipError_t tile_group_of(int layout, int epilogue, TileGroup& g, const TileChoic
 template <int DT>
 bool tile_pair_of(int shape, TilePair& g, hipStream_t s, hipError_t* e) {
   switch (shape) {
+    case 1: return start_pair<DT, 1>(g, s, e);
     case 2: return start_pair<DT, 2>(g, s, e);
     case 3: return start_pair<DT, 3>(g, s, e);
     case 4: return start_pair<DT, 4>(g, s, e);
+    case 7: return start_pair<DT, 7>(g, s, e);
+    case 8: return start_pair<DT, 8>(g, s, e);
     default: return false;
   }
 }
 template <int DT>
 hipError_t tile_down_of(const TileProduct& p, const SelectArgs& select, const TileChoice& c, float* ws, hipStream_t s, bool* selected, int* parts) {
   switch (c.shape) {
-    case 0: case 1: {                                          // whole CUs for a tile: nothing beside it
+    case 1: return start_down<DT, 1>(p, select, c.splits, ws, s, selected, parts);
+    case 2: return start_down<DT, 2>(p, select, c.splits, ws, s, selected, parts);
+    case 3: return start_down<DT, 3>(p, select, c.splits, ws, s, selected, parts);
+    case 4: return start_down<DT, 4>(p, select, c.splits, ws, s, selected, parts);
+    case 7: return start_down<DT, 7>(p, select, c.splits, ws, s, selected, parts);
+    case 8: return start_down<DT, 8>(p, select, c.splits, ws, s, selected, parts);
+    default: {                                                 // tiles of 256 columns: nothing beside them
       *selected = false;
       *parts = 1;
       TileGroup g;
       g.p[g.count++] = p;
       return launch_choice<DT, kNT, kTilePlain>(g, c, ws, true, s);
     }
-    case 2: return start_down<DT, 2>(p, select, c.splits, ws, s, selected, parts);
-    case 3: return start_down<DT, 3>(p, select, c.splits, ws, s, selected, parts);
-    default: return start_down<DT, 4>(p, select, c.splits, ws, s, selected, parts);
   }
 }
 // (each type's kernels are compiled in a file of their own)

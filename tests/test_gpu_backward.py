@@ -698,6 +698,31 @@ def test_mlp_bwd_matches_matmuls(case, dtype, device):
         assert (err.abs().max() <= 4 * ulp * w.abs().max()).item(), (name, (err.abs().max() / w.abs().max()).item())
 
 
+# T, H, I, r: products that take the tiles of 224, 192 and 96 rows: one row past a tile, one short of it and whole tiles; K tails; split K; more tiles than CUs
+LOWER_TILE_CASES = [(65, 136, 520, 17), (449, 136, 4104, 0), (673, 136, 6152, 17), (1537, 136, 4104, 17), (193, 776, 6152, 17), (3361, 264, 520, 8), (2497, 136, 6152, 0),
+                    (2015, 136, 6152, 17), (129, 512, 6152, 64), (200, 1024, 4096, 17), (1344, 264, 2568, 17), (3071, 512, 6144, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", LOWER_TILE_CASES, ids=lambda c: "T%d-H%d-I%d-r%d" % c)
+def test_mlp_on_lower_tiles(case, dtype, device):
+    """Both projections and their gradients against the same products in fp32.  gate, up and their product are rounded once each: half an ulp of each term, and of the
+    result, in the 2-norm; sums in another order are far below that."""
+    T, H, I, _ = case
+    g = torch.Generator(device=device).manual_seed(T * H)
+    n = lambda *s, std: torch.empty(*s, device=device).normal_(0, std, generator=g).to(dtype)
+    x, wg, wu, wd = n(T, H, std=1.0), n(I, H, std=H ** -0.5), n(I, H, std=H ** -0.5), n(H, I, std=I ** -0.5)
+    print(f"mlp on lower tiles T={T} H={H} I={I} {dtype}", flush=True)
+    gate, up = ((x.float() @ w.float().t()).to(dtype).float() for w in (wg, wu))
+    want = (torch.nn.functional.silu(gate) * up).to(dtype).float() @ wd.float().t()
+    err = _ops().hip_omni_mlp_func(x, wg, wu, wd).float() - want
+    eps = torch.finfo(dtype).eps
+    assert (err.norm() <= eps * want.norm()).item(), (err.norm() / want.norm()).item()
+    rows = err.norm(dim=1) / want.norm(dim=1)
+    assert (rows <= 2 * eps).all().item(), rows.max().item()
+    test_mlp_bwd_matches_matmuls(case, dtype, device)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("case", [(64, 512), (1000, 1024), (4100, 1024)], ids=lambda c: "T%d-H%d" % c)
 def test_mlp_bwd_swiglu_is_the_operator(case, dtype, device):

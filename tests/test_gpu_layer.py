@@ -806,6 +806,17 @@ def test_joint_launches_match_the_operators(case, dtype, device):
     assert (got - (mlp + experts)).abs().max().item() <= 4 * eps * max(1.0, float((mlp + experts).abs().max()))
 
 
+# T, H, I, N, k: the joint projections on tiles of 256, 192 and 96 rows of 128 columns, whole and one row past them; the down projection on 96 and 192 rows,
+# split along K and not, with the selection beside it
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", [(613, 1024, 4096, 4096, 16), (97, 136, 2056, 576, 8), (192, 264, 4104, 576, 8), (385, 264, 4104, 576, 8), (768, 776, 2568, 1024, 4),
+                                  (1153, 776, 2568, 576, 8), (1153, 264, 4104, 576, 6), (1200, 1024, 4096, 4096, 16), (1500, 1024, 4096, 1024, 8)],
+                         ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
+def test_joint_launches_on_lower_tiles(case, dtype, device):
+    test_joint_launches_match_the_operators(case, dtype, device)
+
+
+
 def test_layer_with_rows_beyond_the_tile_kernels_reach(device):
     """An intermediate size whose rows put 256 of them beyond 2 GiB: no joint launch, and the result of the operators one by one (MLP in 64 bits)."""
     from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
