@@ -484,101 +484,105 @@ __global__ __launch_bounds__(kSortThreads) void expert_bwd_accumulate_kernel(con
 // `partials[chunk][slot]`, slot 0 if the run starts the chunk, slot 1 otherwise (a chunk has at
 // most one of each); the fix-up kernel then adds an expert's partials in chunk order, so the
 // summation order is fixed and nothing is added atomically.
-template <int DT, int NCH, int G>
-__global__ __launch_bounds__(kBwdWavesPerBlock* kWave, 2) void expert_bwd_weight_kernel(
-    const uint8_t* __restrict__ x, const uint8_t* __restrict__ dy, const float* __restrict__ ds, const float* __restrict__ coef,
-    const int32_t* __restrict__ ids, const int32_t* __restrict__ offsets, const int32_t* __restrict__ sorted_pair_ids,
-    const int32_t* __restrict__ sorted_token_ids, uint8_t* __restrict__ dup, uint8_t* __restrict__ ddown,
-    float* __restrict__ partials, int64_t num_experts, int hidden, int chunk, int num_chunks) {
+//
+// Bound by the gathers: a row pair is read for every pair of the list.  What a wave owns is therefore a chunk of one PART of the columns: up to 1 KiB of
+// the rows of x (for dU) or of dy (for dV), 16 bytes to a lane, and the parts go to the XCDs one after another, so that an XCD gathers from the one or two
+// parts that its L2 holds; with whole rows of both in every wave, all of x and dy went through every L2 and the pass ran at the fabric's 7 TB/s.  A wave's row
+// address and factor are scalars, so a narrower part costs no exchange between lanes.  Rows of up to 512 bytes: x in the lower half of the lanes, dy in the
+// upper.  The chunks, and with them the order of all sums, do not depend on the parts.
+struct WeightPass {
+  const uint8_t *x, *dy;
+  const float *ds, *coef;
+  const int32_t *ids, *offsets, *pair_ids, *token_ids;
+  uint8_t *dup, *ddown;
+  float* partials;
+  int64_t num_experts;
+  int hidden, chunk, num_chunks;
+  int lanes, columns;                // 16-byte lanes of a part; parts of a row of x, and as many of dy (0: both in one part)
+  int blocks, per_xcd;               // blocks of a part; all parts' blocks on an XCD
+};
+template <int DT, bool PAIRED, int G>
+__global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void expert_bwd_weight_kernel(const WeightPass p) {
   constexpr int E = Row16<DT>::kElems;
   const int lane = lane_id();
-  const int ci = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kBwdWavesPerBlock + (threadIdx.x >> 6)));
-  if (ci >= num_chunks) return;
-  const int valid = offsets[num_experts];             // pairs with an id inside the table
-  const int first = ci * chunk, last = min(first + chunk, valid);
+  const int item = ((int)blockIdx.x % kXcds) * p.per_xcd + (int)blockIdx.x / kXcds, part = item / p.blocks;
+  if (part >= (PAIRED ? 1 : 2 * p.columns)) return;
+  const int ci = __builtin_amdgcn_readfirstlane((item - part * p.blocks) * kBwdWavesPerBlock + (int)(threadIdx.x >> 6));
+  if (ci >= p.num_chunks) return;
+  const int valid = p.offsets[p.num_experts];         // pairs with an id inside the table
+  const int first = ci * p.chunk, last = min(first + p.chunk, valid);
   if (first >= last) return;
-  const int64_t row_bytes = int64_t(hidden) * (16 / E);
+  const uint32_t row_bytes = (uint32_t)p.hidden * (16 / E);
 
-  bool live[NCH];
-  int64_t off[NCH];
-  float au[NCH][E], av[NCH][E];
+  const bool second = PAIRED ? lane >= kWave / 2 : part >= p.columns;           // of dy and dV
+  const int in_part = PAIRED ? lane % (kWave / 2) : lane, piece = (PAIRED ? 0 : (second ? part - p.columns : part) * p.lanes) + in_part;
+  const bool live = in_part < p.lanes && piece * E < p.hidden;
+  const uint32_t off = live ? piece * 16u : 0u;       // the other lanes read what the first one does, and store nothing
+  const uint8_t* const rows = second ? p.dy : p.x;
+  uint8_t* const out_rows = second ? p.ddown : p.dup;
+  const float* const factors = PAIRED ? p.ds : second ? p.coef : p.ds;
+  float acc[E];
 #pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    live[c] = (c * kWave + lane) * E < hidden;
-    off[c] = int64_t(c * kWave + lane) * 16;
-#pragma unroll
-    for (int i = 0; i < E; ++i) au[c][i] = av[c][i] = 0.f;
-  }
+  for (int i = 0; i < E; ++i) acc[i] = 0.f;
   // Ends the run [run_first, run_last) of expert e and clears the accumulators.  A run inside the chunk is its expert's whole segment; only the
-  // chunk's first and last run need a look at the pairs beyond it, and those ids are fetched ahead (the segment's offsets, asked for at each
-  // flush, were a wait for memory per run; with them gone and the indices of 64 pairs fetched at once, 32768 pairs over 16384 experts, hidden
-  // 1024: 24.7 -> 23.2 us).
-  const int before = first > 0 ? ids[sorted_pair_ids[first - 1]] : -1, after = last < valid ? ids[sorted_pair_ids[last]] : -1;
+  // chunk's first and last run need a look at the pairs beyond it, and those ids are fetched ahead.
+  const int before = first > 0 ? p.ids[p.pair_ids[first - 1]] : -1, after = last < valid ? p.ids[p.pair_ids[last]] : -1;
   auto flush = [&](int e, int run_first, int run_last) {
     const bool whole = (run_first != first || before != e) && (run_last != last || after != e);
-    if (whole) {
+    if (live) {
+      if (whole) {
+        *(u32x4_t*)(out_rows + (int64_t)e * row_bytes + off) = pack16<DT>(acc);
+      } else {
+        float* out = p.partials + (int64_t(ci) * 2 + (run_first == first ? 0 : 1)) * 2 * p.hidden + (second ? p.hidden : 0) + piece * E;
 #pragma unroll
-      for (int c = 0; c < NCH; ++c)
-        if (live[c]) {
-          *(u32x4_t*)(dup + e * row_bytes + off[c]) = pack16<DT>(au[c]);
-          *(u32x4_t*)(ddown + e * row_bytes + off[c]) = pack16<DT>(av[c]);
-        }
-    } else {
-      float* out = partials + (int64_t(ci) * 2 + (run_first == first ? 0 : 1)) * 2 * hidden;
-#pragma unroll
-      for (int c = 0; c < NCH; ++c)
-        if (live[c]) {
-          const int col = (c * kWave + lane) * E;
-#pragma unroll
-          for (int q = 0; q < E; q += 4) {
-            *(f32x4_t*)(out + col + q) = f32x4_t{au[c][q], au[c][q + 1], au[c][q + 2], au[c][q + 3]};
-            *(f32x4_t*)(out + hidden + col + q) = f32x4_t{av[c][q], av[c][q + 1], av[c][q + 2], av[c][q + 3]};
-          }
-        }
+        for (int q = 0; q < E; q += 4) *(f32x4_t*)(out + q) = f32x4_t{acc[q], acc[q + 1], acc[q + 2], acc[q + 3]};
+      }
     }
 #pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int i = 0; i < E; ++i) au[c][i] = av[c][i] = 0.f;
+    for (int i = 0; i < E; ++i) acc[i] = 0.f;
   };
 
   int run_e = -1, run_first = first;
   for (int p64 = first; p64 < last; p64 += kWave) {   // list order = (expert, pair) order: a fixed summation order
     // lane i holds what belongs to pair p64 + i: the chain pair -> id is walked once for 64 pairs, and the rows of every batch can be asked for at once
-    const int mine = min(p64 + lane, last - 1), my_pid = sorted_pair_ids[mine], my_tok = sorted_token_ids[mine];
-    const int my_e = ids[my_pid];
-    const float my_ds = ds[my_pid], my_coef = coef[my_pid];
-    const int end = min(p64 + kWave, last);
+    const int n = min(kWave, last - p64), mine = p64 + min(lane, n - 1), my_pid = p.pair_ids[mine], my_tok = p.token_ids[mine];
+    const int my_e = p.ids[my_pid];
+    const float my_factor = factors[my_pid], my_coef = PAIRED ? p.coef[my_pid] : 0.f;
     if (run_e < 0) run_e = __builtin_amdgcn_readlane(my_e, 0);
-    for (int p0 = p64; p0 < end; p0 += G) {
-      u32x4_t xr[G][NCH], dyr[G][NCH];
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int64_t at = __builtin_amdgcn_readlane(my_tok, min(p0 + i, end - 1) - p64) * row_bytes;
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-          xr[i][c] = live[c] ? *(const u32x4_t*)(x + at + off[c]) : u32x4_t{0, 0, 0, 0};
-          dyr[i][c] = live[c] ? *(const u32x4_t*)(dy + at + off[c]) : u32x4_t{0, 0, 0, 0};
-        }
+    const int left_e = __shfl_up(my_e, 1, kWave);
+    const uint64_t starts = __ballot(my_e != (lane ? left_e : run_e));          // bit i: pair p64 + i begins a run
+    auto request = [&](int at) __attribute__((always_inline)) {
+      const uint8_t* row = rows + (uint64_t)(uint32_t)__builtin_amdgcn_readlane(my_tok, at) * row_bytes;
+      if constexpr (!PAIRED) asm("" : "+s"(row));     // a scalar base and the lane's 32-bit offset, not a 64-bit address for every lane
+      return *(const u32x4_t*)(row + off);
+    };
+    auto add = [&](int at, const u32x4_t& row) __attribute__((always_inline)) {
+      float factor = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_factor), at));
+      if constexpr (PAIRED) {
+        const float coef = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_coef), at));
+        factor = second ? coef : factor;
       }
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int p = p0 + i;
-        if (p >= end) break;
-        const int e = __builtin_amdgcn_readlane(my_e, p - p64);
-        const float cs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ds), p - p64));
-        const float cc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_coef), p - p64));
-        if (e != run_e) {
-          flush(run_e, run_first, p);
-          run_e = e;
-          run_first = p;
-        }
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-          axpy16<DT>(cs, xr[i][c], au[c]);
-          axpy16<DT>(cc, dyr[i][c], av[c]);
-        }
+      if (starts >> at & 1) {
+        flush(run_e, run_first, p64 + at);
+        run_e = __builtin_amdgcn_readlane(my_e, at);
+        run_first = p64 + at;
       }
+      axpy16<DT>(factor, row, acc);
+    };
+    u32x4_t row[G];
+    int at = 0;
+    for (; at + G <= n; at += G) {
+#pragma unroll
+      for (int i = 0; i < G; ++i) row[i] = request(at + i);
+#pragma unroll
+      for (int i = 0; i < G; ++i) add(at + i, row[i]);
+    }
+    if (at < n) {
+#pragma unroll
+      for (int i = 0; i < G - 1; ++i) row[i] = request(min(at + i, n - 1));
+#pragma unroll
+      for (int i = 0; i < G - 1; ++i)
+        if (at + i < n) add(at + i, row[i]);
     }
   }
   flush(run_e, run_first, last);
@@ -772,9 +776,17 @@ static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, vo
   const int chunk = weight_chunk(P);
   const int num_chunks = (int)((P + chunk - 1) / chunk);
   if (num_chunks > 0) {
-    dim3 grid((unsigned)((num_chunks + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock));
-    hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, NCH, G>), grid, block, 0, s, p.x, p.dy, p.ds, p.coef,
-                       p.ids, offsets, pair_ids, token_ids, (uint8_t*)dup, (uint8_t*)ddown, partials, N, H, chunk, num_chunks);
+    constexpr int E = Row16<DT>::kElems;
+    WeightPass w{p.x, p.dy, p.ds, p.coef, p.ids, offsets, pair_ids, token_ids, (uint8_t*)dup, (uint8_t*)ddown, partials, N, H, chunk, num_chunks};
+    const int pieces = H / E;                          // 16-byte pieces of a row
+    const bool paired = pieces <= kWave / 2;
+    w.columns = paired ? 0 : (pieces + kWave - 1) / kWave;
+    w.lanes = paired ? pieces : (pieces + w.columns - 1) / w.columns;
+    w.blocks = (num_chunks + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock;
+    w.per_xcd = ((paired ? 1 : 2 * w.columns) * w.blocks + kXcds - 1) / kXcds;
+    const dim3 grid((unsigned)(w.per_xcd * kXcds));
+    if (paired) hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, true, 8>), grid, block, 0, s, w);
+    else hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, false, 8>), grid, block, 0, s, w);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   // Rows of up to 4 KiB (16-bit 2048 columns), and up to four columns of a half to a lane: the router's first launch beside the fix-up
