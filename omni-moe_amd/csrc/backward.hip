@@ -476,20 +476,23 @@ __global__ __launch_bounds__(kSortThreads) void expert_bwd_accumulate_kernel(con
 }
 
 // ---- experts, weight pass ----------------------------------------------------------------------
-// The sorted pair list is cut into chunks of `chunk` consecutive pairs, one wave each, whatever the
-// segment lengths: a popular expert's segment is spread over many waves and many rare experts
-// share one.  Inside its chunk a wave sums run after run (a run = the chunk's pairs of one
-// expert).  A run that is the expert's whole segment is rounded and stored straight away.  A run
-// of a segment that crosses the chunk's border is left as an fp32 partial row pair in
-// `partials[chunk][slot]`, slot 0 if the run starts the chunk, slot 1 otherwise (a chunk has at
-// most one of each); the fix-up kernel then adds an expert's partials in chunk order, so the
-// summation order is fixed and nothing is added atomically.
+// The sorted pair list is cut into chunks of `chunk` consecutive pairs, one wave each, whatever the segment lengths: a popular expert's
+// segment is spread over many waves and many rare experts share one.  A wave sums run after run (a run = consecutive pairs of one expert).
+// A segment of up to `chunk` pairs is summed, rounded and stored by the wave of the chunk that it begins in, also beyond that chunk's
+// border; a longer one is cut at the borders, and every wave leaves its run as an fp32 partial row pair in `partials[chunk][slot]`, slot 0
+// if the run starts the chunk, slot 1 otherwise (a chunk has at most one of each); the fix-up kernel then adds an expert's partials in
+// chunk order, so the summation order is fixed and nothing is added atomically.  (With every segment cut at the borders, 65536 pairs over 4096
+// experts left 33 MB of partial rows: weight pass and fix-up 24.3 + 12.1 -> 24.3 + 9.5 us, 32768 over 16384 18.5 + 6.4 -> 16.4 + 4.6; the
+// whole backward at 4096 tokens x 16, hidden 1024, 60.5 -> 54.4, hidden 2048 119.9 -> 102.8.)
 //
 // Bound by the gathers: a row pair is read for every pair of the list.  What a wave owns is therefore a chunk of one PART of the columns: up to 1 KiB of
 // the rows of x (for dU) or of dy (for dV), 16 bytes to a lane, and the parts go to the XCDs one after another, so that an XCD gathers from the one or two
 // parts that its L2 holds; with whole rows of both in every wave, all of x and dy went through every L2 and the pass ran at the fabric's 7 TB/s.  A wave's row
 // address and factor are scalars, so a narrower part costs no exchange between lanes.  Rows of up to 512 bytes: x in the lower half of the lanes, dy in the
-// upper.  The chunks, and with them the order of all sums, do not depend on the parts.
+// upper.  The finished rows pass the L2 by (non-temporal), which is left to the rows that are gathered.  The chunks, and with them the order of all sums, do not depend on the parts.  (4096 tokens x 16, hidden 1024, bf16 37.7 -> 24.3 us, 1024 x 32 over 16384
+// experts 23.7 -> 18.5.  The parts of a chunk one after the other instead, which keeps whole rows together: the whole backward there 54.4 -> 71.6 and 45.9 -> 51.5,
+// at 32768 tokens x 16 over 65536, which no L2 holds, 888 either way.  Four rows in flight, non-temporal: 16384 x 16 over 4096 232.8 -> 227.1, 8192 x 8 over 16384, hidden
+// 2048, 197.5 -> 189.1; sixteen rows or the next batch requested ahead: 1-3 % slower at 1024 and 4096 tokens.)
 struct WeightPass {
   const uint8_t *x, *dy;
   const float *ds, *coef;
@@ -505,12 +508,21 @@ template <int DT, bool PAIRED, int G>
 __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void expert_bwd_weight_kernel(const WeightPass p) {
   constexpr int E = Row16<DT>::kElems;
   const int lane = lane_id();
-  const int item = ((int)blockIdx.x % kXcds) * p.per_xcd + (int)blockIdx.x / kXcds, part = item / p.blocks;
-  if (part >= (PAIRED ? 1 : 2 * p.columns)) return;
-  const int ci = __builtin_amdgcn_readfirstlane((item - part * p.blocks) * kBwdWavesPerBlock + (int)(threadIdx.x >> 6));
+  const int item = ((int)blockIdx.x % kXcds) * p.per_xcd + (int)blockIdx.x / kXcds, parts = PAIRED ? 1 : 2 * p.columns;
+  if (item >= parts * p.blocks) return;
+  const int part = item / p.blocks, ci = __builtin_amdgcn_readfirstlane((item - part * p.blocks) * kBwdWavesPerBlock + (int)(threadIdx.x >> 6));
   if (ci >= p.num_chunks) return;
   const int valid = p.offsets[p.num_experts];         // pairs with an id inside the table
-  const int first = ci * p.chunk, last = min(first + p.chunk, valid);
+  const int border = ci * p.chunk;
+  int first = border, last = min(border + p.chunk, valid);
+  if (first >= last) return;
+  // the segments that the chunk's first and last pair are of
+  auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  const int e0 = uniform(p.ids[p.pair_ids[first]]), e1 = uniform(p.ids[p.pair_ids[last - 1]]);
+  const int begin0 = uniform(p.offsets[e0]), end0 = uniform(p.offsets[e0 + 1]), begin1 = uniform(p.offsets[e1]), end1 = uniform(p.offsets[e1 + 1]);
+  const bool cut0 = end0 - begin0 > p.chunk, cut1 = end1 - begin1 > p.chunk;
+  if (!cut0 && begin0 < border) first = end0;         // the wave that it begins with finishes it
+  if (!cut1) last = end1;
   if (first >= last) return;
   const uint32_t row_bytes = (uint32_t)p.hidden * (16 / E);
 
@@ -524,16 +536,14 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void expert_bwd_weight_ke
   float acc[E];
 #pragma unroll
   for (int i = 0; i < E; ++i) acc[i] = 0.f;
-  // Ends the run [run_first, run_last) of expert e and clears the accumulators.  A run inside the chunk is its expert's whole segment; only the
-  // chunk's first and last run need a look at the pairs beyond it, and those ids are fetched ahead.
-  const int before = first > 0 ? p.ids[p.pair_ids[first - 1]] : -1, after = last < valid ? p.ids[p.pair_ids[last]] : -1;
+  // Ends the run [run_first, run_last) of expert e and clears the accumulators
   auto flush = [&](int e, int run_first, int run_last) {
-    const bool whole = (run_first != first || before != e) && (run_last != last || after != e);
+    const bool whole = (run_first != border || !cut0) && (run_last != last || !cut1);
     if (live) {
       if (whole) {
-        *(u32x4_t*)(out_rows + (int64_t)e * row_bytes + off) = pack16<DT>(acc);
+        __builtin_nontemporal_store(pack16<DT>(acc), (u32x4_t*)(out_rows + (int64_t)e * row_bytes + off));
       } else {
-        float* out = p.partials + (int64_t(ci) * 2 + (run_first == first ? 0 : 1)) * 2 * p.hidden + (second ? p.hidden : 0) + piece * E;
+        float* out = p.partials + (int64_t(ci) * 2 + (run_first == border ? 0 : 1)) * 2 * p.hidden + (second ? p.hidden : 0) + piece * E;
 #pragma unroll
         for (int q = 0; q < E; q += 4) *(f32x4_t*)(out + q) = f32x4_t{acc[q], acc[q + 1], acc[q + 2], acc[q + 3]};
       }
@@ -588,9 +598,8 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void expert_bwd_weight_ke
   flush(run_e, run_first, last);
 }
 
-// One wave per expert: zero rows for an expert nobody selected; for a segment that crosses a chunk
-// border the sum of its partial rows, first chunk to last.  A segment inside one chunk was
-// stored by the pass above.
+// One wave per expert: zero rows for an expert nobody selected; for a segment of more than `chunk` pairs the sum of its partial rows,
+// first chunk to last.  The others were stored by the pass above.
 // R > 0: the launch's first `router_blocks` blocks are the router's (R columns of a half to a lane), which only needs the token pass in front of it: a layer's
 // backward of 4096 tokens x 1024, 64 keys, k = 16 took 7.4 us for the fix-up and 8.2 + 5.0 + 4.1 for the router's three launches behind it; both in one launch
 // 12.2, and 7.0 to finish (1000 tokens x 512, k = 8: 3.8 + 4.9 + 3.6 + 2.8 -> 4.6 + 5.5).
@@ -609,8 +618,8 @@ __global__ __launch_bounds__((R ? norm_waves(R) : kBwdWavesPerBlock) * kWave) vo
   const int64_t e = __builtin_amdgcn_readfirstlane((int)(((int)blockIdx.x - router_blocks) * W + (int)(threadIdx.x >> 6)));
   if (e >= num_experts) return;
   const int begin = offsets[e], end = offsets[e + 1];
+  if (end > begin && end - begin <= chunk) return;
   const int c0 = begin / chunk, c1 = end > begin ? (end - 1) / chunk : c0;
-  if (end > begin && c0 == c1) return;
   const int64_t row_bytes = int64_t(hidden) * (16 / E);
   float au[NCH][E], av[NCH][E];
 #pragma unroll
@@ -785,8 +794,8 @@ static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, vo
     w.blocks = (num_chunks + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock;
     w.per_xcd = ((paired ? 1 : 2 * w.columns) * w.blocks + kXcds - 1) / kXcds;
     const dim3 grid((unsigned)(w.per_xcd * kXcds));
-    if (paired) hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, true, 8>), grid, block, 0, s, w);
-    else hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, false, 8>), grid, block, 0, s, w);
+    if (paired) hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, true, 4>), grid, block, 0, s, w);
+    else hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, false, 4>), grid, block, 0, s, w);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   // Rows of up to 4 KiB (16-bit 2048 columns), and up to four columns of a half to a lane: the router's first launch beside the fix-up

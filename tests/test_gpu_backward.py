@@ -200,6 +200,31 @@ def _check_expert_bwd(case, dtype, device, place=lambda t: t):
         _close(got, ref, dtype, what)
 
 
+# The weight pass's chunks are 16 pairs here: segments of up to 16 (summed by the wave that they begin with) and of more (cut at the borders), at every offset from a
+# border, a last chunk that is short, ids outside the table; rows of half a part (512 bytes), one part and a little more, two, and parts whose last lane is idle
+@pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
+@pytest.mark.parametrize("row", [48, 512, 528, 1024, 1040, 2064, 4096], ids=lambda r: f"B{r}")
+def test_expert_bwd_segments_around_chunk_borders(row, dtype, device):
+    lengths = [16, 1, 15, 0, 16, 17, 3, 16, 32, 33, 2, 16, 5, 47, 15, 16, 16, 48, 0, 31, 7, 1, 1, 16] * 3 + [14]
+    N, k, H = len(lengths), 4, row // torch.empty(0, dtype=dtype).element_size()
+    flat = torch.repeat_interleave(torch.arange(N), torch.tensor(lengths))
+    flat = torch.cat([flat, torch.tensor([-1, N, N + 5] + [N] * ((-3 - flat.numel()) % k))])
+    T = flat.numel() // k
+    g = torch.Generator().manual_seed(row)
+    ids = flat[torch.randperm(flat.numel(), generator=g)].view(T, k).int()
+    x, up, down, gates, _ = oracle.make_expert_inputs(14, T, H, N, k, dtype=dtype, w_std=0.05)
+    dy = torch.randn(T, H, generator=g).to(dtype)
+    print(f"expert bwd segments B={row} {dtype} T={T} N={N}", flush=True)
+    ok = (ids >= 0) & (ids < N)
+    _, wdx, wdu, wdv, wdg = _expert_reference(x, up, down, gates * ok, ids.clamp(0, N - 1), dy)
+    dx, du, dv, dg = _ops().hip_omni_expert_bwd_func(*(t.to(device) for t in (dy, x, up, down, gates, ids)))
+    _close(dx, wdx, dtype, "dx")
+    _close(du, wdu, dtype, "dup_weight")
+    _close(dv, wdv, dtype, "ddown_weight")
+    unused = torch.tensor(lengths) == 0
+    assert not du.cpu()[unused].any() and not dv.cpu()[unused].any()
+
+
 def test_expert_func_autograd(device):
     T, H, N, k = 128, 256, 64, 8
     x, up, down, gates, ids = oracle.make_expert_inputs(13, T, H, N, k, dtype=torch.float32, w_std=0.05)
