@@ -87,8 +87,8 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void router_bwd_kernel(
 // v_readlane; what bounds the pass is that chain, so a wave takes few tokens while there are waves to spare (4096 tokens, 64 keys, k = 16:
 // eight tokens a wave and ds_bpermute exchanges 29 us).
 // Two launches in training: the blocks that finish d(z) add the column sums of their 64 columns themselves, 512 bytes from each block of the first launch, of
-// which there are few (4096 tokens: 256).  Reads nothing that the experts' weight pass leaves, so the layer's backward puts the first
-// launch beside that pass's fix-up (expert_bwd_weight_fixup_kernel).
+// which there are few (4096 tokens: 256).  Neither reads what the experts' weight pass leaves, so the layer's backward puts the first
+// beside that pass and the second beside its fix-up.
 static inline int norm_tokens_per_wave(int64_t num_tokens) {
   const int64_t t = num_tokens / (kBwdWavesPerBlock * 512);
   return (int)(t < 1 ? 1 : t > 8 ? 8 : t);
@@ -245,11 +245,11 @@ __global__ __launch_bounds__(norm_waves(R)* kWave) void router_norm_bwd_kernel(c
 // sums over the `rows` partials in double, sixteen waves side by side, while its first tokens' values are on their way.
 constexpr int kFinishWaves = 16, kFinishRows = 4;               // tokens that a wave has in flight
 template <int DT>
-__global__ __launch_bounds__(kFinishWaves* kWave) void router_norm_bwd_finish_kernel(const RouterPass p, const int rows) {
+__device__ __forceinline__ void router_norm_bwd_finish_block(const RouterPass& p, const int rows, const int block, const int blocks) {
   __shared__ double sums[2][kFinishWaves][kWave];
   __shared__ float means[2][kWave];
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = p.r, per_half = (r + kWave - 1) / kWave, groups = 2 * per_half;
-  const int group = (int)blockIdx.x % groups, part = (int)blockIdx.x / groups, parts = (int)gridDim.x / groups;
+  const int group = block % groups, part = block / groups, parts = blocks / groups;
   const int h = group / per_half, col = (group - h * per_half) * kWave + lane, key = min(col, r - 1);
   const bool live = col < r;
   float zv[kFinishRows], dn[kFinishRows];
@@ -291,6 +291,10 @@ __global__ __launch_bounds__(kFinishWaves* kWave) void router_norm_bwd_finish_ke
       if (live && t < p.num_tokens) Elem<DT>::store(p.dz, at(t), rs * (dn[i] - m1 - (zv[i] - mu) * rs * m2));
     }
   }
+}
+template <int DT>
+__global__ __launch_bounds__(kFinishWaves* kWave) void router_norm_bwd_finish_kernel(const RouterPass p, const int rows) {
+  router_norm_bwd_finish_block<DT>(p, rows, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---- experts, token pass -----------------------------------------------------------------------
@@ -504,13 +508,21 @@ struct WeightPass {
   int lanes, columns;                // 16-byte lanes of a part; parts of a row of x, and as many of dy (0: both in one part)
   int blocks, per_xcd;               // blocks of a part; all parts' blocks on an XCD
 };
-template <int DT, bool PAIRED, int G>
-__global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void expert_bwd_weight_kernel(const WeightPass p) {
-  constexpr int E = Row16<DT>::kElems;
-  const int lane = lane_id();
-  const int item = ((int)blockIdx.x % kXcds) * p.per_xcd + (int)blockIdx.x / kXcds, parts = PAIRED ? 1 : 2 * p.columns;
+// R > 0: the launch's first `router_blocks` blocks (a multiple of eight, so that block % 8 names the XCD of the others too) are the router's, R columns of a half to
+// a lane.
+template <int DT, bool PAIRED, int G, int R>
+__global__ __launch_bounds__((R ? norm_waves(R) : kBwdWavesPerBlock) * kWave) void expert_bwd_weight_kernel(const WeightPass p, const RouterPass router, const int router_blocks) {
+  constexpr int E = Row16<DT>::kElems, W = R ? norm_waves(R) : kBwdWavesPerBlock;
+  if constexpr (R > 0) {
+    if ((int)blockIdx.x < router_blocks) {
+      if ((int)blockIdx.x * W * router.tokens_per_wave < router.num_tokens) router_norm_bwd_block<DT, R>(router, (int)blockIdx.x);
+      return;
+    }
+  }
+  const int lane = lane_id(), at_block = (int)blockIdx.x - router_blocks;
+  const int item = (at_block % kXcds) * p.per_xcd + at_block / kXcds, parts = PAIRED ? 1 : 2 * p.columns;
   if (item >= parts * p.blocks) return;
-  const int part = item / p.blocks, ci = __builtin_amdgcn_readfirstlane((item - part * p.blocks) * kBwdWavesPerBlock + (int)(threadIdx.x >> 6));
+  const int part = item / p.blocks, ci = __builtin_amdgcn_readfirstlane((item - part * p.blocks) * W + (int)(threadIdx.x >> 6));
   if (ci >= p.num_chunks) return;
   const int valid = p.offsets[p.num_experts];         // pairs with an id inside the table
   const int border = ci * p.chunk;
@@ -600,22 +612,21 @@ __global__ __launch_bounds__(kBwdWavesPerBlock* kWave) void expert_bwd_weight_ke
 
 // One wave per expert: zero rows for an expert nobody selected; for a segment of more than `chunk` pairs the sum of its partial rows,
 // first chunk to last.  The others were stored by the pass above.
-// R > 0: the launch's first `router_blocks` blocks are the router's (R columns of a half to a lane), which only needs the token pass in front of it: a layer's
-// backward of 4096 tokens x 1024, 64 keys, k = 16 took 7.4 us for the fix-up and 8.2 + 5.0 + 4.1 for the router's three launches behind it; both in one launch
-// 12.2, and 7.0 to finish (1000 tokens x 512, k = 8: 3.8 + 4.9 + 3.6 + 2.8 -> 4.6 + 5.5).
-template <int DT, int NCH, int R>
-__global__ __launch_bounds__((R ? norm_waves(R) : kBwdWavesPerBlock) * kWave) void expert_bwd_weight_fixup_kernel(
+// FINISH: the launch's first `finish_blocks` blocks finish the router's d(z).  Router and experts, before / now: 4096 tokens x 1024 over 64 x 64, k 16: pass 24.3, fix-up beside
+// the first 9.4, finish 7.3 us -> 25.5 + 8.7; 1000 x 512 over 32 x 32, k 8: 6.2 + 4.7 + 6.0 -> 7.2 + 6.0.
+template <int DT, int NCH, bool FINISH>
+__global__ __launch_bounds__((FINISH ? kFinishWaves : kBwdWavesPerBlock) * kWave) void expert_bwd_weight_fixup_kernel(
     const int32_t* __restrict__ offsets, const float* __restrict__ partials, uint8_t* __restrict__ dup,
-    uint8_t* __restrict__ ddown, int64_t num_experts, int hidden, int chunk, const RouterPass router, const int router_blocks) {
-  constexpr int E = Row16<DT>::kElems, W = R ? norm_waves(R) : kBwdWavesPerBlock;
-  if constexpr (R > 0) {
-    if ((int)blockIdx.x < router_blocks) {
-      router_norm_bwd_block<DT, R>(router, (int)blockIdx.x);
+    uint8_t* __restrict__ ddown, int64_t num_experts, int hidden, int chunk, const RouterPass router, const int router_rows, const int finish_blocks) {
+  constexpr int E = Row16<DT>::kElems, W = FINISH ? kFinishWaves : kBwdWavesPerBlock;
+  if constexpr (FINISH) {
+    if ((int)blockIdx.x < finish_blocks) {
+      router_norm_bwd_finish_block<DT>(router, router_rows, (int)blockIdx.x, finish_blocks);
       return;
     }
   }
   const int lane = lane_id();
-  const int64_t e = __builtin_amdgcn_readfirstlane((int)(((int)blockIdx.x - router_blocks) * W + (int)(threadIdx.x >> 6)));
+  const int64_t e = __builtin_amdgcn_readfirstlane((int)(((int)blockIdx.x - finish_blocks) * W + (int)(threadIdx.x >> 6)));
   if (e >= num_experts) return;
   const int begin = offsets[e], end = offsets[e + 1];
   if (end > begin && end - begin <= chunk) return;
@@ -764,12 +775,15 @@ static hipError_t launch_norm_first(const RouterPass& p, hipStream_t s) {
   else hipLaunchKernelGGL((router_norm_bwd_kernel<DT, 16>), dim3(blocks), dim3(norm_waves(16) * kWave), 0, s, p);
   return hipGetLastError();
 }
+// Blocks that finish d(z): a CU's block for every group of columns, or fewer where 64 tokens to a block are all
+static int finish_blocks(const RouterPass& p) {
+  const int groups = 2 * ((p.r + kWave - 1) / kWave), want = (p.num_tokens + kFinishWaves * kFinishRows - 1) / (kFinishWaves * kFinishRows), most = groups < 256 ? 256 / groups : 1;
+  return groups * (want < most ? want : most);
+}
 template <int DT>
 static hipError_t launch_norm_finish(const RouterPass& p, hipStream_t s) {
   if (!p.training) return hipSuccess;
-  // a CU's block for every group of columns, or fewer where 64 tokens to a block are all
-  const int groups = 2 * ((p.r + kWave - 1) / kWave), want = (p.num_tokens + kFinishWaves * kFinishRows - 1) / (kFinishWaves * kFinishRows), most = groups < 256 ? 256 / groups : 1;
-  hipLaunchKernelGGL(router_norm_bwd_finish_kernel<DT>, dim3((unsigned)(groups * (want < most ? want : most))), dim3(kFinishWaves * kWave), 0, s, p, norm_blocks(p.num_tokens, p.r));
+  hipLaunchKernelGGL(router_norm_bwd_finish_kernel<DT>, dim3((unsigned)finish_blocks(p)), dim3(kFinishWaves * kWave), 0, s, p, norm_blocks(p.num_tokens, p.r));
   return hipGetLastError();
 }
 
@@ -780,10 +794,13 @@ static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, vo
   const int H = p.hidden, k = p.top_k;
   const hipError_t te = p.lanes ? launch_token_split<DT>(p, sort, s) : launch_token_gather<DT, NCH, G>(p, sort, s);
   if (te != hipSuccess) return te;
-  dim3 block(kBwdWavesPerBlock * kWave);
   const size_t P = (size_t)T * (size_t)k;
   const int chunk = weight_chunk(P);
   const int num_chunks = (int)((P + chunk - 1) / chunk);
+  // The router beside: up to four columns of a half to a lane, and, in the second launch, rows of up to 4 KiB (16-bit 2048 columns)
+  const bool first_beside = router && num_chunks > 0 && router->r <= 4 * kWave, finish_beside = router && router->training && NCH <= 4;
+  if (router && !first_beside)
+    if (hipError_t e = launch_norm_first<DT>(*router, s); e != hipSuccess) return e;
   if (num_chunks > 0) {
     constexpr int E = Row16<DT>::kElems;
     WeightPass w{p.x, p.dy, p.ds, p.coef, p.ids, offsets, pair_ids, token_ids, (uint8_t*)dup, (uint8_t*)ddown, partials, N, H, chunk, num_chunks};
@@ -791,32 +808,33 @@ static hipError_t launch_expert_bwd(const TokenPass& p, const SortPass* sort, vo
     const bool paired = pieces <= kWave / 2;
     w.columns = paired ? 0 : (pieces + kWave - 1) / kWave;
     w.lanes = paired ? pieces : (pieces + w.columns - 1) / w.columns;
-    w.blocks = (num_chunks + kBwdWavesPerBlock - 1) / kBwdWavesPerBlock;
-    w.per_xcd = ((paired ? 1 : 2 * w.columns) * w.blocks + kXcds - 1) / kXcds;
-    const dim3 grid((unsigned)(w.per_xcd * kXcds));
-    if (paired) hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, true, 4>), grid, block, 0, s, w);
-    else hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, false, 4>), grid, block, 0, s, w);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    auto start = [&](auto cols) {
+      constexpr int R = decltype(cols)::value, W = R ? norm_waves(R) : kBwdWavesPerBlock;
+      w.blocks = (num_chunks + W - 1) / W;
+      w.per_xcd = ((paired ? 1 : 2 * w.columns) * w.blocks + kXcds - 1) / kXcds;
+      const int router_blocks = R ? (norm_blocks(T, router->r) + kXcds - 1) / kXcds * kXcds : 0;
+      const dim3 grid((unsigned)(router_blocks + w.per_xcd * kXcds)), block(W * kWave);
+      const RouterPass beside = R ? *router : RouterPass{};
+      if (paired) hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, true, 4, R>), grid, block, 0, s, w, beside, router_blocks);
+      else hipLaunchKernelGGL((expert_bwd_weight_kernel<DT, false, 4, R>), grid, block, 0, s, w, beside, router_blocks);
+      return hipGetLastError();
+    };
+    const hipError_t e = !first_beside ? start(std::integral_constant<int, 0>{}) : router->r <= kWave ? start(std::integral_constant<int, 1>{}) : start(std::integral_constant<int, 4>{});
+    if (e != hipSuccess) return e;
   }
-  // Rows of up to 4 KiB (16-bit 2048 columns), and up to four columns of a half to a lane: the router's first launch beside the fix-up
-  const bool beside = router && NCH <= 4 && router->r <= 4 * kWave;
-  auto fixup = [&](auto cols, int router_blocks) {
-    constexpr int R = decltype(cols)::value, W = R ? norm_waves(R) : kBwdWavesPerBlock;
-    hipLaunchKernelGGL((expert_bwd_weight_fixup_kernel<DT, NCH, R>), dim3((unsigned)(router_blocks + (N + W - 1) / W)), dim3(W * kWave), 0, s, offsets, partials, (uint8_t*)dup,
-                       (uint8_t*)ddown, N, H, chunk, router ? *router : RouterPass{}, router_blocks);
+  auto fixup = [&](auto finish) {
+    constexpr bool FINISH = decltype(finish)::value;
+    constexpr int W = FINISH ? kFinishWaves : kBwdWavesPerBlock;
+    const int first = FINISH ? finish_blocks(*router) : 0;
+    hipLaunchKernelGGL((expert_bwd_weight_fixup_kernel<DT, NCH, FINISH>), dim3((unsigned)(first + (N + W - 1) / W)), dim3(W * kWave), 0, s, offsets, partials, (uint8_t*)dup,
+                       (uint8_t*)ddown, N, H, chunk, FINISH ? *router : RouterPass{}, FINISH ? norm_blocks(T, router->r) : 0, first);
     return hipGetLastError();
   };
-  hipError_t e;
   if constexpr (NCH <= 4) {
-    if (beside) e = router->r <= kWave ? fixup(std::integral_constant<int, 1>{}, norm_blocks(T, router->r)) : fixup(std::integral_constant<int, 4>{}, norm_blocks(T, router->r));
-    else e = fixup(std::integral_constant<int, 0>{}, 0);
-  } else {
-    e = fixup(std::integral_constant<int, 0>{}, 0);
+    if (finish_beside) return fixup(std::true_type{});
   }
-  if (e != hipSuccess || !router) return e;
-  if (!beside)
-    if ((e = launch_norm_first<DT>(*router, s)) != hipSuccess) return e;
-  return launch_norm_finish<DT>(*router, s);
+  const hipError_t e = fixup(std::false_type{});
+  return e != hipSuccess || !router ? e : launch_norm_finish<DT>(*router, s);
 }
 
 }  // namespace omni
