@@ -18,6 +18,8 @@
 #include "omni_moe_hip.h"
 #include "select.h"
 
+#include <algorithm>
+
 // defined beside the GEMM kernels: z = x [Wx;Wy]^T, optionally with per-32-row column
 // partial statistics (mean, M2) [ceil(T/32)][2r] of the rounded z
 int omni_gemm_router_projection(const void* x, const void* wx, const void* wy, void* z, float* part_mean, float* part_m2,
@@ -35,6 +37,15 @@ template <int DT, int R, int C>
 __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_packed_kernel(const SelectArgs g) {
   count_batch(g);
   select_packed<DT, R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats);
+}
+
+// Training: the blocks merge the projection's column statistics themselves, W waves to a block.
+template <int DT, int R, int C, int W>
+__global__ __launch_bounds__(W* kWave) void router_select_merge_kernel(const SelectArgs g) {
+  extern __shared__ __align__(16) float stats[];
+  merge_statistics(g, stats, W * kWave);
+  count_batch(g);
+  select_packed<DT, R, C>(g, blockIdx.x * W + (threadIdx.x >> 6), gridDim.x * W, stats);
 }
 
 // More keys per half than a wave's registers hold (r > 1024): 16-bit scores, k' <= 64.  The row is walked in chunks of
@@ -185,6 +196,21 @@ static int select_dispatch(SelectArgs g, hipStream_t s) {
   return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
 }
 
+static int merge_cells(int r, int k) { return (num_cells(k, r < k ? r : k) + kWave - 1) / kWave; }      // candidates per lane
+template <int W>
+static hipError_t launch_select_merge(SelectArgs g, hipStream_t s) {
+  const int cpl = prepare_select(g);
+  const int64_t blocks = std::min<int64_t>(((int64_t)g.num_tokens + W - 1) / W, 256 * 16 / W);
+  auto start = [&](auto cells) {
+    constexpr int C = decltype(cells)::value;
+    const int bytes = 4 * merge_lds_floats(g.r, W * kWave);
+    if (g.dt == kBF16) hipLaunchKernelGGL((router_select_merge_kernel<kBF16, 1, C, W>), dim3((unsigned)blocks), dim3(W * kWave), bytes, s, g);
+    else hipLaunchKernelGGL((router_select_merge_kernel<kF16, 1, C, W>), dim3((unsigned)blocks), dim3(W * kWave), bytes, s, g);
+    return hipGetLastError();
+  };
+  return cpl <= 1 ? start(std::integral_constant<int, 1>{}) : start(std::integral_constant<int, 2>{});
+}
+
 // ---- BatchNorm1d(affine=False) statistics over the T rows of z [T, C] -------------------
 struct BnFinalArgs {
   const float* part_mean;   // [strips][2r] (training)
@@ -329,6 +355,28 @@ int router_fwd(const void* x, const void* weight_x, const void* weight_y,
   // (in training its epilogue also leaves the per-32-row column statistics)
   if (int e = omni_gemm_router_projection(x, weight_x, weight_y, z, training ? part_mean : nullptr, training ? part_m2 : nullptr,
                                           num_tokens, hidden_size, r, dtype, stream, exclusive)) return e;
+  // Training, up to 64 keys per half and 128 KiB of partial statistics: the selecting blocks merge them themselves.  16 waves to a block beyond 2048 tokens (as many
+  // merges as CUs), 8 below (more CUs).  Whole call in three launches / two, top-16 and 64 keys: 1024 tokens 15.0 -> 13.7 us, 2048 15.7 -> 14.4 (16 waves 15.9), 4096
+  // 18.4 -> 17.3 (8 waves 18.5); 32 keys: 256 13.3 -> 11.8, 8192 27.6 -> 25.6.  More keys: 2048 x 100 17.8 -> 23-30, 1500 x 128 21 -> 28-30.  Beside another stream's
+  // kernels, which hide the launch, whole blocks of 16 waves would wait for a CU.
+  const bool merge = training && exclusive && k > 0 && dtype != OMNI_F32 && r <= kWave && merge_here(num_tokens, r) && merge_cells(r, k) <= 2;
+  SelectArgs g{};
+  g.lx = z; g.ly = (const char*)z + (size_t)r * es; g.row_stride = 2 * r;
+  g.scores = scores; g.gates = gates; g.indices = indices;
+  g.num_tokens = (int)num_tokens; g.r = r; g.k = k; g.dt = dtype;
+  if (!training || merge) {
+    g.run_mean[0] = running_mean_x; g.run_mean[1] = running_mean_y;
+    g.run_var[0] = running_var_x; g.run_var[1] = running_var_y;
+    g.stats_out = stats; g.stat_dt = stats_dtype; g.eps = eps;
+  }
+  if (training) {
+    g.count_batch[0] = num_batches_tracked_x; g.count_batch[1] = num_batches_tracked_y;
+  }
+  if (merge) {
+    g.part_mean = part_mean; g.part_m2 = part_m2; g.strips = (int)strips; g.momentum = momentum;
+    const hipError_t err = num_tokens > 2048 ? launch_select_merge<16>(g, s) : launch_select_merge<8>(g, s);
+    return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
+  }
   // Training: one more launch merges the partial statistics and moves the running buffers.  In eval mode the
   // select kernel reads the running buffers itself (and leaves mean and 1/sqrt(var + eps) in `stats`).
   if (training || k == 0) {
@@ -340,18 +388,7 @@ int router_fwd(const void* x, const void* weight_x, const void* weight_y,
     if (err != hipSuccess) return OMNI_ERR_HIP_BASE + (int)err;
     if (k == 0) return OMNI_OK;
   }
-  SelectArgs g{};
-  g.lx = z; g.ly = (const char*)z + (size_t)r * es; g.row_stride = 2 * r;
-  g.scores = scores; g.gates = gates; g.indices = indices;
-  g.num_tokens = (int)num_tokens; g.r = r; g.k = k; g.dt = dtype;
-  if (training) {
-    g.stats = stats;
-    g.count_batch[0] = num_batches_tracked_x; g.count_batch[1] = num_batches_tracked_y;
-  } else {
-    g.run_mean[0] = running_mean_x; g.run_mean[1] = running_mean_y;
-    g.run_var[0] = running_var_x; g.run_var[1] = running_var_y;
-    g.stats_out = stats; g.stat_dt = stats_dtype; g.eps = eps;
-  }
+  if (training) g.stats = stats;
   return select_dispatch(g, s);
 }
 }  // namespace omni

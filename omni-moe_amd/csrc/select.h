@@ -63,9 +63,8 @@ __device__ __forceinline__ ColumnStats column_stats(const ColumnSums& c, int num
 }
 __device__ __forceinline__ float rstd_of(float var, float eps) { return 1.0f / sqrtf(var + eps); }
 
-// Batch statistics for a block of `threads` that selects beside another kernel's tiles: every such block merges all columns (2r of them, a few dozen strips each),
-// which the tiles hide, where a merge of its own is a 4-5 us launch between projection and selection.  (A selection by itself is better off behind that
-// launch: 4096 tokens, 64 keys, blocks of 16 waves that merge first 13 us, against 4.5 + 8.8.)  lds: merge_lds_floats(r, threads) floats, 16-byte aligned; the first 4r hold mean_x, rstd_x,
+// Batch statistics for a block of `threads` that selects beside another kernel's tiles: every such block merges all columns (2r of them, up to a few hundred strips each, eight requested at a time),
+// which the tiles hide, where a merge of its own is a 4-5 us launch between projection and selection.  (A selection by itself: where router_fwd says.)  lds: merge_lds_floats(r, threads) floats, 16-byte aligned; the first 4r hold mean_x, rstd_x,
 // mean_y, rstd_y afterwards.
 __device__ __host__ constexpr int merge_lds_floats(int r, int threads) { return (4 * r + 3) / 4 * 4 + 4 * threads; }
 __device__ __forceinline__ void merge_statistics(const SelectArgs& g, float* lds, const int threads) {
@@ -75,6 +74,7 @@ __device__ __forceinline__ void merge_statistics(const SelectArgs& g, float* lds
     const int part = tid / cols, col = c0 + (parts > 1 ? tid - part * cols : tid);
     if (part < parts && col < cols) {
       ColumnSums c{0., 0.};
+#pragma unroll 8
       for (int strip = part; strip < g.strips; strip += parts) add_strip(c, g.part_mean, g.part_m2, strip, cols, col, g.num_tokens);
       sums[tid] = c;
     }

@@ -130,6 +130,31 @@ def test_router_fwd_matches_oracle(case, training, device):
         assert torch.equal(dbx[0].cpu(), bx.running_mean) and dbx[2].item() == 0
 
 
+# Statistics merged by the selecting blocks: both block sizes, at the border between them, two candidates to a lane, an odd number of keys, a partial strip
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", [(2048, 256, 64, 32), (2049, 256, 64, 32), (4096, 128, 64, 16), (1029, 256, 33, 8), (70, 256, 64, 2), (2, 128, 16, 4)], ids=lambda c: "T%d-H%d-r%d-k%d" % c)
+def test_router_fwd_merges_statistics_where_it_selects(case, dtype, device):
+    """Gates and ids against the oracle (a last-bit difference of a score may pick the other of two nearly equal experts: one in a hundred at most), buffers and counts
+    after two batches."""
+    T, H, r, k = case
+    g = torch.Generator().manual_seed(T + r)
+    wx, wy = ((torch.randn(r, H, generator=g) / H ** 0.5).to(dtype) for _ in range(2))
+    bx, by = oracle.BNState.fresh(r), oracle.BNState.fresh(r)
+    dbx, dby = _bn_buffers(r, torch.float32, device), _bn_buffers(r, torch.float32, device)
+    print(f"router_fwd merged T={T} H={H} r={r} k={k} {dtype}", flush=True)
+    for _ in range(2):
+        x = torch.randn(T, H, generator=g).to(dtype)
+        want_g, want_i, _ = oracle.router_forward(x, wx, wy, bx, by, k, True)
+        got_g, got_i = _ops().hip_omni_router_fwd_func(x.to(device), wx.to(device), wy.to(device), *dbx, *dby, k, training=True)
+        if T > 2:                                       # (two tokens normalise to +-1: every key ties)
+            assert (got_i.cpu().sort(-1).values == want_i.sort(-1).values).float().mean().item() >= 0.99
+            torch.testing.assert_close(got_g.cpu().float(), want_g.float(), rtol=2e-2, atol=2e-2)
+    for d, b in ((dbx, bx), (dby, by)):
+        torch.testing.assert_close(d[0].cpu(), b.running_mean, rtol=1e-3, atol=1e-4)
+        torch.testing.assert_close(d[1].cpu(), b.running_var, rtol=1e-3, atol=1e-4)
+        assert d[2].item() == 2
+
+
 def test_router_fwd_select_is_exact_given_same_logprobs(device):
     """Feeding the oracle's selection the device's own scores must reproduce the device's ids
     bit for bit: run the fused router, rebuild the log-probs it saw from its z, compare."""
