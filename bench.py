@@ -51,10 +51,11 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16, published
 # Bytes that cross the fabric per launch (FETCH_SIZE + WRITE_SIZE of rocprofv3 --pmc, each scaled by a plain copy of
 # known size); counters cannot be read in-process, so these are the figures of the committed summaries named here.
 TRAFFIC_SOURCE = ("profiles/bench_layer_c4_hbm_counters.txt, profiles/expert_c5_hbm_counters.txt; measured on the kernels as of the commit "
-                  "'Split expert passes: no ragged kernels for groups of four lanes, which no cut produces' -- a "
+                  "'Split expert passes: no ragged kernels for groups of four lanes, which no cut produces', the expert backward's as of "
+                  "'Expert weight pass: short segments stay with the wave that begins them, rows of the gradients stored past the L2' -- a "
                   "later change to a kernel's memory access pattern needs a new counter run")
 TRAFFIC_BYTES = {"expert_c3": 132.4e6, "expert_c4": 58.3e6, "expert_gather_c3": 899.2e6, "gateup_c4": 134.4e6, "down_c4": 117.6e6,
-                 "down_plain_c4": 109.2e6, "schedule_c3": 12.4e6, "expert_segment_c3": 927.1e6, "expert_bwd_c3": 1527.8e6,
+                 "down_plain_c4": 109.2e6, "schedule_c3": 12.4e6, "expert_segment_c3": 927.1e6, "expert_bwd_c3": 1325.5e6,
                  "expert_c5_routed": 1030.3e6, "expert_c5_routed_split": 731.5e6, "expert_c5_uniform": 8846.5e6}
 SECTIONS = ("layer", "kernels", "expert_c3", "expert_c5", "layer_c5", "ref_grid", "probe", "train", "cpu")
 
@@ -371,8 +372,8 @@ def main():
                         "timed": "omni_router_fwd through the C ABI with outputs and workspace allocated once, as the layer call runs it; "
                                  "through_python_operator_ms is a loop over layer.route(x), which allocates per call and is host-bound",
                         "algorithmic_flops": 4 * T * H * r, "algorithmic_bytes": (T * H + 2 * r * H + T * k * 3) * 2,
-                        "note": "1.07 GFLOP over 9.7 MB: bounded by launch and memory latency, not by a roofline; training = three dependent "
-                                "launches, eval = two (the select kernel reads the running statistics itself)"})
+                        "note": "1.07 GFLOP over 9.7 MB: bounded by launch and memory latency, not by a roofline; two dependent launches: in training the selecting "
+                                "blocks merge the batch statistics, in eval they read the running ones"})
         out["roofline"] = kernels[0]
 
     if "expert_c3" in sections:
