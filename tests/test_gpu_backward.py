@@ -540,6 +540,45 @@ def test_layer_saved_tensors_through_hooks(dtype, device):
         assert torch.equal(a, b) and torch.equal(a, c)
 
 
+@pytest.mark.parametrize("shape", [(150, 256, 512), (2200, 1024, 4096)], ids=["joint", "schedules"])
+def test_layer_step_same_with_a_second_stream_and_captured(shape, device):
+    """A recording forward and its backward give the same bits on one stream, on two and replayed from a HIP graph, and the output of the call without autograd:
+    that one may sum the experts in another order, so that a result lands on the neighbouring value (half an ulp of either term, far below eps in the 2-norm)."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    torch.manual_seed(5)
+    T, H, I = shape
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", 1024, 8)).to(device=device, dtype=torch.bfloat16).train()
+    x, dy = (torch.randn(1, T, H, device=device).bfloat16() for _ in range(2))
+    leaves = [x.requires_grad_(), *layer.parameters()]
+
+    def step():
+        y = layer(x)
+        return [y.detach(), *torch.autograd.grad(y, leaves, dy)]
+    layer.overlap_branches = False
+    want = step()
+    with torch.no_grad():
+        plain = layer(x).float()
+    assert ((want[0].float() - plain).norm() <= torch.finfo(torch.bfloat16).eps * plain.norm()).item()
+    layer.overlap_branches = True
+    warm = torch.cuda.Stream()
+    warm.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(warm):
+        other = step()
+    torch.cuda.current_stream().wait_stream(warm)
+    assert all(torch.equal(a, b) for a, b in zip(want, other))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step()
+    for _ in range(3):
+        for g in got:
+            g.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(want, got))
+        assert all(torch.equal(a, b) for a, b in zip(want, step()))      # eager work between the replays
+        torch.cuda.synchronize()
+
+
 # T, H, N, k: a backward pass that gathers, one that splits
 @pytest.mark.parametrize("case", [(1000, 512, 1024, 8), (4100, 512, 2050, 16)], ids=["gather", "split"])
 def test_pair_scores_are_kept_where_the_backward_reads_them(case, device):
