@@ -222,7 +222,43 @@ struct BnFinalArgs {
   int num_rows, r, strips, training, stat_dt;
   int count_here;                    // increment num_batches_tracked in this kernel (no select kernel follows; momentum >= 0 only)
   float momentum, eps;               // momentum < 0: cumulative moving average, factor 1 / (batches tracked so far + 1)
+  int parts;                         // 0, or the parts of merge_statistics whose order of the sums is taken
 };
+
+__device__ __forceinline__ double of_lane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane), __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// A column's sums in the order of merge_statistics: part p over the strips p, p + parts, ..., then part after part.  Every lane ends with them.
+// (A lane to a part, where the 64 folded sums use all lanes; eight strips requested ahead make up for it: two-stream layer of hidden 1024 x 4096, 4096 tokens x 64 keys
+// 123.4 us with the folded sums, 123.1 with these, 8192 x 32 keys 211.9 / 212.0.  Strips one after the other: 120.8 / 124.3 at 4096.)
+__device__ __forceinline__ ColumnSums sums_by_parts(const BnFinalArgs& g, const int col) {
+  const int lane = lane_id();
+  ColumnSums all{0., 0.};
+  for (int p0 = 0; p0 < g.parts; p0 += kWave) {
+    ColumnSums c{0., 0.};
+    if (p0 + lane < g.parts) {
+      constexpr int kAhead = 8;                                 // strips requested before the first is waited for
+      for (int first = p0 + lane; first < g.strips; first += kAhead * g.parts) {
+        float mean[kAhead], m2[kAhead];
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+          const int64_t at = int64_t(min(first + j * g.parts, g.strips - 1)) * 2 * g.r + col;
+          mean[j] = g.part_mean[at];
+          m2[j] = g.part_m2[at];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j)
+          if (first + j * g.parts < g.strips) add_strip(c, mean[j], m2[j], first + j * g.parts, g.num_rows);
+      }
+    }
+    for (int q = 0; q < min(kWave, g.parts - p0); ++q) {
+      all.weighted += of_lane(c.weighted, q);
+      all.squares += of_lane(c.squares, q);
+    }
+  }
+  return all;
+}
 
 // One wave per column: merges the strip partials, writes mean and 1/sqrt(var+eps), and in
 // training moves the running buffers (unbiased variance) as nn.BatchNorm1d does.  In eval
@@ -241,15 +277,18 @@ __global__ __launch_bounds__(256) void bn_finalize_kernel(const BnFinalArgs g) {
     const float rm = load_score(g.running_mean[half], key, g.stat_dt), rv = load_score(g.running_var[half], key, g.stat_dt);
     const float f = g.momentum >= 0.f ? g.momentum : 1.0f / (float)(*g.num_batches_tracked[half] + 1);
     ColumnSums c{0., 0.};
-    for (int strip = lane; strip < g.strips; strip += kWave) add_strip(c, g.part_mean, g.part_m2, strip, 2 * g.r, col, g.num_rows);
-    double sum2[2] = {c.weighted, c.squares};
+    if (g.parts) {
+      c = sums_by_parts(g, col);
+    } else {
+      for (int strip = lane; strip < g.strips; strip += kWave) add_strip(c, g.part_mean, g.part_m2, strip, 2 * g.r, col, g.num_rows);
 #pragma unroll
-    for (int m = kWave / 2; m >= 1; m >>= 1) {
-      const double o0 = __shfl_xor(sum2[0], m, kWave), o1 = __shfl_xor(sum2[1], m, kWave);
-      sum2[0] += o0;
-      sum2[1] += o1;
+      for (int m = kWave / 2; m >= 1; m >>= 1) {
+        const double o0 = __shfl_xor(c.weighted, m, kWave), o1 = __shfl_xor(c.squares, m, kWave);
+        c.weighted += o0;
+        c.squares += o1;
+      }
     }
-    const ColumnStats v = column_stats(ColumnSums{sum2[0], sum2[1]}, g.num_rows);
+    const ColumnStats v = column_stats(c, g.num_rows);
     mean = v.mean;
     var = v.var;
     if (lane == 0) {
@@ -358,8 +397,10 @@ int router_fwd(const void* x, const void* weight_x, const void* weight_y,
   // Training, up to 64 keys per half and 128 KiB of partial statistics: the selecting blocks merge them themselves.  16 waves to a block beyond 2048 tokens (as many
   // merges as CUs), 8 below (more CUs).  Whole call in three launches / two, top-16 and 64 keys: 1024 tokens 15.0 -> 13.7 us, 2048 15.7 -> 14.4 (16 waves 15.9), 4096
   // 18.4 -> 17.3 (8 waves 18.5); 32 keys: 256 13.3 -> 11.8, 8192 27.6 -> 25.6.  More keys: 2048 x 100 17.8 -> 23-30, 1500 x 128 21 -> 28-30.  Beside another stream's
-  // kernels, which hide the launch, whole blocks of 16 waves would wait for a CU.
-  const bool merge = training && exclusive && k > 0 && dtype != OMNI_F32 && r <= kWave && merge_here(num_tokens, r) && merge_cells(r, k) <= 2;
+  // kernels, which hide the launch, whole blocks of 16 waves would wait for a CU: there it stays, and takes the blocks' order of the sums, so that the sizes
+  // alone give the bits.
+  const bool block_order = training && k > 0 && dtype != OMNI_F32 && r <= kWave && merge_here(num_tokens, r) && merge_cells(r, k) <= 2, merge = block_order && exclusive;
+  const int merge_waves = num_tokens > 2048 ? 16 : 8;
   SelectArgs g{};
   g.lx = z; g.ly = (const char*)z + (size_t)r * es; g.row_stride = 2 * r;
   g.scores = scores; g.gates = gates; g.indices = indices;
@@ -374,7 +415,7 @@ int router_fwd(const void* x, const void* weight_x, const void* weight_y,
   }
   if (merge) {
     g.part_mean = part_mean; g.part_m2 = part_m2; g.strips = (int)strips; g.momentum = momentum;
-    const hipError_t err = num_tokens > 2048 ? launch_select_merge<16>(g, s) : launch_select_merge<8>(g, s);
+    const hipError_t err = merge_waves == 16 ? launch_select_merge<16>(g, s) : launch_select_merge<8>(g, s);
     return err == hipSuccess ? OMNI_OK : OMNI_ERR_HIP_BASE + (int)err;
   }
   // Training: one more launch merges the partial statistics and moves the running buffers.  In eval mode the
@@ -382,7 +423,7 @@ int router_fwd(const void* x, const void* weight_x, const void* weight_y,
   if (training || k == 0) {
     BnFinalArgs b{part_mean, part_m2, stats, {running_mean_x, running_mean_y}, {running_var_x, running_var_y},
                   {num_batches_tracked_x, num_batches_tracked_y}, (int)num_tokens, r, (int)strips, training ? 1 : 0, stats_dtype,
-                  k == 0 ? 1 : 0, momentum, eps};
+                  k == 0 ? 1 : 0, momentum, eps, block_order ? merge_parts(r, merge_waves * kWave) : 0};
     hipLaunchKernelGGL(bn_finalize_kernel, dim3((2 * r + 3) / 4), dim3(256), 0, s, b);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return OMNI_ERR_HIP_BASE + (int)err;

@@ -51,10 +51,14 @@ constexpr int kBnRows = 32;       // rows per strip: one 32-row MFMA tile of the
 // One column's batch statistics from its strips' sums (mean = sum n_s mean_s / n, M2 = sum M2_s + n_s mean_s^2 - n mean^2, in double: 29 bits more than
 // the fp32 result keeps, so the difference stays exact to fp32 while mean^2 / variance < 2^29).
 struct ColumnSums { double weighted, squares; };
-__device__ __forceinline__ void add_strip(ColumnSums& c, const float* part_mean, const float* part_m2, int strip, int cols, int col, int num_rows) {
-  const double ns = (double)min(kBnRows, num_rows - strip * kBnRows), ms = (double)part_mean[int64_t(strip) * cols + col];
+__device__ __forceinline__ void add_strip(ColumnSums& c, float mean, float m2, int strip, int num_rows) {
+  const double ns = (double)min(kBnRows, num_rows - strip * kBnRows), ms = (double)mean;
   c.weighted += ns * ms;
-  c.squares += (double)part_m2[int64_t(strip) * cols + col] + ns * ms * ms;
+  c.squares += (double)m2 + ns * ms * ms;
+}
+__device__ __forceinline__ void add_strip(ColumnSums& c, const float* part_mean, const float* part_m2, int strip, int cols, int col, int num_rows) {
+  const int64_t at = int64_t(strip) * cols + col;
+  add_strip(c, part_mean[at], part_m2[at], strip, num_rows);
 }
 struct ColumnStats { float mean, var, unbiased; };             // var: biased, normalises the batch
 __device__ __forceinline__ ColumnStats column_stats(const ColumnSums& c, int num_rows) {
@@ -67,8 +71,9 @@ __device__ __forceinline__ float rstd_of(float var, float eps) { return 1.0f / s
 // which the tiles hide, where a merge of its own is a 4-5 us launch between projection and selection.  (A selection by itself: where router_fwd says.)  lds: merge_lds_floats(r, threads) floats, 16-byte aligned; the first 4r hold mean_x, rstd_x,
 // mean_y, rstd_y afterwards.
 __device__ __host__ constexpr int merge_lds_floats(int r, int threads) { return (4 * r + 3) / 4 * 4 + 4 * threads; }
+__device__ __host__ constexpr int merge_parts(int r, int threads) { return threads / (2 * r) > 1 ? threads / (2 * r) : 1; }      // a column's sums are the parts' strided ones, in their order
 __device__ __forceinline__ void merge_statistics(const SelectArgs& g, float* lds, const int threads) {
-  const int cols = 2 * g.r, tid = threadIdx.x, parts = max(threads / cols, 1);
+  const int cols = 2 * g.r, tid = threadIdx.x, parts = merge_parts(g.r, threads);
   ColumnSums* sums = (ColumnSums*)(lds + (4 * g.r + 3) / 4 * 4);
   for (int c0 = 0; c0 < cols; c0 += threads) {                  // (one round up to threads / 2 keys)
     const int part = tid / cols, col = c0 + (parts > 1 ? tid - part * cols : tid);

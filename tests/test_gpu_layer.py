@@ -155,6 +155,46 @@ def test_router_fwd_merges_statistics_where_it_selects(case, dtype, device):
         assert d[2].item() == 2
 
 
+# eight waves a block and sixteen, 4 to 64 sums of a column, an odd number of keys, a partial strip, more than 64 strips
+@pytest.mark.parametrize("case", [(70, 60), (700, 2), (700, 3), (2100, 6), (700, 12), (700, 20), (2100, 33), (1000, 60), (2100, 60)], ids=lambda c: "T%d-r%d" % c)
+def test_batch_statistics_on_one_stream_and_two(case, device):
+    """A layer on one stream merges the batch statistics where it selects, on two in a launch of their own: one order of the double sums, so the same buffers to the
+    bit also where that order shows.  Pairs of strips of values up to 2^59 cancel exactly; what is left beside them (strips of about 1000) loses the bits below
+    2^11 or so in one order and others in another."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, r = case
+    H, I, k = 128, 256, 2
+    print(f"statistics on one stream and two T={T} r={r} k={k}", flush=True)
+    g = torch.Generator().manual_seed(T + r)
+    strips = (T + 31) // 32
+    big = torch.zeros(strips)
+    order = torch.randperm(T // 32, generator=g)
+    for a, b in zip(order[0::4].tolist(), order[1::4].tolist()):        # half of the whole strips in pairs
+        big[a] = (1.0 + torch.rand((), generator=g)) * 2.0 ** torch.randint(50, 59, (), generator=g)
+        big[b] = -big[a]
+    x = torch.randn(T, H, generator=g)
+    x[:, 0] = torch.where(big != 0, big, 1000.0 * torch.randn(strips, generator=g)).repeat_interleave(32)[:T]
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", r * r, k)).to(device=device, dtype=torch.bfloat16)
+    norms = layer.router_norm_x.float(), layer.router_norm_y.float()
+    for w in (layer.router_gate_x.weight, layer.router_gate_y.weight):
+        w.copy_(torch.randn(r, H, generator=g) * H ** -0.5)
+        w[:, 0] = 1.0
+    layer.overlap_min_work = 0
+    x = x.to(device=device, dtype=torch.bfloat16)
+    left = []
+    for two in (False, True):
+        layer.overlap_branches = two
+        for n in norms:
+            n.reset_running_stats()
+        layer(x[None])
+        left.append([b.clone() for n in norms for b in n.buffers()])
+    stats = [b for n in norms for b in (torch.zeros_like(n.running_mean), torch.ones_like(n.running_var), torch.zeros_like(n.num_batches_tracked))]
+    _ops().hip_omni_router_fwd_func(x, layer.router_gate_x.weight, layer.router_gate_y.weight, *stats, k, training=True)
+    assert all(torch.isfinite(b).all() for b in stats)
+    for one, two, alone in zip(*left, stats):
+        assert torch.equal(one, two) and torch.equal(one, alone)
+
+
 def test_router_fwd_select_is_exact_given_same_logprobs(device):
     """Feeding the oracle's selection the device's own scores must reproduce the device's ids
     bit for bit: run the fused router, rebuild the log-probs it saw from its z, compare."""
