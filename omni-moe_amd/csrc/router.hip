@@ -236,22 +236,8 @@ __device__ __forceinline__ ColumnSums sums_by_parts(const BnFinalArgs& g, const 
   ColumnSums all{0., 0.};
   for (int p0 = 0; p0 < g.parts; p0 += kWave) {
     ColumnSums c{0., 0.};
-    if (p0 + lane < g.parts) {
-      constexpr int kAhead = 8;                                 // strips requested before the first is waited for
-      for (int first = p0 + lane; first < g.strips; first += kAhead * g.parts) {
-        float mean[kAhead], m2[kAhead];
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-          const int64_t at = int64_t(min(first + j * g.parts, g.strips - 1)) * 2 * g.r + col;
-          mean[j] = g.part_mean[at];
-          m2[j] = g.part_m2[at];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j)
-          if (first + j * g.parts < g.strips) add_strip(c, mean[j], m2[j], first + j * g.parts, g.num_rows);
-      }
-    }
+    if (p0 + lane < g.parts)
+      for (int first = p0 + lane; first < g.strips; first += 8 * g.parts) add_batch<8>(c, g.part_mean, g.part_m2, first, g.parts, g.strips, 2 * g.r, col, g.num_rows);
     for (int q = 0; q < min(kWave, g.parts - p0); ++q) {
       all.weighted += of_lane(c.weighted, q);
       all.squares += of_lane(c.squares, q);
