@@ -214,6 +214,11 @@ OMNI_API int32_t omni_probe_mfma(const void* operands, float* sink, int32_t num_
  * issue iters x 32 of them (iters * 32 * 16384 flop per wave).  sink: num_blocks * 512 floats, overwritten.  Under the
  * board's power limit this instruction sustains more than the 32x32x16 one on the same operand bits. */
 OMNI_API int32_t omni_probe_mfma16(const void* operands, float* sink, int32_t num_blocks, int32_t iters, void* stream);
+/* Diagnostic: the tiles that a 16-bit layer's joint launches take at these sizes, from the sizes alone (nothing is launched).  pair[2]: rows and columns of
+ * those that the router's projection shares with the gate/up projection (0: a launch for each); down[4]: rows and columns of the down projection's, the
+ * parts of its K, and 1 if the selection runs beside them. */
+OMNI_API int32_t omni_probe_joint_tiles(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t num_expert_sqrt,
+                                        int32_t num_experts_per_token, int32_t* pair, int32_t* down);
 
 /* y[i] = round(y[i] + addend[i]) in place: the layer's final  mlp + experts  (omni_moe.py:102) as a
  * call of its own, for callers that run the two branches on different streams.  num_elements a
@@ -399,13 +404,14 @@ OMNI_API int32_t omni_moe_fwd_algo(const void* x, const void* gate_weight, const
                                    int32_t training, float momentum, float eps, void* workspace, void* stream,
                                    void* side_stream, void* fork_event, void* join_event, int32_t expert_algo);
 
-/* omni_moe_fwd for a differentiable call: the same result, and what the layer's backward pass reads stays with the caller.
+/* omni_moe_fwd for a differentiable call: the same sums and rounding points, and what the layer's backward pass reads stays with the caller.
  *   router_workspace : omni_router_workspace_bytes() bytes, as omni_router_fwd leaves it (z, and the statistics at
  *                      omni_router_workspace_stats_offset())
  *   gates, indices   : [T,k]; scores: NULL, or [T,k] fp32 for the pair scores (where omni_expert_bwd_reads_scores())
  *   gate, up, h      : [T,I], the rounded projections and their SwiGLU product
  *   workspace        : omni_moe_save_workspace_bytes() bytes; free again once the work has run.
- * The expert algorithm is AUTO's; ids beyond the tables add nothing and are no error.  Replaces OmniMoE.forward under autograd (omni_moe.py:60-106). */
+ * The expert algorithm is AUTO's; where scores are kept the experts' sums may run in another order than in omni_moe_fwd.  Ids beyond the tables add
+ * nothing and are no error.  Replaces OmniMoE.forward under autograd (omni_moe.py:60-106). */
 OMNI_API size_t omni_moe_save_workspace_bytes(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int64_t num_experts,
                                               int32_t num_experts_per_token, int32_t dtype);
 OMNI_API int32_t omni_moe_save_fwd(const void* x, const void* gate_weight, const void* up_weight, const void* down_weight,

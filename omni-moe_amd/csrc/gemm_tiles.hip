@@ -58,6 +58,22 @@ static TileChoice choose_down(const TileSize& size, int64_t K, bool may_split) {
   const TileChoice any = choose_tiles(kTilePlain, &size, 1, K, may_split), joint = choose_tiles(kTilePlain, &size, 1, K, may_split, kJointShapes);
   return joint.us <= any.us + kSelectUs ? joint : any;
 }
+// The shape that both products' tiles take least time in, by the figures above, if that is less than a launch for each; -1: it is not
+static int choose_pair(const TileSize& router, const TileSize& mlp, int64_t K) {
+  const TileSize sizes[2] = {router, mlp};
+  const int64_t kt = (K + 63) / 64;
+  int shape = -1;
+  float best = choose_tiles(kTileTwo, sizes, 1, K, false).us + choose_tiles(kTileSwiglu, sizes + 1, 1, K, true).us;
+  for (int i = 0; i < kShapes; ++i) {
+    if (!(kJointShapes >> i & 1)) continue;                    // (256 x 256: 30.6 us at 1024 tokens, where the two launches take 25.8)
+    const ShapeCost &r = kCost[i], &m = i == 4 ? kSwigluCost : kCost[i];
+    if (r.kg > 1 && K < 512) continue;
+    const int64_t n = ((router.M + r.bm - 1) / r.bm) * ((router.N + r.bn - 1) / r.bn) + ((mlp.M + m.bm - 1) / m.bm) * ((mlp.N + m.bn / 2 - 1) / (m.bn / 2));
+    const float us = m.fixed + (float)kt * step_us(m, n);
+    if (us < best) { best = us; shape = i; }
+  }
+  return shape;
+}
 static size_t parts_bytes(const TileChoice& c, int64_t M, int64_t columns) { return c.splits > 1 ? (size_t)c.splits * (size_t)M * (size_t)columns * 4 : 0; }
 
 size_t tile_workspace_bytes(int epilogue, int64_t M, int64_t N, int64_t K) {
@@ -102,19 +118,7 @@ bool launch_tile_pair(int dtype, const TileProduct& router, const TileProduct& m
   TilePair g;
   g.router.p[0] = router;
   g.mlp.p[0] = mlp;
-  // The shape that both products' tiles take least time in, by the figures above, if that is less than a launch for each
-  const TileSize sizes[2] = {{router.M, router.N}, {mlp.M, mlp.N}};
-  const int64_t K = mlp.seg[0].K, kt = (K + 63) / 64;
-  int shape = -1;
-  float best = choose_tiles(kTileTwo, sizes, 1, K, false).us + choose_tiles(kTileSwiglu, sizes + 1, 1, K, true).us;
-  for (int i = 0; i < kShapes; ++i) {
-    if (!(kJointShapes >> i & 1)) continue;                    // (256 x 256: 30.6 us at 1024 tokens, where the two launches take 25.8)
-    const ShapeCost &r = kCost[i], &m = i == 4 ? kSwigluCost : kCost[i];
-    if (r.kg > 1 && K < 512) continue;
-    const int64_t n = ((router.M + r.bm - 1) / r.bm) * ((router.N + r.bn - 1) / r.bn) + ((mlp.M + m.bm - 1) / m.bm) * ((mlp.N + m.bn / 2 - 1) / (m.bn / 2));
-    const float us = m.fixed + (float)kt * step_us(m, n);
-    if (us < best) { best = us; shape = i; }
-  }
+  const int shape = choose_pair(TileSize{router.M, router.N}, TileSize{mlp.M, mlp.N}, mlp.seg[0].K);
   return dtype == kBF16 ? tile_pair_of<kBF16>(shape, g, s, e) : tile_pair_of<kF16>(shape, g, s, e);
 }
 
@@ -127,3 +131,31 @@ hipError_t launch_tile_down(int dtype, const TileProduct& p, const SelectArgs& s
   return dtype == kBF16 ? tile_down_of<kBF16>(p, select, c, (float*)ws, s, selected, parts) : tile_down_of<kF16>(p, select, c, (float*)ws, s, selected, parts);
 }
 }  // namespace omni
+
+extern "C" OMNI_API int32_t omni_probe_joint_tiles(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t num_expert_sqrt, int32_t num_experts_per_token,
+                                                   int32_t* pair, int32_t* down) {
+  using namespace omni;
+  if (num_tokens <= 0 || num_tokens > INT32_MAX / 256 || hidden_size <= 0 || intermediate_size <= 0 || num_expert_sqrt <= 0 || num_experts_per_token <= 0) return OMNI_ERR_SHAPE;
+  if (num_experts_per_token > 128) return OMNI_ERR_TOPK;
+  if (!pair || !down) return OMNI_ERR_NULL;
+  const int shape = choose_pair(TileSize{num_tokens, 2 * (int64_t)num_expert_sqrt}, TileSize{num_tokens, intermediate_size}, hidden_size);
+  const TileChoice c = choose_down(TileSize{num_tokens, hidden_size}, intermediate_size, true);
+  SelectArgs select{};
+  select.r = num_expert_sqrt; select.k = num_experts_per_token;
+  const int cells = prepare_select(select), regs = (num_expert_sqrt + kWave - 1) / kWave, splits = c.splits < kMostDownParts ? c.splits : kMostDownParts;
+  auto plan = [&](auto id) { return plan_down<decltype(id)::value>(num_tokens, hidden_size, intermediate_size, splits, (int)num_tokens, regs, cells); };
+  DownPlan p{0, splits, 0, 0, false};                          // (tiles of 256 columns: nothing beside them)
+  if (c.shape == 1) p = plan(std::integral_constant<int, 1>{});
+  else if (c.shape == 2) p = plan(std::integral_constant<int, 2>{});
+  else if (c.shape == 3) p = plan(std::integral_constant<int, 3>{});
+  else if (c.shape == 4) p = plan(std::integral_constant<int, 4>{});
+  else if (c.shape == 7) p = plan(std::integral_constant<int, 7>{});
+  else if (c.shape == 8) p = plan(std::integral_constant<int, 8>{});
+  pair[0] = shape < 0 ? 0 : kCost[shape].bm;
+  pair[1] = shape < 0 ? 0 : kCost[shape].bn;
+  down[0] = kCost[c.shape].bm;
+  down[1] = kCost[c.shape].bn;
+  down[2] = p.splits;
+  down[3] = p.selected ? 1 : 0;
+  return OMNI_OK;
+}

@@ -858,31 +858,44 @@ static hipError_t launch_choice(TileGroup& g, const TileChoice& c, float* ws, bo
   }
 }
 
+// How the down projection runs on tiles of shape kId: ring steps of a part, parts, tiles of all parts, and the blocks of the selection beside them, if it is
+struct DownPlan { int steps, splits; int64_t tiles, blocks; bool selected; };
+template <int kId>
+static DownPlan plan_down(int64_t M, int64_t N, int K, int splits, int tokens, int regs, int cells) {
+  using S = Shape<kId>;
+  constexpr int kStep = 64 * S::KG, kWaves = S::WM * S::WN * S::KG, BM = S::WM * S::TM * 16, BN = S::WN * S::TN * 16;
+  const int total = (K + kStep - 1) / kStep;
+  const int64_t once = kCost[kId].at_once, want = (tokens + kWaves - 1) / kWaves;
+  const bool joint = total * kStep == K && regs <= 8 && cells <= 2;
+  auto split = [&](int n) {
+    DownPlan p;
+    p.steps = (total + n - 1) / n;
+    p.splits = (total + p.steps - 1) / p.steps;
+    p.tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * p.splits;
+    // the selection takes the places that the last round of tiles leaves free, when they make at most two tokens a wave (of more than 128 keys: one)
+    const int64_t free = (p.tiles + once - 1) / once * once - p.tiles;
+    p.blocks = want < free ? want : free;
+    p.selected = joint && (regs <= 2 ? 2 : 1) * p.blocks * kWaves >= tokens;
+    return p;
+  };
+  // ... for which a product in many splits gives up to a quarter of them (a launch is 5-7 us, a split step 0.2)
+  int n = splits;
+  DownPlan p = split(n);
+  while (!p.selected && n > 1 && n > splits * 3 / 4) p = split(--n);
+  return p.selected ? p : split(splits);
+}
 template <int DT, int kId>
 static hipError_t start_down(TileProduct p, const SelectArgs& select, int splits, float* ws, hipStream_t s, bool* selected, int* parts) {
   using S = Shape<kId>;
   constexpr int kStep = 64 * S::KG, kWaves = S::WM * S::WN * S::KG, kBytes = tile_lds<kId, false>();
-  const int total = (p.seg[0].K + kStep - 1) / kStep;
-  const int64_t once = kCost[kId].at_once, want = (select.num_tokens + kWaves - 1) / kWaves;
   TileSelect g{TileSingle{}, select, (select.r + kWave - 1) / kWave, 0};
   g.cells = prepare_select(g.select);
-  const bool joint = total * kStep == p.seg[0].K && g.regs <= 8 && g.cells <= 2;
-  int64_t tiles = 0, blocks = 0;
-  auto split = [&](int n) {
-    p.steps = (total + n - 1) / n;
-    p.splits = (total + p.steps - 1) / p.steps;
-    p.part = p.splits > 1 ? ws : nullptr;
-    tiles = tile_count<kId, false>(p) * p.splits;
-    // the selection takes the places that the last round of tiles leaves free, when they make at most two tokens a wave (of more than 128 keys: one)
-    const int64_t free = (tiles + once - 1) / once * once - tiles;
-    blocks = want < free ? want : free;
-    return joint && (g.regs <= 2 ? 2 : 1) * blocks * kWaves >= select.num_tokens;
-  };
-  // ... for which a product in many splits gives up to a quarter of them (a launch is 5-7 us, a split step 0.2)
-  int n = splits;
-  while (n > 1 && n > splits * 3 / 4 && !split(n)) --n;
-  *selected = split(n);
-  if (!*selected) split(splits);
+  const DownPlan plan = plan_down<kId>(p.M, p.N, p.seg[0].K, splits, select.num_tokens, g.regs, g.cells);
+  p.steps = plan.steps;
+  p.splits = plan.splits;
+  p.part = p.splits > 1 ? ws : nullptr;
+  const int64_t tiles = plan.tiles, blocks = plan.blocks;
+  *selected = plan.selected;
   *parts = p.splits;
   if (tiles > INT32_MAX / 2) return hipErrorInvalidValue;
   if (*selected) {

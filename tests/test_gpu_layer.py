@@ -871,13 +871,33 @@ def test_joint_launches_match_the_operators(case, dtype, device):
     assert (got - (mlp + experts)).abs().max().item() <= 4 * eps * max(1.0, float((mlp + experts).abs().max()))
 
 
-# T, H, I, N, k: the joint projections on tiles of 256, 192 and 96 rows of 128 columns, whole and one row past them; the down projection on 96 and 192 rows,
-# split along K and not, with the selection beside it
+# T, H, I, N, k: the joint projections on tiles of 256, 192 and 96 rows of 128 columns, whole and one row past them; the down projection on tiles of 64 x 64, 96 x 128 and
+# 128 x 128, split along K and not (test_joint_launches_select_beside_every_tile: the others, and the selection beside each)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("case", [(613, 1024, 4096, 4096, 16), (97, 136, 2056, 576, 8), (192, 264, 4104, 576, 8), (385, 264, 4104, 576, 8), (768, 776, 2568, 1024, 4),
                                   (1153, 776, 2568, 576, 8), (1153, 264, 4104, 576, 6), (1200, 1024, 4096, 4096, 16), (1500, 1024, 4096, 1024, 8)],
                          ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
 def test_joint_launches_on_lower_tiles(case, dtype, device):
+    test_joint_launches_match_the_operators(case, dtype, device)
+
+
+# T, H, I, N, k, and rows, columns and parts of the down projection's tiles beside which the selection runs; of batch statistics the selecting blocks merge (r <= 128)
+DOWN_CASES = [((950, 2048, 4096, 1024, 8), (192, 128, 2)), ((1295, 3128, 128, 64, 8), (192, 128, 1)), ((385, 2208, 7616, 4096, 8), (256, 128, 6)),
+              ((805, 2048, 4096, 1024, 8), (128, 128, 1)), ((583, 520, 4096, 1024, 8), (96, 128, 5)), ((879, 520, 256, 1024, 8), (96, 128, 1)),
+              ((213, 512, 4096, 1024, 8), (64, 64, 7)), ((657, 768, 1024, 1024, 8), (64, 64, 1)), ((694, 1536, 4096, 1024, 8), (128, 128, 2))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case, tiles", DOWN_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_joint_launches_select_beside_every_tile(case, tiles, dtype, device):
+    """The rule's choice is asked for first, so that figures fitted anew cannot take a kernel out of the test unnoticed."""
+    import ctypes
+    import math
+    from omni_moe.ops.hip import _lib
+    T, H, I, N, k = case
+    pair, down = (ctypes.c_int32 * 2)(), (ctypes.c_int32 * 4)()
+    assert _lib.load().omni_probe_joint_tiles(T, H, I, math.isqrt(N), k, ctypes.addressof(pair), ctypes.addressof(down)) == 0
+    assert tuple(down) == (*tiles, 1)
     test_joint_launches_match_the_operators(case, dtype, device)
 
 
