@@ -195,6 +195,26 @@ def test_batch_statistics_on_one_stream_and_two(case, device):
         assert torch.equal(one, two) and torch.equal(one, alone)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", [(300, 128, 16, 8), (2100, 128, 64, 16)], ids=lambda c: "T%d-H%d-r%d-k%d" % c)
+def test_router_fwd_cumulative_average_where_it_selects(case, dtype, device):
+    """momentum=None with the statistics merged by the selecting blocks: the factor 1 / (batches so far + 1) is read before the count moves on."""
+    T, H, r, k = case
+    g = torch.Generator().manual_seed(T)
+    wx, wy = ((torch.randn(r, H, generator=g) / H ** 0.5).to(dtype) for _ in range(2))
+    bx, by = oracle.BNState.fresh(r), oracle.BNState.fresh(r)
+    dbx, dby = _bn_buffers(r, torch.float32, device), _bn_buffers(r, torch.float32, device)
+    print(f"router_fwd cumulative T={T} H={H} r={r} k={k} {dtype}", flush=True)
+    for step in range(3):
+        x = (torch.randn(T, H, generator=g) * (1.0 + step)).to(dtype)
+        oracle.router_forward(x, wx, wy, bx, by, k, True, momentum=None)
+        _ops().hip_omni_router_fwd_func(x.to(device), wx.to(device), wy.to(device), *dbx, *dby, k, training=True, momentum=None)
+        for d, b in ((dbx, bx), (dby, by)):
+            torch.testing.assert_close(d[0].cpu(), b.running_mean, rtol=1e-3, atol=3e-4)       # (three times the spread of the test above in the last batch)
+            torch.testing.assert_close(d[1].cpu(), b.running_var, rtol=1e-3, atol=1e-4)
+            assert d[2].item() == step + 1
+
+
 def test_router_fwd_select_is_exact_given_same_logprobs(device):
     """Feeding the oracle's selection the device's own scores must reproduce the device's ids
     bit for bit: run the fused router, rebuild the log-probs it saw from its z, compare."""
