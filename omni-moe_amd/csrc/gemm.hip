@@ -1129,6 +1129,7 @@ hipError_t launch_f32_joint(const void* x, const void* wx, const void* wy, void*
   const F32Front f{router, mlp, (int)rb};
   constexpr int kDown = SmallF32Lds<kEpiPlain, 2>::kBytes;
   static_assert(kDown >= 4 * merge_lds_floats(kMergeKeys, kGemmThreads), "a block that selects merges statistics there");
+  static_assert(kGemmThreads == kF32MergeThreads, "the order of its sums is also the two-stream schedule's");
   auto start = [&](auto kernel, LdsKernel& entry, int bytes, int64_t blocks, const auto& a) {
     if ((e = entry.ensure()) != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kGemmThreads), bytes, s, a);

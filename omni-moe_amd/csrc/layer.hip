@@ -21,14 +21,15 @@ bool joint_launches_gather(int algo, int64_t T, int H, int64_t N, int k, int dty
 // defined beside the select kernels: whether they take num_expert_sqrt keys per half with top_k and this dtype
 bool select_covers(int r, int k, int dtype);
 int launch_router_select(const SelectArgs& g, hipStream_t s);
-// defined there: omni_router_fwd, with the caller's word on whether the call has the GPU to itself
+// defined there: omni_router_fwd, with the caller's word on whether the call has the GPU to itself, and (0: none) the block size of the joint launches whose order
+// the batch statistics' sums take
 int router_fwd(const void* x, const void* weight_x, const void* weight_y,
                void* running_mean_x, void* running_var_x, int64_t* num_batches_tracked_x,
                void* running_mean_y, void* running_var_y, int64_t* num_batches_tracked_y,
                int32_t training, float momentum, float eps, void* gates, int32_t* indices,
                void* scores, int64_t num_tokens, int32_t hidden_size, int32_t num_expert_sqrt,
                int32_t num_experts_per_token, int32_t dtype, int32_t stats_dtype,
-               void* workspace, void* stream, bool exclusive);
+               void* workspace, void* stream, bool exclusive, int order_threads);
 // defined beside the expert kernels: the gather algorithm with the final add (shared: AUTO's, whose waves may share a token's slots)
 hipError_t launch_gather_add(const void* x, const void* up, const void* down, const void* gates, const int32_t* ids, void* y, const float* parts, int splits, bool shared, int64_t T,
                              int H, int k, int64_t N, int dtype, hipStream_t s);
@@ -255,7 +256,8 @@ static int moe_fwd(const void* x, const void* gate_weight, const void* up_weight
   // for it before this call returns, so that an error leaves no work behind that the caller cannot order.
   const bool alone = side_stream == nullptr;            // one stream: every kernel runs by itself
   int e = router_fwd(x, router_weight_x, router_weight_y, running_mean_x, running_var_x, num_batches_tracked_x, running_mean_y, running_var_y, num_batches_tracked_y,
-                     training, momentum, eps, gates, ids, nullptr, num_tokens, hidden_size, num_expert_sqrt, num_experts_per_token, dtype, stats_dtype, router_ws, branch, alone);
+                     training, momentum, eps, gates, ids, nullptr, num_tokens, hidden_size, num_expert_sqrt, num_experts_per_token, dtype, stats_dtype, router_ws, branch, alone,
+                     f32_sizes ? kF32MergeThreads : 0);
   // Beside the side branch the gate/up projection keeps its one-block-per-tile grid while that is at most two rounds of 256 tiles
   // (CUs come free between the rounds); with more tiles the streaming form wins although it holds every CU (hidden 1024 x
   // intermediate 4096, two streams: 4096 tokens 125.7 against 128.0 us, 6144 tokens 188.9 against 178.5, 8192 tokens 243.5 against 228.7)

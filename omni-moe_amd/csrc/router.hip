@@ -346,14 +346,14 @@ extern "C" OMNI_API size_t omni_router_workspace_stats_offset(int64_t num_tokens
 }
 
 namespace omni {
-// exclusive: nothing is meant to run beside the call
+// exclusive: nothing is meant to run beside the call.  order_threads: 0, or the block size of the joint launches whose order the batch statistics' sums take
 int router_fwd(const void* x, const void* weight_x, const void* weight_y,
                void* running_mean_x, void* running_var_x, int64_t* num_batches_tracked_x,
                void* running_mean_y, void* running_var_y, int64_t* num_batches_tracked_y,
                int32_t training, float momentum, float eps, void* gates, int32_t* indices,
                void* scores, int64_t num_tokens, int32_t hidden_size, int32_t num_expert_sqrt,
                int32_t num_experts_per_token, int32_t dtype, int32_t stats_dtype,
-               void* workspace, void* stream, bool exclusive) {
+               void* workspace, void* stream, bool exclusive, int order_threads) {
   const int r = num_expert_sqrt, k = num_experts_per_token;
   if (num_tokens < 0 || num_tokens > INT32_MAX / 256 || r <= 0 || hidden_size <= 0) return OMNI_ERR_SHAPE;
   if (k < 0 || (int64_t)k > (int64_t)r * r || k > 128 || (k & 1)) return OMNI_ERR_TOPK;
@@ -409,7 +409,7 @@ int router_fwd(const void* x, const void* weight_x, const void* weight_y,
   if (training || k == 0) {
     BnFinalArgs b{part_mean, part_m2, stats, {running_mean_x, running_mean_y}, {running_var_x, running_var_y},
                   {num_batches_tracked_x, num_batches_tracked_y}, (int)num_tokens, r, (int)strips, training ? 1 : 0, stats_dtype,
-                  k == 0 ? 1 : 0, momentum, eps, block_order ? merge_parts(r, merge_waves * kWave) : 0};
+                  k == 0 ? 1 : 0, momentum, eps, order_threads ? merge_parts(r, order_threads) : block_order ? merge_parts(r, merge_waves * kWave) : 0};
     hipLaunchKernelGGL(bn_finalize_kernel, dim3((2 * r + 3) / 4), dim3(256), 0, s, b);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return OMNI_ERR_HIP_BASE + (int)err;
@@ -428,5 +428,5 @@ extern "C" OMNI_API int32_t omni_router_fwd(const void* x, const void* weight_x,
                                             int32_t num_experts_per_token, int32_t dtype, int32_t stats_dtype,
                                             void* workspace, void* stream) {
   return omni::router_fwd(x, weight_x, weight_y, running_mean_x, running_var_x, num_batches_tracked_x, running_mean_y, running_var_y, num_batches_tracked_y, training, momentum, eps,
-                          gates, indices, scores, num_tokens, hidden_size, num_expert_sqrt, num_experts_per_token, dtype, stats_dtype, workspace, stream, true);
+                          gates, indices, scores, num_tokens, hidden_size, num_expert_sqrt, num_experts_per_token, dtype, stats_dtype, workspace, stream, true, 0);
 }

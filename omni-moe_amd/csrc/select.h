@@ -88,6 +88,7 @@ __device__ __forceinline__ float rstd_of(float var, float eps) { return 1.0f / s
 // not unrolled 25.2, now 24.8; 2000 tokens 44.8, 46.8, 43.3).  lds: merge_lds_floats(r, threads) floats, 16-byte aligned; the first 4r hold mean_x, rstd_x,
 // mean_y, rstd_y afterwards.
 __device__ __host__ constexpr int merge_lds_floats(int r, int threads) { return (4 * r + 3) / 4 * 4 + 4 * threads; }
+constexpr int kF32MergeThreads = 256;                         // of a block that merges in the single-precision layer's joint launches
 __device__ __host__ constexpr int merge_parts(int r, int threads) { return threads / (2 * r) > 1 ? threads / (2 * r) : 1; }      // a column's sums are the parts' strided ones, in their order
 __device__ __forceinline__ void merge_statistics(const SelectArgs& g, float* lds, const int threads) {
   const int cols = 2 * g.r, tid = threadIdx.x, parts = merge_parts(g.r, threads);

@@ -155,17 +155,9 @@ def test_router_fwd_merges_statistics_where_it_selects(case, dtype, device):
         assert d[2].item() == 2
 
 
-# eight waves a block and sixteen, 4 to 64 sums of a column, an odd number of keys, a partial strip, more than 64 strips
-@pytest.mark.parametrize("case", [(70, 60), (700, 2), (700, 3), (2100, 6), (700, 12), (700, 20), (2100, 33), (1000, 60), (2100, 60)], ids=lambda c: "T%d-r%d" % c)
-def test_batch_statistics_on_one_stream_and_two(case, device):
-    """A layer on one stream merges the batch statistics where it selects, on two in a launch of their own: one order of the double sums, so the same buffers to the
-    bit also where that order shows.  Pairs of strips of values up to 2^59 cancel exactly; what is left beside them (strips of about 1000) loses the bits below
-    2^11 or so in one order and others in another."""
-    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
-    T, r = case
-    H, I, k = 128, 256, 2
-    print(f"statistics on one stream and two T={T} r={r} k={k}", flush=True)
-    g = torch.Generator().manual_seed(T + r)
+def _cancelling_strips(T, H, g):
+    """Rows whose first column has half of the whole strips of 32 in pairs of +-values up to 2^59, which cancel exactly, and values of about 1000 in the others: every order of the
+    strips' double sums loses other bits of what is left."""
     strips = (T + 31) // 32
     big = torch.zeros(strips)
     order = torch.randperm(T // 32, generator=g)
@@ -174,6 +166,20 @@ def test_batch_statistics_on_one_stream_and_two(case, device):
         big[b] = -big[a]
     x = torch.randn(T, H, generator=g)
     x[:, 0] = torch.where(big != 0, big, 1000.0 * torch.randn(strips, generator=g)).repeat_interleave(32)[:T]
+    return x
+
+
+# eight waves a block and sixteen, 4 to 64 sums of a column, an odd number of keys, a partial strip, more than 64 strips
+@pytest.mark.parametrize("case", [(70, 60), (700, 2), (700, 3), (2100, 6), (700, 12), (700, 20), (2100, 33), (1000, 60), (2100, 60)], ids=lambda c: "T%d-r%d" % c)
+def test_batch_statistics_on_one_stream_and_two(case, device):
+    """A layer on one stream merges the batch statistics where it selects, on two in a launch of their own: one order of the double sums, so the same buffers to the
+    bit also where that order shows."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, r = case
+    H, I, k = 128, 256, 2
+    print(f"statistics on one stream and two T={T} r={r} k={k}", flush=True)
+    g = torch.Generator().manual_seed(T + r)
+    x = _cancelling_strips(T, H, g)
     layer = OmniMoE(OmniMoEConfig(H, I, "silu", r * r, k)).to(device=device, dtype=torch.bfloat16)
     norms = layer.router_norm_x.float(), layer.router_norm_y.float()
     for w in (layer.router_gate_x.weight, layer.router_gate_y.weight):
@@ -509,6 +515,33 @@ def test_layer_fp32_two_streams_equals_one_stream(case, algo, aligned, training,
         layer.overlap_branches = True
         assert _waits_for_side_stream(layer, x)
         assert torch.equal(layer(x), ref)
+
+
+@pytest.mark.parametrize("case", [(70, 64), (512, 32), (700, 64), (1100, 32), (700, 96), (700, 128)], ids=lambda c: "T%d-r%d" % c)
+def test_fp32_batch_statistics_on_one_stream_and_two(case, device):
+    """The joint launches' blocks merge the batch statistics of a small single-precision layer, on two streams a launch of its own: one order of the double sums."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, r = case
+    H, I, k = 128, 256, 8
+    print(f"fp32 statistics on one stream and two T={T} r={r}", flush=True)
+    g = torch.Generator().manual_seed(T + r)
+    x = _cancelling_strips(T, H, g).to(device)[None]
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", r * r, k)).to(device=device)
+    norms = layer.router_norm_x, layer.router_norm_y
+    for w in (layer.router_gate_x.weight, layer.router_gate_y.weight):
+        w.copy_(torch.randn(r, H, generator=g) * H ** -0.5)
+        w[:, 0] = 1.0
+    layer.overlap_min_work = 0
+    left = []
+    for two in (False, True):
+        layer.overlap_branches = two
+        for n in norms:
+            n.reset_running_stats()
+        layer(x)
+        left.append([b.clone() for n in norms for b in n.buffers()])
+    assert all(torch.isfinite(b).all() for b in left[0])
+    for one, two in zip(*left):
+        assert torch.equal(one, two)
 
 
 def test_layer_copies_and_saves_like_a_plain_module(device, tmp_path):
