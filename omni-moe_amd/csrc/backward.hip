@@ -16,9 +16,9 @@
 // every pair, in the organisation that the forward takes at the sizes: gather (one wave owns one token, keeps x_t, dy_t and the fp32 dx
 // accumulator in registers and fetches each selected up and down row once) or split (the rows in eight column slices, one to an XCD).
 // split takes s from the forward where that kept it; gather, which has the up rows in hand for dx, and split without it form it again.  Weight pass: the pairs are grouped by expert with the
-// stable schedule of the forward path; one wave owns one expert, walks its segment and gathers
-// the x and dy rows of the segment's tokens, so every dU/dV row is written exactly once
-// (zeros for experts nobody selected).
+// stable schedule of the forward path; a wave owns a chunk of that list for one part of the columns and
+// gathers the parts of its tokens' x or dy rows; long segments, which several waves share, are added by a fix-up, so every dU/dV row
+// is written exactly once (zeros for experts nobody selected).
 #include "common.h"
 #include "expert_split.h"
 #include "omni_moe_hip.h"
@@ -495,8 +495,8 @@ __global__ __launch_bounds__(kSortThreads) void expert_bwd_accumulate_kernel(con
 // address and factor are scalars, so a narrower part costs no exchange between lanes.  Rows of up to 512 bytes: x in the lower half of the lanes, dy in the
 // upper.  The finished rows pass the L2 by (non-temporal), which is left to the rows that are gathered.  The chunks, and with them the order of all sums, do not depend on the parts.  (4096 tokens x 16, hidden 1024, bf16 37.7 -> 24.3 us, 1024 x 32 over 16384
 // experts 23.7 -> 18.5.  The parts of a chunk one after the other instead, which keeps whole rows together: the whole backward there 54.4 -> 71.6 and 45.9 -> 51.5,
-// at 32768 tokens x 16 over 65536, which no L2 holds, 888 either way.  Four rows in flight, non-temporal: 16384 x 16 over 4096 232.8 -> 227.1, 8192 x 8 over 16384, hidden
-// 2048, 197.5 -> 189.1; sixteen rows or the next batch requested ahead: 1-3 % slower at 1024 and 4096 tokens.)
+// at 32768 tokens x 16 over 65536, which no L2 holds, 888 either way.  A recorded call of the experts, eight rows in flight -> four: 16384 x 16 over 4096 265.0 -> 261.5, 8192 x 8 over 16384,
+// hidden 2048, 221.6 -> 221.1; finished rows through the L2 -> past it: 261.3 -> 261.0 and 232.1 -> 220.7; sixteen rows or the next batch requested ahead: 1-3 % slower at 1024 and 4096 tokens.)
 struct WeightPass {
   const uint8_t *x, *dy;
   const float *ds, *coef;

@@ -50,8 +50,8 @@ hipError_t launch_tile_group(int dtype, int layout, int epilogue, TileGroup& g, 
 // What launch_tile_group wants for one product; K: the sum of its segments, each rounded up to 64
 size_t tile_workspace_bytes(int epilogue, int64_t M, int64_t N, int64_t K);
 
-// The layer's joint launches.  The router's projection (kTileTwo) in front of the gate/up projection (kTileSwiglu, nothing kept), both kNT over the same
-// K; false, and nothing launched, where its tiles would cost a round of their own or the operands are out of reach.
+// The layer's joint launches.  The router's projection (kTileTwo) in front of the gate/up projection (kTileSwiglu; gate and up kept where c2 and c3 say so), both kNT
+// over the same K; false, and nothing launched, where its tiles would cost a round of their own or the operands are out of reach.
 bool launch_tile_pair(int dtype, const TileProduct& router, const TileProduct& mlp, hipStream_t s, hipError_t* e);
 // The down projection (kTilePlain, kNT) and, beside it, the selection, if there is room (*selected).  *parts > 1: its sums are left in ws, [parts][M][N] fp32.
 struct SelectArgs;

@@ -689,7 +689,7 @@ constexpr int kShapes = 9;
 // 300 to 12000 rows, bf16, where the rule's choice takes 0.4 % more than the best shape on average and 9 % at most; about 4 us more for a launch.
 // The lower tiles took, the best of the others / now: gate/up of 3000 x 1024 x 4096 (256 tiles of 256 columns a round) 49.5 / 45.4 us, 613 x 1024 x 4096
 // 17.4 / 15.2; down of 3000 x 4096 x 1024 31.9 / 29.4, 12000 x 1536 x 512 23.7 / 19.6; five weight gradients of 4096 tokens x 1024 x 4096 (200 tiles of
-// 256 rows, 236 of 224) 118 / 107.
+// 256 rows, 236 of 224), in a trace of whole steps, 106 / 101.
 struct ShapeCost { int bm, bn, kg, at_once; float idle, full, fixed; };
 constexpr ShapeCost kCost[kShapes] = {{256, 256, 1, 256, 1.10f, 1.55f, 5.f}, {256, 128, 1, 256, 0.66f, 0.92f, 4.5f}, {128, 128, 1, 512, 0.50f, 1.00f, 4.f},
                                       {128, 128, 1, 256, 0.44f, 0.57f, 4.f}, {64, 64, 2, 256, 0.16f, 0.235f, 4.f}, {224, 256, 1, 256, 1.04f, 1.44f, 5.f},

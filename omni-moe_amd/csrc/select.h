@@ -761,7 +761,8 @@ static inline int num_cells(int k, int kp) {
   return n;
 }
 
-// Whether a joint launch's blocks merge the batch statistics: up to 128 KiB of them to a block
+// Whether the selecting blocks merge the batch statistics: up to 128 KiB of them to a block.  Both sides of the line, the router alone, its own launch / merged in the blocks:
+// 64 keys 4096 tokens 18.4 / 17.3 us, 4200 20.6 / 23.1, 5000 21.2 / 23.8, 8000 25.3 / 26.1; 32 keys 8192 27.6 / 25.6, 8300 23.7 / 25.5, 10000 25.1 / 27.1 (each pair on one box).
 static inline bool merge_here(int64_t num_tokens, int r) { return r <= kMergeKeys && (num_tokens + kBnRows - 1) / kBnRows * 2 * r <= 16384; }
 
 // What select_packed and its kernels want filled in beside the caller's fields; returns the candidate cells per lane
