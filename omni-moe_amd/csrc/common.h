@@ -66,46 +66,48 @@ template <> struct Elem<kF32> {
 // ---- wave-level primitives ---------------------------------------------------
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 
+// Another lane's value by a DPP control under which every lane reads a lane that is there.  With no value to keep and no lane left out, the exchange becomes an
+// operand of the instruction that takes it (where that has such a form), instead of a copy and a move in front of it.
+template <int CTRL> __device__ __forceinline__ int dpp_i(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true); }
+template <int CTRL> __device__ __forceinline__ float dpp_f(float v) { return __int_as_float(dpp_i<CTRL>(__float_as_int(v))); }
+enum : int { kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kQuadXor3 = 0x1B, kRowRor4 = 0x124, kRowXor8 = 0x128, kRowXor15 = 0x140, kRowXor7 = 0x141 };      // quad_perm, row_ror, row_mirror, row_half_mirror
+
 // Over all 64 lanes, in every lane: lane distances 32, 16, 8, 4, 2, 1.  The two swaps leave a lane with its own value and the other's in one order or the
 // other; from distance 8 on a rotation inside 16 lanes reaches the partner, or one that holds the same.  Six steps of register exchanges: through
 // ds_bpermute (__shfl_xor) each step is a round trip to LDS
 // (the layer for one token 19.9 -> 19.2 us, for 48 24.4 -> 23.9, the router stage at 4096 tokens 20.5 -> 20.2).
-template <class Op>
-__device__ __forceinline__ float wave_reduce(float v, Op&& op) {
+__device__ __forceinline__ float wave_sum(float v) {
   const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
-  v = op(__int_as_float((int)s32[0]), __int_as_float((int)s32[1]));
+  v = __int_as_float((int)s32[0]) + __int_as_float((int)s32[1]);
   const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
-  v = op(__int_as_float((int)s16[0]), __int_as_float((int)s16[1]));
-  auto dpp = [&](auto ctrl) __attribute__((always_inline)) {
-    const int i = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, decltype(ctrl)::value, 0xf, 0xf, false));
-  };
-  v = op(v, dpp(std::integral_constant<int, 0x128>{}));        // row_ror:8
-  v = op(v, dpp(std::integral_constant<int, 0x124>{}));        // row_ror:4
-  v = op(v, dpp(std::integral_constant<int, 0x4E>{}));         // quad_perm [2,3,0,1]
-  v = op(v, dpp(std::integral_constant<int, 0xB1>{}));         // quad_perm [1,0,3,2]
+  v = __int_as_float((int)s16[0]) + __int_as_float((int)s16[1]);
+  v += dpp_f<kRowXor8>(v);
+  v += dpp_f<kRowRor4>(v);
+  v += dpp_f<kQuadXor2>(v);
+  return v + dpp_f<kQuadXor1>(v);
+}
+// Spelled out: fmaxf is two instructions more a step, which quiet signalling NaNs (no arithmetic result is one).  The waits are what a DPP operand asks for behind the
+// instruction that wrote it; the last one is for a DPP operand of the compiler's, who does not see what wrote this one.
+__device__ __forceinline__ float wave_max(float v) {
+  const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = fmaxf(__int_as_float((int)s32[0]), __int_as_float((int)s32[1]));
+  const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = fmaxf(__int_as_float((int)s16[0]), __int_as_float((int)s16[1]));
+  asm("s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\ts_nop 1" : "+v"(v));
   return v;
 }
-__device__ __forceinline__ float wave_sum(float v) {
-  return wave_reduce(v, [](float a, float b) { return a + b; });
-}
-__device__ __forceinline__ float wave_max(float v) {
-  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
-}
 
-// Value of lane (lane ^ STRIDE) without touching LDS memory: DPP quad permutes (1, 2), two
-// bank-masked DPP row shifts (4, 8), a ds_swizzle bit pattern (16), v_permlane32_swap (32).
+// Value of lane (lane ^ STRIDE) without touching LDS memory: DPP (1, 2, 8; 4 as 7 and 3), a ds_swizzle bit pattern (16), v_permlane32_swap (32).
 template <int STRIDE>
 __device__ __forceinline__ int xor_lane_i(int v, int lane) {
-  if constexpr (STRIDE == 1) return __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false);
-  else if constexpr (STRIDE == 2) return __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false);
-  else if constexpr (STRIDE == 4) {
-    const int t = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xf, 0x5, false);     // row_shl:4 into banks 0,2
-    return __builtin_amdgcn_update_dpp(t, v, 0x114, 0xf, 0xA, false);            // row_shr:4 into banks 1,3
-  } else if constexpr (STRIDE == 8) {
-    const int t = __builtin_amdgcn_update_dpp(v, v, 0x108, 0xf, 0x3, false);     // row_shl:8 into banks 0,1
-    return __builtin_amdgcn_update_dpp(t, v, 0x118, 0xf, 0xC, false);            // row_shr:8 into banks 2,3
-  } else if constexpr (STRIDE == 16) return __builtin_amdgcn_ds_swizzle(v, 0x401F);
+  if constexpr (STRIDE == 1) return dpp_i<kQuadXor1>(v);
+  else if constexpr (STRIDE == 2) return dpp_i<kQuadXor2>(v);
+  else if constexpr (STRIDE == 4) return dpp_i<kQuadXor3>(dpp_i<kRowXor7>(v));
+  else if constexpr (STRIDE == 8) return dpp_i<kRowXor8>(v);
+  else if constexpr (STRIDE == 16) return __builtin_amdgcn_ds_swizzle(v, 0x401F);
   else {
     const auto sw = __builtin_amdgcn_permlane32_swap(v, v, false, false);         // [lo,lo] and [hi,hi]
     return (lane & 32) ? (int)sw[0] : (int)sw[1];

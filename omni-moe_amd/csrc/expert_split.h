@@ -52,11 +52,11 @@ struct GroupValues {
   }
   template <int E>
   __device__ __forceinline__ int get() const {
-    if constexpr (LPR == 4) return __builtin_amdgcn_update_dpp(v[0], v[0], E * 0x55, 0xf, 0xf, false);                  // quad_perm
-    else if constexpr (LPR == 8) {                                                                                      // row_newbcast, for either half of a row
-      const int t = __builtin_amdgcn_update_dpp(v[0], v[0], 0x150 + E, 0xf, 0x3, false);
+    if constexpr (LPR == 4) return dpp_i<E * 0x55>(v[0]);                       // quad_perm
+    else if constexpr (LPR == 8) {                                                                            // row_newbcast, for either half of a row
+      const int t = dpp_i<0x150 + E>(v[0]);
       return __builtin_amdgcn_update_dpp(t, v[0], 0x158 + E, 0xf, 0xC, false);
-    } else if constexpr (LPR <= 32) return __builtin_amdgcn_update_dpp(v[E / 16], v[E / 16], 0x150 + E % 16, 0xf, 0xf, false);
+    } else if constexpr (LPR <= 32) return dpp_i<0x150 + E % 16>(v[E / 16]);
     else return __builtin_amdgcn_readlane(v[0], E);
   }
 };

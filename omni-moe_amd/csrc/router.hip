@@ -106,9 +106,9 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_chunked_ker
         ky[a] = ok ? make_key<DT>(vy, key) : 0u;
       }
       ktop64_2<RC>(kx, ky, lane);
-      uint32_t x[1] = {max(bx, (uint32_t)__shfl((int)kx[0], 63 - lane, kWave))};
-      uint32_t y[1] = {max(by, (uint32_t)__shfl((int)ky[0], 63 - lane, kWave))};
-      kstages_ct<1, kWave, kWave / 2>(x, y, lane, true);
+      uint32_t x[1] = {max(bx, mirrored<kWave>(kx[0], lane))};
+      uint32_t y[1] = {max(by, mirrored<kWave>(ky[0], lane))};
+      kdistances<1, kWave / 2>(x, y, lane, true);
       bx = c == 0 ? kx[0] : x[0];
       by = c == 0 ? ky[0] : y[0];
     }

@@ -72,6 +72,19 @@ def test_router_select_bit_exact(case, device):
     assert torch.equal(got_i.cpu(), want_i)
 
 
+# more candidates than lanes: whole sorts of 2, 4, 8 and 16 registers to a half, of up to 16 candidates to a lane
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("kind", ["randn", "ties"])
+@pytest.mark.parametrize("r,k", [(66, 66), (128, 100), (129, 128), (256, 66), (300, 128), (512, 80), (513, 128), (1024, 128)])
+def test_router_select_whole_sort_bit_exact(r, k, kind, dtype, device):
+    lx, ly = _router_inputs(37, r, dtype, kind, seed=r + k)
+    want_s, want_i = oracle.router_select(lx, ly, r, k)
+    got_s, got_i = _ops().hip_omni_router_func(lx.to(device), ly.to(device), r, k)
+    torch.cuda.synchronize()
+    assert torch.equal(got_s.cpu().float(), want_s.float())
+    assert torch.equal(got_i.cpu(), want_i)
+
+
 def test_router_select_contract(device):
     hip = _ops()
     lx = torch.zeros(4, 8, device=device)
