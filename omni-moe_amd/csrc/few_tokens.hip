@@ -182,11 +182,12 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel
   const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * Q * TM * 2048;
   if constexpr (kSelect) {
     if ((int)blockIdx.x < g.select_blocks) {
+      __shared__ PrunePool pool;
       const int first = (int)blockIdx.x * kFewWaves + wave, all = g.select_blocks * kFewWaves;
-      if (g.select_regs <= 1) select_packed<DT, 1, C>(g.select, first, all, g.select.stats);
-      else if (g.select_regs <= 2) select_packed<DT, 2, C>(g.select, first, all, g.select.stats);
-      else if (g.select_regs <= 4) select_packed<DT, 4, C>(g.select, first, all, g.select.stats);
-      else select_packed<DT, 8, C>(g.select, first, all, g.select.stats);
+      if (g.select_regs <= 1) select_packed<DT, 1, C>(g.select, first, all, g.select.stats, pool);
+      else if (g.select_regs <= 2) select_packed<DT, 2, C>(g.select, first, all, g.select.stats, pool);
+      else if (g.select_regs <= 4) select_packed<DT, 4, C>(g.select, first, all, g.select.stats, pool);
+      else select_packed<DT, 8, C>(g.select, first, all, g.select.stats, pool);
       return;
     }
   }

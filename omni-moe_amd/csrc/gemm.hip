@@ -1162,7 +1162,7 @@ namespace omni {
 size_t mlp_sums_bytes(int64_t T, int64_t H, int64_t I, int dtype) {
   if (dtype == OMNI_F32 || I % 8 || H % 8) return 0;
   const size_t few = few_tokens_covers(T, H, I, dtype) ? few_tokens_parts_bytes(T, H, I) : 0;
-  return std::max({few, tile_workspace_bytes(kTileSwiglu, T, I, H), tile_workspace_bytes(kTileResidual, T, H, I), tile_down_workspace_bytes(T, H, I)});
+  return std::max({few, tile_workspace_bytes(kNT, kTileSwiglu, T, I, H), tile_workspace_bytes(kNT, kTileResidual, T, H, I), tile_down_workspace_bytes(T, H, I)});
 }
 static size_t mlp_h_bytes(int64_t T, int64_t I, int dtype) { return ((size_t)T * (size_t)I * (dtype == OMNI_F32 ? 4 : 2) + 255) / 256 * 256; }
 

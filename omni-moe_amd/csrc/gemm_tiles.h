@@ -48,7 +48,7 @@ struct TileSingle {
 // hipErrorInvalidValue, and nothing launched, for operands beyond 2 GiB per tile column.
 hipError_t launch_tile_group(int dtype, int layout, int epilogue, TileGroup& g, void* ws, size_t ws_bytes, hipStream_t s, bool exclusive = true);
 // What launch_tile_group wants for one product; K: the sum of its segments, each rounded up to 64
-size_t tile_workspace_bytes(int epilogue, int64_t M, int64_t N, int64_t K);
+size_t tile_workspace_bytes(int layout, int epilogue, int64_t M, int64_t N, int64_t K);
 
 // The layer's joint launches.  The router's projection (kTileTwo) in front of the gate/up projection (kTileSwiglu; gate and up kept where c2 and c3 say so), both kNT
 // over the same K; false, and nothing launched, where its tiles would cost a round of their own or the operands are out of reach.

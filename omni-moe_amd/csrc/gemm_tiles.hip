@@ -4,7 +4,7 @@
 namespace omni {
 
 // (joint: those that share their launch with the layer's router)
-constexpr unsigned kAnyShape = (1u << kShapes) - 1, kJointShapes = 1u << 1 | 1u << 2 | 1u << 3 | 1u << 4 | 1u << 7 | 1u << 8;
+constexpr unsigned kForwardShapes = shapes_of(kNT), kJointShapes = 1u << 1 | 1u << 2 | 1u << 3 | 1u << 4 | 1u << 7 | 1u << 8;
 
 // Microseconds that a launch of n blocks of one shape takes for 64 of K.  Where two blocks share a CU, the CUs with two set the time however few they are
 // (gate/up of 613 x 1024 x 4096 on 128 x 128 tiles, 320 blocks: 19.7 us; 450 rows, 256 blocks: 16.4; 1000 rows, 512 blocks: 21.4).
@@ -37,7 +37,7 @@ static TileChoice choose_of(int epilogue, const TileSize* sizes, int count, int6
 }
 // A call asks for its workspace and then for its launches, a program for the same sizes over and over, and a choice takes 0.6 us: a layer of one token,
 // bound by the host, asked eight times.  Each thread keeps the last few products' choices, which nothing but the sizes goes into.
-static TileChoice choose_tiles(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes = kAnyShape) {
+static TileChoice choose_tiles(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes = kForwardShapes) {
   if (count != 1) return choose_of(epilogue, sizes, count, K, may_split, shapes);
   struct Kept { int64_t M, N, K; uint64_t how; TileChoice choice; };
   constexpr int kKept = 16;
@@ -76,10 +76,10 @@ static int choose_pair(const TileSize& router, const TileSize& mlp, int64_t K) {
 }
 static size_t parts_bytes(const TileChoice& c, int64_t M, int64_t columns) { return c.splits > 1 ? (size_t)c.splits * (size_t)M * (size_t)columns * 4 : 0; }
 
-size_t tile_workspace_bytes(int epilogue, int64_t M, int64_t N, int64_t K) {
+size_t tile_workspace_bytes(int layout, int epilogue, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const TileSize size{M, N};
-  const TileChoice c = choose_tiles(epilogue, &size, 1, K, true);
+  const TileChoice c = choose_tiles(epilogue, &size, 1, K, true, shapes_of(layout));
   return parts_bytes(c, M, epilogue == kTileSwiglu ? 2 * N : N);
 }
 size_t tile_down_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -103,9 +103,9 @@ hipError_t launch_tile_group(int dtype, int layout, int epilogue, TileGroup& g, 
     }
     K = k > K ? k : K;
   }
-  TileChoice c = choose_tiles(epilogue, sizes, g.count, K, ws != nullptr);
+  TileChoice c = choose_tiles(epilogue, sizes, g.count, K, ws != nullptr, shapes_of(layout));
   if (parts_bytes(c, g.p[0].M, epilogue == kTileSwiglu ? 2 * (int64_t)g.p[0].N : g.p[0].N) > ws_bytes)
-    c = choose_tiles(epilogue, sizes, g.count, K, false);
+    c = choose_tiles(epilogue, sizes, g.count, K, false, shapes_of(layout));
   if (dtype == kBF16) return tile_group_of<kBF16>(layout, epilogue, g, c, (float*)ws, exclusive, s);
   if (dtype == kF16) return tile_group_of<kF16>(layout, epilogue, g, c, (float*)ws, exclusive, s);
   return hipErrorInvalidValue;
@@ -144,7 +144,7 @@ extern "C" OMNI_API int32_t omni_probe_joint_tiles(int64_t num_tokens, int32_t h
   select.r = num_expert_sqrt; select.k = num_experts_per_token;
   const int cells = prepare_select(select), regs = (num_expert_sqrt + kWave - 1) / kWave, splits = c.splits < kMostDownParts ? c.splits : kMostDownParts;
   auto plan = [&](auto id) { return plan_down<decltype(id)::value>(num_tokens, hidden_size, intermediate_size, splits, (int)num_tokens, regs, cells); };
-  DownPlan p{0, splits, 0, 0, false};                          // (tiles of 256 columns: nothing beside them)
+  DownPlan p{0, splits, 0, 0, false};                          // (the other shapes: nothing beside them)
   if (c.shape == 1) p = plan(std::integral_constant<int, 1>{});
   else if (c.shape == 2) p = plan(std::integral_constant<int, 2>{});
   else if (c.shape == 3) p = plan(std::integral_constant<int, 3>{});

@@ -55,6 +55,7 @@ template <int DT> __device__ __forceinline__ uint32_t pack16x2(float lo, float h
 template <int TM, int TN, int RA, int RB, int NL, bool kSync>
 struct StepPlan {
   static constexpr int kSlots = TM * TN, kStart = kSync ? TN - 1 : 0, kOps = TM * RA + TN * RB + NL;
+  static constexpr int kSpan = kSync ? (kSlots - kStart + 1) / 2 : kSlots;         // those behind the barrier are waited for soonest: they come in its first half
   static constexpr int kCap = (TM * RA + TN * RB + kSlots - kStart - 1) / (kSlots - kStart), kMost = kCap + 2 * RA + NL;
   int op[kSlots][kMost] = {};
   constexpr StepPlan() {
@@ -69,7 +70,7 @@ struct StepPlan {
         else if (nb < TN * RB) op[s][u++] = 65 + nb++;
         else break;
       }
-      while (nl < NL * (s + 1 - kStart) / (kSlots - kStart)) op[s][u++] = 129 + nl++;
+      while (nl < NL && nl < NL * (s + 1 - kStart) / kSpan) op[s][u++] = 129 + nl++;
     }
   }
   constexpr bool complete() const {
@@ -127,22 +128,36 @@ constexpr int staged_rows(int rows, int waves) {
   return up;
 }
 
-// A block is KG groups of WM x WN waves; a wave owns TM x TN matrix tiles of 16 x 16.  The ring advances 64 * KG of K a step through NS stages;
+// Stages of the two operands in LDS: NS, and one more for the left operand, or for the right one where the left one's does not fit.  The one with a stage
+// more is requested in step 0 of a K tile, half a tile before the barrier that frees the other's: requests are spread over the whole tile, and of two stages the
+// second one's loads have between a half and a whole tile to arrive.  Two stages against two and three, kernels alone: down of 32768 x 2048 x 8192 827 -> 793 us,
+// the three weight gradients of 4096 x 1024 x 4096 95.6 -> 93.2 on 256 rows and 102 -> 94.8 on 224, the SwiGLU backward 58.7 -> 57.3.
+constexpr int kCuLds = 160 * 1024;
+template <int LM, int BN, int KG, int NS>
+struct TileRing {
+  static constexpr bool kLeadA = KG * 128 * (LM * (NS + 1) + BN * NS) <= kCuLds;
+  static constexpr int kAStages = NS + (kLeadA ? 1 : 0), kBStages = NS + (kLeadA ? 0 : 1);
+  static constexpr int kAStage = KG * LM * 128, kBStage = KG * BN * 128, kBFirst = kAStages * kAStage, kBytes = kBFirst + kBStages * kBStage;
+  static_assert(kBytes <= kCuLds, "a block's ring fits its CU");
+};
+
+// A block is KG groups of WM x WN waves; a wave owns TM x TN matrix tiles of 16 x 16.  The ring advances 64 * KG of K a step through NS stages (TileRing);
 // group g multiplies the g-th 64 of each.  kTail: some segment's K is not a multiple of the ring step, and an operand's rows run along K.
 //
 // kStream (one product, one segment, unsplit): the grid may be smaller than the number of output tiles; a block walks its share, and the ring
 // steps of consecutive output tiles form ONE stream through the stages: the next tile's first loads fly while the current one finishes, so
-// only a block's first tile waits for memory before its first matrix instruction.  All of a ring step's loads are then requested in step 1:
-// the epilogue's stores are younger than every load of the next tile's first two ring steps and may stay in flight past its first
-// wait (memory instructions are counted in issue order).
+// only a block's first tile waits for memory before its first matrix instruction.  The epilogue's stores are younger than every load of the next tile's first
+// two ring steps and may stay in flight past its first wait (memory instructions are counted in issue order).
 // (block, blocks): the place in the launch, or in its own part of one that it shares
 template <int DT, int LAY, int WM, int WN, int KG, int TM, int TN, int NS, int EPI, bool kTail, bool kStream, class Group>
 __device__ __forceinline__ void tiles_block(const Group& g, const int block, const int blocks) {
   constexpr bool AC = LAY == kTN, BC = LAY != kNT;             // the operand's K index is its row
   constexpr int NW = WM * WN * KG, BM = WM * TM * 16, BN = WN * TN * 16, BNO = EPI == kTileSwiglu ? BN / 2 : BN;
   constexpr int LM = staged_rows<LAY>(BM, NW);                 // A's rows in a stage, those behind the tile's unread
-  constexpr int kABytes = LM * 128, kSub = (LM + BN) * 128, kStage = KG * kSub;
+  constexpr int kABytes = LM * 128, kBBytes = BN * 128;        // of a group's 64 of K
+  using Ring = TileRing<LM, BN, KG, NS>;
   constexpr int PA = LM / 8 / NW, PB = BN / 8 / NW, LPT = KG * (PA + PB);     // 1 KiB load instructions per wave and ring step
+  constexpr int kLead = KG * (Ring::kLeadA ? PA : PB);         // ... those of the operand with a stage more
   static_assert(LM % (8 * NW) == 0 && BN % (8 * NW) == 0, "the waves share the loads evenly");
   static_assert(TN % (EPI == kTileSwiglu ? 4 : 2) == 0 && TM % KG == 0, "the epilogue takes column tiles in pairs");
   constexpr int RA = AC ? 2 : 1, RB = BC ? 2 : 1;              // LDS reads per fragment
@@ -190,8 +205,9 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
   // their matrices behind them (nothing, once every ring step has been requested: the loads then fetch nothing, which is cheaper than
   // a branch around each -- a scalar branch among the matrix instructions costs a lone wave as much as one of them).
   uint64_t f_a = 0, f_b = 0;
-  int f_aleft = 0, f_bleft = 0, f_astep = 0, f_bstep = 0, f_amore = 0, f_bmore = 0;      // ..more: from one load of a step to the wave's next
-  int f_seg = -1, f_left = 0;                                  // K values of the segment from the cursor on
+  int f_aleft = 0, f_bleft = 0, f_astep = 0, f_bstep = 0, f_amore = 0, f_bmore = 0;      // ..step: for 64 of K; ..more: from one load of a step to the wave's next
+  int f_seg = -1, f_left = 0;                                  // K values of the segment from the cursor on, when its run of steps began
+  int f_run = 0, f_until = 0;                                  // ring steps of that run, and what is left of it: the cursor only moves on by f_astep and f_bstep
   int f_half = 0;                                              // kTileTwo: rows of the fetched tile, counted from the wave's first, that are the first matrix's
   constexpr uint32_t kOutside = 0x80000000u;
   auto scalar = [](int v) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(v); };
@@ -199,6 +215,12 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
     // (readfirstlane returns a signed value)
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32));
     return (uint64_t)lo | ((uint64_t)hi << 32);
+  };
+  int f_steps = 0;                                             // ring steps of the fetched tile, when the run began; none: everything has been requested
+  // up to the end of the segment or the tile, or to a step of less than 64 * KG
+  auto begin_run = [&]() __attribute__((always_inline)) {
+    const int n = min(f_steps, (f_left + 64 * KG - 1) / (64 * KG));
+    f_run = f_until = scalar(kTail && n > 1 && n * 64 * KG > f_left ? n - 1 : n);
   };
   // rows along K: chunks past the segment's K read as zero (the other operands end with their matrix)
   auto mask_tail = [&]() __attribute__((always_inline)) {
@@ -251,6 +273,7 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
 #pragma unroll
     for (int s = 0; s < kOff; ++s) { a_off[s] = a0; b_off[s] = b0; }
     mask_tail();
+    begin_run();
   };
   int tiles = p.steps;                                         // ring steps of one output tile in this block
   {
@@ -264,85 +287,85 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
     }
     tiles = scalar(min(tiles, total - split * p.steps));
     f_seg = scalar(f_seg);
+    f_steps = tiles;
     enter_segment(skip);
   }
-  int f_steps = tiles;                                         // ring steps of the fetched tile from the cursor on; none: everything has been requested
   const uint32_t lds_base = (uint32_t)(uintptr_t)(LdsPtr)lds;
   const uint32_t lds_wave = lds_base + (uint32_t)wave * 1024;
-  int f_stage = 0;                                             // the cursor's stage
+  uint32_t f_ato = lds_wave, f_bto = lds_wave + Ring::kBFirst; // the cursor's stages
   // from B's address to the other matrix's: the up weights, or (Two) the upper half of the columns' as if its rows followed on the first's
   uint64_t to_second = 0;
   if constexpr (EPI == kTileSwiglu) to_second = scalar64((uint64_t)p.b_up - (uint64_t)p.seg[0].b);
   if constexpr (EPI == kTileTwo) to_second = scalar64((uint64_t)p.b_up - (uint64_t)p.seg[0].b - (uint64_t)(N / 2) * (uint64_t)p.seg[0].ldb);
-  // the cursor's ring step as its loads take it (through readfirstlane once more: the compiler does not always see that
-  // they are the same in every lane)
-  uint64_t c_a = 0, c_b = 0;
-  int c_aleft = 0, c_bleft = 0;
-  uint32_t c_to = 0;
-  auto settle = [&]() __attribute__((always_inline)) {
-    c_a = scalar64(f_a);
-    c_b = scalar64(f_b);
-    c_aleft = scalar(max(f_aleft, 0));
-    c_bleft = scalar(max(f_bleft, 0));
-    c_to = (uint32_t)scalar((int)(lds_wave + (uint32_t)f_stage));
+  // load q of an operand's part of the cursor's ring step
+  auto issue_a = [&](auto q_tag) __attribute__((always_inline)) {
+    constexpr int q = decltype(q_tag)::value, s = q / PA, o = q % PA;
+    load_to_lds<s * kABytes + o * NW * 1024>(f_a, f_aleft, f_ato, a_off[s % kOff], s * f_astep + o * f_amore);
   };
-  // load q of it
-  auto issue_one = [&](auto q_tag) __attribute__((always_inline)) {
-    constexpr int q = decltype(q_tag)::value, s = q / (PA + PB), o = q % (PA + PB);
-    if constexpr (o < PA) {
-      load_to_lds<s * kSub + o * NW * 1024>(c_a, c_aleft, c_to, a_off[s % kOff], s * f_astep + o * f_amore);
-    } else {
-      uint64_t base = c_b;
-      constexpr int b = o - PA, row = b * NW * 8, nth = EPI == kTileSwiglu ? row / (TN * 16) : b;
-      if constexpr (EPI == kTileSwiglu) base += ((row + wave * 8) / (TN * 8)) & 1 ? to_second : 0;
-      if constexpr (EPI == kTileTwo) base += row >= f_half ? to_second : 0;     // (the eight rows of a load are of one matrix)
-      load_to_lds<s * kSub + kABytes + b * NW * 1024>(base, c_bleft, c_to, b_off[s % kOff], s * f_bstep + nth * f_bmore);
-    }
+  auto issue_b = [&](auto q_tag) __attribute__((always_inline)) {
+    constexpr int q = decltype(q_tag)::value, s = q / PB, b = q % PB, row = b * NW * 8, nth = EPI == kTileSwiglu ? row / (TN * 16) : b;
+    uint64_t base = f_b;
+    if constexpr (EPI == kTileSwiglu) base += ((row + wave * 8) / (TN * 8)) & 1 ? to_second : 0;
+    if constexpr (EPI == kTileTwo) base += row >= f_half ? to_second : 0;     // (the eight rows of a load are of one matrix)
+    load_to_lds<s * kBBytes + b * NW * 1024>(base, f_bleft, f_bto, b_off[s % kOff], s * f_bstep + nth * f_bmore);
   };
-  auto advance = [&]() __attribute__((always_inline)) {
-    f_stage = f_stage == (NS - 1) * kStage ? 0 : f_stage + kStage;
-    f_left -= 64 * KG;
-    --f_steps;
+  auto issue_lead = [&](auto q_tag) __attribute__((always_inline)) { if constexpr (Ring::kLeadA) issue_a(q_tag); else issue_b(q_tag); };
+  auto issue_other = [&](auto q_tag) __attribute__((always_inline)) { if constexpr (Ring::kLeadA) issue_b(q_tag); else issue_a(q_tag); };
+  // to the next ring step of a run
+  auto move_a = [&]() __attribute__((always_inline)) {
+    f_a += KG * (uint32_t)f_astep;
+    f_aleft -= KG * f_astep;
+    f_ato = f_ato == lds_wave + (Ring::kAStages - 1) * Ring::kAStage ? lds_wave : f_ato + Ring::kAStage;
+  };
+  auto move_b = [&]() __attribute__((always_inline)) {
+    f_b += KG * (uint32_t)f_bstep;
+    f_bleft -= KG * f_bstep;
+    f_bto = f_bto == lds_wave + Ring::kBFirst + (Ring::kBStages - 1) * Ring::kBStage ? lds_wave + Ring::kBFirst : f_bto + Ring::kBStage;
+  };
+  auto move_lead = [&]() __attribute__((always_inline)) { if constexpr (Ring::kLeadA) move_a(); else move_b(); };
+  auto move_other = [&]() __attribute__((always_inline)) { if constexpr (Ring::kLeadA) move_b(); else move_a(); };
+  // where a run has ended
+  auto next_run = [&]() __attribute__((always_inline)) {
+    f_left -= 64 * KG * f_run;
+    f_steps -= f_run;
     if (f_steps > 0) {
       if (f_left <= 0) {
         f_seg = scalar(f_seg + 1);
         enter_segment(0);
       } else {
-        f_a += KG * (uint32_t)f_astep; f_aleft -= KG * f_astep;
-        f_b += KG * (uint32_t)f_bstep; f_bleft -= KG * f_bstep;
         mask_tail();
+        begin_run();
       }
     } else if (kStream && f_tile + blocks < all) {
       f_tile = scalar(f_tile + blocks);
       f_steps = tiles;
       coords(f_tile, fm0, fn0);
       enter_segment(0);
-    } else {
-      f_aleft = f_bleft = 0;
+    } else {                                                   // everything has been requested
+      f_aleft = f_bleft = f_astep = f_bstep = 0;
+      f_until = INT32_MAX;
     }
-    settle();
   };
-  settle();
 
   // ---- fragment reads.  Lane (r16 = lane % 16, g4 = lane / 16) takes the K values 32 ks + 8 g4 .. + 7 of row r16 of a 16-row tile.
   const int r16 = lane & 15, g4 = lane >> 4;
   constexpr int kRowA = AC ? LM * 2 : 128, kRowB = BC ? BN * 2 : 128;
   uint32_t a_addr[AC ? TM : 2], b_addr[BC ? TN : 2];
   const uint32_t tr_row = (uint32_t)(8 * g4 + (r16 >> 2)), tr_in = (uint32_t)(r16 & 3) * 8;       // (piece_of() of the row is the same in every K step and part)
-  const uint32_t my_base = lds_base + (uint32_t)kg * kSub;
+  const uint32_t my_a = lds_base + (uint32_t)(kg * kABytes), my_b = lds_base + (uint32_t)(Ring::kBFirst + kg * kBBytes);
   if constexpr (AC) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) a_addr[i] = my_base + tr_row * kRowA + (uint32_t)((wm * TM + i) ^ piece_of((int)tr_row, LM)) * 32 + tr_in;
+    for (int i = 0; i < TM; ++i) a_addr[i] = my_a + tr_row * kRowA + (uint32_t)((wm * TM + i) ^ piece_of((int)tr_row, LM)) * 32 + tr_in;
   } else {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) a_addr[ks] = my_base + (uint32_t)(wm * TM * 16 + r16) * 128 + (uint32_t)((4 * ks + g4) ^ (r16 >> 1)) * 16;
+    for (int ks = 0; ks < 2; ++ks) a_addr[ks] = my_a + (uint32_t)(wm * TM * 16 + r16) * 128 + (uint32_t)((4 * ks + g4) ^ (r16 >> 1)) * 16;
   }
   if constexpr (BC) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) b_addr[j] = my_base + kABytes + tr_row * kRowB + (uint32_t)((wn * TN + j) ^ piece_of((int)tr_row, BN)) * 32 + tr_in;
+    for (int j = 0; j < TN; ++j) b_addr[j] = my_b + tr_row * kRowB + (uint32_t)((wn * TN + j) ^ piece_of((int)tr_row, BN)) * 32 + tr_in;
   } else {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) b_addr[ks] = my_base + kABytes + (uint32_t)(wn * TN * 16 + r16) * 128 + (uint32_t)((4 * ks + g4) ^ (r16 >> 1)) * 16;
+    for (int ks = 0; ks < 2; ++ks) b_addr[ks] = my_b + (uint32_t)(wn * TN * 16 + r16) * 128 + (uint32_t)((4 * ks + g4) ^ (r16 >> 1)) * 16;
   }
   using Frag = const __attribute__((address_space(3))) u32x4_t*;
   u32x4_t af[TM], bf[2][TN];
@@ -374,34 +397,30 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
 #pragma unroll
       for (int q = 0; q < 4; ++q) acc[i][j][q] = 0.f;
 
-  // ---- K loop.  Step 0 of a K tile reads the fragments of its step 1; then, after the first matrix row of step 1, every wave waits for
-  // its own reads and loads and meets the block: the stage is free, the next one is there; step 1 reads the next stage's first
-  // fragments and requests the first half of the ring step NS ahead (or all of it), the following step 0 its other half.  Behind the last ring step
-  // the reads fetch what nobody uses.
-  // With two stages every load of a ring step goes into step 1: the next wait is for them, and one requested at the end of step 0 would be waited for from
-  // its first cycle on (half of them in step 0: gate/up of 4096 x 4096 x 1024 beside another stream 63.9 -> 60.8 us, keeping gate and up 73.1 -> 68.5, its three
-  // weight gradients on 256 rows 104.6 -> 94.3 and on 224 105.2 -> 99.8, the SwiGLU backward 60.9 -> 59.0).
-  constexpr int kLoads1 = NS == 2 ? LPT : LPT / 2;             // loads in step 1; the rest in the following step 0
-  static_assert(!kStream || kLoads1 == LPT, "a stream's loads are older than the epilogue's stores");
-  using Plan0 = StepPlan<TM, TN, RA, RB, LPT - kLoads1, false>;
-  using Plan1 = StepPlan<TM, TN, RA, RB, kLoads1, true>;
+  // ---- K loop.  Step 0 of a K tile reads the fragments of its step 1 and requests one operand of the ring step NS ahead; then, after the first matrix row of
+  // step 1, every wave waits for its own reads and loads and meets the block: the stage is free, the next one is there; step 1 reads the next stage's first
+  // fragments and requests the other operand.  Behind the last ring step the reads fetch what nobody uses.
+  // The cursor moves between matrix instructions, and where a run of its steps ends, between two K tiles, a branch out of the loop sees to what comes next.
+  using Plan0 = StepPlan<TM, TN, RA, RB, kLead, false>;
+  using Plan1 = StepPlan<TM, TN, RA, RB, LPT - kLead, true>;
   static_assert(Plan0{}.complete() && Plan1{}.complete(), "a step's memory instructions do not fit");
-  auto load_step = [&](auto... q) __attribute__((always_inline)) { (issue_one(q), ...); };
-  auto load_all = [&](auto seq) __attribute__((always_inline)) { with_sequence(load_step, seq); };
+  auto load_lead = [&](auto... q) __attribute__((always_inline)) { (issue_lead(q), ...); };
+  auto load_other = [&](auto... q) __attribute__((always_inline)) { (issue_other(q), ...); };
 #pragma unroll
-  for (int t = 0; t < NS - 1; ++t) {
-    load_all(std::make_integer_sequence<int, LPT>{});
-    advance();
+  for (int t = 0; t < NS; ++t) {
+    with_sequence(load_lead, std::make_integer_sequence<int, kLead>{});
+    with_sequence(load_other, std::make_integer_sequence<int, LPT - kLead>{});
+    move_lead();
+    move_other();
+    if (--f_until == 0) next_run();
   }
-  load_all(std::make_integer_sequence<int, kLoads1>{});         // (the first step 0 requests the others)
-  if constexpr (kStream) advance();
-  vmcnt<(NS - 2) * LPT + kLoads1>();
+  vmcnt<(NS - 1) * LPT>();
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int n = 0; n < TM * RA; ++n) read_a(0, n);
 #pragma unroll
   for (int n = 0; n < TN * RB; ++n) read_b(0, n);
-  int stage = 0;                                               // the one being multiplied
+  int a_stage = 0, b_stage = 0;                                // those being multiplied
   constexpr int kEpiStores = TM * (EPI == kTileSwiglu ? TN / 4 : TN / 2);     // store instructions of a wave's epilogue
   int young = 0;                                               // that many are younger than the loads that the next wait is for
   auto slot0 = [&](auto s_tag) __attribute__((always_inline)) {
@@ -410,7 +429,7 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
     __builtin_amdgcn_sched_barrier(0);
     each_op<Plan0, s>([&](auto op_tag) __attribute__((always_inline)) {
       constexpr int op = decltype(op_tag)::value;
-      if constexpr (op >= 129) issue_one(std::integral_constant<int, kLoads1 + op - 129>{});
+      if constexpr (op >= 129) issue_lead(std::integral_constant<int, op - 129>{});
       else if constexpr (op >= 65) read_b(1, op - 65);
       else if constexpr (op >= 1) read_a(1, op - 1);
     });
@@ -422,17 +441,20 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (s == TN - 1) {
       lds_reads_done();
-      if (kStream && young) vmcnt<(NS - 2) * LPT + kEpiStores>();
-      else vmcnt<(NS - 2) * LPT>();
+      constexpr int kYounger = (NS - 2) * LPT + kLead;
+      if (kStream && young) vmcnt<kYounger + kEpiStores>();
+      else vmcnt<kYounger>();
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
     }
     each_op<Plan1, s>([&](auto op_tag) __attribute__((always_inline)) {
       constexpr int op = decltype(op_tag)::value;
-      if constexpr (op >= 129) issue_one(std::integral_constant<int, op - 129>{});
+      if constexpr (op >= 129) issue_other(std::integral_constant<int, op - 129>{});
       else if constexpr (op >= 65) read_b(0, op - 65);
       else if constexpr (op >= 1) read_a(0, op - 1);
     });
+    if constexpr (s == (TN - 1 + TM * TN - 1) / 2) move_lead();
+    if constexpr (s == TM * TN - 1) move_other();
     __builtin_amdgcn_sched_barrier(0);
   };
   auto all0 = [&](auto... s) __attribute__((always_inline)) { (slot0(s), ...); };
@@ -441,18 +463,25 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
   for (int tile = block - p.first; tile < all; tile += blocks) {
   int m0, n0;
   coords(tile, m0, n0);
+  for (int left = tiles; left > 0;) {
+    const int run = min(left, f_until);
 #pragma clang loop unroll(disable)
-  for (int kt = 0; kt < tiles; ++kt) {
-    with_sequence(all0, std::make_integer_sequence<int, TM * TN>{});
-    stage = stage + 1 == NS ? 0 : stage + 1;
-    const uint32_t move = stage == 0 ? (uint32_t)(-(NS - 1) * kStage) : (uint32_t)kStage;
+    for (int i = run; i > 0; --i) {
+      with_sequence(all0, std::make_integer_sequence<int, TM * TN>{});
+      a_stage = a_stage + 1 == Ring::kAStages ? 0 : a_stage + 1;
+      b_stage = b_stage + 1 == Ring::kBStages ? 0 : b_stage + 1;
+      const uint32_t a_move = a_stage == 0 ? (uint32_t)(-(Ring::kAStages - 1) * Ring::kAStage) : (uint32_t)Ring::kAStage;
+      const uint32_t b_move = b_stage == 0 ? (uint32_t)(-(Ring::kBStages - 1) * Ring::kBStage) : (uint32_t)Ring::kBStage;
 #pragma unroll
-    for (int i = 0; i < (AC ? TM : 2); ++i) a_addr[i] += move;
+      for (int i = 0; i < (AC ? TM : 2); ++i) a_addr[i] += a_move;
 #pragma unroll
-    for (int j = 0; j < (BC ? TN : 2); ++j) b_addr[j] += move;
-    if constexpr (!kStream) advance();
-    with_sequence(all1, std::make_integer_sequence<int, TM * TN>{});
-    if constexpr (kStream) { advance(); young = 0; }
+      for (int j = 0; j < (BC ? TN : 2); ++j) b_addr[j] += b_move;
+      with_sequence(all1, std::make_integer_sequence<int, TM * TN>{});
+      if constexpr (kStream) young = 0;
+    }
+    left -= run;
+    f_until -= run;
+    if (f_until == 0) next_run();
   }
   if constexpr (!kStream) vmcnt<0>();                          // no load may arrive in LDS that the block has given back
 
@@ -687,17 +716,25 @@ template <bool kSwiglu> struct Shape<5, kSwiglu> { enum { WM = 2, WN = 4, KG = 1
 template <bool kSwiglu> struct Shape<6, kSwiglu> { enum { WM = 2, WN = 4, KG = 1, TM = 6, TN = 4, NS = 2 }; };      // 192 x 256, one block to a CU
 template <bool kSwiglu> struct Shape<7, kSwiglu> { enum { WM = 4, WN = 2, KG = 1, TM = 3, TN = 4, NS = 3 }; };      // 192 x 128, one block to a CU
 template <bool kSwiglu> struct Shape<8, kSwiglu> { enum { WM = 2, WN = 2, KG = 1, TM = 3, TN = 4, NS = 4 }; };      // 96 x 128, one block to a CU
-constexpr int kShapes = 9;
+// For long sums of the gradients: a second wave to a SIMD multiplies while the first one's loads are issued, for an exchange of sums at the end.  dy W on 256 tiles,
+// K = 8192: 66.2 us against 71.8; 4096: 33.6 against 32.5.  (Not for x W^T: beside the down projection's eight waves the experts' passes find no room, layer of
+// 4096 tokens on two streams 119.1 -> 121.7 us, and one stream adds up in the order of two.)
+template <bool kSwiglu> struct Shape<9, kSwiglu> { enum { WM = 2, WN = 2, KG = 2, TM = 4, TN = 4, NS = 2 }; };      // 128 x 128, two K groups, one block to a CU
+constexpr int kShapes = 10;
+constexpr unsigned shapes_of(int layout) { return layout == kNN ? (1u << kShapes) - 1 : (1u << 9) - 1; }
 // ... and what a launch of n blocks takes, in microseconds per 64 of K and round of `at_once` blocks: idle + (full - idle) times the share of
 // the chip in use.  Measured on 256 x 256 x 4096 (few blocks) and 4096 x 4096 x 4096 (all CUs busy), the lower tiles and the 64 x 64 one over 57 products of
-// 300 to 12000 rows, bf16, where the rule's choice takes 0.4 % more than the best shape on average and 9 % at most; about 4 us more for a launch.
-// The lower tiles took, the best of the others / now: gate/up of 3000 x 1024 x 4096 (256 tiles of 256 columns a round) 49.5 / 45.4 us, 613 x 1024 x 4096
+// 300 to 12000 rows, bf16, with one ring stage less than now; about 4 us more for a launch.  The times are lower now (tiles of 256 columns by 11 % at the median,
+// two 128 x 128 tiles to a CU 14 %, the others up to 4 %), their order is not: over 174 products (x W^T, dy W, gate/up with SwiGLU; 64 to 12000 rows, 128 to 8192
+// columns, K 256 to 8192) the rule's choice takes 0.24 % more than the best shape on average and 9 % at most, and with figures fitted to those 0.19 and 9.
+// The lower tiles took, the best of the others / theirs: gate/up of 3000 x 1024 x 4096 (256 tiles of 256 columns a round) 49.5 / 45.4 us, 613 x 1024 x 4096
 // 17.4 / 15.2; down of 3000 x 4096 x 1024 31.9 / 29.4, 12000 x 1536 x 512 23.7 / 19.6; five weight gradients of 4096 tokens x 1024 x 4096 (200 tiles of
 // 256 rows, 236 of 224), in a trace of whole steps, 106 / 101.
 struct ShapeCost { int bm, bn, kg, at_once; float idle, full, fixed; };
 constexpr ShapeCost kCost[kShapes] = {{256, 256, 1, 256, 1.10f, 1.55f, 5.f}, {256, 128, 1, 256, 0.66f, 0.92f, 4.5f}, {128, 128, 1, 512, 0.50f, 1.00f, 4.f},
                                       {128, 128, 1, 256, 0.44f, 0.57f, 4.f}, {64, 64, 2, 256, 0.16f, 0.235f, 4.f}, {224, 256, 1, 256, 1.04f, 1.44f, 5.f},
-                                      {192, 256, 1, 256, 0.92f, 1.26f, 5.f}, {192, 128, 1, 256, 0.52f, 0.70f, 4.5f}, {96, 128, 1, 256, 0.36f, 0.47f, 4.f}};
+                                      {192, 256, 1, 256, 0.92f, 1.26f, 5.f}, {192, 128, 1, 256, 0.52f, 0.70f, 4.5f}, {96, 128, 1, 256, 0.36f, 0.47f, 4.f},
+                                      {128, 128, 2, 256, 0.41f, 0.535f, 6.5f}};
 constexpr ShapeCost kSwigluCost = {64, 128, 2, 256, 0.26f, 0.37f, 4.f};
 // A split writes its fp32 sums and a second kernel adds them: its launch, and the two trips
 constexpr float kReduceUs = 3.3f, kPartsOut = 8e6f, kPartsIn = 5e6f;      // us, bytes per us
@@ -708,7 +745,7 @@ struct TileSize { int64_t M, N; };
 template <int DT, int LAY, int kId, int EPI, bool kTail, bool kStream, class Group>
 struct TilesLds {
   using S = Shape<kId, EPI == kTileSwiglu>;
-  static constexpr int kBytes = S::NS * S::KG * (staged_rows<LAY>(S::WM * S::TM * 16, S::WM * S::WN * S::KG) + S::WN * S::TN * 16) * 128;
+  static constexpr int kBytes = TileRing<staged_rows<LAY>(S::WM * S::TM * 16, S::WM * S::WN * S::KG), S::WN * S::TN * 16, S::KG, S::NS>::kBytes;
   static inline LdsKernel entry{(const void*)gemm_tiles_kernel<DT, LAY, S::WM, S::WN, S::KG, S::TM, S::TN, S::NS, EPI, kTail, kStream, Group>, kBytes};
 };
 template <int DT, int LAY, int kId, int EPI, bool kTail, bool kStream, class Group>
@@ -746,18 +783,19 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
     constexpr int kWaves = S::WM * S::WN * S::KG;
     const int first = (int)blockIdx.x * kWaves + (int)(threadIdx.x >> 6), all = select_blocks * kWaves;
     const float* stats = g.select.stats;
+    extern __shared__ __align__(16) uint8_t lds[];             // (the ring of the blocks that multiply takes all of it)
+    PrunePool& pool = *(PrunePool*)(lds + 4 * merge_lds_floats(kMergeKeys, kWaves * kWave));
     if (g.select.part_mean) {                                  // batch statistics: the block merges them first
-      extern __shared__ __align__(16) uint8_t lds[];
       merge_statistics(g.select, (float*)lds, kWaves * kWave);
       stats = (const float*)lds;
     }
     count_batch(g.select);
     auto select = [&](auto cells) {
       constexpr int C = decltype(cells)::value;
-      if (g.regs <= 1) select_packed<DT, 1, C>(g.select, first, all, stats);
-      else if (g.regs <= 2) select_packed<DT, 2, C>(g.select, first, all, stats);
-      else if (g.regs <= 4) select_packed<DT, 4, C>(g.select, first, all, stats);
-      else select_packed<DT, 8, C>(g.select, first, all, stats);
+      if (g.regs <= 1) select_packed<DT, 1, C>(g.select, first, all, stats, pool);
+      else if (g.regs <= 2) select_packed<DT, 2, C>(g.select, first, all, stats, pool);
+      else if (g.regs <= 4) select_packed<DT, 4, C>(g.select, first, all, stats, pool);
+      else select_packed<DT, 8, C>(g.select, first, all, stats, pool);
     };
     if (g.cells <= 1) select(std::integral_constant<int, 1>{});
     else select(std::integral_constant<int, 2>{});
@@ -768,8 +806,8 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
 template <int kId, bool kSwiglu>
 constexpr int tile_lds() {
   using S = Shape<kId, kSwiglu>;
-  constexpr int kBytes = S::NS * S::KG * (staged_rows<kNT>(S::WM * S::TM * 16, S::WM * S::WN * S::KG) + S::WN * S::TN * 16) * 128;
-  static_assert(kBytes >= 4 * merge_lds_floats(kMergeKeys, S::WM * S::WN * S::KG * 64), "a block that selects merges statistics there");
+  constexpr int kBytes = TileRing<staged_rows<kNT>(S::WM * S::TM * 16, S::WM * S::WN * S::KG), S::WN * S::TN * 16, S::KG, S::NS>::kBytes;
+  static_assert(kBytes >= 4 * merge_lds_floats(kMergeKeys, S::WM * S::WN * S::KG * 64) + (int)sizeof(PrunePool), "a block that selects merges statistics and prunes there");
   return kBytes;
 }
 template <auto kKernel, int kBytes>
@@ -858,6 +896,9 @@ static hipError_t launch_choice(TileGroup& g, const TileChoice& c, float* ws, bo
     case 5: return launch_tiles<DT, LAY, 5, EPI>(g, ws, c.splits, exclusive, s);
     case 6: return launch_tiles<DT, LAY, 6, EPI>(g, ws, c.splits, exclusive, s);
     case 7: return launch_tiles<DT, LAY, 7, EPI>(g, ws, c.splits, exclusive, s);
+    case 9:
+      if constexpr (LAY == kNN) return launch_tiles<DT, LAY, 9, EPI>(g, ws, c.splits, exclusive, s);
+      else return hipErrorInvalidValue;
     default: return launch_tiles<DT, LAY, 8, EPI>(g, ws, c.splits, exclusive, s);
   }
 }
@@ -947,7 +988,7 @@ hipError_t tile_down_of(const TileProduct& p, const SelectArgs& select, const Ti
     case 4: return start_down<DT, 4>(p, select, c.splits, ws, s, selected, parts);
     case 7: return start_down<DT, 7>(p, select, c.splits, ws, s, selected, parts);
     case 8: return start_down<DT, 8>(p, select, c.splits, ws, s, selected, parts);
-    default: {                                                 // tiles of 256 columns: nothing beside them
+    default: {                                                 // nothing beside these
       *selected = false;
       *parts = 1;
       TileGroup g;

@@ -16,7 +16,7 @@ static int to_code(hipError_t e) { return e == hipSuccess ? OMNI_OK : e == hipEr
 
 // partial sums of d(h) or of d(x), whichever is more (they are not alive together)
 static size_t sums_bytes(int64_t T, int64_t H, int64_t I, int64_t r) {
-  const size_t dh = tile_workspace_bytes(kTileSwigluBwd, T, I, up64(H)), dx = tile_workspace_bytes(kTileResidual, T, H, 2 * up64(I) + 2 * up64(r));
+  const size_t dh = tile_workspace_bytes(kNN, kTileSwigluBwd, T, I, up64(H)), dx = tile_workspace_bytes(kNN, kTileResidual, T, H, 2 * up64(I) + 2 * up64(r));
   return dh > dx ? dh : dx;
 }
 }  // namespace omni

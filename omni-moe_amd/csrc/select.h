@@ -677,9 +677,9 @@ __device__ __forceinline__ void ktop64_2(uint32_t (&k0)[R], uint32_t (&k1)[R], c
 // every key below it is out; what is left (for scores in no particular order about 42 of 512 keys at kp = 32) goes through LDS into one register and is
 // sorted there.  Two sorts of 64 keys instead of R and the merges: 32768 tokens, 2 x 512 keys, k = 32: 211 -> 165 us.  More than 64 left, or fewer than kp lanes with a key: all of them, as above.
 constexpr int kPruneTop = 32, kPruneWaves = 8;
+typedef uint32_t PrunePool[kPruneWaves][2][kWave];            // in LDS, a block's: a place to each of up to eight waves
 template <int R>
-__device__ __forceinline__ void ktop_pruned_2(uint32_t (&k0)[R], uint32_t (&k1)[R], const int kp, const int lane) {
-  __shared__ uint32_t pool[kPruneWaves][2][kWave];
+__device__ __forceinline__ void ktop_pruned_2(uint32_t (&k0)[R], uint32_t (&k1)[R], const int kp, const int lane, PrunePool& pool) {
   uint32_t (*mine)[kWave] = pool[(threadIdx.x >> 6) % kPruneWaves];
   uint32_t m0[1] = {k0[0]}, m1[1] = {k1[0]};
 #pragma unroll
@@ -729,7 +729,7 @@ __device__ __forceinline__ uint32_t sorted_key(const uint32_t (&v)[R], int i) {
 // Same selection as select_pairs for bf16 / f16 storage, on packed keys: the tokens of wave `wave` of `num_waves`.  stats: g.stats, or what the
 // block merged.
 template <int DT, int R, int C>
-__device__ __forceinline__ void select_packed(const SelectArgs& g, const int wave, const int num_waves, const float* stats) {
+__device__ __forceinline__ void select_packed(const SelectArgs& g, const int wave, const int num_waves, const float* stats, PrunePool& pool) {
   const int lane = lane_id();
   const int r = g.r, k = g.k, kp = g.kp;
 
@@ -771,7 +771,7 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
       ky[a] = key < r ? make_key<DT>(sy[a], key) : 0u;
     }
     if constexpr (R > kUnrollMaxR) {                             // uniform: kp comes with the arguments
-      if (kp <= kPruneTop) ktop_pruned_2<R>(kx, ky, kp, lane);
+      if (kp <= kPruneTop) ktop_pruned_2<R>(kx, ky, kp, lane, pool);
       else if (kp <= kWave) ktop64_2<R>(kx, ky, lane);
       else ksort2<R>(kx, ky, lane);
     } else {
