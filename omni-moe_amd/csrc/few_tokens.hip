@@ -7,10 +7,12 @@
 //   1. the router's projection | gate and up with their SwiGLU product
 //   2. the router's selection  | the down projection, K split over the grid, as fp32 partial sums
 //   3. the experts, the partial sums and the final add, one block per token.
-// 1 token 38.4 -> 18.1 us a call (kernels 6.5 + 5.0 + 4.6), 48 tokens 42.9 -> 21.9 us (9.4 + 6.6 + 5.4), hidden 1024 x intermediate 4096.
+// 1 token 38.4 -> 18.1 us a call, 48 tokens 42.9 -> 21.9 us, hidden 1024 x intermediate 4096; with the weights through LDS as well 17.2 -> 15.3 and 21.0 -> 20.1
+// (calls in a graph; what a program sees at 1 token is the 18 us of host work of a call).
 //
-// Projections.  There is one row tile, so every weight is used once and nothing is gained by staging it through LDS: a lane loads
-// its matrix fragments (8 consecutive K values of a row) straight from memory, all loads of 1024 K values of a block in flight at once.
+// Projections.  There is one row tile, so every weight is used once, and all loads of 1024 K values of a block are in flight at once.  They go through
+// each wave's own LDS all the same, because an instruction that reads eight whole 128-byte lines is faster than the one that a matrix fragment asks for,
+// 64 bytes from each of 16 rows (kWeightsInLds; straight into registers where two blocks would not fit a CU).
 // The eight waves of a block share the K range -- a wave takes 64 of K, a 128-byte line of each row, in turn -- and add up
 // through LDS in wave order.  A block has 32 weight rows: 16 gate and the matching 16 up rows, 16 x and 16 y keys, or 32 rows of the
 // down projection; with K split up to eight ways the latter fill the chip too.
@@ -39,88 +41,124 @@ template <int DT> __device__ __forceinline__ uint32_t pack2(float lo, float hi) 
   if constexpr (DT == kBF16) return pack_bf16(lo, hi); else return pack_f16(lo, hi);
 }
 
-// acc[j][i]: rows 16 i + lane % 16 of `a` ([rows of row_bytes], a_bytes in all, K values a row; TM row tiles, zeros past the matrix) times the 16
+// A wave's LDS: Q units of R8 times eight rows of activations, and the same units of the block's 32 weight rows.  These stay in registers for more than 48 tokens: with
+// them two blocks would not fit a CU (64 tokens 22.1 us; one block to a CU 22.9).
+template <int R8, int Q>
+struct FewStage {
+  static constexpr bool kWeightsInLds = R8 <= 6;
+  static constexpr int kRows = Q * R8 * 1024, kPart = kRows + (kWeightsInLds ? Q * 4096 : 0), kBytes = kFewWaves * kPart;
+};
+
+// acc[j][i]: rows 16 i + lane % 16 of `a` ([rows of row_bytes], a_bytes in all, K values a row; zeros past the matrix, and beyond 8 R8 rows whatever) times the 16
 // rows of weight tile j, columns 4 (lane / 16) .. + 3, over the K units u0 + wave, u0 + wave + 8, .. below u1, Q at a time.
-// Weights: this lane's row b0 or b1, straight into registers, Q units ahead.  Activations: every block reads all of them, from L2, and reads of
-// 64 bytes from each of 16 rows -- what a fragment is -- are slow there (64 tokens, hidden 1024: 15.4 us for launch 1, 10.1 us when an
-// instruction reads 1 KiB on end); so they take whole 128-byte lines of 8 rows into the wave's own `lds` (Q * TM * 2 KiB; position c of row r
-// holds the row's 16-byte piece c ^ (r / 2 % 8), which keeps the fragment reads free of bank conflicts).
+// left[j]: weight rows from b[j] on (at least one; the last one stands in for those past it).  Weights are requested Q units ahead of their use.
+// Every block reads all activations, from L2.  Reads of 64 bytes from each of 16 rows -- what a fragment is -- are slow (activations so, 64 tokens, hidden 1024: 15.4 us
+// for launch 1, 10.1 us when an instruction reads 1 KiB on end; weights so, a call in a graph, hidden 1024 x intermediate 4096: 1 / 8 / 12 / 32 / 48 tokens 17.2 / 18.5 / 18.7 / 20.0 / 21.0 us, by whole lines 15.3 / 16.7 / 17.0 / 18.3 / 20.1;
+// 2048 x 8192, 1 token 35.2 -> 32.5);
+// so both take whole 128-byte lines of 8 rows into the wave's own `lds` (position c of row r holds the row's 16-byte piece c ^ (r / 2 % 8), which
+// keeps the fragment reads free of bank conflicts).
 // kTail: K is no multiple of 64 (but of 8); what is past it reads as zero on both sides.
-template <int DT, int TM, int Q, bool kTail>
-__device__ __forceinline__ void multiply(f32x4_t (&acc)[2][TM], const uint8_t* a, int row_bytes, int a_bytes, const uint8_t* b0, const uint8_t* b1, int K, int u0, int u1,
-                                         int wave, int lane, uint32_t lds) {
+template <int DT, int R8, int Q, bool kTail>
+__device__ __forceinline__ void multiply(f32x4_t (&acc)[2][(R8 + 1) / 2], const uint8_t* a, int row_bytes, int a_bytes, const uint8_t* const (&b)[2], const int (&left)[2], int K,
+                                         int u0, int u1, int wave, int lane, uint32_t lds) {
+  constexpr int TM = (R8 + 1) / 2;
+  using Stage = FewStage<R8, Q>;
   const int r16 = lane & 15, g4 = lane >> 4;
   using Frag = const __attribute__((address_space(3))) u32x4_t*;
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < TM; ++i) acc[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  u32x4_t b[Q][2][2];                                          // [unit][half of it][weight tile]
+  const int row = lane >> 3;
+  // lane's place in the 8 rows that load instruction `part` of unit q brings in, of K step u: r / 2 % 8 = 4 (part % 2) + lane / 16
+  auto offset = [&](int u, int q, int part, int at_row) __attribute__((always_inline)) {
+    const int piece = (lane & 7) ^ (4 * (part & 1) + (lane >> 4)), v = u + q * kFewWaves, k = v * kUnit + piece * 8;
+    return v < u1 && !(kTail && k >= K) ? (uint32_t)(at_row * row_bytes + k * 2) : 0x80000000u;
+  };
+  u32x4_t w[Q][2][2], next[Q][2][2];                           // [unit][half of it][weight tile]
   auto load_weights = [&](int u) __attribute__((always_inline)) {
+    if constexpr (Stage::kWeightsInLds) {
+      auto one = [&](auto n_tag) __attribute__((always_inline)) {
+        constexpr int n = decltype(n_tag)::value, q = n / 4, part = n % 4, j = part / 2;
+        load_to_lds<Stage::kRows + n * 1024>((uint64_t)b[j], min(left[j], 16) * row_bytes, lds, offset(u, q, part, min((part & 1) * 8 + row, left[j] - 1)), 0);
+      };
+      auto all = [&](auto... n) __attribute__((always_inline)) { (one(n), ...); };
+      with_sequence(all, std::make_integer_sequence<int, 4 * Q>{});
+    } else {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int v = u + q * kFewWaves;
+      for (int q = 0; q < Q; ++q) {
+        const int v = u + q * kFewWaves;
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const int k = v * kUnit + ks * 32 + g4 * 8;
-        const bool inside = v < u1 && !(kTail && k >= K);
-        b[q][ks][0] = inside ? *(const u32x4_t*)(b0 + (int64_t)k * 2) : u32x4_t{0, 0, 0, 0};
-        b[q][ks][1] = inside ? *(const u32x4_t*)(b1 + (int64_t)k * 2) : u32x4_t{0, 0, 0, 0};
+        for (int ks = 0; ks < 2; ++ks) {
+          const int k = v * kUnit + ks * 32 + g4 * 8;
+          const bool inside = v < u1 && !(kTail && k >= K);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) next[q][ks][j] = inside ? *(const u32x4_t*)(b[j] + (int64_t)min(r16, left[j] - 1) * row_bytes + (int64_t)k * 2) : u32x4_t{0, 0, 0, 0};
+        }
       }
     }
   };
-  const uint32_t row = (uint32_t)(lane >> 3), from = row * (uint32_t)row_bytes;
   load_weights(u0 + wave);
   for (int u = u0 + wave; u < u1; u += Q * kFewWaves) {
     auto load_rows = [&](auto n_tag) __attribute__((always_inline)) {
-      constexpr int n = decltype(n_tag)::value, q = n / (2 * TM), part = n % (2 * TM);
-      // rows 8 part + lane / 8: r / 2 % 8 = 4 (part % 2) + lane / 16
-      const int piece = (lane & 7) ^ (4 * (part & 1) + (lane >> 4)), k = (u + q * kFewWaves) * kUnit + piece * 8;
-      const bool inside = u + q * kFewWaves < u1 && !(kTail && k >= K);
-      load_to_lds<n * 1024>((uint64_t)a, a_bytes, lds, inside ? from + (uint32_t)(part * 8 * row_bytes + k * 2) : 0x80000000u, 0);
+      constexpr int n = decltype(n_tag)::value, q = n / R8, part = n % R8;
+      load_to_lds<n * 1024>((uint64_t)a, a_bytes, lds, offset(u, q, part, 8 * part + row), 0);
     };
     auto load_all = [&](auto... n) __attribute__((always_inline)) { (load_rows(n), ...); };
-    with_sequence(load_all, std::make_integer_sequence<int, 2 * Q * TM>{});
+    with_sequence(load_all, std::make_integer_sequence<int, Q * R8>{});
     vmcnt<0>();
     __builtin_amdgcn_sched_barrier(0);
-    u32x4_t w[Q][2][2];
+    auto fragment = [&](uint32_t at, int ks, int r) __attribute__((always_inline)) { return *(Frag)(uintptr_t)(lds + at + (uint32_t)(r * 128 + ((4 * ks + g4) ^ ((r >> 1) & 7)) * 16)); };
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) w[q][ks][j] = b[q][ks][j];
-    if (u + Q * kFewWaves < u1) load_weights(u + Q * kFewWaves);
+        for (int j = 0; j < 2; ++j) {
+          if constexpr (Stage::kWeightsInLds) w[q][ks][j] = fragment(Stage::kRows + q * 4096 + j * 2048, ks, r16);
+          else w[q][ks][j] = next[q][ks][j];
+        }
+    if (u + Q * kFewWaves < u1) {
+      if constexpr (Stage::kWeightsInLds) {
+        lds_reads_done();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      load_weights(u + Q * kFewWaves);
+    }
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-          const u32x4_t f = *(Frag)(uintptr_t)(lds + (uint32_t)((q * TM + i) * 2048 + r16 * 128 + ((4 * ks + g4) ^ (r16 >> 1)) * 16));
+          const u32x4_t f = fragment(q * R8 * 1024 + i * 2048, ks, R8 == 1 ? r16 & 7 : r16);
           acc[0][i] = mfma<DT>(w[q][ks][0], f, acc[0][i]);
           acc[1][i] = mfma<DT>(w[q][ks][1], f, acc[1][i]);
         }
     lds_reads_done();                                          // before the next loads overwrite what they read
   }
+  vmcnt<0>();                                                  // (a wave without a unit has asked for zeros)
 }
 
-// The block's eight sums meet in LDS, each at the start of its wave's own Q * TM * 2 KiB
-template <int TM, int Q>
-__device__ __forceinline__ void publish(uint8_t* lds, const f32x4_t (&acc)[2][TM], int wave, int lane) {
+// The block's eight sums meet in LDS, each at the start of its wave's own part of it
+template <int R8, int Q>
+__device__ __forceinline__ void publish(uint8_t* lds, const f32x4_t (&acc)[2][(R8 + 1) / 2], int wave, int lane) {
+  constexpr int TM = (R8 + 1) / 2;
+  static_assert(FewStage<R8, Q>::kPart >= TM * 2048, "a wave's sums fit its part");
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int i = 0; i < TM; ++i) *(f32x4_t*)(lds + wave * Q * TM * 2048 + ((j * TM + i) * kWave + lane) * 16) = acc[j][i];
+    for (int i = 0; i < TM; ++i) *(f32x4_t*)(lds + wave * FewStage<R8, Q>::kPart + ((j * TM + i) * kWave + lane) * 16) = acc[j][i];
   __syncthreads();
 }
 // columns 4 quad .. + 3 of row `row` of weight tile j, all waves
-template <int TM, int Q>
+template <int R8, int Q>
 __device__ __forceinline__ f32x4_t gathered(const uint8_t* lds, int j, int row, int quad) {
+  constexpr int TM = (R8 + 1) / 2;
   f32x4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int w = 0; w < kFewWaves; ++w) {
-    const f32x4_t o = *(const f32x4_t*)(lds + w * Q * TM * 2048 + ((j * TM + row / 16) * kWave + quad * 16 + row % 16) * 16);
+    const f32x4_t o = *(const f32x4_t*)(lds + w * FewStage<R8, Q>::kPart + ((j * TM + row / 16) * kWave + quad * 16 + row % 16) * 16);
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] += o[q];
   }
@@ -134,21 +172,23 @@ struct FrontArgs {
 };
 
 // Launch 1: blocks below router_blocks project 16 keys of each half, the others 16 columns of gate and of up.
-template <int DT, int TM, int Q, bool kTail>
-__global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_front_kernel(const FrontArgs g) {
-  extern __shared__ __align__(16) uint8_t lds[];               // Q * TM * 2 KiB a wave
-  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15;
-  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * Q * TM * 2048;
+template <int DT, int R8, int Q, bool kTail>
+__global__ __launch_bounds__(kFewThreads, Q == 1 || R8 == 1 ? 4 : 2) void few_front_kernel(const FrontArgs g) {
+  extern __shared__ __align__(16) uint8_t lds[];               // FewStage
+  constexpr int TM = (R8 + 1) / 2;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave * FewStage<R8, Q>::kPart);
   const bool router = (int)blockIdx.x < g.router_blocks;
   const int n0 = (router ? (int)blockIdx.x : (int)blockIdx.x - g.router_blocks) * 16, rows = router ? g.r : g.I;
-  const int64_t row_bytes = (int64_t)g.H * 2, b_at = min(n0 + r16, rows - 1) * row_bytes;
+  const int64_t b_at = n0 * ((int64_t)g.H * 2);
   f32x4_t acc[2][TM];
-  multiply<DT, TM, Q, kTail>(acc, g.x, g.H * 2, g.T * g.H * 2, (router ? g.wx : g.wg) + b_at, (router ? g.wy : g.wu) + b_at, g.H, 0, (g.H + kUnit - 1) / kUnit, wave, lane, mine);
-  publish<TM, Q>(lds, acc, wave, lane);
+  multiply<DT, R8, Q, kTail>(acc, g.x, g.H * 2, g.T * g.H * 2, {(router ? g.wx : g.wg) + b_at, (router ? g.wy : g.wu) + b_at}, {rows - n0, rows - n0}, g.H, 0, (g.H + kUnit - 1) / kUnit,
+                             wave, lane, mine);
+  publish<R8, Q>(lds, acc, wave, lane);
   for (int i = threadIdx.x; i < TM * 64; i += kFewThreads) {
     const int row = i >> 2, quad = i & 3, n = n0 + quad * 4;
     if (row >= g.T || n >= rows) continue;
-    const f32x4_t p = gathered<TM, Q>(lds, 0, row, quad), q = gathered<TM, Q>(lds, 1, row, quad);
+    const f32x4_t p = gathered<R8, Q>(lds, 0, row, quad), q = gathered<R8, Q>(lds, 1, row, quad);
     if (router) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -175,14 +215,16 @@ struct MiddleArgs {
 };
 
 // Launch 2: blocks below select_blocks select for eight tokens each, the others multiply 32 output columns over one of the K splits.
-template <int DT, int TM, int Q, bool kTail, bool kSelect, int C>
+template <int DT, int R8, int Q, bool kTail, bool kSelect, int C>
 __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel(const MiddleArgs g) {
-  extern __shared__ __align__(16) uint8_t lds[];               // Q * TM * 2 KiB a wave
-  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15;
-  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wave * Q * TM * 2048;
+  extern __shared__ __align__(16) uint8_t lds[];               // FewStage
+  constexpr int TM = (R8 + 1) / 2;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave * FewStage<R8, Q>::kPart);
   if constexpr (kSelect) {
     if ((int)blockIdx.x < g.select_blocks) {
-      __shared__ PrunePool pool;
+      static_assert(FewStage<R8, Q>::kBytes >= (int)sizeof(PrunePool), "a block that selects prunes there");
+      PrunePool& pool = *(PrunePool*)lds;
       const int first = (int)blockIdx.x * kFewWaves + wave, all = g.select_blocks * kFewWaves;
       if (g.select_regs <= 1) select_packed<DT, 1, C>(g.select, first, all, g.select.stats, pool);
       else if (g.select_regs <= 2) select_packed<DT, 2, C>(g.select, first, all, g.select.stats, pool);
@@ -193,13 +235,14 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel
   }
   const int block = (int)blockIdx.x - (kSelect ? g.select_blocks : 0), split = block / g.groups, n0 = (block - split * g.groups) * 32;
   const int64_t row_bytes = (int64_t)g.I * 2;
+  const int second = min(n0 + 16, g.H - 1);
   f32x4_t acc[2][TM];
-  multiply<DT, TM, Q, kTail>(acc, g.h, g.I * 2, g.T * g.I * 2, g.wd + min(n0 + r16, g.H - 1) * row_bytes, g.wd + min(n0 + 16 + r16, g.H - 1) * row_bytes, g.I, split * g.units,
-                          min((split + 1) * g.units, (g.I + kUnit - 1) / kUnit), wave, lane, mine);
-  publish<TM, Q>(lds, acc, wave, lane);
+  multiply<DT, R8, Q, kTail>(acc, g.h, g.I * 2, g.T * g.I * 2, {g.wd + n0 * row_bytes, g.wd + second * row_bytes}, {g.H - n0, g.H - second}, g.I, split * g.units,
+                             min((split + 1) * g.units, (g.I + kUnit - 1) / kUnit), wave, lane, mine);
+  publish<R8, Q>(lds, acc, wave, lane);
   for (int i = threadIdx.x; i < TM * 128; i += kFewThreads) {
     const int row = i >> 3, quad = i & 7, n = n0 + quad * 4;
-    if (row < g.T && n < g.H) *(f32x4_t*)(g.parts + ((int64_t)split * g.T + row) * g.H + n) = gathered<TM, Q>(lds, quad >> 2, row, quad & 3);
+    if (row < g.T && n < g.H) *(f32x4_t*)(g.parts + ((int64_t)split * g.T + row) * g.H + n) = gathered<R8, Q>(lds, quad >> 2, row, quad & 3);
   }
 }
 
@@ -345,26 +388,23 @@ hipError_t launch_back(const BackArgs& b, hipStream_t s) {
   return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, b.T, s);
 }
 
-template <int DT, int TM>
+template <int DT, int R8>
 hipError_t launch(const FewTokens& f, hipStream_t s) {
   const bool layer = f.up != nullptr;
   const int r = f.select.r;
   const FrontArgs a{(const uint8_t*)f.x, (const uint8_t*)f.wg, (const uint8_t*)f.wu, (const uint8_t*)f.wx, (const uint8_t*)f.wy, (uint8_t*)f.h, (uint8_t*)f.z,
                     f.T, f.H, f.I, r, layer ? (r + 15) / 16 : 0};
   const int64_t front = a.router_blocks + (f.I + 15) / 16;
-  // From 33 tokens on, two K units of a wave in LDS at once are more than half of a CU's: one block to a CU, and blocks beyond 256 wait for a whole round.
-  // One unit at a time then (in turn over three sets of inputs, hidden 1024 x intermediate 4096: 33 tokens 23.5 -> 21.3 us, 48 24.1 -> 21.9, 64 26.2 -> 22.9;
-  // 48 tokens, 2048 x 8192 49.9 -> 43.9).  Where the first launch has no more blocks than CUs both units stay in flight.
-  constexpr bool kWide = TM >= 3;
+  // Beyond eight tokens two K units of a wave in LDS at once are more than half of a CU's: one block to a CU, and blocks beyond 256 wait for a whole round.
+  // One unit at a time then (in turn over three sets of inputs, hidden 1024 x intermediate 4096, weights in registers: 33 tokens 23.5 -> 21.3 us, 48 24.1 -> 21.9, 64
+  // 26.2 -> 22.9; 48 tokens, 2048 x 8192 49.9 -> 43.9).  Where a launch has no more blocks than CUs both units stay in flight, if a wave has two.
   auto units_at_once = [&](bool one, auto&& go) -> hipError_t {
-    if constexpr (kWide) {
-      if (one) return go(std::integral_constant<int, 1>{});
-    }
+    if (one) return go(std::integral_constant<int, 1>{});
     return go(std::integral_constant<int, 2>{});
   };
-  hipError_t e = units_at_once(front > 256, [&](auto q) -> hipError_t {
-    constexpr int Q = decltype(q)::value, kBytes = kFewWaves * Q * TM * 2048;
-    return f.H % kUnit ? start<few_front_kernel<DT, TM, Q, true>, kBytes>(a, front, s) : start<few_front_kernel<DT, TM, Q, false>, kBytes>(a, front, s);
+  hipError_t e = units_at_once((R8 > 1 && front > 256) || f.H <= kFewWaves * kUnit, [&](auto q) -> hipError_t {
+    constexpr int Q = decltype(q)::value, kBytes = FewStage<R8, Q>::kBytes;
+    return f.H % kUnit ? start<few_front_kernel<DT, R8, Q, true>, kBytes>(a, front, s) : start<few_front_kernel<DT, R8, Q, false>, kBytes>(a, front, s);
   });
   if (e != hipSuccess) return e;
 
@@ -375,13 +415,13 @@ hipError_t launch(const FewTokens& f, hipStream_t s) {
   splits = (units + m.units - 1) / m.units;                    // every split has work
   const int cells = prepare_select(m.select);
   const int64_t middle = m.select_blocks + (int64_t)m.groups * splits;
-  e = units_at_once(middle > 256 || m.units <= kFewWaves, [&](auto q) -> hipError_t {           // (a wave may have one unit only)
-    constexpr int Q = decltype(q)::value, kBytes = kFewWaves * Q * TM * 2048;
+  e = units_at_once((R8 > 1 && middle > 256) || m.units <= kFewWaves, [&](auto q) -> hipError_t {           // (a wave may have one unit only)
+    constexpr int Q = decltype(q)::value, kBytes = FewStage<R8, Q>::kBytes;
     auto go = [&](auto tail) -> hipError_t {
       constexpr bool kTail = decltype(tail)::value;
-      if (!layer) return start<few_middle_kernel<DT, TM, Q, kTail, false, 1>, kBytes>(m, middle, s);
-      if (cells <= 1) return start<few_middle_kernel<DT, TM, Q, kTail, true, 1>, kBytes>(m, middle, s);
-      return start<few_middle_kernel<DT, TM, Q, kTail, true, 2>, kBytes>(m, middle, s);
+      if (!layer) return start<few_middle_kernel<DT, R8, Q, kTail, false, 1>, kBytes>(m, middle, s);
+      if (cells <= 1) return start<few_middle_kernel<DT, R8, Q, kTail, true, 1>, kBytes>(m, middle, s);
+      return start<few_middle_kernel<DT, R8, Q, kTail, true, 2>, kBytes>(m, middle, s);
     };
     return f.I % kUnit ? go(std::true_type{}) : go(std::false_type{});
   });
@@ -412,10 +452,11 @@ size_t few_tokens_parts_bytes(int64_t T, int64_t H, int64_t I) { return (size_t)
 hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s) {
   auto go = [&](auto dt) -> hipError_t {
     constexpr int DT = decltype(dt)::value;
-    if (f.T <= 16) return launch<DT, 1>(f, s);
-    if (f.T <= 32) return launch<DT, 2>(f, s);
-    if (f.T <= 48) return launch<DT, 3>(f, s);
-    return launch<DT, 4>(f, s);
+    if (f.T <= 8) return launch<DT, 1>(f, s);
+    if (f.T <= 16) return launch<DT, 2>(f, s);
+    if (f.T <= 32) return launch<DT, 4>(f, s);
+    if (f.T <= 48) return launch<DT, 6>(f, s);
+    return launch<DT, 8>(f, s);
   };
   if (dtype == kBF16) return go(std::integral_constant<int, kBF16>{});
   if (dtype == kF16) return go(std::integral_constant<int, kF16>{});

@@ -762,6 +762,17 @@ def test_mlp_bwd_matches_matmuls(case, dtype, device):
         assert (err.abs().max() <= 4 * ulp * w.abs().max()).item(), (name, (err.abs().max() / w.abs().max()).item())
 
 
+# T, H, I, r: d(x) as sums so long that it takes two K groups on 128 x 128 tiles: whole tiles, rows one past a tile and columns short of one, K tails of the 128 of K that a
+# ring step takes (4104 = 32 * 128 + 8; the router's 64 and 17)
+LONG_SUM_CASES = [(2048, 2048, 4096, 64), (1921, 2040, 4104, 17), (1921, 1928, 4104, 0)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", LONG_SUM_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_mlp_bwd_long_sums(case, dtype, device):
+    test_mlp_bwd_matches_matmuls(case, dtype, device)
+
+
 # T, H, I, r: products that take the tiles of 224, 192 and 96 rows: one row past a tile, one short of it and whole tiles; K tails; split K; more tiles than CUs
 LOWER_TILE_CASES = [(65, 136, 520, 17), (449, 136, 4104, 0), (673, 136, 6152, 17), (1537, 136, 4104, 17), (193, 776, 6152, 17), (3361, 264, 520, 8), (2497, 136, 6152, 0),
                     (2015, 136, 6152, 17), (129, 512, 6152, 64), (200, 1024, 4096, 17), (1344, 264, 2568, 17), (3071, 512, 6144, 64)]

@@ -29,6 +29,18 @@ def _elsewhere(t, device):
     return out
 
 
+# T, H, I, N, k: whole lines of the weights: eight tokens (a half tile of activations) and nine, 16 and 32 and one more; waves without a unit of K (hidden below 512,
+# intermediate below 512), a second column tile of the down projection with 8 columns or none (hidden 520, 528), one and two units of K at a time in either launch
+FEW_TOKEN_LINES = [(8, 1024, 4096, 4096, 16), (9, 528, 4104, 1000, 8), (7, 520, 72, 64, 2), (24, 264, 264, 1024, 8), (32, 1032, 4104, 4096, 16), (10, 2048, 2056, 260, 4),
+                   (28, 1288, 520, 17000, 6), (40, 72, 8200, 900, 4)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", FEW_TOKEN_LINES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
+def test_few_tokens_weights_by_lines(case, dtype, device):
+    test_few_tokens_match_the_operators(case, dtype, device)
+
+
 # the first four are the reference's benchmark grid (tests/test_mlp.py:144-150): intermediate 1024 .. 65536
 MLP_CASES = [(1024, 1024, 1024), (1024, 1024, 4096), (1024, 1024, 16384), (1024, 1024, 65536), (4096, 1024, 4096), (4100, 1024, 4096),
              (333, 256, 1000), (128, 64, 128), (512, 2048, 8192), (5, 8, 8),
