@@ -6,9 +6,9 @@
 // each other shares a launch, by block index:
 //   1. the router's projection | gate and up with their SwiGLU product
 //   2. the router's selection  | the down projection, K split over the grid, as fp32 partial sums
-//   3. the experts, the partial sums and the final add, one block per token.
+//   3. the experts, the partial sums and the final add, one block per token; up to 16 tokens of a small layer in launch 2 (further down).
 // 1 token 38.4 -> 18.1 us a call, 48 tokens 42.9 -> 21.9 us, hidden 1024 x intermediate 4096; with the weights through LDS as well 17.2 -> 15.3 and 21.0 -> 20.1
-// (calls in a graph; what a program sees at 1 token is the 18 us of host work of a call).
+// (calls in a graph; a program sees the 18 us of host work of a call at 1 token, 15.2 with two launches).
 //
 // Projections.  There is one row tile, so every weight is used once, and all loads of 1024 K values of a block are in flight at once.  They go through
 // each wave's own LDS all the same, because an instruction that reads eight whole 128-byte lines is faster than the one that a matrix fragment asks for,
@@ -169,6 +169,8 @@ struct FrontArgs {
   const uint8_t *x, *wg, *wu, *wx, *wy;
   uint8_t *h, *z;
   int T, H, I, r, router_blocks;
+  uint32_t* tickets;                 // [T][groups], or NULL: cleared for launch 2
+  int num_tickets;
 };
 
 // Launch 1: blocks below router_blocks project 16 keys of each half, the others 16 columns of gate and of up.
@@ -179,6 +181,7 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 || R8 == 1 ? 4 : 2) void few_fr
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave * FewStage<R8, Q>::kPart);
   const bool router = (int)blockIdx.x < g.router_blocks;
+  for (int i = (int)blockIdx.x * kFewThreads + (int)threadIdx.x; i < g.num_tickets; i += (int)gridDim.x * kFewThreads) g.tickets[i] = 0;
   const int n0 = (router ? (int)blockIdx.x : (int)blockIdx.x - g.router_blocks) * 16, rows = router ? g.r : g.I;
   const int64_t b_at = n0 * ((int64_t)g.H * 2);
   f32x4_t acc[2][TM];
@@ -206,145 +209,254 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 || R8 == 1 ? 4 : 2) void few_fr
   }
 }
 
+// ---- launch 2, and for few tokens of a small layer launch 3 with it.
+// A call of three launches is 18 us of host work, where the kernels of 1 token, hidden 1024 x intermediate 4096, take 15.  The third one needs every split of the
+// down projection and the token's experts; so a block per token selects and sums up its experts, and whoever comes last adds up: a ticket per token and
+// group of 32 columns, cleared by launch 1, counts the splits and the token's block, and the one that takes the last number finds all parts there and
+// writes y's 32 values.  Nobody waits.  What others read is stored and loaded at agent scope (the XCDs' L2s are not one cache), and a block takes its
+// numbers when its stores have been acknowledged.  Kernels of three launches / two in a graph, and calls as a program makes them: 1 token 15.3 / 14.9, 18.3 / 15.2 us;
+// 12 tokens 17.0 / 16.8; 512 x 2048, 1 token 9.8 / 9.9; but 24 tokens 18.2 / 18.3, 48 19.5 / 20.0, 64 22.3 / 23.4; 2048 x 8192, 1 token 33.6 / 34.0 (merge_launches).
 struct MiddleArgs {
   const uint8_t *h, *wd;
   float* parts;                      // [splits][T][H]
-  int T, H, I, groups, units;        // groups of 32 output columns; K units to a split
-  int select_blocks, select_regs;    // keys per lane
+  int T, H, I, groups, units, splits;    // groups of 32 output columns; K units to a split
+  int select_blocks, select_regs, cells; // the first blocks select, for eight tokens each (merged: for one); keys and candidates per lane
   SelectArgs select;
+  // merged
+  uint32_t* tickets;                 // [T][groups]
+  uint8_t* experts;                  // [T][H] the experts' rounded sums
+  const uint8_t *x, *up, *down;
+  uint8_t* y;
+  uint32_t N;
 };
+constexpr int kMergedTokens = 16, kMergedRow = 1024;           // (a token's block has a thread for four values of a row)
+bool merge_launches(int64_t T, int64_t H, int64_t I) { return T <= kMergedTokens && H <= kMergedRow && H * I <= (1 << 23); }
+__device__ __forceinline__ void store_agent(void* at, uint32_t a, uint32_t b) {
+  __hip_atomic_store((uint64_t*)at, (uint64_t)a | (uint64_t)b << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u32x2_t load_agent(const void* at) {
+  const uint64_t v = __hip_atomic_load((const uint64_t*)at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return u32x2_t{(uint32_t)v, (uint32_t)(v >> 32)};
+}
+__device__ __forceinline__ bool takes_last(const MiddleArgs& g, int t, int group) {           // of the splits' numbers and the token's block's
+  return __hip_atomic_fetch_add(g.tickets + t * g.groups + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)g.splits;
+}
+__device__ __forceinline__ void stores_acknowledged() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+// four columns of a token: y = round(round(sum of the parts in split order) + e)
+template <int DT>
+__device__ __forceinline__ void add_up(const MiddleArgs& g, int t, int n, const u32x2_t e) {
+  u32x2_t part[kMostParts][2];
+#pragma unroll
+  for (int s = 0; s < kMostParts; ++s)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) part[s][q] = load_agent(g.parts + ((int64_t)min(s, g.splits - 1) * g.T + t) * g.H + n + 2 * q);
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < kMostParts; ++s)
+    if (s < g.splits)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] += __uint_as_float(part[s][q / 2][q % 2]);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = Elem<DT>::round(v[q]) + Elem<DT>::load(&e, q);
+  *(u32x2_t*)(g.y + ((int64_t)t * g.H + n) * 2) = u32x2_t{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+}
 
-// Launch 2: blocks below select_blocks select for eight tokens each, the others multiply 32 output columns over one of the K splits.
-template <int DT, int R8, int Q, bool kTail, bool kSelect, int C>
+template <int DT>
+__device__ __forceinline__ void select_tokens(const MiddleArgs& g, int first, int all, PrunePool& pool) {
+  auto select = [&](auto cells) {
+    constexpr int C = decltype(cells)::value;
+    if (g.select_regs <= 1) select_packed<DT, 1, C>(g.select, first, all, g.select.stats, pool);
+    else if (g.select_regs <= 2) select_packed<DT, 2, C>(g.select, first, all, g.select.stats, pool);
+    else if (g.select_regs <= 4) select_packed<DT, 4, C>(g.select, first, all, g.select.stats, pool);
+    else select_packed<DT, 8, C>(g.select, first, all, g.select.stats, pool);
+  };
+  if (g.cells <= 1) select(std::integral_constant<int, 1>{});
+  else select(std::integral_constant<int, 2>{});
+}
+
+// The experts of a token by the block's eight waves, which share its slots so that all its rows are requested at once.  Leaves wave w's sums, in fp32, at
+// sums + w * stride.  NCH 1-KiB pieces of a row; G slots of a wave at once.  Returns the waves that had any.
+struct FewExperts { const uint8_t *x, *up, *down; const void* gates; const int32_t* ids; int H, k; uint32_t N; };
+template <int DT, int NCH, int G>
+__device__ __forceinline__ int share_experts(const FewExperts& g, int t, int wave, int lane, float* sums, int stride) {
+  const int per = (g.k + kFewWaves - 1) / kFewWaves, active = (g.k + per - 1) / per;
+  if (wave >= active) return active;
+  const int64_t row_bytes = (int64_t)g.H * 2;
+  bool live[NCH];
+  u32x4_t xr[NCH];
+  float acc[NCH][8];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    live[c] = (c * kWave + lane) * 8 < g.H;
+    xr[c] = live[c] ? *(const u32x4_t*)(g.x + t * row_bytes + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[c][i] = 0.f;
+  }
+  const int last = min((wave + 1) * per, g.k);
+  for (int j0 = wave * per; j0 < last; j0 += G) {
+    int64_t at[G];
+    float gate[G];
+    bool ok[G];
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      const int j = min(j0 + i, last - 1), id = g.ids[(int64_t)t * g.k + j];
+      gate[i] = Elem<DT>::load(g.gates, (int64_t)t * g.k + j);
+      ok[i] = j0 + i < last && (uint32_t)id < g.N;             // a slot of another wave, or an id outside the table, contributes nothing
+      at[i] = ok[i] ? id * row_bytes : 0;
+    }
+    u32x4_t u[G][NCH], v[G][NCH];
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        u[i][c] = live[c] ? *(const u32x4_t*)(g.up + at[i] + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
+        v[i][c] = live[c] ? *(const u32x4_t*)(g.down + at[i] + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
+      }
+    float s[G];
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      s[i] = 0.f;
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) s[i] = dot16<DT>(xr[c], u[i][c], s[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < G; ++i) s[i] = wave_sum(s[i]);
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      if (!ok[i]) continue;                                    // not even 0 * row: the stand-in row may hold Inf or NaN
+      const float coef = silu_f32(s[i]) * gate[i];
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) axpy16<DT>(coef, v[i][c], acc[c]);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NCH; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (live[c])
+        *(f32x4_t*)(sums + wave * stride + (c * kWave + lane) * 8 + 4 * h) = f32x4_t{acc[c][4 * h], acc[c][4 * h + 1], acc[c][4 * h + 2], acc[c][4 * h + 3]};
+  return active;
+}
+
+template <int DT>
+__device__ __forceinline__ void token_block(const MiddleArgs& g, int t, uint8_t* lds, int wave, int lane) {
+  if (wave == 0) select_tokens<DT>(g, t, g.T, *(PrunePool*)lds);
+  __syncthreads();
+  float* sums = (float*)lds;                                   // [waves][H]
+  const FewExperts f{g.x, g.up, g.down, g.select.gates, g.select.indices, g.H, g.select.k, g.N};
+  const int active = share_experts<DT, kMergedRow / 512, 4>(f, t, wave, lane, sums, g.H);
+  __syncthreads();
+  const int n = (int)threadIdx.x * 4;
+  u32x2_t e{0, 0};
+  if (n < g.H) {
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int w = 0; w < active; ++w) {
+      const f32x4_t o = *(const f32x4_t*)(sums + w * g.H + n);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] += o[q];
+    }
+    e = u32x2_t{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+    store_agent(g.experts + ((int64_t)t * g.H + n) * 2, e[0], e[1]);
+  }
+  stores_acknowledged();
+  uint8_t* last = lds;                                         // (the sums have been read)
+  if ((int)threadIdx.x < g.groups) last[threadIdx.x] = takes_last(g, t, (int)threadIdx.x);
+  __syncthreads();
+  if (n < g.H && last[n >> 5]) add_up<DT>(g, t, n, e);
+}
+
+// Blocks below select_blocks select (merged: and sum up a token's experts), the others multiply 32 output columns over one of the K splits.
+template <int DT, int R8, int Q, bool kMerged>
 __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel(const MiddleArgs g) {
   extern __shared__ __align__(16) uint8_t lds[];               // FewStage
   constexpr int TM = (R8 + 1) / 2;
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave * FewStage<R8, Q>::kPart);
-  if constexpr (kSelect) {
-    if ((int)blockIdx.x < g.select_blocks) {
-      static_assert(FewStage<R8, Q>::kBytes >= (int)sizeof(PrunePool), "a block that selects prunes there");
-      PrunePool& pool = *(PrunePool*)lds;
-      const int first = (int)blockIdx.x * kFewWaves + wave, all = g.select_blocks * kFewWaves;
-      if (g.select_regs <= 1) select_packed<DT, 1, C>(g.select, first, all, g.select.stats, pool);
-      else if (g.select_regs <= 2) select_packed<DT, 2, C>(g.select, first, all, g.select.stats, pool);
-      else if (g.select_regs <= 4) select_packed<DT, 4, C>(g.select, first, all, g.select.stats, pool);
-      else select_packed<DT, 8, C>(g.select, first, all, g.select.stats, pool);
-      return;
-    }
+  static_assert(FewStage<R8, Q>::kBytes >= (int)sizeof(PrunePool), "a block that selects prunes there");
+  static_assert(!kMerged || FewStage<R8, Q>::kBytes >= kFewWaves * kMergedRow * 4, "a token's block has its waves' sums there");
+  if ((int)blockIdx.x < g.select_blocks) {
+    if constexpr (kMerged) token_block<DT>(g, (int)blockIdx.x, lds, wave, lane);
+    else select_tokens<DT>(g, (int)blockIdx.x * kFewWaves + wave, g.select_blocks * kFewWaves, *(PrunePool*)lds);
+    return;
   }
-  const int block = (int)blockIdx.x - (kSelect ? g.select_blocks : 0), split = block / g.groups, n0 = (block - split * g.groups) * 32;
+  const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave * FewStage<R8, Q>::kPart);
+  const int block = (int)blockIdx.x - g.select_blocks, split = block / g.groups, group = block - split * g.groups, n0 = group * 32;
   const int64_t row_bytes = (int64_t)g.I * 2;
   const int second = min(n0 + 16, g.H - 1);
   f32x4_t acc[2][TM];
-  multiply<DT, R8, Q, kTail>(acc, g.h, g.I * 2, g.T * g.I * 2, {g.wd + n0 * row_bytes, g.wd + second * row_bytes}, {g.H - n0, g.H - second}, g.I, split * g.units,
-                             min((split + 1) * g.units, (g.I + kUnit - 1) / kUnit), wave, lane, mine);
+  multiply<DT, R8, Q, true>(acc, g.h, g.I * 2, g.T * g.I * 2, {g.wd + n0 * row_bytes, g.wd + second * row_bytes}, {g.H - n0, g.H - second}, g.I, split * g.units,
+                            min((split + 1) * g.units, (g.I + kUnit - 1) / kUnit), wave, lane, mine);
   publish<R8, Q>(lds, acc, wave, lane);
   for (int i = threadIdx.x; i < TM * 128; i += kFewThreads) {
     const int row = i >> 3, quad = i & 7, n = n0 + quad * 4;
-    if (row < g.T && n < g.H) *(f32x4_t*)(g.parts + ((int64_t)split * g.T + row) * g.H + n) = gathered<R8, Q>(lds, quad >> 2, row, quad & 3);
+    if (row >= g.T || n >= g.H) continue;
+    const f32x4_t v = gathered<R8, Q>(lds, quad >> 2, row, quad & 3);
+    float* out = g.parts + ((int64_t)split * g.T + row) * g.H + n;
+    if constexpr (kMerged) {
+      store_agent(out, __float_as_uint(v[0]), __float_as_uint(v[1]));
+      store_agent(out + 2, __float_as_uint(v[2]), __float_as_uint(v[3]));
+    } else {
+      *(f32x4_t*)out = v;
+    }
+  }
+  if constexpr (kMerged) {
+    stores_acknowledged();
+    uint8_t* last = lds;                                       // (the waves' sums have been read)
+    if ((int)threadIdx.x < g.T) last[threadIdx.x] = takes_last(g, (int)threadIdx.x, group);
+    __syncthreads();
+    for (int i = threadIdx.x; i < g.T * 8; i += kFewThreads) {
+      const int row = i >> 3, n = n0 + (i & 7) * 4;
+      if (n < g.H && last[row]) add_up<DT>(g, row, n, load_agent(g.experts + ((int64_t)row * g.H + n) * 2));
+    }
   }
 }
 
 struct BackArgs {
-  const uint8_t *x, *up, *down, *residual;
-  const void* gates;
-  const int32_t* ids;
+  FewExperts e;
+  const uint8_t* residual;
   const float* parts;
   uint8_t* y;
-  int T, H, k, splits;
-  uint32_t N;
+  int T, splits;
 };
 
-// Launch 3, a block per token: y = round(round(sum of the parts) + round(experts)).  NCH 1-KiB pieces of a row; G slots of a wave at once.
+// Launch 3 where it is one of its own, a block per token: y = round(round(sum of the parts) + round(experts)).  NCH 1-KiB pieces of a row; G slots of a wave at once.
 // splits 0: y holds the rounded sums already.
 // kExperts false: the MLP alone, residual (or nothing) instead of the experts.
 template <int DT, int NCH, int G, bool kExperts>
 __global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const BackArgs g) {
   extern __shared__ __align__(16) float sums[];                // [waves][NCH * 512]
-  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x, H = g.e.H;
   constexpr int kRow = NCH * 512;
   // this thread's first four columns of every part, requested before anything else
   f32x4_t part[kMostParts];
-  const int64_t plane = (int64_t)g.T * g.H;
+  const int64_t plane = (int64_t)g.T * H;
   auto request = [&](int n) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < kMostParts; ++s)
-      if (g.splits) part[s] = *(const f32x4_t*)(g.parts + min(s, g.splits - 1) * plane + (int64_t)t * g.H + min(n, g.H - 4));
+      if (g.splits) part[s] = *(const f32x4_t*)(g.parts + min(s, g.splits - 1) * plane + (int64_t)t * H + min(n, H - 4));
   };
   request(threadIdx.x * 4);
-  const int per = kExperts ? (g.k + kFewWaves - 1) / kFewWaves : 0, active = kExperts ? (g.k + per - 1) / per : 0;
-  if (kExperts && wave < active) {
-    const int64_t row_bytes = (int64_t)g.H * 2;
-    bool live[NCH];
-    u32x4_t xr[NCH];
-    float acc[NCH][8];
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      live[c] = (c * kWave + lane) * 8 < g.H;
-      xr[c] = live[c] ? *(const u32x4_t*)(g.x + t * row_bytes + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[c][i] = 0.f;
-    }
-    const int last = min((wave + 1) * per, g.k);
-    for (int j0 = wave * per; j0 < last; j0 += G) {
-      int64_t at[G];
-      float gate[G];
-      bool ok[G];
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int j = min(j0 + i, last - 1), id = g.ids[(int64_t)t * g.k + j];
-        gate[i] = Elem<DT>::load(g.gates, (int64_t)t * g.k + j);
-        ok[i] = j0 + i < last && (uint32_t)id < g.N;           // a slot of another wave, or an id outside the table, contributes nothing
-        at[i] = ok[i] ? id * row_bytes : 0;
-      }
-      u32x4_t u[G][NCH], v[G][NCH];
-#pragma unroll
-      for (int i = 0; i < G; ++i)
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-          u[i][c] = live[c] ? *(const u32x4_t*)(g.up + at[i] + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
-          v[i][c] = live[c] ? *(const u32x4_t*)(g.down + at[i] + (c * kWave + lane) * 16) : u32x4_t{0, 0, 0, 0};
-        }
-      float s[G];
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        s[i] = 0.f;
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) s[i] = dot16<DT>(xr[c], u[i][c], s[i]);
-      }
-#pragma unroll
-      for (int i = 0; i < G; ++i) s[i] = wave_sum(s[i]);
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        if (!ok[i]) continue;                                  // not even 0 * row: the stand-in row may hold Inf or NaN
-        const float coef = silu_f32(s[i]) * gate[i];
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) axpy16<DT>(coef, v[i][c], acc[c]);
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        *(f32x4_t*)(sums + wave * kRow + (c * kWave + lane) * 8 + 4 * h) = f32x4_t{acc[c][4 * h], acc[c][4 * h + 1], acc[c][4 * h + 2], acc[c][4 * h + 3]};
+  int active = 0;
+  if constexpr (kExperts) {
+    active = share_experts<DT, NCH, G>(g.e, t, wave, lane, sums, kRow);
+    __syncthreads();
   }
-  if (kExperts) __syncthreads();
-  for (int n = threadIdx.x * 4; n < g.H; n += kFewThreads * 4) {
+  for (int n = threadIdx.x * 4; n < H; n += kFewThreads * 4) {
     if (n != (int)threadIdx.x * 4) request(n);
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    float v[4] = {0.f, 0.f, 0.f, 0.f}, e[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < kMostParts; ++s)
       if (s < g.splits)
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] += part[s][q];
-    const int64_t out = ((int64_t)t * g.H + n) * 2;
+    const int64_t out = ((int64_t)t * H + n) * 2;
     if (kExperts && g.splits == 0) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] = Elem<DT>::load(g.y + out, q);
     }
     if (kExperts || g.residual) {
-      float e[4] = {0.f, 0.f, 0.f, 0.f};
       if constexpr (kExperts) {
         for (int w = 0; w < active; ++w) {
           const f32x4_t o = *(const f32x4_t*)(sums + w * kRow + n);
@@ -379,9 +491,26 @@ hipError_t start(const Args& a, int64_t blocks, hipStream_t s) {
   return hipGetLastError();
 }
 
+BackArgs back_args(const FewTokens& f, int splits) {
+  return BackArgs{FewExperts{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, f.select.gates, f.select.indices, f.H, f.select.k, (uint32_t)f.N}, (const uint8_t*)f.residual, f.parts,
+                  (uint8_t*)f.y, f.T, splits};
+}
+// f.parts: the down projection's parts [splits][T][H], and where launches 2 and 3 are one, the experts' rounded sums [T][H] | tickets [T][groups]
+struct FewParts {
+  uint8_t* experts;
+  uint32_t* tickets;
+  size_t bytes;
+  FewParts(float* parts, int64_t T, int64_t H, int64_t I) {
+    const size_t sums = (size_t)few_splits(H, I) * (size_t)T * (size_t)H * 4, rows = ((size_t)T * (size_t)H * 2 + 15) / 16 * 16;
+    experts = (uint8_t*)parts + sums;
+    tickets = (uint32_t*)(experts + rows);
+    bytes = sums + (merge_launches(T, H, I) ? rows + (size_t)T * (size_t)((H + 31) / 32) * 4 : 0);
+  }
+};
+
 template <int DT>
 hipError_t launch_back(const BackArgs& b, hipStream_t s) {
-  const int nch = (b.H + 511) / 512;
+  const int nch = (b.e.H + 511) / 512;
   if (nch <= 1) return start<few_back_kernel<DT, 1, 4, true>, kFewWaves * 1 * 2048>(b, b.T, s);
   if (nch <= 2) return start<few_back_kernel<DT, 2, 4, true>, kFewWaves * 2 * 2048>(b, b.T, s);
   if (nch <= 4) return start<few_back_kernel<DT, 4, 2, true>, kFewWaves * 4 * 2048>(b, b.T, s);
@@ -392,8 +521,10 @@ template <int DT, int R8>
 hipError_t launch(const FewTokens& f, hipStream_t s) {
   const bool layer = f.up != nullptr;
   const int r = f.select.r;
+  const bool merged = layer && merge_launches(f.T, f.H, f.I);
+  const FewParts p(f.parts, f.T, f.H, f.I);
   const FrontArgs a{(const uint8_t*)f.x, (const uint8_t*)f.wg, (const uint8_t*)f.wu, (const uint8_t*)f.wx, (const uint8_t*)f.wy, (uint8_t*)f.h, (uint8_t*)f.z,
-                    f.T, f.H, f.I, r, layer ? (r + 15) / 16 : 0};
+                    f.T, f.H, f.I, r, layer ? (r + 15) / 16 : 0, merged ? p.tickets : nullptr, merged ? f.T * ((f.H + 31) / 32) : 0};
   const int64_t front = a.router_blocks + (f.I + 15) / 16;
   // Beyond eight tokens two K units of a wave in LDS at once are more than half of a CU's: one block to a CU, and blocks beyond 256 wait for a whole round.
   // One unit at a time then (in turn over three sets of inputs, hidden 1024 x intermediate 4096, weights in registers: 33 tokens 23.5 -> 21.3 us, 48 24.1 -> 21.9, 64
@@ -409,26 +540,29 @@ hipError_t launch(const FewTokens& f, hipStream_t s) {
   if (e != hipSuccess) return e;
 
   const int units = (f.I + kUnit - 1) / kUnit;
-  MiddleArgs m{(const uint8_t*)f.h, (const uint8_t*)f.wd, f.parts, f.T, f.H, f.I, (f.H + 31) / 32, 0, layer ? (f.T + kFewWaves - 1) / kFewWaves : 0, (r + kWave - 1) / kWave, f.select};
   int splits = few_splits(f.H, f.I);
+  MiddleArgs m{};
+  m.h = (const uint8_t*)f.h; m.wd = (const uint8_t*)f.wd; m.parts = f.parts; m.T = f.T; m.H = f.H; m.I = f.I;
+  m.groups = (f.H + 31) / 32;
   m.units = (units + splits - 1) / splits;
-  splits = (units + m.units - 1) / m.units;                    // every split has work
-  const int cells = prepare_select(m.select);
+  m.splits = splits = (units + m.units - 1) / m.units;         // every split has work
+  m.tickets = p.tickets; m.experts = p.experts;
+  m.x = (const uint8_t*)f.x; m.up = (const uint8_t*)f.up; m.down = (const uint8_t*)f.down; m.y = (uint8_t*)f.y;
+  m.N = (uint32_t)f.N;
+  m.select = f.select;
+  m.select_regs = (r + kWave - 1) / kWave;
+  m.cells = layer ? prepare_select(m.select) : 0;
+  m.select_blocks = !layer ? 0 : merged ? f.T : (f.T + kFewWaves - 1) / kFewWaves;
   const int64_t middle = m.select_blocks + (int64_t)m.groups * splits;
   e = units_at_once((R8 > 1 && middle > 256) || m.units <= kFewWaves, [&](auto q) -> hipError_t {           // (a wave may have one unit only)
     constexpr int Q = decltype(q)::value, kBytes = FewStage<R8, Q>::kBytes;
-    auto go = [&](auto tail) -> hipError_t {
-      constexpr bool kTail = decltype(tail)::value;
-      if (!layer) return start<few_middle_kernel<DT, R8, Q, kTail, false, 1>, kBytes>(m, middle, s);
-      if (cells <= 1) return start<few_middle_kernel<DT, R8, Q, kTail, true, 1>, kBytes>(m, middle, s);
-      return start<few_middle_kernel<DT, R8, Q, kTail, true, 2>, kBytes>(m, middle, s);
-    };
-    return f.I % kUnit ? go(std::true_type{}) : go(std::false_type{});
+    if constexpr (R8 * 8 <= kMergedTokens) {
+      if (merged) return start<few_middle_kernel<DT, R8, Q, true>, kBytes>(m, middle, s);
+    }
+    return start<few_middle_kernel<DT, R8, Q, false>, kBytes>(m, middle, s);
   });
-  if (e != hipSuccess) return e;
-
-  const BackArgs b{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, (const uint8_t*)f.residual, f.select.gates, f.select.indices, f.parts, (uint8_t*)f.y,
-                   f.T, f.H, f.select.k, splits, (uint32_t)f.N};
+  if (e != hipSuccess || merged) return e;
+  const BackArgs b = back_args(f, splits);
   if (!layer) return start<few_back_kernel<DT, 1, 1, false>, 0>(b, f.T, s);
   return launch_back<DT>(b, s);
 }
@@ -447,7 +581,7 @@ bool few_tokens_aligned(const FewTokens& f) {
     if ((uintptr_t)q % 16) return false;
   return true;
 }
-size_t few_tokens_parts_bytes(int64_t T, int64_t H, int64_t I) { return (size_t)few_splits(H, I) * (size_t)T * (size_t)H * 4; }
+size_t few_tokens_parts_bytes(int64_t T, int64_t H, int64_t I) { return FewParts(nullptr, T, H, I).bytes; }
 
 hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s) {
   auto go = [&](auto dt) -> hipError_t {
@@ -464,8 +598,7 @@ hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s) {
 }
 
 hipError_t launch_few_back(int dtype, const FewTokens& f, int splits, hipStream_t s) {
-  const BackArgs b{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, nullptr, f.select.gates, f.select.indices, f.parts, (uint8_t*)f.y,
-                   f.T, f.H, f.select.k, splits, (uint32_t)f.N};
+  const BackArgs b = back_args(f, splits);
   if (dtype == kBF16) return launch_back<kBF16>(b, s);
   if (dtype == kF16) return launch_back<kF16>(b, s);
   return hipErrorInvalidValue;
