@@ -6,7 +6,7 @@
 // each other shares a launch, by block index:
 //   1. the router's projection | gate and up with their SwiGLU product
 //   2. the router's selection  | the down projection, K split over the grid, as fp32 partial sums
-//   3. the experts, the partial sums and the final add, one block per token; up to 16 tokens of a small layer in launch 2 (further down).
+//   3. the experts, the partial sums and the final add, one block per token; for calls that the host takes longer for in launch 2 (further down).
 // 1 token 38.4 -> 18.1 us a call, 48 tokens 42.9 -> 21.9 us, hidden 1024 x intermediate 4096; with the weights through LDS as well 17.2 -> 15.3 and 21.0 -> 20.1
 // (calls in a graph; a program sees the 18 us of host work of a call at 1 token, 15.2 with two launches).
 //
@@ -224,13 +224,20 @@ struct MiddleArgs {
   SelectArgs select;
   // merged
   uint32_t* tickets;                 // [T][groups]
-  uint8_t* experts;                  // [T][H] the experts' rounded sums
-  const uint8_t *x, *up, *down;
+  uint32_t numbers;                  // of a ticket: the splits and, in the layer, the token's block
+  uint8_t* experts;                  // the layer: [T][H] the experts' rounded sums
+  const uint8_t *x, *up, *down, *residual;   // (residual: the MLP alone, or NULL)
   uint8_t* y;
   uint32_t N;
 };
-constexpr int kMergedTokens = 16, kMergedRow = 1024;           // (a token's block has a thread for four values of a row)
-bool merge_launches(int64_t T, int64_t H, int64_t I) { return T <= kMergedTokens && H <= kMergedRow && H * I <= (1 << 23); }
+// So two launches are for calls whose kernels take less than the host: up to 16 tokens and 2^23 weights a projection (the MLP alone, whose host work is less: 2^22), up to 48
+// tokens and 2^21.  The MLP alone, three / two in a graph: 1 token 512 x 2048 7.4 / 7.4, 16 tokens 7.6 / 8.3, 1024 x 4096 11.5 / 12.7; a call as a program
+// makes it 13.2 / 10.9 at 8 tokens, 512 x 1024.
+constexpr int kMergedTokens = 48, kMergedRow = 1024;           // (a token's block has a thread for four values of a row)
+bool merge_launches(bool layer, int64_t T, int64_t H, int64_t I) {
+  if (layer && H > kMergedRow) return false;
+  return T <= 16 ? H * I <= (layer ? 1 << 23 : 1 << 22) : T <= kMergedTokens && H * I <= (1 << 21);
+}
 __device__ __forceinline__ void store_agent(void* at, uint32_t a, uint32_t b) {
   __hip_atomic_store((uint64_t*)at, (uint64_t)a | (uint64_t)b << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -238,16 +245,16 @@ __device__ __forceinline__ u32x2_t load_agent(const void* at) {
   const uint64_t v = __hip_atomic_load((const uint64_t*)at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return u32x2_t{(uint32_t)v, (uint32_t)(v >> 32)};
 }
-__device__ __forceinline__ bool takes_last(const MiddleArgs& g, int t, int group) {           // of the splits' numbers and the token's block's
-  return __hip_atomic_fetch_add(g.tickets + t * g.groups + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)g.splits;
+__device__ __forceinline__ bool takes_last(const MiddleArgs& g, int t, int group) {
+  return __hip_atomic_fetch_add(g.tickets + t * g.groups + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.numbers - 1;
 }
 __device__ __forceinline__ void stores_acknowledged() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 }
-// four columns of a token: y = round(round(sum of the parts in split order) + e)
+// four columns of a token: y = round(round(sum of the parts in split order) + e), or the rounded sum
 template <int DT>
-__device__ __forceinline__ void add_up(const MiddleArgs& g, int t, int n, const u32x2_t e) {
+__device__ __forceinline__ void add_up(const MiddleArgs& g, int t, int n, const u32x2_t e, bool add = true) {
   u32x2_t part[kMostParts][2];
 #pragma unroll
   for (int s = 0; s < kMostParts; ++s)
@@ -259,8 +266,10 @@ __device__ __forceinline__ void add_up(const MiddleArgs& g, int t, int n, const 
     if (s < g.splits)
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] += __uint_as_float(part[s][q / 2][q % 2]);
+  if (add) {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) v[q] = Elem<DT>::round(v[q]) + Elem<DT>::load(&e, q);
+    for (int q = 0; q < 4; ++q) v[q] = Elem<DT>::round(v[q]) + Elem<DT>::load(&e, q);
+  }
   *(u32x2_t*)(g.y + ((int64_t)t * g.H + n) * 2) = u32x2_t{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
 }
 
@@ -375,7 +384,7 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel
   constexpr int TM = (R8 + 1) / 2;
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   static_assert(FewStage<R8, Q>::kBytes >= (int)sizeof(PrunePool), "a block that selects prunes there");
-  static_assert(!kMerged || FewStage<R8, Q>::kBytes >= kFewWaves * kMergedRow * 4, "a token's block has its waves' sums there");
+  static_assert(FewStage<R8, Q>::kBytes >= kFewWaves * kMergedRow * 4, "a token's block has its waves' sums there");
   if ((int)blockIdx.x < g.select_blocks) {
     if constexpr (kMerged) token_block<DT>(g, (int)blockIdx.x, lds, wave, lane);
     else select_tokens<DT>(g, (int)blockIdx.x * kFewWaves + wave, g.select_blocks * kFewWaves, *(PrunePool*)lds);
@@ -408,7 +417,10 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel
     __syncthreads();
     for (int i = threadIdx.x; i < g.T * 8; i += kFewThreads) {
       const int row = i >> 3, n = n0 + (i & 7) * 4;
-      if (n < g.H && last[row]) add_up<DT>(g, row, n, load_agent(g.experts + ((int64_t)row * g.H + n) * 2));
+      if (n >= g.H || !last[row]) continue;
+      const int64_t at = ((int64_t)row * g.H + n) * 2;
+      if (g.experts) add_up<DT>(g, row, n, load_agent(g.experts + at));
+      else add_up<DT>(g, row, n, g.residual ? *(const u32x2_t*)(g.residual + at) : u32x2_t{0, 0}, g.residual != nullptr);
     }
   }
 }
@@ -504,7 +516,7 @@ struct FewParts {
     const size_t sums = (size_t)few_splits(H, I) * (size_t)T * (size_t)H * 4, rows = ((size_t)T * (size_t)H * 2 + 15) / 16 * 16;
     experts = (uint8_t*)parts + sums;
     tickets = (uint32_t*)(experts + rows);
-    bytes = sums + (merge_launches(T, H, I) ? rows + (size_t)T * (size_t)((H + 31) / 32) * 4 : 0);
+    bytes = sums + (merge_launches(true, T, H, I) || merge_launches(false, T, H, I) ? rows + (size_t)T * (size_t)((H + 31) / 32) * 4 : 0);
   }
 };
 
@@ -521,7 +533,7 @@ template <int DT, int R8>
 hipError_t launch(const FewTokens& f, hipStream_t s) {
   const bool layer = f.up != nullptr;
   const int r = f.select.r;
-  const bool merged = layer && merge_launches(f.T, f.H, f.I);
+  const bool merged = merge_launches(layer, f.T, f.H, f.I);
   const FewParts p(f.parts, f.T, f.H, f.I);
   const FrontArgs a{(const uint8_t*)f.x, (const uint8_t*)f.wg, (const uint8_t*)f.wu, (const uint8_t*)f.wx, (const uint8_t*)f.wy, (uint8_t*)f.h, (uint8_t*)f.z,
                     f.T, f.H, f.I, r, layer ? (r + 15) / 16 : 0, merged ? p.tickets : nullptr, merged ? f.T * ((f.H + 31) / 32) : 0};
@@ -546,7 +558,7 @@ hipError_t launch(const FewTokens& f, hipStream_t s) {
   m.groups = (f.H + 31) / 32;
   m.units = (units + splits - 1) / splits;
   m.splits = splits = (units + m.units - 1) / m.units;         // every split has work
-  m.tickets = p.tickets; m.experts = p.experts;
+  m.tickets = p.tickets; m.numbers = (uint32_t)(layer ? splits + 1 : splits); m.experts = layer ? p.experts : nullptr; m.residual = (const uint8_t*)f.residual;
   m.x = (const uint8_t*)f.x; m.up = (const uint8_t*)f.up; m.down = (const uint8_t*)f.down; m.y = (uint8_t*)f.y;
   m.N = (uint32_t)f.N;
   m.select = f.select;

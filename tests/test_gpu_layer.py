@@ -29,57 +29,6 @@ def _elsewhere(t, device):
     return out
 
 
-# T, H, I, N, k: whole lines of the weights: eight tokens (a half tile of activations) and nine, 16 and 32 and one more; waves without a unit of K (hidden below 512,
-# intermediate below 512), a second column tile of the down projection with 8 columns or none (hidden 520, 528), one and two units of K at a time in either launch
-FEW_TOKEN_LINES = [(8, 1024, 4096, 4096, 16), (9, 528, 4104, 1000, 8), (7, 520, 72, 64, 2), (24, 264, 264, 1024, 8), (32, 1032, 4104, 4096, 16), (10, 2048, 2056, 260, 4),
-                   (28, 1288, 520, 17000, 6), (40, 72, 8200, 900, 4)]
-
-
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("case", FEW_TOKEN_LINES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
-def test_few_tokens_weights_by_lines(case, dtype, device):
-    test_few_tokens_match_the_operators(case, dtype, device)
-
-
-# T, H, I, N, k: two launches up to 16 tokens, hidden 1024 and 2^23 weights a projection, and one past each of the three; one column group and the last of several short;
-# fewer pairs than waves, more than two to a wave; one split of K
-MERGED_LAUNCH_CASES = [(1, 1024, 4096, 4096, 16), (16, 1024, 8192, 4096, 32), (16, 1024, 8200, 4096, 16), (17, 1024, 4096, 4096, 16), (16, 1032, 4096, 4096, 16), (5, 8, 64, 64, 2),
-                       (9, 520, 2056, 90000, 18), (3, 1016, 72, 260, 4)]
-
-
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("case", MERGED_LAUNCH_CASES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
-def test_few_tokens_in_two_launches(case, dtype, device):
-    """Against the operators; then call after call on changing inputs in the same memory, and replays of a graph with eager calls between them: every result has the bits of its
-    input's first one, whoever of a token's blocks came last."""
-    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
-    test_few_tokens_match_the_operators(case, dtype, device)
-    T, H, I, N, k = case
-    layer = OmniMoE(OmniMoEConfig(H, I, "silu", N, k)).to(device=device, dtype=dtype).eval()
-    g = torch.Generator(device=device).manual_seed(T + H)
-    with torch.no_grad():
-        for p in layer.parameters():
-            p.normal_(0.0, H ** -0.5, generator=g)
-        xs = [torch.randn(1, T, H, device=device, generator=g).to(dtype) for _ in range(4)]
-        first = [layer(x).clone() for x in xs]
-        for _ in range(20):
-            again = [layer(x) for x in xs]
-            assert all(torch.equal(a, b) for a, b in zip(first, again))
-        held, stream = xs[0].clone(), torch.cuda.Stream()
-        stream.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(stream):
-            layer(held)
-        torch.cuda.current_stream().wait_stream(stream)
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            y = layer(held)
-        for i in range(8):
-            held.copy_(xs[i % 4])
-            graph.replay()
-            assert torch.equal(y, first[i % 4])
-            assert torch.equal(layer(xs[(i + 1) % 4]), first[(i + 1) % 4])
-
-
 # the first four are the reference's benchmark grid (tests/test_mlp.py:144-150): intermediate 1024 .. 65536
 MLP_CASES = [(1024, 1024, 1024), (1024, 1024, 4096), (1024, 1024, 16384), (1024, 1024, 65536), (4096, 1024, 4096), (4100, 1024, 4096),
              (333, 256, 1000), (128, 64, 128), (512, 2048, 8192), (5, 8, 8),
@@ -896,6 +845,62 @@ def test_few_tokens_match_the_operators(case, dtype, device):
     # ids and gates are those of the router operator: the expert term alone (a zero down projection)
     layer.down_proj.weight.zero_()
     assert (layer(x)[0].double() - experts).abs().max().item() <= 4 * eps * max(1.0, float(experts.abs().max()))
+
+
+# T, H, I, N, k: whole lines of the weights: eight tokens (a half tile of activations) and nine, 16 and 32 and one more; waves without a unit of K (hidden below 512,
+# intermediate below 512), a second column tile of the down projection with 8 columns or none (hidden 520, 528), one and two units of K at a time in either launch
+FEW_TOKEN_LINES = [(8, 1024, 4096, 4096, 16), (9, 528, 4104, 1000, 8), (7, 520, 72, 64, 2), (24, 264, 264, 1024, 8), (32, 1032, 4104, 4096, 16), (10, 2048, 2056, 260, 4),
+                   (28, 1288, 520, 17000, 6), (40, 72, 8200, 900, 4)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", FEW_TOKEN_LINES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
+def test_few_tokens_weights_by_lines(case, dtype, device):
+    test_few_tokens_match_the_operators(case, dtype, device)
+
+
+# T, H, I, N, k: two launches up to 16 tokens, hidden 1024 and 2^23 weights a projection (the MLP alone any hidden and 2^22), and one past each of the three; up to 48 tokens and
+# 2^21, and one past either; one column group and the last of several short; fewer pairs than waves, more than two to a wave; one split of K
+MERGED_LAUNCH_CASES = [(1, 1024, 4096, 4096, 16), (16, 1024, 8192, 4096, 32), (16, 1024, 8200, 4096, 16), (17, 1024, 4096, 4096, 16), (16, 1032, 4096, 4096, 16), (5, 8, 64, 64, 2),
+                       (9, 520, 2056, 90000, 18), (3, 1016, 72, 260, 4), (48, 512, 4096, 1024, 8), (49, 512, 4096, 1024, 8), (48, 520, 4096, 1024, 8), (33, 1024, 2048, 4096, 16),
+                       (20, 264, 520, 1000, 32), (16, 2048, 2048, 1024, 8)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", MERGED_LAUNCH_CASES, ids=lambda c: f"T{c[0]}-H{c[1]}-I{c[2]}-N{c[3]}-k{c[4]}")
+def test_few_tokens_in_two_launches(case, dtype, device):
+    """Against the operators; then call after call on changing inputs in the same memory, and replays of a graph with eager calls between them: every result has the bits of its
+    input's first one, whoever of a token's blocks came last."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    test_few_tokens_match_the_operators(case, dtype, device)
+    T, H, I, N, k = case
+    layer = OmniMoE(OmniMoEConfig(H, I, "silu", N, k)).to(device=device, dtype=dtype).eval()
+    g = torch.Generator(device=device).manual_seed(T + H)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, H ** -0.5, generator=g)
+        xs = [torch.randn(1, T, H, device=device, generator=g).to(dtype) for _ in range(4)]
+        first = [layer(x).clone() for x in xs]
+        mlp = [layer.gate_proj.weight, layer.up_proj.weight, layer.down_proj.weight]
+        alone = [_ops().hip_omni_mlp_func(x[0], *mlp, residual=xs[0][0]).clone() for x in xs]
+        for _ in range(20):
+            again = [layer(x) for x in xs]
+            assert all(torch.equal(a, b) for a, b in zip(first, again))
+            again = [_ops().hip_omni_mlp_func(x[0], *mlp, residual=xs[0][0]) for x in xs]
+            assert all(torch.equal(a, b) for a, b in zip(alone, again))
+        held, stream = xs[0].clone(), torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            layer(held)
+        torch.cuda.current_stream().wait_stream(stream)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = layer(held)
+        for i in range(8):
+            held.copy_(xs[i % 4])
+            graph.replay()
+            assert torch.equal(y, first[i % 4])
+            assert torch.equal(layer(xs[(i + 1) % 4]), first[(i + 1) % 4])
 
 
 # T, H, I: 32-row and 32-column tiles and their remainders, K of one to five tiles of 32 and with a remainder, more and fewer waves than K tiles
