@@ -6,6 +6,8 @@ namespace omni {
 // (joint: those that share their launch with the layer's router)
 constexpr unsigned kForwardShapes = shapes_of(kNT), kJointShapes = 1u << 1 | 1u << 2 | 1u << 3 | 1u << 4 | 1u << 7 | 1u << 8;
 
+constexpr float kJoinedSumUs = 1.8f;
+
 // Microseconds that a launch of n blocks of one shape takes for 64 of K.  Where two blocks share a CU, the CUs with two set the time however few they are
 // (gate/up of 613 x 1024 x 4096 on 128 x 128 tiles, 320 blocks: 19.7 us; 450 rows, 256 blocks: 16.4; 1000 rows, 512 blocks: 21.4).
 static float step_us(const ShapeCost& c, int64_t n) {
@@ -16,7 +18,11 @@ static float step_us(const ShapeCost& c, int64_t n) {
 }
 // The fastest shape and K split by those figures.  K is split for a product on its own only, where every part keeps 256 of K, and the 64 x 64
 // shape (whose two groups also split K) is for K >= 512: shorter sums stay in one order whatever the shape.
-static TileChoice choose_of(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes) {
+// joined: the layer's down projection, whose parts the experts' kernel adds up if they are of a shape that the selection runs beside.  A split costs that kernel's
+// longer wait then instead of a launch (kJoinedSumUs).  Over 36 layers where the figure decides (66 to 2475 tokens, hidden 256 to 1536) the call takes, with a launch's 3.3 us / with 1.8:
+// 197 x 512 x 1536 19.0 / 16.7 us, 221 x 1024 x 2048 23.5 / 21.1, 251 x 1536 x 3072 30.5 / 27.3, 613 x 1024 x 4096 41.2 / 38.8, 2475 x 512 x 2048 44.1 / 41.7, 85 x 256 x 1024
+// 16.5 / 15.2; one loses, 714 x 1280 x 5120 51.2 / 51.6.  With 1.0 or nothing 800 x 768 x 3072 leaves the selection no place, 31.5 / 35.1, and 277 x 256 x 1024 18.8 / 19.5.
+static TileChoice choose_of(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes, bool joined) {
   TileChoice best;
   for (int i = 0; i < kShapes; ++i) {
     if (!(shapes >> i & 1)) continue;
@@ -26,10 +32,11 @@ static TileChoice choose_of(int epilogue, const TileSize* sizes, int count, int6
     int64_t tiles = 0;
     for (int q = 0; q < count; ++q) tiles += ((sizes[q].M + c.bm - 1) / c.bm) * ((sizes[q].N + bn - 1) / bn);
     const int64_t kt = (K + 63) / 64;
-    for (int s = 1; s <= (may_split && count == 1 ? kMostSplits : 1); ++s) {
+    const float sum_us = joined && (kJointShapes >> i & 1) ? kJoinedSumUs : kReduceUs;
+    for (int s = 1; s <= (!may_split || count != 1 ? 1 : joined ? kMostDownParts : kMostSplits); ++s) {
       if (s > 1 && kt / s < 4) break;
       float us = c.fixed + (float)((kt + s - 1) / s) * step_us(c, tiles * s);
-      if (s > 1) us += kReduceUs + (float)s * (float)sizes[0].M * (float)(epilogue == kTileSwiglu ? 2 * sizes[0].N : sizes[0].N) * 4.f * (1.f / kPartsOut + 1.f / kPartsIn);
+      if (s > 1) us += sum_us + (float)s * (float)sizes[0].M * (float)(epilogue == kTileSwiglu ? 2 * sizes[0].N : sizes[0].N) * 4.f * (1.f / kPartsOut + 1.f / kPartsIn);
       if (us < best.us) best = TileChoice{i, s, us};
     }
   }
@@ -37,25 +44,26 @@ static TileChoice choose_of(int epilogue, const TileSize* sizes, int count, int6
 }
 // A call asks for its workspace and then for its launches, a program for the same sizes over and over, and a choice takes 0.6 us: a layer of one token,
 // bound by the host, asked eight times.  Each thread keeps the last few products' choices, which nothing but the sizes goes into.
-static TileChoice choose_tiles(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes = kForwardShapes) {
-  if (count != 1) return choose_of(epilogue, sizes, count, K, may_split, shapes);
+static TileChoice choose_tiles(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes = kForwardShapes, bool joined = false) {
+  if (count != 1) return choose_of(epilogue, sizes, count, K, may_split, shapes, joined);
   struct Kept { int64_t M, N, K; uint64_t how; TileChoice choice; };
   constexpr int kKept = 16;
   static thread_local Kept kept[kKept];                        // (M = 0: none)
   static thread_local int oldest = 0;
-  const uint64_t how = (uint64_t)shapes << 8 | (uint64_t)epilogue << 1 | (may_split ? 1 : 0);
+  const uint64_t how = (uint64_t)shapes << 8 | (uint64_t)joined << 7 | (uint64_t)epilogue << 1 | (may_split ? 1 : 0);
   for (const Kept& k : kept)
     if (k.M == sizes->M && k.N == sizes->N && k.K == K && k.how == how) return k.choice;
   Kept& k = kept[oldest];
   oldest = (oldest + 1) % kKept;
-  k = Kept{sizes->M, sizes->N, K, how, choose_of(epilogue, sizes, count, K, may_split, shapes)};
+  k = Kept{sizes->M, sizes->N, K, how, choose_of(epilogue, sizes, count, K, may_split, shapes, joined)};
   return k.choice;
 }
 
 // The layer's down projection: a shape that takes the selection beside it, unless another one gains more than the selection's own launch costs
 static TileChoice choose_down(const TileSize& size, int64_t K, bool may_split) {
   constexpr float kSelectUs = 6.f;
-  const TileChoice any = choose_tiles(kTilePlain, &size, 1, K, may_split), joint = choose_tiles(kTilePlain, &size, 1, K, may_split, kJointShapes);
+  const TileChoice any = choose_tiles(kTilePlain, &size, 1, K, may_split, kForwardShapes, true),
+                   joint = choose_tiles(kTilePlain, &size, 1, K, may_split, kJointShapes, true);
   return joint.us <= any.us + kSelectUs ? joint : any;
 }
 // The shape that both products' tiles take least time in, by the figures above, if that is less than a launch for each; -1: it is not
@@ -127,7 +135,6 @@ hipError_t launch_tile_down(int dtype, const TileProduct& p, const SelectArgs& s
   const TileSize size{p.M, p.N};
   TileChoice c = choose_down(size, p.seg[0].K, ws != nullptr);
   if (parts_bytes(c, p.M, p.N) > ws_bytes) c = choose_down(size, p.seg[0].K, false);
-  if (c.splits > kMostDownParts) c.splits = kMostDownParts;
   return dtype == kBF16 ? tile_down_of<kBF16>(p, select, c, (float*)ws, s, selected, parts) : tile_down_of<kF16>(p, select, c, (float*)ws, s, selected, parts);
 }
 }  // namespace omni
@@ -142,9 +149,9 @@ extern "C" OMNI_API int32_t omni_probe_joint_tiles(int64_t num_tokens, int32_t h
   const TileChoice c = choose_down(TileSize{num_tokens, hidden_size}, intermediate_size, true);
   SelectArgs select{};
   select.r = num_expert_sqrt; select.k = num_experts_per_token;
-  const int cells = prepare_select(select), regs = (num_expert_sqrt + kWave - 1) / kWave, splits = c.splits < kMostDownParts ? c.splits : kMostDownParts;
-  auto plan = [&](auto id) { return plan_down<decltype(id)::value>(num_tokens, hidden_size, intermediate_size, splits, (int)num_tokens, regs, cells); };
-  DownPlan p{0, splits, 0, 0, false};                          // (the other shapes: nothing beside them)
+  const int cells = prepare_select(select), regs = (num_expert_sqrt + kWave - 1) / kWave;
+  auto plan = [&](auto id) { return plan_down<decltype(id)::value>(num_tokens, hidden_size, intermediate_size, c.splits, (int)num_tokens, regs, cells); };
+  DownPlan p{0, c.splits, 0, 0, false};                          // (the other shapes: nothing beside them)
   if (c.shape == 1) p = plan(std::integral_constant<int, 1>{});
   else if (c.shape == 2) p = plan(std::integral_constant<int, 2>{});
   else if (c.shape == 3) p = plan(std::integral_constant<int, 3>{});

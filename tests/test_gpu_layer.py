@@ -1010,6 +1010,14 @@ def test_joint_launches_select_beside_every_tile(case, tiles, dtype, device):
     test_joint_launches_match_the_operators(case, dtype, device)
 
 
+# down projections in parts because the experts' kernel adds them up: few row tiles, a short one at the end, K in whole steps of a split and not, the most parts and two
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case, tiles", [((613, 1024, 4096, 4096, 16), (96, 128, 3)), ((197, 512, 1536, 576, 4), (64, 64, 6)), ((221, 1024, 2048, 6400, 8), (64, 64, 3)),
+                                         ((207, 1536, 3072, 7744, 16), (64, 64, 2)), ((85, 256, 1024, 3136, 8), (64, 64, 4))], ids=lambda c: "x".join(map(str, c)))
+def test_joint_launches_down_in_parts(case, tiles, dtype, device):
+    test_joint_launches_select_beside_every_tile(case, tiles, dtype, device)
+
+
 
 def test_layer_with_rows_beyond_the_tile_kernels_reach(device):
     """An intermediate size whose rows put 256 of them beyond 2 GiB: no joint launch, and the result of the operators one by one (MLP in 64 bits)."""
