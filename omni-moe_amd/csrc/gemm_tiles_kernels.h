@@ -146,8 +146,9 @@ struct TileRing {
 //
 // kStream (one product, one segment, unsplit): the grid may be smaller than the number of output tiles; a block walks its share, and the ring
 // steps of consecutive output tiles form ONE stream through the stages: the next tile's first loads fly while the current one finishes, so
-// only a block's first tile waits for memory before its first matrix instruction.  The epilogue's stores are younger than every load of the next tile's first
-// two ring steps and may stay in flight past its first wait (memory instructions are counted in issue order).
+// only a block's first tile waits for memory before its first matrix instruction.  A tile's first wait is for the last one's stores too, which have had half a K tile:
+// to let them fly took a branch into the loop, which cost every K tile what this costs one (MI355X, kernels alone, 20 ms of calls: gate/up of 32768 x 2 8192 x 2048
+// 1559 -> 1544 us, of 4474 x 2 4096 x 1024 74.7 -> 73.5; down of 32768 x 2048 x 8192 777 -> 756, of 20000 x 1024 x 2048 92.8 -> 89.6).
 // (block, blocks): the place in the launch, or in its own part of one that it shares
 template <int DT, int LAY, int WM, int WN, int KG, int TM, int TN, int NS, int EPI, bool kTail, bool kStream, class Group>
 __device__ __forceinline__ void tiles_block(const Group& g, const int block, const int blocks) {
@@ -390,12 +391,6 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
   };
 
   f32x4_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc[i][j][q] = 0.f;
 
   // ---- K loop.  Step 0 of a K tile reads the fragments of its step 1 and requests one operand of the ring step NS ahead; then, after the first matrix row of
   // step 1, every wave waits for its own reads and loads and meets the block: the stage is free, the next one is there; step 1 reads the next stage's first
@@ -421,8 +416,6 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
 #pragma unroll
   for (int n = 0; n < TN * RB; ++n) read_b(0, n);
   int a_stage = 0, b_stage = 0;                                // those being multiplied
-  constexpr int kEpiStores = TM * (EPI == kTileSwiglu ? TN / 4 : TN / 2);     // store instructions of a wave's epilogue
-  int young = 0;                                               // that many are younger than the loads that the next wait is for
   // Column tiles back and forth, so that one operand of a matrix instruction is always the one before's: under the power limit less that changes is time
   // (gate/up of 32768 x 2 8192 x 2048 1591 -> 1583 us, down of 32768 x 2048 x 8192 787 -> 784, gate/up of 4096 x 2 4096 x 1024 55.6 -> 55.1; five runs of each in turn)
   auto column = [](int s) constexpr { return s / TN % 2 ? TN - 1 - s % TN : s % TN; };
@@ -447,8 +440,7 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
     if constexpr (s == TN - 1) {
       lds_reads_done();
       constexpr int kYounger = (NS - 2) * LPT + kLead;
-      if (kStream && young) vmcnt<kYounger + kEpiStores>();
-      else vmcnt<kYounger>();
+      vmcnt<kYounger>();
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -468,8 +460,17 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
   for (int tile = block - p.first; tile < all; tile += blocks) {
   int m0, n0;
   coords(tile, m0, n0);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[i][j][q] = 0.f;
   for (int left = tiles; left > 0;) {
     const int run = min(left, f_until);
+    // Nothing of the last tile's epilogue and of next_run() is on its way to a register in here, or the compiler makes every K tile's second matrix instruction
+    // wait for all reads before it
+    if constexpr (kStream) __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
 #pragma clang loop unroll(disable)
     for (int i = run; i > 0; --i) {
       with_sequence(all0, std::make_integer_sequence<int, TM * TN>{});
@@ -482,7 +483,6 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
 #pragma unroll
       for (int j = 0; j < (BC ? TN : 2); ++j) b_addr[j] += b_move;
       with_sequence(all1, std::make_integer_sequence<int, TM * TN>{});
-      if constexpr (kStream) young = 0;
     }
     left -= run;
     f_until -= run;
@@ -625,14 +625,6 @@ __device__ __forceinline__ void tiles_block(const Group& g, const int block, con
     }
   }
   if constexpr (!kStream) return;
-  // every row and column of the wave inside the matrix: each store instruction of the epilogue has been issued
-  young = M - m0 >= BM && N - n0 >= BNO && !(EPI == kTileSwiglu && p.c2);
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc[i][j][q] = 0.f;
   }
   vmcnt<0>();
 }
