@@ -219,6 +219,10 @@ OMNI_API int32_t omni_probe_mfma16(const void* operands, float* sink, int32_t nu
  * parts of its K, and 1 if the selection runs beside them. */
 OMNI_API int32_t omni_probe_joint_tiles(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t num_expert_sqrt,
                                         int32_t num_experts_per_token, int32_t* pair, int32_t* down);
+/* Diagnostic: what a 16-bit product by itself takes in the tile GEMM, from its sizes alone (nothing is launched).  layout 0: x W^T, 1: dy W, 2: dy^T x; epilogue 0: rounded
+ * sums, 1: with a residual, 2: gate and up with SwiGLU (columns: of each), 3: the SwiGLU backward.  choice[4]: rows and columns of a tile, groups of waves that share
+ * its K, parts of K. */
+OMNI_API int32_t omni_probe_tile_choice(int32_t layout, int32_t epilogue, int64_t rows, int64_t columns, int64_t k, int32_t* choice);
 
 /* y[i] = round(y[i] + addend[i]) in place: the layer's final  mlp + experts  (omni_moe.py:102) as a
  * call of its own, for callers that run the two branches on different streams.  num_elements a

@@ -166,3 +166,15 @@ extern "C" OMNI_API int32_t omni_probe_joint_tiles(int64_t num_tokens, int32_t h
   down[3] = p.selected ? 1 : 0;
   return OMNI_OK;
 }
+extern "C" OMNI_API int32_t omni_probe_tile_choice(int32_t layout, int32_t epilogue, int64_t rows, int64_t columns, int64_t k, int32_t* choice) {
+  using namespace omni;
+  if (layout < kNT || layout > kTN || epilogue < kTilePlain || epilogue > kTileSwigluBwd || rows <= 0 || columns <= 0 || k <= 0) return OMNI_ERR_SHAPE;
+  if (!choice) return OMNI_ERR_NULL;
+  const TileSize size{rows, columns};
+  const TileChoice c = choose_tiles(epilogue, &size, 1, k, layout != kTN, shapes_of(layout));
+  choice[0] = kCost[c.shape].bm;
+  choice[1] = kCost[c.shape].bn;
+  choice[2] = kCost[c.shape].kg;
+  choice[3] = c.splits;
+  return OMNI_OK;
+}

@@ -12,9 +12,9 @@
 // PFLOP/s with a block to a tile, 58 % and 1.23 streamed; d(h) with the SwiGLU backward as epilogue 57 us, 0.60 PFLOP/s, half of them its 134 MB).  The
 // 128 x 128 tile: the path from L2 into LDS, which carries 64 bytes per cycle and CU -- what that tile asks for at full matrix rate --
 // and, with one block to a CU, the chain of reads and waits between two barriers.  So a block's waves keep 64 x 64 of the tile each (LDS
-// serves 256 bytes a cycle, and smaller wave tiles read more per product) and, alone on its CU, a block has four ring stages in flight (two groups of four
-// waves with two stages each instead: 4096 x 1024 x 4096 36.4 -> 39.2 us, x 8192 75 -> 94); the 64 x 64 tile has two groups of waves
-// that take every other K tile and add up at the end: one barrier for two K tiles and a second wave to issue while the first waits.
+// serves 256 bytes a cycle, and smaller wave tiles read more per product) and, alone on its CU, a block has three ring stages in flight (TileRing); the 64 x 64 tile
+// has two groups of waves that take every other K tile and add up at the end: one barrier for two K tiles and a second wave to issue while the first waits
+// (and the 128 x 128 tile for the gradients' long sums: Shape<9>).
 // Splitting K over the grid costs a pass over fp32 partial sums (summed in split order: results do not depend on timing).
 #pragma once
 #include "common.h"
@@ -128,14 +128,23 @@ constexpr int staged_rows(int rows, int waves) {
   return up;
 }
 
-// Stages of the two operands in LDS: NS, and one more for the left operand, or for the right one where the left one's does not fit.  The one with a stage
-// more is requested in step 0 of a K tile, half a tile before the barrier that frees the other's: requests are spread over the whole tile, and of two stages the
-// second one's loads have between a half and a whole tile to arrive.  Two stages against two and three, kernels alone: down of 32768 x 2048 x 8192 827 -> 793 us,
-// the three weight gradients of 4096 x 1024 x 4096 95.6 -> 93.2 on 256 rows and 102 -> 94.8 on 224, the SwiGLU backward 58.7 -> 57.3.
+// Stages of the two operands in LDS: NS, and one more for one of them.  That one is requested in step 0 of a K tile, half a tile before the barrier that frees the
+// other's: requests are spread over the whole tile, and of two stages the second one's loads have between a half and a whole tile to arrive.  It is the right operand,
+// in a forward pass the weights, which come from further away, or the left one where a tile has more rows of it, or where the right one's does not fit.
+// Two stages against two and three, kernels alone: down of 32768 x 2048 x 8192 827 -> 793 us, the three weight gradients of 4096 x 1024 x 4096 95.6 -> 93.2 on 256 rows
+// and 102 -> 94.8 on 224, the SwiGLU backward 58.7 -> 57.3.
+// NS is no more than hides memory, for a block requests NS ring steps before its first matrix instruction, at some 20 cycles a load instruction and CU: a stage
+// costs every block 0.1 to 0.3 us.  Equal rings of NS + 1 / NS + 1 and one more for the left operand / as it is, us, weights in the caches, and from memory:
+//   64 x 64     65 x 1024 x 512   4.62 / 4.82 / 4.55   4.80 / 4.92 / 4.79     256 x 2048 x 4096   12.6 / 11.5 / 11.3   20.0 / 20.6 / 19.6
+//   96 x 128    512 x 1024 x 512  6.16 / 6.20 / 6.00   6.11 / 6.33 / 6.02     3000 x 1024 x 4096  28.8 / 27.4 / 26.9   29.6 / 29.1 / 29.1
+//   128 x 128   512 x 1024 x 512  6.91 / 6.93 / 6.77   6.93 / 7.08 / 6.79     4096 x 1024 x 4096  34.5 / 33.3 / 33.0   37.1 / 37.2 / 36.4
+//   256 x 128   2048 x 4096 x 512 12.2 / 12.3 / 11.4   13.3 / 13.5 / 13.0     2048 x 4096 x 1024  18.7 / 18.8 / 18.1   19.8 / 19.7 / 19.3
+//   64 x 128, gate and up   65 x 2 2048 x 512  5.84 / 6.08 / 5.60   7.30 / 7.43 / 7.25     128 x 2 4096 x 1024  7.51 / 7.63 / 6.98   11.2 / 11.3 / 10.9
+// (192 x 128 keeps three: with two 3000 x 2048 x 3072 from memory takes 36.8 -> 40.4.)
 constexpr int kCuLds = 160 * 1024;
 template <int LM, int BN, int KG, int NS>
 struct TileRing {
-  static constexpr bool kLeadA = KG * 128 * (LM * (NS + 1) + BN * NS) <= kCuLds;
+  static constexpr bool kLeadA = LM > 128 ? KG * 128 * (LM * (NS + 1) + BN * NS) <= kCuLds : KG * 128 * (LM * NS + BN * (NS + 1)) > kCuLds;
   static constexpr int kAStages = NS + (kLeadA ? 1 : 0), kBStages = NS + (kLeadA ? 0 : 1);
   static constexpr int kAStage = KG * LM * 128, kBStage = KG * BN * 128, kBFirst = kAStages * kAStage, kBytes = kBFirst + kBStages * kBStage;
   static_assert(kBytes <= kCuLds, "a block's ring fits its CU");
@@ -703,16 +712,20 @@ __global__ __launch_bounds__(256) void tile_reduce_kernel(const TileProduct p) {
 // The tile shapes: waves (rows x columns x K groups), matrix tiles per wave, ring stages.
 template <int kId, bool kSwiglu = false> struct Shape;
 template <bool kSwiglu> struct Shape<0, kSwiglu> { enum { WM = 2, WN = 4, KG = 1, TM = 8, TN = 4, NS = 2 }; };      // 256 x 256, one block to a CU
-template <bool kSwiglu> struct Shape<1, kSwiglu> { enum { WM = 4, WN = 2, KG = 1, TM = 4, TN = 4, NS = 3 }; };      // 256 x 128, one block to a CU
+template <bool kSwiglu> struct Shape<1, kSwiglu> { enum { WM = 4, WN = 2, KG = 1, TM = 4, TN = 4, NS = 2 }; };      // 256 x 128, one block to a CU
 template <bool kSwiglu> struct Shape<2, kSwiglu> { enum { WM = 2, WN = 2, KG = 1, TM = 4, TN = 4, NS = 2 }; };      // 128 x 128, two blocks to a CU
-template <bool kSwiglu> struct Shape<3, kSwiglu> { enum { WM = 2, WN = 2, KG = 1, TM = 4, TN = 4, NS = 4 }; };      // 128 x 128, one block to a CU
-template <> struct Shape<4, false> { enum { WM = 2, WN = 2, KG = 2, TM = 2, TN = 2, NS = 4 }; };                    // 64 x 64, two K groups, one block to a CU
-template <> struct Shape<4, true> { enum { WM = 2, WN = 2, KG = 2, TM = 2, TN = 4, NS = 3 }; };                     // (SwiGLU: 64 x 128, so that a wave holds two column tiles of gate)
+template <bool kSwiglu> struct Shape<3, kSwiglu> { enum { WM = 2, WN = 2, KG = 1, TM = 4, TN = 4, NS = 3 }; };      // 128 x 128, one block to a CU
+template <> struct Shape<4, false> { enum { WM = 2, WN = 2, KG = 2, TM = 2, TN = 2, NS = 3 }; };                    // 64 x 64, two K groups, one block to a CU
+template <> struct Shape<4, true> { enum { WM = 2, WN = 2, KG = 2, TM = 2, TN = 4, NS = 2 }; };                     // (SwiGLU: 64 x 128, so that a wave holds two column tiles of gate)
+template <> struct Shape<10, true> { enum { WM = 2, WN = 2, KG = 2, TM = 2, TN = 4, NS = 3 }; };                    // ... the same for K beyond kShortSum
+// Longer sums of few rows wait for memory.  With two stages / three, weights from memory: 128 x 2 5120 x 1280 14.3 / 14.6 us, 90 x 2 6144 x 1536 14.9 / 14.9, 100 x 2 4096 x 2048
+// 17.3 / 16.9, 100 x 2 8192 x 4096 33.1 / 32.1.
+constexpr int kShortSum = 1536;
 // Lower tiles, for row counts that leave the last round of the ones above half empty
 template <bool kSwiglu> struct Shape<5, kSwiglu> { enum { WM = 2, WN = 4, KG = 1, TM = 7, TN = 4, NS = 2 }; };      // 224 x 256, one block to a CU
 template <bool kSwiglu> struct Shape<6, kSwiglu> { enum { WM = 2, WN = 4, KG = 1, TM = 6, TN = 4, NS = 2 }; };      // 192 x 256, one block to a CU
 template <bool kSwiglu> struct Shape<7, kSwiglu> { enum { WM = 4, WN = 2, KG = 1, TM = 3, TN = 4, NS = 3 }; };      // 192 x 128, one block to a CU
-template <bool kSwiglu> struct Shape<8, kSwiglu> { enum { WM = 2, WN = 2, KG = 1, TM = 3, TN = 4, NS = 4 }; };      // 96 x 128, one block to a CU
+template <bool kSwiglu> struct Shape<8, kSwiglu> { enum { WM = 2, WN = 2, KG = 1, TM = 3, TN = 4, NS = 3 }; };      // 96 x 128, one block to a CU
 // For long sums of the gradients: a second wave to a SIMD multiplies while the first one's loads are issued, for an exchange of sums at the end.  dy W on 256 tiles,
 // K = 8192: 66.2 us against 71.8; 4096: 33.6 against 32.5.  (Not for x W^T: beside the down projection's eight waves the experts' passes find no room, layer of
 // 4096 tokens on two streams 119.1 -> 121.7 us, and one stream adds up in the order of two.)
@@ -758,10 +771,10 @@ static hipError_t start_tiles(const Group& g, int64_t blocks, hipStream_t s) {
 // Up to a few thousand tokens the router's projection and its selection are 6-8 us launches that leave most of the chip idle, and everything waits for
 // them.  The projection's tiles go in front of the gate/up projection's (same tile shape), the selection beside the down projection's.
 struct TilePair { TileSingle router, mlp; };
-template <int DT, int kId, bool kTail>
+template <int DT, int kId, int kMlp, bool kTail>
 __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64, 2) void tile_pair_kernel(const TilePair g) {
   using R = Shape<kId>;
-  using S = Shape<kId, true>;
+  using S = Shape<kMlp, true>;
   if ((int)blockIdx.x < g.mlp.p[0].first)
     tiles_block<DT, kNT, R::WM, R::WN, R::KG, R::TM, R::TN, R::NS, kTileTwo, kTail, false, TileSingle>(g.router, (int)blockIdx.x, (int)gridDim.x);
   else
@@ -817,19 +830,19 @@ static int64_t tile_count(const TileProduct& p) {
   constexpr int BM = S::WM * S::TM * 16, BN = S::WN * S::TN * 16 / (kSwiglu ? 2 : 1);
   return (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
 }
-template <int DT, int kId>
+template <int DT, int kId, int kMlp = kId>
 static bool start_pair(TilePair& g, hipStream_t s, hipError_t* e) {
   using S = Shape<kId>;
-  constexpr int kStep = 64 * S::KG, kBytes = tile_lds<kId, true>() > tile_lds<kId, false>() ? tile_lds<kId, true>() : tile_lds<kId, false>();
+  constexpr int kStep = 64 * S::KG, kBytes = tile_lds<kMlp, true>() > tile_lds<kId, false>() ? tile_lds<kMlp, true>() : tile_lds<kId, false>();
   TileProduct &r = g.router.p[0], &m = g.mlp.p[0];
-  const int64_t rb = tile_count<kId, false>(r), mb = tile_count<kId, true>(m);
+  const int64_t rb = tile_count<kId, false>(r), mb = tile_count<kMlp, true>(m);
   if (rb + mb > INT32_MAX / 2) return false;
   r.steps = m.steps = (r.seg[0].K + kStep - 1) / kStep;
   m.first = (int)rb;
   auto go = [&](auto tail) {
     constexpr bool kTail = decltype(tail)::value;
-    if ((*e = JointLds<tile_pair_kernel<DT, kId, kTail>, kBytes>::entry.ensure()) != hipSuccess) return;
-    hipLaunchKernelGGL((tile_pair_kernel<DT, kId, kTail>), dim3((unsigned)(rb + mb)), dim3(S::WM * S::WN * S::KG * 64), kBytes, s, g);
+    if ((*e = JointLds<tile_pair_kernel<DT, kId, kMlp, kTail>, kBytes>::entry.ensure()) != hipSuccess) return;
+    hipLaunchKernelGGL((tile_pair_kernel<DT, kId, kMlp, kTail>), dim3((unsigned)(rb + mb)), dim3(S::WM * S::WN * S::KG * 64), kBytes, s, g);
     *e = hipGetLastError();
   };
   if (r.seg[0].K % kStep) go(std::true_type{});
@@ -889,7 +902,10 @@ static hipError_t launch_choice(TileGroup& g, const TileChoice& c, float* ws, bo
     case 1: return launch_tiles<DT, LAY, 1, EPI>(g, ws, c.splits, exclusive, s);
     case 2: return launch_tiles<DT, LAY, 2, EPI>(g, ws, c.splits, exclusive, s);
     case 3: return launch_tiles<DT, LAY, 3, EPI>(g, ws, c.splits, exclusive, s);
-    case 4: return launch_tiles<DT, LAY, 4, EPI>(g, ws, c.splits, exclusive, s);
+    case 4:
+      if constexpr (EPI == kTileSwiglu)
+        if (g.p[0].seg[0].K > kShortSum * c.splits) return launch_tiles<DT, LAY, 10, EPI>(g, ws, c.splits, exclusive, s);
+      return launch_tiles<DT, LAY, 4, EPI>(g, ws, c.splits, exclusive, s);
     case 5: return launch_tiles<DT, LAY, 5, EPI>(g, ws, c.splits, exclusive, s);
     case 6: return launch_tiles<DT, LAY, 6, EPI>(g, ws, c.splits, exclusive, s);
     case 7: return launch_tiles<DT, LAY, 7, EPI>(g, ws, c.splits, exclusive, s);
@@ -970,7 +986,7 @@ bool tile_pair_of(int shape, TilePair& g, hipStream_t s, hipError_t* e) {
     case 1: return start_pair<DT, 1>(g, s, e);
     case 2: return start_pair<DT, 2>(g, s, e);
     case 3: return start_pair<DT, 3>(g, s, e);
-    case 4: return start_pair<DT, 4>(g, s, e);
+    case 4: return g.mlp.p[0].seg[0].K > kShortSum ? start_pair<DT, 4, 10>(g, s, e) : start_pair<DT, 4>(g, s, e);
     case 7: return start_pair<DT, 7>(g, s, e);
     case 8: return start_pair<DT, 8>(g, s, e);
     default: return false;

@@ -798,6 +798,25 @@ def test_mlp_on_lower_tiles(case, dtype, device):
     test_mlp_bwd_matches_matmuls(case, dtype, device)
 
 
+def _tile_choice(layout, epilogue, M, N, K):
+    """Rows and columns of the tiles of a product by itself, the groups of waves that share K, its parts: asked for before a test that means one kernel."""
+    import ctypes
+    from omni_moe.ops.hip import _lib
+    out = (ctypes.c_int32 * 4)()
+    assert _lib.load().omni_probe_tile_choice(layout, epilogue, M, N, K, ctypes.addressof(out)) == 0
+    return tuple(out)
+
+
+# T, H, I and the parts of gate and up on tiles of 64 x 64, whose ring has two stages for sums of up to 1536 and three beyond: four ring steps, both sides of the line, a K tail,
+# parts of a long sum
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case, parts", [((65, 512, 4104), 1), ((65, 1536, 2056), 1), ((65, 1544, 4104), 1), ((129, 2056, 2048), 1), ((129, 4096, 520), 8)], ids=str)
+def test_mlp_of_few_rows_on_short_and_long_sums(case, parts, dtype, device):
+    T, H, I = case
+    assert _tile_choice(0, 2, T, I, H) == (64, 64, 2, parts)
+    test_mlp_on_lower_tiles((*case, 0), dtype, device)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("case", [(64, 512), (1000, 1024), (4100, 1024)], ids=lambda c: "T%d-H%d" % c)
 def test_mlp_bwd_swiglu_is_the_operator(case, dtype, device):

@@ -990,6 +990,20 @@ def test_joint_launches_on_lower_tiles(case, dtype, device):
     test_joint_launches_match_the_operators(case, dtype, device)
 
 
+# the joint projections on tiles of 64 x 64, hidden sizes on both sides of the line between two ring stages for gate and up and three
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", [(70, 1536, 3072, 1024, 8), (70, 1544, 3072, 1024, 8), (129, 2048, 1032, 576, 8)], ids=lambda c: "x".join(map(str, c)))
+def test_joint_launches_on_short_and_long_sums(case, dtype, device):
+    import ctypes
+    import math
+    from omni_moe.ops.hip import _lib
+    T, H, I, N, k = case
+    pair, down = (ctypes.c_int32 * 2)(), (ctypes.c_int32 * 4)()
+    assert _lib.load().omni_probe_joint_tiles(T, H, I, math.isqrt(N), k, ctypes.addressof(pair), ctypes.addressof(down)) == 0
+    assert tuple(pair) == (64, 64)
+    test_joint_launches_match_the_operators(case, dtype, device)
+
+
 # T, H, I, N, k, and rows, columns and parts of the down projection's tiles beside which the selection runs; of batch statistics the selecting blocks merge (r <= 128)
 DOWN_CASES = [((950, 2048, 4096, 1024, 8), (192, 128, 2)), ((1295, 3128, 128, 64, 8), (192, 128, 1)), ((385, 2208, 7616, 4096, 8), (256, 128, 6)),
               ((805, 2048, 4096, 1024, 8), (128, 128, 1)), ((583, 520, 4096, 1024, 8), (96, 128, 5)), ((879, 520, 256, 1024, 8), (96, 128, 1)),
