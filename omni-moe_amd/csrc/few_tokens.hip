@@ -378,7 +378,9 @@ __device__ __forceinline__ void token_block(const MiddleArgs& g, int t, uint8_t*
 }
 
 // Blocks below select_blocks select (merged: and sum up a token's experts), the others multiply 32 output columns over one of the K splits.
-template <int DT, int R8, int Q, bool kMerged>
+// kTail: as in multiply().  Weights that go through LDS bear it at no cost; on the way into registers it is a branch around every load (down projection of 64 tokens,
+// 2048 x 8192, 11.7 us with it, 10.7 without).
+template <int DT, int R8, int Q, bool kMerged, bool kTail>
 __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel(const MiddleArgs g) {
   extern __shared__ __align__(16) uint8_t lds[];               // FewStage
   constexpr int TM = (R8 + 1) / 2;
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel
   const int64_t row_bytes = (int64_t)g.I * 2;
   const int second = min(n0 + 16, g.H - 1);
   f32x4_t acc[2][TM];
-  multiply<DT, R8, Q, true>(acc, g.h, g.I * 2, g.T * g.I * 2, {g.wd + n0 * row_bytes, g.wd + second * row_bytes}, {g.H - n0, g.H - second}, g.I, split * g.units,
+  multiply<DT, R8, Q, kTail>(acc, g.h, g.I * 2, g.T * g.I * 2, {g.wd + n0 * row_bytes, g.wd + second * row_bytes}, {g.H - n0, g.H - second}, g.I, split * g.units,
                             min((split + 1) * g.units, (g.I + kUnit - 1) / kUnit), wave, lane, mine);
   publish<R8, Q>(lds, acc, wave, lane);
   for (int i = threadIdx.x; i < TM * 128; i += kFewThreads) {
@@ -425,22 +427,27 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel
   }
 }
 
-struct BackArgs {
-  FewExperts e;
-  const uint8_t* residual;
+// (Kernel arguments come from uncached memory, 64 bytes at a time: behind the experts' the MLP's own were a second trip, down projection's sums of 64 tokens 4.2 -> 4.6 us.)
+struct BackSums {
   const float* parts;
   uint8_t* y;
-  int T, splits;
+  const uint8_t* residual;
+  int T, H, splits;
 };
+struct BackArgs { FewExperts e; BackSums sums; };
 
 // Launch 3 where it is one of its own, a block per token: y = round(round(sum of the parts) + round(experts)).  NCH 1-KiB pieces of a row; G slots of a wave at once.
 // splits 0: y holds the rounded sums already.
 // kExperts false: the MLP alone, residual (or nothing) instead of the experts.
 template <int DT, int NCH, int G, bool kExperts>
-__global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const BackArgs g) {
+__global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const std::conditional_t<kExperts, BackArgs, BackSums> args) {
   extern __shared__ __align__(16) float sums[];                // [waves][NCH * 512]
-  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x, H = g.e.H;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x;
   constexpr int kRow = NCH * 512;
+  BackSums g;
+  if constexpr (kExperts) g = args.sums;
+  else g = args;
+  const int H = g.H;
   // this thread's first four columns of every part, requested before anything else
   f32x4_t part[kMostParts];
   const int64_t plane = (int64_t)g.T * H;
@@ -452,7 +459,7 @@ __global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const BackArgs
   request(threadIdx.x * 4);
   int active = 0;
   if constexpr (kExperts) {
-    active = share_experts<DT, NCH, G>(g.e, t, wave, lane, sums, kRow);
+    active = share_experts<DT, NCH, G>(args.e, t, wave, lane, sums, kRow);
     __syncthreads();
   }
   for (int n = threadIdx.x * 4; n < H; n += kFewThreads * 4) {
@@ -504,8 +511,8 @@ hipError_t start(const Args& a, int64_t blocks, hipStream_t s) {
 }
 
 BackArgs back_args(const FewTokens& f, int splits) {
-  return BackArgs{FewExperts{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, f.select.gates, f.select.indices, f.H, f.select.k, (uint32_t)f.N}, (const uint8_t*)f.residual, f.parts,
-                  (uint8_t*)f.y, f.T, splits};
+  return BackArgs{FewExperts{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, f.select.gates, f.select.indices, f.H, f.select.k, (uint32_t)f.N},
+                  BackSums{f.parts, (uint8_t*)f.y, (const uint8_t*)f.residual, f.T, f.H, splits}};
 }
 // f.parts: the down projection's parts [splits][T][H], and where launches 2 and 3 are one, the experts' rounded sums [T][H] | tickets [T][groups]
 struct FewParts {
@@ -523,10 +530,10 @@ struct FewParts {
 template <int DT>
 hipError_t launch_back(const BackArgs& b, hipStream_t s) {
   const int nch = (b.e.H + 511) / 512;
-  if (nch <= 1) return start<few_back_kernel<DT, 1, 4, true>, kFewWaves * 1 * 2048>(b, b.T, s);
-  if (nch <= 2) return start<few_back_kernel<DT, 2, 4, true>, kFewWaves * 2 * 2048>(b, b.T, s);
-  if (nch <= 4) return start<few_back_kernel<DT, 4, 2, true>, kFewWaves * 4 * 2048>(b, b.T, s);
-  return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, b.T, s);
+  if (nch <= 1) return start<few_back_kernel<DT, 1, 4, true>, kFewWaves * 1 * 2048>(b, b.sums.T, s);
+  if (nch <= 2) return start<few_back_kernel<DT, 2, 4, true>, kFewWaves * 2 * 2048>(b, b.sums.T, s);
+  if (nch <= 4) return start<few_back_kernel<DT, 4, 2, true>, kFewWaves * 4 * 2048>(b, b.sums.T, s);
+  return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, b.sums.T, s);
 }
 
 template <int DT, int R8>
@@ -569,13 +576,16 @@ hipError_t launch(const FewTokens& f, hipStream_t s) {
   e = units_at_once((R8 > 1 && middle > 256) || m.units <= kFewWaves, [&](auto q) -> hipError_t {           // (a wave may have one unit only)
     constexpr int Q = decltype(q)::value, kBytes = FewStage<R8, Q>::kBytes;
     if constexpr (R8 * 8 <= kMergedTokens) {
-      if (merged) return start<few_middle_kernel<DT, R8, Q, true>, kBytes>(m, middle, s);
+      if (merged) return start<few_middle_kernel<DT, R8, Q, true, true>, kBytes>(m, middle, s);
     }
-    return start<few_middle_kernel<DT, R8, Q, false>, kBytes>(m, middle, s);
+    if constexpr (!FewStage<R8, Q>::kWeightsInLds) {
+      if (f.I % kUnit == 0) return start<few_middle_kernel<DT, R8, Q, false, false>, kBytes>(m, middle, s);
+    }
+    return start<few_middle_kernel<DT, R8, Q, false, true>, kBytes>(m, middle, s);
   });
   if (e != hipSuccess || merged) return e;
   const BackArgs b = back_args(f, splits);
-  if (!layer) return start<few_back_kernel<DT, 1, 1, false>, 0>(b, f.T, s);
+  if (!layer) return start<few_back_kernel<DT, 1, 1, false>, 0>(b.sums, f.T, s);
   return launch_back<DT>(b, s);
 }
 
