@@ -427,39 +427,35 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel
   }
 }
 
-// (Kernel arguments come from uncached memory, 64 bytes at a time: behind the experts' the MLP's own were a second trip, down projection's sums of 64 tokens 4.2 -> 4.6 us.)
-struct BackSums {
+struct BackArgs {
+  FewExperts e;
+  const uint8_t* residual;
   const float* parts;
   uint8_t* y;
-  const uint8_t* residual;
-  int T, H, splits;
+  int T, splits;
 };
-struct BackArgs { FewExperts e; BackSums sums; };
 
 // Launch 3 where it is one of its own, a block per token: y = round(round(sum of the parts) + round(experts)).  NCH 1-KiB pieces of a row; G slots of a wave at once.
 // splits 0: y holds the rounded sums already.
 // kExperts false: the MLP alone, residual (or nothing) instead of the experts.
 template <int DT, int NCH, int G, bool kExperts>
-__global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const std::conditional_t<kExperts, BackArgs, BackSums> args) {
+__global__ __launch_bounds__(kFewThreads, 2) void few_back_kernel(const BackArgs g) {
   extern __shared__ __align__(16) float sums[];                // [waves][NCH * 512]
-  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x, H = g.e.H;
   constexpr int kRow = NCH * 512;
-  BackSums g;
-  if constexpr (kExperts) g = args.sums;
-  else g = args;
-  const int H = g.H;
   // this thread's first four columns of every part, requested before anything else
   f32x4_t part[kMostParts];
   const int64_t plane = (int64_t)g.T * H;
   auto request = [&](int n) __attribute__((always_inline)) {
+    if (kExperts && g.splits == 0) return;
+    const float* at = g.parts + (int64_t)t * H + min(n, H - 4);
 #pragma unroll
-    for (int s = 0; s < kMostParts; ++s)
-      if (g.splits) part[s] = *(const f32x4_t*)(g.parts + min(s, g.splits - 1) * plane + (int64_t)t * H + min(n, H - 4));
+    for (int s = 0; s < kMostParts; ++s) part[s] = *(const f32x4_t*)(at + min(s, g.splits - 1) * plane);
   };
   request(threadIdx.x * 4);
   int active = 0;
   if constexpr (kExperts) {
-    active = share_experts<DT, NCH, G>(args.e, t, wave, lane, sums, kRow);
+    active = share_experts<DT, NCH, G>(g.e, t, wave, lane, sums, kRow);
     __syncthreads();
   }
   for (int n = threadIdx.x * 4; n < H; n += kFewThreads * 4) {
@@ -512,7 +508,7 @@ hipError_t start(const Args& a, int64_t blocks, hipStream_t s) {
 
 BackArgs back_args(const FewTokens& f, int splits) {
   return BackArgs{FewExperts{(const uint8_t*)f.x, (const uint8_t*)f.up, (const uint8_t*)f.down, f.select.gates, f.select.indices, f.H, f.select.k, (uint32_t)f.N},
-                  BackSums{f.parts, (uint8_t*)f.y, (const uint8_t*)f.residual, f.T, f.H, splits}};
+                  (const uint8_t*)f.residual, f.parts, (uint8_t*)f.y, f.T, splits};
 }
 // f.parts: the down projection's parts [splits][T][H], and where launches 2 and 3 are one, the experts' rounded sums [T][H] | tickets [T][groups]
 struct FewParts {
@@ -530,10 +526,10 @@ struct FewParts {
 template <int DT>
 hipError_t launch_back(const BackArgs& b, hipStream_t s) {
   const int nch = (b.e.H + 511) / 512;
-  if (nch <= 1) return start<few_back_kernel<DT, 1, 4, true>, kFewWaves * 1 * 2048>(b, b.sums.T, s);
-  if (nch <= 2) return start<few_back_kernel<DT, 2, 4, true>, kFewWaves * 2 * 2048>(b, b.sums.T, s);
-  if (nch <= 4) return start<few_back_kernel<DT, 4, 2, true>, kFewWaves * 4 * 2048>(b, b.sums.T, s);
-  return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, b.sums.T, s);
+  if (nch <= 1) return start<few_back_kernel<DT, 1, 4, true>, kFewWaves * 1 * 2048>(b, b.T, s);
+  if (nch <= 2) return start<few_back_kernel<DT, 2, 4, true>, kFewWaves * 2 * 2048>(b, b.T, s);
+  if (nch <= 4) return start<few_back_kernel<DT, 4, 2, true>, kFewWaves * 4 * 2048>(b, b.T, s);
+  return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, b.T, s);
 }
 
 template <int DT, int R8>
@@ -585,7 +581,7 @@ hipError_t launch(const FewTokens& f, hipStream_t s) {
   });
   if (e != hipSuccess || merged) return e;
   const BackArgs b = back_args(f, splits);
-  if (!layer) return start<few_back_kernel<DT, 1, 1, false>, 0>(b.sums, f.T, s);
+  if (!layer) return start<few_back_kernel<DT, 1, 1, false>, 0>(b, f.T, s);
   return launch_back<DT>(b, s);
 }
 
