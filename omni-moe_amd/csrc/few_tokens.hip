@@ -274,13 +274,13 @@ __device__ __forceinline__ void add_up(const MiddleArgs& g, int t, int n, const 
 }
 
 template <int DT>
-__device__ __forceinline__ void select_tokens(const MiddleArgs& g, int first, int all, PrunePool& pool) {
+__device__ __forceinline__ void select_tokens(const MiddleArgs& g, int first, int all) {
   auto select = [&](auto cells) {
     constexpr int C = decltype(cells)::value;
-    if (g.select_regs <= 1) select_packed<DT, 1, C>(g.select, first, all, g.select.stats, pool);
-    else if (g.select_regs <= 2) select_packed<DT, 2, C>(g.select, first, all, g.select.stats, pool);
-    else if (g.select_regs <= 4) select_packed<DT, 4, C>(g.select, first, all, g.select.stats, pool);
-    else select_packed<DT, 8, C>(g.select, first, all, g.select.stats, pool);
+    if (g.select_regs <= 1) select_packed<DT, 1, C>(g.select, first, all, g.select.stats);
+    else if (g.select_regs <= 2) select_packed<DT, 2, C>(g.select, first, all, g.select.stats);
+    else if (g.select_regs <= 4) select_packed<DT, 4, C>(g.select, first, all, g.select.stats);
+    else select_packed<DT, 8, C>(g.select, first, all, g.select.stats);
   };
   if (g.cells <= 1) select(std::integral_constant<int, 1>{});
   else select(std::integral_constant<int, 2>{});
@@ -352,7 +352,7 @@ __device__ __forceinline__ int share_experts(const FewExperts& g, int t, int wav
 
 template <int DT>
 __device__ __forceinline__ void token_block(const MiddleArgs& g, int t, uint8_t* lds, int wave, int lane) {
-  if (wave == 0) select_tokens<DT>(g, t, g.T, *(PrunePool*)lds);
+  if (wave == 0) select_tokens<DT>(g, t, g.T);
   __syncthreads();
   float* sums = (float*)lds;                                   // [waves][H]
   const FewExperts f{g.x, g.up, g.down, g.select.gates, g.select.indices, g.H, g.select.k, g.N};
@@ -385,11 +385,10 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 ? 4 : 2) void few_middle_kernel
   extern __shared__ __align__(16) uint8_t lds[];               // FewStage
   constexpr int TM = (R8 + 1) / 2;
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  static_assert(FewStage<R8, Q>::kBytes >= (int)sizeof(PrunePool), "a block that selects prunes there");
   static_assert(FewStage<R8, Q>::kBytes >= kFewWaves * kMergedRow * 4, "a token's block has its waves' sums there");
   if ((int)blockIdx.x < g.select_blocks) {
     if constexpr (kMerged) token_block<DT>(g, (int)blockIdx.x, lds, wave, lane);
-    else select_tokens<DT>(g, (int)blockIdx.x * kFewWaves + wave, g.select_blocks * kFewWaves, *(PrunePool*)lds);
+    else select_tokens<DT>(g, (int)blockIdx.x * kFewWaves + wave, g.select_blocks * kFewWaves);
     return;
   }
   const uint32_t mine = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(wave * FewStage<R8, Q>::kPart);

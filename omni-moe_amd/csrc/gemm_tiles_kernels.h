@@ -793,8 +793,7 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
     constexpr int kWaves = S::WM * S::WN * S::KG;
     const int first = (int)blockIdx.x * kWaves + (int)(threadIdx.x >> 6), all = select_blocks * kWaves;
     const float* stats = g.select.stats;
-    extern __shared__ __align__(16) uint8_t lds[];             // (the ring of the blocks that multiply takes all of it)
-    PrunePool& pool = *(PrunePool*)(lds + 4 * merge_lds_floats(kMergeKeys, kWaves * kWave));
+    extern __shared__ __align__(16) uint8_t lds[];             // (the ring of the blocks that multiply)
     if (g.select.part_mean) {                                  // batch statistics: the block merges them first
       merge_statistics(g.select, (float*)lds, kWaves * kWave);
       stats = (const float*)lds;
@@ -802,10 +801,10 @@ __global__ __launch_bounds__(Shape<kId>::WM* Shape<kId>::WN* Shape<kId>::KG * 64
     count_batch(g.select);
     auto select = [&](auto cells) {
       constexpr int C = decltype(cells)::value;
-      if (g.regs <= 1) select_packed<DT, 1, C>(g.select, first, all, stats, pool);
-      else if (g.regs <= 2) select_packed<DT, 2, C>(g.select, first, all, stats, pool);
-      else if (g.regs <= 4) select_packed<DT, 4, C>(g.select, first, all, stats, pool);
-      else select_packed<DT, 8, C>(g.select, first, all, stats, pool);
+      if (g.regs <= 1) select_packed<DT, 1, C>(g.select, first, all, stats);
+      else if (g.regs <= 2) select_packed<DT, 2, C>(g.select, first, all, stats);
+      else if (g.regs <= 4) select_packed<DT, 4, C>(g.select, first, all, stats);
+      else select_packed<DT, 8, C>(g.select, first, all, stats);
     };
     if (g.cells <= 1) select(std::integral_constant<int, 1>{});
     else select(std::integral_constant<int, 2>{});
@@ -817,7 +816,7 @@ template <int kId, bool kSwiglu>
 constexpr int tile_lds() {
   using S = Shape<kId, kSwiglu>;
   constexpr int kBytes = TileRing<staged_rows<kNT>(S::WM * S::TM * 16, S::WM * S::WN * S::KG), S::WN * S::TN * 16, S::KG, S::NS>::kBytes;
-  static_assert(kBytes >= 4 * merge_lds_floats(kMergeKeys, S::WM * S::WN * S::KG * 64) + (int)sizeof(PrunePool), "a block that selects merges statistics and prunes there");
+  static_assert(kBytes >= 4 * merge_lds_floats(kMergeKeys, S::WM * S::WN * S::KG * 64), "a block that selects merges statistics there");
   return kBytes;
 }
 template <auto kKernel, int kBytes>

@@ -36,8 +36,7 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
 template <int DT, int R, int C>
 __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_packed_kernel(const SelectArgs g) {
   count_batch(g);
-  __shared__ PrunePool pool;
-  select_packed<DT, R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats, pool);
+  select_packed<DT, R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats);
 }
 
 // Training: the blocks merge the projection's column statistics themselves, W waves to a block.
@@ -46,8 +45,7 @@ __global__ __launch_bounds__(W* kWave) void router_select_merge_kernel(const Sel
   extern __shared__ __align__(16) float stats[];
   merge_statistics(g, stats, W * kWave);
   count_batch(g);
-  __shared__ PrunePool pool;
-  select_packed<DT, R, C>(g, blockIdx.x * W + (threadIdx.x >> 6), gridDim.x * W, stats, pool);
+  select_packed<DT, R, C>(g, blockIdx.x * W + (threadIdx.x >> 6), gridDim.x * W, stats);
 }
 
 // More keys per half than a wave's registers hold (r > 1024): 16-bit scores, k' <= 64.  The row is walked in chunks of

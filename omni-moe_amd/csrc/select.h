@@ -674,13 +674,21 @@ __device__ __forceinline__ void ktop64_2(uint32_t (&k0)[R], uint32_t (&k1)[R], c
 }
 
 // The same for the kp <= 32 largest alone, from the few keys that can be among them: of 64 lanes' largest keys the kp-th is a bound that kp keys reach, so
-// every key below it is out; what is left (for scores in no particular order about 42 of 512 keys at kp = 32) goes through LDS into one register and is
-// sorted there.  Two sorts of 64 keys instead of R and the merges: 32768 tokens, 2 x 512 keys, k = 32: 211 -> 165 us.  More than 64 left, or fewer than kp lanes with a key: all of them, as above.
-constexpr int kPruneTop = 32, kPruneWaves = 8;
-typedef uint32_t PrunePool[kPruneWaves][2][kWave];            // in LDS, a block's: a place to each of up to eight waves
+// every key below it is out; what is left (for scores in no particular order about 42 of 512 keys at kp = 32) goes into one register and is
+// sorted there.  Two sorts of 64 keys instead of R and the merges: 32768 tokens, 2 x 512 keys, k = 32: 211 -> 165 us.  More than 64 left, or fewer than kp lanes with a key: false, and the keys as they were.
+// The way there is a permutation of the lanes (ds_permute_b32) and no LDS: beside the 256 x 256 tile GEMM, whose ring takes all of a CU's, a block with any finds no place.
+constexpr int kPruneTop = 32;
+// Appends the keys that reach `least` to list[0..n), which has room for them (list: zeros beyond n): in order of lanes, the other lanes' places go round behind them (modulo 64, as
+// the instruction takes them) with a zero each
+__device__ __forceinline__ void kappend(uint32_t& list, int& n, const uint32_t key, const uint32_t least, const int lane) {
+  const uint64_t in = __ballot(key >= least);
+  const int count = __popcll(in), mine = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(in >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in, (uint32_t)n));
+  const int to = key >= least ? mine : 2 * n + count + lane - mine;
+  list |= (uint32_t)__builtin_amdgcn_ds_permute(to * 4, (int)(key >= least ? key : 0u));
+  n += count;
+}
 template <int R>
-__device__ __forceinline__ void ktop_pruned_2(uint32_t (&k0)[R], uint32_t (&k1)[R], const int kp, const int lane, PrunePool& pool) {
-  uint32_t (*mine)[kWave] = pool[(threadIdx.x >> 6) % kPruneWaves];
+__device__ __forceinline__ bool ktop_pruned_2(uint32_t (&k0)[R], uint32_t (&k1)[R], const int kp, const int lane) {
   uint32_t m0[1] = {k0[0]}, m1[1] = {k1[0]};
 #pragma unroll
   for (int a = 1; a < R; ++a) {
@@ -695,25 +703,18 @@ __device__ __forceinline__ void ktop_pruned_2(uint32_t (&k0)[R], uint32_t (&k1)[
     n0 += __popcll(__ballot(k0[a] >= t0));
     n1 += __popcll(__ballot(k1[a] >= t1));
   }
-  if (t0 == 0u || t1 == 0u || n0 > kWave || n1 > kWave) {
-    ktop64_2<R>(k0, k1, lane);
-    return;
-  }
-  int at0 = 0, at1 = 0;
+  if (t0 == 0u || t1 == 0u || n0 > kWave || n1 > kWave) return false;
+  uint32_t x[1] = {0u}, y[1] = {0u};
+  n0 = n1 = 0;
 #pragma unroll
   for (int a = 0; a < R; ++a) {
-    const uint64_t b0 = __ballot(k0[a] >= t0), b1 = __ballot(k1[a] >= t1);
-    if (k0[a] >= t0) mine[0][at0 + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b0 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b0, 0u))] = k0[a];
-    if (k1[a] >= t1) mine[1][at1 + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b1 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b1, 0u))] = k1[a];
-    at0 += __popcll(b0);
-    at1 += __popcll(b1);
+    kappend(x[0], n0, k0[a], t0, lane);
+    kappend(y[0], n1, k1[a], t1, lane);
   }
-  __builtin_amdgcn_wave_barrier();                              // a wave's LDS instructions take effect in order
-  uint32_t x[1] = {lane < n0 ? mine[0][lane] : 0u}, y[1] = {lane < n1 ? mine[1][lane] : 0u};
-  __builtin_amdgcn_wave_barrier();
   ksort2<1>(x, y, lane);
   k0[0] = x[0];
   k1[0] = y[0];
+  return true;
 }
 
 template <int R>
@@ -729,7 +730,7 @@ __device__ __forceinline__ uint32_t sorted_key(const uint32_t (&v)[R], int i) {
 // Same selection as select_pairs for bf16 / f16 storage, on packed keys: the tokens of wave `wave` of `num_waves`.  stats: g.stats, or what the
 // block merged.
 template <int DT, int R, int C>
-__device__ __forceinline__ void select_packed(const SelectArgs& g, const int wave, const int num_waves, const float* stats, PrunePool& pool) {
+__device__ __forceinline__ void select_packed(const SelectArgs& g, const int wave, const int num_waves, const float* stats) {
   const int lane = lane_id();
   const int r = g.r, k = g.k, kp = g.kp;
 
@@ -771,9 +772,8 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
       ky[a] = key < r ? make_key<DT>(sy[a], key) : 0u;
     }
     if constexpr (R > kUnrollMaxR) {                             // uniform: kp comes with the arguments
-      if (kp <= kPruneTop) ktop_pruned_2<R>(kx, ky, kp, lane, pool);
-      else if (kp <= kWave) ktop64_2<R>(kx, ky, lane);
-      else ksort2<R>(kx, ky, lane);
+      if (kp > kWave) ksort2<R>(kx, ky, lane);
+      else if (kp > kPruneTop || !ktop_pruned_2<R>(kx, ky, kp, lane)) ktop64_2<R>(kx, ky, lane);
     } else {
       ksort2<R>(kx, ky, lane);
     }
