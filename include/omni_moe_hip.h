@@ -223,6 +223,10 @@ OMNI_API int32_t omni_probe_joint_tiles(int64_t num_tokens, int32_t hidden_size,
  * sums, 1: with a residual, 2: gate and up with SwiGLU (columns: of each), 3: the SwiGLU backward.  choice[4]: rows and columns of a tile, groups of waves that share
  * its K, parts of K. */
 OMNI_API int32_t omni_probe_tile_choice(int32_t layout, int32_t epilogue, int64_t rows, int64_t columns, int64_t k, int32_t* choice);
+/* Diagnostic: how a 16-bit layer (num_expert_sqrt 0: the MLP alone) of at most 64 tokens runs in eval mode, from its sizes and whether the call is captured into a graph (nothing
+ * is launched).  plan[5]: launches (two or three), rows of activations that a block stages, K units of a wave in LDS at once in the first launch and in the second, parts of
+ * the down projection. */
+OMNI_API int32_t omni_probe_few_tokens(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t num_expert_sqrt, int32_t captured, int32_t* plan);
 
 /* y[i] = round(y[i] + addend[i]) in place: the layer's final  mlp + experts  (omni_moe.py:102) as a
  * call of its own, for callers that run the two branches on different streams.  num_elements a

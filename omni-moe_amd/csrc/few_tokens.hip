@@ -231,12 +231,27 @@ struct MiddleArgs {
   uint32_t N;
 };
 // So two launches are for calls whose kernels take less than the host: up to 16 tokens and 2^23 weights a projection (the MLP alone, whose host work is less: 2^22), up to 48
-// tokens and 2^21.  The MLP alone, three / two in a graph: 1 token 512 x 2048 7.4 / 7.4, 16 tokens 7.6 / 8.3, 1024 x 4096 11.5 / 12.7; a call as a program
-// makes it 13.2 / 10.9 at 8 tokens, 512 x 1024.
+// tokens and 2^21.  The MLP alone, a call as a program makes it, three / two: 16 tokens 1024 x 4096 12.2 / 11.1 us, 8 tokens 512 x 1024 12.4 / 9.7.
+// A graph's replay has no host work, and what is captured takes two launches only where its kernels are no slower for it.  Three / two in a graph, the layer: 1 token 512 x 2048
+// 10.7 / 10.7 us, 16 tokens 768 x 3072 12.7 / 12.7, 48 tokens 1024 x 2048 14.1 / 14.2, 512 x 2048 12.8 / 12.5; but 16 tokens 1024 x 4096 13.8 / 14.5.  The MLP alone: 16 tokens 512 x 1024
+// 8.4 / 8.3; but 32 tokens 9.0 / 9.3, 16 tokens 512 x 2048 8.5 / 9.1, 1024 x 4096 9.1 / 10.8.  Either form leaves the same bits.
 constexpr int kMergedTokens = 48, kMergedRow = 1024;           // (a token's block has a thread for four values of a row)
-bool merge_launches(bool layer, int64_t T, int64_t H, int64_t I) {
+bool merge_launches(bool layer, int64_t T, int64_t H, int64_t I, bool replayed) {
+  const int64_t weights = H * I;
   if (layer && H > kMergedRow) return false;
-  return T <= 16 ? H * I <= (layer ? 1 << 23 : 1 << 22) : T <= kMergedTokens && H * I <= (1 << 21);
+  if (replayed && !layer) return T <= 16 && weights <= 1 << 19;
+  if (T > 16) return T <= kMergedTokens && weights <= 1 << 21;
+  return weights <= (replayed ? 3 << 20 : layer ? 1 << 23 : 1 << 22);
+}
+// Whether the call goes into a graph.  (The null stream is never captured, and asking about it while another stream is being captured is an error.)
+bool is_captured(hipStream_t s) {
+  if (!s) return false;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
 }
 __device__ __forceinline__ void store_agent(void* at, uint32_t a, uint32_t b) {
   __hip_atomic_store((uint64_t*)at, (uint64_t)a | (uint64_t)b << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -518,7 +533,7 @@ struct FewParts {
     const size_t sums = (size_t)few_splits(H, I) * (size_t)T * (size_t)H * 4, rows = ((size_t)T * (size_t)H * 2 + 15) / 16 * 16;
     experts = (uint8_t*)parts + sums;
     tickets = (uint32_t*)(experts + rows);
-    bytes = sums + (merge_launches(true, T, H, I) || merge_launches(false, T, H, I) ? rows + (size_t)T * (size_t)((H + 31) / 32) * 4 : 0);
+    bytes = sums + (merge_launches(true, T, H, I, false) || merge_launches(false, T, H, I, false) ? rows + (size_t)T * (size_t)((H + 31) / 32) * 4 : 0);
   }
 };
 
@@ -531,55 +546,74 @@ hipError_t launch_back(const BackArgs& b, hipStream_t s) {
   return start<few_back_kernel<DT, 8, 1, true>, kFewWaves * 8 * 2048>(b, b.T, s);
 }
 
-template <int DT, int R8>
-hipError_t launch(const FewTokens& f, hipStream_t s) {
-  const bool layer = f.up != nullptr;
-  const int r = f.select.r;
-  const bool merged = merge_launches(layer, f.T, f.H, f.I);
-  const FewParts p(f.parts, f.T, f.H, f.I);
-  const FrontArgs a{(const uint8_t*)f.x, (const uint8_t*)f.wg, (const uint8_t*)f.wu, (const uint8_t*)f.wx, (const uint8_t*)f.wy, (uint8_t*)f.h, (uint8_t*)f.z,
-                    f.T, f.H, f.I, r, layer ? (r + 15) / 16 : 0, merged ? p.tickets : nullptr, merged ? f.T * ((f.H + 31) / 32) : 0};
-  const int64_t front = a.router_blocks + (f.I + 15) / 16;
+// What a call takes, from its sizes; r 0: the MLP alone
+struct FewPlan {
+  int r8;                            // FewStage's
+  bool merged;
+  int front_units, middle_units;     // K units of a wave in LDS at once
+  int splits, units;                 // of the down projection; K units to a split
+  int router_blocks, select_blocks;
+  int64_t front, middle;             // blocks
+};
+FewPlan plan_few(int64_t T, int64_t H, int64_t I, int r, bool replayed) {
+  FewPlan p;
+  p.r8 = T <= 8 ? 1 : T <= 16 ? 2 : T <= 32 ? 4 : T <= 48 ? 6 : 8;
+  p.merged = merge_launches(r > 0, T, H, I, replayed);
+  p.router_blocks = (r + 15) / 16;
+  p.front = p.router_blocks + (I + 15) / 16;
+  const int units = (int)((I + kUnit - 1) / kUnit), most = few_splits(H, I);
+  p.units = (units + most - 1) / most;
+  p.splits = (units + p.units - 1) / p.units;                  // every split has work
+  p.select_blocks = (int)(r == 0 ? 0 : p.merged ? T : (T + kFewWaves - 1) / kFewWaves);
+  p.middle = p.select_blocks + (H + 31) / 32 * p.splits;
   // Beyond eight tokens two K units of a wave in LDS at once are more than half of a CU's: one block to a CU, and blocks beyond 256 wait for a whole round.
   // One unit at a time then (in turn over three sets of inputs, hidden 1024 x intermediate 4096, weights in registers: 33 tokens 23.5 -> 21.3 us, 48 24.1 -> 21.9, 64
   // 26.2 -> 22.9; 48 tokens, 2048 x 8192 49.9 -> 43.9).  Where a launch has no more blocks than CUs both units stay in flight, if a wave has two.
-  auto units_at_once = [&](bool one, auto&& go) -> hipError_t {
-    if (one) return go(std::integral_constant<int, 1>{});
+  p.front_units = (p.r8 > 1 && p.front > 256) || H <= kFewWaves * kUnit ? 1 : 2;
+  p.middle_units = (p.r8 > 1 && p.middle > 256) || p.units <= kFewWaves ? 1 : 2;       // (a wave may have one unit only)
+  return p;
+}
+
+template <int DT, int R8>
+hipError_t launch(const FewTokens& f, const FewPlan& plan, hipStream_t s) {
+  const bool layer = f.up != nullptr, merged = plan.merged;
+  const FewParts p(f.parts, f.T, f.H, f.I);
+  const FrontArgs a{(const uint8_t*)f.x, (const uint8_t*)f.wg, (const uint8_t*)f.wu, (const uint8_t*)f.wx, (const uint8_t*)f.wy, (uint8_t*)f.h, (uint8_t*)f.z,
+                    f.T, f.H, f.I, f.select.r, plan.router_blocks, merged ? p.tickets : nullptr, merged ? f.T * ((f.H + 31) / 32) : 0};
+  auto units_at_once = [&](int units, auto&& go) -> hipError_t {
+    if (units == 1) return go(std::integral_constant<int, 1>{});
     return go(std::integral_constant<int, 2>{});
   };
-  hipError_t e = units_at_once((R8 > 1 && front > 256) || f.H <= kFewWaves * kUnit, [&](auto q) -> hipError_t {
+  hipError_t e = units_at_once(plan.front_units, [&](auto q) -> hipError_t {
     constexpr int Q = decltype(q)::value, kBytes = FewStage<R8, Q>::kBytes;
-    return f.H % kUnit ? start<few_front_kernel<DT, R8, Q, true>, kBytes>(a, front, s) : start<few_front_kernel<DT, R8, Q, false>, kBytes>(a, front, s);
+    return f.H % kUnit ? start<few_front_kernel<DT, R8, Q, true>, kBytes>(a, plan.front, s) : start<few_front_kernel<DT, R8, Q, false>, kBytes>(a, plan.front, s);
   });
   if (e != hipSuccess) return e;
 
-  const int units = (f.I + kUnit - 1) / kUnit;
-  int splits = few_splits(f.H, f.I);
   MiddleArgs m{};
   m.h = (const uint8_t*)f.h; m.wd = (const uint8_t*)f.wd; m.parts = f.parts; m.T = f.T; m.H = f.H; m.I = f.I;
   m.groups = (f.H + 31) / 32;
-  m.units = (units + splits - 1) / splits;
-  m.splits = splits = (units + m.units - 1) / m.units;         // every split has work
-  m.tickets = p.tickets; m.numbers = (uint32_t)(layer ? splits + 1 : splits); m.experts = layer ? p.experts : nullptr; m.residual = (const uint8_t*)f.residual;
+  m.units = plan.units;
+  m.splits = plan.splits;
+  m.tickets = p.tickets; m.numbers = (uint32_t)(layer ? m.splits + 1 : m.splits); m.experts = layer ? p.experts : nullptr; m.residual = (const uint8_t*)f.residual;
   m.x = (const uint8_t*)f.x; m.up = (const uint8_t*)f.up; m.down = (const uint8_t*)f.down; m.y = (uint8_t*)f.y;
   m.N = (uint32_t)f.N;
   m.select = f.select;
-  m.select_regs = (r + kWave - 1) / kWave;
+  m.select_regs = (f.select.r + kWave - 1) / kWave;
   m.cells = layer ? prepare_select(m.select) : 0;
-  m.select_blocks = !layer ? 0 : merged ? f.T : (f.T + kFewWaves - 1) / kFewWaves;
-  const int64_t middle = m.select_blocks + (int64_t)m.groups * splits;
-  e = units_at_once((R8 > 1 && middle > 256) || m.units <= kFewWaves, [&](auto q) -> hipError_t {           // (a wave may have one unit only)
+  m.select_blocks = plan.select_blocks;
+  e = units_at_once(plan.middle_units, [&](auto q) -> hipError_t {
     constexpr int Q = decltype(q)::value, kBytes = FewStage<R8, Q>::kBytes;
     if constexpr (R8 * 8 <= kMergedTokens) {
-      if (merged) return start<few_middle_kernel<DT, R8, Q, true, true>, kBytes>(m, middle, s);
+      if (merged) return start<few_middle_kernel<DT, R8, Q, true, true>, kBytes>(m, plan.middle, s);
     }
     if constexpr (!FewStage<R8, Q>::kWeightsInLds) {
-      if (f.I % kUnit == 0) return start<few_middle_kernel<DT, R8, Q, false, false>, kBytes>(m, middle, s);
+      if (f.I % kUnit == 0) return start<few_middle_kernel<DT, R8, Q, false, false>, kBytes>(m, plan.middle, s);
     }
-    return start<few_middle_kernel<DT, R8, Q, false, true>, kBytes>(m, middle, s);
+    return start<few_middle_kernel<DT, R8, Q, false, true>, kBytes>(m, plan.middle, s);
   });
   if (e != hipSuccess || merged) return e;
-  const BackArgs b = back_args(f, splits);
+  const BackArgs b = back_args(f, m.splits);
   if (!layer) return start<few_back_kernel<DT, 1, 1, false>, 0>(b, f.T, s);
   return launch_back<DT>(b, s);
 }
@@ -601,13 +635,18 @@ bool few_tokens_aligned(const FewTokens& f) {
 size_t few_tokens_parts_bytes(int64_t T, int64_t H, int64_t I) { return FewParts(nullptr, T, H, I).bytes; }
 
 hipError_t launch_few_tokens(int dtype, const FewTokens& f, hipStream_t s) {
+  const bool layer = f.up != nullptr;
+  const int r = layer ? f.select.r : 0;
+  // (asked only where the answer matters)
+  const bool replayed = merge_launches(layer, f.T, f.H, f.I, false) && !merge_launches(layer, f.T, f.H, f.I, true) && is_captured(s);
+  const FewPlan plan = plan_few(f.T, f.H, f.I, r, replayed);
   auto go = [&](auto dt) -> hipError_t {
     constexpr int DT = decltype(dt)::value;
-    if (f.T <= 8) return launch<DT, 1>(f, s);
-    if (f.T <= 16) return launch<DT, 2>(f, s);
-    if (f.T <= 32) return launch<DT, 4>(f, s);
-    if (f.T <= 48) return launch<DT, 6>(f, s);
-    return launch<DT, 8>(f, s);
+    if (plan.r8 == 1) return launch<DT, 1>(f, plan, s);
+    if (plan.r8 == 2) return launch<DT, 2>(f, plan, s);
+    if (plan.r8 == 4) return launch<DT, 4>(f, plan, s);
+    if (plan.r8 == 6) return launch<DT, 6>(f, plan, s);
+    return launch<DT, 8>(f, plan, s);
   };
   if (dtype == kBF16) return go(std::integral_constant<int, kBF16>{});
   if (dtype == kF16) return go(std::integral_constant<int, kF16>{});
@@ -622,3 +661,16 @@ hipError_t launch_few_back(int dtype, const FewTokens& f, int splits, hipStream_
 }
 
 }  // namespace omni
+
+extern "C" OMNI_API int32_t omni_probe_few_tokens(int64_t num_tokens, int32_t hidden_size, int32_t intermediate_size, int32_t num_expert_sqrt, int32_t captured, int32_t* plan) {
+  using namespace omni;
+  if (!few_tokens_covers(num_tokens, hidden_size, intermediate_size, OMNI_BF16) || hidden_size <= 0 || intermediate_size <= 0 || num_expert_sqrt < 0) return OMNI_ERR_SHAPE;
+  if (!plan) return OMNI_ERR_NULL;
+  const FewPlan p = plan_few(num_tokens, hidden_size, intermediate_size, num_expert_sqrt, captured != 0);
+  plan[0] = p.merged ? 2 : 3;
+  plan[1] = p.r8 * 8;
+  plan[2] = p.front_units;
+  plan[3] = p.middle_units;
+  plan[4] = p.splits;
+  return OMNI_OK;
+}

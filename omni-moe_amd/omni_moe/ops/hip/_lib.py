@@ -53,6 +53,7 @@ SIGNATURES = {
     "omni_probe_mfma16": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
     "omni_probe_joint_tiles": (c_int32, [c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
     "omni_probe_tile_choice": (c_int32, [c_int32, c_int32, c_int64, c_int64, c_int64, c_void_p]),
+    "omni_probe_few_tokens": (c_int32, [c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p]),
     "omni_add_inplace": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_void_p]),
     "omni_linear2_fwd": (c_int32, [c_void_p] * 4 + [c_int64, c_int32, c_int32, c_int32, c_void_p]),
     "omni_router_workspace_bytes": (c_size_t, [c_int64, c_int32, c_int32]),

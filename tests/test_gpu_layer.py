@@ -903,6 +903,53 @@ def test_few_tokens_in_two_launches(case, dtype, device):
             assert torch.equal(layer(xs[(i + 1) % 4]), first[(i + 1) % 4])
 
 
+def _few_tokens_plan(T, H, I, r, captured=False):
+    """Launches, staged rows, K units at once in the first launch and the second, parts of the down projection (r 0: the MLP alone)."""
+    import ctypes
+    from omni_moe.ops.hip import _lib
+    out = (ctypes.c_int32 * 5)()
+    assert _lib.load().omni_probe_few_tokens(T, H, I, r, captured, ctypes.addressof(out)) == 0
+    return tuple(out)
+
+
+def _graph_nodes(call):
+    """Nodes of a graph that one call is captured into: its launches."""
+    import ctypes
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        y = call()
+    count = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    graph.replay()
+    torch.cuda.synchronize()
+    return count.value, y
+
+
+# T, H, I of a layer and launches when a program makes the call, when it is captured; the same for its MLP alone.  A replay has no host work, so that two launches are taken only
+# where their kernels are no slower: both sides of the lines at 3 * 2^20 weights a projection, 2^21 beyond 16 tokens, 2^19 for the MLP
+@pytest.mark.parametrize("case, layer, mlp", [((16, 1024, 4096), (2, 3), (2, 3)), ((16, 768, 4096), (2, 2), (2, 3)), ((5, 768, 4104), (2, 3), (2, 3)), ((48, 1024, 2048), (2, 2), (2, 3)),
+                                              ((16, 512, 1024), (2, 2), (2, 2)), ((17, 512, 1024), (2, 2), (2, 3)), ((16, 520, 1024), (2, 2), (2, 3)), ((2, 2048, 4096), (3, 3), (3, 3))], ids=str)
+def test_captured_calls_of_few_tokens_take_the_launches_that_replay_faster(case, layer, mlp, device):
+    """... and leave the bits of the call that a program makes."""
+    from omni_moe.modules.omni_moe import OmniMoE, OmniMoEConfig
+    T, H, I = case
+    assert tuple(_few_tokens_plan(T, H, I, 16, c)[0] for c in (False, True)) == layer
+    assert tuple(_few_tokens_plan(T, H, I, 0, c)[0] for c in (False, True)) == mlp
+    module = OmniMoE(OmniMoEConfig(H, I, "silu", 256, 8)).to(device=device, dtype=torch.bfloat16).eval()
+    g = torch.Generator(device=device).manual_seed(T + I)
+    with torch.no_grad():
+        for p in module.parameters():
+            p.normal_(0.0, H ** -0.5, generator=g)
+        x = torch.randn(1, T, H, device=device, generator=g).bfloat16()
+        alone = lambda: _ops().hip_omni_mlp_func(x[0], module.gate_proj.weight, module.up_proj.weight, module.down_proj.weight)
+        for call, launches in ((lambda: module(x), layer), (alone, mlp)):
+            want = call()
+            nodes, y = _graph_nodes(call)
+            assert nodes == launches[1]
+            assert torch.equal(y, want)
+
+
 # T, H, I: 32-row and 32-column tiles and their remainders, K of one to five tiles of 32 and with a remainder, more and fewer waves than K tiles
 @pytest.mark.parametrize("case", [(1, 4, 4), (33, 36, 100), (512, 256, 1024), (100, 1028, 68), (640, 160, 96), (65, 128, 132),
                    # 256 and 288 blocks of the SwiGLU product (two ring stages, one), 512 and 544 of the down projection
