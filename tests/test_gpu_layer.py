@@ -912,6 +912,26 @@ def _few_tokens_plan(T, H, I, r, captured=False):
     return tuple(out)
 
 
+# T, H, I, N, k and the plan: at most eight tokens in three launches (hidden past 1024), one and two K units of a wave at once; more than eight units to a part in two launches and
+# in three; 64 tokens, whose weights stay in registers, with two units at once and no K tail
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case, plan", [((1, 2048, 8192, 4096, 16), (3, 8, 2, 2, 4)), ((8, 4096, 520, 1024, 4), (3, 8, 2, 2, 1)), ((5, 1032, 4104, 576, 8), (3, 8, 2, 2, 7)),
+                                        ((8, 1040, 264, 256, 8), (3, 8, 2, 1, 1)), ((8, 2048, 8200, 1000, 4), (3, 8, 2, 2, 4)), ((8, 256, 8192, 1024, 8), (2, 8, 1, 2, 8)),
+                                        ((3, 264, 7944, 256, 4), (2, 8, 1, 2, 8)), ((64, 768, 8192, 256, 4), (3, 64, 1, 2, 8))], ids=str)
+def test_few_tokens_on_every_plan(case, plan, dtype, device):
+    T, H, I, N, _ = case
+    assert _few_tokens_plan(T, H, I, int(N ** 0.5)) == plan
+    test_few_tokens_match_the_operators(case, dtype, device)
+
+
+# ... and of the MLP alone, which takes two launches for other sizes
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case, plan", [((8, 8200, 512), (3, 8, 2, 1, 1)), ((7, 2048, 8192), (3, 8, 2, 2, 4)), ((8, 1040, 520), (2, 8, 2, 2, 1)), ((6, 512, 512), (2, 8, 1, 1, 1))], ids=str)
+def test_mlp_of_few_tokens_on_every_plan(case, plan, dtype, device):
+    assert _few_tokens_plan(*case, 0) == plan
+    test_mlp_matches_oracle(case, dtype, device)
+
+
 def _graph_nodes(call):
     """Nodes of a graph that one call is captured into: its launches."""
     import ctypes
