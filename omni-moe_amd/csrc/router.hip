@@ -33,8 +33,12 @@ __global__ __launch_bounds__(kRouterWaves* kWave) void router_select_kernel(cons
   select_pairs<R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats);
 }
 
+// Waves to a SIMD that the registers have to leave room for, where a few more of them would cost one (router of 32768 tokens, hidden 256, 1000 keys a half, top-16: with 169
+// registers, two waves, 435 us; with 168, three, 355)
+template <int R, int C>
+constexpr int kSelectWaves = R == 16 && C <= 4 ? 3 : 1;
 template <int DT, int R, int C>
-__global__ __launch_bounds__(kRouterWaves* kWave) void router_select_packed_kernel(const SelectArgs g) {
+__global__ __launch_bounds__(kRouterWaves* kWave, (kSelectWaves<R, C>)) void router_select_packed_kernel(const SelectArgs g) {
   count_batch(g);
   select_packed<DT, R, C>(g, blockIdx.x * kRouterWaves + (threadIdx.x >> 6), gridDim.x * kRouterWaves, g.stats);
 }

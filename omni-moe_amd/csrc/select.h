@@ -764,6 +764,9 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
       normalise_half<DT, R>(sx, g, norm, stats, 0, r, lane);
       normalise_half<DT, R>(sy, g, norm, stats, 1, r, lane);
     }
+    // (With most keys the sorts' masks are made anew for each token: held from one to the next they are six registers where there are none to spare, kSelectWaves)
+    int here = lane;
+    if constexpr (R > 8) asm volatile("" : "+v"(here));
     uint32_t kx[R], ky[R];
 #pragma unroll
     for (int a = 0; a < R; ++a) {
@@ -772,10 +775,10 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
       ky[a] = key < r ? make_key<DT>(sy[a], key) : 0u;
     }
     if constexpr (R > kUnrollMaxR) {                             // uniform: kp comes with the arguments
-      if (kp > kWave) ksort2<R>(kx, ky, lane);
-      else if (kp > kPruneTop || !ktop_pruned_2<R>(kx, ky, kp, lane)) ktop64_2<R>(kx, ky, lane);
+      if (kp > kWave) ksort2<R>(kx, ky, here);
+      else if (kp > kPruneTop || !ktop_pruned_2<R>(kx, ky, kp, here)) ktop64_2<R>(kx, ky, here);
     } else {
-      ksort2<R>(kx, ky, lane);
+      ksort2<R>(kx, ky, here);
     }
 
     uint32_t ck[C];
@@ -786,7 +789,7 @@ __device__ __forceinline__ void select_packed(const SelectArgs& g, const int wav
       const float va = key_score<DT>(sorted_key<R>(kx, a)), vb = key_score<DT>(sorted_key<R>(ky, b));
       ck[c] = ok ? make_key<DT>(Elem<DT>::round(va + vb), cell[c]) : 0u;
     }
-    ksort<C>(ck, lane);
+    ksort<C>(ck, here);
 
     constexpr int kOut = (C >= 2) ? 2 : 1;          // k <= 128 -> winners live in regs 0..1
 #pragma unroll

@@ -53,3 +53,11 @@ def test_selection_beside_the_large_tiles_takes_no_lds(kernels):
     assert len(found) >= 32
     for k in found:
         assert k[".group_segment_fixed_size"] == 0, k[".name"]
+
+
+def test_selection_of_most_keys_leaves_room_for_three_waves(kernels):
+    """More than 512 keys a half, up to 256 candidates: with a few more registers than 168 a SIMD holds two waves instead of three, which took 14 % longer."""
+    found = [k for k in kernels if any(f"router_select_packed_kernelILi{dt}ELi16ELi{c}E" in k[".name"] for dt in (0, 1) for c in (1, 2, 4))]
+    assert len(found) == 6
+    for k in found:
+        assert k[".vgpr_count"] + k.get(".agpr_count", 0) <= 168, k[".name"]
