@@ -723,7 +723,7 @@ MLP_BWD_CASES = [(1, 8, 8, 0), (77, 64, 136, 7), (200, 72, 264, 17), (129, 520, 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("case", MLP_BWD_CASES, ids=lambda c: "T%d-H%d-I%d-r%d" % c)
-def test_mlp_bwd_matches_matmuls(case, dtype, device):
+def test_mlp_bwd_matches_matmuls(case, dtype, device, with_addend=True):
     """omni_mlp_bwd against the same products in fp32 on the same stored operands.  Both round d(h), d(gate) and d(up) to the storage type; sums in
     another order move a last bit of some of them, so an output is within one rounding (2^-9 bf16, 2^-12 f16, relative) of the reference in the
     2-norm, and within a few of the largest value anywhere."""
@@ -744,7 +744,9 @@ def test_mlp_bwd_matches_matmuls(case, dtype, device):
     gf, sig = gate.float(), torch.sigmoid(gate.float())
     dup = rnd(dh * gf * sig)
     dgate = rnd(dh * (gf * sig * (1 - sig) + sig) * up.float())
-    dx = rnd(dgate @ wg.float() + dup @ wu.float() + dz[:, 0, :r].float() @ rx.float() + dz[:, 1, :r].float() @ ry.float()) + addend.float()
+    dx = rnd(dgate @ wg.float() + dup @ wu.float() + dz[:, 0, :r].float() @ rx.float() + dz[:, 1, :r].float() @ ry.float())
+    if with_addend:
+        dx = dx + addend.float()
     want = [dx, dgate.t() @ x.float(), dup.t() @ x.float(), dy.float().t() @ h.float()]
     if r:
         want += [dz[:, 0, :r].float().t() @ x.float(), dz[:, 1, :r].float().t() @ x.float()]
@@ -754,12 +756,25 @@ def test_mlp_bwd_matches_matmuls(case, dtype, device):
     ws = torch.empty(lib.omni_mlp_bwd_workspace_bytes(T, H, I, r, dt), device=device, dtype=torch.uint8)
     print(f"mlp_bwd T={T} H={H} I={I} r={r} {dtype}", flush=True)
     args = [t.data_ptr() for t in (dy, x, wg, wu, wd, gate, up, h)] + ([dz.data_ptr(), rx.data_ptr(), ry.data_ptr()] if r else [None] * 3)
-    _lib.check(lib.omni_mlp_bwd(*args, addend.data_ptr(), *ptrs, T, H, I, r, dt, ws.data_ptr(), _lib.stream_ptr()), "omni_mlp_bwd")
+    _lib.check(lib.omni_mlp_bwd(*args, addend.data_ptr() if with_addend else None, *ptrs, T, H, I, r, dt, ws.data_ptr(), _lib.stream_ptr()), "omni_mlp_bwd")
     ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     for name, a, w in zip(("dx", "dWg", "dWu", "dWd", "dWx", "dWy"), got, want):
         err = a.float() - w
         assert (err.norm() <= ulp * w.norm()).item(), (name, (err.norm() / w.norm()).item())
         assert (err.abs().max() <= 4 * ulp * w.abs().max()).item(), (name, (err.abs().max() / w.abs().max()).item())
+
+
+def _tile_choice(layout, epilogue, M, N, K):
+    """Rows and columns of the tiles of a product by itself, the groups of waves that share K, its parts: asked for before a test that means one kernel."""
+    import ctypes
+    from omni_moe.ops.hip import _lib
+    out = (ctypes.c_int32 * 4)()
+    assert _lib.load().omni_probe_tile_choice(layout, epilogue, M, N, K, ctypes.addressof(out)) == 0
+    return tuple(out)
+
+
+def _up64(n):
+    return (n + 63) // 64 * 64
 
 
 # T, H, I, r: d(x) as sums so long that it takes two K groups on 128 x 128 tiles: whole tiles, rows one past a tile and columns short of one, K tails of the 128 of K that a
@@ -769,7 +784,19 @@ LONG_SUM_CASES = [(2048, 2048, 4096, 64), (1921, 2040, 4104, 17), (1921, 1928, 4
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("case", LONG_SUM_CASES, ids=lambda c: "x".join(map(str, c)))
-def test_mlp_bwd_long_sums(case, dtype, device):
+@pytest.mark.parametrize("with_addend", [True, False], ids=["addend", "alone"])
+def test_mlp_bwd_long_sums(with_addend, case, dtype, device):
+    T, H, I, r = case
+    assert _tile_choice(1, 1 if with_addend else 0, T, H, 2 * _up64(I) + 2 * _up64(r)) == (128, 128, 2, 1)
+    test_mlp_bwd_matches_matmuls(case, dtype, device, with_addend)
+
+
+# ... and d(h) of a wide hidden size, the SwiGLU backward behind the exchange of the two groups' sums
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", [(2048, 8192, 2048, 0), (1921, 8200, 2040, 17)], ids=lambda c: "x".join(map(str, c)))
+def test_mlp_bwd_long_sums_of_the_hidden_gradient(case, dtype, device):
+    T, H, I, _ = case
+    assert _tile_choice(1, 3, T, I, _up64(H)) == (128, 128, 2, 1)
     test_mlp_bwd_matches_matmuls(case, dtype, device)
 
 
@@ -796,15 +823,6 @@ def test_mlp_on_lower_tiles(case, dtype, device):
     rows = err.norm(dim=1) / want.norm(dim=1)
     assert (rows <= 2 * eps).all().item(), rows.max().item()
     test_mlp_bwd_matches_matmuls(case, dtype, device)
-
-
-def _tile_choice(layout, epilogue, M, N, K):
-    """Rows and columns of the tiles of a product by itself, the groups of waves that share K, its parts: asked for before a test that means one kernel."""
-    import ctypes
-    from omni_moe.ops.hip import _lib
-    out = (ctypes.c_int32 * 4)()
-    assert _lib.load().omni_probe_tile_choice(layout, epilogue, M, N, K, ctypes.addressof(out)) == 0
-    return tuple(out)
 
 
 # T, H, I and the parts of gate and up on tiles of 64 x 64, whose ring has two stages for sums of up to 1536 and three beyond: four ring steps, both sides of the line, a K tail,
