@@ -1,7 +1,8 @@
 /* A plain C caller that runs compute entries of libomni_moe_hip.so on the GPU: omni_router_select on device buffers
  * it allocates and fills through the HIP runtime's C API, checked against a scalar loop over the same inputs; then
+ * omni_mlp_fwd eagerly and, at the same size, captured (other launches: a replay has no host work), which leaves the same bits; then
  * omni_init(), and straight after it -- no eager call came before -- HIP-graph captures of
- *   - omni_linear_fwd at a shape whose kernel needs 128 KiB of dynamic LDS: without omni_init() the call would have
+ *   - omni_linear_fwd at a shape whose kernel needs 112 KiB of dynamic LDS (64 are free to use): without omni_init() the call would have
  *     to raise that kernel's limit with hipFuncSetAttribute inside the capture; omni_init() has done it for every kernel,
  *   - omni_schedule and omni_schedule_noalloc side by side (the second on the device scratch that omni_init() resolved),
  * each replayed three times and checked against scalar loops.
@@ -27,7 +28,7 @@ static uint16_t bf16_of_int(int v) { float f = (float)v; uint32_t u; memcpy(&u, 
 static float float_of_bf16(uint16_t b) { uint32_t u = (uint32_t)b << 16; float f; memcpy(&f, &u, 4); return f; }
 
 /* omni_linear_fwd inside a stream capture, straight after omni_init().  2048 x 2048 outputs make the library pick its
- * 128 x 128 tile, whose kernel needs 128 KiB of dynamic LDS.  Operands are small integers, so every product and sum is
+ * 128 x 128 tile, whose kernel needs 112 KiB of dynamic LDS.  Operands are small integers, so every product and sum is
  * exact and the result must equal the scalar loop bit for bit. */
 static int captured_gemm(void) {
   uint16_t* x = (uint16_t*)malloc((size_t)GM * GK * 2); uint16_t* w = (uint16_t*)malloc((size_t)GN * GK * 2);
@@ -110,6 +111,46 @@ static int captured_schedule(void) {
   return 0;
 }
 
+/* omni_mlp_fwd of few tokens, eagerly in two launches and then captured, where it takes three; no omni_init() before: what ran eagerly can be captured */
+static int captured_mlp(void) {
+  enum { N = 16, H = 512, I = 2048 };
+  const size_t nx = (size_t)N * H, nw = (size_t)I * H;
+  uint16_t* v = (uint16_t*)malloc((nx + 3 * nw) * 2);
+  uint16_t* want = (uint16_t*)malloc(nx * 2); uint16_t* got = (uint16_t*)malloc(nx * 2);
+  if (!v || !want || !got) return 40;
+  uint32_t s = 99u;
+  for (size_t i = 0; i < nx + 3 * nw; ++i) { s = s * 1664525u + 1013904223u; v[i] = bf16_of_int((int)((s >> 12) % 5) - 2); }
+  uint8_t *d, *dy, *ws;
+  CHECK(hipMalloc((void**)&d, (nx + 3 * nw) * 2)); CHECK(hipMalloc((void**)&dy, nx * 2)); CHECK(hipMalloc((void**)&ws, omni_mlp_workspace_bytes(N, H, I, OMNI_BF16)));
+  CHECK(hipMemcpy(d, v, (nx + 3 * nw) * 2, hipMemcpyHostToDevice));
+  hipStream_t stream; hipGraph_t graph; hipGraphExec_t exec;
+  CHECK(hipStreamCreate(&stream));
+  int32_t code = omni_mlp_fwd(d, d + nx * 2, d + (nx + nw) * 2, d + (nx + 2 * nw) * 2, NULL, dy, N, H, I, OMNI_BF16, ws, stream);
+  if (code != OMNI_OK) { printf("omni_mlp_fwd: %s\n", omni_error_string(code)); return 41; }
+  CHECK(hipStreamSynchronize(stream));
+  CHECK(hipMemcpy(want, dy, nx * 2, hipMemcpyDeviceToHost));
+  CHECK(hipStreamBeginCapture(stream, hipStreamCaptureModeGlobal));
+  code = omni_mlp_fwd(d, d + nx * 2, d + (nx + nw) * 2, d + (nx + 2 * nw) * 2, NULL, dy, N, H, I, OMNI_BF16, ws, stream);
+  const hipError_t end = hipStreamEndCapture(stream, &graph);
+  if (code != OMNI_OK) { printf("omni_mlp_fwd under capture: %s\n", omni_error_string(code)); return 42; }
+  CHECK(end);
+  size_t nodes = 0;
+  CHECK(hipGraphGetNodes(graph, NULL, &nodes));
+  if (nodes != 3) { printf("omni_mlp_fwd captured: %d launches, want 3\n", (int)nodes); return 43; }
+  CHECK(hipGraphInstantiate(&exec, graph, NULL, NULL, 0));
+  for (int rep = 0; rep < 3; ++rep) {
+    CHECK(hipMemset(dy, 0xff, nx * 2));
+    CHECK(hipGraphLaunch(exec, stream));
+    CHECK(hipStreamSynchronize(stream));
+    CHECK(hipMemcpy(got, dy, nx * 2, hipMemcpyDeviceToHost));
+    if (memcmp(got, want, nx * 2)) { printf("mlp replay %d differs from the eager call\n", rep); return 44; }
+  }
+  CHECK(hipGraphExecDestroy(exec)); CHECK(hipGraphDestroy(graph)); CHECK(hipStreamDestroy(stream));
+  CHECK(hipFree(d)); CHECK(hipFree(dy)); CHECK(hipFree(ws));
+  free(v); free(want); free(got);
+  return 0;
+}
+
 int main(void) {
   /* fp32 logits with distinct values, so that ties play no part */
   static float lx[T * R], ly[T * R];
@@ -146,6 +187,8 @@ int main(void) {
     }
   }
   CHECK(hipFree(dlx)); CHECK(hipFree(dly)); CHECK(hipFree(dscores)); CHECK(hipFree(dids));
+  const int mlp = captured_mlp();
+  if (mlp) return mlp;
   int32_t init = omni_init();
   if (init != OMNI_OK) { printf("omni_init: %s\n", omni_error_string(init)); return 20; }
   if (omni_init() != OMNI_OK) { printf("second omni_init failed\n"); return 21; }

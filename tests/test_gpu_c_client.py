@@ -1,6 +1,7 @@
 """The C ABI from plain C on the GPU: tests/c_abi_gpu_client.c allocates device buffers with the HIP runtime's C API, calls
-omni_router_select through include/omni_moe_hip.h and checks ids and scores against a scalar loop; it then calls omni_init()
-and captures, without any eager call before, a GEMM whose kernel needs 128 KiB of dynamic LDS and the two schedule entry
+omni_router_select through include/omni_moe_hip.h and checks ids and scores against a scalar loop; it runs omni_mlp_fwd
+of few tokens eagerly and captures the same size, which takes other launches and leaves the same bits; it then calls omni_init()
+and captures, without any eager call before, a GEMM whose kernel needs 112 KiB of dynamic LDS and the two schedule entry
 points into HIP graphs, and checks three replays of each."""
 import os
 import subprocess
