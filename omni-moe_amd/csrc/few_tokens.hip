@@ -1,4 +1,4 @@
-// The layer (reference omni_moe/modules/omni_moe.py:60-106) for at most 64 tokens, as in decoding: three launches.
+// The layer (reference omni_moe/modules/omni_moe.py:60-106) for at most 64 tokens, as in decoding: three launches, or two.
 //
 // What bounds it.  The weights' one trip through memory (25 MB at hidden 1024 x intermediate 4096: 5 us) and, above all, the chain of
 // dependent launches: as six kernels -- projection, select, gate/up, experts, down projection, its partial sums -- the stages
@@ -6,9 +6,9 @@
 // each other shares a launch, by block index:
 //   1. the router's projection | gate and up with their SwiGLU product
 //   2. the router's selection  | the down projection, K split over the grid, as fp32 partial sums
-//   3. the experts, the partial sums and the final add, one block per token; for calls that the host takes longer for in launch 2 (further down).
+//   3. the experts, the partial sums and the final add, one block per token; in launch 2 where the host takes longer for a launch than the kernels do (merge_launches).
 // 1 token 38.4 -> 18.1 us a call, 48 tokens 42.9 -> 21.9 us, hidden 1024 x intermediate 4096; with the weights through LDS as well 17.2 -> 15.3 and 21.0 -> 20.1
-// (calls in a graph; a program sees the 18 us of host work of a call at 1 token, 15.2 with two launches).
+// (three launches in a graph; a program sees the 18 us of host work of a call at 1 token, 15.2 with two launches).
 //
 // Projections.  There is one row tile, so every weight is used once, and all loads of 1024 K values of a block are in flight at once.  They go through
 // each wave's own LDS all the same, because an instruction that reads eight whole 128-byte lines is faster than the one that a matrix fragment asks for,
@@ -214,8 +214,8 @@ __global__ __launch_bounds__(kFewThreads, Q == 1 || R8 == 1 ? 4 : 2) void few_fr
 // down projection and the token's experts; so a block per token selects and sums up its experts, and whoever comes last adds up: a ticket per token and
 // group of 32 columns, cleared by launch 1, counts the splits and the token's block, and the one that takes the last number finds all parts there and
 // writes y's 32 values.  Nobody waits.  What others read is stored and loaded at agent scope (the XCDs' L2s are not one cache), and a block takes its
-// numbers when its stores have been acknowledged.  Kernels of three launches / two in a graph, and calls as a program makes them: 1 token 15.3 / 14.9, 18.3 / 15.2 us;
-// 12 tokens 17.0 / 16.8; 512 x 2048, 1 token 9.8 / 9.9; but 24 tokens 18.2 / 18.3, 48 19.5 / 20.0, 64 22.3 / 23.4; 2048 x 8192, 1 token 33.6 / 34.0 (merge_launches).
+// numbers when its stores have been acknowledged.  Three launches / two as a program makes the call, 1 token: 18.3 / 15.2 us.  Replayed from a graph the kernels of two
+// take up to 5 % more, of the MLP alone up to 19 %; merge_launches has the figures.
 struct MiddleArgs {
   const uint8_t *h, *wd;
   float* parts;                      // [splits][T][H]

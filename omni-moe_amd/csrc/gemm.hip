@@ -622,7 +622,7 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_nt_dma_kernel(const GemmArgs 
 // (w % TM, w / TM) with the common epilogue.  Needs K % 64 == 0; worth it while there are fewer tiles than CUs.
 // TM = 1 where that makes at most 256 blocks and nothing runs beside the launch: every CU may have one, which loads three quarters as much, with three
 // stages in flight instead of two (router stage of 1000 / 2048 / 4096 tokens, hidden 1024, 64 keys: 16.3 / 16.8 / 19.3 -> 15.6 / 16.3 / 18.5 us).  Beside gate/up,
-// whose tiles take 128 KiB of LDS of a CU, blocks of both kinds wait for one another: the 4096-token layer on two streams 118 -> 130 us.
+// whose 256 x 256 tiles take all of a CU's LDS, blocks of both kinds wait for one another: the 4096-token layer on two streams 118 -> 130 us.
 template <int DT, int EPI, int TM>
 __global__ __launch_bounds__(kGemmThreads, 1) void gemm_ksplit_kernel(const GemmArgs g) {
   constexpr int kRow = 128, kATile = 32 * TM * kRow, kBTile = 64 * kRow, PA = 4 * TM, PB = 8;      // a K tile of each operand, in 1-KiB loads

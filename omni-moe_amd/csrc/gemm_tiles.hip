@@ -16,8 +16,8 @@ static float step_us(const ShapeCost& c, int64_t n) {
   const float used = n >= c.at_once ? 1.f : n > kCus ? 0.86f + 0.14f * (float)(n - kCus) / (c.at_once - kCus) : (float)n / c.at_once;
   return (float)rounds * (c.idle + (c.full - c.idle) * used);
 }
-// The fastest shape and K split by those figures.  K is split for a product on its own only, where every part keeps 256 of K, and the 64 x 64
-// shape (whose two groups also split K) is for K >= 512: shorter sums stay in one order whatever the shape.
+// The fastest shape and K split by those figures.  K is split for a product on its own only, where every part keeps 256 of K, and the shapes
+// whose two groups also split K (64 x 64; for dy W 128 x 128) are for K >= 512: shorter sums stay in one order whatever the shape.
 // joined: the layer's down projection, whose parts the experts' kernel adds up if they are of a shape that the selection runs beside.  A split costs that kernel's
 // longer wait then instead of a launch (kJoinedSumUs).  Over 36 layers where the figure decides (66 to 2475 tokens, hidden 256 to 1536) the call takes, with a launch's 3.3 us / with 1.8:
 // 197 x 512 x 1536 19.0 / 16.7 us, 221 x 1024 x 2048 23.5 / 21.1, 251 x 1536 x 3072 30.5 / 27.3, 613 x 1024 x 4096 41.2 / 38.8, 2475 x 512 x 2048 44.1 / 41.7, 85 x 256 x 1024

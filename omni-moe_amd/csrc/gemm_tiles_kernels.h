@@ -7,9 +7,10 @@
 // come out of LDS through the transposing read ds_read_b64_tr_b16 (within 16 lanes, lane i names 8 bytes, 4 elements, of row i / 4 of
 // a 4 x 16 block and receives column i of it; two of them give a lane the 8 consecutive K values of v_mfma_f32_16x16x32).
 //
-// What bounds it.  The 256 x 256 tile at K = 2048 and more: the matrix pipelines under the board's power limit (gate/up at 32768 x 2 8192 x 2048: busy 70 % of
-// the cycles at 1.90 GHz, 1.40 PFLOP/s); at K = 1024 the 16 ring steps between its fill and its epilogue (4096 x 2 4096 x 1024: 51 % at 2.08 GHz, 1.11
-// PFLOP/s with a block to a tile, 58 % and 1.23 streamed; d(h) with the SwiGLU backward as epilogue 57 us, 0.60 PFLOP/s, half of them its 134 MB).  The
+// What bounds it.  The 256 x 256 tile at K = 2048 and more: the matrix pipelines under the board's power limit (gate/up at 32768 x 2 8192 x 2048: busy 74 % of
+// the cycles at 1.88 GHz, 1.32 PFLOP/s in the layer, 1.45 in a counter run, which leaves gaps between launches); at K = 1024 the 16 ring steps between its fill and its epilogue
+// (4096 x 2 4096 x 1024: 57 % at 1.92 GHz, 1.14 PFLOP/s with a block to a tile, 58 % and 1.16 streamed; d(h) with the SwiGLU backward as epilogue 57 us, 0.60
+// PFLOP/s, half of them its 134 MB).  The
 // 128 x 128 tile: the path from L2 into LDS, which carries 64 bytes per cycle and CU -- what that tile asks for at full matrix rate --
 // and, with one block to a CU, the chain of reads and waits between two barriers.  So a block's waves keep 64 x 64 of the tile each (LDS
 // serves 256 bytes a cycle, and smaller wave tiles read more per product) and, alone on its CU, a block has three ring stages in flight (TileRing); the 64 x 64 tile
@@ -131,8 +132,8 @@ constexpr int staged_rows(int rows, int waves) {
 // Stages of the two operands in LDS: NS, and one more for one of them.  That one is requested in step 0 of a K tile, half a tile before the barrier that frees the
 // other's: requests are spread over the whole tile, and of two stages the second one's loads have between a half and a whole tile to arrive.  It is the right operand,
 // in a forward pass the weights, which come from further away, or the left one where a tile has more rows of it, or where the right one's does not fit.
-// Two stages against two and three, kernels alone: down of 32768 x 2048 x 8192 827 -> 793 us, the three weight gradients of 4096 x 1024 x 4096 95.6 -> 93.2 on 256 rows
-// and 102 -> 94.8 on 224, the SwiGLU backward 58.7 -> 57.3.
+// Kernels in traces of whole calls, from equal rings of two stages (with half of a step's requests just before the wait for them) to this one, mean of 45 launches each:
+// down of 32768 x 2048 x 8192 844 -> 791 us, gate/up there 1668 -> 1662; the five weight gradients of a 4096-token step 102 -> 94, its SwiGLU backward 59.4 -> 57.4, its d(x) 81 -> 75.
 // NS is no more than hides memory, for a block requests NS ring steps before its first matrix instruction, at some 20 cycles a load instruction and CU: a stage
 // costs every block 0.1 to 0.3 us.  Equal rings of NS + 1 / NS + 1 and one more for the left operand / as it is, us, weights in the caches, and from memory:
 //   64 x 64     65 x 1024 x 512   4.62 / 4.82 / 4.55   4.80 / 4.92 / 4.79     256 x 2048 x 4096   12.6 / 11.5 / 11.3   20.0 / 20.6 / 19.6
@@ -734,9 +735,10 @@ constexpr int kShapes = 10;
 constexpr unsigned shapes_of(int layout) { return layout == kNN ? (1u << kShapes) - 1 : (1u << 9) - 1; }
 // ... and what a launch of n blocks takes, in microseconds per 64 of K and round of `at_once` blocks: idle + (full - idle) times the share of
 // the chip in use.  Measured on 256 x 256 x 4096 (few blocks) and 4096 x 4096 x 4096 (all CUs busy), the lower tiles and the 64 x 64 one over 57 products of
-// 300 to 12000 rows, bf16, with one ring stage less than now; about 4 us more for a launch.  The times are lower now (tiles of 256 columns by 11 % at the median,
-// two 128 x 128 tiles to a CU 14 %, the others up to 4 %), their order is not: over 174 products (x W^T, dy W, gate/up with SwiGLU; 64 to 12000 rows, 128 to 8192
-// columns, K 256 to 8192) the rule's choice takes 0.24 % more than the best shape on average and 9 % at most, and with figures fitted to those 0.19 and 9.
+// 300 to 12000 rows, bf16, with equal rings of both operands; about 4 us more for a launch.  The times are lower now, and not all by the same share: over 174 products
+// (x W^T, gate/up with SwiGLU, dy W; 64 to 12000 rows, 128 to 8192 columns, K 256 to 8192; weights in the caches) the rule's choice takes 1.9 / 1.1 / 1.2 % more than the
+// best shape and split on average.  The most: 150 x 1496 x 6848, 96 x 128 in ten parts 15.6 us where 64 x 64 in three takes 12.9; gate/up of 293 x 2 2840 x 6912 17 %;
+// the rest 10 % at most.  Figures fitted to the present kernels would be the way to these.
 // The lower tiles took, the best of the others / theirs: gate/up of 3000 x 1024 x 4096 (256 tiles of 256 columns a round) 49.5 / 45.4 us, 613 x 1024 x 4096
 // 17.4 / 15.2; down of 3000 x 4096 x 1024 31.9 / 29.4, 12000 x 1536 x 512 23.7 / 19.6; five weight gradients of 4096 tokens x 1024 x 4096 (200 tiles of
 // 256 rows, 236 of 224), in a trace of whole steps, 106 / 101.

@@ -177,7 +177,7 @@ static int moe_fwd(const void* x, const void* gate_weight, const void* up_weight
 
   hipStream_t main_s = (hipStream_t)stream;
   // Up to a certain size the layer is joint launches on the caller's stream: stages that do not depend on each other share one.
-  //   * at most 64 tokens in eval mode (four row tiles, what a wave has registers and LDS for): few_tokens.hip, three launches; 64 tokens 44 -> 27 us (hidden 1024, bf16).
+  //   * at most 64 tokens in eval mode (four row tiles, what a wave has registers and LDS for): few_tokens.hip, two or three launches; 64 tokens 44 -> 27 us (hidden 1024, bf16).
   //   * up to 2^33 token x hidden x intermediate (2048 tokens at 1024 x 4096), beyond which gate/up fills the chip for several rounds and two streams are the
   //     better overlap: projection | gate/up, selection | down projection, experts and add.  The bound is this rule's own: a side stream that is given
   //     does not move it (OmniMoE.overlap_min_work, the least work that OmniMoE gives one for, is the same number so that the two schedules meet).
