@@ -19,9 +19,9 @@ static float step_us(const ShapeCost& c, int64_t n) {
 // The fastest shape and K split by those figures.  K is split for a product on its own only, where every part keeps 256 of K, and the shapes
 // whose two groups also split K (64 x 64; for dy W 128 x 128) are for K >= 512: shorter sums stay in one order whatever the shape.
 // joined: the layer's down projection, whose parts the experts' kernel adds up if they are of a shape that the selection runs beside.  A split costs that kernel's
-// longer wait then instead of a launch (kJoinedSumUs).  Over 36 layers where the figure decides (66 to 2475 tokens, hidden 256 to 1536) the call takes, with a launch's 3.3 us / with 1.8:
-// 197 x 512 x 1536 19.0 / 16.7 us, 221 x 1024 x 2048 23.5 / 21.1, 251 x 1536 x 3072 30.5 / 27.3, 613 x 1024 x 4096 41.2 / 38.8, 2475 x 512 x 2048 44.1 / 41.7, 85 x 256 x 1024
-// 16.5 / 15.2; one loses, 714 x 1280 x 5120 51.2 / 51.6.  With 1.0 or nothing 800 x 768 x 3072 leaves the selection no place, 31.5 / 35.1, and 277 x 256 x 1024 18.8 / 19.5.
+// longer wait then instead of a launch (kJoinedSumUs).  Layers in a graph, with a launch's 3.3 us / with 1.8: 197 x 512 x 1536 18.4 / 16.1 us, 221 x 1024 x 2048 23.8 / 21.0,
+// 251 x 1536 x 3072 30.4 / 26.9, 613 x 1024 x 4096 40.0 / 37.8, 2475 x 512 x 2048 48.2 / 45.5, 85 x 256 x 1024 15.6 / 14.2, 714 x 1280 x 5120 55.6 / 55.1; of 20 none is slower by more
+// than 0.3 %.  With 1.0 391 x 1024 x 2048 gains (26.0 -> 25.3) and 583 x 1280 x 3840 (43.1 -> 42.6), but 800 x 768 x 3072 leaves the selection no place, 33.7 -> 37.1.
 static TileChoice choose_of(int epilogue, const TileSize* sizes, int count, int64_t K, bool may_split, unsigned shapes, bool joined) {
   TileChoice best;
   for (int i = 0; i < kShapes; ++i) {
@@ -59,14 +59,17 @@ static TileChoice choose_tiles(int epilogue, const TileSize* sizes, int count, i
   return k.choice;
 }
 
-// The layer's down projection: a shape that takes the selection beside it, unless another one gains more than the selection's own launch costs
+// The layer's down projection: a shape that takes the selection beside it, unless another one gains more than the selection's own launch costs.  (That seldom decides: over the
+// 56 layers below, 0 us for that launch or any price makes none faster, and two slower by 2 %.)
 static TileChoice choose_down(const TileSize& size, int64_t K, bool may_split) {
   constexpr float kSelectUs = 6.f;
   const TileChoice any = choose_tiles(kTilePlain, &size, 1, K, may_split, kForwardShapes, true),
                    joint = choose_tiles(kTilePlain, &size, 1, K, may_split, kJointShapes, true);
   return joint.us <= any.us + kSelectUs ? joint : any;
 }
-// The shape that both products' tiles take least time in, by the figures above, if that is less than a launch for each; -1: it is not
+// The shape that both products' tiles take least time in, by the figures above, if that is less than a launch for each; -1: it is not.
+// Over 56 layers in a graph (65 to 3000 tokens, hidden 256 to 2048, 24 to 128 keys) a launch for each instead is slower by more than 1.5 % in 47 and faster in none (130 x 1536 x 3072
+// 23.8 / 31.2 us); one launch always is faster in none.
 static int choose_pair(const TileSize& router, const TileSize& mlp, int64_t K) {
   const TileSize sizes[2] = {router, mlp};
   const int64_t kt = (K + 63) / 64;
