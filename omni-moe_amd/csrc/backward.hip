@@ -298,7 +298,7 @@ __global__ __launch_bounds__(kFinishWaves* kWave) void router_norm_bwd_finish_ke
 }
 
 // ---- experts, token pass -----------------------------------------------------------------------
-// Both organisations are bound as the forward's are: gather by the rows' trip over the fabric, split by the vector-memory path on rows that an XCD's
+// Both organisations are bound as the forward's are: gather by the rows' trip over the fabric, split on the chip, by loads and arithmetic on rows that an XCD's
 // L2 holds; split needs the sums over the slices in between, so the forward keeps its <x, U> (4 bytes a pair) and only <dy, V> is formed here.
 // The sort of the pairs, which only the weight pass needs, runs beside: the token pass comes in two launches whose first blocks sort, the count
 // pass beside the first and the scatter pass beside the second.  All blocks have the sort's threads.
